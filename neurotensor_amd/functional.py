@@ -328,6 +328,11 @@ def unfold2d_backward(col, output_size, kernel_size, dilation=1, padding=0, stri
 
 def conv2d_backward(image, kernel, grad, stride=1, padding=0, dilation=1, groups=1):
     """conv_dimage + conv_dkernel for dim == 2 (conv.cpp:318-346, 444-471): returns (d_image, d_kernel)."""
+    return _conv2d_gradients(image, kernel, grad, stride, padding, dilation, groups)
+
+
+def _conv2d_gradients(image, kernel, grad, stride, padding, dilation, groups, want_dx=True):
+    """want_dx=False: (None, d_kernel) -- the transposed convolution's backward has no use for the other one."""
     _require_device(image, kernel, grad)
     s, p, d = _pair(stride), _pair(padding), _pair(dilation)
     x = image.reshape((1,) + tuple(image.shape)) if image.dim() == 3 else image.reshape((-1,) + tuple(image.shape[-3:]))
@@ -346,12 +351,12 @@ def conv2d_backward(image, kernel, grad, stride=1, padding=0, dilation=1, groups
     Wo = (W + 2 * p[1] - d[1] * (kw - 1) - 1) // s[1] + 1
     if g.numel() != B * O * Ho * Wo:
         raise ValueError(f"grad has {g.numel()} elements, expected {(B, O, Ho, Wo)}")
-    dx = torch.empty_like(x)
+    dx = torch.empty_like(x) if want_dx else None
     dw = torch.empty_like(w)
     ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=x.device)
-    check(L.ntg_conv2d_backward_dev(dt, x.data_ptr(), w.data_ptr(), g.data_ptr(), dx.data_ptr(), dw.data_ptr(), ws.data_ptr(), ws_bytes,
+    check(L.ntg_conv2d_backward_dev(dt, x.data_ptr(), w.data_ptr(), g.data_ptr(), dx.data_ptr() if want_dx else None, dw.data_ptr(), ws.data_ptr(), ws_bytes,
                                     B, C, H, W, O, kh, kw, s[0], s[1], p[0], p[1], d[0], d[1], groups, 0, _stream()))
-    return dx.reshape(image.shape), dw.reshape(kernel.shape)
+    return dx.reshape(image.shape) if want_dx else None, dw.reshape(kernel.shape)
 
 
 def conv1d(image, kernel, stride=1, padding=0, dilation=1, groups=1):
@@ -436,7 +441,7 @@ def conv_transpose2d_backward(image, kernel, grad, stride=1, padding=0, output_p
     w = kernel.reshape((1,) + tuple(kernel.shape)) if kernel.dim() == 3 else kernel
     g = grad.reshape((x.shape[0], w.shape[1] * groups) + tuple(grad.shape[-2:])).contiguous()
     dx = conv2d(g, w, s, p, d, groups)
-    _, dw = conv2d_backward(g, w, x.contiguous(), s, p, d, groups)
+    _, dw = _conv2d_gradients(g, w, x.contiguous(), s, p, d, groups, want_dx=False)
     return dx.reshape(image.shape), dw.reshape(kernel.shape)
 
 
@@ -505,6 +510,11 @@ def convnd(image, kernel, stride=1, padding=0, dilation=1, groups=1):
 
 def convnd_backward(image, kernel, grad, stride=1, padding=0, dilation=1, groups=1):
     """conv_dimage + conv_dkernel for 1..4 spatial axes (conv.cpp:318-535): returns (d_image, d_kernel)."""
+    return _convnd_gradients(image, kernel, grad, stride, padding, dilation, groups)
+
+
+def _convnd_gradients(image, kernel, grad, stride, padding, dilation, groups, want_dx=True):
+    """want_dx=False: (None, d_kernel)."""
     _require_device(image, kernel, grad)
     nd = kernel.dim() - 2
     s, p, d = _ntuple(stride, nd), _ntuple(padding, nd), _ntuple(dilation, nd)
@@ -518,9 +528,9 @@ def convnd_backward(image, kernel, grad, stride=1, padding=0, dilation=1, groups
     ws_bytes = L.ntg_convnd_workspace_bytes(dt, B, C, O, nd, *geo, groups, 1)
     if ws_bytes < 0:
         raise ValueError("invalid convolution geometry")
-    dx, dw = torch.empty_like(x), torch.empty_like(w)
+    dx, dw = torch.empty_like(x) if want_dx else None, torch.empty_like(w)
     ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=x.device)
-    check(L.ntg_convnd_backward_dev(dt, x.data_ptr(), w.data_ptr(), g.data_ptr(), dx.data_ptr(), dw.data_ptr(), ws.data_ptr(), ws_bytes,
+    check(L.ntg_convnd_backward_dev(dt, x.data_ptr(), w.data_ptr(), g.data_ptr(), dx.data_ptr() if want_dx else None, dw.data_ptr(), ws.data_ptr(), ws_bytes,
                                     B, C, O, nd, *geo, groups, 0, _stream()))
     return dx, dw
 
@@ -577,7 +587,7 @@ def conv_transposend_backward(image, kernel, grad, stride=1, padding=0, output_p
     with image and output gradient exchanged."""
     g = grad.contiguous()
     dx = convnd(g, kernel, stride, padding, dilation, groups)
-    _, dw = convnd_backward(g, kernel, image.contiguous(), stride, padding, dilation, groups)
+    _, dw = _convnd_gradients(g, kernel, image.contiguous(), stride, padding, dilation, groups, want_dx=False)
     return dx.reshape(image.shape), dw
 
 
