@@ -218,9 +218,11 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams p) {
     constexpr int A_TILE_BYTES = GA::TILE_BYTES, STAGE_BYTES = GA::TILE_BYTES + G::TILE_BYTES;
     constexpr int WTM = GA::WT, WTN = G::WT;             // a wavefront's share of the tile: WTM rows x WTN columns
     constexpr bool GATHER4 = CONV == 1 || CONV == 2;     // op(B) gathered element by element from an NCHW image
-    constexpr bool GATHER16 = CONV == 3 || CONV == 5;    // op(B) = col^T gathered in 16-byte pieces from a channels-last image
-    constexpr bool HALO = CONV == 5;                     // ... whose copy carries the padding as pixels of zeros: every tap of every window exists
-    constexpr bool GATHERW = CONV == 4;                  // op(B) = col^T of a channels-last image, 16-byte pieces along the channels (weight gradient)
+    constexpr bool GATHER16 = CONV == 3 || CONV == 5 || CONV == 6;   // op(B) = col^T gathered in 16-byte pieces from a channels-last image
+    constexpr bool HALO = CONV == 5 || CONV == 6;        // ... whose copy carries the padding as pixels of zeros: every tap of every window exists
+    constexpr bool DEPTH = CONV == 6;                    // ... over three spatial axes
+    constexpr bool GATHERW = CONV == 4 || CONV == 7;     // op(B) = col^T of a channels-last image, 16-byte pieces along the channels (weight gradient)
+    constexpr bool DEPTHW = CONV == 7;                   // ... of a bordered copy over two or three axes, pixel by division (no table of window origins)
     constexpr bool A_KC = !TA, B_KC = GATHER4 ? false : GATHER16 ? true : GATHERW ? false : TB;
     constexpr int BK = G::BK;
     static_assert(!GATHER4 || (ES == 4 && !TA && RAGGED), "gathered operands: Float32, A stored [m][k], guarded edges");
@@ -236,7 +238,7 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams p) {
     __shared__ __attribute__((aligned(1024))) char st2[STAGE_BYTES];
     __shared__ __attribute__((aligned(1024))) char st3[RING3 ? 1024 : STAGE_BYTES];
     // channels-last weight gradient: byte offset of every output pixel's window origin inside one (bordered) image
-    constexpr int DW_TABLE = CONV == 4 ? dw_table_entries(WB) : 1;
+    constexpr int DW_TABLE = CONV == 4 ? dw_table_entries(WB) : 1;   // (CONV = 7 has none)
     __shared__ int dw_tab[DW_TABLE];
 
     if (p.gate && *p.gate != p.gate_want) return;       // (uniform: the other kernel of a gated pair does this product)
@@ -306,9 +308,13 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams p) {
 
     // ---- DMA sources: uniform tile base (advances by adv bytes per K-step) + per-lane offsets ----
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-    const int KT = (p.K + BK - 1) / BK;
+    int K = p.K;
+    if constexpr (GATHERW) {
+        if (p.conv.k_ranges && p.conv.k_total - b * p.K < K) K = p.conv.k_total - b * p.K;      // (uniform) the last k range is what is left
+    }
+    const int KT = (K + BK - 1) / BK;
     const int last = KT - 1;
-    const int kr = p.K - last * BK;                                  // k that exist in the last K-step (a multiple of one chunk)
+    const int kr = K - last * BK;                                    // k that exist in the last K-step (a multiple of one chunk, or the gathered operand is zero past it)
     const int mvalid = p.M - m0 < GA::BM ? p.M - m0 : GA::BM;
     const int nvalid = p.N - n0 < G::BN ? p.N - n0 : G::BN;
     uint32_t offA[WBM * KD], offB[WBN * KD];      // K-steps before the last
@@ -431,16 +437,20 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams p) {
     // taps of one tap row (the row padded to p.conv.kq_pad taps with zero weights): a lane's 16-byte slot then belongs to
     // tap q + tq3 of the step, which shifts its address and its validity bit.
     uint32_t lanepart3[WB], cmask3[WB], tq3[WB];
-    int k3_c0 = 0, k3_q = 0, k3_r = 0, k3_up = 0, k3_k = 0, k3_cg = 1;
+    // Three spatial axes (CONV = 6, bordered copies only): the depth is one more digit of the output pixel, set up once per lane,
+    // and of the tap, one more carry of the uniform counters.  An instantiation of its own: as a digit that is always zero the
+    // carry cost the two-axis kernel 4 % (64 x 256 x 56 x 56, 3 x 3 BFloat16: 272 -> 284 us).
+    int k3_c0 = 0, k3_q = 0, k3_r = 0, k3_t = 0, k3_up = 0, k3_k = 0, k3_cg = 1;
     if constexpr (GATHER16) {
         const ConvGeom& g = p.conv;
-        k3_cg = p.K / g.k_rc;
+        k3_cg = p.K / g.k_drc;
         k3_up = -(g.p_r * g.W + g.p_c) * g.chan * ES;
 #pragma unroll
         for (int x = 0; x < WB; ++x) {
             const int row = 16 * (wave * WB + x) + (lane >> 2);
             const int n = n0 + row;
-            const uint32_t l = (n < p.N ? (uint32_t)n : 0u) + (uint32_t)g.n_base;
+            const uint32_t ld = (n < p.N ? (uint32_t)n : 0u) + (uint32_t)g.n_base;
+            const uint32_t od = DEPTH ? fast_div(ld, g.div_howo) : 0u, l = DEPTH ? ld - od * (uint32_t)g.HoWo : ld;
             const uint32_t oh = fast_div(l, g.div_wo), ow = l - oh * (uint32_t)g.Wo;
             const int ih0 = (int)oh * g.s_r - g.p_r, iw0 = (int)ow * g.s_c - g.p_c;
             uint32_t m = 0;
@@ -458,7 +468,8 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams p) {
                 cho -= tq * cb;
             }
             tq3[x] = tq;
-            lanepart3[x] = (oh * (uint32_t)g.s_r * (uint32_t)g.W + ow * (uint32_t)g.s_c + tq * (uint32_t)g.d_c) * (uint32_t)g.chan * (uint32_t)ES + cho;
+            lanepart3[x] = ((od * (uint32_t)g.s_d * (uint32_t)g.H + oh * (uint32_t)g.s_r) * (uint32_t)g.W + ow * (uint32_t)g.s_c + tq * (uint32_t)g.d_c) *
+                           (uint32_t)g.chan * (uint32_t)ES + cho;
         }
     }
     // instruction x (0 .. WB - 1) of this wavefront's share of the NEXT gathered tile; the K-step's counters move on after the last
@@ -490,8 +501,17 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams p) {
                 up = w0 ? up - g.k_c * g.d_c * g.chan * ES + g.d_r * g.W * g.chan * ES : up;
                 const bool w1 = r >= g.k_r;
                 r = w1 ? 0 : r;
-                c0 = w1 ? c0 + BK : c0;
-                up = w1 ? up - g.k_r * g.d_r * g.W * g.chan * ES + BK * ES : up;
+                if constexpr (DEPTH) {
+                    int t = w1 ? k3_t + 1 : k3_t;
+                    up = w1 ? up + (g.d_d * g.H - g.k_r * g.d_r) * g.W * g.chan * ES : up;
+                    const bool w2 = t >= g.k_d;
+                    k3_t = w2 ? 0 : t;
+                    c0 = w2 ? c0 + BK : c0;
+                    up = w2 ? up - g.k_d * g.d_d * g.H * g.W * g.chan * ES + BK * ES : up;
+                } else {
+                    c0 = w1 ? c0 + BK : c0;
+                    up = w1 ? up - g.k_r * g.d_r * g.W * g.chan * ES + BK * ES : up;
+                }
                 k3_c0 = c0; k3_up = up; k3_q = q; k3_r = r; k3_k += BK;
             }
             if (!(HALO && g.tap_inner) && x == WB - 1) {
@@ -507,6 +527,11 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams p) {
                 q = w1 ? 0 : q;
                 up = w1 ? up - qend * g.d_c * g.chan * ES + g.d_r * g.W * g.chan * ES : up;
                 r = w1 ? r + 1 : r;
+                if constexpr (DEPTH) {
+                    const bool w2 = r >= g.k_r;
+                    r = w2 ? 0 : r;
+                    up = w2 ? up + (g.d_d * g.H - g.k_r * g.d_r) * g.W * g.chan * ES : up;
+                }
                 k3_c0 = merged ? 0 : c0; k3_up = up; k3_q = q; k3_r = r; k3_k += BK;
             }
         }
@@ -517,8 +542,10 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams p) {
     // WB 16-byte DMA instructions per wavefront; a lane's 16 bytes are channels c .. of ONE tap for the whole K loop
     // (tap reach and byte offset kept per lane), and its k-row moves on by BK output pixels per K-step: the pixel is
     // split into (row, column) with one multiply-shift division per instruction.  Padding and k >= K read zeros.
-    // Several images may share one K loop (p.conv.fold_L = output pixels per image, 0: one image): k then counts the
-    // output pixels of consecutive images, and one more division gives the image, p.conv.fold_stride elements apart.
+    // Items that are k ranges (p.conv.k_ranges, fold_L = output pixels per image) count k through the output pixels of all
+    // images, and one more division gives the image, p.conv.fold_stride elements apart.
+    // CONV = 7: the copy carries its padding as zeros (the only form for three spatial axes, and what large output planes take),
+    // which needs no validity test; without the table its LDS lets a fourth 64 x 64 workgroup onto the CU.
     int krow4[WB], noff4[WB];
     uint32_t tap4[WB];
     int k4_k = 0, k4_base = 0;
@@ -526,7 +553,7 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams p) {
         const ConvGeom& g = p.conv;
         constexpr int CH = G::CHUNKS;
         if (g.k_ranges) k4_base = b * p.K;                         // this item's first output pixel, counted through the images
-        const uint32_t cgc = (uint32_t)(g.n_total ? g.n_total : p.N) / (uint32_t)g.k_rc;   // channels of the slice: N = taps * channels
+        const uint32_t cgc = (uint32_t)(g.n_total ? g.n_total : p.N) / (uint32_t)g.k_drc;  // channels of the slice: N = taps * channels
 #pragma unroll
         for (int x = 0; x < WB; ++x) {
             const int j = wave * WB + x;
@@ -534,11 +561,13 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams p) {
             const int chunk = (lane % CH) ^ (ES == 2 ? 2 * (krow & 3) : 8 * (krow & 1));
             const int n = n0 + chunk * G::VEL;
             const uint32_t nn = (n < p.N ? (uint32_t)n : 0u) + (uint32_t)g.n_base;
-            const uint32_t t = nn / cgc, c = nn - t * cgc;
+            const uint32_t td = nn / cgc, c = nn - td * cgc;
+            const uint32_t d = fast_div(td, g.div_krc), t = td - d * (uint32_t)g.k_rc;
             const uint32_t r = fast_div(t, g.div_kc), q = t - r * (uint32_t)g.k_c;
             krow4[x] = n < p.N ? krow : 0x40000000;                       // columns past the edge: never inside
             tap4[x] = (r * (uint32_t)g.d_r) | ((q * (uint32_t)g.d_c) << 16);
-            noff4[x] = (((int)(r * (uint32_t)g.d_r) - g.p_r) * g.W + ((int)(q * (uint32_t)g.d_c) - g.p_c)) * g.chan * ES + (int)c * ES;
+            noff4[x] = (((int)(d * (uint32_t)g.d_d * (uint32_t)g.H + r * (uint32_t)g.d_r) - g.p_r) * g.W + ((int)(q * (uint32_t)g.d_c) - g.p_c)) * g.chan * ES +
+                       (int)c * ES;
         }
     }
     // Table form (p.conv.pix_table = output pixels per image, at most DW_TABLE - BK; the copy of the image carries its padding
@@ -551,7 +580,7 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams p) {
     int64_t t4_img = 0, t4_imgn = 0;
     if constexpr (GATHERW) {
         const ConvGeom& g = p.conv;
-        if (g.pix_table) {                                        // (uniform)
+        if (!DEPTHW && g.pix_table) {                             // (uniform)
             const int Lp = g.pix_table;
             for (int i = tid; i < Lp + BK; i += 256) {
                 const uint32_t oh = fast_div((uint32_t)i, g.div_wo), ow = (uint32_t)i - oh * (uint32_t)g.Wo;
@@ -574,9 +603,9 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams p) {
         if constexpr (GATHERW) {
             const ConvGeom& g = p.conv;
             const char* img = reinterpret_cast<const char*>(B);
-            if (g.pix_table) {                                     // (uniform)
+            if (!DEPTHW && g.pix_table) {                          // (uniform)
                 const uint32_t lk = (uint32_t)(k4_k + krow4[x]);
-                const char* src = lk < (uint32_t)p.K ? img + (t4_img + (int64_t)(pre4[x] + noff4[x])) : reinterpret_cast<const char*>(ring_zero_word);
+                const char* src = lk < (uint32_t)K ? img + (t4_img + (int64_t)(pre4[x] + noff4[x])) : reinterpret_cast<const char*>(ring_zero_word);
                 asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
                              :: "s"(lds_tile + (uint32_t)(wave_u * WB + x) * 1024u), "v"(src) : "memory");
                 const int pn = t4_pixn < g.pix_table ? t4_pixn : g.pix_table;      // (K-steps past the end: the zeros behind the table)
@@ -591,15 +620,26 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams p) {
             }
             const uint32_t lk = (uint32_t)(k4_k + krow4[x]), l = lk + (uint32_t)k4_base;
             uint32_t li = l, im = 0u;
-            if (g.fold_L) {                                        // (uniform)
+            if (g.k_ranges) {                                      // (uniform)
                 im = fast_div(l, g.div_fold);
                 li = l - im * (uint32_t)g.fold_L;
             }
-            const uint32_t oh = fast_div(li, g.div_wo), ow = li - oh * (uint32_t)g.Wo;
-            const int ih0 = (int)oh * g.s_r - g.p_r, iw0 = (int)ow * g.s_c - g.p_c;
-            const bool ok = (lk < (uint32_t)p.K) & ((uint32_t)(ih0 + (int)(tap4[x] & 0xffffu)) < (uint32_t)g.H) &
-                            ((uint32_t)(iw0 + (int)(tap4[x] >> 16)) < (uint32_t)g.W);
-            const int off = (int)((oh * (uint32_t)g.s_r * (uint32_t)g.W + ow * (uint32_t)g.s_c) * (uint32_t)g.chan * (uint32_t)ES) + noff4[x];
+            bool ok = lk < (uint32_t)K;
+            uint32_t oh, ow;
+            if constexpr (DEPTHW) {
+                const uint32_t od = fast_div(li, g.div_howo);
+                li -= od * (uint32_t)g.HoWo;
+                oh = fast_div(li, g.div_wo);
+                ow = li - oh * (uint32_t)g.Wo;
+                oh = oh * (uint32_t)g.s_r + od * (uint32_t)(g.s_d * g.H);
+            } else {
+                oh = fast_div(li, g.div_wo);
+                ow = li - oh * (uint32_t)g.Wo;
+                oh *= (uint32_t)g.s_r;
+                const int ih0 = (int)oh - g.p_r, iw0 = (int)ow * g.s_c - g.p_c;
+                ok = ok & ((uint32_t)(ih0 + (int)(tap4[x] & 0xffffu)) < (uint32_t)g.H) & ((uint32_t)(iw0 + (int)(tap4[x] >> 16)) < (uint32_t)g.W);
+            }
+            const int off = (int)((oh * (uint32_t)g.W + ow * (uint32_t)g.s_c) * (uint32_t)g.chan * (uint32_t)ES) + noff4[x];
             const char* src = ok ? img + ((int64_t)im * g.fold_stride * ES + (int64_t)off) : reinterpret_cast<const char*>(ring_zero_word);
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
                          :: "s"(lds_tile + (uint32_t)(wave_u * WB + x) * 1024u), "v"(src) : "memory");
@@ -623,7 +663,7 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams p) {
     // multiply k = (0, 1), (2, 3), (4, 5), (6, 7) in that order and every output element is the reference's own chain
     // c = fma(a_k, b_k, c) in ascending k.  Both layouts are therefore read one dword per element, element e = k 2 e + lane / 32
     // (a 16-byte read of a K-major row would hand a lane four consecutive k, and rearranging them with cross-lane moves in the
-    // MFMA stream was measured 4 % slower per K-major operand).  The channels-last convolution (CONV = 3 / 5: both operands
+    // MFMA stream was measured 4 % slower per K-major operand).  The channels-last convolution (CONV = 3 / 5 / 6: both operands
     // K-major), whose k runs taps-outermost and so cannot be the reference's order anyway, keeps the 16-byte reads: element e
     // of both operands is k = e (lanes 0..31) | 4 + e (lanes 32..63), the same pairs on both sides.
     // K-major: block b of the wavefront, row = wbase + 32 b + lane%32, slot (2 ks + lane/32) ^ ((row>>1)&3)
@@ -711,7 +751,7 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams p) {
         }
         if constexpr (GATHERW && A_KC) {
             if (p.conv.a_steps) {                                  // (uniform) K-step counted through the images -> image, step inside it
-                const uint32_t gs = (uint32_t)(b * KT + kc), im = fast_div(gs, p.conv.div_a_steps);
+                const uint32_t gs = (uint32_t)(b * (p.K / BK) + kc), im = fast_div(gs, p.conv.div_a_steps);
                 return tile_src(baseA + ((int64_t)im * p.conv.a_image_stride * ES + (int64_t)(gs - im * (uint32_t)p.conv.a_steps) * advA));
             }
         }
@@ -1220,7 +1260,7 @@ static hipError_t launch_ring_conv_cfg(bool tb, const GemmParams& pin, hipStream
     return hipGetLastError();
 }
 
-// ... from a channels-last image that carries its padding as zero pixels (CONV = 5)
+// ... from a channels-last image that carries its padding as zero pixels (CONV = 5; three spatial axes: 6)
 template <int DT, int WB>
 static hipError_t launch_ring_nhwc_halo_cfg(const GemmParams& pin, hipStream_t s) {
     constexpr int TE = RingGeom<WB, (int)sizeof(typename Elem<DT>::T)>::BM;
@@ -1230,7 +1270,8 @@ static hipError_t launch_ring_nhwc_halo_cfg(const GemmParams& pin, hipStream_t s
     const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n * p.batch;
     if (blocks <= 0) return hipSuccess;
     if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 5>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+    if (p.conv.k_d > 1 || p.conv.D > 1) hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 6>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 5>), dim3((unsigned)blocks), dim3(256), 0, s, p);
     return hipGetLastError();
 }
 
@@ -1249,7 +1290,7 @@ static hipError_t launch_ring_nhwc_cfg(const GemmParams& pin, hipStream_t s) {
     return hipGetLastError();
 }
 
-// weight gradient of a convolution with op(B) gathered from a channels-last image (see CONV = 4)
+// weight gradient of a convolution with op(B) gathered from a channels-last image (see CONV = 4 and 7)
 template <int DT, int WB, bool TA = false>
 static hipError_t launch_ring_nhwc_dw_cfg(const GemmParams& pin, hipStream_t s) {
     constexpr int TE = RingGeom<WB, (int)sizeof(typename Elem<DT>::T)>::BM;
@@ -1261,7 +1302,8 @@ static hipError_t launch_ring_nhwc_dw_cfg(const GemmParams& pin, hipStream_t s) 
     if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
     // (more output pixels per image than the table holds: the divisions per instruction, which serve a bordered copy as well)
     if (p.conv.pix_table + 64 > dw_table_entries(WB)) p.conv.pix_table = 0;
-    hipLaunchKernelGGL((gemm_ring_kernel<DT, TA, false, true, WB, 4>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+    if (p.conv.halo && !p.conv.pix_table) hipLaunchKernelGGL((gemm_ring_kernel<DT, TA, false, true, WB, 7>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((gemm_ring_kernel<DT, TA, false, true, WB, 4>), dim3((unsigned)blocks), dim3(256), 0, s, p);
     return hipGetLastError();
 }
 
@@ -1300,7 +1342,7 @@ static hipError_t launch_ring16_planned(const GemmParams& p, hipStream_t s, Laun
 // of their own (see ring16_column_split); each part planned over the batch like any other
 template <class Launch>
 static hipError_t launch_conv_nhwc16_planned(const GemmParams& p, hipStream_t s, Launch&& launch) {
-    if (p.conv.k_ranges) return launch(ring16_tile_edge(p.M, p.N, p.K, p.batch), p);     // items are k ranges: one launch, planned by the caller
+    if (p.conv.tile_edge) return launch(p.conv.tile_edge, p);                              // items are k ranges: one launch, planned by the caller
     const int64_t head_cols = p.cmode == C_PARTIAL ? 0 : ring16_column_split(p.M, p.N, p.K, p.batch);
     if (head_cols == 0) return launch_ring16_planned(p, s, launch);
     GemmParams head = p, tail = p;

@@ -53,15 +53,14 @@ struct ConvGeom {
     int k_d, k_r, k_c, k_rc, k_drc, Wo, HoWo;
     int last;                // index of the last element of the image slice at p.B (loads are clamped to it)
     FastDiv div_kdrc, div_krc, div_kc, div_wo, div_howo;
-    // channels-last weight gradient with several images per K loop: output pixels per image (0: one image per item),
-    // its divider, and the elements from one image to the next
+    // channels-last weight gradient, items = k ranges: output pixels per image, its divider, and the elements from one image to the next
     int fold_L;
     FastDiv div_fold;
     int64_t fold_stride;
     // channels-last convolution of few channels: taps of one tap row per K-step (0 / 1: one tap) and the padded row length
     int tap_step, kq_pad;
-    // channels-last convolution: the copy of the image carries the padding as pixels of zeros (H, W, chan describe the padded
-    // image, p_r = p_c = 0), so the gather needs no validity test
+    // channels-last convolution: the copy of the image carries the padding as pixels of zeros (D, H, W, chan describe the padded
+    // image, all paddings 0), so the gather needs no validity test; the form that three spatial axes take
     int halo;
     // ... and k runs (64-byte run of channels, tap, channel inside the run) instead of (tap, channel): the taps of a run reach
     // the same pixels while they are in L2 (unit strides; the weights are permuted to match)
@@ -69,16 +68,18 @@ struct ConvGeom {
     // channels-last convolution and weight gradient: column n of this launch is column n + n_base of the whole product
     // (a launch on the trailing columns); n_total = columns of the whole product (0: this launch has them all)
     int n_base, n_total;
-    // channels-last weight gradient, items = k ranges: the k axis is the output pixels of ALL images counted through, item b
-    // covers pixels [b K, (b + 1) K) of it (K a whole number of K-steps, and so is an image: a K-step never straddles two).
-    // The gathered operand finds image and pixel by division (fold_L, fold_stride as above); dY, read where it lies as
-    // [image][out channel][pixel], jumps a_image_stride elements after every a_steps K-steps.  0: off.
-    int k_ranges, a_steps;
+    // channels-last weight gradient, items = k ranges: the k axis is the output pixels of ALL images counted through (k_total of
+    // them), item b covers pixels [b K, (b + 1) K) of it, the last one what is left (K is a whole number of K-steps).  The gathered
+    // operand finds image and pixel by division (fold_L, fold_stride).  dY read where it lies as [image][out channel][pixel] (an image
+    // is whole K-steps then) jumps a_image_stride elements after every a_steps K-steps; read from a channels-last copy, it is one
+    // [pixel][out channel] matrix (a_steps = 0).  k_ranges = 0: one product per image.
+    int k_ranges, k_total, a_steps;
     FastDiv div_a_steps;
     int64_t a_image_stride;
     // channels-last weight gradient on a copy that carries the padding as pixels of zeros (H, W describe the padded image,
     // p_r = p_c = 0): output pixels per image when the kernel keeps their window origins in an LDS table, 0: off
     int pix_table;
+    int tile_edge;           // channels-last weight gradient: the tile the caller planned with (0: the launcher's own choice)
 };
 
 struct GemmParams {
@@ -341,9 +342,14 @@ hipError_t launch_splitk_reduce(int dtype, const void* part, int splits, const G
 // conv2d backward helpers (unfold2d.hip): ordered sum of per-image weight gradients; weights of
 // the gradient-to-image convolution
 hipError_t launch_reduce_batch(int dtype, const void* part, void* out, int64_t batch, int64_t n, int accumulate, hipStream_t s);
-// Where the pixels of a channels-last copy go when the copy carries a border of zero pixels: pixel (h, w) of a W-wide image is
-// pixel (h + top) * Wp + (w + left) of a padded image of Hp x Wp pixels.  nullptr / Wp == 0: no border.
-struct HaloMap { int64_t W, H, Wp, Hp, top, left; };
+// Where the pixels of a channels-last copy go when the copy carries a border of zero pixels: pixel (d, h, w) of a D x H x W image
+// is pixel ((d + front) * Hp + h + top) * Wp + (w + left) of a padded image of Dp x Hp x Wp pixels (two axes: D = Dp = 1,
+// front = 0).  nullptr / Wp == 0: no border.
+struct HaloMap {
+    int64_t W, H, Wp, Hp, top, left, D, Dp, front;
+    __host__ __device__ int64_t vol() const { return Dp * Hp * Wp; }
+    __host__ __device__ int64_t border() const { return vol() - D * H * W; }
+};
 // A weight permutation that the launch of a channels-last copy can take along (its blocks share the elements after
 // their tiles): kind 1 = launch_weights_channels_last(w, wp, rows = a, cg, cgp, taps, chunk), kind 2 =
 // launch_flip_weights_channels_last(w, wp, groups = a, og, ogp, cg, taps, chunk).
@@ -379,8 +385,9 @@ struct IntPlanesParams { int M, N, K, Kp, Np, batch; int64_t lda, ldb, sA, sB; i
 hipError_t launch_int_split_planes(int planes, const void* A, const void* B, void* a_planes, void* b_planes, const IntPlanesParams& q, hipStream_t s);
 hipError_t launch_int_combine(int planes, const void* parts, const GemmParams& p, int Np, hipStream_t s);
 hipError_t launch_conv_nhwc_dw(int dtype, bool ta, const GemmParams& p, hipStream_t s);   // ta: A (the output gradient) stored [k][m]
-hipError_t launch_reduce_batch_taps_last(int dtype, const void* part, void* out, int64_t batch, int64_t rows, int64_t cg, int64_t cgp,
-                                         int64_t taps, int accumulate, hipStream_t s);   // part rows hold cgp >= cg channels per tap
+// part rows hold cgp >= cg channels per tap; part_f32: the partial sums are Float32 whatever the dtype
+hipError_t launch_reduce_batch_taps_last(int dtype, bool part_f32, const void* part, void* out, int64_t batch, int64_t rows, int64_t cg, int64_t cgp,
+                                         int64_t taps, int accumulate, hipStream_t s);
 hipError_t launch_flip_weights(int64_t elem_size, const void* w, void* wt, int64_t groups, int64_t og, int64_t cg, int64_t taps, hipStream_t s);
 
 // padded copies of operands whose rows are not 16-byte multiples (pad_copy.hip); es = 1, 2, 4 or 8 bytes per element, sizes in elements

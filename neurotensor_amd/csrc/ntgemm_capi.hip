@@ -1201,8 +1201,9 @@ static int conv_forward_pointwise(int dtype, const void* image, const void* kern
 // Byte offsets inside a channels-last image are formed in 32 bits from two terms (the pixel of the window origin, and the
 // tap reach with the padding taken off): both must stay below 2^30
 static bool conv_nhwc_offsets_fit(int64_t channels, int64_t es, const Geo3& g) {
-    const int64_t pr = g.p[1] < 0 ? -g.p[1] : g.p[1], pc = g.p[2] < 0 ? -g.p[2] : g.p[2];
-    const int64_t reach = ((pr + g.k[1] * g.d[1]) * g.sz[2] + pc + g.k[2] * g.d[2]) * channels * es;
+    auto mag = [](int64_t v) { return v < 0 ? -v : v; };
+    const int64_t pd = mag(g.p[0]), pr = mag(g.p[1]), pc = mag(g.p[2]);
+    const int64_t reach = (((pd + g.k[0] * g.d[0]) * g.sz[1] + pr + g.k[1] * g.d[1]) * g.sz[2] + pc + g.k[2] * g.d[2]) * channels * es;
     return channels * g.vol() * es < (1LL << 30) && reach < (1LL << 30);
 }
 // A K-step of the channels-last kernel is 64 bytes of channels of one tap, so the copy pads the channels of each group
@@ -1214,7 +1215,7 @@ static int64_t nhwc_padded_channels(int64_t es, int64_t cg) {
     const int64_t step = 64 / es, cgp = (cg + step - 1) / step * step;
     return cg > 0 && cgp <= (es == 2 ? 4 : 1) * cg ? cgp : 0;
 }
-// The channels-last copy carries the convolution's padding as a border of zero pixels (two axes, non-negative padding):
+// The channels-last copy carries the convolution's padding as a border of zero pixels (non-negative padding):
 // the padded image is as large as the windows reach, every tap of every window then exists, and the kernel's gather needs
 // neither a validity test nor a per-lane address select -- its DMA is that of a stored operand.  gp describes the padded
 // image with padding 0 (what the kernel is told); hm where the copy puts the pixels.
@@ -1223,13 +1224,20 @@ static HaloPlan conv_halo(const Geo3& g) {
     HaloPlan h;
     std::memset(&h.hm, 0, sizeof h.hm);
     h.on = false; h.gp = g; h.vol = g.vol();
-    if (g.nd != 2 || g.p[1] < 0 || g.p[2] < 0) return h;
-    const int64_t need_h = (g.o[1] - 1) * g.s[1] + (g.k[1] - 1) * g.d[1] + 1, need_w = (g.o[2] - 1) * g.s[2] + (g.k[2] - 1) * g.d[2] + 1;
-    const int64_t Hp = std::max(need_h, g.p[1] + g.sz[1]), Wp = std::max(need_w, g.p[2] + g.sz[2]);
-    if (Hp * Wp > 2 * g.sz[1] * g.sz[2] + 64) return h;               // (a border larger than the image: not worth the copy)
-    h.hm.W = g.sz[2]; h.hm.H = g.sz[1]; h.hm.Wp = Wp; h.hm.Hp = Hp; h.hm.top = g.p[1]; h.hm.left = g.p[2];
-    h.gp.sz[1] = Hp; h.gp.sz[2] = Wp; h.gp.p[1] = 0; h.gp.p[2] = 0;
-    h.vol = Hp * Wp;
+    int64_t ext[3];                                                   // the padded image: as far as the windows reach, and the image itself
+    for (int a = 0; a < 3; ++a) {
+        if (g.p[a] < 0) return h;
+        ext[a] = std::max((g.o[a] - 1) * g.s[a] + (g.k[a] - 1) * g.d[a] + 1, g.p[a] + g.sz[a]);
+    }
+    const int64_t vol = ext[0] * ext[1] * ext[2];
+    // (a border larger than the image: not worth the copy on two axes, where the validity bits serve; three axes have no such form,
+    //  and the element-wise gather they fall back to loses more than the copy of three times the image costs)
+    if (vol > (g.nd == 3 ? 4 : 2) * g.vol() + 64) return h;
+    h.hm.W = g.sz[2]; h.hm.H = g.sz[1]; h.hm.D = g.sz[0];
+    h.hm.Wp = ext[2]; h.hm.Hp = ext[1]; h.hm.Dp = ext[0];
+    h.hm.left = g.p[2]; h.hm.top = g.p[1]; h.hm.front = g.p[0];
+    for (int a = 0; a < 3; ++a) { h.gp.sz[a] = ext[a]; h.gp.p[a] = 0; }
+    h.vol = vol;
     h.on = true;
     return h;
 }
@@ -1254,9 +1262,11 @@ static int64_t conv_nhwc_merged_workspace(int dtype, int64_t batch, int64_t out_
 }
 static bool conv_nhwc_ok(int dtype, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
     if (dtype != ntg::DT_F32 && dtype != ntg::DT_F16 && dtype != ntg::DT_BF16) return false;
-    if (g.nd != 2 || !conv_implicit_g(dtype, channels, g)) return false;
+    if (!conv_implicit_g(dtype, channels, g)) return false;
+    const HaloPlan halo = conv_halo(g);
+    if (g.nd == 3 && !halo.on) return false;                          // (three axes: the bordered copy is the only form)
     const int64_t es = ntg::elem_size(dtype), cgp = nhwc_padded_channels(es, channels / groups);
-    return cgp > 0 && out_channels > 0 && conv_nhwc_offsets_fit(groups * cgp, es, g) && conv_nhwc_offsets_fit(groups * cgp, es, conv_halo(g).gp);
+    return cgp > 0 && out_channels > 0 && conv_nhwc_offsets_fit(groups * cgp, es, g) && conv_nhwc_offsets_fit(groups * cgp, es, halo.gp);
 }
 static int64_t conv_nhwc_workspace(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
     const int64_t es = ntg::elem_size(dtype), cgp = nhwc_padded_channels(es, channels / groups);
@@ -1270,7 +1280,7 @@ static int conv_forward_nhwc(int dtype, const void* image, const void* kernel, v
     HaloPlan halo = conv_halo(g);
     if (mt) { halo.on = false; halo.vol = vol; halo.gp = g; }                    // (the merged-tap form keeps its validity bits)
     const int64_t volp = halo.vol;                                               // pixels per image of the copy
-    const bool tap_inner = halo.on && g.s[1] == 1 && g.s[2] == 1;                // (neighbouring taps share pixels only at unit strides)
+    const bool tap_inner = halo.on && g.s[0] == 1 && g.s[1] == 1 && g.s[2] == 1;   // (neighbouring taps share pixels only at unit strides)
     char* ws_img = static_cast<char*>(ws);
     char* ws_w = ws_img + align_up((size_t)(batch * chp * volp * es), 256);
     const ntg::HaloMap* hm = halo.on ? &halo.hm : nullptr;
@@ -1381,7 +1391,7 @@ static int conv_dimage_nhwc(int dtype, const void* kernel, const void* grad_out,
     const Geo3 t = geo_dimage(g);
     const HaloPlan halo = conv_halo(t);                                         // (the "image" of this convolution is dY)
     const int64_t Lp = halo.vol;
-    const bool tap_inner = halo.on && t.s[1] == 1 && t.s[2] == 1;
+    const bool tap_inner = halo.on;                                             // (all strides are 1)
     char* ws_gy = static_cast<char*>(ws);
     char* ws_w = ws_gy + align_up((size_t)(batch * ochp * Lp * es), 256);
     const ntg::HaloMap* hm = halo.on ? &halo.hm : nullptr;
@@ -1526,165 +1536,161 @@ static int conv_dimage_phases(int dtype, const PhasePlan& pp, const void* kernel
     return NTG_OK;
 }
 
-// dW through the channels-last kernel: the image is copied to [B][pixel][C]; per image and group
-// P_{b,g} [og][(taps, c)] = dY_{b,g} [og, L] . col^T gathered 16 bytes of channels at a time; the per-image results are
-// summed in batch order into the kernel's [O][c][taps] layout.  The copy pads the channels of a group to whole 16-byte
-// runs; dY is read where it lies or from a channels-last copy of its own (below).
-// Large output planes with 16-byte rows: dY is read where it lies, one image per K loop (measured faster from about 512
-// pixels: no copy, one LDS read per block instead of the transposing ones).  Otherwise, when the out channels of a group
-// are a 16-byte multiple, dY goes through its own channels-last copy: as a [pixel][out channel] matrix the images follow
-// each other, so several of them can share one K loop.
-static bool conv_dkernel_nhwc_copies_dy(int dtype, int64_t out_channels, int64_t groups, const Geo3& g) {
-    const int64_t es = ntg::elem_size(dtype);
-    if ((g.L() * es) % 16 == 0 && g.L() >= 512) return false;
-    return ((out_channels / groups) * es) % 16 == 0;
-}
-// Images per K loop: the largest divisor of the batch that still leaves two workgroups per CU (128 x 128 tiles), so that
-// fewer per-image results are written and summed (64 images of a 3 x 3 x 256 x 256 layer: 16 partial sums instead of 64;
-// 7 x 7 maps: K = 784 instead of 49).
-static int64_t conv_dkernel_fold(int64_t batch, int64_t og, int64_t n, int64_t groups, int64_t L) {
-    const int64_t tiles = ((og + 127) / 128) * ((n + 127) / 128) * groups;
-    int64_t best = 1;
-    for (int64_t f = 2; f <= batch; ++f) {
-        if (batch % f) continue;
-        if ((batch / f) * tiles < 512 || f * L >= (1LL << 30)) break;
-        best = f;
-    }
-    return best;
-}
-// 16-bit, dY read where it lies: instead of one product per image, the output pixels of all images counted through are cut
-// into `ranges` equal k ranges (whole K-steps; an image is whole K-steps too) so that tiles x ranges fill whole rounds
-// over the CUs: 64 images of a 3 x 3 x 256 x 256 layer on 56 x 56 maps are 9 tiles x 28 ranges = 252 tiles of 7168 pixels
-// in one round (235 us + 10 us for adding 28 partial sums), against 512 + 256 tiles in three rounds (217 + 46 us, + 18 us
-// for 64 partial sums).  Returns the number of ranges, 0: one product per image.
-// The estimate prices the gathering kernel as measured on that layer: 0.41 of a CU's MFMA peak on 256 x 256 tiles, 0.35 on
-// 128 x 128 tiles when two workgroups share a CU and 0.245 when one has it alone; it has to be 5 % ahead.
-static double dkernel16_cost_us(int edge, int64_t tiles, int64_t K) {
-    const double cu_flops_per_us = 9.77e6, area = (double)edge * edge;
-    if (edge == 256) return (double)((tiles + 255) / 256) * (2.0 * area * (double)K / (cu_flops_per_us * 0.41) + 6.0);
-    if (edge == 128) {
-        if (tiles <= 256) return 2.0 * area * (double)K / (cu_flops_per_us * 0.245) + 3.0;
-        return (double)((tiles + 511) / 512) * (4.0 * area * (double)K / (cu_flops_per_us * 0.35) + 3.0);
-    }
-    return (double)((tiles + 1023) / 1024) * (8.0 * area * (double)K / (cu_flops_per_us * 0.2) + 2.0);
-}
-static double dkernel16_plan_cost_us(int64_t M, int64_t N, int64_t K, int64_t batch) {
-    const ntg::Ring16Plan pl = ntg::ring16_plan(M, N, K, batch);
-    if (pl.head >= batch) return dkernel16_cost_us(pl.edge, ntg::ring16_tiles(pl.edge, M, N, batch), K);
-    return dkernel16_cost_us(pl.edge, ntg::ring16_tiles(pl.edge, M, N, pl.head), K) +
-           dkernel16_cost_us(pl.tail_edge, ntg::ring16_tiles(pl.tail_edge, M, N, batch - pl.head), K) + 2.0;
-}
-static int64_t conv_dkernel_ranges(int dtype, int64_t batch, int64_t og, int64_t out_channels, int64_t N, int64_t L) {
-    const int64_t es = ntg::elem_size(dtype), bk = 64 / es;
-    if (es != 2 || batch < 2 || L % bk != 0 || batch * L >= (1LL << 30)) return 0;
-    auto reduce_us = [&](int64_t items) { return 3.0 + (double)items * (double)(out_channels * N * es) / 4.0e6; };
-    const int64_t hc = ntg::ring16_column_split(og, N, L, batch);
-    const double cur = (hc ? dkernel16_plan_cost_us(og, hc, L, batch) + dkernel16_plan_cost_us(og, N - hc, L, batch) + 2.0
-                           : dkernel16_plan_cost_us(og, N, L, batch)) + reduce_us(batch);
-    const int64_t steps = batch * L / bk;
-    // measurement and test knob: NTG_DW_RANGES=r forces r ranges where r is admissible, 0 forces one product per image
-    if (const char* env = std::getenv("NTG_DW_RANGES")) {
-        const int64_t r = std::atoll(env);
-        return r > 0 && r <= batch && steps % r == 0 ? r : 0;
-    }
-    int64_t best = 0;
-    double best_us = 0.95 * cur;
-    for (int64_t r = 1; r <= batch; ++r) {
-        if (steps % r != 0 || steps / r < 16) continue;
-        const int64_t kr = steps / r * bk;
-        const int edge = ntg::ring16_tile_edge(og, N, kr, r);
-        const double us = dkernel16_cost_us(edge, ntg::ring16_tiles(edge, og, N, r), kr) + reduce_us(r);
-        if (us < best_us) { best_us = us; best = r; }
-    }
-    return best;
-}
+// dW through the channels-last kernel: the image is copied to [B][pixel][C]; the output pixels of ALL images counted through are
+// cut into k ranges, and per range and group  P [og][(taps, c)] = dY [og, pixels] . col^T  gathered 16 bytes of channels at a
+// time; the ranges' partial sums are added in order into the kernel's [O][c][taps] layout.  The copy pads the channels of a group to
+// whole 16-byte runs and carries the convolution's padding as pixels of zeros.
 static int64_t dkernel_padded_channels(int64_t es, int64_t cg) { const int64_t v = 16 / es; return (cg + v - 1) / v * v; }
-// The copy of the image carries the padding as a border of zero pixels where the plain 16-byte copy serves it (whole
-// 16-byte runs of channels): the gather then needs no validity test, and keeps the window origins in a table.
 static HaloPlan dkernel_halo(int64_t es, int64_t cg, int64_t groups, const Geo3& g) {
     HaloPlan h = conv_halo(g);
-    if (h.on && (dkernel_padded_channels(es, cg) != cg || !conv_nhwc_offsets_fit(groups * cg, es, h.gp))) {
+    if (h.on && !conv_nhwc_offsets_fit(groups * dkernel_padded_channels(es, cg), es, h.gp)) {
         h.on = false; h.gp = g; h.vol = g.vol();
     }
     return h;
 }
-static bool conv_dkernel_nhwc_ok(int dtype, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
-    if (dtype != ntg::DT_F32 && dtype != ntg::DT_F16 && dtype != ntg::DT_BF16) return false;
-    if (g.nd != 2 || !conv_implicit_g(dtype, channels, g)) return false;
-    const int64_t es = ntg::elem_size(dtype), cg = channels / groups;
-    if (g.k[1] * g.d[1] >= 32768 || g.k[2] * g.d[2] >= 32768) return false;      // tap reach packed in 16 bits
-    // rows of dY that are 16-byte multiples are read where they lie; otherwise dY is copied channels-last too and read
-    // as a [pixel][out channel] operand, which needs the out channels of a group to be a 16-byte multiple
-    const bool a_ok = (g.L() * es) % 16 == 0 || conv_dkernel_nhwc_copies_dy(dtype, out_channels, groups, g);
-    // the channels of a group are gathered in 16-byte runs: the copy pads them to whole runs (RGB: 3 -> 8 or 4)
-    const int64_t cgp = dkernel_padded_channels(es, cg);
-    return a_ok && cgp <= 4 * cg && out_channels > 0 && cgp * g.taps() < 0x7fffffffLL && conv_nhwc_offsets_fit(groups * cgp, es, g);
+// What a launch of the gathering kernel takes, from the timings of the layers below: microseconds for `tiles` tiles of
+// edge x edge with K output pixels each, by how many workgroups share a CU.  16-bit: 0.41 of a CU's MFMA peak on 256 x 256 tiles;
+// 0.35 on 128 x 128 tiles when two workgroups share a CU, 0.245 when one has it alone; a 64 x 64 tile alone on its CU
+// takes 9 ns per pixel, several of them 4.2 ns each.  Float32: 27 ns per pixel for a 64 x 64 tile alone, 15.4 ns each for
+// several; 128 x 128: 70 and 60.
+static double dkernel_cost_us(int64_t es, int edge, int64_t tiles, int64_t K) {
+    const double w = (double)((tiles + 255) / 256), k = (double)K;
+    if (es == 4) return edge == 128 ? 4.0 + k * std::max(0.070, 0.060 * w) : 3.0 + k * std::max(0.027, 0.0154 * w);
+    const double cu_flops_per_us = 9.77e6, area = (double)edge * edge;
+    if (edge == 256) return w * (2.0 * area * k / (cu_flops_per_us * 0.41) + 6.0);
+    if (edge == 128) {
+        if (tiles <= 256) return 2.0 * area * k / (cu_flops_per_us * 0.245) + 3.0;
+        return (double)((tiles + 511) / 512) * (4.0 * area * k / (cu_flops_per_us * 0.35) + 3.0);
+    }
+    return 3.0 + k * std::max(0.009, 0.0042 * w);
 }
-static int64_t conv_dkernel_nhwc_workspace(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
+// How dW is cut up: `ranges` k ranges of `kr` output pixels (0: one product per image), tiles of edge x edge (0: the launcher's choice), dY read where it
+// lies (its rows 16-byte multiples, an image a whole number of K-steps) or through a channels-last copy of its own (the out
+// channels of a group a 16-byte multiple; any range then), the partial sums in the element type or in Float32.
+// One product per image left a small layer on a handful of workgroups, each with the whole image as its k (3 x 3 x 3 x 32 -> 64
+// channels on 4 volumes of 32^3 in Float32: 56 workgroups of 32768 pixels, 1285 us), and a 7 x 7 map of 64 images with 64
+// times the partial sums it needs; the ranges are chosen so that tiles x ranges fill whole rounds over the CUs, against the
+// cost of writing and reading the partial sums (4 TB/s) and of the copy of dY.
+struct DkernelPlan { bool ok, copy_dy, part_f32; int64_t ranges, kr, items; int edge; };
+static DkernelPlan plan_dkernel(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
+    DkernelPlan pl;
+    std::memset(&pl, 0, sizeof pl);
+    if (dtype != ntg::DT_F32 && dtype != ntg::DT_F16 && dtype != ntg::DT_BF16) return pl;
+    if (!conv_implicit_g(dtype, channels, g) || out_channels <= 0 || batch <= 0) return pl;
+    const int64_t es = ntg::elem_size(dtype), bk = 64 / es, cg = channels / groups, og = out_channels / groups, L = g.L();
+    if (g.k[1] * g.d[1] >= 32768 || g.k[2] * g.d[2] >= 32768) return pl;         // tap reach packed in 16 bits
+    const int64_t cgp = dkernel_padded_channels(es, cg), N = cgp * g.taps();
+    if (cgp > 4 * cg || N >= 0x7fffffffLL || !conv_nhwc_offsets_fit(groups * cgp, es, g)) return pl;
+    if (g.nd == 3 && !dkernel_halo(es, cg, groups, g).on) return pl;             // (three axes: the bordered copy is the only form)
+    const bool rows_16 = (L * es) % 16 == 0, og_16 = (og * es) % 16 == 0;
+    const int64_t total = batch * L, steps = (total + bk - 1) / bk;
+    const bool countable = total < (1LL << 30);
+    const bool lies = rows_16 && L % bk == 0 && countable, copied = og_16 && countable;
+    if (!rows_16 && !copied) return pl;
+    pl.ok = true;
+    pl.items = batch;
+    // measurement and test knob: NTG_DW_RANGES=r forces r ranges of dY where it lies where r is admissible, 0 one product per image
+    const char* env = std::getenv("NTG_DW_RANGES");
+    if (env && rows_16) {
+        const int64_t r = std::atoll(env);
+        if (lies && r > 0 && steps % r == 0) {
+            pl.ranges = pl.items = r;
+            pl.kr = total / r;
+            pl.edge = es == 2 ? ntg::ring16_tile_edge(og, N, pl.kr, r) : 64;
+        }
+    } else {
+        double best = 0.0;
+        const auto consider = [&](bool copy, int64_t ranges, int64_t items, int64_t kr, int edge) {
+            const int64_t tiles = ((og + edge - 1) / edge) * ((N + edge - 1) / edge) * items;
+            // (the groups' launches run one behind the other)
+            const double us = (copy ? 4.0 + 2.0 * (double)(total * out_channels * es) / 4.5e6 : 0.0) + groups * dkernel_cost_us(es, edge, tiles, kr) + 4.0 +
+                              2.0 * (double)(items * out_channels * N * (es == 2 && items > batch ? 4 : es)) / 4.0e6;
+            if (pl.edge && us >= best) return;
+            best = us;
+            pl.copy_dy = copy; pl.ranges = ranges; pl.items = items; pl.kr = kr; pl.edge = edge;
+        };
+        for (int edge : {256, 128, 64}) {
+            if (es == 4 && edge == 256) continue;
+            if (rows_16) consider(false, 0, batch, L, edge);
+            const int64_t tiles = ((og + edge - 1) / edge) * ((N + edge - 1) / edge) * groups;
+            for (int64_t target : {256, 512, 768, 1024, 1536, 2048}) {
+                const int64_t want = std::min(std::max<int64_t>(target / tiles, 1), std::max<int64_t>(steps / 8, 1));
+                const int64_t per = (steps + want - 1) / want, r = (steps + per - 1) / per;
+                if (lies) consider(false, r, r, per * bk, edge);
+                if (copied) consider(true, r, r, per * bk, edge);
+            }
+        }
+    }
+    // (at most one rounding per image, as many as the reference's own per-image products take; more partial sums stay in Float32)
+    pl.part_f32 = es == 2 && pl.items > batch;
+    return pl;
+}
+static int64_t conv_dkernel_nhwc_workspace(int dtype, const DkernelPlan& pl, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
     const int64_t es = ntg::elem_size(dtype);
-    const int64_t gy = conv_dkernel_nhwc_copies_dy(dtype, out_channels, groups, g) ? (int64_t)align_up((size_t)(batch * out_channels * g.L() * es), 256) : 0;
+    const int64_t gy = pl.copy_dy ? (int64_t)align_up((size_t)(batch * out_channels * g.L() * es), 256) : 0;
     const int64_t cgp = dkernel_padded_channels(es, channels / groups);
     return (int64_t)align_up((size_t)(batch * groups * cgp * dkernel_halo(es, channels / groups, groups, g).vol * es), 256) + gy +
-           batch * out_channels * cgp * g.taps() * es;
+           pl.items * out_channels * cgp * g.taps() * (pl.part_f32 ? 4 : es);
 }
-static int conv_dkernel_nhwc(int dtype, const void* image, const void* grad_out, void* d_kernel, void* ws, int64_t batch,
+static int conv_dkernel_nhwc(int dtype, const DkernelPlan& pl, const void* image, const void* grad_out, void* d_kernel, void* ws, int64_t batch,
                              int64_t channels, int64_t out_channels, const Geo3& g, int64_t groups, int accumulate, hipStream_t hs) {
-    const int64_t es = ntg::elem_size(dtype), cg = channels / groups, og = out_channels / groups;
+    const int64_t es = ntg::elem_size(dtype), bk = 64 / es, cg = channels / groups, og = out_channels / groups;
     const int64_t cgp = dkernel_padded_channels(es, cg), chp = groups * cgp;      // channels per group / per pixel in the copy
     const int64_t L = g.L(), taps = g.taps(), vol = g.vol(), N = taps * cgp;
     const HaloPlan halo = dkernel_halo(es, cg, groups, g);
     const int64_t volp = halo.vol;                                                         // pixels per image of the copy
-    const bool copy_dy = conv_dkernel_nhwc_copies_dy(dtype, out_channels, groups, g);      // dY read as [pixel][out channel] from its own copy
-    const int64_t ranges = copy_dy ? 0 : conv_dkernel_ranges(dtype, batch, og, out_channels, N, L);
-    const int64_t fold = copy_dy ? conv_dkernel_fold(batch, og, N, groups, L) : 1, items = ranges ? ranges : batch / fold;
     char* ws_img = static_cast<char*>(ws);
     char* ws_gy = ws_img + align_up((size_t)(batch * chp * volp * es), 256);
-    char* ws_part = ws_gy + (copy_dy ? align_up((size_t)(batch * out_channels * L * es), 256) : 0);
+    char* ws_part = ws_gy + (pl.copy_dy ? align_up((size_t)(batch * out_channels * L * es), 256) : 0);
+    const ntg::HaloMap* hm = halo.on ? &halo.hm : nullptr;
     bool took_along = false;
-    hipError_t e = cgp == cg ? ntg::launch_nchw_to_nhwc(es, image, ws_img, batch, channels, vol, hs, halo.on ? &halo.hm : nullptr, nullptr, &took_along)
-                             : ntg::launch_nchw_to_nhwc_padded(es, image, ws_img, batch, groups, cg, cgp, vol, hs);
+    hipError_t e = cgp == cg ? ntg::launch_nchw_to_nhwc(es, image, ws_img, batch, channels, vol, hs, hm, nullptr, &took_along)
+                             : ntg::launch_nchw_to_nhwc_padded(es, image, ws_img, batch, groups, cg, cgp, vol, hs, hm);
     if (e == hipSuccess && halo.on && volp != vol && !took_along) e = ntg::launch_halo_zero(es, ws_img, batch, chp, halo.hm, hs);
-    if (e == hipSuccess && copy_dy) e = ntg::launch_nchw_to_nhwc(es, grad_out, ws_gy, batch, out_channels, L, hs);
+    if (e == hipSuccess && pl.copy_dy) e = ntg::launch_nchw_to_nhwc(es, grad_out, ws_gy, batch, out_channels, L, hs);
     if (e != hipSuccess) return hip_fail(e, "channels-last copy launch");
+    const int64_t pes = pl.part_f32 ? 4 : es;
     for (int64_t gi = 0; gi < groups; ++gi) {
         ntg::GemmParams p;
         std::memset(&p, 0, sizeof p);
-        p.M = (int)og; p.K = (int)(fold * L); p.N = (int)N; p.batch = (int)items;
-        if (copy_dy) {
+        p.M = (int)og; p.K = (int)(pl.ranges ? pl.kr : L); p.N = (int)N; p.batch = (int)pl.items;
+        if (pl.copy_dy) {
             p.A = ws_gy + gi * og * es;
             p.lda = out_channels;
+            p.sA = pl.kr * out_channels;
         } else {
             p.A = static_cast<const char*>(grad_out) + gi * og * L * es;
             p.lda = L;
+            p.sA = pl.ranges ? 0 : out_channels * L;
         }
         p.B = ws_img + gi * cgp * es;
-        p.C = ws_part + gi * og * N * es;
+        p.C = ws_part + gi * og * N * pes;
         p.ldb = chp; p.ldc = N;
-        p.sA = fold * out_channels * L; p.sB = fold * chp * volp; p.sC = out_channels * N;
-        p.cmode = ntg::C_OVERWRITE;
+        p.sB = pl.ranges ? 0 : chp * volp; p.sC = out_channels * N;
+        p.cmode = pl.part_f32 ? ntg::C_PARTIAL : ntg::C_OVERWRITE;
         p.vecA_ok = 1; p.vecB_ok = 1;
         fill_conv_geom(p.conv, cgp, halo.gp);
         p.conv.chan = (int)chp;                    // elements from one pixel to the next
-        if (fold > 1 || ranges) {
+        p.conv.halo = halo.on ? 1 : 0;
+        if (halo.on && g.nd == 2 && L < (1 << 20) && (pl.ranges == 0 || L % bk == 0)) p.conv.pix_table = (int)L;     // (a K-step inside one image: see the kernel)
+        p.conv.tile_edge = pl.edge;
+        if (pl.ranges) {
+            p.conv.k_ranges = 1;
+            p.conv.k_total = (int)(batch * L);
             p.conv.fold_L = (int)L;
             p.conv.div_fold = ntg::make_fastdiv((uint32_t)L);
             p.conv.fold_stride = chp * volp;
+            if (!pl.copy_dy) {
+                p.conv.a_steps = (int)(L / bk);
+                p.conv.div_a_steps = ntg::make_fastdiv((uint32_t)(L / bk));
+                p.conv.a_image_stride = out_channels * L;
+            }
         }
-        if (halo.on && fold == 1 && L < (1 << 20)) p.conv.pix_table = (int)L;     // (a K-step inside one image: see the kernel)
-        if (ranges) {
-            const int64_t bk = 64 / es;
-            p.K = (int)(batch * L / ranges);
-            p.sA = 0; p.sB = 0;
-            p.conv.k_ranges = 1;
-            p.conv.a_steps = (int)(L / bk);
-            p.conv.div_a_steps = ntg::make_fastdiv((uint32_t)(L / bk));
-            p.conv.a_image_stride = out_channels * L;
-        }
-        e = ntg::launch_conv_nhwc_dw(dtype, copy_dy, p, hs);
+        e = ntg::launch_conv_nhwc_dw(dtype, pl.copy_dy, p, hs);
         if (e != hipSuccess) return hip_fail(e, "channels-last conv_dkernel launch");
     }
     // (groups are consecutive row blocks of both layouts, so one pass covers them all)
-    e = ntg::launch_reduce_batch_taps_last(dtype, ws_part, d_kernel, items, out_channels, cg, cgp, taps, accumulate, hs);
+    e = ntg::launch_reduce_batch_taps_last(dtype, pl.part_f32, ws_part, d_kernel, pl.items, out_channels, cg, cgp, taps, accumulate, hs);
     if (e != hipSuccess) return hip_fail(e, "weight gradient reduction launch");
     return NTG_OK;
 }
@@ -1734,7 +1740,7 @@ static int conv_dkernel_from_col(int dtype, const char* gy, char* col, void* d_k
 }
 
 // Which backward gradients run as implicit GEMMs, and the workspace the call needs.
-struct ConvBackwardPlan { bool gather_dw, gather_dx, nhwc_dx, nhwc_dw, phase_dx; int64_t need, need_nhwc_dx, need_nhwc_dw, need_phase_dx; PhasePlan phases; };
+struct ConvBackwardPlan { bool gather_dw, gather_dx, nhwc_dx, nhwc_dw, phase_dx; int64_t need, need_nhwc_dx, need_nhwc_dw, need_phase_dx; PhasePlan phases; DkernelPlan dkernel; };
 // reference_order (Float32 through the host entry points): the forms whose sums are the reference's own, bit for bit -- the
 // image gradient as W^T . dY into the col matrix + col2im (conv.cpp:318-346; the implicit forms run one chain over out
 // channels and taps where the reference rounds in between), the weight gradient per image with k = the output pixels +
@@ -1752,10 +1758,12 @@ static ConvBackwardPlan plan_conv_backward_g(int dtype, bool want_dx, bool want_
     if (want_dx) need = std::max(need, pl.gather_dx ? out_channels * cg * taps * es : col);
     pl.need = need;
     // the channels-last form of dX is taken when the caller's workspace also holds the copy of dY
-    pl.nhwc_dx = pl.gather_dx && g.nd == 2 && conv_dimage_nhwc_ok(dtype, channels, out_channels, groups, g);
+    pl.nhwc_dx = pl.gather_dx && conv_dimage_nhwc_ok(dtype, channels, out_channels, groups, g);
     pl.need_nhwc_dx = pl.nhwc_dx ? conv_dimage_nhwc_workspace(dtype, batch, channels, out_channels, groups, g) : 0;
-    pl.nhwc_dw = pl.gather_dw && !reference_order && conv_dkernel_nhwc_ok(dtype, channels, out_channels, groups, g);
-    pl.need_nhwc_dw = pl.nhwc_dw ? conv_dkernel_nhwc_workspace(dtype, batch, channels, out_channels, groups, g) : 0;
+    std::memset(&pl.dkernel, 0, sizeof pl.dkernel);
+    if (pl.gather_dw && !reference_order) pl.dkernel = plan_dkernel(dtype, batch, channels, out_channels, groups, g);
+    pl.nhwc_dw = pl.dkernel.ok;
+    pl.need_nhwc_dw = pl.nhwc_dw ? conv_dkernel_nhwc_workspace(dtype, pl.dkernel, batch, channels, out_channels, groups, g) : 0;
     // strides > 1: dX phase by phase instead of GEMM + col2im, again when the workspace allows
     std::memset(&pl.phases, 0, sizeof pl.phases);
     if (want_dx && !pl.gather_dx && !reference_order && conv_implicit_g(dtype, out_channels, geo_dimage(g)))
@@ -2020,7 +2028,7 @@ static int conv2d_backward_dev_impl(int dtype, const void* image, const void* ke
     }
     if (gather_dw) {
         if (plan.nhwc_dw && workspace_bytes >= plan.need_nhwc_dw && ((reinterpret_cast<uintptr_t>(ws) | reinterpret_cast<uintptr_t>(grad_out)) & 15) == 0)
-            rc = conv_dkernel_nhwc(dtype, image, grad_out, d_kernel, ws, batch, channels, out_channels, geo, groups, accumulate, hs);
+            rc = conv_dkernel_nhwc(dtype, plan.dkernel, image, grad_out, d_kernel, ws, batch, channels, out_channels, geo, groups, accumulate, hs);
         else
             rc = conv_dkernel_gather(dtype, image, grad_out, d_kernel, ws, batch, channels, out_channels, geo, groups, accumulate, hs);
         if (rc) return rc;
@@ -2304,7 +2312,11 @@ int64_t ntg_convnd_workspace_bytes(int dtype, int64_t batch, int64_t channels, i
     }
     if (ndim == 3) {
         const Geo3 g = geo_from(u);
-        if (backward) return plan_conv_backward_g(dtype, true, true, batch, channels, out_channels, g, groups).need;
+        if (backward) {
+            const ConvBackwardPlan pl = plan_conv_backward_g(dtype, true, true, batch, channels, out_channels, g, groups);
+            return std::max(std::max(pl.need, pl.need_phase_dx), std::max(pl.need_nhwc_dx, pl.need_nhwc_dw));
+        }
+        if (conv_nhwc_ok(dtype, channels, out_channels, groups, g)) return conv_nhwc_workspace(dtype, batch, channels, out_channels, groups, g);
         if (conv_implicit_g(dtype, channels, g)) return 0;
     }
     return u.total * es + (backward ? complex_dkernel_extra(dtype, batch, out_channels, (channels / groups) * u.taps, u.total * es) : 0);
@@ -2329,6 +2341,9 @@ int ntg_convnd_dev(int dtype, const void* image, const void* kernel, void* out, 
     if (!image || !kernel || !out) return fail(NTG_ERR_INVALID_ARGUMENT, "null pointer");
     if (ndim == 3) {
         const Geo3 g = geo_from(u);
+        if (conv_nhwc_ok(dtype, channels, out_channels, groups, g) && workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
+            workspace_bytes >= conv_nhwc_workspace(dtype, batch, channels, out_channels, groups, g))
+            return conv_forward_nhwc(dtype, image, kernel, out, workspace, batch, channels, out_channels, g, groups, static_cast<hipStream_t>(stream));
         if (conv_implicit_g(dtype, channels, g))      // three axes, floating dtype: gathered inside the GEMM, no col buffer
             return conv_forward_gather(dtype, image, kernel, out, batch, channels, out_channels, g, groups, static_cast<hipStream_t>(stream));
     }
@@ -2354,10 +2369,12 @@ int ntg_convnd_dev(int dtype, const void* image, const void* kernel, void* out, 
     return NTG_OK;
 }
 
-int ntg_convnd_backward_dev(int dtype, const void* image, const void* kernel, const void* grad_out, void* d_image, void* d_kernel,
-                            void* workspace, int64_t workspace_bytes, int64_t batch, int64_t channels, int64_t out_channels, int ndim,
-                            const int64_t* size, const int64_t* kernel_size, const int64_t* stride, const int64_t* padding,
-                            const int64_t* dilation, int64_t groups, int accumulate, void* stream) {
+// channels_last = false (Float32 through the host entry point): the element-wise gathering forms, whose weight gradient sums the
+// output pixels of each image in ascending order like the reference
+static int convnd_backward_dev_impl(int dtype, const void* image, const void* kernel, const void* grad_out, void* d_image, void* d_kernel,
+                                    void* workspace, int64_t workspace_bytes, int64_t batch, int64_t channels, int64_t out_channels, int ndim,
+                                    const int64_t* size, const int64_t* kernel_size, const int64_t* stride, const int64_t* padding,
+                                    const int64_t* dilation, int64_t groups, int accumulate, void* stream, bool channels_last) {
     const int64_t es = ntg::elem_size(dtype);
     if (es == 0) return fail(NTG_ERR_UNSUPPORTED_DTYPE, "dtype %d is not supported", dtype);
     int rc = check_groups(channels, out_channels, groups);
@@ -2380,14 +2397,23 @@ int ntg_convnd_backward_dev(int dtype, const void* image, const void* kernel, co
         if (need > 0 && (!workspace || workspace_bytes < need))
             return fail(NTG_ERR_INVALID_ARGUMENT, "workspace of %lld bytes needed, %lld given", (long long)need, (long long)workspace_bytes);
         if (plan.gather_dw) {
-            rc = conv_dkernel_gather(dtype, image, grad_out, d_kernel, workspace, batch, channels, out_channels, g, groups, accumulate,
-                                     static_cast<hipStream_t>(stream));
+            if (channels_last && plan.nhwc_dw && workspace_bytes >= plan.need_nhwc_dw &&
+                ((reinterpret_cast<uintptr_t>(workspace) | reinterpret_cast<uintptr_t>(grad_out)) & 15) == 0)
+                rc = conv_dkernel_nhwc(dtype, plan.dkernel, image, grad_out, d_kernel, workspace, batch, channels, out_channels, g, groups, accumulate,
+                                       static_cast<hipStream_t>(stream));
+            else
+                rc = conv_dkernel_gather(dtype, image, grad_out, d_kernel, workspace, batch, channels, out_channels, g, groups, accumulate,
+                                         static_cast<hipStream_t>(stream));
             if (rc) return rc;
             d_kernel = nullptr;
         }
         if (plan.gather_dx) {
-            rc = conv_dimage_gather(dtype, kernel, grad_out, d_image, workspace, batch, channels, out_channels, g, groups, accumulate,
-                                    static_cast<hipStream_t>(stream));
+            if (channels_last && plan.nhwc_dx && workspace_bytes >= plan.need_nhwc_dx && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0)
+                rc = conv_dimage_nhwc(dtype, kernel, grad_out, d_image, workspace, batch, channels, out_channels, g, groups, accumulate,
+                                      static_cast<hipStream_t>(stream));
+            else
+                rc = conv_dimage_gather(dtype, kernel, grad_out, d_image, workspace, batch, channels, out_channels, g, groups, accumulate,
+                                        static_cast<hipStream_t>(stream));
             if (rc) return rc;
             d_image = nullptr;
         }
@@ -2420,6 +2446,14 @@ int ntg_convnd_backward_dev(int dtype, const void* image, const void* kernel, co
         if (e != hipSuccess) return hip_fail(e, "col2imnd launch");
     }
     return NTG_OK;
+}
+
+int ntg_convnd_backward_dev(int dtype, const void* image, const void* kernel, const void* grad_out, void* d_image, void* d_kernel,
+                            void* workspace, int64_t workspace_bytes, int64_t batch, int64_t channels, int64_t out_channels, int ndim,
+                            const int64_t* size, const int64_t* kernel_size, const int64_t* stride, const int64_t* padding,
+                            const int64_t* dilation, int64_t groups, int accumulate, void* stream) {
+    return convnd_backward_dev_impl(dtype, image, kernel, grad_out, d_image, d_kernel, workspace, workspace_bytes, batch, channels, out_channels, ndim,
+                                    size, kernel_size, stride, padding, dilation, groups, accumulate, stream, true);
 }
 
 // output size of the transposed convolution per axis; the geometry of the convolution it is the adjoint of
@@ -2488,7 +2522,9 @@ int ntg_convnd(int dtype, const void* image, const void* kernel, void* out, int6
     if (!image || !kernel || !out) return fail(NTG_ERR_INVALID_ARGUMENT, "null pointer");
     const size_t im_bytes = (size_t)(batch * channels * u.vol * es), k_bytes = (size_t)(out_channels * (channels / groups) * u.taps * es);
     const size_t o_bytes = (size_t)(batch * out_channels * u.L * es);
-    const int64_t wsb = ntg_convnd_workspace_bytes(dtype, batch, channels, out_channels, ndim, size, kernel_size, stride, padding, dilation, groups, 0);
+    int64_t wsb = ntg_convnd_workspace_bytes(dtype, batch, channels, out_channels, ndim, size, kernel_size, stride, padding, dilation, groups, 0);
+    // (Float32 at the reference's seam keeps the gathering kernels and with them im2col's order of k, see ntg_conv2d)
+    if (dtype == ntg::DT_F32 && ndim == 3 && conv_implicit_g(dtype, channels, geo_from(u))) wsb = 0;
     ntg::HostSession mem;
     const size_t o_k = align_up(im_bytes, 256), o_o = o_k + align_up(k_bytes, 256), o_ws = o_o + align_up(o_bytes, 256);
     HIP_TRY(mem.reserve(o_ws + (size_t)wsb));
@@ -2530,9 +2566,9 @@ int ntg_convnd_backward(int dtype, const void* image, const void* kernel, const 
     HIP_TRY(mem.upload(o_g, grad_out, g_bytes));
     if (accumulate && d_image) HIP_TRY(mem.upload(o_di, d_image, im_bytes));
     if (accumulate && d_kernel) HIP_TRY(mem.upload(o_dk, d_kernel, k_bytes));
-    rc = ntg_convnd_backward_dev(dtype, mem.at(0), mem.at(o_k), mem.at(o_g), d_image ? mem.at(o_di) : nullptr, d_kernel ? mem.at(o_dk) : nullptr,
-                                 mem.at(o_ws), wsb, batch, channels, out_channels, ndim, size, kernel_size, stride, padding, dilation, groups,
-                                 accumulate, mem.stream());
+    rc = convnd_backward_dev_impl(dtype, mem.at(0), mem.at(o_k), mem.at(o_g), d_image ? mem.at(o_di) : nullptr, d_kernel ? mem.at(o_dk) : nullptr,
+                                  mem.at(o_ws), wsb, batch, channels, out_channels, ndim, size, kernel_size, stride, padding, dilation, groups,
+                                  accumulate, mem.stream(), dtype != ntg::DT_F32);
     if (rc) return rc;
     if (d_image) HIP_TRY(mem.download(d_image, o_di, im_bytes));
     if (d_kernel) HIP_TRY(mem.download(d_kernel, o_dk, k_bytes));

@@ -41,59 +41,58 @@ __global__ void __launch_bounds__(256) reduce_batch_sum_first_kernel(const T* __
     }
 }
 
-// The same ordered sum for per-image weight gradients held channels-last, part[b][o][t][c], into the kernel's own layout
-// out[o][c][t]: threads follow the partial sums (coalesced reads of the large side), the small result is written scattered.
-template <class T, class Acc>
-__global__ void __launch_bounds__(256) reduce_batch_taps_last_kernel(const T* __restrict__ part, T* __restrict__ out, const int64_t batch,
+// The same sum for partial weight gradients held channels-last, part[b][o][t][c], into the kernel's own layout out[o][c][t]: a
+// thread owns 16 bytes of consecutive channels of one (row, tap) and every SLICES-th of the partial sums (four reads in flight),
+// the slices of a column group are added through LDS in slice order.  Bound by the reads of the partial sums; with one slice a
+// small gradient (3 x 3 x 3 x 32 x 64: 55296 elements, 54 workgroups) over hundreds of partial sums would be one long chain of
+// memory latencies on a few CUs, so SLICES grows until the launch has about 1024 workgroups (28 partial sums of 589824 BFloat16
+// elements: 16 slices of 8-byte reads 15.1 us, one slice of 16-byte reads 10.6).  The order of the additions depends on the sizes only.
+template <class T, class P, int SLICES>
+__global__ void __launch_bounds__(256) reduce_batch_taps_last_kernel(const P* __restrict__ part, T* __restrict__ out, const int64_t batch,
                                                                      const int64_t rows, const int64_t cg, const int64_t cgp, const int64_t taps,
                                                                      const int accumulate) {
-    const int64_t n = rows * cgp * taps;                  // (the partial sums hold cgp >= cg channels per tap, the rest padding)
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const int64_t c = i % cgp, t = (i / cgp) % taps, o = i / (cgp * taps);
-        if (c >= cg) continue;
-        T* dst = out + (o * cg + c) * taps + t;
-        Acc acc = accumulate ? (Acc)*dst : (Acc)0;
-        for (int64_t b = 0; b < batch; ++b) acc += (Acc)part[b * n + i];
-        *dst = (T)acc;
-    }
-}
-
-// The same with 16-byte loads: a thread owns VEC consecutive channels of one (row, tap) and keeps four partial-sum
-// loads in flight; the order of the additions per element is unchanged.  Needs cg % VEC == 0 and aligned partial sums.
-template <class T, class Acc>
-__global__ void __launch_bounds__(256) reduce_batch_taps_last_vec_kernel(const T* __restrict__ part, T* __restrict__ out, const int64_t batch,
-                                                                         const int64_t rows, const int64_t cg, const int64_t taps, const int accumulate) {
-    constexpr int VEC = 16 / (int)sizeof(T);
-    typedef T TV __attribute__((ext_vector_type(VEC)));
-    const int64_t n = rows * cg * taps, nv = n / VEC;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nv; v += stride) {
-        const int64_t i = v * VEC;
-        const int64_t c = i % cg, t = (i / cg) % taps, o = i / (cg * taps);
-        T* dst = out + (o * cg + c) * taps + t;
-        Acc acc[VEC];
+    constexpr int VEC = 16 / (int)sizeof(P);
+    typedef P PV __attribute__((ext_vector_type(VEC)));
+    constexpr int COLS = 256 / SLICES;                    // column groups of VEC elements per workgroup
+    __shared__ float sums[SLICES > 1 ? 256 * VEC : 1];
+    const int64_t n = rows * cgp * taps, nv = n / VEC;    // (the partial sums hold cgp >= cg channels per tap, the rest padding; cgp % VEC == 0)
+    const int col = (int)threadIdx.x % COLS, sl = (int)threadIdx.x / COLS;
+    const int64_t v = (int64_t)blockIdx.x * COLS + col;
+    const int64_t i = v * VEC;
+    float acc[VEC] = {};
+    if (v < nv) {
+        const P* pp = part + i;
+        int64_t b = sl;
+        for (; b + 3 * SLICES < batch; b += 4 * SLICES) {
+            PV x[4];
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) acc[e] = accumulate ? (Acc)dst[(int64_t)e * taps] : (Acc)0;
-        const T* pp = part + i;
-        int64_t b = 0;
-        for (; b + 4 <= batch; b += 4) {
-            TV x[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) x[u] = *reinterpret_cast<const TV*>(pp + (b + u) * n);
+            for (int u = 0; u < 4; ++u) x[u] = *reinterpret_cast<const PV*>(pp + (b + u * SLICES) * n);
 #pragma unroll
             for (int u = 0; u < 4; ++u)
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) acc[e] += (Acc)x[u][e];
+                for (int e = 0; e < VEC; ++e) acc[e] += (float)x[u][e];
         }
-        for (; b < batch; ++b) {
-            const TV x = *reinterpret_cast<const TV*>(pp + b * n);
+        for (; b < batch; b += SLICES) {
+            const PV x = *reinterpret_cast<const PV*>(pp + b * n);
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) acc[e] += (Acc)x[e];
+            for (int e = 0; e < VEC; ++e) acc[e] += (float)x[e];
         }
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) dst[(int64_t)e * taps] = (T)acc[e];
     }
+    if constexpr (SLICES > 1) {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) sums[(e * SLICES + sl) * COLS + col] = acc[e];
+        __syncthreads();
+        if (sl != 0) return;
+        for (int o = 1; o < SLICES; ++o)
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) acc[e] += sums[(e * SLICES + o) * COLS + col];
+    }
+    if (v >= nv) return;
+    const int64_t c = i % cgp, t = (i / cgp) % taps, o = i / (cgp * taps);
+    T* dst = out + (o * cg + c) * taps + t;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e)
+        if (c + e < cg) dst[(int64_t)e * taps] = (T)(accumulate ? (float)dst[(int64_t)e * taps] + acc[e] : acc[e]);
 }
 
 // Split-K epilogue: C (+)= sum over the k ranges of part[s][m][n], s ascending, starting from C0 (the incoming C, the
@@ -266,26 +265,31 @@ hipError_t launch_reduce_batch(int dtype, const void* part, void* out, int64_t b
     return hipGetLastError();
 }
 
-hipError_t launch_reduce_batch_taps_last(int dtype, const void* part, void* out, int64_t batch, int64_t rows, int64_t cg, int64_t cgp,
+template <class T, class P>
+static void launch_reduce_taps_last_t(const void* part, void* out, int64_t batch, int64_t rows, int64_t cg, int64_t cgp, int64_t taps, int accumulate, hipStream_t s) {
+    const int64_t nv = rows * cgp * taps / (16 / (int64_t)sizeof(P));
+#define NTG_TAPS_LAST(S) \
+    hipLaunchKernelGGL((reduce_batch_taps_last_kernel<T, P, S>), dim3((unsigned)((nv * S + 255) / 256)), dim3(256), 0, s, (const P*)part, (T*)out, batch, rows, cg, cgp, taps, accumulate)
+    if (nv >= 256 * 1024 || batch < 8) NTG_TAPS_LAST(1);
+    else if (nv * 4 >= 256 * 1024 || batch < 32) NTG_TAPS_LAST(4);
+    else NTG_TAPS_LAST(16);
+#undef NTG_TAPS_LAST
+}
+hipError_t launch_reduce_batch_taps_last(int dtype, bool part_f32, const void* part, void* out, int64_t batch, int64_t rows, int64_t cg, int64_t cgp,
                                          int64_t taps, int accumulate, hipStream_t s) {
     const int64_t n = rows * cgp * taps;
     if (n == 0) return hipSuccess;
-    const int64_t vec = 16 / elem_size(dtype);
-    if (cgp == cg && cg % vec == 0 && (reinterpret_cast<uintptr_t>(part) & 15) == 0) {
-        const dim3 g(grid_for(n / vec)), b(256);
-        switch (dtype) {
-        case DT_F32: hipLaunchKernelGGL((reduce_batch_taps_last_vec_kernel<float, float>), g, b, 0, s, (const float*)part, (float*)out, batch, rows, cg, taps, accumulate); break;
-        case DT_F16: hipLaunchKernelGGL((reduce_batch_taps_last_vec_kernel<_Float16, float>), g, b, 0, s, (const _Float16*)part, (_Float16*)out, batch, rows, cg, taps, accumulate); break;
-        case DT_BF16: hipLaunchKernelGGL((reduce_batch_taps_last_vec_kernel<__bf16, float>), g, b, 0, s, (const __bf16*)part, (__bf16*)out, batch, rows, cg, taps, accumulate); break;
-        default: return hipErrorInvalidValue;
-        }
-        return hipGetLastError();
-    }
-    const dim3 g(grid_for(n)), b(256);
+    if (cgp % (part_f32 || dtype == DT_F32 ? 4 : 8) != 0 || (reinterpret_cast<uintptr_t>(part) & 15) != 0 || n / 64 >= 0x7fffffffLL) return hipErrorInvalidValue;
     switch (dtype) {
-    case DT_F32: hipLaunchKernelGGL((reduce_batch_taps_last_kernel<float, float>), g, b, 0, s, (const float*)part, (float*)out, batch, rows, cg, cgp, taps, accumulate); break;
-    case DT_F16: hipLaunchKernelGGL((reduce_batch_taps_last_kernel<_Float16, float>), g, b, 0, s, (const _Float16*)part, (_Float16*)out, batch, rows, cg, cgp, taps, accumulate); break;
-    case DT_BF16: hipLaunchKernelGGL((reduce_batch_taps_last_kernel<__bf16, float>), g, b, 0, s, (const __bf16*)part, (__bf16*)out, batch, rows, cg, cgp, taps, accumulate); break;
+    case DT_F32: launch_reduce_taps_last_t<float, float>(part, out, batch, rows, cg, cgp, taps, accumulate, s); break;
+    case DT_F16:
+        if (part_f32) launch_reduce_taps_last_t<_Float16, float>(part, out, batch, rows, cg, cgp, taps, accumulate, s);
+        else launch_reduce_taps_last_t<_Float16, _Float16>(part, out, batch, rows, cg, cgp, taps, accumulate, s);
+        break;
+    case DT_BF16:
+        if (part_f32) launch_reduce_taps_last_t<__bf16, float>(part, out, batch, rows, cg, cgp, taps, accumulate, s);
+        else launch_reduce_taps_last_t<__bf16, __bf16>(part, out, batch, rows, cg, cgp, taps, accumulate, s);
+        break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -306,28 +310,51 @@ hipError_t launch_flip_weights(int64_t es, const void* w, void* wt, int64_t grou
 
 // out[b][p][c] = in[b][c][p]: an image batch from channel planes to channels-last, 64 x 64 tiles through LDS so that
 // both the loads (along p) and the stores (along c) are coalesced.
-// Where pixel p of the source image goes in a copy that carries a border of zero pixels (Wp == 0: no border, Pp == P)
-struct PixRemap { int64_t Pp; uint32_t W, Wp, off0; };
+// Where pixel p of the source image goes in a copy that carries a border of zero pixels (on == 0: no border, Pp == P): every row
+// skips the Wp - W border pixels beside it, every depth slice the Hp - H border rows
+struct PixRemap { int64_t Pp; FastDiv div_w, div_hw; uint32_t on, row_skip, slice_skip, off0; };
 __device__ __forceinline__ int64_t remap_pixel(const PixRemap& r, int64_t p) {
-    return r.Wp ? p + (int64_t)((uint32_t)p / r.W) * (r.Wp - r.W) + r.off0 : p;
+    if (!r.on) return p;
+    uint32_t skip = fast_div((uint32_t)p, r.div_w) * r.row_skip + r.off0;      // (a padded image has fewer than 2^31 pixels)
+    if (r.slice_skip) skip += fast_div((uint32_t)p, r.div_hw) * r.slice_skip;   // (uniform)
+    return p + skip;
 }
 static PixRemap make_remap(const HaloMap* h, int64_t P) {
     PixRemap r;
-    r.Pp = P; r.W = 1; r.Wp = 0; r.off0 = 0;
-    if (h && h->Wp) { r.Pp = h->Hp * h->Wp; r.W = (uint32_t)h->W; r.Wp = (uint32_t)h->Wp; r.off0 = (uint32_t)(h->top * h->Wp + h->left); }
+    std::memset(&r, 0, sizeof r);
+    r.Pp = P;
+    if (h && h->Wp) {
+        r.Pp = h->vol(); r.on = 1;
+        r.div_w = make_fastdiv((uint32_t)h->W); r.div_hw = make_fastdiv((uint32_t)(h->H * h->W));
+        r.row_skip = (uint32_t)(h->Wp - h->W); r.slice_skip = (uint32_t)((h->Hp - h->H) * h->Wp);
+        r.off0 = (uint32_t)((h->front * h->Hp + h->top) * h->Wp + h->left);
+    }
     return r;
 }
 
-// zeros the border pixels of a channels-last copy [B][Hp * Wp][C] (16-byte pieces; C * sizeof(T) a multiple of 16).
-// Only the border is visited: its pixels are numbered top rows, bottom rows, then the left and right pieces of the
-// image's rows.
+// zeros the border pixels of a channels-last copy [B][Dp * Hp * Wp][C] (16-byte pieces; C * sizeof(T) a multiple of 16).
+// Only the border is visited: its pixels are numbered front slices, back slices, then slice by slice the top rows, the bottom
+// rows and the left and right pieces of the image's rows.
 // (vectors first, first + step, ... of the per_image 16-byte vectors of one image's border)
 __device__ __forceinline__ void zero_border_vectors(uint4* __restrict__ img, const uint32_t per_image, const uint32_t vec_per_pixel, const HaloMap& h,
                                                     const uint32_t first, const uint32_t step) {
     const uint32_t top_n = (uint32_t)(h.top * h.Wp), bot_n = (uint32_t)((h.Hp - h.top - h.H) * h.Wp), side = (uint32_t)(h.Wp - h.W);
+    const uint32_t slice = (uint32_t)(h.Hp * h.Wp), slice_n = slice - (uint32_t)(h.H * h.W);
+    const uint32_t front_n = (uint32_t)h.front * slice, back_n = (uint32_t)(h.Dp - h.front - h.D) * slice;
     for (uint32_t i = first; i < per_image; i += step) {
-        uint32_t j = i / vec_per_pixel, pix;
+        uint32_t j = i / vec_per_pixel, pix, d0 = 0u;
         const uint32_t v = i - j * vec_per_pixel;
+        if (h.Dp > 1) {                                               // (uniform)
+            if (j < front_n + back_n) {
+                pix = j < front_n ? j : j + (uint32_t)h.D * slice;
+                img[(int64_t)pix * vec_per_pixel + v] = make_uint4(0u, 0u, 0u, 0u);
+                continue;
+            }
+            j -= front_n + back_n;
+            const uint32_t d = j / slice_n;
+            j -= d * slice_n;
+            d0 = ((uint32_t)h.front + d) * slice;
+        }
         if (j < top_n) pix = j;
         else if (j < top_n + bot_n) pix = (uint32_t)((h.top + h.H) * h.Wp) + (j - top_n);
         else {
@@ -335,22 +362,22 @@ __device__ __forceinline__ void zero_border_vectors(uint4* __restrict__ img, con
             const uint32_t row = j / side, c = j - row * side;
             pix = (uint32_t)((h.top + row) * h.Wp) + (c < (uint32_t)h.left ? c : (uint32_t)h.W + c);
         }
-        img[(int64_t)pix * vec_per_pixel + v] = make_uint4(0u, 0u, 0u, 0u);
+        img[(int64_t)(d0 + pix) * vec_per_pixel + v] = make_uint4(0u, 0u, 0u, 0u);
     }
 }
 __global__ void __launch_bounds__(256) halo_zero_kernel(uint4* __restrict__ out, const uint32_t per_image, const uint32_t vec_per_pixel, const HaloMap h) {
-    zero_border_vectors(out + (int64_t)blockIdx.y * (h.Hp * h.Wp) * vec_per_pixel, per_image, vec_per_pixel, h, blockIdx.x * 256u + threadIdx.x, gridDim.x * 256u);
+    zero_border_vectors(out + (int64_t)blockIdx.y * h.vol() * vec_per_pixel, per_image, vec_per_pixel, h, blockIdx.x * 256u + threadIdx.x, gridDim.x * 256u);
 }
 hipError_t launch_halo_zero(int64_t es, void* out, int64_t batch, int64_t C, const HaloMap& h, hipStream_t s) {
     if ((C * es) % 16 != 0 || (reinterpret_cast<uintptr_t>(out) & 15) != 0) return hipErrorInvalidValue;
-    const int64_t vpp = C * es / 16, border = h.Hp * h.Wp - h.H * h.W, per_image = border * vpp;
+    const int64_t vpp = C * es / 16, border = h.border(), per_image = border * vpp;
     if (batch <= 0 || per_image <= 0) return hipSuccess;
-    if (per_image > 0x7fffffffLL || h.Hp * h.Wp > 0x7fffffffLL) return hipErrorInvalidValue;
+    if (per_image > 0x7fffffffLL || h.vol() > 0x7fffffffLL) return hipErrorInvalidValue;
     const int64_t gx = std::min<int64_t>((per_image + 255) / 256, 64);
     for (int64_t b0 = 0; b0 < batch; b0 += 65535) {
         const int64_t nb = std::min<int64_t>(batch - b0, 65535);
         hipLaunchKernelGGL(halo_zero_kernel, dim3((unsigned)gx, (unsigned)nb), dim3(256), 0, s,
-                           (uint4*)out + b0 * h.Hp * h.Wp * vpp, (uint32_t)per_image, (uint32_t)vpp, h);
+                           (uint4*)out + b0 * h.vol() * vpp, (uint32_t)per_image, (uint32_t)vpp, h);
     }
     return hipGetLastError();
 }
@@ -461,8 +488,8 @@ hipError_t launch_nchw_to_nhwc(int64_t es, const void* in, void* out, int64_t ba
     std::memset(&ex, 0, sizeof ex);
     if (vec_ok && (es == 2 || es == 4) && took_along) {
         // (the caller acts on *took_along: without it the copy stays what it was)
-        const int64_t vpp = C * es / 16, border = halo && halo->Wp ? halo->Hp * halo->Wp - halo->H * halo->W : 0;
-        if (border * vpp <= 0x7fffffffLL && (!halo || halo->Hp * halo->Wp <= 0x7fffffffLL)) {
+        const int64_t vpp = C * es / 16, border = halo && halo->Wp ? halo->border() : 0;
+        if (border * vpp <= 0x7fffffffLL && (!halo || halo->vol() <= 0x7fffffffLL)) {
             if (border > 0) { ex.h = *halo; ex.border_vecs = (uint32_t)(border * vpp); ex.vpp = (uint32_t)vpp; }
             if (job && job->kind) {
                 ex.job = *job;

@@ -810,3 +810,45 @@ def test_conv2d_backward_fp32_host_entry_is_the_reference_bit_for_bit(geom):
     dcol = _dcol_plane(oracle, w, g, B, C, O, kh, kw, groups, None)
     want = _col2im_onto(dx0, dcol, (H, W), (kh, kw), dl, pd, st)
     assert np.array_equal(dx.view(np.uint32), np.ascontiguousarray(want).view(np.uint32)), (geom, "d_image +=")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("geom", [
+    # (B, C, size, O, kernel, stride, padding, dilation, groups)
+    (2, 32, (6, 7, 5), 16, (3, 3, 3), 1, 1, 1, 1),                    # three axes, odd planes (element-wise stores), dY through its copy
+    (3, 64, (4, 5, 8), 72, (3, 2, 1), (1, 2, 1), (1, 1, 0), (1, 1, 2), 2),   # groups, a stride and a dilation; the outputs end inside a tile
+    (1, 32, (1, 9, 16), 8, (1, 3, 3), 1, (0, 1, 1), 1, 1),            # a depth of one: the border has no front
+    (2, 16, (9, 4, 16), 128, (1, 1, 3), 1, (2, 0, 1), 1, 1),          # padding along the depth alone
+    (5, 16, (7, 7), 48, (3, 3), 1, 1, 1, 1),                          # weight gradient over 245 pixels: the last k range is 5 of them short
+    (1, 24, (33, 40), 64, (5, 3), (2, 1), (2, 1), 1, 1),              # one image, channels that end inside a 64-byte run
+    (9, 3, (70, 66), 16, (7, 7), 2, 3, 1, 1),                         # three channels, more output pixels than the window table holds
+    (3, 32, (1, 1), 32, (1, 1), 2, 0, 1, 1),                          # one output pixel per image
+], ids=lambda g: "x".join(map(str, g)))
+def test_channels_last_convolutions_over_two_and_three_axes(geom, dtype):
+    """Forward, image gradient and weight gradient (k ranges through all images) on the channels-last kernels at the edges of
+    their ranges, against float64 on the CPU.  Bounds: 16-bit results are one rounding of a Float32 sum (HALF_REL covers the weight
+    gradient's second one); a Float32 sum of K random products is off by about sqrt(K) * 2^-24 of the results' root mean square,
+    six of which (the largest of some 10^5 values) stay below 1e-6 * sqrt(K) of it."""
+    B, C, size, O, k, s, p, d, groups = geom
+    nd = len(size)
+    rng = np.random.default_rng(11 + B + C + O + sum(size))
+    x = torch.from_numpy(rng.standard_normal((B, C) + size)).to(dtype)
+    w = torch.from_numpy(rng.standard_normal((O, C // groups) + k)).to(dtype)
+    conv = torch.nn.functional.conv3d if nd == 3 else torch.nn.functional.conv2d
+    rx, rw = x.double().requires_grad_(True), w.double().requires_grad_(True)
+    ry = conv(rx, rw, None, s, p, d, groups)
+    g = torch.from_numpy(rng.standard_normal(tuple(ry.shape))).to(dtype)
+    ry.backward(g.double())
+    fwd, bwd = (F.conv3d, F.conv3d_backward) if nd == 3 else (F.conv2d, F.conv2d_backward)
+    y = fwd(x.to(DEV), w.to(DEV), stride=s, padding=p, dilation=d, groups=groups)
+    dx, dw = bwd(x.to(DEV), w.to(DEV), g.to(DEV), stride=s, padding=p, dilation=d, groups=groups)
+    taps = int(np.prod(k))
+    for name, got, want, depth in (("y", y, ry.detach(), C // groups * taps), ("dx", dx, rx.grad, O // groups * taps),
+                                   ("dw", dw, rw.grad, ry.numel() // O)):
+        got = got.double().cpu()
+        assert got.shape == want.shape and bool(torch.isfinite(got).all()), name
+        if dtype == torch.float32:
+            bound = 1e-6 * max(depth, 1) ** 0.5 * max(want.square().mean().sqrt().item(), 1.0)
+        else:
+            bound = HALF_REL * max(want.abs().max().item(), 1e-3)
+        assert (got - want).abs().max().item() <= bound, (name, (got - want).abs().max().item(), bound)
