@@ -25,6 +25,11 @@ hipError_t launch_conv_nhwc_bf16(const GemmParams& p, hipStream_t s) {
         return launch_ring_nhwc_cfg<DT_BF16, 2>(q, s);
     });
 }
+hipError_t launch_conv_nhwc_items_bf16(int edge, const GemmParams& p, int64_t blocks, hipStream_t s) {
+    if (edge == 256) return launch_ring_items_cfg<DT_BF16, 4>(p, blocks, s);
+    if (edge == 64) return launch_ring_items_cfg<DT_BF16, 1>(p, blocks, s);
+    return launch_ring_items_cfg<DT_BF16, 2>(p, blocks, s);
+}
 hipError_t launch_conv_nhwc_dw_bf16(bool ta, const GemmParams& p, hipStream_t s) {
     return launch_conv_nhwc16_planned(p, s, [&](int te, const GemmParams& q) {
         if (ta) {

@@ -203,7 +203,7 @@ __device__ __forceinline__ uint32_t lds_addr_of(const char* p) {
 constexpr int dw_table_entries(int wb) { return wb == 4 ? 6144 : 3584; }
 
 template <int DT, bool TA, bool TB, bool RAGGED, int WB_, int CONV = 0, int WBN_ = 0, int KD_ = 1>
-__global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams p) {
+__global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams pin) {
     using E = Elem<DT>;
     using T = typename E::T;
     constexpr int ES = sizeof(T);
@@ -218,9 +218,10 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams p) {
     constexpr int A_TILE_BYTES = GA::TILE_BYTES, STAGE_BYTES = GA::TILE_BYTES + G::TILE_BYTES;
     constexpr int WTM = GA::WT, WTN = G::WT;             // a wavefront's share of the tile: WTM rows x WTN columns
     constexpr bool GATHER4 = CONV == 1 || CONV == 2;     // op(B) gathered element by element from an NCHW image
-    constexpr bool GATHER16 = CONV == 3 || CONV == 5 || CONV == 6;   // op(B) = col^T gathered in 16-byte pieces from a channels-last image
-    constexpr bool HALO = CONV == 5 || CONV == 6;        // ... whose copy carries the padding as pixels of zeros: every tap of every window exists
-    constexpr bool DEPTH = CONV == 6;                    // ... over three spatial axes
+    constexpr bool ITEMS = CONV == 8;                    // several convolutions of one bordered image in one launch, each described by a RingItem
+    constexpr bool GATHER16 = CONV == 3 || CONV == 5 || CONV == 6 || ITEMS;   // op(B) = col^T gathered in 16-byte pieces from a channels-last image
+    constexpr bool HALO = CONV == 5 || CONV == 6 || ITEMS;   // ... whose copy carries the padding as pixels of zeros: every tap of every window exists
+    constexpr bool DEPTH = CONV == 6 || ITEMS;           // ... over three spatial axes
     constexpr bool GATHERW = CONV == 4 || CONV == 7;     // op(B) = col^T of a channels-last image, 16-byte pieces along the channels (weight gradient)
     constexpr bool DEPTHW = CONV == 7;                   // ... of a bordered copy over two or three axes, pixel by division (no table of window origins)
     constexpr bool A_KC = !TA, B_KC = GATHER4 ? false : GATHER16 ? true : GATHERW ? false : TB;
@@ -241,13 +242,36 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams p) {
     constexpr int DW_TABLE = CONV == 4 ? dw_table_entries(WB) : 1;   // (CONV = 7 has none)
     __shared__ int dw_tab[DW_TABLE];
 
-    if (p.gate && *p.gate != p.gate_want) return;       // (uniform: the other kernel of a gated pair does this product)
+    if (pin.gate && *pin.gate != pin.gate_want) return; // (uniform: the other kernel of a gated pair does this product)
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
 
-    const int lid = p.group_m < 0 ? (int)blockIdx.x : xcd_contiguous_id(blockIdx.x, gridDim.x);      // (group_m != 0: measurement only, see ring_tile_order_override)
+    int lid = pin.group_m < 0 ? (int)blockIdx.x : xcd_contiguous_id(blockIdx.x, gridDim.x);      // (group_m != 0: measurement only, see ring_tile_order_override)
+    typename std::conditional<ITEMS, GemmParams, const GemmParams&>::type p = pin;
+    if constexpr (ITEMS) {
+        // this workgroup's product: the last item whose first workgroup is not behind it
+        const __attribute__((address_space(4))) RingItem* it = (const __attribute__((address_space(4))) RingItem*)pin.conv.items;
+        int lo = 0, hi = pin.conv.n_items;
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (lid >= it[mid].first) lo = mid;
+            else hi = mid;
+        }
+        it += lo;
+        lid -= it->first;
+        p.A = static_cast<const T*>(pin.A) + it->a;
+        p.B = static_cast<const T*>(pin.B) + it->b;
+        p.C = static_cast<T*>(pin.C) + it->c;
+        p.K = it->K; p.lda = it->K;
+        p.N = it->N; p.tiles_n = it->tiles_n;
+        p.ldc = it->ldc; p.sC = pin.sC * it->ldc;              // (sC: channels of an image)
+        p.conv.k_d = it->k_d; p.conv.k_r = it->k_r; p.conv.k_c = it->k_c;
+        p.conv.Wo = it->Wo; p.conv.HoWo = it->HoWo;
+        p.conv.div_wo.m = it->div_wo.m; p.conv.div_wo.s1 = it->div_wo.s1; p.conv.div_wo.s2 = it->div_wo.s2;
+        p.conv.div_howo.m = it->div_howo.m; p.conv.div_howo.s1 = it->div_howo.s1; p.conv.div_howo.s2 = it->div_howo.s2;
+    }
     const int tiles = p.tiles_m * p.tiles_n;
     const int b = lid / tiles;
     int tm, tn;
@@ -1272,6 +1296,18 @@ static hipError_t launch_ring_nhwc_halo_cfg(const GemmParams& pin, hipStream_t s
     if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
     if (p.conv.k_d > 1 || p.conv.D > 1) hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 6>), dim3((unsigned)blocks), dim3(256), 0, s, p);
     else hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 5>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+    return hipGetLastError();
+}
+
+// several such convolutions in one launch (CONV = 8)
+template <int DT, int WB>
+static hipError_t launch_ring_items_cfg(const GemmParams& pin, int64_t blocks, hipStream_t s) {
+    constexpr int TE = RingGeom<WB, (int)sizeof(typename Elem<DT>::T)>::BM;
+    GemmParams p = pin;
+    p.tiles_m = (p.M + TE - 1) / TE;
+    if (blocks <= 0) return hipSuccess;
+    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 8>), dim3((unsigned)blocks), dim3(256), 0, s, p);
     return hipGetLastError();
 }
 

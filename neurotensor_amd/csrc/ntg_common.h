@@ -32,7 +32,7 @@ enum CMode : int {
 // Unsigned division by a divisor fixed at launch (round-up multiplier form): exact for every
 // 32-bit n.  q = (t + ((n - t) >> s1)) >> s2  with  t = mulhi(m, n).
 struct FastDiv { uint32_t m, s1, s2; };
-static inline FastDiv make_fastdiv(uint32_t d) {
+__host__ __device__ static inline FastDiv make_fastdiv(uint32_t d) {
     uint32_t l = 0;
     while ((1ull << l) < d) ++l;
     FastDiv f;
@@ -79,6 +79,9 @@ struct ConvGeom {
     // channels-last weight gradient on a copy that carries the padding as pixels of zeros (H, W describe the padded image,
     // p_r = p_c = 0): output pixels per image when the kernel keeps their window origins in an LDS table, 0: off
     int pix_table;
+    // channels-last convolution, several products in one launch: their table in device memory (see RingItem)
+    const struct RingItem* items;
+    int n_items;
     int tile_edge;           // channels-last weight gradient: the tile the caller planned with (0: the launcher's own choice)
 };
 
@@ -367,19 +370,30 @@ hipError_t launch_nchw_to_nhwc_padded(int64_t es, const void* in, void* out, int
 hipError_t launch_flip_weights_channels_last(int64_t es, const void* w, void* wt, int64_t groups, int64_t og, int64_t ogp, int64_t cg, int64_t taps, hipStream_t s, int64_t chunk = 0);
 // channels-last convolution (image [B][pixel][C], weights [O][(r, q, c)]); F16 / BF16 / F32, two spatial axes
 hipError_t launch_conv_nhwc(int dtype, const GemmParams& p, hipStream_t s);
-// Image gradient of a strided convolution as one stride-1 convolution per phase of the image (see conv_dimage_phases):
-// where the phase planes lie in the temporary buffer (element offsets; -1: the phase has no taps) and how image
-// coordinates map to them.  Strides up to 4.
+// Image gradient of a strided convolution as one stride-1 convolution per phase of the image (see conv_dimage_phases), up to
+// three axes, strides up to 4 (slowest axis first; two axes: everything of axis 0 is 1 or 0).  Phase (e0, e1, e2) is number
+// (e0 s1 + e1) s2 + e2; along an axis it holds n[e] image positions from a0[e] on, M[e] taps, and its windows start org[e]
+// pixels inside the bordered copy of dY.  plane_off: where its planes [batch][channels][ld] lie in the temporary buffer, w_off:
+// where its weights lie (elements; plane_off -1: the phase has no taps or no positions).
+#define NTG_MAX_PHASES 64
 struct PhaseLayout {
-    int H, W, p_r, p_c, s_r, s_c;
-    uint32_t total;              // batch * channels * H * W
-    int a0r[4], a0c[4], hp[4], wp[4];
-    int64_t off[16];
-    FastDiv div_w, div_h, div_sr, div_sc;
+    int sz[3], k[3], s[3], p[3], yp[3];              // image, kernel, strides, paddings; the bordered copy of dY
+    int M[3][4], a0[3][4], n[3][4], org[3][4];
+    int groups, og, ogp, cg, batch, phases, chunk;   // chunk: channels in 64 bytes (k order: run, tap, channel inside the run)
+    int tile_rows, tile_cols, vel;                   // of the launch; elements per 16 bytes: a plane's pitch is a multiple
+    FastDiv div_s[3], div_rows[3];
+    int64_t plane_off[NTG_MAX_PHASES], w_off[NTG_MAX_PHASES];
 };
-hipError_t launch_phase_weights(int64_t es, const void* w, void* wt, int64_t groups, int64_t og, int64_t ogp, int64_t cg, int64_t k_r, int64_t k_c,
-                                int64_t er, int64_t ec, int64_t s_r, int64_t s_c, int64_t Mr, int64_t Mc, hipStream_t s);
+__host__ __device__ static inline int phase_plane(const PhaseLayout& q, int e0, int e1, int e2) {
+    const int n = q.n[0][e0] * q.n[1][e1] * q.n[2][e2];
+    return (n + q.vel - 1) / q.vel * q.vel;
+}
+// One product of a launch that computes several convolutions of one bordered channels-last image (phases and groups): what
+// differs from item to item.  Offsets in elements from GemmParams::A / B / C; `first` = first workgroup.
+struct RingItem { int64_t a, b, c; int K, N, ldc, k_d, k_r, k_c, Wo, HoWo, first, tiles_n; FastDiv div_wo, div_howo; };
+hipError_t launch_phase_setup(int64_t es, const void* w, void* wt, RingItem* items, const PhaseLayout& q, hipStream_t s);
 hipError_t launch_phase_interleave(int dtype, const void* tmp, void* im, const PhaseLayout& q, int accumulate, hipStream_t s);
+hipError_t launch_conv_nhwc_items(int dtype, int edge, const GemmParams& p, int64_t blocks, hipStream_t s);
 // 16-, 32- and 64-bit integer products on the 8-bit matrix pipe as byte planes (see gemm_mfma_i8.hip); planes = bytes per element
 struct IntPlanesParams { int M, N, K, Kp, Np, batch; int64_t lda, ldb, sA, sB; int ta, tb; };
 hipError_t launch_int_split_planes(int planes, const void* A, const void* B, void* a_planes, void* b_planes, const IntPlanesParams& q, hipStream_t s);

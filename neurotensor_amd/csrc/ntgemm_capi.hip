@@ -55,6 +55,17 @@ hipError_t launch_conv_nhwc(int dtype, const GemmParams& p, hipStream_t s) {
     }
 }
 
+hipError_t launch_conv_nhwc_items_f32(int edge, const GemmParams& p, int64_t blocks, hipStream_t s);
+hipError_t launch_conv_nhwc_items_f16(int edge, const GemmParams& p, int64_t blocks, hipStream_t s);
+hipError_t launch_conv_nhwc_items_bf16(int edge, const GemmParams& p, int64_t blocks, hipStream_t s);
+hipError_t launch_conv_nhwc_items(int dtype, int edge, const GemmParams& p, int64_t blocks, hipStream_t s) {
+    switch (dtype) {
+    case DT_F32: return launch_conv_nhwc_items_f32(edge, p, blocks, s);
+    case DT_F16: return launch_conv_nhwc_items_f16(edge, p, blocks, s);
+    case DT_BF16: return launch_conv_nhwc_items_bf16(edge, p, blocks, s);
+    default: return hipErrorInvalidValue;
+    }
+}
 hipError_t launch_conv_nhwc_dw_f32(bool ta, const GemmParams& p, hipStream_t s);
 hipError_t launch_conv_nhwc_dw_f16(bool ta, const GemmParams& p, hipStream_t s);
 hipError_t launch_conv_nhwc_dw_bf16(bool ta, const GemmParams& p, hipStream_t s);
@@ -1428,110 +1439,140 @@ static int conv_dimage_nhwc(int dtype, const void* kernel, const void* grad_out,
     return NTG_OK;
 }
 
-// dX of a convolution with strides > 1 (dilation 1), without the col matrix: the image rows y with (y + p) mod s = e
+// dX of a convolution with strides > 1 (dilation 1), without the col matrix: the image positions y with (y + p) mod s = e
 // form one phase; they receive only the taps i = e + s m (m = 0 .. M_e - 1), and, with a = (y + p) / s,
 //   dX[y] = sum_m dY[a - m] W[e + s m],
-// a stride-1 convolution of dY with the M_e reversed taps.  So every phase (er, ec) is one channels-last convolution
-// (the forward kernel) of the shared channels-last copy of dY with its own small kernel, written to a plane of the
-// phase's rows and columns in the workspace; a last pass interleaves the planes into dX.  Exactly the products of the
-// reference's GEMM + col2im, none wasted on the zeros a dilated gradient would hold.
+// a stride-1 convolution of dY with the M_e reversed taps.  So every phase (one per residue of each axis) is one channels-last
+// convolution of the shared bordered copy of dY with its own small kernel, written to a plane of the phase's positions in the
+// workspace; a last pass interleaves the planes into dX.  Exactly the products of the reference's GEMM + col2im, none wasted on
+// the zeros a dilated gradient would hold.  All phases (and groups) are items of ONE launch: a phase alone is a small product
+// (32 x 64 x 56 x 56 by 4 x 4 at stride 2: 416 tiles of k = 512), and four launches with a weight permutation each took 58 us
+// where the one takes 20.
 struct PhasePlan {
     bool ok;
-    int64_t Mr[4], Mc[4], a0r[4], a0c[4], hp[4], wp[4];
-    int64_t ogp, gy_bytes, w_bytes, tmp_bytes;
+    int edge;
+    int64_t gy_bytes, w_bytes, item_bytes, tmp_bytes, blocks;
+    ntg::HaloMap hm;
+    ntg::PhaseLayout lay;
+    int64_t bytes() const { return gy_bytes + w_bytes + item_bytes + tmp_bytes; }
 };
-static Geo3 phase_geo(const Geo3& g, const PhasePlan& pp, int er, int ec) {
-    // image = the dY plane, kernel Mr x Mc, stride 1, padding (M - 1) - a0 (first row of the plane is a0), outputs hp x wp
-    return Geo3{2, {1, g.o[1], g.o[2]}, {1, pp.Mr[er], pp.Mc[ec]}, {1, 1, 1}, {0, pp.Mr[er] - 1 - pp.a0r[er], pp.Mc[ec] - 1 - pp.a0c[ec]},
-                {1, 1, 1}, {1, pp.hp[er], pp.wp[ec]}};
-}
 static PhasePlan plan_dimage_phases(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
     PhasePlan pp;
     std::memset(&pp, 0, sizeof pp);
     if (dtype != ntg::DT_F32 && dtype != ntg::DT_F16 && dtype != ntg::DT_BF16) return pp;
-    if (g.nd != 2 || g.d[1] != 1 || g.d[2] != 1 || (g.s[1] == 1 && g.s[2] == 1) || g.s[1] > 4 || g.s[2] > 4 || g.p[1] < 0 || g.p[2] < 0) return pp;
-    if (g.k[1] > 8 * g.s[1] || g.k[2] > 8 * g.s[2]) return pp;
-    const int64_t es = ntg::elem_size(dtype), og = out_channels / groups;
-    pp.ogp = nhwc_padded_channels(es, og);
-    if (pp.ogp == 0 || batch * channels * g.vol() >= 0x7fffffffLL) return pp;
+    if (g.s[0] == 1 && g.s[1] == 1 && g.s[2] == 1) return pp;
+    for (int a = 0; a < 3; ++a)
+        if (g.d[a] != 1 || g.s[a] > 4 || g.p[a] < 0 || g.sz[a] >= (1 << 24) || g.k[a] >= (1 << 16)) return pp;
+    const int64_t es = ntg::elem_size(dtype), vel = 16 / es, og = out_channels / groups, cg = channels / groups;
+    const int64_t ogp = nhwc_padded_channels(es, og), ochp = groups * ogp;
+    if (ogp == 0 || batch * channels * (g.vol() + 64 * vel) >= 0x7fffffffLL) return pp;
     // the image channels of a group are the rows of these products: with a handful of them (an RGB input layer) a 64-row
     // tile is mostly padding, and the GEMM over (channel, tap) rows followed by col2im is the better form
-    if (channels / groups < 16) return pp;
-    for (int ax = 1; ax <= 2; ++ax) {
-        int64_t* M = ax == 1 ? pp.Mr : pp.Mc;
-        int64_t* a0 = ax == 1 ? pp.a0r : pp.a0c;
-        int64_t* n = ax == 1 ? pp.hp : pp.wp;
+    if (cg < 16) return pp;
+    ntg::PhaseLayout& q = pp.lay;
+    int64_t front[3];
+    for (int ax = 0; ax < 3; ++ax) {
+        q.sz[ax] = (int)g.sz[ax]; q.k[ax] = (int)g.k[ax]; q.s[ax] = (int)g.s[ax]; q.p[ax] = (int)g.p[ax];
+        q.div_s[ax] = ntg::make_fastdiv((uint32_t)g.s[ax]);
+        q.div_rows[ax] = ntg::make_fastdiv((uint32_t)g.sz[ax]);
+        front[ax] = 0;
         for (int64_t e = 0; e < g.s[ax]; ++e) {
-            M[e] = e < g.k[ax] ? (g.k[ax] - e + g.s[ax] - 1) / g.s[ax] : 0;
+            q.M[ax][e] = (int)(e < g.k[ax] ? (g.k[ax] - e + g.s[ax] - 1) / g.s[ax] : 0);
             // image positions y = s a + e - p in [0, size): a from a0
-            a0[e] = g.p[ax] > e ? (g.p[ax] - e + g.s[ax] - 1) / g.s[ax] : 0;
+            q.a0[ax][e] = (int)(g.p[ax] > e ? (g.p[ax] - e + g.s[ax] - 1) / g.s[ax] : 0);
             const int64_t last = g.sz[ax] - 1 + g.p[ax] - e;                      // largest s a
-            n[e] = last >= 0 && last / g.s[ax] >= a0[e] ? last / g.s[ax] - a0[e] + 1 : 0;
+            q.n[ax][e] = (int)(last >= 0 && last / g.s[ax] >= q.a0[ax][e] ? last / g.s[ax] - q.a0[ax][e] + 1 : 0);
+            // the window of the phase's first position begins (M - 1) - a0 before dY (behind it if negative)
+            if (q.M[ax][e] && q.n[ax][e]) front[ax] = std::max<int64_t>(front[ax], q.M[ax][e] - 1 - q.a0[ax][e]);
         }
+        int64_t ext = front[ax] + g.o[ax];
+        for (int64_t e = 0; e < g.s[ax]; ++e) {
+            q.org[ax][e] = (int)(front[ax] - (q.M[ax][e] - 1 - q.a0[ax][e]));
+            if (q.M[ax][e] && q.n[ax][e]) ext = std::max<int64_t>(ext, q.org[ax][e] + q.n[ax][e] - 1 + q.M[ax][e]);
+        }
+        q.yp[ax] = (int)ext;
     }
-    int64_t wmax = 0, tmp = 0;
-    for (int64_t er = 0; er < g.s[1]; ++er)
-        for (int64_t ec = 0; ec < g.s[2]; ++ec) {
-            if (pp.Mr[er] == 0 || pp.Mc[ec] == 0 || pp.hp[er] == 0 || pp.wp[ec] == 0) continue;
-            if (!conv_nhwc_ok(dtype, out_channels, channels, groups, phase_geo(g, pp, (int)er, (int)ec))) return pp;
-            wmax += (int64_t)align_up((size_t)(channels * pp.Mr[er] * pp.Mc[ec] * pp.ogp * es), 256);
-            tmp += (int64_t)align_up((size_t)(batch * channels * pp.hp[er] * pp.wp[ec] * es), 256);
-        }
-    pp.gy_bytes = (int64_t)align_up((size_t)(batch * groups * pp.ogp * g.L() * es), 256);
-    pp.w_bytes = wmax;
-    pp.tmp_bytes = tmp;
+    const int64_t volp = (int64_t)q.yp[0] * q.yp[1] * q.yp[2];
+    const Geo3 reach = {g.nd, {q.yp[0], q.yp[1], q.yp[2]}, {g.k[0], g.k[1], g.k[2]}, {1, 1, 1}, {0, 0, 0}, {1, 1, 1}, {1, 1, 1}};
+    if (volp > 4 * g.L() + 64 || !conv_nhwc_offsets_fit(ochp, es, reach) || ogp * g.taps() >= 0x7fffffffLL) return pp;
+    pp.hm.W = g.o[2]; pp.hm.H = g.o[1]; pp.hm.D = g.o[0];
+    pp.hm.Wp = q.yp[2]; pp.hm.Hp = q.yp[1]; pp.hm.Dp = q.yp[0];
+    pp.hm.left = front[2]; pp.hm.top = front[1]; pp.hm.front = front[0];
+    q.groups = (int)groups; q.og = (int)og; q.ogp = (int)ogp; q.cg = (int)cg; q.batch = (int)batch;
+    q.chunk = (int)(64 / es); q.vel = (int)vel;
+    int64_t w_elems = 0, tmp_elems = 0, n_max = 0, k_max = 0;
+    for (int ph = 0; ph < NTG_MAX_PHASES; ++ph) q.plane_off[ph] = -1;
+    for (int e0 = 0; e0 < q.s[0]; ++e0)
+        for (int e1 = 0; e1 < q.s[1]; ++e1)
+            for (int e2 = 0; e2 < q.s[2]; ++e2) {
+                const int64_t taps = (int64_t)q.M[0][e0] * q.M[1][e1] * q.M[2][e2], n = (int64_t)q.n[0][e0] * q.n[1][e1] * q.n[2][e2];
+                if (taps == 0 || n == 0) continue;
+                const int ph = (e0 * q.s[1] + e1) * q.s[2] + e2;
+                q.w_off[ph] = w_elems;
+                q.plane_off[ph] = tmp_elems;
+                w_elems += channels * taps * ogp;                                 // (ogp is a multiple of 64 bytes)
+                tmp_elems += batch * channels * ntg::phase_plane(q, e0, e1, e2);
+                n_max = std::max(n_max, n); k_max = std::max(k_max, taps * ogp);
+                ++q.phases;
+            }
+    if (q.phases == 0) return pp;
+    // one tile for all items, as if they were equal
+    const int64_t items = (int64_t)q.phases * groups;
+    if (es == 4) {
+        const int64_t t128 = ((cg + 127) / 128) * ((n_max + 127) / 128) * batch * items, t64 = ((cg + 63) / 64) * ((n_max + 63) / 64) * batch * items;
+        pp.edge = 1.07 * 0.25 * (double)((t64 + 255) / 256) < (double)((t128 + 255) / 256) ? 64 : 128;
+    } else {
+        pp.edge = ntg::ring16_tile_edge(cg, n_max, k_max, batch * items);
+    }
+    q.tile_rows = q.tile_cols = pp.edge;
+    const int64_t tiles_m = (cg + pp.edge - 1) / pp.edge;
+    for (int e0 = 0; e0 < q.s[0]; ++e0)
+        for (int e1 = 0; e1 < q.s[1]; ++e1)
+            for (int e2 = 0; e2 < q.s[2]; ++e2) {
+                if (q.plane_off[(e0 * q.s[1] + e1) * q.s[2] + e2] < 0) continue;
+                const int64_t n = (int64_t)q.n[0][e0] * q.n[1][e1] * q.n[2][e2];
+                pp.blocks += tiles_m * ((n + pp.edge - 1) / pp.edge) * batch * groups;
+            }
+    if (pp.blocks > 0x7fffffffLL) return pp;
+    pp.gy_bytes = (int64_t)align_up((size_t)(batch * ochp * volp * es), 256);
+    pp.w_bytes = (int64_t)align_up((size_t)(w_elems * es), 256);
+    pp.item_bytes = (int64_t)align_up((size_t)items * sizeof(ntg::RingItem), 256);
+    pp.tmp_bytes = (int64_t)align_up((size_t)(tmp_elems * es), 256);
     pp.ok = true;
     return pp;
 }
 static int conv_dimage_phases(int dtype, const PhasePlan& pp, const void* kernel, const void* grad_out, void* d_image, void* ws, int64_t batch,
                               int64_t channels, int64_t out_channels, const Geo3& g, int64_t groups, int accumulate, hipStream_t hs) {
-    const int64_t es = ntg::elem_size(dtype), cg = channels / groups, og = out_channels / groups;
-    const int64_t ogp = pp.ogp, ochp = groups * ogp, L = g.L();
+    const ntg::PhaseLayout& q = pp.lay;
+    const int64_t es = ntg::elem_size(dtype), og = q.og, ogp = q.ogp, ochp = groups * ogp, L = g.L();
     char* ws_gy = static_cast<char*>(ws);
     char* ws_w = ws_gy + pp.gy_bytes;
-    char* ws_tmp = ws_w + pp.w_bytes;
-    hipError_t e = ogp == og ? ntg::launch_nchw_to_nhwc(es, grad_out, ws_gy, batch, out_channels, L, hs)
-                             : ntg::launch_nchw_to_nhwc_padded(es, grad_out, ws_gy, batch, groups, og, ogp, L, hs);
+    char* ws_items = ws_w + pp.w_bytes;
+    char* ws_tmp = ws_items + pp.item_bytes;
+    bool took_along = false;
+    hipError_t e = ogp == og ? ntg::launch_nchw_to_nhwc(es, grad_out, ws_gy, batch, out_channels, L, hs, &pp.hm, nullptr, &took_along)
+                             : ntg::launch_nchw_to_nhwc_padded(es, grad_out, ws_gy, batch, groups, og, ogp, L, hs, &pp.hm);
+    if (e == hipSuccess && pp.hm.border() > 0 && !took_along) e = ntg::launch_halo_zero(es, ws_gy, batch, ochp, pp.hm, hs);
     if (e != hipSuccess) return hip_fail(e, "channels-last copy launch");
-    ntg::PhaseLayout lay;
-    std::memset(&lay, 0, sizeof lay);
-    lay.H = (int)g.sz[1]; lay.W = (int)g.sz[2]; lay.p_r = (int)g.p[1]; lay.p_c = (int)g.p[2]; lay.s_r = (int)g.s[1]; lay.s_c = (int)g.s[2];
-    lay.total = (uint32_t)(batch * channels * g.vol());
-    lay.div_w = ntg::make_fastdiv((uint32_t)lay.W); lay.div_h = ntg::make_fastdiv((uint32_t)lay.H);
-    lay.div_sr = ntg::make_fastdiv((uint32_t)lay.s_r); lay.div_sc = ntg::make_fastdiv((uint32_t)lay.s_c);
-    for (int i = 0; i < 4; ++i) { lay.a0r[i] = (int)pp.a0r[i]; lay.a0c[i] = (int)pp.a0c[i]; lay.hp[i] = (int)pp.hp[i]; lay.wp[i] = (int)pp.wp[i]; }
-    for (int i = 0; i < 16; ++i) lay.off[i] = -1;
-    int64_t w_off = 0, t_off = 0;
-    for (int64_t er = 0; er < g.s[1]; ++er)
-        for (int64_t ec = 0; ec < g.s[2]; ++ec) {
-            if (pp.Mr[er] == 0 || pp.Mc[ec] == 0 || pp.hp[er] == 0 || pp.wp[ec] == 0) continue;
-            const Geo3 t = phase_geo(g, pp, (int)er, (int)ec);
-            const int64_t taps = pp.Mr[er] * pp.Mc[ec], K = taps * ogp, plane = pp.hp[er] * pp.wp[ec];
-            char* wph = ws_w + w_off;
-            char* tph = ws_tmp + t_off;
-            e = ntg::launch_phase_weights(es, kernel, wph, groups, og, ogp, cg, g.k[1], g.k[2], er, ec, g.s[1], g.s[2], pp.Mr[er], pp.Mc[ec], hs);
-            if (e != hipSuccess) return hip_fail(e, "phase weight launch");
-            for (int64_t gi = 0; gi < groups; ++gi) {
-                ntg::GemmParams p;
-                std::memset(&p, 0, sizeof p);
-                p.M = (int)cg; p.K = (int)K; p.N = (int)plane; p.batch = (int)batch;
-                p.A = wph + gi * cg * K * es;
-                p.B = ws_gy + gi * ogp * es;
-                p.C = tph + gi * cg * plane * es;
-                p.lda = K; p.ldb = ochp; p.ldc = plane;
-                p.sA = 0; p.sB = ochp * L; p.sC = channels * plane;
-                p.cmode = ntg::C_OVERWRITE;
-                p.vecA_ok = 1; p.vecB_ok = 1;
-                fill_conv_geom(p.conv, ogp, t);
-                p.conv.chan = (int)ochp;
-                e = ntg::launch_conv_nhwc(dtype, p, hs);
-                if (e != hipSuccess) return hip_fail(e, "phase convolution launch");
-            }
-            lay.off[er * g.s[2] + ec] = t_off / es;
-            w_off += (int64_t)align_up((size_t)(channels * taps * ogp * es), 256);
-            t_off += (int64_t)align_up((size_t)(batch * channels * plane * es), 256);
-        }
-    e = ntg::launch_phase_interleave(dtype, ws_tmp, d_image, lay, accumulate, hs);
+    ntg::RingItem* items = reinterpret_cast<ntg::RingItem*>(ws_items);
+    e = ntg::launch_phase_setup(es, kernel, ws_w, items, q, hs);
+    if (e != hipSuccess) return hip_fail(e, "phase weight launch");
+    ntg::GemmParams p;
+    std::memset(&p, 0, sizeof p);
+    p.M = q.cg; p.batch = (int)batch;
+    p.A = ws_w; p.B = ws_gy; p.C = ws_tmp;
+    p.ldb = ochp; p.sB = ochp * pp.hm.vol(); p.sC = channels;
+    p.cmode = ntg::C_OVERWRITE;
+    p.vecA_ok = 1; p.vecB_ok = 1;
+    p.conv.D = q.yp[0]; p.conv.H = q.yp[1]; p.conv.W = q.yp[2]; p.conv.chan = (int)ochp;
+    p.conv.s_d = p.conv.s_r = p.conv.s_c = 1;
+    p.conv.d_d = p.conv.d_r = p.conv.d_c = 1;
+    p.conv.k_drc = 1;                                      // (the items set their own taps; k runs taps-inner, which does not use it)
+    p.conv.halo = 1; p.conv.tap_inner = 1;
+    p.conv.items = items; p.conv.n_items = q.phases * (int)groups;
+    e = ntg::launch_conv_nhwc_items(dtype, pp.edge, p, pp.blocks, hs);
+    if (e != hipSuccess) return hip_fail(e, "phase convolution launch");
+    e = ntg::launch_phase_interleave(dtype, ws_tmp, d_image, q, accumulate, hs);
     if (e != hipSuccess) return hip_fail(e, "phase interleave launch");
     return NTG_OK;
 }
@@ -1766,10 +1807,10 @@ static ConvBackwardPlan plan_conv_backward_g(int dtype, bool want_dx, bool want_
     pl.need_nhwc_dw = pl.nhwc_dw ? conv_dkernel_nhwc_workspace(dtype, pl.dkernel, batch, channels, out_channels, groups, g) : 0;
     // strides > 1: dX phase by phase instead of GEMM + col2im, again when the workspace allows
     std::memset(&pl.phases, 0, sizeof pl.phases);
-    if (want_dx && !pl.gather_dx && !reference_order && conv_implicit_g(dtype, out_channels, geo_dimage(g)))
+    if (want_dx && !pl.gather_dx && !reference_order)
         pl.phases = plan_dimage_phases(dtype, batch, channels, out_channels, groups, g);
     pl.phase_dx = pl.phases.ok;
-    pl.need_phase_dx = pl.phase_dx ? pl.phases.gy_bytes + pl.phases.w_bytes + pl.phases.tmp_bytes : 0;
+    pl.need_phase_dx = pl.phase_dx ? pl.phases.bytes() : 0;
     return pl;
 }
 
@@ -2414,6 +2455,12 @@ static int convnd_backward_dev_impl(int dtype, const void* image, const void* ke
             else
                 rc = conv_dimage_gather(dtype, kernel, grad_out, d_image, workspace, batch, channels, out_channels, g, groups, accumulate,
                                         static_cast<hipStream_t>(stream));
+            if (rc) return rc;
+            d_image = nullptr;
+        }
+        if (d_image && channels_last && plan.phase_dx && workspace_bytes >= plan.need_phase_dx && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0) {
+            rc = conv_dimage_phases(dtype, plan.phases, kernel, grad_out, d_image, workspace, batch, channels, out_channels, g, groups, accumulate,
+                                    static_cast<hipStream_t>(stream));
             if (rc) return rc;
             d_image = nullptr;
         }

@@ -539,70 +539,147 @@ hipError_t launch_flip_weights_channels_last(int64_t es, const void* w, void* wt
     return hipGetLastError();
 }
 
-// Weights of one phase of a strided convolution's image gradient: the taps i = er + s_r (Mr-1-mr), j = ec + s_c (Mc-1-mc)
-// of w [g*og + oc][c][k_r][k_c], as wt[g][c][(mr, mc)][oc] with the out channels padded with zeros from og to ogp.
-struct PhaseWeights { int64_t groups, og, ogp, cg, k_r, k_c, er, ec, s_r, s_c, Mr, Mc; };
+// Weights of all phases of a strided convolution's image gradient, and the table of their products.  Phase e has the taps
+// e + s (M - 1 - m) of w [g*og + oc][c][taps], reversed, as wt[g][c][(run, m0, m1, m2, oc in run)] with the out channels padded with
+// zeros from og to ogp and in runs of `chunk` (see ConvGeom::tap_inner).  One thread per (group, image channel, tap, out channel):
+// every tap belongs to one phase.  The first threads write the table.
 template <class T>
-__global__ void __launch_bounds__(256) phase_weights_kernel(const T* __restrict__ w, T* __restrict__ wt, const PhaseWeights q) {
-    const int64_t total = q.groups * q.cg * q.Mr * q.Mc * q.ogp;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += stride) {
-        const int64_t oc = idx % q.ogp;
+__global__ void __launch_bounds__(256) phase_setup_kernel(const T* __restrict__ w, T* __restrict__ wt, RingItem* __restrict__ items, const PhaseLayout q) {
+    const int taps = q.k[0] * q.k[1] * q.k[2];
+    const int64_t total = (int64_t)q.groups * q.cg * taps * q.ogp;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x, first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    for (int64_t idx = first; idx < total; idx += stride) {
+        const int oc = (int)(idx % q.ogp);
         int64_t r = idx / q.ogp;
-        const int64_t mc = r % q.Mc;
-        r /= q.Mc;
-        const int64_t mr = r % q.Mr;
-        r /= q.Mr;
-        const int64_t c = r % q.cg, g = r / q.cg;
-        const int64_t i = q.er + q.s_r * (q.Mr - 1 - mr), j = q.ec + q.s_c * (q.Mc - 1 - mc);
-        wt[idx] = oc < q.og ? w[(((g * q.og + oc) * q.cg + c) * q.k_r + i) * q.k_c + j] : (T)0;
+        int tap = (int)(r % taps);
+        const int src_tap = tap;
+        r /= taps;                                                     // g * cg + c
+        int e[3], m[3];
+#pragma unroll
+        for (int a = 2; a >= 0; --a) {
+            const int i = tap % q.k[a];
+            tap /= q.k[a];
+            e[a] = i % q.s[a];
+            m[a] = q.M[a][e[a]] - 1 - i / q.s[a];
+        }
+        const int ph = (e[0] * q.s[1] + e[1]) * q.s[2] + e[2];
+        if (q.plane_off[ph] < 0) continue;
+        const int ptaps = q.M[0][e[0]] * q.M[1][e[1]] * q.M[2][e[2]], t = (m[0] * q.M[1][e[1]] + m[1]) * q.M[2][e[2]] + m[2];
+        const int64_t g = r / q.cg, c = r - g * q.cg;
+        wt[q.w_off[ph] + r * ptaps * q.ogp + ((int64_t)(oc / q.chunk) * ptaps + t) * q.chunk + oc % q.chunk] =
+            oc < q.og ? w[((g * q.og + oc) * q.cg + c) * taps + src_tap] : (T)0;
+    }
+    // item (live phase, group)
+    for (int64_t i = first; i < (int64_t)q.phases * q.groups; i += stride) {
+        const int want = (int)(i / q.groups), g = (int)(i % q.groups);
+        const int tiles_m = (q.cg + q.tile_rows - 1) / q.tile_rows;
+        int64_t start = 0;
+        int live = 0;
+        for (int ph = 0; ph < q.s[0] * q.s[1] * q.s[2]; ++ph) {
+            if (q.plane_off[ph] < 0) continue;
+            const int e2 = ph % q.s[2], e1 = ph / q.s[2] % q.s[1], e0 = ph / (q.s[2] * q.s[1]);
+            const int N = q.n[0][e0] * q.n[1][e1] * q.n[2][e2], tiles_n = (N + q.tile_cols - 1) / q.tile_cols;
+            const int64_t per_group = (int64_t)tiles_m * tiles_n * q.batch;
+            if (live++ < want) { start += per_group * q.groups; continue; }
+            const int ptaps = q.M[0][e0] * q.M[1][e1] * q.M[2][e2], ochp = q.groups * q.ogp;
+            RingItem it;
+            it.K = ptaps * q.ogp; it.N = N; it.ldc = phase_plane(q, e0, e1, e2);
+            it.a = q.w_off[ph] + (int64_t)g * q.cg * it.K;
+            it.b = (((int64_t)q.org[0][e0] * q.yp[1] + q.org[1][e1]) * q.yp[2] + q.org[2][e2]) * ochp + (int64_t)g * q.ogp;
+            it.c = q.plane_off[ph] + (int64_t)g * q.cg * it.ldc;
+            it.k_d = q.M[0][e0]; it.k_r = q.M[1][e1]; it.k_c = q.M[2][e2];
+            it.Wo = q.n[2][e2]; it.HoWo = q.n[1][e1] * q.n[2][e2];
+            it.first = (int)(start + per_group * g); it.tiles_n = tiles_n;
+            it.div_wo = make_fastdiv((uint32_t)it.Wo); it.div_howo = make_fastdiv((uint32_t)it.HoWo);
+            items[i] = it;
+            break;
+        }
     }
 }
 
-hipError_t launch_phase_weights(int64_t es, const void* w, void* wt, int64_t groups, int64_t og, int64_t ogp, int64_t cg, int64_t k_r, int64_t k_c,
-                                int64_t er, int64_t ec, int64_t s_r, int64_t s_c, int64_t Mr, int64_t Mc, hipStream_t s) {
-    const PhaseWeights q{groups, og, ogp, cg, k_r, k_c, er, ec, s_r, s_c, Mr, Mc};
-    const int64_t total = groups * cg * Mr * Mc * ogp;
-    if (total == 0) return hipSuccess;
+hipError_t launch_phase_setup(int64_t es, const void* w, void* wt, RingItem* items, const PhaseLayout& q, hipStream_t s) {
+    const int64_t total = (int64_t)q.groups * q.cg * q.k[0] * q.k[1] * q.k[2] * q.ogp;
     const dim3 g(grid_for(total)), t(256);
     switch (es) {
-    case 2: hipLaunchKernelGGL(phase_weights_kernel<uint16_t>, g, t, 0, s, (const uint16_t*)w, (uint16_t*)wt, q); break;
-    case 4: hipLaunchKernelGGL(phase_weights_kernel<uint32_t>, g, t, 0, s, (const uint32_t*)w, (uint32_t*)wt, q); break;
+    case 2: hipLaunchKernelGGL(phase_setup_kernel<uint16_t>, g, t, 0, s, (const uint16_t*)w, (uint16_t*)wt, items, q); break;
+    case 4: hipLaunchKernelGGL(phase_setup_kernel<uint32_t>, g, t, 0, s, (const uint32_t*)w, (uint32_t*)wt, items, q); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
 
-// im[b][c][y][x] (+)= the element of the phase plane that holds it: phase (er, ec) = ((y + p_r) % s_r, (x + p_c) % s_c)
-// stores the image rows y = s_r (a0 + a) + er - p_r as its rows a (columns likewise); phases without taps contribute zero.
-template <class T, class Acc>
-__global__ void __launch_bounds__(256) phase_interleave_kernel(const T* __restrict__ tmp, T* __restrict__ im, const PhaseLayout q, const int accumulate) {
+// im[b][c][z][y][x] (+)= the element of the phase plane that holds it: phase e = (position + p) % s per axis stores the image
+// positions s (a0 + a) + e - p as its positions a; phases without taps contribute zero.  A thread does V consecutive elements of
+// an image row (16 bytes in one store where the rows allow it): the divisions are made once per row piece and the column phase
+// advances by counting -- one element per thread with all its divisions took 19.8 us where this takes the time of the memory
+// traffic (Float16 32 x 64 x 56 x 56).
+template <class T, int V, bool STORE16>
+__global__ void __launch_bounds__(256) phase_interleave_kernel(const T* __restrict__ tmp, T* __restrict__ im, const PhaseLayout q, const uint32_t total,
+                                                               const FastDiv div_pieces, const int accumulate) {
     const uint32_t idx = blockIdx.x * 256u + threadIdx.x;
-    if (idx >= q.total) return;
-    const uint32_t t = fast_div(idx, q.div_w), x = idx - t * (uint32_t)q.W;
-    const uint32_t bc = fast_div(t, q.div_h), y = t - bc * (uint32_t)q.H;
-    const uint32_t Y = y + (uint32_t)q.p_r, X = x + (uint32_t)q.p_c;
-    const uint32_t ar = fast_div(Y, q.div_sr), er = Y - ar * (uint32_t)q.s_r;
-    const uint32_t ac = fast_div(X, q.div_sc), ec = X - ac * (uint32_t)q.s_c;
-    Acc v = accumulate ? (Acc)im[idx] : (Acc)0;
-    const int ph = (int)(er * (uint32_t)q.s_c + ec);
-    if (q.off[ph] >= 0) {
-        const int a = (int)ar - q.a0r[er], b = (int)ac - q.a0c[ec];      // inside the plane by construction
-        v += (Acc)tmp[q.off[ph] + ((int64_t)bc * q.hp[er] + a) * q.wp[ec] + b];
+    if (idx >= total) return;
+    const uint32_t pieces = (uint32_t)(q.sz[2] + V - 1) / V;
+    const uint32_t row = fast_div(idx, div_pieces), x0 = (idx - row * pieces) * V;
+    const uint32_t t1 = fast_div(row, q.div_rows[1]), y = row - t1 * (uint32_t)q.sz[1];
+    const uint32_t bc = fast_div(t1, q.div_rows[0]), z = t1 - bc * (uint32_t)q.sz[0];
+    const uint32_t Z = z + (uint32_t)q.p[0], Y = y + (uint32_t)q.p[1], X = x0 + (uint32_t)q.p[2];
+    const uint32_t az = fast_div(Z, q.div_s[0]), ez = Z - az * (uint32_t)q.s[0];
+    const uint32_t ay = fast_div(Y, q.div_s[1]), ey = Y - ay * (uint32_t)q.s[1];
+    uint32_t ax = fast_div(X, q.div_s[2]), ex = X - ax * (uint32_t)q.s[2];
+    const int rz = (int)az - q.a0[0][ez], ry = (int)ay - q.a0[1][ey];
+    const int rphase = (int)((ez * (uint32_t)q.s[1] + ey) * (uint32_t)q.s[2]);
+    constexpr int64_t none = -(1LL << 62);
+    // (the row's place in the planes of each column phase)
+    int64_t rowoff[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        rowoff[e] = e < q.s[2] && q.plane_off[rphase + e] >= 0
+                  ? q.plane_off[rphase + e] + (int64_t)bc * phase_plane(q, (int)ez, (int)ey, e) + ((int64_t)rz * q.n[1][ey] + ry) * q.n[2][e] - q.a0[2][e] : none;
+    T* dst = im + (int64_t)row * q.sz[2] + x0;
+    T v[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        const int64_t o = ex == 0u ? rowoff[0] : ex == 1u ? rowoff[1] : ex == 2u ? rowoff[2] : rowoff[3];
+        const bool ok = (int)x0 + i < q.sz[2];
+        float f = ok && o != none ? (float)tmp[o + ax] : 0.0f;
+        if (accumulate && ok) f += (float)dst[i];
+        v[i] = (T)f;
+        if (++ex == (uint32_t)q.s[2]) { ex = 0u; ++ax; }
     }
-    im[idx] = (T)v;
+    if constexpr (STORE16) {
+        typedef T TV __attribute__((ext_vector_type(V)));
+        TV o;
+#pragma unroll
+        for (int i = 0; i < V; ++i) o[i] = v[i];
+        *reinterpret_cast<TV*>(dst) = o;
+    } else {
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+            if ((int)x0 + i < q.sz[2]) dst[i] = v[i];
+    }
 }
 
+template <class T>
+static hipError_t launch_phase_interleave_t(const void* tmp, void* im, const PhaseLayout& q, int accumulate, hipStream_t s) {
+    constexpr int V16 = 16 / (int)sizeof(T), V = 4;
+    const int64_t rows = (int64_t)q.batch * q.groups * q.cg * q.sz[0] * q.sz[1];
+    const bool vec = q.sz[2] % V16 == 0 && (reinterpret_cast<uintptr_t>(im) & 15) == 0;
+    const int64_t pieces = vec ? q.sz[2] / V16 : (q.sz[2] + V - 1) / V, total = rows * pieces;
+    if (total == 0) return hipSuccess;
+    if (total >= 0x7fffffffLL) return hipErrorInvalidValue;
+    const dim3 g((unsigned)((total + 255) / 256)), t(256);
+    const FastDiv dp = make_fastdiv((uint32_t)pieces);
+    if (vec) hipLaunchKernelGGL((phase_interleave_kernel<T, V16, true>), g, t, 0, s, (const T*)tmp, (T*)im, q, (uint32_t)total, dp, accumulate);
+    else hipLaunchKernelGGL((phase_interleave_kernel<T, V, false>), g, t, 0, s, (const T*)tmp, (T*)im, q, (uint32_t)total, dp, accumulate);
+    return hipGetLastError();
+}
 hipError_t launch_phase_interleave(int dtype, const void* tmp, void* im, const PhaseLayout& q, int accumulate, hipStream_t s) {
-    if (q.total == 0) return hipSuccess;
-    const dim3 g((q.total + 255u) / 256u), t(256);
     switch (dtype) {
-    case DT_F32: hipLaunchKernelGGL((phase_interleave_kernel<float, float>), g, t, 0, s, (const float*)tmp, (float*)im, q, accumulate); break;
-    case DT_F16: hipLaunchKernelGGL((phase_interleave_kernel<_Float16, float>), g, t, 0, s, (const _Float16*)tmp, (_Float16*)im, q, accumulate); break;
-    case DT_BF16: hipLaunchKernelGGL((phase_interleave_kernel<__bf16, float>), g, t, 0, s, (const __bf16*)tmp, (__bf16*)im, q, accumulate); break;
+    case DT_F32: return launch_phase_interleave_t<float>(tmp, im, q, accumulate, s);
+    case DT_F16: return launch_phase_interleave_t<_Float16>(tmp, im, q, accumulate, s);
+    case DT_BF16: return launch_phase_interleave_t<__bf16>(tmp, im, q, accumulate, s);
     default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
 
 // wp[o][t][c] = w[o][c][t]: convolution weights with the channel index fastest (the k order of the channels-last gather),

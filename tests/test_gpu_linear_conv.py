@@ -823,6 +823,12 @@ def test_conv2d_backward_fp32_host_entry_is_the_reference_bit_for_bit(geom):
     (1, 24, (33, 40), 64, (5, 3), (2, 1), (2, 1), 1, 1),              # one image, channels that end inside a 64-byte run
     (9, 3, (70, 66), 16, (7, 7), 2, 3, 1, 1),                         # three channels, more output pixels than the window table holds
     (3, 32, (1, 1), 32, (1, 1), 2, 0, 1, 1),                          # one output pixel per image
+    # image gradients by phases of the strides, all in one launch:
+    (2, 32, (12, 15), 32, (2, 2), 2, 1, 1, 1),                        # a window that begins behind the first output (padding beyond the taps)
+    (2, 32, (11, 9), 64, (1, 2), (3, 4), 0, 1, 2),                    # phases without taps, groups, odd rows
+    (3, 16, (17, 16), 40, (5, 3), (4, 1), (2, 1), 1, 1),              # a stride along one axis, out channels that end inside a 64-byte run
+    (2, 32, (7, 6, 9), 32, (3, 2, 4), 2, (1, 0, 1), 1, 1),            # three axes, eight phases of unequal sizes
+    (1, 64, (5, 9, 8), 64, (1, 3, 3), (1, 2, 2), (0, 1, 1), 1, 2),
 ], ids=lambda g: "x".join(map(str, g)))
 def test_channels_last_convolutions_over_two_and_three_axes(geom, dtype):
     """Forward, image gradient and weight gradient (k ranges through all images) on the channels-last kernels at the edges of
