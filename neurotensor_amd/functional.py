@@ -29,7 +29,8 @@ def ntg_dtype(t):
 
 
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current stream's handle (torch.cuda.current_stream() builds a Stream object first: 2.9 us of an 11 us call)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _require_device(*ts):
@@ -64,23 +65,19 @@ def _logical(a_shape, b_shape, ta, tb):
 def _launch(a, b, c, m, k, n, ta, tb, batches, sa, sb, sc, c_mode, bias=None, bias_strides=(0, 0, 0),
             a_off=0, b_off=0, c_off=0, bias_off=0, relu=False):
     es = a.element_size()
-    d = GemmDesc()
-    d.dtype = ntg_dtype(a)
-    d.transpose_a, d.transpose_b, d.c_mode = int(ta), int(tb), c_mode
-    d.m, d.k, d.n = m, k, n
-    d.batches = batches
-    d.stride_a, d.stride_b, d.stride_c = sa, sb, sc
-    if bias is not None:
-        d.bias = bias.data_ptr() + bias_off * es
-        d.bias_batch_stride, d.bias_row_stride, d.bias_col_stride = bias_strides
+    # (in the order of the structure's fields: one call instead of an attribute store each)
+    d = GemmDesc(ntg_dtype(a), ta, tb, c_mode, m, k, n, 0, 0, 0, batches, sa, sb, sc,
+                 None if bias is None else bias.data_ptr() + bias_off * es, *bias_strides)
+    ref = ctypes.byref(d)
     L = load()
-    ws_bytes = L.ntg_gemm_workspace_bytes(ctypes.byref(d))      # > 0: few output tiles, deep k -> split along k
-    ws = None
+    ws_bytes = L.ntg_gemm_workspace_bytes(ref)      # > 0: few output tiles, deep k -> split along k
     if ws_bytes > 0:
         ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=a.device)
         d.workspace, d.workspace_bytes = ws.data_ptr(), ws_bytes
-    entry = L.ntg_gemm_relu_dev if relu else L.ntg_gemm_dev
-    check(entry(ctypes.byref(d), a.data_ptr() + a_off * es, b.data_ptr() + b_off * es, c.data_ptr() + c_off * es, _stream()))
+    status = (L.ntg_gemm_relu_dev if relu else L.ntg_gemm_dev)(ref, a.data_ptr() + a_off * es, b.data_ptr() + b_off * es, c.data_ptr() + c_off * es,
+                                                               _stream())
+    if status:
+        check(status)
 
 
 def matmult(a, b, out=None, transpose_a=False, transpose_b=False, accumulate=None):
@@ -94,6 +91,15 @@ def matmult(a, b, out=None, transpose_a=False, transpose_b=False, accumulate=Non
         raise ValueError(f"Expected tensors to have dims greater than 1, but instead had dims of {a.dim()} and {b.dim()}")
     if a.dtype != b.dtype:
         raise ValueError(f"Expected both tensors to have the same dtype but got {a.dtype} and {b.dtype}")   # :868
+    if out is None and a.dim() == 2 and b.dim() == 2:
+        # two matrices: what the rules below come down to, without their bookkeeping
+        a_st, ta = _as_matrix_view(a, bool(transpose_a))
+        b_st, tb = _as_matrix_view(b, bool(transpose_b))
+        m, k, n = _logical(a_st.shape, b_st.shape, ta, tb)
+        c = torch.empty((m, n), dtype=a.dtype, device=a.device)
+        if m and n:
+            _launch(a_st, b_st, c, m, k, n, ta, tb, 1, m * k, k * n, m * n, _lib.C_OVERWRITE)
+        return c
     a_st, ta = _as_matrix_view(a, bool(transpose_a))
     b_st, tb = _as_matrix_view(b, bool(transpose_b))
     m, k, n = _logical(a_st.shape, b_st.shape, ta, tb)
@@ -184,6 +190,15 @@ def linear(x, w, bias, transpose_a=False, transpose_b=False, _relu=False):
     def unsq(t):      # unsqueeze_as, matmult_cpu.cpp:1712-1713
         return t.reshape((1,) * (nd - t.dim()) + tuple(t.shape))
 
+    if x.dim() == 2 and w.dim() == 2 and bias.dim() == 1:
+        # a layer's own call: one bias row for a matrix (what the rules below come down to)
+        x_st, ta = _as_matrix_view(x, bool(transpose_a))
+        w_st, tb = _as_matrix_view(w, bool(transpose_b))
+        m, k, n = _logical(x_st.shape, w_st.shape, ta, tb)
+        if bias.shape[0] == n and m and n:
+            out = torch.empty((m, n), dtype=x.dtype, device=x.device)
+            _launch(x_st, w_st, out, m, k, n, ta, tb, 1, m * k, k * n, m * n, _lib.C_BIAS, bias=bias.contiguous(), bias_strides=(0, 0, 1), relu=_relu)
+            return out
     x, w, bias = unsq(x), unsq(w), unsq(bias)
     x_st, ta = _as_matrix_view(x, bool(transpose_a))
     w_st, tb = _as_matrix_view(w, bool(transpose_b))
