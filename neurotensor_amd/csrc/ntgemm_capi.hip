@@ -1584,7 +1584,11 @@ static int conv_dimage_phases(int dtype, const PhasePlan& pp, const void* kernel
 static int64_t dkernel_padded_channels(int64_t es, int64_t cg) { const int64_t v = 16 / es; return (cg + v - 1) / v * v; }
 static HaloPlan dkernel_halo(int64_t es, int64_t cg, int64_t groups, const Geo3& g) {
     HaloPlan h = conv_halo(g);
-    if (h.on && !conv_nhwc_offsets_fit(groups * dkernel_padded_channels(es, cg), es, h.gp)) {
+    const int64_t cgp = dkernel_padded_channels(es, cg);
+    // (a copy that pads the channels grows by its border as well: on one and two axes only where that is a quarter of it at most, as
+    //  it is from 17 x 17 pixels on for a 3 x 3 window; smaller planes keep the validity tests and their workspace)
+    const bool wide_border = g.nd < 3 && cgp != cg && 4 * h.vol > 5 * g.vol();
+    if (h.on && (wide_border || !conv_nhwc_offsets_fit(groups * cgp, es, h.gp))) {
         h.on = false; h.gp = g; h.vol = g.vol();
     }
     return h;
