@@ -405,8 +405,15 @@ hipError_t launch_reduce_batch_taps_last(int dtype, bool part_f32, const void* p
 hipError_t launch_flip_weights(int64_t elem_size, const void* w, void* wt, int64_t groups, int64_t og, int64_t cg, int64_t taps, hipStream_t s);
 
 // padded copies of operands whose rows are not 16-byte multiples (pad_copy.hip); es = 1, 2, 4 or 8 bytes per element, sizes in elements
-hipError_t launch_pad_copy(int64_t es, const void* src, int64_t ld_src, int64_t s_src, void* dst, int64_t ld_dst, int64_t s_dst,
-                           int64_t rows, int64_t cols, int64_t rows_dst, int64_t batch, hipStream_t s);
+// The copies of one product into rows padded with zeros (pad_copies_kernel); first, row_blocks and sh are the launcher's.
+struct PadJob {
+    const void* src; int64_t ld_src, s_src;
+    void* dst; int64_t ld_dst, s_dst;
+    int64_t rows, cols, rows_dst, batch;
+    uint32_t first, row_blocks; int sh;
+};
+struct PadJobs { PadJob job[3]; int n; };
+hipError_t launch_pad_copies(int64_t es, PadJobs jobs, hipStream_t s);
 hipError_t launch_unpad_copy(int64_t es, const void* src, int64_t ld_src, int64_t s_src, void* dst, int64_t ld_dst, int64_t s_dst,
                              int64_t rows, int64_t cols, int64_t batch, hipStream_t s);
 hipError_t launch_bias_fill(int64_t es, const void* bias, int64_t bs, int64_t rs, int64_t cs, void* dst, int64_t ld_dst, int64_t s_dst,

@@ -356,34 +356,37 @@ static int run_padded(const ntg::GemmParams& p, const PadPlan& pl, int dtype, bo
     ntg::GemmParams q = p;
     q.M = pl.Mp; q.K = pl.Kp; q.N = pl.Np;
     hipError_t e;
+    ntg::PadJobs jobs;
+    std::memset(&jobs, 0, sizeof jobs);
+    const int64_t itemsA = p.sA == 0 ? 1 : p.batch, itemsB = p.sB == 0 ? 1 : p.batch;
+    auto copy = [&](const void* src, int64_t ld_src, int64_t s_src, void* dst, int64_t ld_dst, int64_t rows, int64_t cols, int64_t rows_dst, int64_t items) {
+        ntg::PadJob& j = jobs.job[jobs.n++];
+        j.src = src; j.ld_src = ld_src; j.s_src = s_src;
+        j.dst = dst; j.ld_dst = ld_dst; j.s_dst = rows_dst * ld_dst;
+        j.rows = rows; j.cols = cols; j.rows_dst = rows_dst; j.batch = items;
+    };
     if (pl.padA) {
-        e = ntg::launch_pad_copy(es, p.A, p.lda, p.sA, a2, pl.lda2, pl.rowsA2 * pl.lda2, ta ? p.K : p.M, ta ? p.M : p.K, pl.rowsA2, p.sA == 0 ? 1 : p.batch, s);
-        if (e != hipSuccess) return hip_fail(e, "padded copy of A");
+        copy(p.A, p.lda, p.sA, a2, pl.lda2, ta ? p.K : p.M, ta ? p.M : p.K, pl.rowsA2, itemsA);
         q.A = a2; q.lda = pl.lda2; q.sA = p.sA == 0 ? 0 : pl.rowsA2 * pl.lda2;
-    }
-    if (pl.padB) {
-        e = ntg::launch_pad_copy(es, p.B, p.ldb, p.sB, b2, pl.ldb2, pl.rowsB2 * pl.ldb2, tb ? p.N : p.K, tb ? p.K : p.N, pl.rowsB2, p.sB == 0 ? 1 : p.batch, s);
-        if (e != hipSuccess) return hip_fail(e, "padded copy of B");
-        q.B = b2; q.ldb = pl.ldb2; q.sB = p.sB == 0 ? 0 : pl.rowsB2 * pl.ldb2;
-    }
-    if (pl.stripA) {
-        e = ntg::launch_pad_copy(es, static_cast<const char*>(p.A) + (int64_t)pl.strip_k0 * p.lda * es, p.lda, p.sA, a2, p.lda, (int64_t)pl.strip_rows * p.lda,
-                                 p.K - pl.strip_k0, p.M, pl.strip_rows, p.sA == 0 ? 1 : p.batch, s);
-        if (e != hipSuccess) return hip_fail(e, "copy of A's last k-rows");
+    } else if (pl.stripA) {
+        copy(static_cast<const char*>(p.A) + (int64_t)pl.strip_k0 * p.lda * es, p.lda, p.sA, a2, p.lda, p.K - pl.strip_k0, p.M, pl.strip_rows, itemsA);
         q.tailA = a2; q.s_tailA = p.sA == 0 ? 0 : (int64_t)pl.strip_rows * p.lda; q.tail_k0 = pl.strip_k0;
     }
-    if (pl.stripB) {
-        e = ntg::launch_pad_copy(es, static_cast<const char*>(p.B) + (int64_t)pl.strip_k0 * p.ldb * es, p.ldb, p.sB, b2, p.ldb, (int64_t)pl.strip_rows * p.ldb,
-                                 p.K - pl.strip_k0, p.N, pl.strip_rows, p.sB == 0 ? 1 : p.batch, s);
-        if (e != hipSuccess) return hip_fail(e, "copy of B's last k-rows");
+    if (pl.padB) {
+        copy(p.B, p.ldb, p.sB, b2, pl.ldb2, tb ? p.N : p.K, tb ? p.K : p.N, pl.rowsB2, itemsB);
+        q.B = b2; q.ldb = pl.ldb2; q.sB = p.sB == 0 ? 0 : pl.rowsB2 * pl.ldb2;
+    } else if (pl.stripB) {
+        copy(static_cast<const char*>(p.B) + (int64_t)pl.strip_k0 * p.ldb * es, p.ldb, p.sB, b2, p.ldb, p.K - pl.strip_k0, p.N, pl.strip_rows, itemsB);
         q.tailB = b2; q.s_tailB = p.sB == 0 ? 0 : (int64_t)pl.strip_rows * p.ldb; q.tail_k0 = pl.strip_k0;
+    }
+    if (pl.padC && p.cmode == ntg::C_ACCUMULATE) copy(p.C, p.ldc, p.sC, c2, pl.Np, p.M, p.N, pl.Mp, p.batch);
+    if (jobs.n) {
+        e = ntg::launch_pad_copies(es, jobs, s);
+        if (e != hipSuccess) return hip_fail(e, "padded copies");
     }
     if (pl.padC) {
         const int64_t sc2 = (int64_t)pl.Mp * pl.Np;
-        if (p.cmode == ntg::C_ACCUMULATE) {
-            e = ntg::launch_pad_copy(es, p.C, p.ldc, p.sC, c2, pl.Np, sc2, p.M, p.N, pl.Mp, p.batch, s);
-            if (e != hipSuccess) return hip_fail(e, "padded copy of C");
-        } else if (p.cmode == ntg::C_BIAS) {
+        if (p.cmode == ntg::C_BIAS) {
             // the bias becomes the initial accumulator in the padded layout (reading it at padded indices would leave its array)
             e = ntg::launch_bias_fill(es, p.bias, p.bias_bs, p.bias_rs, p.bias_cs, c2, pl.Np, sc2, p.M, p.N, pl.Mp, p.batch, s);
             if (e != hipSuccess) return hip_fail(e, "bias fill");

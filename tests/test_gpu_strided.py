@@ -223,6 +223,18 @@ def test_rows_that_are_not_16_byte_multiples_through_padded_copies(name):
             run_case(rng, name, 2320, 1001, 2056, True, False, (0, 0, 0), _lib.C_OVERWRITE, workspace=True, one_rounding=True)
             run_case(rng, name, 264, 1001, 2304, False, False, (0, 0, 0), _lib.C_ACCUMULATE, batches=33, workspace=True, one_rounding=True)
 
+
+@pytest.mark.parametrize("name,m,k,n", [("bf16", 264, 4097, 2001), ("i8", 40, 8193, 1003), ("f32", 700, 4097, 1501)])
+def test_padded_copies_of_one_launch_with_rows_of_several_pieces(name, m, k, n):
+    """A, B and the C that is added to are jobs of one copy launch: rows of more than 256 chunks (several pieces) beside shorter ones,
+    no job a whole number of blocks, and the operands in both orders."""
+    rng = np.random.default_rng(8150 + k)
+    half = name == "bf16"
+    run_case(rng, name, m, k, n, False, True, (0, 0, 0), _lib.C_ACCUMULATE, workspace=True, one_rounding=half)
+    run_case(rng, name, m, k, n, True, False, ODD, _lib.C_ACCUMULATE, base=1, workspace=True, one_rounding=half)
+    run_case(rng, name, m, k, n, False, False, (3, 5, 0), _lib.C_ACCUMULATE, batches=2, gap=1, bcast_b=True, workspace=True, one_rounding=half)
+
+
 def _random_dim(rng, hi):
     """sizes that sit on, just below and just above the tile edges, tiny ones, multiples of 8 and anything else"""
     kind = int(rng.integers(0, 4))
