@@ -1788,7 +1788,7 @@ static int conv_dkernel_from_col(int dtype, const char* gy, char* col, void* d_k
 }
 
 // Which backward gradients run as implicit GEMMs, and the workspace the call needs.
-struct ConvBackwardPlan { bool gather_dw, gather_dx, nhwc_dx, nhwc_dw, phase_dx; int64_t need, need_nhwc_dx, need_nhwc_dw, need_phase_dx; PhasePlan phases; DkernelPlan dkernel; };
+struct ConvBackwardPlan { bool gather_dw, gather_dx, nhwc_dx, nhwc_dw, phase_dx; int64_t need, need_nhwc_dx, need_nhwc_dw, need_phase_dx, need_wt_dx, wt_offset; PhasePlan phases; DkernelPlan dkernel; };
 // reference_order (Float32 through the host entry points): the forms whose sums are the reference's own, bit for bit -- the
 // image gradient as W^T . dY into the col matrix + col2im (conv.cpp:318-346; the implicit forms run one chain over out
 // channels and taps where the reference rounds in between), the weight gradient per image with k = the output pixels +
@@ -1818,6 +1818,16 @@ static ConvBackwardPlan plan_conv_backward_g(int dtype, bool want_dx, bool want_
         pl.phases = plan_dimage_phases(dtype, batch, channels, out_channels, groups, g);
     pl.phase_dx = pl.phases.ok;
     pl.need_phase_dx = pl.phase_dx ? pl.phases.bytes() : 0;
+    // strides > 1 on few channels: W^T . dY + col2im.  W_g is stored [og][channels of the group * taps]; where those rows miss the
+    // 16-byte rule (3 channels by 7 x 7: 147) the product would go to the register-staged kernel, so W is copied to [..][og] behind the col matrix
+    // and dY and col, whose rows keep the rule, stay where they are.  Float32 32 x 3 x 224 x 224 from 7 x 7 at stride 2, 64 out channels
+    // (3.8 * 10^9 multiply-adds, 236 MB written): 203 us there, 152 us here and 9 us for the copy -- the two meet at 0.65 * 10^9: from 2^30 on.
+    pl.wt_offset = (int64_t)align_up((size_t)col, 256);
+    const int64_t og = out_channels / groups, add = cg * taps;
+    const bool wt = want_dx && !pl.gather_dx && !pl.phase_dx && !reference_order && g.nd <= 2 &&
+                    (dtype == ntg::DT_F32 || dtype == ntg::DT_F16 || dtype == ntg::DT_BF16) && add > 32 && (add * es) % 16 != 0 && (og * es) % 16 == 0 &&
+                    (g.L() * es) % 16 == 0 && (double)batch * (double)(og * add) * (double)g.L() >= 1073741824.0;
+    pl.need_wt_dx = wt ? pl.wt_offset + groups * og * add * es : 0;
     return pl;
 }
 
@@ -2011,7 +2021,7 @@ int64_t ntg_conv2d_backward_workspace_bytes(int dtype, int64_t batch, int64_t ch
     // the larger of what the call needs at least and what lets dX take its channels-last form (copy of dY + flipped weights)
     const ConvBackwardPlan pl = plan_conv_backward(dtype, true, true, batch, channels, height, width, out_channels, k_r, k_c, s_r, s_c, p_r, p_c,
                                                    d_r, d_c, groups, Ho, Wo);
-    return std::max(std::max(pl.need, pl.need_phase_dx), std::max(pl.need_nhwc_dx, pl.need_nhwc_dw));
+    return std::max(std::max(std::max(pl.need, pl.need_phase_dx), pl.need_wt_dx), std::max(pl.need_nhwc_dx, pl.need_nhwc_dw));
 }
 
 static int conv2d_backward_dev_impl(int dtype, const void* image, const void* kernel, const void* grad_out,
@@ -2103,14 +2113,20 @@ static int conv2d_backward_dev_impl(int dtype, const void* image, const void* ke
         if (rc) return rc;
     }
     if (d_image) {
-        // d_col_{b,g} [add, L] = W_g^T . dY_{b,g}   (W_g stored [og, add] -> transpose_a), then col2im
+        // d_col_{b,g} [add, L] = W_g^T . dY_{b,g}   (W_g stored [og, add] -> transpose_a, or its copy [add, og]), then col2im
+        const bool wt = plan.need_wt_dx > 0 && workspace_bytes >= plan.need_wt_dx &&
+                        ((reinterpret_cast<uintptr_t>(ws) | reinterpret_cast<uintptr_t>(grad_out)) & 15) == 0;
+        if (wt) {
+            hipError_t e = ntg::launch_nchw_to_nhwc(es, kern, ws + plan.wt_offset, groups, og, add, hs);
+            if (e != hipSuccess) return hip_fail(e, "transposed weights launch");
+        }
         for (int64_t g = 0; g < groups; ++g) {
             std::memset(&d, 0, sizeof d);
-            d.dtype = dtype; d.transpose_a = 1; d.c_mode = NTG_C_OVERWRITE;
+            d.dtype = dtype; d.transpose_a = wt ? 0 : 1; d.c_mode = NTG_C_OVERWRITE;
             d.m = add; d.k = og; d.n = L;
-            d.lda = add; d.ldb = L; d.ldc = L; d.batches = batch;
+            d.lda = wt ? og : add; d.ldb = L; d.ldc = L; d.batches = batch;
             d.stride_a = 0; d.stride_b = out_channels * L; d.stride_c = ckk * L;
-            rc = ntg_gemm_dev(&d, kern + g * og * add * es, gy + g * og * L * es, ws + g * add * L * es, stream);
+            rc = ntg_gemm_dev(&d, (wt ? ws + plan.wt_offset : kern) + g * og * add * es, gy + g * og * L * es, ws + g * add * L * es, stream);
             if (rc) return rc;
         }
         rc = ntg_unfold2d_backward_dev(dtype, ws, d_image, batch, channels, height, width, k_r, k_c, s_r, s_c, p_r, p_c, d_r, d_c,

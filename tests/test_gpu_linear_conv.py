@@ -858,3 +858,31 @@ def test_channels_last_convolutions_over_two_and_three_axes(geom, dtype):
         else:
             bound = HALF_REL * max(want.abs().max().item(), 1e-3)
         assert (got - want).abs().max().item() <= bound, (name, (got - want).abs().max().item(), bound)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("geom", [
+    # (B, C, size, O, kernel, stride, padding, dilation, groups)
+    (18, 3, (159, 160), 64, (7, 7), 2, 3, 1, 1),                      # 147 weights per out channel, every fourth column a remainder of the tap loop
+    (26, 6, (160, 159), 128, (5, 7), (2, 2), (2, 3), 1, 2),           # groups: 105 weights each
+    (4, 3, (192, 250), 72, (9, 11), (1, 3), (4, 5), 1, 1),            # a stride along one axis, rows of up to 4 taps
+    (18, 3, (160, 160), 64, (7, 7), 2, 6, 2, 1),                      # dilated: a test per tap
+], ids=lambda g: "x".join(map(str, g)))
+def test_strided_image_gradient_on_few_channels_through_the_transposed_weights(geom, dtype):
+    """W^T . dY with W copied to rows that keep the 16-byte rule, then col2im, against float64 on the CPU: the bounds of the
+    channels-last convolutions above (a 16-bit col entry is rounded once, and at most 44 of them are added in Float32)."""
+    B, C, size, O, k, s, p, d, groups = geom
+    rng = np.random.default_rng(17 + O + sum(size))
+    x = torch.from_numpy(rng.standard_normal((B, C) + size)).to(dtype)
+    w = torch.from_numpy(rng.standard_normal((O, C // groups) + k)).to(dtype)
+    rx = x.double().requires_grad_(True)
+    ry = torch.nn.functional.conv2d(rx, w.double(), None, s, p, d, groups)
+    g = torch.from_numpy(rng.standard_normal(tuple(ry.shape))).to(dtype)
+    want, = torch.autograd.grad(ry, rx, g.double())
+    dx, _ = F.conv2d_backward(x.to(DEV), w.to(DEV), g.to(DEV), stride=s, padding=p, dilation=d, groups=groups)
+    got = dx.double().cpu()
+    if dtype == torch.float32:
+        bound = 1e-6 * (O // groups * int(np.prod(k))) ** 0.5 * want.square().mean().sqrt().item()
+    else:
+        bound = HALF_REL * want.abs().max().item()
+    assert got.shape == want.shape and (got - want).abs().max().item() <= bound, ((got - want).abs().max().item(), bound)
