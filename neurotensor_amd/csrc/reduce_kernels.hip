@@ -542,18 +542,22 @@ hipError_t launch_flip_weights_channels_last(int64_t es, const void* w, void* wt
 // Weights of all phases of a strided convolution's image gradient, and the table of their products.  Phase e has the taps
 // e + s (M - 1 - m) of w [g*og + oc][c][taps], reversed, as wt[g][c][(run, m0, m1, m2, oc in run)] with the out channels padded with
 // zeros from og to ogp and in runs of `chunk` (see ConvGeom::tap_inner).  One thread per (group, image channel, tap, out channel):
-// every tap belongs to one phase.  The first threads write the table.
-template <class T>
-__global__ void __launch_bounds__(256) phase_setup_kernel(const T* __restrict__ w, T* __restrict__ wt, RingItem* __restrict__ items, const PhaseLayout q) {
+// every tap belongs to one phase.  The table, one thread an item, is the work of the blocks behind those of the weights: an item is a
+// walk over the phases and four 64-bit divisions, which behind a weight of its own was the kernel's whole length; index arithmetic in
+// 32 bits (I) where the weights allow it, as a 64-bit division is some hundred instructions and a weight takes three
+// (Float16 128 x 64 x 4 x 4 at stride 2: 9.5 -> 8.2 us, the rest the latency of its strided reads).
+template <class T, class I>
+__global__ void __launch_bounds__(256) phase_setup_kernel(const T* __restrict__ w, T* __restrict__ wt, RingItem* __restrict__ items, const PhaseLayout q,
+                                                          const uint32_t weight_blocks) {
     const int taps = q.k[0] * q.k[1] * q.k[2];
     const int64_t total = (int64_t)q.groups * q.cg * taps * q.ogp;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x, first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    for (int64_t idx = first; idx < total; idx += stride) {
-        const int oc = (int)(idx % q.ogp);
-        int64_t r = idx / q.ogp;
-        int tap = (int)(r % taps);
+    const int64_t stride = (int64_t)weight_blocks * 256;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; blockIdx.x < weight_blocks && i < total; i += stride) {
+        const I idx = (I)i, row = idx / (I)q.ogp, gc = row / (I)taps;
+        const int oc = (int)(idx - row * (I)q.ogp);
+        int tap = (int)(row - gc * (I)taps);
         const int src_tap = tap;
-        r /= taps;                                                     // g * cg + c
+        const int64_t r = (int64_t)gc;                                 // g * cg + c
         int e[3], m[3];
 #pragma unroll
         for (int a = 2; a >= 0; --a) {
@@ -565,12 +569,14 @@ __global__ void __launch_bounds__(256) phase_setup_kernel(const T* __restrict__ 
         const int ph = (e[0] * q.s[1] + e[1]) * q.s[2] + e[2];
         if (q.plane_off[ph] < 0) continue;
         const int ptaps = q.M[0][e[0]] * q.M[1][e[1]] * q.M[2][e[2]], t = (m[0] * q.M[1][e[1]] + m[1]) * q.M[2][e[2]] + m[2];
-        const int64_t g = r / q.cg, c = r - g * q.cg;
+        const int64_t g = (int64_t)(gc / (I)q.cg), c = r - g * q.cg;
         wt[q.w_off[ph] + r * ptaps * q.ogp + ((int64_t)(oc / q.chunk) * ptaps + t) * q.chunk + oc % q.chunk] =
             oc < q.og ? w[((g * q.og + oc) * q.cg + c) * taps + src_tap] : (T)0;
     }
     // item (live phase, group)
-    for (int64_t i = first; i < (int64_t)q.phases * q.groups; i += stride) {
+    if (blockIdx.x < weight_blocks) return;
+    const int64_t i = (int64_t)(blockIdx.x - weight_blocks) * 256 + threadIdx.x;
+    if (i < (int64_t)q.phases * q.groups) {
         const int want = (int)(i / q.groups), g = (int)(i % q.groups);
         const int tiles_m = (q.cg + q.tile_rows - 1) / q.tile_rows;
         int64_t start = 0;
@@ -599,10 +605,20 @@ __global__ void __launch_bounds__(256) phase_setup_kernel(const T* __restrict__ 
 
 hipError_t launch_phase_setup(int64_t es, const void* w, void* wt, RingItem* items, const PhaseLayout& q, hipStream_t s) {
     const int64_t total = (int64_t)q.groups * q.cg * q.k[0] * q.k[1] * q.k[2] * q.ogp;
-    const dim3 g(grid_for(total)), t(256);
+    const uint32_t wb = (uint32_t)grid_for(total);
+    const int64_t ib = ((int64_t)q.phases * q.groups + 255) / 256;
+    if (ib > 0x3fffffffLL) return hipErrorInvalidValue;
+    const dim3 g(wb + (uint32_t)ib), t(256);
+    const bool narrow = total <= 0x7fffffffLL;
     switch (es) {
-    case 2: hipLaunchKernelGGL(phase_setup_kernel<uint16_t>, g, t, 0, s, (const uint16_t*)w, (uint16_t*)wt, items, q); break;
-    case 4: hipLaunchKernelGGL(phase_setup_kernel<uint32_t>, g, t, 0, s, (const uint32_t*)w, (uint32_t*)wt, items, q); break;
+    case 2:
+        if (narrow) hipLaunchKernelGGL((phase_setup_kernel<uint16_t, uint32_t>), g, t, 0, s, (const uint16_t*)w, (uint16_t*)wt, items, q, wb);
+        else hipLaunchKernelGGL((phase_setup_kernel<uint16_t, int64_t>), g, t, 0, s, (const uint16_t*)w, (uint16_t*)wt, items, q, wb);
+        break;
+    case 4:
+        if (narrow) hipLaunchKernelGGL((phase_setup_kernel<uint32_t, uint32_t>), g, t, 0, s, (const uint32_t*)w, (uint32_t*)wt, items, q, wb);
+        else hipLaunchKernelGGL((phase_setup_kernel<uint32_t, int64_t>), g, t, 0, s, (const uint32_t*)w, (uint32_t*)wt, items, q, wb);
+        break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
