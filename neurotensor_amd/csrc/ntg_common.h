@@ -399,8 +399,8 @@ struct IntPlanesParams { int M, N, K, Kp, Np, batch; int64_t lda, ldb, sA, sB; i
 hipError_t launch_int_split_planes(int planes, const void* A, const void* B, void* a_planes, void* b_planes, const IntPlanesParams& q, hipStream_t s);
 hipError_t launch_int_combine(int planes, const void* parts, const GemmParams& p, int Np, hipStream_t s);
 hipError_t launch_conv_nhwc_dw(int dtype, bool ta, const GemmParams& p, hipStream_t s);   // ta: A (the output gradient) stored [k][m]
-// part rows hold cgp >= cg channels per tap; part_f32: the partial sums are Float32 whatever the dtype
-hipError_t launch_reduce_batch_taps_last(int dtype, bool part_f32, const void* part, void* out, int64_t batch, int64_t rows, int64_t cg, int64_t cgp,
+// part rows hold cgp >= cg channels per tap; the partial sums are Float32 whatever the dtype
+hipError_t launch_reduce_batch_taps_last(int dtype, const void* part, void* out, int64_t batch, int64_t rows, int64_t cg, int64_t cgp,
                                          int64_t taps, int accumulate, hipStream_t s);
 hipError_t launch_flip_weights(int64_t elem_size, const void* w, void* wt, int64_t groups, int64_t og, int64_t cg, int64_t taps, hipStream_t s);
 

@@ -1614,12 +1614,14 @@ static double dkernel_cost_us(int64_t es, int edge, int64_t tiles, int64_t K) {
 }
 // How dW is cut up: `ranges` k ranges of `kr` output pixels (0: one product per image), tiles of edge x edge (0: the launcher's choice), dY read where it
 // lies (its rows 16-byte multiples, an image a whole number of K-steps) or through a channels-last copy of its own (the out
-// channels of a group a 16-byte multiple; any range then), the partial sums in the element type or in Float32.
+// channels of a group a 16-byte multiple; any range then).  The partial sums are Float32 whatever the type, so that a 16-bit gradient
+// is rounded once (rounded to 16 bits each, they left sqrt(2) of one rounding's error in the sum: BFloat16 2 x 256 x 32 x 32 -> 1024
+// channels by 3 x 3 2.45e-3 against 1.66e-3).
 // One product per image left a small layer on a handful of workgroups, each with the whole image as its k (3 x 3 x 3 x 32 -> 64
 // channels on 4 volumes of 32^3 in Float32: 56 workgroups of 32768 pixels, 1285 us), and a 7 x 7 map of 64 images with 64
 // times the partial sums it needs; the ranges are chosen so that tiles x ranges fill whole rounds over the CUs, against the
 // cost of writing and reading the partial sums (4 TB/s) and of the copy of dY.
-struct DkernelPlan { bool ok, copy_dy, part_f32; int64_t ranges, kr, items; int edge; };
+struct DkernelPlan { bool ok, copy_dy; int64_t ranges, kr, items; int edge; };
 static DkernelPlan plan_dkernel(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
     DkernelPlan pl;
     std::memset(&pl, 0, sizeof pl);
@@ -1652,7 +1654,7 @@ static DkernelPlan plan_dkernel(int dtype, int64_t batch, int64_t channels, int6
             const int64_t tiles = ((og + edge - 1) / edge) * ((N + edge - 1) / edge) * items;
             // (the groups' launches run one behind the other)
             const double us = (copy ? 4.0 + 2.0 * (double)(total * out_channels * es) / 4.5e6 : 0.0) + groups * dkernel_cost_us(es, edge, tiles, kr) + 4.0 +
-                              2.0 * (double)(items * out_channels * N * (es == 2 && items > batch ? 4 : es)) / 4.0e6;
+                              2.0 * (double)(items * out_channels * N * 4) / 4.0e6;
             if (pl.edge && us >= best) return;
             best = us;
             pl.copy_dy = copy; pl.ranges = ranges; pl.items = items; pl.kr = kr; pl.edge = edge;
@@ -1669,8 +1671,6 @@ static DkernelPlan plan_dkernel(int dtype, int64_t batch, int64_t channels, int6
             }
         }
     }
-    // (at most one rounding per image, as many as the reference's own per-image products take; more partial sums stay in Float32)
-    pl.part_f32 = es == 2 && pl.items > batch;
     return pl;
 }
 static int64_t conv_dkernel_nhwc_workspace(int dtype, const DkernelPlan& pl, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
@@ -1678,7 +1678,7 @@ static int64_t conv_dkernel_nhwc_workspace(int dtype, const DkernelPlan& pl, int
     const int64_t gy = pl.copy_dy ? (int64_t)align_up((size_t)(batch * out_channels * g.L() * es), 256) : 0;
     const int64_t cgp = dkernel_padded_channels(es, channels / groups);
     return (int64_t)align_up((size_t)(batch * groups * cgp * dkernel_halo(es, channels / groups, groups, g).vol * es), 256) + gy +
-           pl.items * out_channels * cgp * g.taps() * (pl.part_f32 ? 4 : es);
+           pl.items * out_channels * cgp * g.taps() * 4;
 }
 static int conv_dkernel_nhwc(int dtype, const DkernelPlan& pl, const void* image, const void* grad_out, void* d_kernel, void* ws, int64_t batch,
                              int64_t channels, int64_t out_channels, const Geo3& g, int64_t groups, int accumulate, hipStream_t hs) {
@@ -1697,7 +1697,6 @@ static int conv_dkernel_nhwc(int dtype, const DkernelPlan& pl, const void* image
     if (e == hipSuccess && halo.on && volp != vol && !took_along) e = ntg::launch_halo_zero(es, ws_img, batch, chp, halo.hm, hs);
     if (e == hipSuccess && pl.copy_dy) e = ntg::launch_nchw_to_nhwc(es, grad_out, ws_gy, batch, out_channels, L, hs);
     if (e != hipSuccess) return hip_fail(e, "channels-last copy launch");
-    const int64_t pes = pl.part_f32 ? 4 : es;
     for (int64_t gi = 0; gi < groups; ++gi) {
         ntg::GemmParams p;
         std::memset(&p, 0, sizeof p);
@@ -1712,10 +1711,10 @@ static int conv_dkernel_nhwc(int dtype, const DkernelPlan& pl, const void* image
             p.sA = pl.ranges ? 0 : out_channels * L;
         }
         p.B = ws_img + gi * cgp * es;
-        p.C = ws_part + gi * og * N * pes;
+        p.C = ws_part + gi * og * N * 4;
         p.ldb = chp; p.ldc = N;
         p.sB = pl.ranges ? 0 : chp * volp; p.sC = out_channels * N;
-        p.cmode = pl.part_f32 ? ntg::C_PARTIAL : ntg::C_OVERWRITE;
+        p.cmode = ntg::C_PARTIAL;
         p.vecA_ok = 1; p.vecB_ok = 1;
         fill_conv_geom(p.conv, cgp, halo.gp);
         p.conv.chan = (int)chp;                    // elements from one pixel to the next
@@ -1738,7 +1737,7 @@ static int conv_dkernel_nhwc(int dtype, const DkernelPlan& pl, const void* image
         if (e != hipSuccess) return hip_fail(e, "channels-last conv_dkernel launch");
     }
     // (groups are consecutive row blocks of both layouts, so one pass covers them all)
-    e = ntg::launch_reduce_batch_taps_last(dtype, pl.part_f32, ws_part, d_kernel, pl.items, out_channels, cg, cgp, taps, accumulate, hs);
+    e = ntg::launch_reduce_batch_taps_last(dtype, ws_part, d_kernel, pl.items, out_channels, cg, cgp, taps, accumulate, hs);
     if (e != hipSuccess) return hip_fail(e, "weight gradient reduction launch");
     return NTG_OK;
 }

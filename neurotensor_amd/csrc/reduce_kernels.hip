@@ -45,14 +45,14 @@ __global__ void __launch_bounds__(256) reduce_batch_sum_first_kernel(const T* __
 // thread owns 16 bytes of consecutive channels of one (row, tap) and every SLICES-th of the partial sums (four reads in flight),
 // the slices of a column group are added through LDS in slice order.  Bound by the reads of the partial sums; with one slice a
 // small gradient (3 x 3 x 3 x 32 x 64: 55296 elements, 54 workgroups) over hundreds of partial sums would be one long chain of
-// memory latencies on a few CUs, so SLICES grows until the launch has about 1024 workgroups (28 partial sums of 589824 BFloat16
-// elements: 16 slices of 8-byte reads 15.1 us, one slice of 16-byte reads 10.6).  The order of the additions depends on the sizes only.
-template <class T, class P, int SLICES>
-__global__ void __launch_bounds__(256) reduce_batch_taps_last_kernel(const P* __restrict__ part, T* __restrict__ out, const int64_t batch,
+// memory latencies on a few CUs, so SLICES grows until the launch has about 1024 workgroups (28 partial sums of 589824 elements,
+// 66 MB: four slices, 16.1 us).  The order of the additions depends on the sizes only.
+template <class T, int SLICES>
+__global__ void __launch_bounds__(256) reduce_batch_taps_last_kernel(const float* __restrict__ part, T* __restrict__ out, const int64_t batch,
                                                                      const int64_t rows, const int64_t cg, const int64_t cgp, const int64_t taps,
                                                                      const int accumulate) {
-    constexpr int VEC = 16 / (int)sizeof(P);
-    typedef P PV __attribute__((ext_vector_type(VEC)));
+    constexpr int VEC = 4;
+    typedef float PV __attribute__((ext_vector_type(VEC)));
     constexpr int COLS = 256 / SLICES;                    // column groups of VEC elements per workgroup
     __shared__ float sums[SLICES > 1 ? 256 * VEC : 1];
     const int64_t n = rows * cgp * taps, nv = n / VEC;    // (the partial sums hold cgp >= cg channels per tap, the rest padding; cgp % VEC == 0)
@@ -61,7 +61,7 @@ __global__ void __launch_bounds__(256) reduce_batch_taps_last_kernel(const P* __
     const int64_t i = v * VEC;
     float acc[VEC] = {};
     if (v < nv) {
-        const P* pp = part + i;
+        const float* pp = part + i;
         int64_t b = sl;
         for (; b + 3 * SLICES < batch; b += 4 * SLICES) {
             PV x[4];
@@ -70,12 +70,12 @@ __global__ void __launch_bounds__(256) reduce_batch_taps_last_kernel(const P* __
 #pragma unroll
             for (int u = 0; u < 4; ++u)
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) acc[e] += (float)x[u][e];
+                for (int e = 0; e < VEC; ++e) acc[e] += x[u][e];
         }
         for (; b < batch; b += SLICES) {
             const PV x = *reinterpret_cast<const PV*>(pp + b * n);
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) acc[e] += (float)x[e];
+            for (int e = 0; e < VEC; ++e) acc[e] += x[e];
         }
     }
     if constexpr (SLICES > 1) {
@@ -265,31 +265,25 @@ hipError_t launch_reduce_batch(int dtype, const void* part, void* out, int64_t b
     return hipGetLastError();
 }
 
-template <class T, class P>
+template <class T>
 static void launch_reduce_taps_last_t(const void* part, void* out, int64_t batch, int64_t rows, int64_t cg, int64_t cgp, int64_t taps, int accumulate, hipStream_t s) {
-    const int64_t nv = rows * cgp * taps / (16 / (int64_t)sizeof(P));
+    const int64_t nv = rows * cgp * taps / 4;
 #define NTG_TAPS_LAST(S) \
-    hipLaunchKernelGGL((reduce_batch_taps_last_kernel<T, P, S>), dim3((unsigned)((nv * S + 255) / 256)), dim3(256), 0, s, (const P*)part, (T*)out, batch, rows, cg, cgp, taps, accumulate)
+    hipLaunchKernelGGL((reduce_batch_taps_last_kernel<T, S>), dim3((unsigned)((nv * S + 255) / 256)), dim3(256), 0, s, (const float*)part, (T*)out, batch, rows, cg, cgp, taps, accumulate)
     if (nv >= 256 * 1024 || batch < 8) NTG_TAPS_LAST(1);
     else if (nv * 4 >= 256 * 1024 || batch < 32) NTG_TAPS_LAST(4);
     else NTG_TAPS_LAST(16);
 #undef NTG_TAPS_LAST
 }
-hipError_t launch_reduce_batch_taps_last(int dtype, bool part_f32, const void* part, void* out, int64_t batch, int64_t rows, int64_t cg, int64_t cgp,
+hipError_t launch_reduce_batch_taps_last(int dtype, const void* part, void* out, int64_t batch, int64_t rows, int64_t cg, int64_t cgp,
                                          int64_t taps, int accumulate, hipStream_t s) {
     const int64_t n = rows * cgp * taps;
     if (n == 0) return hipSuccess;
-    if (cgp % (part_f32 || dtype == DT_F32 ? 4 : 8) != 0 || (reinterpret_cast<uintptr_t>(part) & 15) != 0 || n / 64 >= 0x7fffffffLL) return hipErrorInvalidValue;
+    if (cgp % 4 != 0 || (reinterpret_cast<uintptr_t>(part) & 15) != 0 || n / 64 >= 0x7fffffffLL) return hipErrorInvalidValue;
     switch (dtype) {
-    case DT_F32: launch_reduce_taps_last_t<float, float>(part, out, batch, rows, cg, cgp, taps, accumulate, s); break;
-    case DT_F16:
-        if (part_f32) launch_reduce_taps_last_t<_Float16, float>(part, out, batch, rows, cg, cgp, taps, accumulate, s);
-        else launch_reduce_taps_last_t<_Float16, _Float16>(part, out, batch, rows, cg, cgp, taps, accumulate, s);
-        break;
-    case DT_BF16:
-        if (part_f32) launch_reduce_taps_last_t<__bf16, float>(part, out, batch, rows, cg, cgp, taps, accumulate, s);
-        else launch_reduce_taps_last_t<__bf16, __bf16>(part, out, batch, rows, cg, cgp, taps, accumulate, s);
-        break;
+    case DT_F32: launch_reduce_taps_last_t<float>(part, out, batch, rows, cg, cgp, taps, accumulate, s); break;
+    case DT_F16: launch_reduce_taps_last_t<_Float16>(part, out, batch, rows, cg, cgp, taps, accumulate, s); break;
+    case DT_BF16: launch_reduce_taps_last_t<__bf16>(part, out, batch, rows, cg, cgp, taps, accumulate, s); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -1,0 +1,69 @@
+"""How far the convolutions' gradients are from their sums in 64 bits, and what their rarer forms return."""
+import itertools
+
+import pytest
+import torch
+
+from neurotensor_amd import functional as F
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def randn(shape, dtype, seed, scale=1.0):
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(seed)
+    return (torch.randn(shape, device=DEV, generator=gen) * scale).to(dtype)
+
+
+def windows(x, k, s, p, d, out):
+    """(tap, the [B, C, *out] elements that it meets) for every tap of the window."""
+    nd = len(k)
+    xp = torch.nn.functional.pad(x, [q for a in reversed(range(nd)) for q in (p[a], p[a])])
+    for t in itertools.product(*[range(i) for i in k]):
+        yield t, xp[(slice(None), slice(None)) + tuple(slice(t[a] * d[a], t[a] * d[a] + (out[a] - 1) * s[a] + 1, s[a]) for a in range(nd))]
+
+
+def exact_dw(x, g, k, s, p, d, groups):
+    """The weight gradient in Float64: one product of matrices per tap and group."""
+    x, g = x.double(), g.double()
+    O, cg, og = g.shape[1], x.shape[1] // groups, g.shape[1] // groups
+    dw = torch.zeros((O, cg) + tuple(k), device=x.device, dtype=torch.float64)
+    for t, win in windows(x, k, s, p, d, g.shape[2:]):
+        for gi in range(groups):
+            xg = win[:, gi * cg:(gi + 1) * cg].transpose(0, 1).reshape(cg, -1).t().contiguous()
+            gg = g[:, gi * og:(gi + 1) * og].transpose(0, 1).reshape(og, -1).contiguous()
+            dw[(slice(gi * og, (gi + 1) * og), slice(None)) + t] = gg @ xg
+    return dw
+
+
+def relative(got, want):
+    return ((got.double() - want).norm() / want.norm()).item()
+
+
+def backward(nd):
+    return {1: F.conv1d_backward, 2: F.conv2d_backward, 3: F.conv3d_backward}[nd]
+
+
+@pytest.mark.parametrize("geom", [
+    # (B, C, size, O, kernel, stride, padding, groups)
+    (2, 256, (32, 32), 1024, (3, 3), 1, 1, 1),      # two k ranges in 256 x 256 tiles
+    (64, 512, (14, 14), 512, (7, 7), 1, 3, 1),      # a few ranges over 64 images
+    (64, 256, (28, 28), 256, (3, 3), 1, 1, 1),      # as many as fill the CUs
+    (26, 96, (13, 13, 13), 256, (3, 3, 3), 1, 1, 1),
+    (6, 24, (9, 9, 9), 64, (3, 3, 3), 2, 1, 1),
+    (10, 128, (19, 19), 48, (7, 7), 1, 3, 1),       # rows that miss the 16-byte rule: dY through its copy
+    (16, 16, (7, 17), 32, (3, 3), 1, 1, 4),
+    (2, 192, (40, 40), 256, (3, 3), 2, 1, 1),
+], ids=lambda g: "x".join(map(str, g)))
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_16_bit_weight_gradients_are_rounded_once(geom, dtype):
+    """A gradient that is one rounding of its Float32 sum is as far from the exact sum as that sum's own rounding (the Float32 chain
+    adds some 1e-6 of it); a second rounding, of partial sums, makes that sqrt(2) times as much.  1.1 lies between."""
+    B, C, size, O, k, s, p, groups = geom
+    nd = len(size)
+    out = [(size[a] + 2 * p - k[a]) // s + 1 for a in range(nd)]
+    x, w, g = randn((B, C) + size, dtype, 1), randn((O, C // groups) + k, dtype, 2, 0.05), randn([B, O] + out, dtype, 3)
+    _, dw = backward(nd)(x, w, g, stride=s, padding=p, groups=groups)
+    want = exact_dw(x, g, k, (s,) * nd, (p,) * nd, (1,) * nd, groups)
+    assert relative(dw, want) <= 1.1 * relative(want.to(dtype), want), (relative(dw, want), relative(want.to(dtype), want))
