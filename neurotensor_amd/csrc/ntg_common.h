@@ -358,7 +358,8 @@ struct HaloMap {
 // launch_flip_weights_channels_last(w, wp, groups = a, og, ogp, cg, taps, chunk).
 struct WeightsJob { int kind; const void* w; void* wp; int64_t a, og, ogp, cg, cgp, taps, chunk; };
 // With `halo`, pixels go to their places inside the bordered copy.  When the 16-byte kernel serves the copy it also zeroes
-// the border and runs `job` in the same launch and sets *took_along; otherwise the caller launches those two itself.
+// the border in the same launch, runs `job` (there too, or where the blocks are too few for it in a launch of its own) and
+// sets *took_along; otherwise the caller launches those two itself.
 hipError_t launch_nchw_to_nhwc(int64_t elem_size, const void* in, void* out, int64_t batch, int64_t C, int64_t P, hipStream_t s, const HaloMap* halo = nullptr,
                                const WeightsJob* job = nullptr, bool* took_along = nullptr);
 hipError_t launch_halo_zero(int64_t elem_size, void* out, int64_t batch, int64_t C, const HaloMap& halo, hipStream_t s);   // zeros the border pixels

@@ -488,6 +488,16 @@ hipError_t launch_nchw_to_nhwc(int64_t es, const void* in, void* out, int64_t ba
             if (job && job->kind) {
                 ex.job = *job;
                 ex.job_total = job->kind == 1 ? job->a * job->cgp * job->taps : job->a * job->ogp * job->cg * job->taps;
+                // Small images have few blocks, and an element is a chain of divisions and a strided read, about 0.55 us: eight a thread
+                // take as long as a launch, beyond that the permutation goes out on its own (Float32 1 x 512 x 4 x 4 x 4 -> 128
+                // channels by 3 x 3 x 3, eight blocks: 864 elements a thread, image gradient 1960 us; on its own 84 us).
+                if (ex.job_total > 8 * 256 * gx * gy * std::min<int64_t>(batch, 65535)) {
+                    const WeightsJob& j = *job;
+                    const hipError_t e = j.kind == 1 ? launch_weights_channels_last(es, j.w, j.wp, j.a, j.cg, j.cgp, j.taps, s, j.chunk)
+                                                     : launch_flip_weights_channels_last(es, j.w, j.wp, j.a, j.og, j.ogp, j.cg, j.taps, s, j.chunk);
+                    if (e != hipSuccess) return e;
+                    ex.job.kind = 0;
+                }
             }
             *took_along = true;
         }

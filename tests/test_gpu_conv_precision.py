@@ -1,4 +1,4 @@
-"""How far the convolutions' gradients are from their sums in 64 bits, and what their rarer forms return."""
+"""How far the convolutions' gradients are from their sums in 64 bits, and what their rarer forms return and take."""
 import itertools
 
 import pytest
@@ -67,3 +67,33 @@ def test_16_bit_weight_gradients_are_rounded_once(geom, dtype):
     _, dw = backward(nd)(x, w, g, stride=s, padding=p, groups=groups)
     want = exact_dw(x, g, k, (s,) * nd, (p,) * nd, (1,) * nd, groups)
     assert relative(dw, want) <= 1.1 * relative(want.to(dtype), want), (relative(dw, want), relative(want.to(dtype), want))
+
+
+def microseconds(fn, passes=10):
+    for _ in range(3):
+        fn()
+    best = float("inf")
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(passes):
+            fn()
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b) / passes * 1e3)
+    return best
+
+
+@pytest.mark.parametrize("nd", [2, 3])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_many_weights_over_one_small_image(nd, dtype):
+    """A single small image (a copy of eight blocks beside a million weights) takes no longer than sixteen of them, and gives the
+    first of the sixteen's results bit for bit."""
+    size, k = (4,) * nd, (3,) * nd
+    x, w, g = randn((16, 512) + size, dtype, 1), randn((192, 512) + k, dtype, 2, 0.02), randn((16, 192) + size, dtype, 3)
+    fwd = {2: F.conv2d, 3: F.conv3d}[nd]
+    calls = (lambda n: fwd(x[:n], w, padding=1), lambda n: backward(nd)(x[:n], w, g[:n], padding=1)[0])
+    for call in calls:
+        assert torch.equal(call(1)[0], call(16)[0])
+        one, sixteen = microseconds(lambda: call(1)), microseconds(lambda: call(16))
+        assert one <= 1.2 * sixteen, (one, sixteen)
