@@ -1213,11 +1213,14 @@ static int conv_forward_pointwise(int dtype, const void* image, const void* kern
 // channels of one tap, and the kernel's DMA gathers the operand in 16-byte pieces instead of element by element.
 
 // Byte offsets inside a channels-last image are formed in 32 bits from two terms (the pixel of the window origin, and the
-// tap reach with the padding taken off): both must stay below 2^30
+// tap reach with the padding taken off): both must stay below 2^30.  The tap counters run to the first tap behind the window, so
+// the reach is k d and not (k - 1) d; over two axes there is no depth to step through (counted as one whole slice it refused
+// images within one window's reach of 2^30 bytes).
 static bool conv_nhwc_offsets_fit(int64_t channels, int64_t es, const Geo3& g) {
     auto mag = [](int64_t v) { return v < 0 ? -v : v; };
     const int64_t pd = mag(g.p[0]), pr = mag(g.p[1]), pc = mag(g.p[2]);
-    const int64_t reach = (((pd + g.k[0] * g.d[0]) * g.sz[1] + pr + g.k[1] * g.d[1]) * g.sz[2] + pc + g.k[2] * g.d[2]) * channels * es;
+    const int64_t slices = g.nd == 3 ? pd + g.k[0] * g.d[0] : 0;
+    const int64_t reach = ((slices * g.sz[1] + pr + g.k[1] * g.d[1]) * g.sz[2] + pc + g.k[2] * g.d[2]) * channels * es;
     return channels * g.vol() * es < (1LL << 30) && reach < (1LL << 30);
 }
 // A K-step of the channels-last kernel is 64 bytes of channels of one tap, so the copy pads the channels of each group

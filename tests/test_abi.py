@@ -97,6 +97,9 @@ def test_argument_errors_do_not_need_a_device():
     assert fast(_lib.FLOAT32, 4, 64, 8, 8, 32, 1, 1, 1, 1, 0, 0, 1, 1, 1) == 0                            # 1x1: product in place
     assert fast(_lib.FLOAT32, 4, 64, 7, 7, 32, 1, 1, 1, 1, 0, 0, 1, 1, 1) == 50176 + 32 * 64 * 4   # rows of 196 bytes
     assert fast(_lib.FLOAT32, 1, 16, 2, 2, 8, 3, 3, 1, 1, 0, 0, 1, 1, 1) == -1                            # kernel larger than the image
+    # the copy of an image may come as close to 2^30 bytes as a window's rows allow: 2896 x 2896 pixels of 128 bytes are 2^30 - 229376
+    assert fast(_lib.BFLOAT16, 1, 64, 2896, 2896, 32, 3, 3, 1, 1, 0, 0, 1, 1, 1) == 2896 * 2896 * 128 + 32 * 64 * 9 * 2
+    assert fast(_lib.BFLOAT16, 1, 64, 2897, 2897, 32, 3, 3, 1, 1, 0, 0, 1, 1, 1) == 0
     # per-image weight gradients [B, O, C/g * taps] instead of the im2col matrix
     # (the larger figure: channels-last copy of the image with the 2 channels of each group padded to 4, per-image results)
     assert lib.ntg_conv2d_backward_workspace_bytes(_lib.FLOAT32, 2, 4, 8, 8, 6, 3, 3, 1, 1, 1, 1, 1, 1, 2) == 2 * 2 * 4 * 64 * 4 + 2 * 6 * 4 * 9 * 4
