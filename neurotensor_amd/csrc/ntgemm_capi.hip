@@ -1471,7 +1471,8 @@ static PhasePlan plan_dimage_phases(int dtype, int64_t batch, int64_t channels, 
         if (g.d[a] != 1 || g.s[a] > 4 || g.p[a] < 0 || g.sz[a] >= (1 << 24) || g.k[a] >= (1 << 16)) return pp;
     const int64_t es = ntg::elem_size(dtype), vel = 16 / es, og = out_channels / groups, cg = channels / groups;
     const int64_t ogp = nhwc_padded_channels(es, og), ochp = groups * ogp;
-    if (ogp == 0 || batch * channels * (g.vol() + 64 * vel) >= 0x7fffffffLL) return pp;
+    // (the interleaving pass counts image elements in 32 bits; one image's planes, whose pitches are 16-byte multiples, are indexed in 32 bits)
+    if (ogp == 0 || batch * channels * g.vol() >= 0x7fffffffLL || channels * (g.vol() + 64 * vel) >= 0x7fffffffLL) return pp;
     // the image channels of a group are the rows of these products: with a handful of them (an RGB input layer) a 64-row
     // tile is mostly padding, and the GEMM over (channel, tap) rows followed by col2im is the better form
     if (cg < 16) return pp;
@@ -1500,7 +1501,12 @@ static PhasePlan plan_dimage_phases(int dtype, int64_t batch, int64_t channels, 
     }
     const int64_t volp = (int64_t)q.yp[0] * q.yp[1] * q.yp[2];
     const Geo3 reach = {g.nd, {q.yp[0], q.yp[1], q.yp[2]}, {g.k[0], g.k[1], g.k[2]}, {1, 1, 1}, {0, 0, 0}, {1, 1, 1}, {1, 1, 1}};
-    if (volp > 4 * g.L() + 64 || !conv_nhwc_offsets_fit(ochp, es, reach) || ogp * g.taps() >= 0x7fffffffLL) return pp;
+    // A border of many times dY: in Float32 the col matrix is the faster form (32 x 128 x 8 x 256 from 8 x 8 at stride 2, one row of 125
+    // outputs, 256 out channels: 231 us against 541 by phases).  In 16 bits it is slower (247 against 128 us; a small one, 4 x 32 x 8 x 64,
+    // 18 against 27) and rounds every entry of the col matrix besides the sum (2.4e-3 from the exact gradient against 1.7e-3), so the
+    // phases keep what they served over two axes with windows of up to 8 taps, whose border is at most 7 positions on each side.
+    const bool keep = es == 2 && g.nd == 2 && g.k[1] <= 8 && g.k[2] <= 8;
+    if ((!keep && volp > 4 * g.L() + 64) || !conv_nhwc_offsets_fit(ochp, es, reach) || ogp * g.taps() >= 0x7fffffffLL) return pp;
     pp.hm.W = g.o[2]; pp.hm.H = g.o[1]; pp.hm.D = g.o[0];
     pp.hm.Wp = q.yp[2]; pp.hm.Hp = q.yp[1]; pp.hm.Dp = q.yp[0];
     pp.hm.left = front[2]; pp.hm.top = front[1]; pp.hm.front = front[0];

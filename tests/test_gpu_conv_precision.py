@@ -19,7 +19,7 @@ def randn(shape, dtype, seed, scale=1.0):
 def windows(x, k, s, p, d, out):
     """(tap, the [B, C, *out] elements that it meets) for every tap of the window."""
     nd = len(k)
-    xp = torch.nn.functional.pad(x, [q for a in reversed(range(nd)) for q in (p[a], p[a])])
+    xp = torch.nn.functional.pad(x, [q for a in reversed(range(nd)) for q in (p[a], p[a])]) if any(p) else x
     for t in itertools.product(*[range(i) for i in k]):
         yield t, xp[(slice(None), slice(None)) + tuple(slice(t[a] * d[a], t[a] * d[a] + (out[a] - 1) * s[a] + 1, s[a]) for a in range(nd))]
 
@@ -35,6 +35,20 @@ def exact_dw(x, g, k, s, p, d, groups):
             gg = g[:, gi * og:(gi + 1) * og].transpose(0, 1).reshape(og, -1).contiguous()
             dw[(slice(gi * og, (gi + 1) * og), slice(None)) + t] = gg @ xg
     return dw
+
+
+def exact_dx(size, w, g, k, s, p, d, groups):
+    """The image gradient in Float64: one product of matrices per tap and group, added at the elements that the tap meets."""
+    w, g = w.double(), g.double()
+    B, O, out = g.shape[0], g.shape[1], tuple(g.shape[2:])
+    cg, og = w.shape[1], O // groups
+    dx = torch.zeros((B, cg * groups) + tuple(size[a] + 2 * p[a] for a in range(len(size))), device=w.device, dtype=torch.float64)
+    for t, win in windows(dx, k, s, (0,) * len(k), d, out):
+        for gi in range(groups):
+            gg = g[:, gi * og:(gi + 1) * og].transpose(0, 1).reshape(og, -1)
+            col = w[(slice(gi * og, (gi + 1) * og), slice(None)) + t].t().contiguous() @ gg
+            win[:, gi * cg:(gi + 1) * cg] += col.reshape((cg, B) + out).transpose(0, 1)
+    return dx[(slice(None), slice(None)) + tuple(slice(p[a], p[a] + size[a]) for a in range(len(size)))]
 
 
 def relative(got, want):
@@ -97,3 +111,23 @@ def test_many_weights_over_one_small_image(nd, dtype):
         assert torch.equal(call(1)[0], call(16)[0])
         one, sixteen = microseconds(lambda: call(1)), microseconds(lambda: call(16))
         assert one <= 1.2 * sixteen, (one, sixteen)
+
+
+@pytest.mark.parametrize("geom", [
+    # (B, C, size, O, kernel, stride, padding, groups)
+    (4, 32, (8, 64), 32, (8, 8), 2, (0, 0), 1),            # one row of outputs: the border is 7 times dY
+    (3, 64, (9, 130), 48, (8, 7), (2, 3), (0, 3), 2),
+    (2, 32, (7, 40), 32, (7, 4), (1, 4), (0, 1), 1),       # a stride along one axis: a border of 6 rows on each side of one row
+    (4096, 1024, (4, 4), 16, (3, 3), 2, (1, 1), 1),        # four million planes of four elements
+], ids=lambda g: "x".join(map(str, g)))
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_16_bit_strided_image_gradients_are_rounded_once(geom, dtype):
+    """Image gradients by phases of the strides are one rounding of their Float32 sums (bound as above); the GEMM + col2im form rounds
+    every entry of the col matrix and then their sum."""
+    B, C, size, O, k, s, p, groups = geom
+    s = s if isinstance(s, tuple) else (s, s)
+    out = [(size[a] + 2 * p[a] - k[a]) // s[a] + 1 for a in range(2)]
+    x, w, g = randn((B, C) + size, dtype, 1), randn((O, C // groups) + k, dtype, 2, 0.05), randn([B, O] + out, dtype, 3)
+    dx, _ = F.conv2d_backward(x, w, g, stride=s, padding=p, groups=groups)
+    want = exact_dx(size, w, g, k, s, p, (1, 1), groups)
+    assert relative(dx, want) <= 1.1 * relative(want.to(dtype), want), (relative(dx, want), relative(want.to(dtype), want))
