@@ -1658,6 +1658,11 @@ static DkernelPlan plan_dkernel(int dtype, int64_t batch, int64_t channels, int6
             pl.edge = es == 2 ? ntg::ring16_tile_edge(og, N, pl.kr, r) : 64;
         }
     } else {
+        // A range has the pixels of an image at least, where those are two to eight K-steps: it is one Float32 chain, and over small maps
+        // ranges longer than the reference's chains cost time -- groups run one behind the other -- and digits (22 x 23 x 69 -> 4 by 5 at
+        // stride 3: 1.2e-7 from the exact gradient in chains of one image, 2.1e-7 in three ranges of 176 pixels), while shorter ones
+        // ask for a larger workspace than one gradient per image.
+        const int64_t shortest = std::min<int64_t>(8, std::max<int64_t>(2, (L + bk - 1) / bk));
         double best = 0.0;
         const auto consider = [&](bool copy, int64_t ranges, int64_t items, int64_t kr, int edge) {
             const int64_t tiles = ((og + edge - 1) / edge) * ((N + edge - 1) / edge) * items;
@@ -1673,10 +1678,7 @@ static DkernelPlan plan_dkernel(int dtype, int64_t batch, int64_t channels, int6
             if (rows_16) consider(false, 0, batch, L, edge);
             const int64_t tiles = ((og + edge - 1) / edge) * ((N + edge - 1) / edge) * groups;
             for (int64_t target : {256, 512, 768, 1024, 1536, 2048}) {
-                // (ranges of two K-steps at least: a range is one Float32 chain, and over small maps longer ones cost time -- groups run one
-                //  behind the other -- and digits: 22 x 23 x 69 -> 4 by 5 at stride 3 is 1.2e-7 from the exact gradient in the reference's
-                //  chains of one image, 2.1e-7 in three ranges of 176 pixels)
-                const int64_t want = std::min(std::max<int64_t>(target / tiles, 1), std::max<int64_t>(steps / 2, 1));
+                const int64_t want = std::min(std::max<int64_t>(target / tiles, 1), std::max<int64_t>(steps / shortest, 1));
                 const int64_t per = (steps + want - 1) / want, r = (steps + per - 1) / per;
                 if (lies) consider(false, r, r, per * bk, edge);
                 if (copied) consider(true, r, r, per * bk, edge);
