@@ -353,9 +353,17 @@ int ntg_conv_transpose2d(int dtype, const void* input, const void* kernel, void*
  * size / kernel_size / stride / padding / dilation / output_padding point to `ndim` values, slowest axis first
  * (depth, rows, columns).  image [batch, channels, size...], kernel [out_channels, channels/groups, kernel_size...]
  * (transposed: [in_channels, out_channels/groups, kernel_size...]).  ndim 1 and 2 run on the conv2d entry points above;
- * ndim 3 gathers the unfolded operand inside the GEMM for the floating dtypes (workspace as for conv2d); ndim 4, the
- * integer dtypes and kernels wider than 8 taps unfold into the workspace like the reference.  `backward` selects the
- * workspace of the gradient call. */
+ * ndim 4, the integer dtypes and kernels wider than 8 taps unfold into the workspace like the reference.  ndim 3 in the
+ * floating dtypes gathers the unfolded operand inside the GEMM, in one of two orders of summation:
+ *   with ntg_convnd_workspace_bytes -- element by element: a Float32 result is unfold + matmult bit for bit, a weight
+ *     gradient sums the output pixels of one image in ascending order and then the images (like the host entry points);
+ *   with ntg_convnd_fast_workspace_bytes -- Float32 / Float16 / BFloat16 from channels-last copies that carry the padding:
+ *     k runs (channels of one 64-byte run, tap) in the forward call and the image gradient, which at strides > 1 is one
+ *     convolution per residue of the image position; the weight gradient's sums run through the pixels of all images in
+ *     equal ranges, `accumulate` adds the incoming value last.  Where there is no such form the two figures are equal.
+ * ndim <= 2: the first is ntg_conv2d_forward_workspace_bytes, the second ntg_conv2d_fast_workspace_bytes; both are
+ * ntg_conv2d_backward_workspace_bytes for the gradients.  `backward` selects the workspace of the gradient call.  The
+ * calls accept every amount from the first figure on; ntg_conv_transposend_workspace_bytes is that of the fast forms. */
 int ntg_unfoldnd_dev(int dtype, const void* image, void* col, int64_t batch, int64_t channels, int ndim, const int64_t* size,
                      const int64_t* kernel_size, const int64_t* stride, const int64_t* padding, const int64_t* dilation, void* stream);
 int ntg_unfoldnd_backward_dev(int dtype, const void* col, void* image, int64_t batch, int64_t channels, int ndim, const int64_t* size,
@@ -364,6 +372,9 @@ int ntg_unfoldnd_backward_dev(int dtype, const void* col, void* image, int64_t b
 int64_t ntg_convnd_workspace_bytes(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int ndim, const int64_t* size,
                                    const int64_t* kernel_size, const int64_t* stride, const int64_t* padding, const int64_t* dilation,
                                    int64_t groups, int backward);
+int64_t ntg_convnd_fast_workspace_bytes(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int ndim, const int64_t* size,
+                                        const int64_t* kernel_size, const int64_t* stride, const int64_t* padding, const int64_t* dilation,
+                                        int64_t groups, int backward);
 int ntg_convnd_dev(int dtype, const void* image, const void* kernel, void* out, void* workspace, int64_t workspace_bytes,
                    int64_t batch, int64_t channels, int64_t out_channels, int ndim, const int64_t* size, const int64_t* kernel_size,
                    const int64_t* stride, const int64_t* padding, const int64_t* dilation, int64_t groups, void* stream);

@@ -82,6 +82,7 @@ SIGNATURES = {
     "ntg_unfoldnd_dev": (_ci, [_ci, _vp, _vp, _i64, _i64, _ci] + [_pi64] * 5 + [_vp]),
     "ntg_unfoldnd_backward_dev": (_ci, [_ci, _vp, _vp, _i64, _i64, _ci] + [_pi64] * 5 + [_ci, _vp]),
     "ntg_convnd_workspace_bytes": (_i64, [_ci, _i64, _i64, _i64, _ci] + [_pi64] * 5 + [_i64, _ci]),
+    "ntg_convnd_fast_workspace_bytes": (_i64, [_ci, _i64, _i64, _i64, _ci] + [_pi64] * 5 + [_i64, _ci]),
     "ntg_convnd_dev": (_ci, [_ci, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _ci] + [_pi64] * 5 + [_i64, _vp]),
     "ntg_convnd_backward_dev": (_ci, [_ci, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _ci] + [_pi64] * 5 + [_i64, _ci, _vp]),
     "ntg_conv_transposend_workspace_bytes": (_i64, [_ci, _i64, _i64, _i64, _ci] + [_pi64] * 6 + [_i64]),

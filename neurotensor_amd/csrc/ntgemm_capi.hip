@@ -2389,14 +2389,31 @@ int64_t ntg_convnd_workspace_bytes(int dtype, int64_t batch, int64_t channels, i
     }
     if (ndim == 3) {
         const Geo3 g = geo_from(u);
-        if (backward) {
-            const ConvBackwardPlan pl = plan_conv_backward_g(dtype, true, true, batch, channels, out_channels, g, groups);
-            return std::max(std::max(pl.need, pl.need_phase_dx), std::max(pl.need_nhwc_dx, pl.need_nhwc_dw));
-        }
-        if (conv_nhwc_ok(dtype, channels, out_channels, groups, g)) return conv_nhwc_workspace(dtype, batch, channels, out_channels, groups, g);
+        if (backward) return plan_conv_backward_g(dtype, true, true, batch, channels, out_channels, g, groups).need;
         if (conv_implicit_g(dtype, channels, g)) return 0;
     }
     return u.total * es + (backward ? complex_dkernel_extra(dtype, batch, out_channels, (channels / groups) * u.taps, u.total * es) : 0);
+}
+
+int64_t ntg_convnd_fast_workspace_bytes(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int ndim, const int64_t* size,
+                                        const int64_t* kernel_size, const int64_t* stride, const int64_t* padding, const int64_t* dilation,
+                                        int64_t groups, int backward) {
+    const int64_t least = ntg_convnd_workspace_bytes(dtype, batch, channels, out_channels, ndim, size, kernel_size, stride, padding, dilation, groups, backward);
+    if (least < 0) return least;
+    if (ndim <= 2) {
+        const Geo2 g = as_2d(ndim, size, kernel_size, stride, padding, dilation);
+        return backward ? least : ntg_conv2d_fast_workspace_bytes(dtype, batch, channels, g.h, g.w, out_channels, g.kr, g.kc, g.sr, g.sc, g.pr, g.pc, g.dr, g.dc, groups);
+    }
+    if (ndim != 3) return least;
+    ntg::UnfoldNdParams u;
+    if (fill_nd(u, batch, channels, ndim, size, kernel_size, stride, padding, dilation)) return -1;
+    const Geo3 g = geo_from(u);
+    if (backward) {
+        const ConvBackwardPlan pl = plan_conv_backward_g(dtype, true, true, batch, channels, out_channels, g, groups);
+        const int64_t fast = std::max(pl.need_phase_dx, std::max(pl.need_nhwc_dx, pl.need_nhwc_dw));
+        return fast > 0 ? std::max(fast, least + 256) : least;        // (more than `least` is what asks for the fast forms)
+    }
+    return conv_nhwc_ok(dtype, channels, out_channels, groups, g) ? conv_nhwc_workspace(dtype, batch, channels, out_channels, groups, g) : least;
 }
 
 int ntg_convnd_dev(int dtype, const void* image, const void* kernel, void* out, void* workspace, int64_t workspace_bytes,
@@ -2473,8 +2490,11 @@ static int convnd_backward_dev_impl(int dtype, const void* image, const void* ke
         need = plan.need;
         if (need > 0 && (!workspace || workspace_bytes < need))
             return fail(NTG_ERR_INVALID_ARGUMENT, "workspace of %lld bytes needed, %lld given", (long long)need, (long long)workspace_bytes);
+        // a workspace of ntg_convnd_workspace_bytes asks for the reference's order, even where a fast form would fit into it
+        const bool fast = channels_last && workspace_bytes > ntg_convnd_workspace_bytes(dtype, batch, channels, out_channels, ndim, size, kernel_size, stride,
+                                                                                        padding, dilation, groups, 1);
         if (plan.gather_dw) {
-            if (channels_last && plan.nhwc_dw && workspace_bytes >= plan.need_nhwc_dw &&
+            if (fast && plan.nhwc_dw && workspace_bytes >= plan.need_nhwc_dw &&
                 ((reinterpret_cast<uintptr_t>(workspace) | reinterpret_cast<uintptr_t>(grad_out)) & 15) == 0)
                 rc = conv_dkernel_nhwc(dtype, plan.dkernel, image, grad_out, d_kernel, workspace, batch, channels, out_channels, g, groups, accumulate,
                                        static_cast<hipStream_t>(stream));
@@ -2485,7 +2505,7 @@ static int convnd_backward_dev_impl(int dtype, const void* image, const void* ke
             d_kernel = nullptr;
         }
         if (plan.gather_dx) {
-            if (channels_last && plan.nhwc_dx && workspace_bytes >= plan.need_nhwc_dx && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0)
+            if (fast && plan.nhwc_dx && workspace_bytes >= plan.need_nhwc_dx && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0)
                 rc = conv_dimage_nhwc(dtype, kernel, grad_out, d_image, workspace, batch, channels, out_channels, g, groups, accumulate,
                                       static_cast<hipStream_t>(stream));
             else
@@ -2494,7 +2514,7 @@ static int convnd_backward_dev_impl(int dtype, const void* image, const void* ke
             if (rc) return rc;
             d_image = nullptr;
         }
-        if (d_image && channels_last && plan.phase_dx && workspace_bytes >= plan.need_phase_dx && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0) {
+        if (d_image && fast && plan.phase_dx && workspace_bytes >= plan.need_phase_dx && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0) {
             rc = conv_dimage_phases(dtype, plan.phases, kernel, grad_out, d_image, workspace, batch, channels, out_channels, g, groups, accumulate,
                                     static_cast<hipStream_t>(stream));
             if (rc) return rc;
@@ -2566,7 +2586,7 @@ int64_t ntg_conv_transposend_workspace_bytes(int dtype, int64_t batch, int64_t i
         return ntg_conv_transpose2d_workspace_bytes(dtype, batch, in_channels, g.h, g.w, out_channels, g.kr, g.kc, g.sr, g.sc, g.pr, g.pc, g.dr, g.dc,
                                                     ndim == 1 ? 0 : output_padding[0], output_padding[ndim - 1], groups);
     }
-    return ntg_convnd_workspace_bytes(dtype, batch, out_channels, in_channels, ndim, os, kernel_size, stride, padding, dilation, groups, 1);
+    return ntg_convnd_fast_workspace_bytes(dtype, batch, out_channels, in_channels, ndim, os, kernel_size, stride, padding, dilation, groups, 1);
 }
 
 int ntg_conv_transposend_dev(int dtype, const void* input, const void* kernel, void* out, void* workspace, int64_t workspace_bytes,
@@ -2605,9 +2625,9 @@ int ntg_convnd(int dtype, const void* image, const void* kernel, void* out, int6
     if (!image || !kernel || !out) return fail(NTG_ERR_INVALID_ARGUMENT, "null pointer");
     const size_t im_bytes = (size_t)(batch * channels * u.vol * es), k_bytes = (size_t)(out_channels * (channels / groups) * u.taps * es);
     const size_t o_bytes = (size_t)(batch * out_channels * u.L * es);
-    int64_t wsb = ntg_convnd_workspace_bytes(dtype, batch, channels, out_channels, ndim, size, kernel_size, stride, padding, dilation, groups, 0);
-    // (Float32 at the reference's seam keeps the gathering kernels and with them im2col's order of k, see ntg_conv2d)
-    if (dtype == ntg::DT_F32 && ndim == 3 && conv_implicit_g(dtype, channels, geo_from(u))) wsb = 0;
+    // (Float32 at the reference's seam keeps the gathering kernels and with them im2col's order of k, see ntg_conv2d; so do one and two axes)
+    const int64_t wsb = (dtype == ntg::DT_F32 || ndim != 3 ? ntg_convnd_workspace_bytes : ntg_convnd_fast_workspace_bytes)(
+        dtype, batch, channels, out_channels, ndim, size, kernel_size, stride, padding, dilation, groups, 0);
     ntg::HostSession mem;
     const size_t o_k = align_up(im_bytes, 256), o_o = o_k + align_up(k_bytes, 256), o_ws = o_o + align_up(o_bytes, 256);
     HIP_TRY(mem.reserve(o_ws + (size_t)wsb));
@@ -2639,7 +2659,9 @@ int ntg_convnd_backward(int dtype, const void* image, const void* kernel, const 
     }
     const size_t im_bytes = (size_t)(batch * channels * u.vol * es), k_bytes = (size_t)(out_channels * (channels / groups) * u.taps * es);
     const size_t g_bytes = (size_t)(batch * out_channels * u.L * es);
-    const int64_t wsb = ntg_convnd_workspace_bytes(dtype, batch, channels, out_channels, ndim, size, kernel_size, stride, padding, dilation, groups, 1);
+    // (Float32 takes the forms that follow the reference's order and reserves no more than those use)
+    const int64_t wsb = (dtype == ntg::DT_F32 ? ntg_convnd_workspace_bytes : ntg_convnd_fast_workspace_bytes)(
+        dtype, batch, channels, out_channels, ndim, size, kernel_size, stride, padding, dilation, groups, 1);
     ntg::HostSession mem;
     const size_t o_k = align_up(im_bytes, 256), o_g = o_k + align_up(k_bytes, 256), o_di = o_g + align_up(g_bytes, 256);
     const size_t o_dk = o_di + align_up(im_bytes, 256), o_ws = o_dk + align_up(k_bytes, 256);

@@ -514,7 +514,8 @@ def convnd(image, kernel, stride=1, padding=0, dilation=1, groups=1):
     L = load()
     dt = ntg_dtype(x)
     geo = (_i64arr(size), _i64arr(k), _i64arr(s), _i64arr(p), _i64arr(d))
-    ws_bytes = L.ntg_convnd_workspace_bytes(dt, B, C, O, nd, *geo, groups, 0)
+    # (one and two axes keep im2col's order of k here; conv1d and conv2d are their fast forms)
+    ws_bytes = (L.ntg_convnd_fast_workspace_bytes if nd == 3 else L.ntg_convnd_workspace_bytes)(dt, B, C, O, nd, *geo, groups, 0)
     if ws_bytes < 0:
         raise ValueError("invalid convolution geometry")
     y = torch.empty((B, O) + out, dtype=x.dtype, device=x.device)
@@ -540,7 +541,7 @@ def _convnd_gradients(image, kernel, grad, stride, padding, dilation, groups, wa
     L = load()
     dt = ntg_dtype(x)
     geo = (_i64arr(size), _i64arr(k), _i64arr(s), _i64arr(p), _i64arr(d))
-    ws_bytes = L.ntg_convnd_workspace_bytes(dt, B, C, O, nd, *geo, groups, 1)
+    ws_bytes = L.ntg_convnd_fast_workspace_bytes(dt, B, C, O, nd, *geo, groups, 1)
     if ws_bytes < 0:
         raise ValueError("invalid convolution geometry")
     dx, dw = torch.empty_like(x) if want_dx else None, torch.empty_like(w)

@@ -1112,7 +1112,7 @@ Tensor conv3d(const Tensor& image, const Tensor& kernel, utils::my_n_tuple<3> s,
     Tensor y({xv.B, O, out[0], out[1], out[2]}, x.dtype(), dev);
     const int dt = static_cast<int>(x.dtype());
     if (dev == DeviceType::HIP) {
-        const int64_t wsb = ntg_convnd_workspace_bytes(dt, xv.B, xv.C, O, 3, xv.size, wv.size, s.data(), p.data(), d.data(), groups, 0);
+        const int64_t wsb = ntg_convnd_fast_workspace_bytes(dt, xv.B, xv.C, O, 3, xv.size, wv.size, s.data(), p.data(), d.data(), groups, 0);
         utils::throw_exception(wsb >= 0, "conv3d output would be empty");
         check_status(ntg_convnd_dev(dt, x.data_ptr(), w.data_ptr(), y.data_ptr(), device_workspace(wsb), wsb, xv.B, xv.C, O, 3, xv.size, wv.size,
                                     s.data(), p.data(), d.data(), groups, nullptr));
@@ -1134,7 +1134,7 @@ ConvGrads conv3d_backward(const Tensor& image, const Tensor& kernel, const Tenso
     ConvGrads out{Tensor(image.shape(), x.dtype(), dev), Tensor(kernel.shape(), x.dtype(), dev)};
     const int dt = static_cast<int>(x.dtype());
     if (dev == DeviceType::HIP) {
-        const int64_t wsb = ntg_convnd_workspace_bytes(dt, xv.B, xv.C, wv.B, 3, xv.size, wv.size, s.data(), p.data(), d.data(), groups, 1);
+        const int64_t wsb = ntg_convnd_fast_workspace_bytes(dt, xv.B, xv.C, wv.B, 3, xv.size, wv.size, s.data(), p.data(), d.data(), groups, 1);
         utils::throw_exception(wsb >= 0, "conv3d backward: geometry has no output");
         check_status(ntg_convnd_backward_dev(dt, x.data_ptr(), w.data_ptr(), g.data_ptr(), out.d_image.data_ptr(), out.d_kernel.data_ptr(),
                                              device_workspace(wsb), wsb, xv.B, xv.C, wv.B, 3, xv.size, wv.size, s.data(), p.data(), d.data(), groups, 0, nullptr));

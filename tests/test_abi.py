@@ -117,6 +117,20 @@ def test_argument_errors_do_not_need_a_device():
     assert lib.ntg_convnd_workspace_bytes(_lib.FLOAT32, 2, 3, 4, 3, arr(5, 6, 7), arr(2, 3, 2), arr(1, 2, 1), arr(1, 0, 2), arr(2, 1, 1), 1, 0) == 0
     assert lib.ntg_convnd_workspace_bytes(_lib.INT32, 2, 3, 4, 3, arr(5, 6, 7), arr(2, 3, 2), arr(1, 2, 1), arr(1, 0, 2), arr(2, 1, 1), 1, 0) \
         == 2 * 3 * 12 * (5 * 2 * 10) * 4
+    # three axes: the reference's order without a copy of the image; the fast forms' copies have a query of their own
+    one = (arr(1, 1, 1), arr(1, 1, 1), arr(1, 1, 1))
+    assert lib.ntg_convnd_workspace_bytes(_lib.FLOAT32, 2, 32, 16, 3, arr(5, 6, 7), arr(3, 3, 3), *one, 1, 0) == 0
+    assert lib.ntg_convnd_fast_workspace_bytes(_lib.FLOAT32, 2, 32, 16, 3, arr(5, 6, 7), arr(3, 3, 3), *one, 1, 0) \
+        == 2 * 7 * 8 * 9 * 32 * 4 + 16 * 32 * 27 * 4
+    least = lib.ntg_convnd_workspace_bytes(_lib.FLOAT32, 2, 32, 16, 3, arr(5, 6, 7), arr(3, 3, 3), *one, 1, 1)
+    assert least == 2 * 16 * 32 * 27 * 4                                               # one weight gradient per image
+    assert lib.ntg_convnd_fast_workspace_bytes(_lib.FLOAT32, 2, 32, 16, 3, arr(5, 6, 7), arr(3, 3, 3), *one, 1, 1) > least
+    for size, k in (((9, 8), (3, 3)), ((9,), (3,))):                                   # one and two axes: the conv2d queries
+        geo, h, w = (arr(*size), arr(*k)) + tuple(arr(*[1] * len(k)) for _ in range(3)), (1,) * (2 - len(k)), len(k)
+        row = h + size + (16,) + h + k + (1, 1) + (0,) * len(h) + (1,) * w + (1, 1, 1)
+        assert lib.ntg_convnd_fast_workspace_bytes(_lib.FLOAT32, 2, 32, 16, w, *geo, 1, 0) == fast(_lib.FLOAT32, 2, 32, *row)
+    assert lib.ntg_convnd_fast_workspace_bytes(_lib.INT32, 2, 3, 4, 3, arr(5, 6, 7), arr(2, 3, 2), arr(1, 2, 1), arr(1, 0, 2), arr(2, 1, 1), 1, 0) \
+        == lib.ntg_convnd_workspace_bytes(_lib.INT32, 2, 3, 4, 3, arr(5, 6, 7), arr(2, 3, 2), arr(1, 2, 1), arr(1, 0, 2), arr(2, 1, 1), 1, 0)
     assert lib.ntg_convnd_workspace_bytes(_lib.FLOAT32, 2, 3, 4, 5, arr(5, 6, 7), arr(2, 3, 2), arr(1, 2, 1), arr(1, 0, 2), arr(2, 1, 1), 1, 0) == -1
     assert lib.ntg_convnd(_lib.FLOAT32, p, p, p, 1, 3, 4, 3, arr(5, 6, 7), arr(2, 3, 9), arr(1, 1, 1), arr(0, 0, 0), arr(1, 1, 1), 1) == 1
     assert b"sliding blocks" in lib.ntg_last_error()

@@ -159,3 +159,39 @@ def test_16_bit_strided_image_gradients_are_rounded_once(geom, dtype):
     dx, _ = F.conv2d_backward(x, w, g, stride=s, padding=p, groups=groups)
     want = exact_dx(size, w, g, k, s, p, (1, 1), groups)
     assert relative(dx, want) <= 1.1 * relative(want.to(dtype), want), (relative(dx, want), relative(want.to(dtype), want))
+
+
+def _arr(v):
+    return (ctypes.c_int64 * len(v))(*v)
+
+
+@pytest.mark.parametrize("geom", [
+    # (B, C, size, O, kernel, stride, padding, dilation, groups)
+    (2, 32, (6, 7, 8), 48, (3, 3, 3), (1, 1, 1), (1, 1, 1), (1, 1, 1), 1),
+    (3, 32, (5, 8, 12), 32, (3, 2, 3), (1, 2, 1), (1, 0, 1), (1, 1, 2), 2),
+    (1, 64, (8, 8, 8), 32, (2, 2, 2), (2, 2, 2), (0, 0, 0), (1, 1, 1), 1),
+    (70, 16, (4, 4, 4), 16, (3, 3, 3), (1, 1, 1), (1, 1, 1), (1, 1, 1), 1),   # the weight gradient's ranges fit into the smaller workspace
+], ids=lambda g: "x".join(map(str, g)))
+def test_fp32_three_axes_keep_the_reference_order_in_the_smaller_workspace(geom):
+    """Device calls with ntg_convnd_workspace_bytes of workspace sum in the order of the host entry points: the same bits.  Either
+    gradient alone takes the form that it takes beside the other."""
+    B, C, size, O, k, s, p, d, groups = geom
+    out = tuple((size[a] + 2 * p[a] - d[a] * (k[a] - 1) - 1) // s[a] + 1 for a in range(3))
+    x, w, g = randn((B, C) + size, torch.float32, 1), randn((O, C // groups) + k, torch.float32, 2, 0.05), randn((B, O) + out, torch.float32, 3)
+    hx, hw, hg = (t.cpu().numpy() for t in (x, w, g))
+    hy, hdx, hdw = np.empty((B, O) + out, np.float32), np.empty_like(hx), np.empty_like(hw)
+    vp = lambda a: a.ctypes.data_as(ctypes.c_void_p)
+    geo = tuple(_arr(v) for v in (size, k, s, p, d))
+    lib = _lib.load()
+    _lib.check(lib.ntg_convnd(_lib.FLOAT32, vp(hx), vp(hw), vp(hy), B, C, O, 3, *geo, groups))
+    _lib.check(lib.ntg_convnd_backward(_lib.FLOAT32, vp(hx), vp(hw), vp(hg), vp(hdx), vp(hdw), B, C, O, 3, *geo, groups, 0))
+    st = torch.cuda.current_stream().cuda_stream
+    fwd, bwd = (lib.ntg_convnd_workspace_bytes(_lib.FLOAT32, B, C, O, 3, *geo, groups, b) for b in (0, 1))
+    ws = torch.empty((max(fwd, bwd, 1),), dtype=torch.uint8, device=DEV)
+    y, dx, dw, dx1, dw1 = torch.empty((B, O) + out, device=DEV), torch.empty_like(x), torch.empty_like(w), torch.empty_like(x), torch.empty_like(w)
+    _lib.check(lib.ntg_convnd_dev(_lib.FLOAT32, x.data_ptr(), w.data_ptr(), y.data_ptr(), ws.data_ptr(), fwd, B, C, O, 3, *geo, groups, st))
+    for pdx, pdw in ((dx, dw), (dx1, None), (None, dw1)):
+        _lib.check(lib.ntg_convnd_backward_dev(_lib.FLOAT32, x.data_ptr(), w.data_ptr(), g.data_ptr(), None if pdx is None else pdx.data_ptr(),
+                                               None if pdw is None else pdw.data_ptr(), ws.data_ptr(), bwd, B, C, O, 3, *geo, groups, 0, st))
+    for got, want in ((y, hy), (dx, hdx), (dw, hdw), (dx1, hdx), (dw1, hdw)):
+        assert torch.equal(got.cpu(), torch.from_numpy(want))
