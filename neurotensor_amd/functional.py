@@ -28,9 +28,17 @@ def ntg_dtype(t):
         raise ValueError(f"dtype {t.dtype} has no matmult on this backend")
 
 
-def _stream():
-    """The current stream's handle (torch.cuda.current_stream() builds a Stream object first: 2.9 us of an 11 us call)."""
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+try:
+    # (torch.cuda.current_stream() builds a Stream object first: 2.9 us of an 11 us call.  Both names are private to torch.)
+    from torch._C import _cuda_getCurrentRawStream, _cuda_getDevice
+except ImportError:
+    def _stream():
+        """The current stream's handle."""
+        return torch.cuda.current_stream().cuda_stream
+else:
+    def _stream():
+        """The current stream's handle."""
+        return _cuda_getCurrentRawStream(_cuda_getDevice())
 
 
 def _require_device(*ts):

@@ -201,3 +201,17 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "libntgemm.so"))
     with pytest.raises(RuntimeError, match="not built"):
         _lib.load()
+
+
+def test_current_stream_without_the_private_names_of_torch(monkeypatch):
+    """functional takes the stream's handle from two private functions of torch; a torch without them serves the public way."""
+    import importlib
+
+    import torch
+
+    from neurotensor_amd import functional as F
+    with monkeypatch.context() as m:
+        m.delattr(torch._C, "_cuda_getCurrentRawStream")
+        m.setattr(torch.cuda, "current_stream", lambda: type("Stream", (), {"cuda_stream": 77})())
+        assert importlib.reload(F)._stream() == 77
+    importlib.reload(F)
