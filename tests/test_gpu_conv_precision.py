@@ -195,3 +195,83 @@ def test_fp32_three_axes_keep_the_reference_order_in_the_smaller_workspace(geom)
                                                None if pdw is None else pdw.data_ptr(), ws.data_ptr(), bwd, B, C, O, 3, *geo, groups, 0, st))
     for got, want in ((y, hy), (dx, hdx), (dw, hdw), (dx1, hdx), (dw1, hdw)):
         assert torch.equal(got.cpu(), torch.from_numpy(want))
+
+
+def exact_y(x, w, s, p, d, out, groups):
+    """The convolution in Float64: one product of matrices per tap and group."""
+    x, w = x.double(), w.double()
+    B, O = x.shape[0], w.shape[0]
+    cg, og = w.shape[1], O // groups
+    y = torch.zeros((B, O) + tuple(out), device=w.device, dtype=torch.float64)
+    for t, win in windows(x, w.shape[2:], s, p, d, out):
+        for gi in range(groups):
+            xg = win[:, gi * cg:(gi + 1) * cg].transpose(0, 1).reshape(cg, -1)
+            part = w[(slice(gi * og, (gi + 1) * og), slice(None)) + t].contiguous() @ xg
+            y[:, gi * og:(gi + 1) * og] += part.reshape((og, B) + tuple(out)).transpose(0, 1)
+    return y
+
+
+@pytest.mark.parametrize("geom,dtype", [
+    # (B, C, size, O, kernel, stride, groups), and the tiles that the planners choose:
+    ((4, 128, (32, 32, 32), 128, (3, 3, 3), 1, 1), torch.float32),      # 128 x 128 in all three
+    ((4, 128, (31, 33, 31), 128, (3, 3, 3), 1, 1), torch.float32),      # ... dY through its copy, outputs that end inside a tile
+    ((16, 128, (16, 16, 16), 128, (3, 3, 3), 2, 1), torch.float32),     # the phases 128 x 128
+    ((16, 64, (16, 16, 16), 256, (3, 3, 3), 1, 2), torch.float32),      # groups: forward 128 x 128
+    ((16, 32, (16, 16, 17), 256, (3, 3, 3), 1, 1), torch.bfloat16),     # forward 256 x 256 and the last 256 outputs on 64 x 64, dW 128 x 128
+    ((16, 256, (16, 16, 17), 32, (3, 3, 3), 1, 1), torch.float16),      # the same of the image gradient
+    ((16, 256, (16, 16, 16), 32, (3, 3, 3), 2, 1), torch.bfloat16),     # the phases 256 x 256
+    ((16, 128, (16, 16, 16), 32, (3, 3, 3), 2, 1), torch.float16),      # the phases 128 x 128
+    ((8, 256, (15, 17, 17), 256, (3, 3, 3), 1, 1), torch.bfloat16),     # 256 x 256 in all three, dY through its copy
+    ((24, 256, (16, 16, 16), 256, (1, 3, 3), 1, 1), torch.float16),     # 256 x 256, the last eight images 128 x 128; dW 256 x 256
+    ((16, 64, (16, 16, 16), 256, (3, 3, 3), 1, 2), torch.bfloat16),     # groups: 128 x 128 in all three
+], ids=str)
+def test_three_axes_on_the_large_tiles(geom, dtype):
+    """Three axes at sizes that reach the 128- and 256-row tiles of the channels-last kernels, against Float64.  16 bits: one
+    rounding (bound as above).  Float32: each of the K roundings of a sum of K random products errs by 2^-24 of a partial sum at most, which is
+    no larger than the results in the mean, and independent errors add up as sqrt(K): sqrt(K) * 2^-24 of the results' norm."""
+    B, C, size, O, k, s, groups = geom
+    p = tuple(i // 2 for i in k)
+    out = tuple((size[a] + 2 * p[a] - k[a]) // s + 1 for a in range(3))
+    x, w, g = randn((B, C) + size, dtype, 1), randn((O, C // groups) + k, dtype, 2, 0.05), randn((B, O) + out, dtype, 3)
+    y = F.conv3d(x, w, stride=s, padding=p, groups=groups)
+    dx, dw = F.conv3d_backward(x, w, g, stride=s, padding=p, groups=groups)
+    taps = k[0] * k[1] * k[2]
+    for name, got, exact, depth in (("y", y, lambda: exact_y(x, w, (s,) * 3, p, (1,) * 3, out, groups), C // groups * taps),
+                                    ("dx", dx, lambda: exact_dx(size, w, g, k, (s,) * 3, p, (1,) * 3, groups), O // groups * taps),
+                                    ("dw", dw, lambda: exact_dw(x, g, k, (s,) * 3, p, (1,) * 3, groups), B * out[0] * out[1] * out[2])):
+        want = exact()
+        bound = 2.0 ** -24 * depth ** 0.5 if dtype == torch.float32 else 1.1 * relative(want.to(dtype), want)
+        assert relative(got, want) <= bound, (name, relative(got, want), bound)
+        # (no element is off on its own: a misplaced one differs by about its neighbours' size)
+        worst = ((got.double() - want).abs().max() / want.square().mean().sqrt()).item()
+        assert worst <= (1e-6 * depth ** 0.5 if dtype == torch.float32 else 0.06), (name, worst)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("geom", [
+    # (B, C, size, O, kernel, stride, groups)
+    (2, 32, (6, 7, 8), 48, (3, 3, 3), 1, 1),
+    (3, 32, (9, 8, 11), 64, (3, 3, 3), 2, 2),
+], ids=str)
+def test_three_axes_gradients_add_to_what_is_there(geom, dtype):
+    """accumulate = 1 on the channels-last forms.  16 bits: Float32 sums with the incoming value in them, rounded once -- but the image
+    gradient at strides > 1 is rounded in its phase's plane first, an error of sqrt(1 + 1/2) of one rounding where both terms are of one
+    size; bounds of 1.1 times these.  Float32 as above."""
+    B, C, size, O, k, s, groups = geom
+    p = (1,) * 3
+    out = tuple((size[a] + 2 - k[a]) // s + 1 for a in range(3))
+    x, w, g = randn((B, C) + size, dtype, 1), randn((O, C // groups) + k, dtype, 2, 0.05), randn((B, O) + out, dtype, 3)
+    want_dx, want_dw = exact_dx(size, w, g, k, (s,) * 3, p, (1,) * 3, groups), exact_dw(x, g, k, (s,) * 3, p, (1,) * 3, groups)
+    dx0 = randn(x.shape, dtype, 4, want_dx.std().item())
+    dw0 = randn(w.shape, dtype, 5, want_dw.std().item())
+    dx, dw = dx0.clone(), dw0.clone()
+    lib, code = _lib.load(), F.ntg_dtype(x)
+    geo = tuple(_arr(v) for v in (size, k, (s,) * 3, p, (1,) * 3))
+    need = lib.ntg_convnd_fast_workspace_bytes(code, B, C, O, 3, *geo, groups, 1)
+    ws = torch.empty((need,), dtype=torch.uint8, device=DEV)
+    _lib.check(lib.ntg_convnd_backward_dev(code, x.data_ptr(), w.data_ptr(), g.data_ptr(), dx.data_ptr(), dw.data_ptr(), ws.data_ptr(), need,
+                                           B, C, O, 3, *geo, groups, 1, torch.cuda.current_stream().cuda_stream))
+    for name, got, want, depth, roundings in (("dx", dx, dx0.double() + want_dx, O // groups * 27, 1.5 if s > 1 else 1.0),
+                                              ("dw", dw, dw0.double() + want_dw, B * out[0] * out[1] * out[2], 1.0)):
+        bound = 2.0 ** -24 * depth ** 0.5 if dtype == torch.float32 else 1.1 * roundings ** 0.5 * relative(want.to(dtype), want)
+        assert relative(got, want) <= bound, (name, relative(got, want), bound)
