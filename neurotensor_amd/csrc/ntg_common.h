@@ -65,9 +65,8 @@ struct ConvGeom {
     // ... and k runs (64-byte run of channels, tap, channel inside the run) instead of (tap, channel): the taps of a run reach
     // the same pixels while they are in L2 (unit strides; the weights are permuted to match)
     int tap_inner;
-    // channels-last convolution and weight gradient: column n of this launch is column n + n_base of the whole product
-    // (a launch on the trailing columns); n_total = columns of the whole product (0: this launch has them all)
-    int n_base, n_total;
+    // channels-last convolution: column n of this launch is column n + n_base of the whole product (a launch on the trailing columns)
+    int n_base;
     // channels-last weight gradient, items = k ranges: the k axis is the output pixels of ALL images counted through (k_total of
     // them), item b covers pixels [b K, (b + 1) K) of it, the last one what is left (K is a whole number of K-steps).  The gathered
     // operand finds image and pixel by division (fold_L, fold_stride).  dY read where it lies as [image][out channel][pixel] (an image
@@ -82,7 +81,7 @@ struct ConvGeom {
     // channels-last convolution, several products in one launch: their table in device memory (see RingItem)
     const struct RingItem* items;
     int n_items;
-    int tile_edge;           // channels-last weight gradient: the tile the caller planned with (0: the launcher's own choice)
+    int tile_edge;           // channels-last weight gradient: the edge of the tile the caller planned with
 };
 
 struct GemmParams {
@@ -369,7 +368,7 @@ hipError_t launch_weights_channels_last_rows(int64_t es, const void* w, void* wp
 hipError_t launch_nchw_to_nhwc_padded(int64_t es, const void* in, void* out, int64_t batch, int64_t groups, int64_t cg, int64_t cgp, int64_t P, hipStream_t s,
                                       const HaloMap* halo = nullptr);
 hipError_t launch_flip_weights_channels_last(int64_t es, const void* w, void* wt, int64_t groups, int64_t og, int64_t ogp, int64_t cg, int64_t taps, hipStream_t s, int64_t chunk = 0);
-// channels-last convolution (image [B][pixel][C], weights [O][(r, q, c)]); F16 / BF16 / F32, two spatial axes
+// channels-last convolution (image [B][pixel][C], weights [O][(r, q, c)]); F16 / BF16 / F32, up to three spatial axes
 hipError_t launch_conv_nhwc(int dtype, const GemmParams& p, hipStream_t s);
 // Image gradient of a strided convolution as one stride-1 convolution per phase of the image (see conv_dimage_phases), up to
 // three axes, strides up to 4 (slowest axis first; two axes: everything of axis 0 is 1 or 0).  Phase (e0, e1, e2) is number

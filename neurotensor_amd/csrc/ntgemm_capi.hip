@@ -1621,7 +1621,7 @@ static double dkernel_cost_us(int64_t es, int edge, int64_t tiles, int64_t K) {
     }
     return 3.0 + k * std::max(0.009, 0.0042 * w);
 }
-// How dW is cut up: `ranges` k ranges of `kr` output pixels (0: one product per image), tiles of edge x edge (0: the launcher's choice), dY read where it
+// How dW is cut up: `ranges` k ranges of `kr` output pixels (0: one product per image), tiles of edge x edge, dY read where it
 // lies (its rows 16-byte multiples, an image a whole number of K-steps) or through a channels-last copy of its own (the out
 // channels of a group a 16-byte multiple; any range then).  The partial sums are Float32 whatever the type, so that a 16-bit gradient
 // is rounded once (rounded to 16 bits each, they left sqrt(2) of one rounding's error in the sum: BFloat16 2 x 256 x 32 x 32 -> 1024
@@ -1647,16 +1647,13 @@ static DkernelPlan plan_dkernel(int dtype, int64_t batch, int64_t channels, int6
     const bool lies = rows_16 && L % bk == 0 && countable, copied = og_16 && countable;
     if (!rows_16 && !copied) return pl;
     pl.ok = true;
-    pl.items = batch;
     // measurement and test knob: NTG_DW_RANGES=r forces r ranges of dY where it lies where r is admissible, 0 one product per image
-    const char* env = std::getenv("NTG_DW_RANGES");
-    if (env && rows_16) {
-        const int64_t r = std::atoll(env);
-        if (lies && r > 0 && steps % r == 0) {
-            pl.ranges = pl.items = r;
-            pl.kr = total / r;
-            pl.edge = es == 2 ? ntg::ring16_tile_edge(og, N, pl.kr, r) : 64;
-        }
+    const char* env = rows_16 ? std::getenv("NTG_DW_RANGES") : nullptr;
+    const int64_t forced = env ? std::atoll(env) : 0;
+    if (lies && forced > 0 && steps % forced == 0) {
+        pl.ranges = pl.items = forced;
+        pl.kr = total / forced;
+        pl.edge = es == 2 ? ntg::ring16_tile_edge(og, N, pl.kr, forced) : 64;
     } else {
         // A range has the pixels of an image at least, where those are two to eight K-steps: it is one Float32 chain, and over small maps
         // ranges longer than the reference's chains cost time -- groups run one behind the other -- and digits (22 x 23 x 69 -> 4 by 5 at
@@ -1676,6 +1673,7 @@ static DkernelPlan plan_dkernel(int dtype, int64_t batch, int64_t channels, int6
         for (int edge : {256, 128, 64}) {
             if (es == 4 && edge == 256) continue;
             if (rows_16) consider(false, 0, batch, L, edge);
+            if (env) continue;
             const int64_t tiles = ((og + edge - 1) / edge) * ((N + edge - 1) / edge) * groups;
             for (int64_t target : {256, 512, 768, 1024, 1536, 2048}) {
                 const int64_t want = std::min(std::max<int64_t>(target / tiles, 1), std::max<int64_t>(steps / shortest, 1));
