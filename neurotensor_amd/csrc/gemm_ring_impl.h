@@ -202,8 +202,12 @@ __device__ __forceinline__ uint32_t lds_addr_of(const char* p) {
 // on the smaller tiles, so that two workgroups still share a CU)
 constexpr int dw_table_entries(int wb) { return wb == 4 ? 6144 : 3584; }
 
+// Wavefronts per SIMD that an instantiation must leave room for (0: as the compiler sees fit): the 128 x 128 weight gradient in Float32 holds a
+// second set of sums (SEGMENTS below) and, unasked, takes a few registers more than two workgroups a CU can have.
+constexpr int ring_min_waves(int dt, int wb, int conv) { return dt == DT_F32 && wb == 2 && (conv == 4 || conv == 7) ? 2 : 0; }
+
 template <int DT, bool TA, bool TB, bool RAGGED, int WB_, int CONV = 0, int WBN_ = 0, int KD_ = 1>
-__global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams pin) {
+__global__ void __launch_bounds__(256, ring_min_waves(DT, WB_, CONV)) gemm_ring_kernel(const GemmParams pin) {
     using E = Elem<DT>;
     using T = typename E::T;
     constexpr int ES = sizeof(T);
@@ -1021,6 +1025,33 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams pin) {
       }
     };
 
+    // Float32 weight gradients and image gradients by phases: the chain ends every p.conv.k_segment K-steps (a power of two, 0: never) and its
+    // sum is added to the sum of the chains before it.  One chain through all pixels, or all taps and out channels, errs by sqrt(K) roundings
+    // of partial sums that grow to the result's size, where a product per image, or per tap, added up errs by far less
+    // (Float32 7 x 128 x 8^3 -> 48 by 3 x 3 x 3 at stride 2: 2.4e-7 from the exact image gradient against 1.3e-7).  The additions hide behind
+    // the other wavefronts' matrix instructions: 4 x 32 x 32^3 -> 64 by 3 x 3 x 3, a step of 531 us before, 528 with them.
+    constexpr bool SEGMENTS = (ITEMS || GATHERW) && ES == 4;
+    float sum[SEGMENTS ? WBM : 1][SEGMENTS ? WBN : 1][16] = {};
+    const int segment_mask = SEGMENTS ? p.conv.k_segment - 1 : 0;
+    auto end_segment = [&](int kt) __attribute__((always_inline)) {
+        if constexpr (SEGMENTS) {
+            if (((kt + 1) & segment_mask) == 0) {                  // (uniform)
+#pragma unroll
+                for (int i = 0; i < WBM; ++i)
+#pragma unroll
+                    for (int j = 0; j < WBN; ++j)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            // (one element after the other: read out together, the accumulators would take their number of registers once more)
+                            float t = acc[i][j][r];
+                            asm volatile("" : "+v"(t));
+                            sum[i][j][r] += t;
+                            asm volatile("" : "+v"(sum[i][j][r]));
+                            acc[i][j][r] = 0.0f;
+                        }
+            }
+        }
+    };
     if constexpr (RING3) {
         for (int kt = 0; kt < KT; kt += 3) {
             iteration_deep3(kt, st0, st1, st2);
@@ -1036,10 +1067,22 @@ __global__ void __launch_bounds__(256) gemm_ring_kernel(const GemmParams pin) {
             if (kt + 3 < KT) iteration_deep(kt + 3, st3, st0, st2);
         } else {
             iteration(kt, st0, st1, st3);
+            end_segment(kt);
             if (kt + 1 < KT) iteration(kt + 1, st1, st2, st0);
+            end_segment(kt + 1);
             if (kt + 2 < KT) iteration(kt + 2, st2, st3, st1);
+            end_segment(kt + 2);
             if (kt + 3 < KT) iteration(kt + 3, st3, st0, st2);
+            end_segment(kt + 3);
         }
+    }
+    if constexpr (SEGMENTS) {
+#pragma unroll
+        for (int i = 0; i < WBM; ++i)
+#pragma unroll
+            for (int j = 0; j < WBN; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[i][j][r] += sum[i][j][r];
     }
     NTG_WAIT_VMCNT(0);              // clamped tail DMAs have landed
     __builtin_amdgcn_s_barrier();   // all fragment reads done: LDS is free for the epilogue

@@ -81,6 +81,7 @@ struct ConvGeom {
     // channels-last convolution, several products in one launch: their table in device memory (see RingItem)
     const struct RingItem* items;
     int n_items;
+    int k_segment;           // Float32 weight gradients and `items`: K-steps of one chain of multiply-adds (a power of two; 0: all of them)
     int tile_edge;           // channels-last weight gradient: the edge of the tile the caller planned with
 };
 

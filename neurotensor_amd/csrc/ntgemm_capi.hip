@@ -1445,6 +1445,14 @@ static int conv_dimage_nhwc(int dtype, const void* kernel, const void* grad_out,
     return NTG_OK;
 }
 
+// Float32: K-steps (16 multiply-adds) of one chain in a gathered product that stands for shorter ones of `n` multiply-adds each, added
+// up: the largest power of two within n, from one K-step to sixteen (256 multiply-adds; longer chains gain no time).
+static int chain_steps(int64_t n) {
+    int steps = 1;
+    while (steps < 16 && 32 * steps <= n) steps *= 2;
+    return steps;
+}
+
 // dX of a convolution with strides > 1 (dilation 1), without the col matrix: the image positions y with (y + p) mod s = e
 // form one phase; they receive only the taps i = e + s m (m = 0 .. M_e - 1), and, with a = (y + p) / s,
 //   dX[y] = sum_m dY[a - m] W[e + s m],
@@ -1582,6 +1590,7 @@ static int conv_dimage_phases(int dtype, const PhasePlan& pp, const void* kernel
     p.conv.k_drc = 1;                                      // (the items set their own taps; k runs taps-inner, which does not use it)
     p.conv.halo = 1; p.conv.tap_inner = 1;
     p.conv.items = items; p.conv.n_items = q.phases * (int)groups;
+    if (g.nd == 3) p.conv.k_segment = chain_steps(og);
     e = ntg::launch_conv_nhwc_items(dtype, pp.edge, p, pp.blocks, hs);
     if (e != hipSuccess) return hip_fail(e, "phase convolution launch");
     e = ntg::launch_phase_interleave(dtype, ws_tmp, d_image, q, accumulate, hs);
@@ -1655,10 +1664,9 @@ static DkernelPlan plan_dkernel(int dtype, int64_t batch, int64_t channels, int6
         pl.kr = total / forced;
         pl.edge = es == 2 ? ntg::ring16_tile_edge(og, N, pl.kr, forced) : 64;
     } else {
-        // A range has the pixels of an image at least, where those are two to eight K-steps: it is one Float32 chain, and over small maps
-        // ranges longer than the reference's chains cost time -- groups run one behind the other -- and digits (22 x 23 x 69 -> 4 by 5 at
-        // stride 3: 1.2e-7 from the exact gradient in chains of one image, 2.1e-7 in three ranges of 176 pixels), while shorter ones
-        // ask for a larger workspace than one gradient per image.
+        // A range has the pixels of an image at least, where those are two to eight K-steps: over small maps longer ranges are few and cost
+        // time, as the groups run one behind the other (58 x 64 x 17 -> 64 by 5 in 8 groups: backward 136 us, 108 with short ranges), while
+        // shorter ones ask for a larger workspace than one gradient per image.
         const int64_t shortest = std::min<int64_t>(8, std::max<int64_t>(2, (L + bk - 1) / bk));
         double best = 0.0;
         const auto consider = [&](bool copy, int64_t ranges, int64_t items, int64_t kr, int edge) {
@@ -1733,6 +1741,7 @@ static int conv_dkernel_nhwc(int dtype, const DkernelPlan& pl, const void* image
         p.conv.halo = halo.on ? 1 : 0;
         if (halo.on && g.nd == 2 && L < (1 << 20) && (pl.ranges == 0 || L % bk == 0)) p.conv.pix_table = (int)L;     // (a K-step inside one image: see the kernel)
         p.conv.tile_edge = pl.edge;
+        p.conv.k_segment = chain_steps(L);
         if (pl.ranges) {
             p.conv.k_ranges = 1;
             p.conv.k_total = (int)(batch * L);
