@@ -1461,7 +1461,7 @@ static int chain_steps(int64_t n) {
 // workspace; a last pass interleaves the planes into dX.  Exactly the products of the reference's GEMM + col2im, none wasted on
 // the zeros a dilated gradient would hold.  All phases (and groups) are items of ONE launch: a phase alone is a small product
 // (32 x 64 x 56 x 56 by 4 x 4 at stride 2: 416 tiles of k = 512), and four launches with a weight permutation each took 58 us
-// where the one takes 20.
+// where the one takes 25 and the set-up of all phases' weights 8.
 struct PhasePlan {
     bool ok;
     int edge;
@@ -1606,22 +1606,26 @@ static int64_t dkernel_padded_channels(int64_t es, int64_t cg) { const int64_t v
 static HaloPlan dkernel_halo(int64_t es, int64_t cg, int64_t groups, const Geo3& g) {
     HaloPlan h = conv_halo(g);
     const int64_t cgp = dkernel_padded_channels(es, cg);
-    // (a copy that pads the channels grows by its border as well: on one and two axes only where that is a quarter of it at most, as
-    //  it is from 17 x 17 pixels on for a 3 x 3 window; smaller planes keep the validity tests and their workspace)
+    // (a copy that pads the channels grows by its border as well, which takes a launch of its own: on one and two axes only where the border
+    //  is a quarter of the image at most, as it is from 17 x 17 pixels on for a 3 x 3 window.  Validity tests against the border, us per
+    //  weight gradient: Float32 64 x 3 x 16 x 16 -> 64 by 3 x 3 20.1 | 23.1, 256 x 6 x 16 x 16 -> 96 35.9 | 36.5, 64 x 60 x 16 x 16 -> 128
+    //  41.9 | 41.9, 256 x 3 x 32 x 32 -> 64 by 5 x 5 56.2 | 55.3; BFloat16 20.4 | 23.2, 20.3 | 23.0, 25.2 | 27.7, 37.6 | 37.7)
     const bool wide_border = g.nd < 3 && cgp != cg && 4 * h.vol > 5 * g.vol();
     if (h.on && (wide_border || !conv_nhwc_offsets_fit(groups * cgp, es, h.gp))) {
         h.on = false; h.gp = g; h.vol = g.vol();
     }
     return h;
 }
-// What a launch of the gathering kernel takes, from the timings of the layers below: microseconds for `tiles` tiles of
-// edge x edge with K output pixels each, by how many workgroups share a CU.  16-bit: 0.41 of a CU's MFMA peak on 256 x 256 tiles;
-// 0.35 on 128 x 128 tiles when two workgroups share a CU, 0.245 when one has it alone; a 64 x 64 tile alone on its CU
-// takes 9 ns per pixel, several of them 4.2 ns each.  Float32: 27 ns per pixel for a 64 x 64 tile alone, 15.4 ns each for
-// several; 128 x 128: 70 and 60.
+// What a launch of the gathering kernel takes: microseconds for `tiles` tiles of edge x edge with K output pixels each, by how many
+// workgroups share a CU; the writes of the partial sums are the caller's.  Float32, from profiles/conv_weight_gradient_gather_sweep.txt without
+// those writes (4.7 TB/s): 8 us and, per pixel, 29 ns for a 64 x 64 tile alone on its CU, 22 ns each for several; 128 x 128: 79 and 68, so large
+// tiles where the gradient has the rows and columns for them (64 x 128 x 28 x 28 -> 128 by 3 x 3, a step: 438 us on
+// 64 x 64 tiles, 419).  16-bit: 0.41 of a CU's MFMA
+// peak on 256 x 256 tiles; 0.35 on 128 x 128 tiles when two workgroups share a CU, 0.245 when one has it alone; a 64 x 64 tile 9 ns per
+// pixel alone, 4.2 ns each for several, and 3 us (the sweep reads 0.46, 0.41, 0.29, 7.5 and 5.1 ns, and 8 us).
 static double dkernel_cost_us(int64_t es, int edge, int64_t tiles, int64_t K) {
     const double w = (double)((tiles + 255) / 256), k = (double)K;
-    if (es == 4) return edge == 128 ? 4.0 + k * std::max(0.070, 0.060 * w) : 3.0 + k * std::max(0.027, 0.0154 * w);
+    if (es == 4) return 8.0 + k * (edge == 128 ? std::max(0.079, 0.068 * w) : std::max(0.029, 0.022 * w));
     const double cu_flops_per_us = 9.77e6, area = (double)edge * edge;
     if (edge == 256) return w * (2.0 * area * k / (cu_flops_per_us * 0.41) + 6.0);
     if (edge == 128) {
@@ -1840,8 +1844,10 @@ static ConvBackwardPlan plan_conv_backward_g(int dtype, bool want_dx, bool want_
     pl.need_phase_dx = pl.phase_dx ? pl.phases.bytes() : 0;
     // strides > 1 on few channels: W^T . dY + col2im.  W_g is stored [og][channels of the group * taps]; where those rows miss the
     // 16-byte rule (3 channels by 7 x 7: 147) the product would go to the register-staged kernel, so W is copied to [..][og] behind the col matrix
-    // and dY and col, whose rows keep the rule, stay where they are.  Float32 32 x 3 x 224 x 224 from 7 x 7 at stride 2, 64 out channels
-    // (3.8 * 10^9 multiply-adds, 236 MB written): 203 us there, 152 us here and 9 us for the copy -- the two meet at 0.65 * 10^9: from 2^30 on.
+    // and dY and col, whose rows keep the rule, stay where they are.  From 2^30 multiply-adds on, where every layer timed gains; us per backward
+    // call as stored | transposed, at n * 2^30 multiply-adds: Float32 3 x 224 x 224 -> 64 by 7 x 7 at stride 2 n = 0.22 57 | 57, 0.44 80 | 73,
+    // 1.76 214 | 181, 3.52 405 | 352; 3 x 256 x 256 -> 32 by 5 x 5 0.29 76 | 78, 1.17 237 | 230; BFloat16 0.22 49 | 48, 1.76 213 | 128, 3.52 362 | 209.
+    // (The two meet near 0.25: between that and 2^30 the copy would gain up to a third.)
     pl.wt_offset = (int64_t)align_up((size_t)col, 256);
     const int64_t og = out_channels / groups, add = cg * taps;
     const bool wt = want_dx && !pl.gather_dx && !pl.phase_dx && !reference_order && g.nd <= 2 &&

@@ -309,3 +309,18 @@ def test_fp32_gradients_are_as_close_as_sums_per_tap_and_per_image(geom):
     for name, got, host, want in checks:
         ours, reference = relative(got, want), relative(torch.from_numpy(host).to(DEV), want)
         assert ours <= 1.15 * reference, (name, ours, reference)
+
+
+def test_fp32_weight_gradient_takes_the_large_tiles_where_they_are_faster(monkeypatch):
+    """128 x 128 tiles take 77 % of the time of four 64 x 64 ones (profiles/conv_weight_gradient_gather_sweep.txt): the planned gradient of this
+    layer is faster than fourteen ranges on 64 x 64 tiles (the knob's tile), which a plan that charged both alike chose; by 15 % without
+    the copy of the image."""
+    x, w, g = (randn(s, torch.float32, i) for i, s in enumerate(((64, 128, 28, 28), (128, 128, 3, 3), (64, 128, 28, 28))))
+    call = lambda: F._conv2d_gradients(x, w, g, 1, 1, 1, 1, want_dx=False)[1]
+    planned, small = [], []
+    for _ in range(2):
+        monkeypatch.delenv("NTG_DW_RANGES", raising=False)
+        planned.append(microseconds(call))
+        monkeypatch.setenv("NTG_DW_RANGES", "14")
+        small.append(microseconds(call))
+    assert min(planned) <= 0.96 * min(small), (planned, small)
