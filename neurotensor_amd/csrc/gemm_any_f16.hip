@@ -1,0 +1,5 @@
+// Float16 instantiations of the product on rows that start anywhere.
+#include "gemm_any_impl.h"
+namespace ntg {
+hipError_t launch_gemm_any_f16(bool ta, bool tb, const GemmParams& p, hipStream_t s) { return launch_any<DT_F16>(ta, tb, p, s); }
+}  // namespace ntg

@@ -102,6 +102,7 @@ struct GemmParams {
     // A and B of it lie at item * sA + range * sAk (sB, sBk); C (the partial sums) at b * sC.  0: a plain batch.
     int krange_items;
     int64_t sAk, sBk;
+    int k_total;             // k ranges of unequal length (gemm_any_impl.h): K is a range's length, the last one has what is left of k_total; 0: all equal
     int M, N, K, batch;      // logical sizes (after the transpose flags)
     int cmode;
     int tiles_m, tiles_n;
@@ -189,6 +190,13 @@ static inline int ring16_tile_edge(int64_t M, int64_t N, int64_t K, int64_t batc
     return best;
 }
 
+// Products on rows that start anywhere: every contiguous extent holds a 16-byte chunk, 32-bit lane offsets (128 rows below 1 GiB).
+static inline bool any_eligible(const GemmParams& p, int dtype, bool ta, bool tb) {
+    const int es = dtype == DT_F32 ? 4 : dtype == DT_F16 || dtype == DT_BF16 ? 2 : dtype == DT_I8 || dtype == DT_U8 ? 1 : 0;
+    if (es == 0) return false;
+    const int64_t vel = 16 / es, ldmax = (int64_t)(1 << 23) / es;
+    return p.K > 0 && (ta ? p.M : p.K) >= vel && (tb ? p.K : p.N) >= vel && p.lda < ldmax && p.ldb < ldmax;
+}
 // A batched product whose tiles fill the 256 CUs a whole number of times plus a small rest would spend a full tile time
 // on that rest.  The plan then gives the first `head` items the chosen tile (as many as fit in whole rounds) and the
 // remaining ones a tile chosen for them alone (usually the next smaller one, spread over all CUs), as two launches; the
@@ -311,6 +319,8 @@ hipError_t launch_gemm_mfma(int dtype, bool ta, bool tb, const GemmParams& p, hi
 // epilogue applies GemmParams::act
 hipError_t launch_gemm_ring_only(int dtype, bool ta, bool tb, const GemmParams& p, hipStream_t s, bool* taken);
 // C[b][m][n] = max(C[b][m][n], 0) in place (floating dtypes)
+// Float16 / BFloat16 / Float32 / Int8 on rows that start anywhere (gemm_any_impl.h); the caller has checked any_eligible()
+hipError_t launch_gemm_any(int dtype, bool ta, bool tb, const GemmParams& p, hipStream_t s);
 hipError_t launch_relu_inplace(int dtype, void* C, int64_t ldc, int64_t sC, int64_t M, int64_t N, int64_t batch, hipStream_t s);
 hipError_t launch_gemm_valu(int dtype, bool ta, bool tb, const GemmParams& p, hipStream_t s);
 hipError_t launch_gemm_mfma_i8(int dtype, bool ta, bool tb, const GemmParams& p, hipStream_t s);   // Int8 / UInt8: MFMA where rows are 16-byte multiples
@@ -340,7 +350,8 @@ hipError_t launch_unfoldnd(int64_t elem_size, const void* im, void* col, const U
 hipError_t launch_col2imnd(int dtype, const void* col, void* im, const UnfoldNdParams& u, int accumulate, hipStream_t s);
 
 // split-K: out (+)= sum over s of part[s] (s ascending), fp32 accumulation for the 16-bit dtypes whose partials are float
-hipError_t launch_splitk_reduce(int dtype, const void* part, int splits, const GemmParams& p, hipStream_t s);
+// (rows of the partial sums lie ldp elements apart)
+hipError_t launch_splitk_reduce(int dtype, const void* part, int splits, const GemmParams& p, int64_t ldp, hipStream_t s);
 
 // conv2d backward helpers (unfold2d.hip): ordered sum of per-image weight gradients; weights of
 // the gradient-to-image convolution

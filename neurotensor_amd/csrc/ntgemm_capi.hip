@@ -38,6 +38,19 @@ hipError_t launch_gemm_ring_only(int dtype, bool ta, bool tb, const GemmParams& 
     default: return hipSuccess;
     }
 }
+hipError_t launch_gemm_any_f32(bool ta, bool tb, const GemmParams& p, hipStream_t s);
+hipError_t launch_gemm_any_f16(bool ta, bool tb, const GemmParams& p, hipStream_t s);
+hipError_t launch_gemm_any_bf16(bool ta, bool tb, const GemmParams& p, hipStream_t s);
+hipError_t launch_gemm_any_i8(bool ta, bool tb, const GemmParams& p, hipStream_t s);
+hipError_t launch_gemm_any(int dtype, bool ta, bool tb, const GemmParams& p, hipStream_t s) {
+    switch (dtype) {
+    case DT_I8: case DT_U8: return launch_gemm_any_i8(ta, tb, p, s);
+    case DT_F32: return launch_gemm_any_f32(ta, tb, p, s);
+    case DT_F16: return launch_gemm_any_f16(ta, tb, p, s);
+    case DT_BF16: return launch_gemm_any_bf16(ta, tb, p, s);
+    default: return hipErrorInvalidValue;
+    }
+}
 hipError_t launch_conv_mfma_f32(bool tb, int nd, const GemmParams& p, hipStream_t s);
 hipError_t launch_conv_mfma_f64(bool tb, int nd, const GemmParams& p, hipStream_t s);
 hipError_t launch_conv_mfma_f16(bool tb, int nd, const GemmParams& p, hipStream_t s);
@@ -175,6 +188,10 @@ int launch_gemm(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s) {
             e = ntg::launch_gemm_ring_only(dtype, ta, tb, q, s, &taken);
             if (e != hipSuccess) return hip_fail(e, "gemm launch");
             if (taken) return NTG_OK;
+            if (ntg::any_eligible(p, dtype, ta, tb)) {
+                e = ntg::launch_gemm_any(dtype, ta, tb, q, s);
+                return e == hipSuccess ? NTG_OK : hip_fail(e, "gemm launch");
+            }
         }
     }
     const auto finish = [&]() -> int {
@@ -297,7 +314,7 @@ static int run_int_planes(const ntg::GemmParams& p, const IntPlanesPlan& pl, boo
 // single rounding for the 16-bit floats), the product runs on the DMA-fed kernel, and a result whose own rows are not
 // 16-byte multiples is computed into a padded copy and copied back.  Taken for products large enough to repay the copies.
 struct PadPlan {
-    bool ok, padA, padB, padC;
+    bool ok, pays, padA, padB, padC;   // ok: it can be done; pays: nothing else is faster
     bool stripA, stripB;            // the operand stays where it is, only its last k-rows are copied (and continued with zeros)
     int strip_k0, strip_rows;
     int Mp, Kp, Np;
@@ -311,8 +328,8 @@ static PadPlan plan_pad(const ntg::GemmParams& p, int dtype, bool ta, bool tb) {
     const bool wide = dtype == ntg::DT_F32 || dtype == ntg::DT_F64;
     if ((!half && !byte && !wide) || p.Aptr || p.Bptr || p.Cptr || p.M <= 32) return pl;
     const int64_t es = ntg::elem_size(dtype), ve = 16 / es;
-    // from where the faster kernel repays the copies: 8-bit against the vector ALU (40 x), 16-bit against the register-staged
-    // kernel at half the rate, Float32 / Float64 against the register-staged kernel at 0.8 - 0.85 of the DMA-fed one
+    // From where a faster kernel repays the copies: 8-bit against the vector ALU (40 x), 16-bit against the register-staged
+    // kernel at half the rate, Float32 / Float64 against the register-staged kernel at 0.8 - 0.85 of the DMA-fed one.
     const double macs = (double)p.M * p.N * p.K * p.batch;
     if (macs < (byte ? 268435456.0 : half ? 2147483648.0 : dtype == ntg::DT_F32 ? 4294967296.0 : 8589934592.0)) return pl;
     auto up = [&](int64_t v) { return (v + ve - 1) / ve * ve; };
@@ -346,6 +363,11 @@ static PadPlan plan_pad(const ntg::GemmParams& p, int dtype, bool ta, bool tb) {
     if (pl.padB) pl.b_bytes = (int64_t)align_up((size_t)((p.sB == 0 ? 1 : p.batch) * pl.rowsB2 * pl.ldb2 * es), 256);
     if (pl.padC) pl.c_bytes = (int64_t)align_up((size_t)((int64_t)p.batch * pl.Mp * pl.Np * es), 256);
     pl.ok = true;
+    // The kernel that takes rows as they lie (gemm_any_impl.h) makes whole copies pay later; where only the last k-rows are copied they are as good
+    // as free.  Copies against no copies: Float16 1023 x 1537 x 2049 (3.2e9) 31.0 us against 31.3, BFloat16 2813 x 803 x 2240 (5.1e9) 29.2 against 26.7,
+    // 2049^3 (8.6e9) 51.1 against 51.8, 3618 x 739 x 9392 (2.5e10) 79 against 96; Float32 2049^3 211 against 187, 1504 x 727 x 8952 (9.8e9) 180 against
+    // 191; Int8 2049^3 36.6 against 33.9, 1002 x 256 x 2432 12.2 against 7.5.  (The workspace is offered as if they paid: what a caller keeps stays enough.)
+    pl.pays = !(pl.padA || pl.padB || pl.padC) || !ntg::any_eligible(p, dtype, ta, tb) || macs >= (byte ? 1.7e10 : half ? 3.0e9 : dtype == ntg::DT_F32 ? 9.0e9 : 0.0);
     return pl;
 }
 static int run_padded(const ntg::GemmParams& p, const PadPlan& pl, int dtype, bool ta, bool tb, void* ws, hipStream_t s) {
@@ -458,6 +480,42 @@ SplitPlan plan_splitk(const ntg::GemmParams& p, int dtype, bool ta) {
     return none;
 }
 
+// k ranges of a product whose rows miss the 16-byte rule by their SIZES (gemm_any_impl.h serves it): as plan_splitk a function of one item's
+// sizes and pitches only.  kc is a whole number of K-steps, the last range is what is left.  Rows of the partial sums hold whole 16-byte chunks.
+struct AnySplitPlan { int splits; int64_t kc, ldp, bytes; };
+AnySplitPlan plan_any_split(const ntg::GemmParams& p, int dtype, bool ta, bool tb) {
+    AnySplitPlan none{1, p.K, 0, 0};
+    if (p.batch < 1 || p.batch > 65535 || p.Aptr || p.Bptr || p.Cptr || p.keep_k_order || !ntg::any_eligible(p, dtype, ta, tb)) return none;
+    const bool byte = dtype == ntg::DT_I8 || dtype == ntg::DT_U8;
+    if (p.M <= 32 && !byte) return none;                           // the streaming kernels take these
+    const int64_t es = ntg::elem_size(dtype), ve = 16 / es, bk = 128 / es;
+    if (p.K % ve == 0 && p.N % ve == 0 && (!ta || p.M % ve == 0) && p.lda % ve == 0 && p.ldb % ve == 0 && p.ldc % ve == 0) return none;
+    const int64_t tiles = ((p.M + 63) / 64) * ((p.N + 63) / 64), steps = (p.K + bk - 1) / bk;
+    if (tiles > 255) return none;
+    // A workgroup alone on its CU spends 0.28 / 0.71 / 0.43 us (16-bit / Float32 / Int8) on each K-step, several on one CU 0.18 / 0.45 / 0.25 us
+    // each; a launch costs about 2.5 us, the second pass 4 us + the partial sums written and read at 4 TB/s.  Of 2 .. 32 ranges the choice was the
+    // best measured one or within 10 % of it on fourteen shapes (BFloat16 576 x 3797 x 448, ranges 1 / 2 / 4 / 8: 19.6 / 16.5 / 13.0 / 14.5 us;
+    // 448 x 3704 x 166: 25.9 us whole, 10.4 in eight ranges; Float32 128 x 6463 x 720: 146 us whole, 24 in 21 ranges).
+    const double alone = byte ? 0.43 : es == 2 ? 0.28 : 0.71, shared = byte ? 0.25 : es == 2 ? 0.18 : 0.45;
+    auto estimate_us = [&](int64_t sp, int64_t per) {
+        const int64_t wgs = tiles * sp;
+        const double second_pass = sp == 1 ? 0.0 : 4.0 + 8.0 * (double)sp * (double)p.M * (double)p.N / 4.0e6;
+        return 2.5 + (double)per * (wgs <= 256 ? alone : shared * (double)((wgs + 255) / 256)) + second_pass;
+    };
+    const double whole_us = estimate_us(1, steps);
+    double best_us = 0.95 * whole_us;
+    AnySplitPlan pl = none;
+    for (int64_t sp = 2; sp <= 32 && sp <= steps / 2; ++sp) {
+        const int64_t per = (steps + sp - 1) / sp, ranges = (steps + per - 1) / per;
+        const double us = estimate_us(ranges, per);
+        if (us < best_us) { best_us = us; pl.splits = (int)ranges; pl.kc = per * bk; }
+    }
+    if (pl.splits < 2) return none;
+    pl.ldp = (p.N + 3) / 4 * 4;
+    pl.bytes = (int64_t)pl.splits * p.batch * p.M * pl.ldp * 4;
+    return pl;
+}
+
 int run_gemm(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s, void* workspace = nullptr, int64_t workspace_bytes = 0) {
     const int64_t es = ntg::elem_size(dtype);
     if (es == 0) return fail(NTG_ERR_UNSUPPORTED_DTYPE, "dtype %d is not supported by the gfx950 matmult backend", dtype);
@@ -477,7 +535,7 @@ int run_gemm(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s, void
                 q.batch = 1;
                 q.C = static_cast<char*>(p.C) + (int64_t)b * p.sC * es;
                 if (p.bias) q.bias = static_cast<const char*>(p.bias) + (int64_t)b * p.bias_bs * es;
-                e = ntg::launch_splitk_reduce(dtype, nullptr, 0, q, s);     // C0 plus no partial sums
+                e = ntg::launch_splitk_reduce(dtype, nullptr, 0, q, q.N, s);     // C0 plus no partial sums
             }
         }
         if (e != hipSuccess) return hip_fail(e, "empty-k launch");
@@ -489,8 +547,32 @@ int run_gemm(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s, void
             return run_int_planes(p, ip, ta, tb, workspace, s);
     }
     {
+        const AnySplitPlan ap = plan_any_split(p, dtype, ta, tb);
+        if (ap.splits > 1 && workspace && workspace_bytes >= ap.bytes && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0) {
+            // launch index = range * batch + item
+            ntg::GemmParams q = p;
+            q.K = (int)ap.kc;
+            q.k_total = p.K;
+            q.C = workspace;
+            q.ldc = ap.ldp;
+            q.sC = (int64_t)p.M * ap.ldp;
+            q.cmode = ntg::C_PARTIAL;
+            q.bias = nullptr;
+            q.act = ntg::ACT_NONE;
+            q.batch = ap.splits * p.batch;
+            q.krange_items = p.batch;
+            q.sAk = ta ? ap.kc * p.lda : ap.kc;
+            q.sBk = tb ? ap.kc : ap.kc * p.ldb;
+            hipError_t e = ntg::launch_gemm_any(dtype, ta, tb, q, s);
+            if (e != hipSuccess) return hip_fail(e, "gemm launch");
+            e = ntg::launch_splitk_reduce(dtype, workspace, ap.splits, p, ap.ldp, s);
+            if (e != hipSuccess) return hip_fail(e, "split-K reduction launch");
+            return NTG_OK;
+        }
+    }
+    {
         const PadPlan pp = plan_pad(p, dtype, ta, tb);
-        if (pp.ok && workspace && workspace_bytes >= pp.bytes() && (reinterpret_cast<uintptr_t>(workspace) & 255) == 0)
+        if (pp.ok && pp.pays && workspace && workspace_bytes >= pp.bytes() && (reinterpret_cast<uintptr_t>(workspace) & 255) == 0)
             return run_padded(p, pp, dtype, ta, tb, workspace, s);
     }
     const SplitPlan plan = plan_splitk(p, dtype, ta);
@@ -519,7 +601,7 @@ int run_gemm(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s, void
             int rc = launch_gemm(q, dtype, ta, tb, s);
             if (rc) return rc;
         }
-        hipError_t e = ntg::launch_splitk_reduce(dtype, workspace, plan.splits, p, s);
+        hipError_t e = ntg::launch_splitk_reduce(dtype, workspace, plan.splits, p, p.N, s);
         if (e != hipSuccess) return hip_fail(e, "split-K reduction launch");
         return NTG_OK;
     }
@@ -644,8 +726,9 @@ int64_t ntg_gemm_workspace_bytes(const ntg_gemm_desc* d) {
         return ip.ok ? ip.bytes() : 0;
     }
     {
+        const AnySplitPlan ap = plan_any_split(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0);
         const PadPlan pp = plan_pad(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0);      // pointers taken as 16-byte aligned
-        if (pp.ok) return pp.bytes();
+        if (pp.ok || ap.splits > 1) return std::max<int64_t>(ap.bytes, pp.ok ? pp.bytes() : 0);
     }
     return plan_splitk(p, d->dtype, d->transpose_a != 0).bytes;      // pointers taken as 16-byte aligned
 }

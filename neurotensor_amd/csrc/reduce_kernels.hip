@@ -98,50 +98,59 @@ __global__ void __launch_bounds__(256) reduce_batch_taps_last_kernel(const float
 // Split-K epilogue: C (+)= sum over the k ranges of part[s][m][n], s ascending, starting from C0 (the incoming C, the
 // broadcast bias, or zero).  One rounding to T at the end.
 template <class T, class P, class Acc>
-__global__ void __launch_bounds__(256) splitk_reduce_kernel(const P* __restrict__ part, const int splits, const int64_t split_stride, const GemmParams p) {
+__global__ void __launch_bounds__(256) splitk_reduce_kernel(const P* __restrict__ part, const int splits, const int64_t split_stride, const int64_t ldp, const GemmParams p) {
     const int64_t total = (int64_t)p.M * p.N;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     const int64_t b = blockIdx.y;                                      // item of the batch: its partial sums follow the previous item's
     T* C = static_cast<T*>(p.C) + b * p.sC;
     const T* bias = static_cast<const T*>(p.bias) + b * p.bias_bs;
-    part += b * total;
+    part += b * ((int64_t)p.M * ldp);
     for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += stride) {
         const int64_t m = idx / p.N, n = idx - m * p.N;
         T* cp = C + m * p.ldc + n;
         Acc acc = (Acc)0;
         if (p.cmode == C_ACCUMULATE) acc = (Acc)*cp;
         else if (p.cmode == C_BIAS) acc = (Acc)bias[m * p.bias_rs + n * p.bias_cs];
-        for (int s = 0; s < splits; ++s) acc += (Acc)part[(int64_t)s * split_stride + idx];
+        for (int s = 0; s < splits; ++s) acc += (Acc)part[(int64_t)s * split_stride + m * ldp + n];
         if (p.act == ACT_RELU) acc = acc > (Acc)0 ? acc : (Acc)0;
         *cp = (T)acc;
     }
 }
 
-// The same sum, four consecutive columns per thread with 16-byte accesses to the partial sums (rows of C and of the
-// partial matrices must start on a multiple of four elements); the partial loads of four k ranges are in flight together.
+// The same sum, four consecutive columns per thread with 16-byte accesses to the partial sums, whose rows lie ldp elements apart (a multiple
+// of four); C may start anywhere.  The partial loads of four k ranges are in flight together.
 template <class T, class P, class Acc>
-__global__ void __launch_bounds__(256) splitk_reduce_vec_kernel(const P* __restrict__ part, const int splits, const int64_t split_stride, const GemmParams p) {
-    typedef T TV __attribute__((ext_vector_type(4)));
+__global__ void __launch_bounds__(256) splitk_reduce_vec_kernel(const P* __restrict__ part, const int splits, const int64_t split_stride, const uint32_t ldp, const GemmParams p) {
+    typedef T TV __attribute__((ext_vector_type(4), aligned(sizeof(T))));
     typedef P PV __attribute__((ext_vector_type(4)));
-    const int64_t nq = p.N / 4, total = (int64_t)p.M * p.N, quads = (int64_t)p.M * nq;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    const uint32_t nq = ldp / 4, quads = (uint32_t)p.M * nq;
+    const uint32_t stride = gridDim.x * blockDim.x;
     const int64_t b = blockIdx.y;
     T* C = static_cast<T*>(p.C) + b * p.sC;
     const T* bias = static_cast<const T*>(p.bias) + b * p.bias_bs;
-    part += b * total;
-    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < quads; q += stride) {
-        const int64_t m = q / nq, n = (q - m * nq) * 4;
-        TV* cp = reinterpret_cast<TV*>(C + m * p.ldc + n);
+    part += b * ((int64_t)p.M * ldp);
+    for (uint32_t q = blockIdx.x * blockDim.x + threadIdx.x; q < quads; q += stride) {
+        const uint32_t m = q / nq, n = (q - m * nq) * 4;
+        if (n >= (uint32_t)p.N) continue;
+        const bool whole = n + 4 <= (uint32_t)p.N;
+        T* ce = C + (int64_t)m * p.ldc + n;
         Acc acc[4] = {(Acc)0, (Acc)0, (Acc)0, (Acc)0};
         if (p.cmode == C_ACCUMULATE) {
-            const TV c0 = *cp;
+            if (whole) {
+                const TV c0 = *reinterpret_cast<const TV*>(ce);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[e] = (Acc)c0[e];
+                for (int e = 0; e < 4; ++e) acc[e] = (Acc)c0[e];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < (uint32_t)p.N) acc[e] = (Acc)ce[e];
+            }
         } else if (p.cmode == C_BIAS) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[e] = (Acc)bias[m * p.bias_rs + (n + e) * p.bias_cs];
+            for (int e = 0; e < 4; ++e)
+                if (n + e < (uint32_t)p.N) acc[e] = (Acc)bias[(int64_t)m * p.bias_rs + (int64_t)(n + e) * p.bias_cs];
         }
-        const P* pp = part + q * 4;
+        const P* pp = part + (int64_t)q * 4;
         int s = 0;
         for (; s + 4 <= splits; s += 4) {
             PV v[4];
@@ -160,19 +169,23 @@ __global__ void __launch_bounds__(256) splitk_reduce_vec_kernel(const P* __restr
         TV o;
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[e] = (T)((p.act == ACT_RELU && !(acc[e] > (Acc)0)) ? (Acc)0 : acc[e]);
-        *cp = o;
+        if (whole) *reinterpret_cast<TV*>(ce) = o;
+        else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (n + e < (uint32_t)p.N) ce[e] = o[e];
+        }
     }
 }
 
-// p.batch items (at most 65535 per call): item b's partial sums start b * M * N elements into every k range's block, the
-// ranges' blocks lie p.batch * M * N elements apart
+// p.batch items (at most 65535 per call): item b's partial sums start b * M * ldp elements into every k range's block, the
+// ranges' blocks lie p.batch * M * ldp elements apart
 template <class T, class P, class Acc>
-static void launch_splitk_reduce_t(const void* part, int splits, const GemmParams& p, hipStream_t s) {
-    const int64_t total = (int64_t)p.M * p.N, split_stride = total * p.batch;
-    const bool vec = p.N % 4 == 0 && p.ldc % 4 == 0 && p.sC % 4 == 0 && (reinterpret_cast<uintptr_t>(p.C) % (4 * sizeof(T))) == 0 &&
-                     (reinterpret_cast<uintptr_t>(part) % (4 * sizeof(P))) == 0;
-    if (vec) hipLaunchKernelGGL((splitk_reduce_vec_kernel<T, P, Acc>), dim3(grid_for(total / 4), (unsigned)p.batch), dim3(256), 0, s, (const P*)part, splits, split_stride, p);
-    else hipLaunchKernelGGL((splitk_reduce_kernel<T, P, Acc>), dim3(grid_for(total), (unsigned)p.batch), dim3(256), 0, s, (const P*)part, splits, split_stride, p);
+static void launch_splitk_reduce_t(const void* part, int splits, const GemmParams& p, int64_t ldp, hipStream_t s) {
+    const int64_t total = (int64_t)p.M * ldp, split_stride = total * p.batch;
+    const bool vec = ldp % 4 == 0 && total < (1LL << 31) && (reinterpret_cast<uintptr_t>(part) % (4 * sizeof(P))) == 0;
+    if (vec) hipLaunchKernelGGL((splitk_reduce_vec_kernel<T, P, Acc>), dim3(grid_for(total / 4), (unsigned)p.batch), dim3(256), 0, s, (const P*)part, splits, split_stride, (uint32_t)ldp, p);
+    else hipLaunchKernelGGL((splitk_reduce_kernel<T, P, Acc>), dim3(grid_for((int64_t)p.M * p.N), (unsigned)p.batch), dim3(256), 0, s, (const P*)part, splits, split_stride, ldp, p);
 }
 
 // C[b][m][n] = C[b][m][n] > 0 ? C[b][m][n] : 0 -- relu_ = clamp_(x, 0) of the reference (activation_functions.cpp:143,
@@ -214,15 +227,16 @@ hipError_t launch_relu_inplace(int dtype, void* C, int64_t ldc, int64_t sC, int6
     return hipGetLastError();
 }
 
-hipError_t launch_splitk_reduce(int dtype, const void* part, int splits, const GemmParams& p, hipStream_t s) {
+hipError_t launch_splitk_reduce(int dtype, const void* part, int splits, const GemmParams& p, int64_t ldp, hipStream_t s) {
     const int64_t total = (int64_t)p.M * p.N;
     if (total == 0 || p.batch < 1) return hipSuccess;
     if (p.batch > 65535) return hipErrorInvalidValue;
     switch (dtype) {
-    case DT_F32: launch_splitk_reduce_t<float, float, float>(part, splits, p, s); break;
-    case DT_F64: launch_splitk_reduce_t<double, double, double>(part, splits, p, s); break;
-    case DT_F16: launch_splitk_reduce_t<_Float16, float, float>(part, splits, p, s); break;
-    case DT_BF16: launch_splitk_reduce_t<__bf16, float, float>(part, splits, p, s); break;
+    case DT_F32: launch_splitk_reduce_t<float, float, float>(part, splits, p, ldp, s); break;
+    case DT_F64: launch_splitk_reduce_t<double, double, double>(part, splits, p, ldp, s); break;
+    case DT_F16: launch_splitk_reduce_t<_Float16, float, float>(part, splits, p, ldp, s); break;
+    case DT_BF16: launch_splitk_reduce_t<__bf16, float, float>(part, splits, p, ldp, s); break;
+    case DT_I8: case DT_U8: launch_splitk_reduce_t<uint8_t, int, int>(part, splits, p, ldp, s); break;      // (the low 8 bits, either signedness)
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -1,0 +1,110 @@
+"""Products whose rows start anywhere (odd sizes, views inside a 16-byte chunk): whole and cut into k ranges, at the edges of tiles, K-steps and chunks.
+
+Exact for Int8 (wrapping) and Float32 without a workspace (the reference's chain, bit for bit).  Otherwise against the product in 64 bits: one
+rounding to the type (half a last place: 2^-11 Float16, 2^-8 BFloat16, relative) on a sum whose k multiply-adds each err by 2^-24 of sum |a||b| at most.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from neurotensor_amd import _lib
+from neurotensor_amd import functional as F
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+DTYPES = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32, "i8": torch.int8}
+UNIT = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8, "f32": 2.0 ** -24}
+TRANS = [(False, False), (False, True), (True, False), (True, True)]
+# one element past / before a tile, a K-step, a chunk; one row; the shortest rows that hold a chunk; k ranges with a short last one
+SIZES = [(33, 17, 17), (63, 65, 64), (64, 63, 65), (65, 129, 127), (40, 16, 19), (1, 33, 18), (129, 257, 31), (1700, 40, 1030),
+         (70, 2049, 66), (37, 3001, 130), (200, 1100, 77)]
+
+
+def values(shape, name, gen):
+    if name == "i8":
+        return torch.randint(-128, 128, shape, dtype=torch.int8, generator=gen)
+    return torch.randn(*shape, generator=gen).to(DTYPES[name])
+
+
+def check(got, a, b, c0, name, k):
+    if name == "i8":
+        want = torch.matmul(a.double(), b.double()).to(torch.int64) + (0 if c0 is None else c0.to(torch.int64))
+        assert torch.equal(((want + 128) % 256 - 128).to(torch.int8), got)
+        return
+    exact = torch.matmul(a.double(), b.double()) + (0 if c0 is None else c0.double())
+    terms = torch.matmul(a.double().abs(), b.double().abs()) + (0 if c0 is None else c0.double().abs())
+    bound = UNIT[name] * exact.abs() + (k + 40) * 2.0 ** -24 * terms + (2.0 ** -24 if name == "f16" else 0)      # (40: the sums of k ranges; Float16's smallest step)
+    assert ((got.double() - exact).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("name", sorted(DTYPES))
+@pytest.mark.parametrize("ta,tb", TRANS)
+def test_sizes_at_the_edges(name, ta, tb):
+    gen = torch.Generator().manual_seed(5)
+    for m, k, n in SIZES:
+        a, b = values((k, m) if ta else (m, k), name, gen), values((n, k) if tb else (k, n), name, gen)
+        got = F.matmult(a.to(DEV), b.to(DEV), None, ta, tb).cpu()
+        check(got, a.t() if ta else a, b.t() if tb else b, None, name, k)
+
+
+@pytest.mark.parametrize("name", sorted(DTYPES))
+def test_batches_pitches_and_what_is_added_to(name):
+    """Items of a batch are the same bits alone, rows lie further apart than they are long, C is added to and starts inside a chunk."""
+    lib = _lib.load()
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    gen = torch.Generator().manual_seed(6)
+    for m, k, n in ((66, 70, 37), (45, 2051, 97)):
+        batch, lda, ldb, ldc = 3, k + 2, n + 1, n + 3
+        a, b, c0 = values((batch, m, lda), name, gen), values((batch, k, ldb), name, gen), values((1 + batch * m * ldc,), name, gen)
+        ta, tb, one = a.to(DEV), b.to(DEV), c0.to(DEV)
+        both = [c0.to(DEV), one]
+        for c, items in ((both[0], [(0, batch)]), (both[1], [(i, 1) for i in range(batch)])):
+            for first, count in items:
+                d = _lib.GemmDesc()
+                d.dtype, d.c_mode, d.m, d.k, d.n, d.batches = F.ntg_dtype(ta), _lib.C_ACCUMULATE, m, k, n, count
+                d.lda, d.ldb, d.ldc, d.stride_a, d.stride_b, d.stride_c = lda, ldb, ldc, m * lda, k * ldb, m * ldc
+                need = lib.ntg_gemm_workspace_bytes(ctypes.byref(d))
+                ws = torch.empty(max(need, 1), dtype=torch.uint8, device=DEV)
+                d.workspace, d.workspace_bytes = ws.data_ptr(), need
+                es = c.element_size()
+                _lib.check(lib.ntg_gemm_dev(ctypes.byref(d), ta[first].data_ptr(), tb[first].data_ptr(), c.data_ptr() + (1 + first * m * ldc) * es, st))
+        torch.cuda.synchronize()
+        assert torch.equal(both[0].view(torch.uint8), both[1].view(torch.uint8))
+        got, before = both[0].cpu()[1:].view(batch, m, ldc), c0[1:].view(batch, m, ldc)
+        assert torch.equal(got[..., n:], before[..., n:])                # what lies between the rows stays
+        check(got[..., :n], a[..., :k], b[..., :n], before[..., :n], name, k)
+
+
+@pytest.mark.parametrize("name", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("relu", [False, True])
+def test_bias_and_relu(name, relu):
+    gen = torch.Generator().manual_seed(7)
+    for m, k, n in ((37, 67, 129), (65, 2001, 100), (300, 300, 333)):
+        x, w, bias = values((m, k), name, gen), values((n, k), name, gen), values((n,), name, gen)
+        got = (F.linear_relu if relu else F.linear)(x.to(DEV), w.to(DEV), bias.to(DEV), False, True).cpu()
+        if relu:
+            assert (got >= 0).all()
+            keep = got > 0
+            plain = F.linear(x.to(DEV), w.to(DEV), bias.to(DEV), False, True).cpu()
+            assert torch.equal(got, torch.where(plain > 0, plain, torch.zeros_like(plain))) and keep.any()
+        else:
+            check(got, x, w.t(), bias, name, k)
+
+
+def test_float32_without_workspace_is_the_reference_chain_bit_for_bit():
+    lib = _lib.load()
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    rng = np.random.default_rng(8)
+    for (m, k, n), (ta, tb) in zip(((65, 67, 130), (70, 131, 33), (130, 35, 65), (61, 1003, 63)), TRANS):
+        a, b, c0 = (rng.standard_normal(s).astype(np.float32) for s in ((m, k), (k, n), (m, n)))
+        sa, sb = np.ascontiguousarray(a.T) if ta else a, np.ascontiguousarray(b.T) if tb else b
+        da, db, dc = (torch.from_numpy(v).to(DEV) for v in (sa, sb, c0))
+        d = _lib.GemmDesc()
+        d.dtype, d.transpose_a, d.transpose_b, d.c_mode = _lib.FLOAT32, int(ta), int(tb), _lib.C_ACCUMULATE
+        d.m, d.k, d.n, d.batches = m, k, n, 1
+        _lib.check(lib.ntg_gemm_dev(ctypes.byref(d), da.data_ptr(), db.data_ptr(), dc.data_ptr(), st))
+        want = oracle.matmult2d(sa, sb, c0.copy(), ta, tb)
+        assert np.array_equal(dc.cpu().numpy().view(np.uint32), want.view(np.uint32))
