@@ -181,8 +181,7 @@ typedef struct ntg_gemm_desc {
     const void* bias;           /* device pointer, NTG_C_BIAS only */
     int64_t bias_batch_stride, bias_row_stride, bias_col_stride;   /* elements; 0 = broadcast */
     void* workspace;            /* optional device scratch, 256-byte aligned, ntg_gemm_workspace_bytes(desc) bytes: lets a   */
-    int64_t workspace_bytes;    /* single product with few output tiles and a deep k be split along k (deterministic), and  */
-                                /* a large 16/32/64-bit integer product run as byte planes on the 8-bit matrix pipe (bit-exact) */
+    int64_t workspace_bytes;    /* product with few output tiles and a deep k be split along k (deterministic) */
     int64_t flags;              /* NTG_GEMM_* bits below; 0 for none */
 } ntg_gemm_desc;
 
@@ -192,7 +191,7 @@ typedef struct ntg_gemm_desc {
  * kernel read from a misaligned address (wrong results, not a fault).  Without the vouch, floating-point and 8-bit
  * batches of some size (from 8 GFLOP; Float32 and Float64 from 32, 8-bit integers from 1) have their entries looked at on the device: one small kernel sets a
  * flag, then the product is launched on both kernel families and the one the flag does not name returns at once -- two
- * extra launches (about 4 us), the same bits; smaller batches run on the register-staged kernels.  The flags live in a static
+ * extra launches (about 4 us), the same bits; smaller batches run on the kernels that take rows as they lie.  The flags live in a static
  * array of the library's device code: make the first such call on a device outside a stream capture. */
 #define NTG_GEMM_PTRS_ALIGNED16 1
 /* Keep the reference's order of summation: never split this product along k (workspace or not), and run products of up to 32
@@ -207,10 +206,10 @@ typedef struct ntg_gemm_desc {
  * for shapes such as [256, 8192] x [8192, 8192] (planned from one item's sizes, so a batch is offered its item's split with
  * the partial sums of every item); zero-padded copies of large 8-bit, 16-bit, Float32 and Float64 operands whose rows, pitches
  * or base pointers are not 16-byte multiples, so that they run on the DMA-fed kernels (same results: zeros add nothing);
- * or, for large Int16 / Int32 / Int64 products and their unsigned forms, the
- * 3 / 10 / 36 products of balanced byte planes on v_mfma_i32_32x32x32_i8, whose sum modulo 2^W is the reference's wrapping
- * result (nt/mp/simde_traits/simde_traits_avx2.h:810-812, :444-446, :523-540: multiply and add in the element type).  Without a workspace the same result is computed by the
- * plain kernels.  The reference has no counterpart: its k loop is always serial (nt_matmult.hpp:196). */
+ * or, for large Int16 / Int32 / Int64 products and their unsigned forms, room for k ranges (these run as 3 / 10 / 36 products of balanced
+ * digits on v_mfma_i32_32x32x32_i8 with or without it; the sum modulo 2^W is the reference's wrapping result,
+ * nt/mp/simde_traits/simde_traits_avx2.h:810-812, :444-446, :523-540: multiply and add in the element type).  It is the largest any form takes: a
+ * product may use less.  Without a workspace the same result is computed by the plain kernels.  The reference has no counterpart: its k loop is always serial (nt_matmult.hpp:196). */
 int64_t ntg_gemm_workspace_bytes(const ntg_gemm_desc* desc);
 
 /* nt_matmult<T> on device buffers: C += op(A).op(B), dense leading dimensions. */

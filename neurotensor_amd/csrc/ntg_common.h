@@ -319,6 +319,8 @@ hipError_t launch_gemm_mfma(int dtype, bool ta, bool tb, const GemmParams& p, hi
 // epilogue applies GemmParams::act
 hipError_t launch_gemm_ring_only(int dtype, bool ta, bool tb, const GemmParams& p, hipStream_t s, bool* taken);
 // C[b][m][n] = max(C[b][m][n], 0) in place (floating dtypes)
+// Int16 / 32 / 64 and unsigned on the 8-bit matrix pipe (planes = bytes of an element; gemm_int_impl.h)
+hipError_t launch_gemm_int(int planes, bool ta, bool tb, const GemmParams& p, hipStream_t s);
 // Float16 / BFloat16 / Float32 / Int8 on rows that start anywhere (gemm_any_impl.h); the caller has checked any_eligible()
 hipError_t launch_gemm_any(int dtype, bool ta, bool tb, const GemmParams& p, hipStream_t s);
 hipError_t launch_relu_inplace(int dtype, void* C, int64_t ldc, int64_t sC, int64_t M, int64_t N, int64_t batch, hipStream_t s);
@@ -406,10 +408,6 @@ struct RingItem { int64_t a, b, c; int K, N, ldc, k_d, k_r, k_c, Wo, HoWo, first
 hipError_t launch_phase_setup(int64_t es, const void* w, void* wt, RingItem* items, const PhaseLayout& q, hipStream_t s);
 hipError_t launch_phase_interleave(int dtype, const void* tmp, void* im, const PhaseLayout& q, int accumulate, hipStream_t s);
 hipError_t launch_conv_nhwc_items(int dtype, int edge, const GemmParams& p, int64_t blocks, hipStream_t s);
-// 16-, 32- and 64-bit integer products on the 8-bit matrix pipe as byte planes (see gemm_mfma_i8.hip); planes = bytes per element
-struct IntPlanesParams { int M, N, K, Kp, Np, batch; int64_t lda, ldb, sA, sB; int ta, tb; };
-hipError_t launch_int_split_planes(int planes, const void* A, const void* B, void* a_planes, void* b_planes, const IntPlanesParams& q, hipStream_t s);
-hipError_t launch_int_combine(int planes, const void* parts, const GemmParams& p, int Np, hipStream_t s);
 hipError_t launch_conv_nhwc_dw(int dtype, bool ta, const GemmParams& p, hipStream_t s);   // ta: A (the output gradient) stored [k][m]
 // part rows hold cgp >= cg channels per tap; the partial sums are Float32 whatever the dtype
 hipError_t launch_reduce_batch_taps_last(int dtype, const void* part, void* out, int64_t batch, int64_t rows, int64_t cg, int64_t cgp,

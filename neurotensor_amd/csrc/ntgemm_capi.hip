@@ -167,6 +167,22 @@ bool is_complex_dtype(int dt) { return dt == ntg::DT_C32 || dt == ntg::DT_C64 ||
 // integers and the complex types: computed lane by lane on the vector ALU, bit-exact; no matrix-pipe or gathering forms
 bool is_valu_dtype(int dt) { return is_int_dtype(dt) || is_complex_dtype(dt); }
 
+// 16-, 32- and 64-bit integers on the 8-bit matrix pipe (gemm_int_impl.h): bytes per element
+static int int_planes_of(int dtype) {
+    switch (dtype) {
+    case ntg::DT_I16: case ntg::DT_U16: return 2;
+    case ntg::DT_I32: case ntg::DT_U32: return 4;
+    case ntg::DT_I64: case ntg::DT_U64: return 8;
+    default: return 0;
+    }
+}
+// Every contiguous extent holds the eight elements of a group, 32-bit lane offsets, 32-bit sums of a shift's products (P K 2^14 < 2^31).
+// What misses this runs on the vector ALU, bit for bit the same.
+static bool int_pipe_eligible(const ntg::GemmParams& p, int dtype, bool ta, bool tb) {
+    const int64_t P = int_planes_of(dtype);
+    return P != 0 && p.K > 0 && (ta ? p.M : p.K) >= 8 && (tb ? p.K : p.N) >= 8 && P * (int64_t)p.K < (1 << 17) && p.lda * P < (1 << 23) && p.ldb * P < (1 << 23);
+}
+
 // Fills the derived fields and launches the kernel family for the dtype.
 int launch_gemm(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s) {
     const int64_t es = ntg::elem_size(dtype);
@@ -201,6 +217,8 @@ int launch_gemm(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s) {
     };
     if (dtype == ntg::DT_I8 || dtype == ntg::DT_U8) {
         e = ntg::launch_gemm_mfma_i8(dtype, ta, tb, p, s);
+    } else if (int_pipe_eligible(p, dtype, ta, tb)) {
+        e = ntg::launch_gemm_int(int_planes_of(dtype), ta, tb, p, s);
     } else if (is_int_dtype(dtype)) {
         e = ntg::launch_gemm_valu(dtype, ta, tb, p, s);
     } else if (is_complex_dtype(dtype)) {
@@ -232,80 +250,6 @@ int launch_gemm(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s) {
 // (the reference's batched == per-item rule, tests/src/matmult_test.cpp:108-189).  A batch whose items are split runs one
 // batched launch per k range into [splits][batch][M][N] and one reduction over all items.
 struct SplitPlan { int splits; int64_t kc; int64_t bytes; };
-
-// 16-, 32- and 64-bit integers on the 8-bit matrix pipe (byte planes, gemm_mfma_i8.hip): P (P + 1) / 2 8-bit products
-// (P bytes per element) instead of the vector ALU's multiply-adds, plus the passes that split the operands and
-// recombine the partial sums.  Taken when the caller supplies the workspace and an estimate of both times favours it.
-// Measured on MI355X: the vector-ALU kernel spends about 0.07 us (16- and 32-bit; 0.13 us 64-bit) per k on each round of
-// 64 x 64 tiles over the 256 CUs, plus as much once; the plane form costs its P + 3 launches (17 / 30 / 55 us for
-// P = 2 / 4 / 8), the 8-bit products at about 10^9 multiply-adds per us, and the partial sums written and read at 4 TB/s.
-struct IntPlanesPlan {
-    bool ok; int planes, Kp, Np; int64_t a_bytes, b_bytes, p_bytes;
-    int64_t bytes() const { return a_bytes + b_bytes + p_bytes; }
-};
-static int int_planes_of(int dtype) {
-    switch (dtype) {
-    case ntg::DT_I16: case ntg::DT_U16: return 2;
-    case ntg::DT_I32: case ntg::DT_U32: return 4;
-    case ntg::DT_I64: case ntg::DT_U64: return 8;
-    default: return 0;
-    }
-}
-static IntPlanesPlan plan_int_planes(const ntg::GemmParams& p, int dtype) {
-    IntPlanesPlan pl;
-    std::memset(&pl, 0, sizeof pl);
-    const int P = int_planes_of(dtype);
-    if (P == 0 || p.Aptr || p.Bptr || p.Cptr) return pl;
-    if (p.M < 128 || p.N < 128 || p.K < 64) return pl;
-    pl.planes = P;
-    pl.Kp = (p.K + 15) / 16 * 16;
-    pl.Np = (p.N + 15) / 16 * 16;
-    {
-        const double macs = (double)p.M * p.N * p.K * p.batch;
-        const double rounds = (double)(((int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch + 255) / 256);
-        const double valu_us = (double)p.K * (P == 8 ? 0.13 : P == 4 ? 0.07 : 0.055) * (rounds + 1.0);
-        const double planes_us = (P == 8 ? 55.0 : P == 4 ? 30.0 : 17.0) + macs * (P * (P + 1) / 2) / 1.0e9 +
-                                 8.0 * P * p.batch * (double)p.M * pl.Np / 4.0e6;
-        if (planes_us > 0.8 * valu_us) return pl;
-    }
-    if ((int64_t)P * pl.Kp >= (1 << 17) || pl.Np >= (1 << 23)) return pl;     // 32-bit partial sums: P K 2^14 < 2^31
-    pl.a_bytes = (int64_t)align_up((size_t)((p.sA == 0 ? 1 : p.batch) * (int64_t)p.M * P * pl.Kp), 256);
-    pl.b_bytes = (int64_t)align_up((size_t)((p.sB == 0 ? 1 : p.batch) * (int64_t)P * pl.Kp * pl.Np), 256);
-    pl.p_bytes = (int64_t)P * p.batch * p.M * pl.Np * 4;
-    pl.ok = true;
-    return pl;
-}
-static int run_int_planes(const ntg::GemmParams& p, const IntPlanesPlan& pl, bool ta, bool tb, void* ws, hipStream_t s) {
-    const int P = pl.planes;
-    char* a_pl = static_cast<char*>(ws);
-    char* b_pl = a_pl + pl.a_bytes;
-    char* parts = b_pl + pl.b_bytes;
-    ntg::IntPlanesParams q;
-    q.M = p.M; q.N = p.N; q.K = p.K; q.Kp = pl.Kp; q.Np = pl.Np; q.batch = p.batch;
-    q.lda = p.lda; q.ldb = p.ldb; q.sA = p.sA; q.sB = p.sB; q.ta = ta; q.tb = tb;
-    hipError_t e = ntg::launch_int_split_planes(P, p.A, p.B, a_pl, b_pl, q, s);
-    if (e != hipSuccess) return hip_fail(e, "byte-plane split launch");
-    const int64_t per = (int64_t)p.M * pl.Np;
-    for (int sh = 0; sh < P; ++sh) {
-        ntg::GemmParams g;
-        std::memset(&g, 0, sizeof g);
-        g.M = p.M; g.N = pl.Np; g.K = (sh + 1) * pl.Kp; g.batch = p.batch;
-        g.A = a_pl;
-        g.B = b_pl + (int64_t)(P - 1 - sh) * pl.Kp * pl.Np;
-        g.C = parts + (int64_t)sh * p.batch * per * 4;
-        g.lda = (int64_t)P * pl.Kp; g.ldb = pl.Np; g.ldc = pl.Np;
-        g.sA = p.sA == 0 ? 0 : (int64_t)p.M * P * pl.Kp;
-        g.sB = p.sB == 0 ? 0 : (int64_t)P * pl.Kp * pl.Np;
-        g.sC = per;
-        g.cmode = ntg::C_PARTIAL;
-        g.vecA_ok = 1; g.vecB_ok = 1;
-        e = ntg::launch_gemm_mfma_i8(ntg::DT_I8, false, false, g, s);
-        if (e != hipSuccess) return hip_fail(e, "byte-plane product launch");
-    }
-    e = ntg::launch_int_combine(P, parts, p, pl.Np, s);
-    if (e != hipSuccess) return hip_fail(e, "byte-plane combine launch");
-    return NTG_OK;
-}
 
 // Padded copies.  The DMA-fed kernels need 16-byte rows (leading dimensions, batch strides, base pointers, and K, N -- M
 // under transpose_a -- multiples of one 16-byte chunk); a product that misses this falls to the vector ALU
@@ -482,7 +426,41 @@ SplitPlan plan_splitk(const ntg::GemmParams& p, int dtype, bool ta) {
 
 // k ranges of a product whose rows miss the 16-byte rule by their SIZES (gemm_any_impl.h serves it): as plan_splitk a function of one item's
 // sizes and pitches only.  kc is a whole number of K-steps, the last range is what is left.  Rows of the partial sums hold whole 16-byte chunks.
+// The integers of more than a byte likewise (gemm_int_impl.h).
 struct AnySplitPlan { int splits; int64_t kc, ldp, bytes; };
+// Room that ntg_gemm_workspace_bytes offers large integer products (and ntg_gemm_noalloc_dev takes them with or refuses them for): the digits of both
+// operands and the 32-bit sums of every shift.  The product itself needs none; its k ranges take what they use of it.
+static int64_t int_workspace_bytes(const ntg::GemmParams& p, int dtype) {
+    const int P = int_planes_of(dtype);
+    if (P == 0 || p.Aptr || p.Bptr || p.Cptr || p.M < 128 || p.N < 128 || p.K < 64) return 0;
+    const int64_t Kp = (p.K + 15) / 16 * 16, Np = (p.N + 15) / 16 * 16;
+    const double macs = (double)p.M * p.N * p.K * p.batch;
+    const double rounds = (double)(((int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch + 255) / 256);
+    const double valu_us = (double)p.K * (P == 8 ? 0.13 : P == 4 ? 0.07 : 0.055) * (rounds + 1.0);
+    const double planes_us = (P == 8 ? 55.0 : P == 4 ? 30.0 : 17.0) + macs * (P * (P + 1) / 2) / 1.0e9 + 8.0 * P * p.batch * (double)p.M * Np / 4.0e6;
+    if (planes_us > 0.8 * valu_us || P * Kp >= (1 << 17) || Np >= (1 << 23)) return 0;
+    return (int64_t)align_up((size_t)((p.sA == 0 ? 1 : p.batch) * (int64_t)p.M * P * Kp), 256) +
+           (int64_t)align_up((size_t)((p.sB == 0 ? 1 : p.batch) * (int64_t)P * Kp * Np), 256) + (int64_t)P * p.batch * p.M * Np * 4;
+}
+// A workgroup alone on its CU spends 0.35 / 0.48 / 1.4 us (16 / 32 / 64 bits) on each K-step of 32, several 0.17 / 0.35 / 1.3 us each (Int32 200 x 3000 x 200
+// whole 48 us, 8 / 16 ranges 12.4 / 10.8; Int16 709 x 3136 x 450, ranges 1 / 4 / 8 / 16: 36 / 16.9 / 15.8 / 19.4; Int64 576 x 3968 x 281, 1 / 4 / 8: 183 / 53 / 58).
+// The sums wrap, so their order is nobody's concern: the batch counts among the tiles.  room: bytes of workspace there are.
+AnySplitPlan plan_int_split(const ntg::GemmParams& p, int dtype, bool ta, bool tb, int64_t room) {
+    AnySplitPlan pl{1, p.K, (p.N + 3) / 4 * 4, 0};
+    if (p.batch < 1 || p.batch > 65535 || p.Aptr || p.Bptr || p.Cptr || !int_pipe_eligible(p, dtype, ta, tb)) return pl;
+    const int P = int_planes_of(dtype);
+    const int64_t steps = (p.K + 31) / 32, tiles = ((p.M + 63) / 64) * ((p.N + 63) / 64) * (int64_t)p.batch;
+    if (tiles > 255) return pl;
+    const int64_t per_range = (int64_t)p.batch * p.M * pl.ldp * P;
+    const double alone = P == 2 ? 0.35 : P == 4 ? 0.48 : 1.4, shared = P == 2 ? 0.17 : P == 4 ? 0.35 : 1.3;
+    double best_us = 0.95 * (double)steps * alone;
+    for (int64_t sp = 2; sp <= 32 && sp <= steps / 2 && sp * per_range <= room; ++sp) {
+        const int64_t per = (steps + sp - 1) / sp, ranges = (steps + per - 1) / per, wgs = tiles * ranges;
+        const double us = (double)per * (wgs <= 256 ? alone : shared * (double)((wgs + 255) / 256)) + 4.0 + 2.0 * (double)ranges * (double)per_range / 4.0e6;
+        if (us < best_us) { best_us = us; pl.splits = (int)ranges; pl.kc = per * 32; pl.bytes = ranges * per_range; }
+    }
+    return pl;
+}
 AnySplitPlan plan_any_split(const ntg::GemmParams& p, int dtype, bool ta, bool tb) {
     AnySplitPlan none{1, p.K, 0, 0};
     if (p.batch < 1 || p.batch > 65535 || p.Aptr || p.Bptr || p.Cptr || p.keep_k_order || !ntg::any_eligible(p, dtype, ta, tb)) return none;
@@ -508,6 +486,7 @@ AnySplitPlan plan_any_split(const ntg::GemmParams& p, int dtype, bool ta, bool t
     for (int64_t sp = 2; sp <= 32 && sp <= steps / 2; ++sp) {
         const int64_t per = (steps + sp - 1) / sp, ranges = (steps + per - 1) / per;
         const double us = estimate_us(ranges, per);
+        if (ranges * (int64_t)p.M * ((p.N + 3) / 4 * 4) * 4 > (int64_t)NTG_NOALLOC_SCRATCH_BYTES) break;      // (an item fits where nothing is allocated)
         if (us < best_us) { best_us = us; pl.splits = (int)ranges; pl.kc = per * bk; }
     }
     if (pl.splits < 2) return none;
@@ -541,13 +520,8 @@ int run_gemm(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s, void
         if (e != hipSuccess) return hip_fail(e, "empty-k launch");
         return NTG_OK;
     }
-    if (int_planes_of(dtype)) {
-        const IntPlanesPlan ip = plan_int_planes(p, dtype);
-        if (ip.ok && workspace && workspace_bytes >= ip.bytes() && (reinterpret_cast<uintptr_t>(workspace) & 255) == 0)
-            return run_int_planes(p, ip, ta, tb, workspace, s);
-    }
     {
-        const AnySplitPlan ap = plan_any_split(p, dtype, ta, tb);
+        const AnySplitPlan ap = int_planes_of(dtype) ? plan_int_split(p, dtype, ta, tb, workspace ? workspace_bytes : 0) : plan_any_split(p, dtype, ta, tb);
         if (ap.splits > 1 && workspace && workspace_bytes >= ap.bytes && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0) {
             // launch index = range * batch + item
             ntg::GemmParams q = p;
@@ -556,14 +530,14 @@ int run_gemm(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s, void
             q.C = workspace;
             q.ldc = ap.ldp;
             q.sC = (int64_t)p.M * ap.ldp;
-            q.cmode = ntg::C_PARTIAL;
+            q.cmode = int_planes_of(dtype) ? ntg::C_OVERWRITE : ntg::C_PARTIAL;      // (sums in the element type: wrapping)
             q.bias = nullptr;
             q.act = ntg::ACT_NONE;
             q.batch = ap.splits * p.batch;
             q.krange_items = p.batch;
             q.sAk = ta ? ap.kc * p.lda : ap.kc;
             q.sBk = tb ? ap.kc : ap.kc * p.ldb;
-            hipError_t e = ntg::launch_gemm_any(dtype, ta, tb, q, s);
+            hipError_t e = int_planes_of(dtype) ? ntg::launch_gemm_int(int_planes_of(dtype), ta, tb, q, s) : ntg::launch_gemm_any(dtype, ta, tb, q, s);
             if (e != hipSuccess) return hip_fail(e, "gemm launch");
             e = ntg::launch_splitk_reduce(dtype, workspace, ap.splits, p, ap.ldp, s);
             if (e != hipSuccess) return hip_fail(e, "split-K reduction launch");
@@ -721,10 +695,7 @@ int64_t ntg_gemm_workspace_bytes(const ntg_gemm_desc* d) {
     ntg::GemmParams p;
     if (desc_to_params(d, p)) return -1;
     if (p.M == 0 || p.N == 0 || p.batch == 0) return 0;
-    if (int_planes_of(d->dtype)) {
-        const IntPlanesPlan ip = plan_int_planes(p, d->dtype);
-        return ip.ok ? ip.bytes() : 0;
-    }
+    if (int_planes_of(d->dtype)) return int_workspace_bytes(p, d->dtype);
     {
         const AnySplitPlan ap = plan_any_split(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0);
         const PadPlan pp = plan_pad(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0);      // pointers taken as 16-byte aligned
@@ -742,7 +713,15 @@ int ntg_gemm_noalloc_dev(const ntg_gemm_desc* d, const void* dA, const void* dB,
     if (p.batch > 1 && p.sC == 0) return fail(NTG_ERR_INVALID_ARGUMENT, "stride_c must be non-zero for a batch (outputs may not alias)");
     const int64_t need = ntg_gemm_workspace_bytes(d);
     if (need < 0) return fail(NTG_ERR_INVALID_ARGUMENT, "bad descriptor");
-    if (need > (int64_t)NTG_NOALLOC_SCRATCH_BYTES)
+    // k ranges of rows that start anywhere are planned for one item: a batch whose sums do not fit goes out in groups that do, the same bits
+    int group = p.batch;
+    if (need > (int64_t)NTG_NOALLOC_SCRATCH_BYTES && p.batch > 1) {
+        const bool ta = d->transpose_a != 0, tb = d->transpose_b != 0;
+        const AnySplitPlan ap = plan_any_split(p, d->dtype, ta, tb);
+        const PadPlan pp = plan_pad(p, d->dtype, ta, tb);
+        if (ap.splits > 1 && !(pp.ok && pp.bytes() > (int64_t)NTG_NOALLOC_SCRATCH_BYTES)) group = (int)((int64_t)NTG_NOALLOC_SCRATCH_BYTES / (ap.bytes / p.batch));
+    }
+    if (need > (int64_t)NTG_NOALLOC_SCRATCH_BYTES && group == p.batch)
         return fail(NTG_ERR_INVALID_ARGUMENT, "this product's workspace form needs %lld bytes, the static scratch of ntg_gemm_noalloc_dev holds %lld: "
                     "call ntg_gemm_dev with a workspace of the caller's, or ntg_gemm_dev without a workspace (the plain kernels: they allocate "
                     "nothing either, but a split along k is then not taken and floating-point sums may differ in their last bits)",
@@ -761,7 +740,16 @@ int ntg_gemm_noalloc_dev(const ntg_gemm_desc* d, const void* dA, const void* dB,
     }
     const bool ordered = capture == hipStreamCaptureStatusNone;
     if (ordered && st->used && st->last_stream != s) HIP_TRY(hipStreamWaitEvent(s, st->done, 0));     // the previous user of the array finishes first
-    rc = run_gemm(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0, s, st->ptr, need);
+    const int64_t es = ntg::elem_size(d->dtype);
+    for (int first = 0; first < p.batch && rc == NTG_OK; first += group) {
+        ntg::GemmParams q = p;
+        q.batch = std::min(group, p.batch - first);
+        q.A = static_cast<const char*>(p.A) + first * p.sA * es;
+        q.B = static_cast<const char*>(p.B) + first * p.sB * es;
+        q.C = static_cast<char*>(p.C) + first * p.sC * es;
+        if (p.bias) q.bias = static_cast<const char*>(p.bias) + first * p.bias_bs * es;
+        rc = run_gemm(q, d->dtype, d->transpose_a != 0, d->transpose_b != 0, s, st->ptr, std::min<int64_t>(need, NTG_NOALLOC_SCRATCH_BYTES));
+    }
     if (ordered) {
         HIP_TRY(hipEventRecord(st->done, s));
         st->last_stream = s;

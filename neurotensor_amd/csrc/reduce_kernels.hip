@@ -237,6 +237,9 @@ hipError_t launch_splitk_reduce(int dtype, const void* part, int splits, const G
     case DT_F16: launch_splitk_reduce_t<_Float16, float, float>(part, splits, p, ldp, s); break;
     case DT_BF16: launch_splitk_reduce_t<__bf16, float, float>(part, splits, p, ldp, s); break;
     case DT_I8: case DT_U8: launch_splitk_reduce_t<uint8_t, int, int>(part, splits, p, ldp, s); break;      // (the low 8 bits, either signedness)
+    case DT_I16: case DT_U16: launch_splitk_reduce_t<uint16_t, uint16_t, uint16_t>(part, splits, p, ldp, s); break;
+    case DT_I32: case DT_U32: launch_splitk_reduce_t<uint32_t, uint32_t, uint32_t>(part, splits, p, ldp, s); break;
+    case DT_I64: case DT_U64: launch_splitk_reduce_t<uint64_t, uint64_t, uint64_t>(part, splits, p, ldp, s); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -108,3 +108,28 @@ def test_float32_without_workspace_is_the_reference_chain_bit_for_bit():
         _lib.check(lib.ntg_gemm_dev(ctypes.byref(d), da.data_ptr(), db.data_ptr(), dc.data_ptr(), st))
         want = oracle.matmult2d(sa, sb, c0.copy(), ta, tb)
         assert np.array_equal(dc.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+INTS = {"i16": (np.int16, torch.int16), "i32": (np.int32, torch.int32), "i64": (np.int64, torch.int64)}
+
+
+@pytest.mark.parametrize("name", sorted(INTS))
+@pytest.mark.parametrize("ta,tb", TRANS)
+def test_wide_integers_from_digits(name, ta, tb):
+    """The whole range of values, wrapping: edges of tiles, K-steps and groups of eight, k ranges, both tile heights, a broadcast operand, C added to."""
+    rng = np.random.default_rng(9)
+    npdt, dt = INTS[name]
+    full = lambda *shape: rng.integers(-2**63, 2**63 - 1, shape, dtype=np.int64, endpoint=True).astype(npdt)
+    for m, k, n, batch in ((33, 9, 8, 1), (8, 8, 9, 1), (63, 33, 65, 1), (65, 31, 63, 2), (1, 40, 70, 1), (129, 64, 66, 1), (140, 1031, 150, 1), (200, 40, 299, 64), (5, 7, 6, 1)):
+        lead = (batch,) if batch > 1 else ()
+        a, b = full(*lead, *((k, m) if ta else (m, k))), full(*((n, k) if tb else (k, n)))
+        c0 = full(*lead, m, n)
+        a[..., 0, 0], b[0, 0] = np.iinfo(npdt).min, np.iinfo(npdt).min
+        A = (np.swapaxes(a, -1, -2) if ta else a).astype(np.int64).view(np.uint64)
+        B = (b.T if tb else b).astype(np.int64).view(np.uint64)
+        want = A @ B
+        got = F.matmult(torch.from_numpy(a).to(DEV), torch.from_numpy(b).to(DEV), None, ta, tb).cpu().numpy()
+        assert np.array_equal(got, want.astype(npdt)), (m, k, n)
+        out = torch.from_numpy(c0.copy()).to(DEV)
+        F.matmult(torch.from_numpy(a).to(DEV), torch.from_numpy(b).to(DEV), out, ta, tb)
+        assert np.array_equal(out.cpu().numpy(), (want + c0.astype(np.int64).view(np.uint64)).astype(npdt)), (m, k, n)
