@@ -7,9 +7,11 @@
 //
 //   * 64 x 64, 128 x 64 or 128 x 128 tiles, four wavefronts of WBM x WBN blocks of 32 x 32; a K-step is 128 bytes of k per row.
 //   * DEPTH K-steps of loads in flight per thread (registers), two LDS stages, one barrier per K-step: while a K-step is multiplied the next one
-//     is written to the other stage.  Every load is unconditional: a
-//     chunk that the end of its row cuts off is loaded from the row's last 16 bytes and shifted into place on its way to LDS, which
-//     also fills it up with zeros (rows past the edge repeat the last one; their sums are never stored).
+//     is written to the other stage.  Every load is unconditional.  In the last K-step a chunk that the end of its row cuts off is loaded from the
+//     row's last 16 bytes and shifted into place on its way to LDS, which also fills it up with zeros; before it nothing is shifted, also on the
+//     edge of M and N, so one loop serves every tile (shifting there behind a test per chunk made the compiler wait for each load by itself, and
+//     the tiles on the edge set the pace: 1023 x 1537 x 1985 on 128 x 128 31.3 -> 26.5 us).  Rows past the edge
+//     repeat the last one; their sums are never stored.
 //   * The sums go through LDS to memory, eight consecutive columns per lane.
 //   * k ranges (krange_items, k_total): the last range is what is left, ranges write sums in 32 bits (C_PARTIAL).
 //
@@ -48,10 +50,10 @@ struct AnyOperand {
     int64_t adv;
     uint32_t pitch;                                      // bytes from a stored row to the next
     uint32_t off[KC ? NV : 1];                           // byte offsets of the chunks (M/N-contiguous: of the first, the others RSTEP rows apart)
-    uint32_t last_step;                                  // K-contiguous: what the last K-step adds to them
+    uint32_t last_step;                                  // what the last K-step adds to them
     int krow, kr;                                        // M/N-contiguous: k-row of the first chunk; k-rows that exist in the last K-step
-    int lds, cut;                                        // LDS bytes of the first chunk; bytes to shift down by (16: nothing of it exists): K-contiguous: in the last K-step
-    bool edge;                                           // (uniform) some chunk is cut off in every K-step
+    int lds, cut;                                        // LDS bytes of the first chunk; bytes to shift it down by in the last K-step (16: nothing of it exists)
+    bool cut_last;                                       // (uniform) some chunk of the last K-step does not exist as a whole
 
     __device__ __forceinline__ void setup(const NTG_GLOBAL char* first, int64_t ld, int mn0, int MN, int K, int last, int tid) {
         kr = K - last * BK;
@@ -60,7 +62,7 @@ struct AnyOperand {
             base = first + (int64_t)mn0 * ld * ES;
             base_last = base + (int64_t)(K - BK) * ES;
             adv = 128;
-            edge = false;
+            cut_last = kr < BK;
             const int row = tid >> 3, slot = tid & 7;
             const int k = last * BK + slot * VEL, at = k < K - VEL ? k : K - VEL;           // (K - BK <= at: what base_last lacks is not negative)
             last_step = (uint32_t)((at - (K - BK) - slot * VEL) * ES);
@@ -77,14 +79,16 @@ struct AnyOperand {
             base = first + (int64_t)mn0 * ES - 16;
             base_last = base + (int64_t)last * BK * ld * ES;
             adv = (int64_t)BK * ld * ES;
-            edge = mn0 + 64 * WB > MN;
+            cut_last = kr < BK || mn0 + 64 * WB > MN;
             krow = tid / CH;
-            const int c = tid % CH, mn = mn0 + c * VEL, at = mn < MN - VEL ? mn : MN - VEL;
+            // A chunk that the end of its row cuts off runs on into the next k-row, which holds a chunk at least: the columns past the edge are sums
+            // of their own, which nobody stores.  Only the last k-row has none behind it: the last K-step loads that chunk from the row's last 16 bytes.
+            const int c = tid % CH, mn = mn0 + c * VEL, at = mn < MN - VEL ? mn : MN - VEL, on = mn < MN ? mn : MN - VEL;
             cut = (mn - at) * ES < 16 ? (mn - at) * ES : 16;
-            off[0] = (uint32_t)krow * pitch + (uint32_t)((at - mn0 + VEL) * ES);
+            off[0] = (uint32_t)krow * pitch + (uint32_t)((on - mn0 + VEL) * ES);
+            last_step = (uint32_t)((at - on) * ES);
             const int sw = ES == 2 ? 2 * (krow & 3) : ES == 4 ? 8 * (krow & 1) : mn8_swizzle<CH>(krow);      // (the same for krow + RSTEP)
             lds = krow * ROW + ((c ^ sw) << 4);
-            last_step = 0;
         }
     }
     __device__ __forceinline__ void load(u32x4& v, int i, int kt, int last) const {
@@ -96,14 +100,14 @@ struct AnyOperand {
             // (the last k-row once more in the place of those that do not exist)
             int k = krow + RSTEP * i;
             if (l) k = k < kr ? k : kr - 1;
-            o = off[0] + (uint32_t)(k - krow) * pitch;
+            o = off[0] + (uint32_t)(k - krow) * pitch + (l ? last_step : 0u);
         }
         v = *(const NTG_GLOBAL u32x4_any*)(b + o);
     }
-    // cut: some chunk of this K-step does not exist as a whole (uniform)
-    __device__ __forceinline__ void store(char* tile, const u32x4& v, int i, bool cut_off, bool lastk) const {
+    // cut_off: the last K-step, and some chunk of it does not exist as a whole (uniform)
+    __device__ __forceinline__ void store(char* tile, const u32x4& v, int i, bool cut_off) const {
         char* to = tile + lds + RSTEP * (KC ? 128 : ROW) * i;
-        if (cut_off) *reinterpret_cast<u32x4*>(to) = shift_down(v, KC ? (lastk ? cut : 0) : !lastk || krow + RSTEP * i < kr ? cut : 16);
+        if (cut_off) *reinterpret_cast<u32x4*>(to) = shift_down(v, KC || krow + RSTEP * i < kr ? cut : 16);
         else *reinterpret_cast<u32x4*>(to) = v;
     }
 };
@@ -167,7 +171,6 @@ __global__ void __launch_bounds__(256, WBM == 1 ? 3 : 2) gemm_any_kernel(const G
     }
 
     const int KT = (K + BK - 1) / BK, last = KT - 1;
-    const bool cut_k = K - last * BK < BK;
     OA a;
     OB bb;
     a.setup(A, p.lda, m0, p.M, K, last, tid);
@@ -230,11 +233,11 @@ __global__ void __launch_bounds__(256, WBM == 1 ? 3 : 2) gemm_any_kernel(const G
     };
     // K-step kt out of its stage; behind each quarter's matrix instructions a quarter of the chunks of K-step kt + 1 (set d) goes to the other
     // stage, which was last read before this K-step's barrier, and with MORE the loads of K-step kt + 1 + DEPTH take their registers
-    auto step = [&](int kt, int d, auto more_tag, bool special) __attribute__((always_inline)) {
-        constexpr bool MORE = decltype(more_tag)::value;
+    auto step = [&](int kt, int d, auto more_tag) __attribute__((always_inline)) {
+        constexpr bool MORE = decltype(more_tag)::value;         // (false: kt + 1 may be the last K-step)
         const char* sa = lds + (kt & 1) * STAGE;
         char* nx = lds + (~kt & 1) * STAGE;
-        const bool lastk = special && cut_k && kt + 1 == last, cut_a = lastk || (special && a.edge), cut_b = lastk || (special && bb.edge);
+        const bool lastk = !MORE && kt + 1 == last, cut_a = lastk && a.cut_last, cut_b = lastk && bb.cut_last;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
@@ -266,15 +269,15 @@ __global__ void __launch_bounds__(256, WBM == 1 ? 3 : 2) gemm_any_kernel(const G
                         E::mma(acc[i][j], fb[ks & 1][j], fa[ks & 1][i]);
                     }
                 }
-            if (!special || kt < last) {
+            if (MORE || kt < last) {
 #pragma unroll
                 for (int c = ks * (NVA + NVB) / 4; c < (ks + 1) * (NVA + NVB) / 4; ++c) {       // A's chunks, then B's
                     const int i = c < NVA ? c : c - NVA;
                     if (c < NVA) {
-                        a.store(nx, ra[d][i], i, cut_a, lastk);
+                        a.store(nx, ra[d][i], i, cut_a);
                         if constexpr (MORE) a.load(ra[d][i], i, kt + 1 + DEPTH, last);
                     } else {
-                        bb.store(nx + TILE_A, rb[d][i], i, cut_b, lastk);
+                        bb.store(nx + TILE_A, rb[d][i], i, cut_b);
                         if constexpr (MORE) bb.load(rb[d][i], i, kt + 1 + DEPTH, last);
                     }
                 }
@@ -282,32 +285,26 @@ __global__ void __launch_bounds__(256, WBM == 1 ? 3 : 2) gemm_any_kernel(const G
         }
     };
     {
-        const bool lastk = cut_k && last == 0, edge = lastk || a.edge, edge_b = lastk || bb.edge;
+        const bool cut_a = last == 0 && a.cut_last, cut_b = last == 0 && bb.cut_last;
 #pragma unroll
         for (int i = 0; i < NVA; ++i) {
-            a.store(lds, ra[0][i], i, edge, lastk);
+            a.store(lds, ra[0][i], i, cut_a);
             a.load(ra[0][i], i, DEPTH, last);
         }
 #pragma unroll
         for (int i = 0; i < NVB; ++i) {
-            bb.store(lds + TILE_A, rb[0][i], i, edge_b, lastk);
+            bb.store(lds + TILE_A, rb[0][i], i, cut_b);
             bb.load(rb[0][i], i, DEPTH, last);
         }
     }
     // (K-step kt + 1 is in set (kt + 1) % DEPTH; the rounds end before the last K-step is written to LDS)
     int kt = 0;
-    if (a.edge || bb.edge) {                                       // (uniform) a tile on the edge of an operand stored along it
-        for (; kt + DEPTH <= last - 1; kt += DEPTH)
+    for (; kt + DEPTH <= last - 1; kt += DEPTH)
 #pragma unroll
-            for (int d = 0; d < DEPTH; ++d) step(kt + d, (d + 1) % DEPTH, std::true_type{}, true);
-    } else {
-        for (; kt + DEPTH <= last - 1; kt += DEPTH)
-#pragma unroll
-            for (int d = 0; d < DEPTH; ++d) step(kt + d, (d + 1) % DEPTH, std::true_type{}, false);
-    }
+        for (int d = 0; d < DEPTH; ++d) step(kt + d, (d + 1) % DEPTH, std::true_type{});
 #pragma unroll
     for (int d = 0; d < DEPTH + 1; ++d)
-        if (kt + d <= last) step(kt + d, (d + 1) % DEPTH, std::false_type{}, true);     // (uniform)
+        if (kt + d <= last) step(kt + d, (d + 1) % DEPTH, std::false_type{});     // (uniform)
 
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();                                  // all fragments read: LDS is free for the sums
@@ -415,13 +412,14 @@ static hipError_t launch_any_wb(bool ta, bool tb, const GemmParams& pin, hipStre
 }
 template <int DT>
 static hipError_t launch_any(bool ta, bool tb, const GemmParams& p, hipStream_t s) {
-    // 128 x 128 tiles where these reach three quarters of the CUs (BFloat16 3618 x 739 x 9392: 96 us against 139 on 64 x 64; 2429 x 1536 x 157,
-    // 38 tiles: 28 against 14), 128 x 64 where those put one on each CU at most and 64 x 64 more than one (Float16 1023 x 1537 x 1985: 21.3 us against
-    // 25.2 and 31.3 on 128 x 128; 624 x 1024 x 51 by 47 16.0 against 16.8).  Float32 always on 64 x 64: the matrix pipe is its bound on either and
-    // the smaller tile spreads evenly (2049^3: 188 us against 274).
+    // 128 x 128 tiles where these reach three quarters of the CUs (BFloat16 3618 x 739 x 9392: 84 us against 112 on 128 x 64 and 126 on 64 x 64;
+    // 2429 x 1536 x 157, 38 tiles: 23 against 12), 128 x 64 where those put one on each CU at most and 64 x 64 more than one (Float16 1023 x 1537 x
+    // 1985: 18.6 us against 21.6 and 26.5 on 128 x 128), and 128 x 128 again from half of the CUs on where 128 x 64 would need a second round (1023 x 1537
+    // x 2049, 136 tiles: 26.7 against 30 on either; 1337 x 777 x 1555, 143 tiles: 18.2, 19.0 and 17.6).  Float32 always on 64 x 64: the matrix pipe
+    // is its bound on either and the smaller tile spreads evenly (2049^3: 188 us against 274).
     if constexpr (DT != DT_F32) {
         auto tiles = [&](int r, int c) { return (int64_t)((p.M + r - 1) / r) * ((p.N + c - 1) / c) * p.batch; };
-        if (p.M > 64 && p.N > 64 && tiles(128, 128) >= 192) return launch_any_wb<DT, 2, 2>(ta, tb, p, s);
+        if (p.M > 64 && p.N > 64 && (tiles(128, 128) >= 192 || (tiles(128, 128) >= 128 && tiles(128, 64) > 256))) return launch_any_wb<DT, 2, 2>(ta, tb, p, s);
         if (p.M > 64 && tiles(64, 64) > 256 && tiles(128, 64) <= 256) return launch_any_wb<DT, 2, 1>(ta, tb, p, s);
     }
     return launch_any_wb<DT, 1, 1>(ta, tb, p, s);

@@ -308,10 +308,12 @@ static PadPlan plan_pad(const ntg::GemmParams& p, int dtype, bool ta, bool tb) {
     if (pl.padC) pl.c_bytes = (int64_t)align_up((size_t)((int64_t)p.batch * pl.Mp * pl.Np * es), 256);
     pl.ok = true;
     // The kernel that takes rows as they lie (gemm_any_impl.h) makes whole copies pay later; where only the last k-rows are copied they are as good
-    // as free.  Copies against no copies: Float16 1023 x 1537 x 2049 (3.2e9) 31.0 us against 31.3, BFloat16 2813 x 803 x 2240 (5.1e9) 29.2 against 26.7,
-    // 2049^3 (8.6e9) 51.1 against 51.8, 3618 x 739 x 9392 (2.5e10) 79 against 96; Float32 2049^3 211 against 187, 1504 x 727 x 8952 (9.8e9) 180 against
-    // 191; Int8 2049^3 36.6 against 33.9, 1002 x 256 x 2432 12.2 against 7.5.  (The workspace is offered as if they paid: what a caller keeps stays enough.)
-    pl.pays = !(pl.padA || pl.padB || pl.padC) || !ntg::any_eligible(p, dtype, ta, tb) || macs >= (byte ? 1.7e10 : half ? 3.0e9 : dtype == ntg::DT_F32 ? 9.0e9 : 0.0);
+    // as free.  Copies against no copies: Float16 1023 x 1537 x 2049 (3.2e9) 30.4 us against 26.7, 27 x 1704 x 229 x 960 (1.0e10) 64 against 56, 8 x 1201 x
+    // 1301 x 903 (1.1e10) 57.2 against 53.7, 2049^3 (8.6e9) 50.4 against 49.7; BFloat16 2813 x 803 x 2240 (5.1e9) 28.0 against 23.3, 8192 x 999 x 999
+    // A^T.B (8.2e9) 40.8 against 29.8, 3618 x 739 x 9392 (2.5e10) 73 against 84, 4095^3 145 against 192; Float32 2049^3 211 against 187, 1504 x 727 x
+    // 8952 (9.8e9) 180 against 191; Int8 2049^3 36.7 against 33.3, 1002 x 257 x 2431 14.8 against 9.8.  (The workspace is offered as if they paid:
+    // what a caller keeps stays enough.)
+    pl.pays = !(pl.padA || pl.padB || pl.padC) || !ntg::any_eligible(p, dtype, ta, tb) || macs >= (byte ? 1.7e10 : half ? 1.6e10 : dtype == ntg::DT_F32 ? 9.0e9 : 0.0);
     return pl;
 }
 static int run_padded(const ntg::GemmParams& p, const PadPlan& pl, int dtype, bool ta, bool tb, void* ws, hipStream_t s) {

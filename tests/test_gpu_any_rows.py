@@ -20,7 +20,7 @@ UNIT = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8, "f32": 2.0 ** -24}
 TRANS = [(False, False), (False, True), (True, False), (True, True)]
 # one element past / before a tile, a K-step, a chunk; one row; the shortest rows that hold a chunk; k ranges with a short last one
 SIZES = [(33, 17, 17), (63, 65, 64), (64, 63, 65), (65, 129, 127), (40, 16, 19), (1, 33, 18), (129, 257, 31), (1700, 40, 1030),
-         (70, 2049, 66), (37, 3001, 130), (200, 1100, 77)]
+         (70, 2049, 66), (37, 3001, 130), (200, 1100, 77), (1025, 401, 2049)]
 
 
 def values(shape, name, gen):
@@ -48,6 +48,19 @@ def test_sizes_at_the_edges(name, ta, tb):
         a, b = values((k, m) if ta else (m, k), name, gen), values((n, k) if tb else (k, n), name, gen)
         got = F.matmult(a.to(DEV), b.to(DEV), None, ta, tb).cpu()
         check(got, a.t() if ta else a, b.t() if tb else b, None, name, k)
+
+
+@pytest.mark.parametrize("name", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("ta,tb", TRANS)
+def test_infinities_stay_in_their_row_and_column(name, ta, tb):
+    """What a chunk on the edge reads of the next k-row reaches no sum."""
+    gen = torch.Generator().manual_seed(9)
+    for m, k, n in ((67, 300, 69), (131, 1100, 130)):
+        a, b = values((m, k), name, gen).abs() + 1, values((k, n), name, gen).abs() + 1
+        a[0, 1:] = float("inf")
+        b[1:, 0] = float("inf")
+        got = F.matmult((a.t() if ta else a).contiguous().to(DEV), (b.t() if tb else b).contiguous().to(DEV), None, ta, tb).cpu()
+        assert torch.isinf(got[0]).all() and torch.isinf(got[:, 0]).all() and torch.isfinite(got[1:, 1:]).all()
 
 
 @pytest.mark.parametrize("name", sorted(DTYPES))
