@@ -204,7 +204,8 @@ typedef struct ntg_gemm_desc {
 
 /* Bytes of workspace with which ntg_gemm_dev runs its faster form (0: there is none for this product): a split along k
  * for shapes such as [256, 8192] x [8192, 8192] (planned from one item's sizes, so a batch is offered its item's split with
- * the partial sums of every item); zero-padded copies of large 8-bit, 16-bit, Float32 and Float64 operands whose rows, pitches
+ * the partial sums of every item; a batch of rows that miss the 16-byte rule and that fills the GPU by itself runs its items' ranges without
+ * going through memory: 256 bytes are asked for, which give the leave to change the order of summation and are not written); zero-padded copies of large 8-bit, 16-bit, Float32 and Float64 operands whose rows, pitches
  * or base pointers are not 16-byte multiples, so that they run on the DMA-fed kernels (same results: zeros add nothing);
  * or, for large Int16 / Int32 / Int64 products and their unsigned forms, room for k ranges (these run as 3 / 10 / 36 products of balanced
  * digits on v_mfma_i32_32x32x32_i8 with or without it; the sum modulo 2^W is the reference's wrapping result,

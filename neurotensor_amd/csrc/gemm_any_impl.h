@@ -14,6 +14,8 @@
 //     repeat the last one; their sums are never stored.
 //   * The sums go through LDS to memory, eight consecutive columns per lane.
 //   * k ranges (krange_items, k_total): the last range is what is left, ranges write sums in 32 bits (C_PARTIAL).
+//   * FOLD (fold_steps): a batch whose tiles fill the CUs runs the k ranges of its item inside one workgroup, which adds up each range's sums in
+//     registers, from C0 or the bias on, as the second pass over partial sums does: the bits of the item alone, nothing through memory.
 //
 // What bounds it: the latency of the loads where few tiles have a deep k (hence the k ranges, and 64 x 64 tiles that put several workgroups
 // on every CU), the LDS of the CU where there are many (64 x 64 tiles read 256 bytes of LDS per cycle of MFMA, twice what it delivers).
@@ -112,7 +114,7 @@ struct AnyOperand {
     }
 };
 
-template <int DT, bool TA, bool TB, int WBM, int WBN>
+template <int DT, bool TA, bool TB, int WBM, int WBN, bool FOLD>
 __global__ void __launch_bounds__(256, WBM == 1 ? 3 : 2) gemm_any_kernel(const GemmParams p) {
     using E = Elem<DT>;
     using T = typename E::T;
@@ -145,14 +147,17 @@ __global__ void __launch_bounds__(256, WBM == 1 ? 3 : 2) gemm_any_kernel(const G
     const gptr_mut<char> C = (gptr_mut<char>)(p.Cptr ? static_cast<char*>(((gptr<void*>)p.Cptr)[b]) : static_cast<char*>(p.C) + (int64_t)b * p.sC * ces);
     const NTG_GLOBAL T* bias = (const NTG_GLOBAL T*)static_cast<const T*>(p.bias) + (int64_t)b * p.bias_bs;
 
-    AccV acc[WBM][WBN];
+    AccV acc[WBM][WBN], tot[FOLD ? WBM : 1][FOLD ? WBN : 1];
 #pragma unroll
     for (int i = 0; i < WBM; ++i)
 #pragma unroll
         for (int j = 0; j < WBN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = (AccS)0;
-    if constexpr (CHAIN) {
+            for (int r = 0; r < 16; ++r) {
+                acc[i][j][r] = (AccS)0;
+                if constexpr (FOLD) tot[i][j][r] = (AccS)0;
+            }
+    if constexpr (CHAIN || FOLD) {
         if (p.cmode == C_ACCUMULATE || p.cmode == C_BIAS) {        // (uniform)
             const bool from_c = p.cmode == C_ACCUMULATE;
 #pragma unroll
@@ -165,7 +170,9 @@ __global__ void __launch_bounds__(256, WBM == 1 ? 3 : 2) gemm_any_kernel(const G
                         int m = m0 + wm * WTM + 32 * i + (lane & 31), n = n0 + wn * WTN + 32 * j + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
                         m = m < p.M ? m : p.M - 1;
                         n = n < p.N ? n : p.N - 1;
-                        acc[i][j][r] = from_c ? ((gptr<float>)C)[(int64_t)m * p.ldc + n] : bias[(int64_t)m * p.bias_rs + (int64_t)n * p.bias_cs];
+                        const AccS c0 = (AccS)(from_c ? ((gptr<T>)C)[(int64_t)m * p.ldc + n] : bias[(int64_t)m * p.bias_rs + (int64_t)n * p.bias_cs]);
+                        if constexpr (FOLD) tot[i][j][r] = c0;
+                        else acc[i][j][r] = c0;
                     }
         }
     }
@@ -231,6 +238,7 @@ __global__ void __launch_bounds__(256, WBM == 1 ? 3 : 2) gemm_any_kernel(const G
             }
         }
     };
+    int fold_at = p.fold_steps - 1;                                // FOLD: the K-step that ends the range
     // K-step kt out of its stage; behind each quarter's matrix instructions a quarter of the chunks of K-step kt + 1 (set d) goes to the other
     // stage, which was last read before this K-step's barrier, and with MORE the loads of K-step kt + 1 + DEPTH take their registers
     auto step = [&](int kt, int d, auto more_tag) __attribute__((always_inline)) {
@@ -283,6 +291,20 @@ __global__ void __launch_bounds__(256, WBM == 1 ? 3 : 2) gemm_any_kernel(const G
                 }
             }
         }
+        if constexpr (FOLD) {
+            if (kt == fold_at || kt == last) {                     // (uniform)
+                fold_at += p.fold_steps;
+#pragma unroll
+                for (int i = 0; i < WBM; ++i)
+#pragma unroll
+                    for (int j = 0; j < WBN; ++j)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            tot[i][j][r] += acc[i][j][r];
+                            acc[i][j][r] = (AccS)0;
+                        }
+            }
+        }
     };
     {
         const bool cut_a = last == 0 && a.cut_last, cut_b = last == 0 && bb.cut_last;
@@ -321,8 +343,8 @@ __global__ void __launch_bounds__(256, WBM == 1 ? 3 : 2) gemm_any_kernel(const G
 #pragma unroll
             for (int rq = 0; rq < 4; ++rq) {
                 const int row = wm * WTM + 32 * i + (lane & 31), slot = (wn * WTN + 32 * j) / 4 + 2 * rq + (lane >> 5);
-                *reinterpret_cast<accx4*>(lds + row * SROW + ((slot ^ (row & 7)) << 4)) =
-                    accx4{acc[i][j][4 * rq], acc[i][j][4 * rq + 1], acc[i][j][4 * rq + 2], acc[i][j][4 * rq + 3]};
+                const AccV& s = FOLD ? tot[FOLD ? i : 0][FOLD ? j : 0] : acc[i][j];
+                *reinterpret_cast<accx4*>(lds + row * SROW + ((slot ^ (row & 7)) << 4)) = accx4{s[4 * rq], s[4 * rq + 1], s[4 * rq + 2], s[4 * rq + 3]};
             }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -344,7 +366,7 @@ __global__ void __launch_bounds__(256, WBM == 1 ? 3 : 2) gemm_any_kernel(const G
             continue;
         }
         NTG_GLOBAL T* cp = (NTG_GLOBAL T*)C + (int64_t)m * p.ldc + n;
-        if constexpr (!CHAIN) {
+        if constexpr (!CHAIN && !FOLD) {
             if (p.cmode == C_ACCUMULATE) {
                 if (whole) {
                     if constexpr (ES == 2) {
@@ -396,7 +418,7 @@ __global__ void __launch_bounds__(256, WBM == 1 ? 3 : 2) gemm_any_kernel(const G
     }
 }
 
-template <int DT, int WBM, int WBN>
+template <int DT, int WBM, int WBN, bool FOLD>
 static hipError_t launch_any_wb(bool ta, bool tb, const GemmParams& pin, hipStream_t s) {
     GemmParams p = pin;
     p.tiles_m = (p.M + 64 * WBM - 1) / (64 * WBM);
@@ -404,14 +426,14 @@ static hipError_t launch_any_wb(bool ta, bool tb, const GemmParams& pin, hipStre
     const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n * p.batch;
     if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
     const dim3 g((unsigned)blocks), t(256);
-    if (ta && tb) hipLaunchKernelGGL((gemm_any_kernel<DT, true, true, WBM, WBN>), g, t, 0, s, p);
-    else if (ta) hipLaunchKernelGGL((gemm_any_kernel<DT, true, false, WBM, WBN>), g, t, 0, s, p);
-    else if (tb) hipLaunchKernelGGL((gemm_any_kernel<DT, false, true, WBM, WBN>), g, t, 0, s, p);
-    else hipLaunchKernelGGL((gemm_any_kernel<DT, false, false, WBM, WBN>), g, t, 0, s, p);
+    if (ta && tb) hipLaunchKernelGGL((gemm_any_kernel<DT, true, true, WBM, WBN, FOLD>), g, t, 0, s, p);
+    else if (ta) hipLaunchKernelGGL((gemm_any_kernel<DT, true, false, WBM, WBN, FOLD>), g, t, 0, s, p);
+    else if (tb) hipLaunchKernelGGL((gemm_any_kernel<DT, false, true, WBM, WBN, FOLD>), g, t, 0, s, p);
+    else hipLaunchKernelGGL((gemm_any_kernel<DT, false, false, WBM, WBN, FOLD>), g, t, 0, s, p);
     return hipGetLastError();
 }
-template <int DT>
-static hipError_t launch_any(bool ta, bool tb, const GemmParams& p, hipStream_t s) {
+template <int DT, bool FOLD>
+static hipError_t launch_any_tile(bool ta, bool tb, const GemmParams& p, hipStream_t s) {
     // 128 x 128 tiles where these reach three quarters of the CUs (BFloat16 3618 x 739 x 9392: 84 us against 112 on 128 x 64 and 126 on 64 x 64;
     // 2429 x 1536 x 157, 38 tiles: 23 against 12), 128 x 64 where those put one on each CU at most and 64 x 64 more than one (Float16 1023 x 1537 x
     // 1985: 18.6 us against 21.6 and 26.5 on 128 x 128), and 128 x 128 again from half of the CUs on where 128 x 64 would need a second round (1023 x 1537
@@ -419,10 +441,16 @@ static hipError_t launch_any(bool ta, bool tb, const GemmParams& p, hipStream_t 
     // is its bound on either and the smaller tile spreads evenly (2049^3: 188 us against 274).
     if constexpr (DT != DT_F32) {
         auto tiles = [&](int r, int c) { return (int64_t)((p.M + r - 1) / r) * ((p.N + c - 1) / c) * p.batch; };
-        if (p.M > 64 && p.N > 64 && (tiles(128, 128) >= 192 || (tiles(128, 128) >= 128 && tiles(128, 64) > 256))) return launch_any_wb<DT, 2, 2>(ta, tb, p, s);
-        if (p.M > 64 && tiles(64, 64) > 256 && tiles(128, 64) <= 256) return launch_any_wb<DT, 2, 1>(ta, tb, p, s);
+        if (p.M > 64 && p.N > 64 && (tiles(128, 128) >= 192 || (tiles(128, 128) >= 128 && tiles(128, 64) > 256))) return launch_any_wb<DT, 2, 2, FOLD>(ta, tb, p, s);
+        if (p.M > 64 && tiles(64, 64) > 256 && tiles(128, 64) <= 256) return launch_any_wb<DT, 2, 1, FOLD>(ta, tb, p, s);
     }
-    return launch_any_wb<DT, 1, 1>(ta, tb, p, s);
+    return launch_any_wb<DT, 1, 1, FOLD>(ta, tb, p, s);
+}
+template <int DT>
+static hipError_t launch_any(bool ta, bool tb, const GemmParams& p, hipStream_t s) {
+    if constexpr (DT != DT_I8)
+        if (p.fold_steps) return launch_any_tile<DT, true>(ta, tb, p, s);
+    return launch_any_tile<DT, false>(ta, tb, p, s);
 }
 
 }  // namespace ntg

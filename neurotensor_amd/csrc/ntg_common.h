@@ -103,6 +103,7 @@ struct GemmParams {
     int krange_items;
     int64_t sAk, sBk;
     int k_total;             // k ranges of unequal length (gemm_any_impl.h): K is a range's length, the last one has what is left of k_total; 0: all equal
+    int fold_steps;          // k ranges inside one workgroup (gemm_any_impl.h): K-steps in each but the last; 0: none
     int M, N, K, batch;      // logical sizes (after the transpose flags)
     int cmode;
     int tiles_m, tiles_n;

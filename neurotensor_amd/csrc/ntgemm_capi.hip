@@ -429,7 +429,10 @@ SplitPlan plan_splitk(const ntg::GemmParams& p, int dtype, bool ta) {
 // k ranges of a product whose rows miss the 16-byte rule by their SIZES (gemm_any_impl.h serves it): as plan_splitk a function of one item's
 // sizes and pitches only.  kc is a whole number of K-steps, the last range is what is left.  Rows of the partial sums hold whole 16-byte chunks.
 // The integers of more than a byte likewise (gemm_int_impl.h).
-struct AnySplitPlan { int splits; int64_t kc, ldp, bytes; };
+// inside: a workgroup runs all ranges of its tile (the sums of these are added in registers, in the order of the second pass: the same bits).  It needs
+// no room; 256 bytes stand for the caller's leave to change the order of summation, which a workspace is.
+struct AnySplitPlan { int splits; int64_t kc, ldp, bytes; bool inside; };
+constexpr int64_t INSIDE_BYTES = 256;
 // Room that ntg_gemm_workspace_bytes offers large integer products (and ntg_gemm_noalloc_dev takes them with or refuses them for): the digits of both
 // operands and the 32-bit sums of every shift.  The product itself needs none; its k ranges take what they use of it.
 static int64_t int_workspace_bytes(const ntg::GemmParams& p, int dtype) {
@@ -448,7 +451,7 @@ static int64_t int_workspace_bytes(const ntg::GemmParams& p, int dtype) {
 // whole 48 us, 8 / 16 ranges 12.4 / 10.8; Int16 709 x 3136 x 450, ranges 1 / 4 / 8 / 16: 36 / 16.9 / 15.8 / 19.4; Int64 576 x 3968 x 281, 1 / 4 / 8: 183 / 53 / 58).
 // The sums wrap, so their order is nobody's concern: the batch counts among the tiles.  room: bytes of workspace there are.
 AnySplitPlan plan_int_split(const ntg::GemmParams& p, int dtype, bool ta, bool tb, int64_t room) {
-    AnySplitPlan pl{1, p.K, (p.N + 3) / 4 * 4, 0};
+    AnySplitPlan pl{1, p.K, (p.N + 3) / 4 * 4, 0, false};
     if (p.batch < 1 || p.batch > 65535 || p.Aptr || p.Bptr || p.Cptr || !int_pipe_eligible(p, dtype, ta, tb)) return pl;
     const int P = int_planes_of(dtype);
     const int64_t steps = (p.K + 31) / 32, tiles = ((p.M + 63) / 64) * ((p.N + 63) / 64) * (int64_t)p.batch;
@@ -464,37 +467,57 @@ AnySplitPlan plan_int_split(const ntg::GemmParams& p, int dtype, bool ta, bool t
     return pl;
 }
 AnySplitPlan plan_any_split(const ntg::GemmParams& p, int dtype, bool ta, bool tb) {
-    AnySplitPlan none{1, p.K, 0, 0};
-    if (p.batch < 1 || p.batch > 65535 || p.Aptr || p.Bptr || p.Cptr || p.keep_k_order || !ntg::any_eligible(p, dtype, ta, tb)) return none;
+    AnySplitPlan none{1, p.K, 0, 0, false};
     const bool byte = dtype == ntg::DT_I8 || dtype == ntg::DT_U8;
+    if (p.batch < 1 || (byte && p.batch > 65535) || p.Aptr || p.Bptr || p.Cptr || p.keep_k_order || !ntg::any_eligible(p, dtype, ta, tb)) return none;
     if (p.M <= 32 && !byte) return none;                           // the streaming kernels take these
     const int64_t es = ntg::elem_size(dtype), ve = 16 / es, bk = 128 / es;
     if (p.K % ve == 0 && p.N % ve == 0 && (!ta || p.M % ve == 0) && p.lda % ve == 0 && p.ldb % ve == 0 && p.ldc % ve == 0) return none;
-    const int64_t tiles = ((p.M + 63) / 64) * ((p.N + 63) / 64), steps = (p.K + bk - 1) / bk;
+    // (the ranges of a float are one item's: an item comes out bit for bit the same alone and in a batch.  Bytes wrap: the batch counts among the tiles)
+    const int64_t items = byte ? p.batch : 1;
+    const int64_t tiles = ((p.M + 63) / 64) * ((p.N + 63) / 64) * items, steps = (p.K + bk - 1) / bk;
     if (tiles > 255) return none;
     // A workgroup alone on its CU spends 0.28 / 0.71 / 0.43 us (16-bit / Float32 / Int8) on each K-step, several on one CU 0.18 / 0.45 / 0.25 us
     // each; a launch costs about 2.5 us, the second pass 4 us + the partial sums written and read at 4 TB/s.  Of 2 .. 32 ranges the choice was the
     // best measured one or within 10 % of it on fourteen shapes (BFloat16 576 x 3797 x 448, ranges 1 / 2 / 4 / 8: 19.6 / 16.5 / 13.0 / 14.5 us;
     // 448 x 3704 x 166: 25.9 us whole, 10.4 in eight ranges; Float32 128 x 6463 x 720: 146 us whole, 24 in 21 ranges).
     const double alone = byte ? 0.43 : es == 2 ? 0.28 : 0.71, shared = byte ? 0.25 : es == 2 ? 0.18 : 0.45;
-    auto estimate_us = [&](int64_t sp, int64_t per) {
-        const int64_t wgs = tiles * sp;
-        const double second_pass = sp == 1 ? 0.0 : 4.0 + 8.0 * (double)sp * (double)p.M * (double)p.N / 4.0e6;
+    auto estimate_us = [&](int64_t tls, int64_t its, int64_t sp, int64_t per) {
+        const int64_t wgs = tls * sp;
+        const double second_pass = sp == 1 ? 0.0 : 4.0 + 8.0 * (double)sp * (double)its * (double)p.M * (double)p.N / 4.0e6;
         return 2.5 + (double)per * (wgs <= 256 ? alone : shared * (double)((wgs + 255) / 256)) + second_pass;
     };
-    const double whole_us = estimate_us(1, steps);
+    const double whole_us = estimate_us(tiles, items, 1, steps);
     double best_us = 0.95 * whole_us;
     AnySplitPlan pl = none;
     for (int64_t sp = 2; sp <= 32 && sp <= steps / 2; ++sp) {
         const int64_t per = (steps + sp - 1) / sp, ranges = (steps + per - 1) / per;
-        const double us = estimate_us(ranges, per);
-        if (ranges * (int64_t)p.M * ((p.N + 3) / 4 * 4) * 4 > (int64_t)NTG_NOALLOC_SCRATCH_BYTES) break;      // (an item fits where nothing is allocated)
+        const double us = estimate_us(tiles, items, ranges, per);
+        if (ranges * items * (int64_t)p.M * ((p.N + 3) / 4 * 4) * 4 > (int64_t)NTG_NOALLOC_SCRATCH_BYTES) break;      // (fits where nothing is allocated)
         if (us < best_us) { best_us = us; pl.splits = (int)ranges; pl.kc = per * bk; }
     }
     if (pl.splits < 2) return none;
     pl.ldp = (p.N + 3) / 4 * 4;
     pl.bytes = (int64_t)pl.splits * p.batch * p.M * pl.ldp * 4;
+    if (!byte && p.batch > 1) {
+        // A batch: the items' ranges through memory, or inside a workgroup once the batch gives the CUs enough tiles (and where the sums would take more than
+        // 64 MiB).  Measured in 2 .. 64 items of six shapes, the choice is the better one or within 10 % of it: Float16 128 x 6463 x 721 through memory / inside,
+        // 6 items 30.7 / 37.0 us, 10 items 44.3 / 38.6, 32 items 148 / 113; Float32 200 x 1501 x 201, 6 items 25.9 / 36.7, 16 items 48.7 / 37.3, 64 items 175 /
+        // 114; Float16 1000 x (70 x 2049 x 66) 237 / 135, Float32 64 x (128 x 6463 x 720) 892 / 740.  A K-step inside takes at least 0.33 / 0.71 us (16-bit / Float32).
+        const int64_t all = tiles * p.batch;
+        const double rounds = (double)all / 256.0;
+        const double inside_us = es == 2 ? 5.5 + (double)steps * std::max(0.33, 0.3 * rounds) : 2.5 + (double)steps * std::max(0.71, 0.3 + 0.62 * rounds);
+        pl.inside = p.batch > 65535 || pl.bytes > (int64_t)NTG_NOALLOC_SCRATCH_BYTES || inside_us <= estimate_us(all, p.batch, pl.splits, pl.kc / bk);
+        if (pl.inside) pl.bytes = INSIDE_BYTES;
+    }
     return pl;
+}
+
+// the k ranges of a float's item inside one workgroup a tile: no workspace
+static int run_ranges_inside(ntg::GemmParams p, const AnySplitPlan& ap, int dtype, bool ta, bool tb, hipStream_t s) {
+    p.fold_steps = (int)(ap.kc * ntg::elem_size(dtype) / 128);
+    const hipError_t e = ntg::launch_gemm_any(dtype, ta, tb, p, s);
+    return e == hipSuccess ? NTG_OK : hip_fail(e, "gemm launch");
 }
 
 int run_gemm(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s, void* workspace = nullptr, int64_t workspace_bytes = 0) {
@@ -524,7 +547,10 @@ int run_gemm(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s, void
     }
     {
         const AnySplitPlan ap = int_planes_of(dtype) ? plan_int_split(p, dtype, ta, tb, workspace ? workspace_bytes : 0) : plan_any_split(p, dtype, ta, tb);
-        if (ap.splits > 1 && workspace && workspace_bytes >= ap.bytes && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0) {
+        const bool offered = ap.splits > 1 && workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0;
+        if (offered && workspace_bytes >= INSIDE_BYTES && (ap.inside || workspace_bytes < ap.bytes) && !is_int_dtype(dtype))
+            return run_ranges_inside(p, ap, dtype, ta, tb, s);
+        if (offered && !ap.inside && workspace_bytes >= ap.bytes) {
             // launch index = range * batch + item
             ntg::GemmParams q = p;
             q.K = (int)ap.kc;
@@ -700,8 +726,9 @@ int64_t ntg_gemm_workspace_bytes(const ntg_gemm_desc* d) {
     if (int_planes_of(d->dtype)) return int_workspace_bytes(p, d->dtype);
     {
         const AnySplitPlan ap = plan_any_split(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0);
+        if (ap.splits > 1) return ap.bytes;                        // (no padded copies beside k ranges)
         const PadPlan pp = plan_pad(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0);      // pointers taken as 16-byte aligned
-        if (pp.ok || ap.splits > 1) return std::max<int64_t>(ap.bytes, pp.ok ? pp.bytes() : 0);
+        if (pp.ok) return pp.bytes();
     }
     return plan_splitk(p, d->dtype, d->transpose_a != 0).bytes;      // pointers taken as 16-byte aligned
 }
@@ -715,15 +742,7 @@ int ntg_gemm_noalloc_dev(const ntg_gemm_desc* d, const void* dA, const void* dB,
     if (p.batch > 1 && p.sC == 0) return fail(NTG_ERR_INVALID_ARGUMENT, "stride_c must be non-zero for a batch (outputs may not alias)");
     const int64_t need = ntg_gemm_workspace_bytes(d);
     if (need < 0) return fail(NTG_ERR_INVALID_ARGUMENT, "bad descriptor");
-    // k ranges of rows that start anywhere are planned for one item: a batch whose sums do not fit goes out in groups that do, the same bits
-    int group = p.batch;
-    if (need > (int64_t)NTG_NOALLOC_SCRATCH_BYTES && p.batch > 1) {
-        const bool ta = d->transpose_a != 0, tb = d->transpose_b != 0;
-        const AnySplitPlan ap = plan_any_split(p, d->dtype, ta, tb);
-        const PadPlan pp = plan_pad(p, d->dtype, ta, tb);
-        if (ap.splits > 1 && !(pp.ok && pp.bytes() > (int64_t)NTG_NOALLOC_SCRATCH_BYTES)) group = (int)((int64_t)NTG_NOALLOC_SCRATCH_BYTES / (ap.bytes / p.batch));
-    }
-    if (need > (int64_t)NTG_NOALLOC_SCRATCH_BYTES && group == p.batch)
+    if (need > (int64_t)NTG_NOALLOC_SCRATCH_BYTES)
         return fail(NTG_ERR_INVALID_ARGUMENT, "this product's workspace form needs %lld bytes, the static scratch of ntg_gemm_noalloc_dev holds %lld: "
                     "call ntg_gemm_dev with a workspace of the caller's, or ntg_gemm_dev without a workspace (the plain kernels: they allocate "
                     "nothing either, but a split along k is then not taken and floating-point sums may differ in their last bits)",
@@ -742,16 +761,7 @@ int ntg_gemm_noalloc_dev(const ntg_gemm_desc* d, const void* dA, const void* dB,
     }
     const bool ordered = capture == hipStreamCaptureStatusNone;
     if (ordered && st->used && st->last_stream != s) HIP_TRY(hipStreamWaitEvent(s, st->done, 0));     // the previous user of the array finishes first
-    const int64_t es = ntg::elem_size(d->dtype);
-    for (int first = 0; first < p.batch && rc == NTG_OK; first += group) {
-        ntg::GemmParams q = p;
-        q.batch = std::min(group, p.batch - first);
-        q.A = static_cast<const char*>(p.A) + first * p.sA * es;
-        q.B = static_cast<const char*>(p.B) + first * p.sB * es;
-        q.C = static_cast<char*>(p.C) + first * p.sC * es;
-        if (p.bias) q.bias = static_cast<const char*>(p.bias) + first * p.bias_bs * es;
-        rc = run_gemm(q, d->dtype, d->transpose_a != 0, d->transpose_b != 0, s, st->ptr, std::min<int64_t>(need, NTG_NOALLOC_SCRATCH_BYTES));
-    }
+    rc = run_gemm(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0, s, st->ptr, need);
     if (ordered) {
         HIP_TRY(hipEventRecord(st->done, s));
         st->last_stream = s;

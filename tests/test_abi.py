@@ -196,6 +196,27 @@ def test_split_k_planner_needs_no_device():
     assert lib.ntg_gemm_workspace_bytes(ctypes.byref(d)) == 8192 * 8192 * 2 + 128 * 8192 * 2
 
 
+def test_k_ranges_of_odd_rows_take_a_bounded_workspace():
+    """A batch of odd rows that fills the chip by itself runs its items' k ranges inside one workgroup and needs no room (256 bytes: the leave to change
+    the order); what goes through memory stays under 64 MiB; the sums of bytes wrap, so a batch of them is not cut at all."""
+    lib = _lib.load()
+
+    def ws(dtype, m, k, n, batches):
+        d = _lib.GemmDesc()
+        d.dtype, d.c_mode, d.m, d.k, d.n, d.batches = dtype, _lib.C_OVERWRITE, m, k, n, batches
+        d.stride_a, d.stride_b, d.stride_c = m * k, k * n, m * n
+        return lib.ntg_gemm_workspace_bytes(ctypes.byref(d))
+
+    one = ws(_lib.FLOAT32, 200, 1001, 201, 1)
+    assert one > 0 and one % (200 * 204 * 4) == 0
+    assert ws(_lib.FLOAT32, 200, 1001, 201, 2) == 2 * one
+    assert ws(_lib.FLOAT32, 200, 1001, 201, 40) == 256
+    assert ws(_lib.FLOAT16, 70, 2049, 66, 200) == 256 and ws(_lib.BFLOAT16, 70, 2049, 66, 70000) == 256
+    for batches in range(1, 80):
+        assert 256 <= ws(_lib.FLOAT32, 128, 6463, 721, batches) <= _lib.NOALLOC_SCRATCH_BYTES
+    assert ws(_lib.INT8, 256, 1793, 39, 1) > 0 and ws(_lib.INT8, 256, 1793, 39, 14) == 0
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "_lib", None)
     monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "libntgemm.so"))

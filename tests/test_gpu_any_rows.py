@@ -91,6 +91,59 @@ def test_batches_pitches_and_what_is_added_to(name):
         check(got[..., :n], a[..., :k], b[..., :n], before[..., :n], name, k)
 
 
+def product(lib, a, b, c, m, k, n, batch, strides, ta, tb, mode, bias=None, relu=False, entry="dev", first=0):
+    """Items first .. first + batch - 1 of one call; the bytes of workspace that it was offered."""
+    es = c.element_size()
+    d = _lib.GemmDesc()
+    d.dtype, d.transpose_a, d.transpose_b, d.c_mode = F.ntg_dtype(c), int(ta), int(tb), mode
+    d.m, d.k, d.n, d.batches = m, k, n, batch
+    d.stride_a, d.stride_b, d.stride_c = strides
+    if bias is not None:
+        d.bias, d.bias_batch_stride, d.bias_col_stride = bias.data_ptr() + first * n * es, n, 1
+    need = lib.ntg_gemm_workspace_bytes(ctypes.byref(d))
+    ws = torch.empty(max(need, 1), dtype=torch.uint8, device=DEV)
+    if entry == "dev":
+        d.workspace, d.workspace_bytes = ws.data_ptr(), need
+    call = lib.ntg_gemm_noalloc_dev if entry == "noalloc" else lib.ntg_gemm_relu_dev if relu else lib.ntg_gemm_dev
+    _lib.check(call(ctypes.byref(d), a.data_ptr() + first * strides[0] * es, b.data_ptr() + first * strides[1] * es, c.data_ptr() + first * strides[2] * es,
+                    ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    torch.cuda.synchronize()
+    return need
+
+
+# batches that fill the chip by themselves; ranges of whole and of broken length, a last K-step that is cut
+FULL = [(70, 2049, 66, 200), (129, 2057, 130, 64), (200, 2501, 77, 70), (40, 3001, 201, 200), (128, 2002, 250, 130)]
+
+
+@pytest.mark.parametrize("name", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("ta,tb", TRANS)
+def test_a_batch_that_fills_the_chip_takes_no_room_and_gives_the_bits_of_its_items(name, ta, tb):
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(12)
+    for (m, k, n, batch), mode, relu, shared in zip(FULL, (_lib.C_ACCUMULATE, _lib.C_BIAS, _lib.C_OVERWRITE, _lib.C_BIAS, _lib.C_ACCUMULATE),
+                                                    (False, True, False, False, True), (False, False, True, True, False)):
+        a, b = values((batch, m, k), name, gen), values((1 if shared else batch, k, n), name, gen)
+        c0, bias = values((batch, m, n), name, gen), values((batch, n), name, gen)
+        da, db = (a.transpose(1, 2) if ta else a).contiguous().to(DEV), (b.transpose(1, 2) if tb else b).contiguous().to(DEV)
+        dbias = bias.to(DEV) if mode == _lib.C_BIAS else None
+        strides = (m * k, 0 if shared else k * n, m * n)
+        together, alone = c0.to(DEV), c0.to(DEV)
+        room = product(lib, da, db, together, m, k, n, batch, strides, ta, tb, mode, dbias, relu)
+        some = [0, 1, batch // 2, batch - 1]
+        for i in some:
+            one = product(lib, da, db, alone, m, k, n, 1, strides, ta, tb, mode, dbias, relu, first=i)
+            assert one >= 2 * m * n * 4 and room == 256                  # the item alone is cut into ranges that go through memory
+            assert torch.equal(together[i].view(torch.uint8), alone[i].view(torch.uint8)), (m, k, n, i)
+        start = c0 if mode == _lib.C_ACCUMULATE else bias[:, None, :].expand(batch, m, n) if mode == _lib.C_BIAS else torch.zeros_like(c0)
+        if relu:
+            assert (together >= 0).all() and (together > 0).any()
+        else:
+            check(together.cpu()[some], a[some], b.expand(batch, k, n)[some], start[some], name, k)
+            unallocated = c0.to(DEV)
+            product(lib, da, db, unallocated, m, k, n, batch, strides, ta, tb, mode, dbias, entry="noalloc")
+            assert torch.equal(unallocated.view(torch.uint8), together.view(torch.uint8))
+
+
 @pytest.mark.parametrize("name", ["f16", "bf16", "f32"])
 @pytest.mark.parametrize("relu", [False, True])
 def test_bias_and_relu(name, relu):
