@@ -245,8 +245,11 @@ int ntg_gemm_relu_dev(const ntg_gemm_desc* desc, const void* dA, const void* dB,
  * stream.  Calls on different streams or from different threads are ordered by the library: a call is enqueued as a whole
  * (a mutex per GPU) and makes its stream wait for an event recorded behind the previous user's last kernel.  A stream under
  * capture takes no part in that ordering (an event recorded inside a capture cannot be waited for from outside): graphs
- * that contain such calls must not run while other users of the array are in flight.  The first call on a device looks the
- * array's address up (hipGetSymbolAddress) and creates the event: make that call before a stream capture begins. */
+ * that contain calls which use the array must not run while other users of it are in flight.  Under capture only the split along k of
+ * 16-byte rows and the padded copies use it: rows that miss the 16-byte rule run their k ranges inside one workgroup and integers are not cut, the same
+ * bits (few tiles with a deep k are slower that way: BFloat16 448 x 3704 x 166 20 us against 10; ntg_gemm_dev with a workspace of the graph's own
+ * is not).  The first call that uses the array on a device looks its
+ * address up (hipGetSymbolAddress) and creates the event: make that call before a stream capture begins. */
 #define NTG_NOALLOC_SCRATCH_BYTES (64ll << 20)
 int ntg_gemm_noalloc_dev(const ntg_gemm_desc* desc, const void* dA, const void* dB, void* dC, void* stream);
 

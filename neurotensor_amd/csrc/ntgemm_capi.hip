@@ -749,19 +749,25 @@ int ntg_gemm_noalloc_dev(const ntg_gemm_desc* d, const void* dA, const void* dB,
                     (long long)need, (long long)NTG_NOALLOC_SCRATCH_BYTES);
     p.A = dA; p.B = dB; p.C = dC;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (need == 0) return run_gemm(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0, s);      // the plain kernels: the array is not used
-    ntg::NoallocState* st = nullptr;
-    rc = ntg::noalloc_state_of_current_device(&st);
-    if (rc) return rc;
-    std::lock_guard<std::mutex> lock(st->mutex);
+    const bool ta = d->transpose_a != 0, tb = d->transpose_b != 0;
+    if (need == 0) return run_gemm(p, d->dtype, ta, tb, s);      // the plain kernels: the array is not used
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &capture) != hipSuccess) {      // (e.g. the default stream while another stream captures)
         (void)hipGetLastError();
         capture = hipStreamCaptureStatusActive;
     }
     const bool ordered = capture == hipStreamCaptureStatusNone;
+    // k ranges of rows that start anywhere, and of integers, have forms of the same bits that keep nothing in memory.  They are taken under capture, where
+    // nothing orders the users of the array (an odd row must not decide whether a graph may run beside them), and where they are the faster ones anyway.
+    const AnySplitPlan ap = plan_any_split(p, d->dtype, ta, tb);
+    if (ap.splits > 1 && !is_int_dtype(d->dtype) && (ap.inside || !ordered)) return run_ranges_inside(p, ap, d->dtype, ta, tb, s);
+    if (!ordered && (int_planes_of(d->dtype) || ap.splits > 1)) return run_gemm(p, d->dtype, ta, tb, s);
+    ntg::NoallocState* st = nullptr;
+    rc = ntg::noalloc_state_of_current_device(&st);
+    if (rc) return rc;
+    std::lock_guard<std::mutex> lock(st->mutex);
     if (ordered && st->used && st->last_stream != s) HIP_TRY(hipStreamWaitEvent(s, st->done, 0));     // the previous user of the array finishes first
-    rc = run_gemm(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0, s, st->ptr, need);
+    rc = run_gemm(p, d->dtype, ta, tb, s, st->ptr, need);
     if (ordered) {
         HIP_TRY(hipEventRecord(st->done, s));
         st->last_stream = s;

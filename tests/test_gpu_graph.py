@@ -1,6 +1,8 @@
 """The device entry points under HIP graph capture: they allocate nothing, never synchronise and take their stream as an
 argument, so a chain of them can be captured once and replayed.  Every replay is checked against the eager result of the
 same inputs, with eager work and synchronisation between the replays."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -57,3 +59,38 @@ def test_capture_and_replay():
         torch.cuda.synchronize()
         for i, (g, w) in enumerate(zip(got, want)):
             assert torch.equal(g, w), (rep, i, (g.float() - w.float()).abs().max().item())
+
+
+def _kernel_nodes(graph):
+    """How many nodes a captured graph has, from the runtime that torch loaded."""
+    path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64.so" in line)
+    hip, count = ctypes.CDLL(path), ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(count)) == 0
+    return count.value
+
+
+@pytest.mark.parametrize("dtype,batch,m,k,n", [(torch.bfloat16, 1, 448, 3701, 166), (torch.float16, 3, 70, 2049, 66), (torch.float32, 1, 128, 2463, 721),
+                                               (torch.int8, 1, 256, 1793, 39), (torch.int32, 1, 200, 3000, 200)])
+def test_captured_noalloc_calls_on_odd_rows_leave_the_shared_array_alone(dtype, batch, m, k, n):
+    """A graph of such calls may run beside other users of the array: one kernel, no second pass over sums in memory, and the bits of a workspace."""
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(k)
+    draw = (lambda *s: torch.randint(-100, 100, s, generator=gen).to(dtype)) if dtype in (torch.int8, torch.int32) else (lambda *s: torch.randn(*s, generator=gen).to(dtype))
+    a, b, c = draw(batch, m, k).to(DEV), draw(batch, k, n).to(DEV), torch.zeros(batch, m, n, dtype=dtype, device=DEV)
+    d = _lib.GemmDesc()
+    d.dtype, d.m, d.k, d.n, d.batches = F.ntg_dtype(a), m, k, n, batch
+    d.stride_a, d.stride_b, d.stride_c = m * k, k * n, m * n
+    assert lib.ntg_gemm_workspace_bytes(ctypes.byref(d)) > 0
+    call = lambda: _lib.check(lib.ntg_gemm_noalloc_dev(ctypes.byref(d), a.data_ptr(), b.data_ptr(), c.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        call()
+    assert _kernel_nodes(graph) == 1
+    for _ in range(3):
+        a.copy_(draw(batch, m, k))
+        c.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c, F.matmult(a, b))
