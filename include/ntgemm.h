@@ -207,7 +207,7 @@ typedef struct ntg_gemm_desc {
  * the partial sums of every item; a batch of rows that miss the 16-byte rule and that fills the GPU by itself runs its items' ranges without
  * going through memory: 256 bytes are asked for, which give the leave to change the order of summation and are not written); zero-padded copies of large 8-bit, 16-bit, Float32 and Float64 operands whose rows, pitches
  * or base pointers are not 16-byte multiples, so that they run on the DMA-fed kernels (same results: zeros add nothing);
- * or, for large Int16 / Int32 / Int64 products and their unsigned forms, room for k ranges (these run as 3 / 10 / 36 products of balanced
+ * or, for Int16 / Int32 / Int64 products and their unsigned forms with few tiles and a deep k, room for k ranges (these products run as 3 / 10 / 36 products of balanced
  * digits on v_mfma_i32_32x32x32_i8 with or without it; the sum modulo 2^W is the reference's wrapping result,
  * nt/mp/simde_traits/simde_traits_avx2.h:810-812, :444-446, :523-540: multiply and add in the element type).  It is the largest any form takes: a
  * product may use less.  Without a workspace the same result is computed by the plain kernels.  The reference has no counterpart: its k loop is always serial (nt_matmult.hpp:196). */

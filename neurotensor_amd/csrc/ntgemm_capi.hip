@@ -433,20 +433,6 @@ SplitPlan plan_splitk(const ntg::GemmParams& p, int dtype, bool ta) {
 // no room; 256 bytes stand for the caller's leave to change the order of summation, which a workspace is.
 struct AnySplitPlan { int splits; int64_t kc, ldp, bytes; bool inside; };
 constexpr int64_t INSIDE_BYTES = 256;
-// Room that ntg_gemm_workspace_bytes offers large integer products (and ntg_gemm_noalloc_dev takes them with or refuses them for): the digits of both
-// operands and the 32-bit sums of every shift.  The product itself needs none; its k ranges take what they use of it.
-static int64_t int_workspace_bytes(const ntg::GemmParams& p, int dtype) {
-    const int P = int_planes_of(dtype);
-    if (P == 0 || p.Aptr || p.Bptr || p.Cptr || p.M < 128 || p.N < 128 || p.K < 64) return 0;
-    const int64_t Kp = (p.K + 15) / 16 * 16, Np = (p.N + 15) / 16 * 16;
-    const double macs = (double)p.M * p.N * p.K * p.batch;
-    const double rounds = (double)(((int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch + 255) / 256);
-    const double valu_us = (double)p.K * (P == 8 ? 0.13 : P == 4 ? 0.07 : 0.055) * (rounds + 1.0);
-    const double planes_us = (P == 8 ? 55.0 : P == 4 ? 30.0 : 17.0) + macs * (P * (P + 1) / 2) / 1.0e9 + 8.0 * P * p.batch * (double)p.M * Np / 4.0e6;
-    if (planes_us > 0.8 * valu_us || P * Kp >= (1 << 17) || Np >= (1 << 23)) return 0;
-    return (int64_t)align_up((size_t)((p.sA == 0 ? 1 : p.batch) * (int64_t)p.M * P * Kp), 256) +
-           (int64_t)align_up((size_t)((p.sB == 0 ? 1 : p.batch) * (int64_t)P * Kp * Np), 256) + (int64_t)P * p.batch * p.M * Np * 4;
-}
 // A workgroup alone on its CU spends 0.35 / 0.48 / 1.4 us (16 / 32 / 64 bits) on each K-step of 32, several 0.17 / 0.35 / 1.3 us each (Int32 200 x 3000 x 200
 // whole 48 us, 8 / 16 ranges 12.4 / 10.8; Int16 709 x 3136 x 450, ranges 1 / 4 / 8 / 16: 36 / 16.9 / 15.8 / 19.4; Int64 576 x 3968 x 281, 1 / 4 / 8: 183 / 53 / 58).
 // The sums wrap, so their order is nobody's concern: the batch counts among the tiles.  room: bytes of workspace there are.
@@ -723,7 +709,10 @@ int64_t ntg_gemm_workspace_bytes(const ntg_gemm_desc* d) {
     ntg::GemmParams p;
     if (desc_to_params(d, p)) return -1;
     if (p.M == 0 || p.N == 0 || p.batch == 0) return 0;
-    if (int_planes_of(d->dtype)) return int_workspace_bytes(p, d->dtype);
+    if (int_planes_of(d->dtype)) {
+        if (p.M < 128 || p.N < 128 || p.K < 64) return 0;
+        return plan_int_split(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0, NTG_NOALLOC_SCRATCH_BYTES).bytes;
+    }
     {
         const AnySplitPlan ap = plan_any_split(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0);
         if (ap.splits > 1) return ap.bytes;                        // (no padded copies beside k ranges)

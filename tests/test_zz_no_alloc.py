@@ -1,4 +1,4 @@
-"""ntg_gemm_noalloc_dev (the entry point that allocates nothing: its split-K partial sums, integer byte planes and padded
+"""ntg_gemm_noalloc_dev (the entry point that allocates nothing: its split-K partial sums, k ranges of integers and padded
 copies live in a fixed array inside the library's device code) against ntg_gemm_dev with a caller-owned workspace, through the C ABI.
 
 Both run the same kernels in the same order, so every result must be bit-identical -- for the floating dtypes too.
@@ -85,9 +85,9 @@ def test_noalloc_entry_point_matches_the_workspace_entry_point():
         (np.float16, 520, 4096, 1032, True, False, BIAS), (np.float16, 128, 2048, 512, False, False, OV),
         (np.float32, 256, 4096, 2048, False, True, ACC), (np.float32, 64, 4096, 256, True, True, OV),
         (np.float64, 256, 4096, 1024, False, False, OV), (np.float64, 64, 2048, 256, False, True, BIAS),
-        (np.int16, 640, 520, 712, False, False, ACC), (np.int16, 256, 200, 264, True, False, OV),
-        (np.int32, 512, 512, 512, False, True, OV), ("u32", 320, 392, 328, False, False, BIAS),
-        (np.int64, 768, 520, 776, True, True, ACC), ("u64", 512, 512, 520, False, False, OV),
+        (np.int16, 300, 3000, 264, False, False, ACC), (np.int16, 136, 2000, 200, True, False, OV),
+        (np.int32, 300, 3000, 264, False, True, OV), ("u32", 136, 2000, 200, False, False, BIAS),
+        (np.int64, 640, 520, 712, True, True, ACC), ("u64", 256, 200, 264, False, False, OV),
     ]
     sizes = []
     for (dtype, m, k, n, ta, tb, mode) in calls:
@@ -95,8 +95,8 @@ def test_noalloc_entry_point_matches_the_workspace_entry_point():
     assert all(b < a for a, b in zip(sizes[0::2], sizes[1::2])), sizes      # the second call of each pair is the smaller one
     # the first product once more after all the others: same bits as a fresh caller-owned workspace gives
     _both(lib, rng, "bf16", 256, 4096, 2048, False, False, OV)
-    # a batch of integer products (planes of every item in the array)
-    _both(lib, rng, np.int16, 256, 256, 256, False, False, ACC, batches=3)
+    # a batch of integer products (the ranges of every item in the array)
+    _both(lib, rng, np.int16, 200, 1000, 260, False, False, ACC, batches=3)
     # padded copies (rows that are not 16-byte multiples: A, B and C copied into the array, the bias written as the padded
     # C's starting value, the result copied back), a larger product before a smaller one, then the 8-bit form
     big = _both(lib, rng, "bf16", 2048, 1001, 2044, False, False, BIAS)
@@ -110,14 +110,20 @@ def test_noalloc_entry_point_matches_the_workspace_entry_point():
     # products that have no workspace form run on the plain kernels
     _both(lib, rng, np.float32, 512, 512, 512, False, False, ACC, expect_workspace=False)
     _both(lib, rng, "bf16", 100, 72, 48, False, True, OV, expect_workspace=False)
+    # integers split their digits between their loads and LDS: no room for these
+    _both(lib, rng, np.int16, 640, 520, 712, False, False, ACC, expect_workspace=False)
+    _both(lib, rng, np.int16, 256, 256, 256, False, False, ACC, batches=3, expect_workspace=False)
+    _both(lib, rng, np.int32, 512, 512, 512, False, True, OV, expect_workspace=False)
+    _both(lib, rng, np.int32, 1024, 1024, 1024, False, False, ACC, batches=8, expect_workspace=False)
+    _both(lib, rng, np.int64, 768, 520, 776, True, True, ACC, expect_workspace=False)
 
 
 def test_noalloc_entry_point_rejects_what_does_not_fit():
     lib = _lib.load()
-    # Int32 batch 8 x 1024^3 as byte planes needs 192 MiB
-    a = torch.zeros((8, 1024, 1024), dtype=torch.int32, device=DEV)
-    c = torch.zeros((8, 1024, 1024), dtype=torch.int32, device=DEV)
-    d = _desc(a, 1024, 1024, 1024, False, False, _lib.C_ACCUMULATE, 8)
+    # padded copies of A, B and C of two BFloat16 products of 4095^3 need 191 MiB
+    a = torch.ones((2, 4095, 4095), dtype=torch.bfloat16, device=DEV)
+    c = torch.zeros((2, 4095, 4095), dtype=torch.bfloat16, device=DEV)
+    d = _desc(a, 4095, 4095, 4095, False, False, _lib.C_ACCUMULATE, 2)
     need = lib.ntg_gemm_workspace_bytes(ctypes.byref(d))
     assert need > _lib.NOALLOC_SCRATCH_BYTES
     st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
