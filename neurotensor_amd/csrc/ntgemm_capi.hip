@@ -445,6 +445,9 @@ AnySplitPlan plan_int_split(const ntg::GemmParams& p, int dtype, bool ta, bool t
     const int64_t per_range = (int64_t)p.batch * p.M * pl.ldp * P;
     const double alone = P == 2 ? 0.35 : P == 4 ? 0.48 : 1.4, shared = P == 2 ? 0.17 : P == 4 ? 0.35 : 1.3;
     double best_us = 0.95 * (double)steps * alone;
+    // (The second launch and its workspace take a host about 5 us, 8.3 -> 13.5 us a call through the Python face: what the GPU does meanwhile stays whole.
+    //  64 x k x 64 through that face, whole / ranges: Int32 k = 384 9.0 / 13.9 us, 1000 17.7 / 13.6, 4096 59 / 13.6; Int16 k = 1000 10.3 / 13.5, 2048 17.0 / 13.7.)
+    if (best_us < 13.0) return pl;
     for (int64_t sp = 2; sp <= 32 && sp <= steps / 2 && sp * per_range <= room; ++sp) {
         const int64_t per = (steps + sp - 1) / sp, ranges = (steps + per - 1) / per, wgs = tiles * ranges;
         const double us = (double)per * (wgs <= 256 ? alone : shared * (double)((wgs + 255) / 256)) + 4.0 + 2.0 * (double)ranges * (double)per_range / 4.0e6;
@@ -709,10 +712,7 @@ int64_t ntg_gemm_workspace_bytes(const ntg_gemm_desc* d) {
     ntg::GemmParams p;
     if (desc_to_params(d, p)) return -1;
     if (p.M == 0 || p.N == 0 || p.batch == 0) return 0;
-    if (int_planes_of(d->dtype)) {
-        if (p.M < 128 || p.N < 128 || p.K < 64) return 0;
-        return plan_int_split(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0, NTG_NOALLOC_SCRATCH_BYTES).bytes;
-    }
+    if (int_planes_of(d->dtype)) return plan_int_split(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0, NTG_NOALLOC_SCRATCH_BYTES).bytes;
     {
         const AnySplitPlan ap = plan_any_split(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0);
         if (ap.splits > 1) return ap.bytes;                        // (no padded copies beside k ranges)

@@ -199,3 +199,31 @@ def test_wide_integers_from_digits(name, ta, tb):
         out = torch.from_numpy(c0.copy()).to(DEV)
         F.matmult(torch.from_numpy(a).to(DEV), torch.from_numpy(b).to(DEV), out, ta, tb)
         assert np.array_equal(out.cpu().numpy(), (want + c0.astype(np.int64).view(np.uint64)).astype(npdt)), (m, k, n)
+
+
+@pytest.mark.parametrize("name", sorted(INTS))
+@pytest.mark.parametrize("ta,tb", TRANS)
+def test_wide_integers_with_a_side_under_a_tile_are_cut_into_k_ranges(name, ta, tb):
+    """Few tiles and a deep k, down to the smallest sides; the last range is shorter than a group of eight."""
+    lib = _lib.load()
+    rng = np.random.default_rng(10)
+    npdt, dt = INTS[name]
+    full = lambda *shape: rng.integers(-2**63, 2**63 - 1, shape, dtype=np.int64, endpoint=True).astype(npdt)
+    for m, n, batch in ((64, 64, 1), (8, 8, 1), (9, 300, 1), (40, 70, 3)):
+        d = _lib.GemmDesc()
+        d.dtype, d.transpose_a, d.transpose_b, d.m, d.n, d.batches = F.ntg_dtype(torch.empty(0, dtype=dt)), int(ta), int(tb), m, n, batch
+        for k in range(1300, 1500):
+            d.k, d.stride_a, d.stride_b, d.stride_c = k, m * k, k * n, m * n
+            ranges = lib.ntg_gemm_workspace_bytes(ctypes.byref(d)) // (batch * m * ((n + 3) // 4 * 4) * np.dtype(npdt).itemsize)
+            assert ranges >= 2
+            steps = (k + 31) // 32
+            if 0 < k - (ranges - 1) * -(-steps // ranges) * 32 < 8:
+                break
+        else:
+            assert False, "no k with a short last range"
+        a, b, c0 = full(batch, *((k, m) if ta else (m, k))), full(batch, *((n, k) if tb else (k, n))), full(batch, m, n)
+        A = (np.swapaxes(a, -1, -2) if ta else a).astype(np.int64).view(np.uint64)
+        B = (np.swapaxes(b, -1, -2) if tb else b).astype(np.int64).view(np.uint64)
+        out = torch.from_numpy(c0.copy()).to(DEV)
+        F.matmult(torch.from_numpy(a).to(DEV), torch.from_numpy(b).to(DEV), out, ta, tb)
+        assert np.array_equal(out.cpu().numpy(), (A @ B + c0.astype(np.int64).view(np.uint64)).astype(npdt)), (m, k, n)

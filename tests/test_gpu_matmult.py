@@ -239,7 +239,7 @@ def test_wide_integers_on_the_8bit_matrix_pipe_bit_exact(code, npdt):
     lib = _lib.load()
     st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     rng = np.random.default_rng(4200)
-    sizes = ((4, 520, 2057, 522), (2, 136, 1033, 138))
+    sizes = ((4, 520, 2057, 522), (2, 136, 1321, 138))
     full = lambda shape: rng.integers(0, 2**64, shape, dtype=np.uint64).astype(npdt)      # (keeps the low bits)
     cases = list(zip(TRANS, (_lib.C_OVERWRITE, _lib.C_ACCUMULATE, _lib.C_BIAS, _lib.C_ACCUMULATE), (False, True, False, False)))
     for (batch, m, k, n), ((ta, tb), mode, bcast_b) in itertools.product(sizes, cases):

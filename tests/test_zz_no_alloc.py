@@ -87,7 +87,7 @@ def test_noalloc_entry_point_matches_the_workspace_entry_point():
         (np.float64, 256, 4096, 1024, False, False, OV), (np.float64, 64, 2048, 256, False, True, BIAS),
         (np.int16, 300, 3000, 264, False, False, ACC), (np.int16, 136, 2000, 200, True, False, OV),
         (np.int32, 300, 3000, 264, False, True, OV), ("u32", 136, 2000, 200, False, False, BIAS),
-        (np.int64, 640, 520, 712, True, True, ACC), ("u64", 256, 200, 264, False, False, OV),
+        (np.int64, 640, 520, 712, True, True, ACC), ("u64", 256, 392, 264, False, False, OV),
     ]
     sizes = []
     for (dtype, m, k, n, ta, tb, mode) in calls:
@@ -96,7 +96,7 @@ def test_noalloc_entry_point_matches_the_workspace_entry_point():
     # the first product once more after all the others: same bits as a fresh caller-owned workspace gives
     _both(lib, rng, "bf16", 256, 4096, 2048, False, False, OV)
     # a batch of integer products (the ranges of every item in the array)
-    _both(lib, rng, np.int16, 200, 1000, 260, False, False, ACC, batches=3)
+    _both(lib, rng, np.int16, 200, 1400, 260, False, False, ACC, batches=3)
     # padded copies (rows that are not 16-byte multiples: A, B and C copied into the array, the bias written as the padded
     # C's starting value, the result copied back), a larger product before a smaller one, then the 8-bit form
     big = _both(lib, rng, "bf16", 2048, 1001, 2044, False, False, BIAS)
