@@ -177,9 +177,13 @@ static int int_planes_of(int dtype) {
     }
 }
 // Every contiguous extent holds the eight elements of a group, 32-bit lane offsets, 32-bit sums of a shift's products (P K 2^14 < 2^31).
-// What misses this runs on the vector ALU, bit for bit the same.
+// What misses this runs on the vector ALU, bit for bit the same; so does Int64 of up to 16 k, one pass of that kernel and half a K-step here, on more than
+// 256 tiles (one wavefront a SIMD here): 4096 x 16 x 4096 64 us against 76, 2048 x 16 x 2048 20.3 / 21.8, 1500 x 8 x 1500 14.9 / 17.9, 1024 x (16 x 16 x 16)
+// 13.5 / 16.8, but 1024 x 16 x 1024 10.2 / 7.4; from 17 k on the digits win on any number of tiles (4096 x 20 x 4096 87 / 76, 2048 x 20 x 2048 27 / 22).  Int16 and
+// Int32 win everywhere (4096 x 8 x 4096 25 / 20 and 34 / 22.5, 4096 x (8 x 8 x 8) 19 / 12 and 23 / 20).
 static bool int_pipe_eligible(const ntg::GemmParams& p, int dtype, bool ta, bool tb) {
     const int64_t P = int_planes_of(dtype);
+    if (P == 8 && p.K <= 16 && (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch > 256) return false;
     return P != 0 && p.K > 0 && (ta ? p.M : p.K) >= 8 && (tb ? p.K : p.N) >= 8 && P * (int64_t)p.K < (1 << 17) && p.lda * P < (1 << 23) && p.ldb * P < (1 << 23);
 }
 

@@ -227,3 +227,12 @@ def test_wide_integers_with_a_side_under_a_tile_are_cut_into_k_ranges(name, ta, 
         out = torch.from_numpy(c0.copy()).to(DEV)
         F.matmult(torch.from_numpy(a).to(DEV), torch.from_numpy(b).to(DEV), out, ta, tb)
         assert np.array_equal(out.cpu().numpy(), (A @ B + c0.astype(np.int64).view(np.uint64)).astype(npdt)), (m, k, n)
+
+
+def test_int64_of_few_k_on_either_side_of_the_line():
+    """16 and 17 k on 256 and more tiles: the vector ALU's kernel and the digits give the wrapping result."""
+    rng = np.random.default_rng(11)
+    for m, k, n, batch in ((1024, 16, 1024, 1), (1025, 16, 1024, 1), (1025, 17, 1024, 1), (70, 8, 40, 200), (16, 17, 16, 300)):
+        a, b = (rng.integers(-2**63, 2**63 - 1, s, dtype=np.int64, endpoint=True) for s in ((batch, m, k), (batch, k, n)))
+        got = F.matmult(torch.from_numpy(a).to(DEV), torch.from_numpy(b).to(DEV)).cpu().numpy()
+        assert np.array_equal(got, (a.view(np.uint64) @ b.view(np.uint64)).view(np.int64)), (m, k, n, batch)
