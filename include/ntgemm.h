@@ -189,7 +189,7 @@ typedef struct ntg_gemm_desc {
  * tables live in device memory, so the host side of the library cannot look; with the vouch (and rows that are 16-byte
  * multiples) a table batch runs on the DMA-fed kernels like its strided twin.  An entry that breaks the promise makes the
  * kernel read from a misaligned address (wrong results, not a fault).  Without the vouch, floating-point and 8-bit
- * batches of some size (from 8 GFLOP; Float32 and Float64 from 32, 8-bit integers from 1) have their entries looked at on the device: one small kernel sets a
+ * batches of some size (from 12 GFLOP; Float32 from 6, Float64 from 32, 8-bit integers from 60) have their entries looked at on the device: one small kernel sets a
  * flag, then the product is launched on both kernel families and the one the flag does not name returns at once -- two
  * extra launches (about 4 us), the same bits; smaller batches run on the kernels that take rows as they lie.  The flags live in a static
  * array of the library's device code: make the first such call on a device outside a stream capture. */

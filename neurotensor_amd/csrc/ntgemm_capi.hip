@@ -791,16 +791,18 @@ static int next_gate_slot(int** out) {
 
 // Pointer tables without the caller's vouch: the entries' alignment is a fact of device memory, so it is found out there.  A
 // one-workgroup kernel ORs the low bits of all entries into a flag; then the product is launched twice, on the DMA-fed
-// kernel (which needs 16-byte entries) and on the register-staged one (which does not), each returning at once unless the
-// flag names it.  The two kernels give the same bits, so nothing depends on which one runs.  Worth two extra launches
-// (about 4 us) only for products that take a few times that; the floating types that have both kernels, more than 32 rows.
+// kernel (which needs 16-byte entries) and on the one that takes rows as they lie (Float64: register-staged), each returning at
+// once unless the flag names it.  The two kernels give the same bits, so nothing depends on which one runs.  Worth two extra
+// launches (about 4 us) only where the DMA-fed kernel gains more; the types that have both kernels, more than 32 rows.
 static bool gated_tables_pay(const ntg::GemmParams& p, int dtype) {
     const bool byte = dtype == ntg::DT_I8 || dtype == ntg::DT_U8;
     if (dtype != ntg::DT_F32 && dtype != ntg::DT_F64 && dtype != ntg::DT_F16 && dtype != ntg::DT_BF16 && !byte) return false;
     if (p.M <= 32 || p.K <= 0 || p.act != ntg::ACT_NONE) return false;
     const double flops = 2.0 * (double)p.M * (double)p.N * (double)p.K * (double)p.batch;
-    // (8-bit: the kernel that needs no alignment is the vector ALU's, 40 x slower: the check pays almost at once)
-    return flops >= (byte ? 1.0e9 : dtype == ntg::DT_F32 || dtype == ntg::DT_F64 ? 3.2e10 : 8.0e9);
+    // Checked / rows as they lie, aligned tables: Int8 8 x 512^3 12.3 us / 7.2, 128 x (256 x 2048 x 256) 36 / 27, 24 x 1024^3 42 / 41, 32 x 1024^3 49 / 53, 4 x 2048^3
+    // 40 / 48; BFloat16 64 x (256 x 1024 x 256) 23.0 / 18.1, 8 x (1024 x 512 x 1024) 17.2 / 17.6, 6 x 1024^3 23.2 / 25.1, 32 x 1024^3 73 / 91; Float32 64 x 256^3 28.1 /
+    // 24.7, 16 x 512^3 42 / 41, 4 x 1024^3 71.5 / 75.2, 16 x 1024^3 244 / 279.  (Float64 still weighs against the register-staged kernel.)
+    return flops >= (byte ? 6.0e10 : dtype == ntg::DT_F32 ? 6.0e9 : dtype == ntg::DT_F64 ? 3.2e10 : 1.2e10);
 }
 static int launch_gemm_tables_gated(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s) {
     int* flag = nullptr;

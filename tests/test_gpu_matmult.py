@@ -1309,11 +1309,11 @@ def test_host_entry_points_fp32_are_the_reference_chain_bit_for_bit(shape):
 @pytest.mark.parametrize("dtype", ["bf16", np.float32, np.int8, np.float64], ids=["bf16", "fp32", "int8", "fp64"])
 def test_pointer_tables_without_a_vouch_find_their_alignment_on_the_device(dtype):
     """ntg_gemm_ptrs_dev without NTG_GEMM_PTRS_ALIGNED16 on products large enough to pay for it: a small kernel looks at the
-    tables' entries, and the product runs on the DMA-fed kernel when all of them are 16-byte multiples, on the register-staged
-    one otherwise (8-bit integers: the vector ALU's; both are launched, one of them returns at once).  Aligned tables, then
+    tables' entries, and the product runs on the DMA-fed kernel when all of them are 16-byte multiples, on the one that takes
+    rows as they lie otherwise (Float64: the register-staged one; both are launched, one of them returns at once).  Aligned tables, then
     tables with one entry moved by one element: in both cases every item has the bits of the item alone."""
     bf = dtype == "bf16"
-    m, k, n, nb = (2048, 1024, 2048, 5) if dtype in (np.float32, np.float64) else (1024, 1024, 1024, 6)
+    m, k, n, nb = (2048, 1024, 2048, 5) if dtype in (np.float32, np.float64) else (1024, 1024, 1024, 30 if dtype == np.int8 else 6)
     rng = np.random.default_rng(60606)
     lib = _lib.load()
     st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
