@@ -201,6 +201,11 @@ typedef struct ntg_gemm_desc {
  * 32 rows that is given no workspace.  The host-pointer entry points set it for Float32 themselves (the transfers hide what
  * the faster forms would gain); ntg_gemm_workspace_bytes honours it. */
 #define NTG_GEMM_KEEP_K_ORDER 2
+/* ntg_gemm_ptrs_dev only: every item is to have the bits that ntg_gemm_dev gives it alone with the workspace it is offered.  With this flag
+ * ntg_gemm_workspace_bytes answers for a list of desc->batches items: 0 = one call of ntg_gemm_ptrs_dev does it; otherwise the bytes of ONE item's workspace,
+ * with which the items go out one by one through ntg_gemm_dev (no launch over tables has their order of summation, or the list is so short that this is the
+ * faster way).  Items whose order the tables do not have are refused by ntg_gemm_ptrs_dev (NTG_ERR_INVALID_ARGUMENT). */
+#define NTG_GEMM_PTRS_ITEM_ORDER 4
 
 /* Bytes of workspace with which ntg_gemm_dev runs its faster form (0: there is none for this product): a split along k
  * for shapes such as [256, 8192] x [8192, 8192] (planned from one item's sizes, so a batch is offered its item's split with

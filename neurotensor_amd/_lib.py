@@ -19,6 +19,7 @@ BFLOAT16, UINT64 = 100, 101
 C_OVERWRITE, C_ACCUMULATE, C_BIAS = 0, 1, 2
 GEMM_PTRS_ALIGNED16 = 1               # NTG_GEMM_PTRS_ALIGNED16
 GEMM_KEEP_K_ORDER = 2                 # NTG_GEMM_KEEP_K_ORDER
+GEMM_PTRS_ITEM_ORDER = 4              # NTG_GEMM_PTRS_ITEM_ORDER
 NOALLOC_SCRATCH_BYTES = 64 << 20      # NTG_NOALLOC_SCRATCH_BYTES
 DIAG_MFMA_OPERAND_BYTES = 128 << 10   # NTG_DIAG_MFMA_OPERAND_BYTES
 DIAG_MFMA_FLOPS_PER_PASS = 8388608    # NTG_DIAG_MFMA_FLOPS_PER_PASS

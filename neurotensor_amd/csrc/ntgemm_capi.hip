@@ -435,19 +435,34 @@ SplitPlan plan_splitk(const ntg::GemmParams& p, int dtype, bool ta) {
 // The integers of more than a byte likewise (gemm_int_impl.h).
 // inside: a workgroup runs all ranges of its tile (the sums of these are added in registers, in the order of the second pass: the same bits).  It needs
 // no room; 256 bytes stand for the caller's leave to change the order of summation, which a workspace is.
-struct AnySplitPlan { int splits; int64_t kc, ldp, bytes; bool inside; };
+struct AnySplitPlan { int splits; int64_t kc, ldp, bytes; bool inside; double us; };      // us: estimated, where splits > 1
 constexpr int64_t INSIDE_BYTES = 256;
+// microseconds of a K-step on a 64 x 64 tile: of a workgroup alone on its CU, of each of several (measured, see the planners)
+struct KStepUs { double alone, shared; };
+static KStepUs k_step_us(int dtype) {
+    switch (int_planes_of(dtype)) {
+    case 2: return {0.35, 0.17};
+    case 4: return {0.48, 0.35};
+    case 8: return {1.4, 1.3};
+    default: return dtype == ntg::DT_F32 ? KStepUs{0.71, 0.45} : ntg::elem_size(dtype) == 2 ? KStepUs{0.28, 0.18} : KStepUs{0.43, 0.25};
+    }
+}
+// ... with all k ranges of a float's tile in one workgroup
+static double inside_us(int64_t es, int64_t tiles, int64_t steps) {
+    const double rounds = (double)tiles / 256.0;
+    return es == 2 ? 5.5 + (double)steps * std::max(0.33, 0.3 * rounds) : 2.5 + (double)steps * std::max(0.71, 0.3 + 0.62 * rounds);
+}
 // A workgroup alone on its CU spends 0.35 / 0.48 / 1.4 us (16 / 32 / 64 bits) on each K-step of 32, several 0.17 / 0.35 / 1.3 us each (Int32 200 x 3000 x 200
 // whole 48 us, 8 / 16 ranges 12.4 / 10.8; Int16 709 x 3136 x 450, ranges 1 / 4 / 8 / 16: 36 / 16.9 / 15.8 / 19.4; Int64 576 x 3968 x 281, 1 / 4 / 8: 183 / 53 / 58).
 // The sums wrap, so their order is nobody's concern: the batch counts among the tiles.  room: bytes of workspace there are.
 AnySplitPlan plan_int_split(const ntg::GemmParams& p, int dtype, bool ta, bool tb, int64_t room) {
-    AnySplitPlan pl{1, p.K, (p.N + 3) / 4 * 4, 0, false};
+    AnySplitPlan pl{1, p.K, (p.N + 3) / 4 * 4, 0, false, 0.0};
     if (p.batch < 1 || p.batch > 65535 || p.Aptr || p.Bptr || p.Cptr || !int_pipe_eligible(p, dtype, ta, tb)) return pl;
     const int P = int_planes_of(dtype);
     const int64_t steps = (p.K + 31) / 32, tiles = ((p.M + 63) / 64) * ((p.N + 63) / 64) * (int64_t)p.batch;
     if (tiles > 255) return pl;
     const int64_t per_range = (int64_t)p.batch * p.M * pl.ldp * P;
-    const double alone = P == 2 ? 0.35 : P == 4 ? 0.48 : 1.4, shared = P == 2 ? 0.17 : P == 4 ? 0.35 : 1.3;
+    const auto [alone, shared] = k_step_us(dtype);
     double best_us = 0.95 * (double)steps * alone;
     // (The second launch and its workspace take a host about 5 us, 8.3 -> 13.5 us a call through the Python face: what the GPU does meanwhile stays whole.
     //  64 x k x 64 through that face, whole / ranges: Int32 k = 384 9.0 / 13.9 us, 1000 17.7 / 13.6, 4096 59 / 13.6; Int16 k = 1000 10.3 / 13.5, 2048 17.0 / 13.7.)
@@ -455,12 +470,12 @@ AnySplitPlan plan_int_split(const ntg::GemmParams& p, int dtype, bool ta, bool t
     for (int64_t sp = 2; sp <= 32 && sp <= steps / 2 && sp * per_range <= room; ++sp) {
         const int64_t per = (steps + sp - 1) / sp, ranges = (steps + per - 1) / per, wgs = tiles * ranges;
         const double us = (double)per * (wgs <= 256 ? alone : shared * (double)((wgs + 255) / 256)) + 4.0 + 2.0 * (double)ranges * (double)per_range / 4.0e6;
-        if (us < best_us) { best_us = us; pl.splits = (int)ranges; pl.kc = per * 32; pl.bytes = ranges * per_range; }
+        if (us < best_us) { best_us = us; pl.splits = (int)ranges; pl.kc = per * 32; pl.bytes = ranges * per_range; pl.us = us; }
     }
     return pl;
 }
 AnySplitPlan plan_any_split(const ntg::GemmParams& p, int dtype, bool ta, bool tb) {
-    AnySplitPlan none{1, p.K, 0, 0, false};
+    AnySplitPlan none{1, p.K, 0, 0, false, 0.0};
     const bool byte = dtype == ntg::DT_I8 || dtype == ntg::DT_U8;
     if (p.batch < 1 || (byte && p.batch > 65535) || p.Aptr || p.Bptr || p.Cptr || p.keep_k_order || !ntg::any_eligible(p, dtype, ta, tb)) return none;
     if (p.M <= 32 && !byte) return none;                           // the streaming kernels take these
@@ -474,7 +489,7 @@ AnySplitPlan plan_any_split(const ntg::GemmParams& p, int dtype, bool ta, bool t
     // each; a launch costs about 2.5 us, the second pass 4 us + the partial sums written and read at 4 TB/s.  Of 2 .. 32 ranges the choice was the
     // best measured one or within 10 % of it on fourteen shapes (BFloat16 576 x 3797 x 448, ranges 1 / 2 / 4 / 8: 19.6 / 16.5 / 13.0 / 14.5 us;
     // 448 x 3704 x 166: 25.9 us whole, 10.4 in eight ranges; Float32 128 x 6463 x 720: 146 us whole, 24 in 21 ranges).
-    const double alone = byte ? 0.43 : es == 2 ? 0.28 : 0.71, shared = byte ? 0.25 : es == 2 ? 0.18 : 0.45;
+    const auto [alone, shared] = k_step_us(dtype);
     auto estimate_us = [&](int64_t tls, int64_t its, int64_t sp, int64_t per) {
         const int64_t wgs = tls * sp;
         const double second_pass = sp == 1 ? 0.0 : 4.0 + 8.0 * (double)sp * (double)its * (double)p.M * (double)p.N / 4.0e6;
@@ -487,7 +502,7 @@ AnySplitPlan plan_any_split(const ntg::GemmParams& p, int dtype, bool ta, bool t
         const int64_t per = (steps + sp - 1) / sp, ranges = (steps + per - 1) / per;
         const double us = estimate_us(tiles, items, ranges, per);
         if (ranges * items * (int64_t)p.M * ((p.N + 3) / 4 * 4) * 4 > (int64_t)NTG_NOALLOC_SCRATCH_BYTES) break;      // (fits where nothing is allocated)
-        if (us < best_us) { best_us = us; pl.splits = (int)ranges; pl.kc = per * bk; }
+        if (us < best_us) { best_us = us; pl.splits = (int)ranges; pl.kc = per * bk; pl.us = us; }
     }
     if (pl.splits < 2) return none;
     pl.ldp = (p.N + 3) / 4 * 4;
@@ -498,9 +513,7 @@ AnySplitPlan plan_any_split(const ntg::GemmParams& p, int dtype, bool ta, bool t
         // 6 items 30.7 / 37.0 us, 10 items 44.3 / 38.6, 32 items 148 / 113; Float32 200 x 1501 x 201, 6 items 25.9 / 36.7, 16 items 48.7 / 37.3, 64 items 175 /
         // 114; Float16 1000 x (70 x 2049 x 66) 237 / 135, Float32 64 x (128 x 6463 x 720) 892 / 740.  A K-step inside takes at least 0.33 / 0.71 us (16-bit / Float32).
         const int64_t all = tiles * p.batch;
-        const double rounds = (double)all / 256.0;
-        const double inside_us = es == 2 ? 5.5 + (double)steps * std::max(0.33, 0.3 * rounds) : 2.5 + (double)steps * std::max(0.71, 0.3 + 0.62 * rounds);
-        pl.inside = p.batch > 65535 || pl.bytes > (int64_t)NTG_NOALLOC_SCRATCH_BYTES || inside_us <= estimate_us(all, p.batch, pl.splits, pl.kc / bk);
+        pl.inside = p.batch > 65535 || pl.bytes > (int64_t)NTG_NOALLOC_SCRATCH_BYTES || inside_us(es, all, steps) <= estimate_us(all, p.batch, pl.splits, pl.kc / bk);
         if (pl.inside) pl.bytes = INSIDE_BYTES;
     }
     return pl;
@@ -511,6 +524,27 @@ static int run_ranges_inside(ntg::GemmParams p, const AnySplitPlan& ap, int dtyp
     p.fold_steps = (int)(ap.kc * ntg::elem_size(dtype) / 128);
     const hipError_t e = ntg::launch_gemm_any(dtype, ta, tb, p, s);
     return e == hipSuccess ? NTG_OK : hip_fail(e, "gemm launch");
+}
+
+// A list of p.batch products behind pointer tables whose items are to have the bits that they have alone with their workspace (NTG_GEMM_PTRS_ITEM_ORDER).
+// 0: one launch over the tables does that; else the workspace of one item, the list goes out item by item.  Integers have the same bits in any order; k ranges
+// of odd rows run inside a workgroup; a split of 16-byte rows, and padded copies, are for single products only.  Where both ways are open the list's length
+// decides: an item takes its own time and two launches, 9 us at least.  Item by item / one launch: BFloat16 448 x 3704 x 166 A^T.B, 2 items 22 / 21 us, 16 items 178 /
+// 33, 64 items 774 / 80; Int32 200 x 3001 x 200, 2 items 23 / 50, 8 items 94 / 53; Int64 64 x 4096 x 64, 8 items 119 / 134, 16 items 237 / 134.
+static int64_t table_item_bytes(const ntg::GemmParams& p, int dtype, bool ta, bool tb) {
+    ntg::GemmParams one = p;
+    one.batch = 1;
+    const bool wide = int_planes_of(dtype) != 0;
+    const AnySplitPlan ap = wide ? plan_int_split(one, dtype, ta, tb, NTG_NOALLOC_SCRATCH_BYTES) : plan_any_split(one, dtype, ta, tb);
+    if (ap.splits > 1) {
+        const int64_t bk = wide ? 32 : 128 / ntg::elem_size(dtype), steps = (p.K + bk - 1) / bk, tiles = (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
+        const KStepUs c = k_step_us(dtype);
+        const double table_us = is_int_dtype(dtype) ? 2.5 + (double)steps * (tiles <= 256 ? c.alone : c.shared * (double)((tiles + 255) / 256))
+                                                    : inside_us(ntg::elem_size(dtype), tiles, steps);
+        return table_us <= (double)p.batch * std::max(9.0, ap.us + 4.0) ? 0 : ap.bytes;
+    }
+    const PadPlan pp = plan_pad(one, dtype, ta, tb);
+    return pp.ok && pp.pays ? pp.bytes() : plan_splitk(one, dtype, ta).bytes;
 }
 
 int run_gemm(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s, void* workspace = nullptr, int64_t workspace_bytes = 0) {
@@ -716,6 +750,7 @@ int64_t ntg_gemm_workspace_bytes(const ntg_gemm_desc* d) {
     ntg::GemmParams p;
     if (desc_to_params(d, p)) return -1;
     if (p.M == 0 || p.N == 0 || p.batch == 0) return 0;
+    if (d->flags & NTG_GEMM_PTRS_ITEM_ORDER) return table_item_bytes(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0);
     if (int_planes_of(d->dtype)) return plan_int_split(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0, NTG_NOALLOC_SCRATCH_BYTES).bytes;
     {
         const AnySplitPlan ap = plan_any_split(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0);
@@ -830,8 +865,17 @@ static int gemm_ptrs(const ntg_gemm_desc* d, const void* const* dA, const void* 
     if (rc) return rc;
     if (p.M == 0 || p.N == 0 || p.batch == 0) return NTG_OK;
     if (!dA || !dB || !dC) return fail(NTG_ERR_INVALID_ARGUMENT, "null pointer table");
+    AnySplitPlan item{1, p.K, 0, 0, false, 0.0};
+    if ((d->flags & NTG_GEMM_PTRS_ITEM_ORDER) && !is_int_dtype(d->dtype)) {
+        ntg::GemmParams one = p;
+        one.batch = 1;
+        item = plan_any_split(one, d->dtype, d->transpose_a != 0, d->transpose_b != 0);
+        if (item.splits == 1 && plan_splitk(one, d->dtype, d->transpose_a != 0).splits > 1)
+            return fail(NTG_ERR_INVALID_ARGUMENT, "no launch over pointer tables sums these items in the order that each has alone: run them one by one (ntg_gemm_workspace_bytes says so)");
+    }
     p.Aptr = dA; p.Bptr = dB; p.Cptr = dC;
     p.ptrs_aligned = aligned ? 1 : 0;
+    if (item.splits > 1) return run_ranges_inside(p, item, d->dtype, d->transpose_a != 0, d->transpose_b != 0, static_cast<hipStream_t>(stream));
     if (!aligned && gated_tables_pay(p, d->dtype))
         return launch_gemm_tables_gated(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0, static_cast<hipStream_t>(stream));
     return run_gemm(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0, static_cast<hipStream_t>(stream));
@@ -1042,14 +1086,13 @@ int ntg_matmult_batch(int dtype, const void* const* A, const void* const* B, voi
     else d.stride_a = d.stride_b = 0;
     const size_t ws_off = off;
     int64_t ws_bytes = strided ? ntg_gemm_workspace_bytes(&d) : 0;
-    // A pattern of repeated pointers runs as ONE table batch, which has no workspace form.  Where an item on its own would
-    // be given one that changes the order of summation over k (a split), the items go out one by one in that form instead,
-    // so that an item comes out bit for bit the same alone and in any batch (tests/src/matmult_test.cpp:108-189).
+    // A pattern of repeated pointers runs as ONE table batch.  Where an item on its own would be given a workspace form whose order of
+    // summation over k the tables do not have (a split), the items go out one by one in that form instead, so that an item comes out
+    // bit for bit the same alone and in any batch (tests/src/matmult_test.cpp:108-189).
     bool per_item = false;
     if (!strided) {
-        ntg_gemm_desc one = d;
-        one.batches = 1;
-        const int64_t wb = ntg_gemm_workspace_bytes(&one);
+        d.flags |= NTG_GEMM_PTRS_ITEM_ORDER;
+        const int64_t wb = ntg_gemm_workspace_bytes(&d);
         if (wb > 0) { per_item = true; ws_bytes = wb; }
     }
     if (ws_bytes > 0) off += (size_t)ws_bytes;

@@ -540,7 +540,7 @@ static void device_gemm(int dt, int64_t es, bool ta, bool tb, int mode, int64_t 
             d.bias_row_stride = brow > 1 ? bcol : 0;
             d.bias_col_stride = bcol > 1 ? 1 : 0;
         }
-        const int64_t wsb = ntg_gemm_workspace_bytes(&d);      // > 0: a faster form exists (split along k, byte planes)
+        const int64_t wsb = ntg_gemm_workspace_bytes(&d);      // > 0: a faster form exists (split along k, padded copies)
         if (wsb > 0) { d.workspace = device_workspace(wsb); d.workspace_bytes = wsb; }
         const char* a_i = A + (na > 1 ? (i0 % na) * m * k * es : 0);
         const char* b_i = B + (nb > 1 ? (i0 % nb) * k * n * es : 0);
@@ -681,13 +681,15 @@ Tensor matmult(const TensorList& a, const TensorList& b, bool trans_a, bool tran
             check_status(ntg_gemm_dev(&d, tab[0], tab[(size_t)total], const_cast<void*>(tab[(size_t)(2 * total)]), nullptr));
             return c;
         }
-        // (2) Any other list: where one item on its own would be given a workspace form (a split along k changes the order of
-        // summation), the items go out one by one in that form, so that an item comes out bit for bit the same alone and in a
-        // list (tests/src/matmult_test.cpp:108-189) ...
+        // (2) Any other list: where one item on its own would be given a workspace form that a launch over pointer tables does not have
+        // (a split along k changes the order of summation), the items go out one by one in that form, so that an item comes out bit
+        // for bit the same alone and in a list (tests/src/matmult_test.cpp:108-189) ...
+        d.flags |= NTG_GEMM_PTRS_ITEM_ORDER;
         {
             ntg_gemm_desc one = d;
-            one.batches = 1;
             if (with_workspace(one) > 0) {
+                one.batches = 1;
+                one.flags = 0;
                 for (int64_t t = 0; t < total; ++t)
                     check_status(ntg_gemm_dev(&one, tab[(size_t)t], tab[(size_t)(total + t)], const_cast<void*>(tab[(size_t)(2 * total + t)]), nullptr));
                 return c;

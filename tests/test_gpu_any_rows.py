@@ -236,3 +236,54 @@ def test_int64_of_few_k_on_either_side_of_the_line():
         a, b = (rng.integers(-2**63, 2**63 - 1, s, dtype=np.int64, endpoint=True) for s in ((batch, m, k), (batch, k, n)))
         got = F.matmult(torch.from_numpy(a).to(DEV), torch.from_numpy(b).to(DEV)).cpu().numpy()
         assert np.array_equal(got, (a.view(np.uint64) @ b.view(np.uint64)).view(np.int64)), (m, k, n, batch)
+
+
+@pytest.mark.parametrize("name", sorted(DTYPES) + sorted(INTS))
+@pytest.mark.parametrize("ta,tb", TRANS)
+def test_lists_behind_pointer_tables_have_the_bits_of_their_items(name, ta, tb):
+    """Repeated pointers in no order, entries inside a chunk, C added to: one launch for a long list; a list whose items are split
+    along k on 16-byte rows is refused."""
+    lib = _lib.load()
+    rng, gen = np.random.default_rng(13), torch.Generator().manual_seed(13)
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    if name in INTS:
+        draw = lambda *s: torch.from_numpy(rng.integers(-2**63, 2**63 - 1, s, dtype=np.int64, endpoint=True).astype(INTS[name][0]))
+    else:
+        draw = lambda *s: values(s, name, gen)
+    m, k, n, mats = 67, 4051, 97, 3
+    d = _lib.GemmDesc()
+    d.transpose_a, d.transpose_b, d.c_mode, d.m, d.k, d.n = int(ta), int(tb), _lib.C_ACCUMULATE, m, k, n
+    a, b = draw(mats, m * k + 3), draw(mats, k * n + 3)                  # (odd pitches: the matrices start anywhere)
+    da, db = a.to(DEV), b.to(DEV)
+    d.dtype = F.ntg_dtype(da)
+    for items in (60, 2):
+        d.flags, d.batches = _lib.GEMM_PTRS_ITEM_ORDER, items
+        ia, ib = rng.integers(0, mats, items), rng.integers(0, mats, items)
+        c0 = draw(items, m * n + 1)
+        c, alone = c0.to(DEV), c0.to(DEV)
+        need = lib.ntg_gemm_workspace_bytes(ctypes.byref(d))
+        assert need == 0 or items == 2
+        tab = torch.tensor([da[i].data_ptr() for i in ia] + [db[i].data_ptr() for i in ib] + [x.data_ptr() for x in c], dtype=torch.int64, device=DEV)
+        _lib.check(lib.ntg_gemm_ptrs_dev(ctypes.byref(d), tab.data_ptr(), tab.data_ptr() + 8 * items, tab.data_ptr() + 16 * items, st))
+        d.flags, d.batches = 0, 1
+        one = lib.ntg_gemm_workspace_bytes(ctypes.byref(d))
+        assert one > 0 and need in (0, one)
+        ws = torch.empty(one, dtype=torch.uint8, device=DEV)
+        d.workspace, d.workspace_bytes = ws.data_ptr(), one
+        for j in range(items):
+            _lib.check(lib.ntg_gemm_dev(ctypes.byref(d), da[ia[j]].data_ptr(), db[ib[j]].data_ptr(), alone[j].data_ptr(), st))
+        d.workspace, d.workspace_bytes = None, 0
+        torch.cuda.synchronize()
+        assert torch.equal(c.view(torch.uint8), alone.view(torch.uint8))
+        assert torch.equal(c[:, m * n:].cpu(), c0[:, m * n:])
+        j = items - 1
+        left, right = a[ia[j], :m * k].view(k, m).t() if ta else a[ia[j], :m * k].view(m, k), b[ib[j], :k * n].view(n, k).t() if tb else b[ib[j], :k * n].view(k, n)
+        if name in INTS:
+            want = left.numpy().astype(np.int64).view(np.uint64) @ right.numpy().astype(np.int64).view(np.uint64) + c0[j, :m * n].view(m, n).numpy().astype(np.int64).view(np.uint64)
+            assert np.array_equal(c[j, :m * n].cpu().view(m, n).numpy(), want.astype(INTS[name][0]))
+        else:
+            check(c[j, :m * n].cpu().view(m, n), left, right, c0[j, :m * n].view(m, n), name, k)
+    if name in ("f16", "bf16", "f32"):
+        d.flags, d.batches, d.m, d.k, d.n = _lib.GEMM_PTRS_ITEM_ORDER, 2, 64, 8192, 64
+        assert lib.ntg_gemm_workspace_bytes(ctypes.byref(d)) > 0
+        assert lib.ntg_gemm_ptrs_dev(ctypes.byref(d), tab.data_ptr(), tab.data_ptr() + 16, tab.data_ptr() + 32, st) == 1
