@@ -210,12 +210,12 @@ typedef struct ntg_gemm_desc {
 /* Bytes of workspace with which ntg_gemm_dev runs its faster form (0: there is none for this product): a split along k
  * for shapes such as [256, 8192] x [8192, 8192] (planned from one item's sizes, so a batch is offered its item's split with
  * the partial sums of every item; a batch of rows that miss the 16-byte rule and that fills the GPU by itself runs its items' ranges without
- * going through memory: 256 bytes are asked for, which give the leave to change the order of summation and are not written); zero-padded copies of large 8-bit, 16-bit, Float32 and Float64 operands whose rows, pitches
- * or base pointers are not 16-byte multiples, so that they run on the DMA-fed kernels (same results: zeros add nothing);
+ * going through memory: 256 bytes are asked for, which give the leave to change the order of summation and are not written); zero-padded copies of 8-bit, 16-bit, Float32 and Float64 operands whose rows, pitches
+ * or base pointers are not 16-byte multiples, where these repay the copies (from 1.7e10, 1.6e10, 9e9 and 8.6e9 multiply-adds on; smaller products run on
+ * rows as they lie), so that they run on the DMA-fed kernels (same results: zeros add nothing);
  * or, for Int16 / Int32 / Int64 products and their unsigned forms with few tiles and a deep k, room for k ranges (these products run as 3 / 10 / 36 products of balanced
  * digits on v_mfma_i32_32x32x32_i8 with or without it; the sum modulo 2^W is the reference's wrapping result,
- * nt/mp/simde_traits/simde_traits_avx2.h:810-812, :444-446, :523-540: multiply and add in the element type).  It is the largest any form takes: a
- * product may use less.  Without a workspace the same result is computed by the plain kernels.  The reference has no counterpart: its k loop is always serial (nt_matmult.hpp:196). */
+ * nt/mp/simde_traits/simde_traits_avx2.h:810-812, :444-446, :523-540: multiply and add in the element type).  Without a workspace the same result is computed by the plain kernels.  The reference has no counterpart: its k loop is always serial (nt_matmult.hpp:196). */
 int64_t ntg_gemm_workspace_bytes(const ntg_gemm_desc* desc);
 
 /* nt_matmult<T> on device buffers: C += op(A).op(B), dense leading dimensions. */
@@ -240,8 +240,7 @@ int ntg_gemm_relu_dev(const ntg_gemm_desc* desc, const void* dA, const void* dB,
 /* ntg_gemm_dev for callers that cannot allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc): it has NO counterpart in the reference.  Same arguments, results bit-identical to
  * ntg_gemm_dev called with a workspace of ntg_gemm_workspace_bytes(desc) bytes; desc->workspace and desc->workspace_bytes
- * are ignored.  The split along k, the byte-plane products of the wide integers and the padded copies of unaligned 8- and
- * 16-bit operands keep their intermediate data in a fixed array of NTG_NOALLOC_SCRATCH_BYTES bytes that is part of the
+ * are ignored.  The split along k and the padded copies of unaligned operands keep their intermediate data in a fixed array of NTG_NOALLOC_SCRATCH_BYTES bytes that is part of the
  * library's device code (every GPU the library runs on holds its copy until the process ends); the call itself allocates and
  * frees no memory.  A product whose workspace form needs more than that is rejected with NTG_ERR_INVALID_ARGUMENT: use
  * ntg_gemm_dev with your own workspace, or -- it allocates nothing either -- ntg_gemm_dev with workspace = NULL, which runs

@@ -315,8 +315,7 @@ static PadPlan plan_pad(const ntg::GemmParams& p, int dtype, bool ta, bool tb) {
     // as free.  Copies against no copies: Float16 1023 x 1537 x 2049 (3.2e9) 30.4 us against 26.7, 27 x 1704 x 229 x 960 (1.0e10) 64 against 56, 8 x 1201 x
     // 1301 x 903 (1.1e10) 57.2 against 53.7, 2049^3 (8.6e9) 50.4 against 49.7; BFloat16 2813 x 803 x 2240 (5.1e9) 28.0 against 23.3, 8192 x 999 x 999
     // A^T.B (8.2e9) 40.8 against 29.8, 3618 x 739 x 9392 (2.5e10) 73 against 84, 4095^3 145 against 192; Float32 2049^3 211 against 187, 1504 x 727 x
-    // 8952 (9.8e9) 180 against 191; Int8 2049^3 36.7 against 33.3, 1002 x 257 x 2431 14.8 against 9.8.  (The workspace is offered as if they paid:
-    // what a caller keeps stays enough.)
+    // 8952 (9.8e9) 180 against 191; Int8 2049^3 36.7 against 33.3, 1002 x 257 x 2431 14.8 against 9.8.
     pl.pays = !(pl.padA || pl.padB || pl.padC) || !ntg::any_eligible(p, dtype, ta, tb) || macs >= (byte ? 1.7e10 : half ? 1.6e10 : dtype == ntg::DT_F32 ? 9.0e9 : 0.0);
     return pl;
 }
@@ -756,7 +755,7 @@ int64_t ntg_gemm_workspace_bytes(const ntg_gemm_desc* d) {
         const AnySplitPlan ap = plan_any_split(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0);
         if (ap.splits > 1) return ap.bytes;                        // (no padded copies beside k ranges)
         const PadPlan pp = plan_pad(p, d->dtype, d->transpose_a != 0, d->transpose_b != 0);      // pointers taken as 16-byte aligned
-        if (pp.ok) return pp.bytes();
+        if (pp.ok && pp.pays) return pp.bytes();
     }
     return plan_splitk(p, d->dtype, d->transpose_a != 0).bytes;      // pointers taken as 16-byte aligned
 }

@@ -177,24 +177,25 @@ def test_split_k_planner_needs_no_device():
     assert ws(_lib.BFLOAT16, 1536, 4096, 1536) == 0
     # rows that are not 16-byte multiples cannot use the kernel that writes fp32 partial sums; products this large are
     # offered padded copies of the operands that need them instead (B and C for n = 8190, A for a pitch of 8196)
-    assert ws(_lib.BFLOAT16, 128, 8192, 8190) == 8192 * 8192 * 2 + 128 * 8192 * 2 and ws(_lib.BFLOAT16, 128, 8192, 8192, lda=8196) == 128 * 8192 * 2
-    assert ws(_lib.BFLOAT16, 128, 1024, 1022) == 0 and ws(_lib.BFLOAT16, 128, 1024, 1024, lda=1028) == 0      # too small to repay the copies
-    # 8-bit integers: the alternative is the vector ALU, so the padded form starts earlier
-    # (k 1001 -> 1008, n 530 -> 544; the copies of A and B have rows of whole 128-byte lines: 1024 and 640 bytes)
-    assert ws(_lib.INT8, 520, 1001, 530) == 520 * 1024 + 1008 * 640 + 520 * 544 + (256 - 520 * 1024 % 256) % 256 + (256 - 1008 * 640 % 256) % 256 + (256 - 520 * 544 % 256) % 256
+    assert ws(_lib.BFLOAT16, 256, 8192, 8190) == 8192 * 8192 * 2 + 256 * 8192 * 2 and ws(_lib.BFLOAT16, 256, 8192, 8192, lda=8196) == 256 * 8192 * 2
+    for k, n, lda in ((8192, 8190, 0), (8192, 8192, 8196), (1024, 1022, 0), (1024, 1024, 1028)):                # too small to repay the copies
+        assert ws(_lib.BFLOAT16, 128, k, n, lda=lda) == 0
+    # (k 2601 -> 2608, n 2602 -> 2608; the copies of A and B have rows of whole 128-byte lines: 2688 bytes)
+    assert ws(_lib.INT8, 2600, 2601, 2602) == sum(-(-b // 256) * 256 for b in (2600 * 2688, 2608 * 2688, 2600 * 2608))
+    assert ws(_lib.INT8, 520, 1001, 530) == 0
     assert ws(_lib.INT8, 100, 101, 103) == 0 and ws(_lib.INT32, 100, 101, 103) == 0
     # fp32 / fp64, 64 x 64 tiles: 16 tiles and k = 1024 -> eight ranges of 128; 256 or more tiles -> none
     assert ranges(_lib.FLOAT32, 256, 1024, 256, 4) == 8
     assert ranges(_lib.FLOAT64, 256, 1024, 256, 8) == 8
     assert ws(_lib.FLOAT32, 1024, 4096, 1024) == 0 and ws(_lib.FLOAT64, 1024, 4096, 1024) == 0
     assert ws(_lib.FLOAT32, 768, 768, 768) == 0
-    # NTG_GEMM_KEEP_K_ORDER: no split along k is offered (padded copies and byte planes keep the order and stay on offer)
+    # NTG_GEMM_KEEP_K_ORDER: no split along k is offered (padded copies keep the order and stay on offer)
     d = _lib.GemmDesc()
     d.dtype, d.c_mode, d.flags = _lib.FLOAT32, _lib.C_OVERWRITE, _lib.GEMM_KEEP_K_ORDER
     d.m, d.k, d.n, d.batches = 256, 1024, 256, 1
     assert lib.ntg_gemm_workspace_bytes(ctypes.byref(d)) == 0
-    d.dtype, d.m, d.k, d.n = _lib.BFLOAT16, 128, 8192, 8190
-    assert lib.ntg_gemm_workspace_bytes(ctypes.byref(d)) == 8192 * 8192 * 2 + 128 * 8192 * 2
+    d.dtype, d.m, d.k, d.n = _lib.BFLOAT16, 256, 8192, 8190
+    assert lib.ntg_gemm_workspace_bytes(ctypes.byref(d)) == 8192 * 8192 * 2 + 256 * 8192 * 2
 
 
 def test_k_ranges_of_odd_rows_take_a_bounded_workspace():

@@ -101,8 +101,10 @@ def test_relu_epilogue_with_workspace_forms(name):
         for mode in (_lib.C_OVERWRITE, _lib.C_BIAS, _lib.C_ACCUMULATE):
             run_pair(lib, st, dt, m, k, n, False, False, mode, workspace=True)
     if dt in (torch.float16, torch.bfloat16):
-        run_pair(lib, st, dt, 2048, 1001, 2048, False, False, _lib.C_BIAS, workspace=True)
-        run_pair(lib, st, dt, 2048, 1024, 2044, False, True, _lib.C_ACCUMULATE, workspace=True)
+        run_pair(lib, st, dt, 2600, 2501, 2608, False, False, _lib.C_BIAS, workspace=True)
+        run_pair(lib, st, dt, 2600, 2504, 2604, False, True, _lib.C_ACCUMULATE, workspace=True)
+        run_pair(lib, st, dt, 2048, 1001, 2048, False, False, _lib.C_BIAS)                  # too small to repay the copies
+        run_pair(lib, st, dt, 2048, 1024, 2044, False, True, _lib.C_ACCUMULATE)
 
 
 def test_relu_epilogue_argument_errors():

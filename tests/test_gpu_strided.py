@@ -191,18 +191,20 @@ def test_16bit_results_are_rounded_once_on_ragged_k(name):
 
 @pytest.mark.parametrize("name", ["bf16", "f16", "i8", "u8", "f32", "f64"])
 def test_rows_that_are_not_16_byte_multiples_through_padded_copies(name):
-    """Large 8-bit, 16-bit, Float32 and Float64 products whose pitches, sizes or base pointers miss the 16-byte rule are offered
-    a workspace (ntg_gemm_workspace_bytes) with which the operands are copied into zero-padded rows and the DMA-fed kernel runs:
+    """8-bit, 16-bit, Float32 and Float64 products whose pitches, sizes or base pointers miss the 16-byte rule, with the workspace that
+    they are offered: the operands are copied into zero-padded rows and the DMA-fed kernel runs (Float64, and where only the last k-rows
+    are copied; the other types copy whole operands from larger products on, see below, and are read as they lie here):
     every flag pair, the three C modes, batches with a broadcast operand, odd k / n / m and odd base pointers;
     integers bit-exact against the oracle, 16-bit floats held to one rounding, Float32 / Float64 within their bound."""
     rng = np.random.default_rng(8100 + list(DTYPES).index(name))
     half = name in ("bf16", "f16")
     m, k, n = (1304, 1001, 1702) if half else (1700, 1501, 1702) if name == "f32" else (2100, 2001, 2053) if name == "f64" else (520, 1001, 530)
     modes = (_lib.C_ACCUMULATE, _lib.C_BIAS, _lib.C_OVERWRITE, _lib.C_ACCUMULATE)
+    whole = True if name == "f64" else "offered"              # a copy of a whole operand
     for (ta, tb), mode in zip(TRANS, modes):
-        run_case(rng, name, m, k, n, ta, tb, (0, 0, 0), mode, workspace=True, one_rounding=half)             # odd k: A and B padded, C as it lies
-    run_case(rng, name, m + 3, k + 7, n + 1, True, False, ODD, _lib.C_BIAS, base=1, workspace=True, one_rounding=half)   # everything odd, C padded too
-    run_case(rng, name, m, k + 7, n - 6, False, True, (0, 8, 5), _lib.C_ACCUMULATE, batches=2, gap=3, workspace=True, one_rounding=half)
+        run_case(rng, name, m, k, n, ta, tb, (0, 0, 0), mode, workspace=whole, one_rounding=half)            # odd k: A and B padded, C as it lies
+    run_case(rng, name, m + 3, k + 7, n + 1, True, False, ODD, _lib.C_BIAS, base=1, workspace=whole, one_rounding=half)   # everything odd, C padded too
+    run_case(rng, name, m, k + 7, n - 6, False, True, (0, 8, 5), _lib.C_ACCUMULATE, batches=2, gap=3, workspace=whole, one_rounding=half)
     run_case(rng, name, m, 1008, n - 6, False, False, (0, 0, 0), _lib.C_OVERWRITE, batches=2, bcast_b=True, base=3, workspace=64 << 20, one_rounding=half)   # only the base pointers are odd
     if True:
         # only k misses the chunk and an operand stored [k][m] / [k][n] keeps the 16-byte rule: it is read where it lies and only
@@ -212,28 +214,77 @@ def test_rows_that_are_not_16_byte_multiples_through_padded_copies(name):
         m2, n2 = (1700, 1704) if f32 else (1304, 1712) if half else (2100, 2056) if name == "f64" else (528, 544)
         ks = (1501, 1502, 1503, 1535) if f32 else (1001, 1003, 1017, 1087) if half else (2001, 2003, 2005, 2047) if name == "f64" else (1001, 1009, 1023, 1090)
         for (ta, tb), mode, k2 in zip(TRANS, modes, ks):
-            run_case(rng, name, m2, k2, n2, ta, tb, (0, 0, 0), mode, workspace=True, one_rounding=half,
+            run_case(rng, name, m2, k2, n2, ta, tb, (0, 0, 0), mode, workspace=True if ta and not tb else whole, one_rounding=half,
                      flags=_lib.GEMM_KEEP_K_ORDER if f32 else 0, f32_bits=f32)
-        run_case(rng, name, m2, ks[0], n2, False, False, (0, 16, 16), _lib.C_ACCUMULATE, batches=2, gap=16, workspace=True, one_rounding=half)
+        run_case(rng, name, m2, ks[0], n2, False, False, (0, 16, 16), _lib.C_ACCUMULATE, batches=2, gap=16, workspace=whole, one_rounding=half)
         run_case(rng, name, m2, ks[1] + 8, n2, True, False, (16, 0, 0), _lib.C_BIAS, batches=3, bcast_b=True, workspace=True, one_rounding=half)
         if f32:
             run_case(rng, name, 520, 16385, 512, False, False, (0, 0, 0), _lib.C_OVERWRITE, workspace=True)          # few tiles, a deep k
         if half:
             # products that go out as two launches with shifted operand pointers (rows / columns split, a batch in two parts)
-            run_case(rng, name, 2056, 1001, 2320, False, False, (0, 0, 0), _lib.C_ACCUMULATE, workspace=True, one_rounding=True)
+            run_case(rng, name, 2056, 1001, 2320, False, False, (0, 0, 0), _lib.C_ACCUMULATE, workspace=whole, one_rounding=True)
             run_case(rng, name, 2320, 1001, 2056, True, False, (0, 0, 0), _lib.C_OVERWRITE, workspace=True, one_rounding=True)
             run_case(rng, name, 264, 1001, 2304, False, False, (0, 0, 0), _lib.C_ACCUMULATE, batches=33, workspace=True, one_rounding=True)
 
 
-@pytest.mark.parametrize("name,m,k,n", [("bf16", 264, 4097, 2001), ("i8", 40, 8193, 1003), ("f32", 700, 4097, 1501)])
-def test_padded_copies_of_one_launch_with_rows_of_several_pieces(name, m, k, n):
-    """A, B and the C that is added to are jobs of one copy launch: rows of more than 256 chunks (several pieces) beside shorter ones,
-    no job a whole number of blocks, and the operands in both orders."""
-    rng = np.random.default_rng(8150 + k)
-    half = name == "bf16"
-    run_case(rng, name, m, k, n, False, True, (0, 0, 0), _lib.C_ACCUMULATE, workspace=True, one_rounding=half)
-    run_case(rng, name, m, k, n, True, False, ODD, _lib.C_ACCUMULATE, base=1, workspace=True, one_rounding=half)
-    run_case(rng, name, m, k, n, False, False, (3, 5, 0), _lib.C_ACCUMULATE, batches=2, gap=1, bcast_b=True, workspace=True, one_rounding=half)
+def copies_against_rows_as_they_lie(rng, name, m, k, n, ta, tb, pads, mode, batches=1, gap=0, base=0, bcast_b=False):
+    """The call with room for padded copies and the call without: the same bytes, between the rows of C too; some rows against 64 bits."""
+    npdt, code, _ = DTYPES[name]
+    es = np.dtype(npdt).itemsize
+    ra, ca = (k, m) if ta else (m, k)
+    rb, cb = (n, k) if tb else (k, n)
+    lda, ldb, ldc = ca + pads[0], cb + pads[1], n + pads[2]
+    sA, sB, sC = ra * lda + gap, (0 if bcast_b else rb * ldb + gap), m * ldc + gap
+    bufA, bufB = fill(rng, name, base + batches * (ra * lda + gap) + 8, 0.5), fill(rng, name, base + batches * (rb * ldb + gap) + 8, 0.5)
+    bufC, bias = fill(rng, name, base + batches * sC + 8), fill(rng, name, n)
+    dA, dB, dbias = upload(bufA), upload(bufB), upload(bias)
+    d = _lib.GemmDesc()
+    d.dtype, d.transpose_a, d.transpose_b, d.c_mode = code, int(ta), int(tb), mode
+    d.m, d.k, d.n, d.batches = m, k, n, batches
+    d.lda, d.ldb, d.ldc, d.stride_a, d.stride_b, d.stride_c = lda, ldb, ldc, sA, sB, sC
+    if mode == _lib.C_BIAS:
+        d.bias, d.bias_col_stride = dbias.data_ptr(), 1
+    lib = _lib.load()
+    need = lib.ntg_gemm_workspace_bytes(ctypes.byref(d))
+    assert need > 0 or base, (name, m, k, n)                # (the query takes the pointers as aligned)
+    need = need or 192 << 20
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    results = []
+    for room in (need, 0):
+        dC = upload(bufC)
+        d.workspace, d.workspace_bytes = (ws.data_ptr() if room else None), room
+        _lib.check(lib.ntg_gemm_dev(ctypes.byref(d), dA.data_ptr() + base * es, dB.data_ptr() + base * es, dC.data_ptr() + base * es,
+                                    ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        torch.cuda.synchronize()
+        results.append(dC.cpu().numpy().view(npdt))
+    assert results[0].tobytes() == results[1].tobytes(), (name, m, k, n, ta, tb, mode)
+    for bi in {0, batches - 1}:
+        rows = np.array([0, m // 2, m - 1])
+        al, bl = sub(bufA, base + bi * sA, ra, ca, lda), np.ascontiguousarray(sub(bufB, base + bi * sB, rb, cb, ldb))
+        al = np.ascontiguousarray(al[:, rows].T if ta else al[rows])
+        start = sub(bufC, base + bi * sC, m, n, ldc)[rows] if mode == _lib.C_ACCUMULATE else np.broadcast_to(bias, (3, n)) if mode == _lib.C_BIAS else np.zeros((3, n), npdt)
+        got = np.ascontiguousarray(sub(results[0], base + bi * sC, m, n, ldc)[rows])
+        if name in FLOATS:
+            exact = widen(name, al) @ (widen(name, bl).T if tb else widen(name, bl)) + widen(name, np.ascontiguousarray(start))
+            tol = HALF_REL * np.abs(exact).max() if name in ("bf16", "f16") else float_tol(k, widen(name, al), widen(name, bl))
+            assert np.abs(widen(name, got) - exact).max() <= tol
+        else:
+            exact = al.astype(np.int64) @ (bl.T if tb else bl).astype(np.int64) + start.astype(np.int64)
+            assert np.array_equal(got, exact.astype(npdt))
+
+
+@pytest.mark.parametrize("name", ["bf16", "f16", "i8", "f32"])
+def test_padded_copies_of_whole_operands(name):
+    """From where whole copies pay: every flag pair and C mode, A, B and the C that is added to in one copy launch (rows of more than 256 chunks beside
+    shorter ones, no job a whole number of blocks), batches with a broadcast operand, everything odd, only the base pointers odd."""
+    rng = np.random.default_rng(8150 + list(DTYPES).index(name))
+    m, k, n = (2100, 2101, 2102) if name == "f32" else (2600, 2601, 2602)
+    for (ta, tb), mode in zip(TRANS, (_lib.C_ACCUMULATE, _lib.C_BIAS, _lib.C_OVERWRITE, _lib.C_ACCUMULATE)):
+        copies_against_rows_as_they_lie(rng, name, m, k, n, ta, tb, (0, 0, 0), mode)
+    copies_against_rows_as_they_lie(rng, name, m + 3, k + 8, n + 1, True, False, ODD, _lib.C_BIAS, base=1)
+    copies_against_rows_as_they_lie(rng, name, 1032, 8209, 2101, False, True, (3, 5, 0), _lib.C_ACCUMULATE)
+    copies_against_rows_as_they_lie(rng, name, m, k, n // 2, False, False, (3, 5, 1), _lib.C_ACCUMULATE, batches=2, gap=3, bcast_b=True)
+    copies_against_rows_as_they_lie(rng, name, 2608, 2624, 2640, False, False, (0, 0, 0), _lib.C_OVERWRITE, base=3)
 
 
 def _random_dim(rng, hi):

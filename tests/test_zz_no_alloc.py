@@ -99,11 +99,13 @@ def test_noalloc_entry_point_matches_the_workspace_entry_point():
     _both(lib, rng, np.int16, 200, 1400, 260, False, False, ACC, batches=3)
     # padded copies (rows that are not 16-byte multiples: A, B and C copied into the array, the bias written as the padded
     # C's starting value, the result copied back), a larger product before a smaller one, then the 8-bit form
-    big = _both(lib, rng, "bf16", 2048, 1001, 2044, False, False, BIAS)
-    small = _both(lib, rng, "bf16", 1032, 2001, 1048, False, True, ACC)
+    big = _both(lib, rng, "bf16", 2800, 2501, 2604, False, False, BIAS)
+    small = _both(lib, rng, "bf16", 2600, 2501, 2568, False, True, ACC)
     assert small < big, (small, big)
-    _both(lib, rng, np.float16, 2048, 1001, 2044, True, False, ACC)
-    _both(lib, rng, np.int8, 520, 1001, 530, False, False, ACC)
+    _both(lib, rng, np.float16, 2800, 2501, 2604, True, False, ACC)
+    _both(lib, rng, np.int8, 2600, 2601, 2602, False, False, ACC)
+    for dtype, m, k, n in (("bf16", 2048, 1001, 2044), ("bf16", 1032, 2001, 1048), (np.float16, 2048, 1001, 2044), (np.int8, 520, 1001, 530)):
+        _both(lib, rng, dtype, m, k, n, False, False, ACC, expect_workspace=False)                          # too small to repay the copies
     # a batch whose items are split along k (the partial sums of every item and k range in the array)
     _both(lib, rng, "bf16", 256, 4096, 512, False, False, ACC, batches=3)
     _both(lib, rng, np.float32, 64, 4096, 256, False, True, BIAS, batches=5)
