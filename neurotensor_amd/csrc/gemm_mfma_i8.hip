@@ -8,7 +8,6 @@ hipError_t launch_gemm_mfma_i8(int dtype, bool ta, bool tb, const GemmParams& p,
     if ((p.tailA || p.tailB) && !ring_eligible(p, ta, 1)) return hipErrorInvalidValue;     // (only the DMA-fed kernel reads copied tail rows)
     if (!ring_eligible(p, ta, 1)) {
         if (any_eligible(p, dtype, ta, tb)) return launch_gemm_any(dtype, ta, tb, p, s);
-        if (p.cmode == C_PARTIAL) return hipErrorInvalidValue;      // (only the DMA-fed kernel writes 32-bit sums)
         return launch_gemm_valu(dtype, ta, tb, p, s);
     }
     // (an MN-major 192-row tile of bytes has 12 chunks per k-row, which the chunk swizzle of the transposing reads does not fit)
@@ -22,7 +21,7 @@ hipError_t launch_gemm_mfma_i8(int dtype, bool ta, bool tb, const GemmParams& p,
         if (ring16_deep128(ring16_tiles(128, q.M, q.N, q.batch), q.K / 2)) return launch_ring_wb<DT_I8, 2, 0, 2>(ta, tb, q, s);
         return launch_ring_wb<DT_I8, 2>(ta, tb, q, s);
     };
-    if (p.batch == 1 && p.cmode != C_PARTIAL) {
+    if (p.batch == 1) {
         // (the estimate of the 16-bit kernel: a K-step of 64 bytes per row is 64 k here, so the same tile takes half the steps)
         const Ring16Split sp = ring16_split(p.M, p.N, p.K, rect);
         if (sp.axis) {

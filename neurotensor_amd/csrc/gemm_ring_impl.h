@@ -1264,7 +1264,7 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, WB_, CONV)) gemm_ring_
         else epilogue(std::integral_constant<int, C_OVERWRITE>{});
     } else {
         if (p.cmode == C_ACCUMULATE) epilogue(std::integral_constant<int, C_ACCUMULATE>{});
-        else if (p.cmode == C_PARTIAL) epilogue(std::integral_constant<int, C_PARTIAL>{});
+        else if (ES != 1 && p.cmode == C_PARTIAL) epilogue(std::integral_constant<int, C_PARTIAL>{});
         else if (p.cmode == C_BIAS) epilogue(std::integral_constant<int, C_BIAS>{});
         else epilogue(std::integral_constant<int, C_OVERWRITE>{});
     }

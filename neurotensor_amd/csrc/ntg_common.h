@@ -26,7 +26,7 @@ enum CMode : int {
     C_OVERWRITE = 0,   // C  = op(A).op(B)          (caller knows C would be zeros)
     C_ACCUMULATE = 1,  // C += op(A).op(B)          (contract of nt_matmult, nt_matmult.hpp:370-378)
     C_BIAS = 2,        // C  = bias (+) op(A).op(B) (cpu::linear, matmult_cpu.cpp:1637-1647)
-    C_PARTIAL = 3      // internal: write the 32-bit accumulators (fp32 sums of a split-K range; integer sums of 8-bit operands) to a 4-byte matrix at C; DMA-fed kernels and gemm_any_impl.h
+    C_PARTIAL = 3      // internal: write the 32-bit accumulators of a k range to a 4-byte matrix at C: fp32 sums (DMA-fed kernels, gemm_any_impl.h), integer sums of 8-bit operands (gemm_any_impl.h)
 };
 
 // Unsigned division by a divisor fixed at launch (round-up multiplier form): exact for every

@@ -461,7 +461,7 @@ AnySplitPlan plan_int_split(const ntg::GemmParams& p, int dtype, bool ta, bool t
     const int64_t steps = (p.K + 31) / 32, tiles = ((p.M + 63) / 64) * ((p.N + 63) / 64) * (int64_t)p.batch;
     if (tiles > 255) return pl;
     const int64_t per_range = (int64_t)p.batch * p.M * pl.ldp * P;
-    const auto [alone, shared] = k_step_us(dtype);
+    const double alone = k_step_us(dtype).alone, shared = k_step_us(dtype).shared;
     double best_us = 0.95 * (double)steps * alone;
     // (The second launch and its workspace take a host about 5 us, 8.3 -> 13.5 us a call through the Python face: what the GPU does meanwhile stays whole.
     //  64 x k x 64 through that face, whole / ranges: Int32 k = 384 9.0 / 13.9 us, 1000 17.7 / 13.6, 4096 59 / 13.6; Int16 k = 1000 10.3 / 13.5, 2048 17.0 / 13.7.)
@@ -488,7 +488,7 @@ AnySplitPlan plan_any_split(const ntg::GemmParams& p, int dtype, bool ta, bool t
     // each; a launch costs about 2.5 us, the second pass 4 us + the partial sums written and read at 4 TB/s.  Of 2 .. 32 ranges the choice was the
     // best measured one or within 10 % of it on fourteen shapes (BFloat16 576 x 3797 x 448, ranges 1 / 2 / 4 / 8: 19.6 / 16.5 / 13.0 / 14.5 us;
     // 448 x 3704 x 166: 25.9 us whole, 10.4 in eight ranges; Float32 128 x 6463 x 720: 146 us whole, 24 in 21 ranges).
-    const auto [alone, shared] = k_step_us(dtype);
+    const double alone = k_step_us(dtype).alone, shared = k_step_us(dtype).shared;
     auto estimate_us = [&](int64_t tls, int64_t its, int64_t sp, int64_t per) {
         const int64_t wgs = tls * sp;
         const double second_pass = sp == 1 ? 0.0 : 4.0 + 8.0 * (double)sp * (double)its * (double)p.M * (double)p.N / 4.0e6;
