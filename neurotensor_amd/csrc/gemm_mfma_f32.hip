@@ -244,10 +244,8 @@ hipError_t launch_gemm_mfma_f32(bool ta, bool tb, const GemmParams& p, hipStream
     if (ring_eligible(p, ta, 4))
         return ring_f32_tile_edge(p) == 64 ? launch_ring_wb<DT_F32, 1>(ta, tb, p, s) : launch_ring_wb<DT_F32, 2>(ta, tb, p, s);
     if (any_eligible(p, DT_F32, ta, tb)) return launch_gemm_any(DT_F32, ta, tb, p, s);
-    // rows that are not 16-byte aligned (or pointer tables): register-staged kernel, 128 x 128 x 32 tiles unless that
-    // leaves most of the 256 CUs idle; then 64 x 64 x 32
-    const int64_t big_tiles = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
-    if (big_tiles >= 192 && p.M > 64 && p.N > 64) return launch_trans<DT_F32, 2, 2, 32>(ta, tb, p, s);   // a 128-wide tile would be half empty
+    // rows shorter than a 16-byte chunk, pitches from 8 MiB on: register-staged kernel, 64 x 64 x 32 (128 x 128: 2048 x 3 x 2048 11.9 us against 9.6, 2048 x 2048 x
+    // 2048 at such a pitch 167 / 161)
     return launch_trans<DT_F32, 1, 1, 32>(ta, tb, p, s);
 }
 hipError_t launch_gemm_ring_only_f32(bool ta, bool tb, const GemmParams& p, hipStream_t s, bool* taken) {
