@@ -269,6 +269,7 @@ struct PadPlan {
     int64_t lda2, ldb2, rowsA2, rowsB2, a_bytes, b_bytes, c_bytes;
     int64_t bytes() const { return a_bytes + b_bytes + c_bytes; }
 };
+SplitPlan plan_splitk(const ntg::GemmParams& p, int dtype, bool ta);
 static PadPlan plan_pad(const ntg::GemmParams& p, int dtype, bool ta, bool tb) {
     PadPlan pl;
     std::memset(&pl, 0, sizeof pl);
@@ -279,7 +280,10 @@ static PadPlan plan_pad(const ntg::GemmParams& p, int dtype, bool ta, bool tb) {
     // From where a faster kernel repays the copies: 8-bit against the vector ALU (40 x), 16-bit against the register-staged
     // kernel at half the rate, Float32 / Float64 against the register-staged kernel at 0.8 - 0.85 of the DMA-fed one.
     const double macs = (double)p.M * p.N * p.K * p.batch;
-    if (macs < (byte ? 268435456.0 : half ? 2147483648.0 : dtype == ntg::DT_F32 ? 4294967296.0 : 8589934592.0)) return pl;
+    const double from = byte ? 268435456.0 : half ? 2147483648.0 : dtype == ntg::DT_F32 ? 4294967296.0 : 8589934592.0;
+    if (macs < from) return pl;
+    // (an item that alone is too small for copies, and is split along k instead, keeps that order of summation in a batch that is not: Float64)
+    if (macs / p.batch < from && plan_splitk(p, dtype, ta).splits > 1) return pl;
     auto up = [&](int64_t v) { return (v + ve - 1) / ve * ve; };
     pl.Kp = (int)up(p.K); pl.Np = (int)up(p.N); pl.Mp = ta ? (int)up(p.M) : p.M;
     auto misaligned = [&](const void* ptr, int64_t ld, int64_t stride) {

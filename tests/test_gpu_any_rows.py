@@ -287,3 +287,17 @@ def test_lists_behind_pointer_tables_have_the_bits_of_their_items(name, ta, tb):
         d.flags, d.batches, d.m, d.k, d.n = _lib.GEMM_PTRS_ITEM_ORDER, 2, 64, 8192, 64
         assert lib.ntg_gemm_workspace_bytes(ctypes.byref(d)) > 0
         assert lib.ntg_gemm_ptrs_dev(ctypes.byref(d), tab.data_ptr(), tab.data_ptr() + 16, tab.data_ptr() + 32, st) == 1
+
+
+def test_float64_items_that_are_split_alone_are_split_in_a_batch_too_large_for_it_to_matter():
+    """128 items of an odd n are enough multiply-adds for padded copies, one is not and goes out in k ranges: the same bits."""
+    lib = _lib.load()
+    m, k, n, batch = 64, 4096, 257, 128
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    a, b = (torch.randn(batch, *s, generator=gen, device=DEV, dtype=torch.float64) for s in ((m, k), (k, n)))
+    together, alone = (torch.zeros(batch, m, n, device=DEV, dtype=torch.float64) for _ in range(2))
+    strides = (m * k, k * n, m * n)
+    product(lib, a, b, together, m, k, n, batch, strides, False, False, _lib.C_OVERWRITE)
+    for i in (0, batch - 1):
+        assert product(lib, a, b, alone, m, k, n, 1, strides, False, False, _lib.C_OVERWRITE, first=i) > 0
+        assert torch.equal(together[i], alone[i])
