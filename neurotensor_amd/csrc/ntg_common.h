@@ -101,9 +101,9 @@ struct GemmParams {
     // A batch whose items are each split into k ranges (split-K of a batch): launch index b = range * krange_items + item,
     // A and B of it lie at item * sA + range * sAk (sB, sBk); C (the partial sums) at b * sC.  0: a plain batch.
     int krange_items;
+    int fold_steps;          // k ranges inside one workgroup (gemm_any_impl.h): K-steps in each but the last; 0: none
     int64_t sAk, sBk;
     int k_total;             // k ranges of unequal length (gemm_any_impl.h): K is a range's length, the last one has what is left of k_total; 0: all equal
-    int fold_steps;          // k ranges inside one workgroup (gemm_any_impl.h): K-steps in each but the last; 0: none
     int M, N, K, batch;      // logical sizes (after the transpose flags)
     int cmode;
     int tiles_m, tiles_n;
@@ -117,14 +117,14 @@ struct GemmParams {
     int tail_k0;
     int keep_k_order;        // never split along k (the caller wants the one chain per element in ascending k)
     // Pointer tables whose entries' alignment the library found out on the device (see gemm_ptrs): the product is launched on
-    // the DMA-fed kernel AND on the register-staged one; a kernel whose gate_want differs from *gate returns at once.
+    // the DMA-fed kernel AND on the one that takes rows as they lie; a kernel whose gate_want differs from *gate returns at once.
     const int* gate;
     int gate_want;
     int ptrs_aligned;        // pointer tables only: the caller vouches that every entry is a multiple of 16 bytes (the tables
                              // live in device memory, the host cannot look); lets table batches onto the DMA-fed kernels
     int group_m;             // DMA-fed kernels: tile rows per group of the tile order (0: the default, 4; see tile_coords)
     int act;                 // ACT_RELU: the stored result is max(result, 0) (relu_ of the reference = clamp_(x, 0): NaN and -0 become +0);
-                             // honoured by the DMA-fed Float16 / BFloat16 / Float32 kernels and the split-K reduction only
+                             // honoured by the DMA-fed Float16 / BFloat16 / Float32 kernels, gemm_any_impl.h and the split-K reduction only
     ConvGeom conv;           // used by the implicit-im2col kernels only: B = image, op(B) = col or col^T
 };
 enum { ACT_NONE = 0, ACT_RELU = 1 };
@@ -319,11 +319,11 @@ hipError_t launch_gemm_mfma(int dtype, bool ta, bool tb, const GemmParams& p, hi
 // Float16 / BFloat16 / Float32 on the DMA-fed kernel or not at all (*taken = false, nothing launched): the kernel whose
 // epilogue applies GemmParams::act
 hipError_t launch_gemm_ring_only(int dtype, bool ta, bool tb, const GemmParams& p, hipStream_t s, bool* taken);
-// C[b][m][n] = max(C[b][m][n], 0) in place (floating dtypes)
 // Int16 / 32 / 64 and unsigned on the 8-bit matrix pipe (planes = bytes of an element; gemm_int_impl.h)
 hipError_t launch_gemm_int(int planes, bool ta, bool tb, const GemmParams& p, hipStream_t s);
 // Float16 / BFloat16 / Float32 / Int8 on rows that start anywhere (gemm_any_impl.h); the caller has checked any_eligible()
 hipError_t launch_gemm_any(int dtype, bool ta, bool tb, const GemmParams& p, hipStream_t s);
+// C[b][m][n] = max(C[b][m][n], 0) in place (floating dtypes)
 hipError_t launch_relu_inplace(int dtype, void* C, int64_t ldc, int64_t sC, int64_t M, int64_t N, int64_t batch, hipStream_t s);
 hipError_t launch_gemm_valu(int dtype, bool ta, bool tb, const GemmParams& p, hipStream_t s);
 hipError_t launch_gemm_mfma_i8(int dtype, bool ta, bool tb, const GemmParams& p, hipStream_t s);   // Int8 / UInt8: MFMA where rows are 16-byte multiples
