@@ -464,7 +464,7 @@ def main():
         run("mid_bf16_2048x4096x4096", G(torch.bfloat16, 2048, 4096, 4096, scale=0.05, mode=_lib.C_OVERWRITE), 2.0 * 2048 * 4096 * 4096,
             PEAK_TFLOPS["bf16"])
         # a batch as a strided launch and as device pointer tables whose entries the caller vouches for (ntg_gemm_ptrs_dev with
-        # NTG_GEMM_PTRS_ALIGNED16: the same DMA-fed kernels; without the vouch the register-staged ones)
+        # NTG_GEMM_PTRS_ALIGNED16: the same DMA-fed kernels; without the vouch a check on the device comes first)
         fb = 2.0 * 32 * 1024 ** 3
         run("batch_bf16_32x1024_strided", G(torch.bfloat16, 1024, 1024, 1024, batch=32, scale=0.05, mode=_lib.C_OVERWRITE), fb, PEAK_TFLOPS["bf16"])
 

@@ -19,6 +19,8 @@
 //
 // What bounds it: the latency of the loads where few tiles have a deep k (hence the k ranges, and 64 x 64 tiles that put several workgroups
 // on every CU), the LDS of the CU where there are many (64 x 64 tiles read 256 bytes of LDS per cycle of MFMA, twice what it delivers).
+// Operands that no cache holds arrive at the latency of the two or three K-steps in flight: Float16 1023 x 1537 x 2049 26.8 us in cache, 28.5 cycled through
+// 0.8 GB, 32.6 alone behind a sweep of the caches (padded copies, which stream them in: 29.5, 31 and 34.6).
 // Measured, the register-staged kernel with element-wise loads (or the vector ALU, Int8) before -> now: BFloat16 448 x 3704 x 166 A^T.B 263 -> 10.8 us,
 // 576 x 3797 x 448 226 -> 12.8, 2429 x 1536 x 157 77 -> 13.5, 3712 x 543 x 448 45 -> 9.9; Float32 128 x 6463 x 720 218 -> 24,
 // 1000 x 774 x 64 35 -> 9.8, 2049^3 213 (padded copies) -> 187; Int8 256 x 1792 x 39 198 -> 8.2 us.
@@ -436,9 +438,10 @@ template <int DT, bool FOLD>
 static hipError_t launch_any_tile(bool ta, bool tb, const GemmParams& p, hipStream_t s) {
     // 128 x 128 tiles where these reach three quarters of the CUs (BFloat16 3618 x 739 x 9392: 84 us against 112 on 128 x 64 and 126 on 64 x 64;
     // 2429 x 1536 x 157, 38 tiles: 23 against 12), 128 x 64 where those put one on each CU at most and 64 x 64 more than one (Float16 1023 x 1537 x
-    // 1985: 18.6 us against 21.6 and 26.5 on 128 x 128), and 128 x 128 again from half of the CUs on where 128 x 64 would need a second round (1023 x 1537
-    // x 2049, 136 tiles: 26.7 against 30 on either; 1337 x 777 x 1555, 143 tiles: 18.2, 19.0 and 17.6).  Float32 always on 64 x 64: the matrix pipe
-    // is its bound on either and the smaller tile spreads evenly (2049^3: 188 us against 274).
+    // 1985: 18.6 us against 21.6 and 26.5 on 128 x 128), and 128 x 128 again from half of the CUs on where 128 x 64 would need a second round.  That last line
+    // on 21 shapes of 128 .. 191 tiles, single and batched, every storage form, BFloat16 and Int8: the best of the three or within 2 % of it (BFloat16 1023 x
+    // 1537 x 2049 26.8 us, 29.4 on 128 x 64, 29.3 on 64 x 64; 1281 x 3001 x 1667 43.6 / 52.2 / 51.4; 6 x (513 x 1537 x 641) 27.3 / 31.6 / 29.5; 2049 x 515 x 1281 14.6 / 15.2 /
+    // 14.3).  Float32 always on 64 x 64: the matrix pipe is its bound on either and the smaller tile spreads evenly (2049^3: 188 us against 274).
     if constexpr (DT != DT_F32) {
         auto tiles = [&](int r, int c) { return (int64_t)((p.M + r - 1) / r) * ((p.N + c - 1) / c) * p.batch; };
         if (p.M > 64 && p.N > 64 && (tiles(128, 128) >= 192 || (tiles(128, 128) >= 128 && tiles(128, 64) > 256))) return launch_any_wb<DT, 2, 2, FOLD>(ta, tb, p, s);

@@ -14,9 +14,10 @@
 //   * The products of one shift i + j have accumulators of their own (P sets, 32-bit sums: P K 2^14 < 2^31), folded together at the end.
 //   * 64 x 64 tiles, 128 x 64 where they are many; four wavefronts of 1 x 1 or 2 x 1 blocks of 32 x 32.  (128 x 128 with one workgroup per CU was
 //     measured slower: Int32 8 x 1024^3 97.6 us.)
-// Bound: vector instructions, LDS and the matrix pipe's P (P + 1) / 2 products about evenly.  Before, the digits went through memory (a pass that split each
-// operand, P products writing 32-bit sums, a pass that added these) or the product ran on the vector ALU: Int32 8 x 1024^3 158 -> 84 us, 80 x 1088 x 152
-// 150 -> 20; Int16 23 x 58 x 3008 x 3072 1040 -> 114; Int64 1024^3 135 -> 41, 16 x 824 x 3454 x 80 1219 -> 236 us.
+// Bound: vector instructions, LDS and the matrix pipe's P (P + 1) / 2 products about evenly; Int32 on 128 x 64 tiles spills 34 to 53 of its 256 registers (140 to 176
+// bytes a lane, none for A.B^T): two workgroups on a CU leave no more.  Before, the digits went through memory (a pass that split each
+// operand, P products writing 32-bit sums, a pass that added these) or the product ran on the vector ALU: Int32 8 x 1024^3 147 -> 84 us, 80 x 1088 x 152
+// 150 -> 20; Int16 23 x 58 x 3008 x 3072 1040 -> 121; Int64 1024^3 135 -> 41, 16 x 824 x 3454 x 80 1219 -> 236 us.
 #pragma once
 #include "gemm_any_impl.h"
 

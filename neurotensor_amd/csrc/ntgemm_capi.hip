@@ -256,8 +256,8 @@ int launch_gemm(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s) {
 struct SplitPlan { int splits; int64_t kc; int64_t bytes; };
 
 // Padded copies.  The DMA-fed kernels need 16-byte rows (leading dimensions, batch strides, base pointers, and K, N -- M
-// under transpose_a -- multiples of one 16-byte chunk); a product that misses this falls to the vector ALU
-// (8-bit: 40 x slower) or the register-staged kernel (16-bit: half the rate; Float32 / Float64: 0.8 - 0.85 of it).  With a workspace the operands that need it
+// under transpose_a -- multiples of one 16-byte chunk); a product that misses this runs on rows as they lie (gemm_any_impl.h), Float64 on
+// the register-staged kernel at 0.8 of the rate.  With a workspace the operands that need it
 // are copied into rows padded with zeros to whole chunks (zero products add nothing: bit-identical integers, the same
 // single rounding for the 16-bit floats), the product runs on the DMA-fed kernel, and a result whose own rows are not
 // 16-byte multiples is computed into a padded copy and copied back.  Taken for products large enough to repay the copies.
@@ -277,8 +277,8 @@ static PadPlan plan_pad(const ntg::GemmParams& p, int dtype, bool ta, bool tb) {
     const bool wide = dtype == ntg::DT_F32 || dtype == ntg::DT_F64;
     if ((!half && !byte && !wide) || p.Aptr || p.Bptr || p.Cptr || p.M <= 32) return pl;
     const int64_t es = ntg::elem_size(dtype), ve = 16 / es;
-    // From where a faster kernel repays the copies: 8-bit against the vector ALU (40 x), 16-bit against the register-staged
-    // kernel at half the rate, Float32 / Float64 against the register-staged kernel at 0.8 - 0.85 of the DMA-fed one.
+    // From where copies of an operand's last k-rows, as good as free, pay; Float64: from where whole copies pay against the register-staged kernel.
+    // (Whole copies of the other types: see below.)
     const double macs = (double)p.M * p.N * p.K * p.batch;
     const double from = byte ? 268435456.0 : half ? 2147483648.0 : dtype == ntg::DT_F32 ? 4294967296.0 : 8589934592.0;
     if (macs < from) return pl;
@@ -433,8 +433,8 @@ SplitPlan plan_splitk(const ntg::GemmParams& p, int dtype, bool ta) {
     return none;
 }
 
-// k ranges of a product whose rows miss the 16-byte rule by their SIZES (gemm_any_impl.h serves it): as plan_splitk a function of one item's
-// sizes and pitches only.  kc is a whole number of K-steps, the last range is what is left.  Rows of the partial sums hold whole 16-byte chunks.
+// k ranges of a product whose rows miss the 16-byte rule by their SIZES (gemm_any_impl.h serves it): for floats, as plan_splitk, a function of one
+// item's sizes and pitches only.  kc is a whole number of K-steps, the last range is what is left.  Rows of the partial sums hold whole 16-byte chunks.
 // The integers of more than a byte likewise (gemm_int_impl.h).
 // inside: a workgroup runs all ranges of its tile (the sums of these are added in registers, in the order of the second pass: the same bits).  It needs
 // no room; 256 bytes stand for the caller's leave to change the order of summation, which a workspace is.
@@ -1973,7 +1973,7 @@ static ConvBackwardPlan plan_conv_backward_g(int dtype, bool want_dx, bool want_
     pl.phase_dx = pl.phases.ok;
     pl.need_phase_dx = pl.phase_dx ? pl.phases.bytes() : 0;
     // strides > 1 on few channels: W^T . dY + col2im.  W_g is stored [og][channels of the group * taps]; where those rows miss the
-    // 16-byte rule (3 channels by 7 x 7: 147) the product would go to the register-staged kernel, so W is copied to [..][og] behind the col matrix
+    // 16-byte rule (3 channels by 7 x 7: 147) the product would run on rows as they lie, so W is copied to [..][og] behind the col matrix
     // and dY and col, whose rows keep the rule, stay where they are.  From 2^30 multiply-adds on, where every layer timed gains; us per backward
     // call as stored | transposed, at n * 2^30 multiply-adds: Float32 3 x 224 x 224 -> 64 by 7 x 7 at stride 2 n = 0.22 57 | 57, 0.44 80 | 73,
     // 1.76 214 | 181, 3.52 405 | 352; 3 x 256 x 256 -> 32 by 5 x 5 0.29 76 | 78, 1.17 237 | 230; BFloat16 0.22 49 | 48, 1.76 213 | 128, 3.52 362 | 209.
