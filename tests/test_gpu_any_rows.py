@@ -69,8 +69,8 @@ def test_batches_pitches_and_what_is_added_to(name):
     lib = _lib.load()
     st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     gen = torch.Generator().manual_seed(6)
-    for m, k, n in ((66, 70, 37), (45, 2051, 97)):
-        batch, lda, ldb, ldc = 3, k + 2, n + 1, n + 3
+    for m, k, n, batch in ((66, 70, 37, 3), (45, 2051, 97, 3), (45, 2051, 97, 160)):       # (160: the ranges of a float inside a workgroup)
+        lda, ldb, ldc = k + 2, n + 1, n + 3
         a, b, c0 = values((batch, m, lda), name, gen), values((batch, k, ldb), name, gen), values((1 + batch * m * ldc,), name, gen)
         ta, tb, one = a.to(DEV), b.to(DEV), c0.to(DEV)
         both = [c0.to(DEV), one]
