@@ -286,6 +286,7 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, WB_, CONV)) gemm_ring_
     const T* A = p.Aptr ? static_cast<const T*>(p.Aptr[b]) : static_cast<const T*>(p.A) + operand_offset(p, b, p.sA, p.sAk);
     const T* B = p.Bptr ? static_cast<const T*>(p.Bptr[b]) : static_cast<const T*>(p.B) + operand_offset(p, b, p.sB, p.sBk);
     T* C = p.Cptr ? static_cast<T*>(p.Cptr[b]) : static_cast<T*>(p.C) + (int64_t)b * p.sC;
+    const int item = GATHERW && p.krange_items ? b / p.krange_items : b;      // (weight gradient: the k range or image; its groups follow each other)
 
     using AccV = typename E::AccV;
     using AccS = typename E::AccS;
@@ -338,7 +339,7 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, WB_, CONV)) gemm_ring_
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     int K = p.K;
     if constexpr (GATHERW) {
-        if (p.conv.k_ranges && p.conv.k_total - b * p.K < K) K = p.conv.k_total - b * p.K;      // (uniform) the last k range is what is left
+        if (p.conv.k_ranges && p.conv.k_total - item * p.K < K) K = p.conv.k_total - item * p.K;      // (uniform) the last k range is what is left
     }
     const int KT = (K + BK - 1) / BK;
     const int last = KT - 1;
@@ -580,7 +581,7 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, WB_, CONV)) gemm_ring_
     if constexpr (GATHERW) {
         const ConvGeom& g = p.conv;
         constexpr int CH = G::CHUNKS;
-        if (g.k_ranges) k4_base = b * p.K;                         // this item's first output pixel, counted through the images
+        if (g.k_ranges) k4_base = item * p.K;                      // this item's first output pixel, counted through the images
         const uint32_t cgc = (uint32_t)p.N / (uint32_t)g.k_drc;  // channels of the slice: N = taps * channels
 #pragma unroll
         for (int x = 0; x < WB; ++x) {
@@ -779,7 +780,7 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, WB_, CONV)) gemm_ring_
         }
         if constexpr (GATHERW && A_KC) {
             if (p.conv.a_steps) {                                  // (uniform) K-step counted through the images -> image, step inside it
-                const uint32_t gs = (uint32_t)(b * (p.K / BK) + kc), im = fast_div(gs, p.conv.div_a_steps);
+                const uint32_t gs = (uint32_t)(item * (p.K / BK) + kc), im = fast_div(gs, p.conv.div_a_steps);
                 return tile_src(baseA + ((int64_t)im * p.conv.a_image_stride * ES + (int64_t)(gs - im * (uint32_t)p.conv.a_steps) * advA));
             }
         }
@@ -1391,11 +1392,11 @@ static hipError_t launch_ring_wb(bool ta, bool tb, const GemmParams& p, hipStrea
     return tb ? launch_ring_cfg<DT, false, true, WB, WBN, KD>(p, s) : launch_ring_cfg<DT, false, false, WB, WBN, KD>(p, s);
 }
 
-// items [b0, b0 + nb) of a strided batch as a product of their own
+// items [b0, b0 + nb) of a strided batch as a product of their own (of a batch in groups: whole images, b0 a multiple of krange_items)
 static inline GemmParams ring_batch_range(const GemmParams& p, int64_t es, int b0, int nb) {
     GemmParams q = p;
-    q.A = static_cast<const char*>(p.A) + (int64_t)b0 * p.sA * es;
-    q.B = static_cast<const char*>(p.B) + (int64_t)b0 * p.sB * es;
+    q.A = static_cast<const char*>(p.A) + (p.krange_items ? (int64_t)(b0 / p.krange_items) * p.sAk : (int64_t)b0 * p.sA) * es;
+    q.B = static_cast<const char*>(p.B) + (p.krange_items ? (int64_t)(b0 / p.krange_items) * p.sBk : (int64_t)b0 * p.sB) * es;
     q.C = static_cast<char*>(p.C) + (int64_t)b0 * p.sC * es;
     if (p.bias) q.bias = static_cast<const char*>(p.bias) + (int64_t)b0 * p.bias_bs * es;
     if (p.tailA) q.tailA = static_cast<const char*>(p.tailA) + (int64_t)b0 * p.s_tailA * es;
@@ -1410,6 +1411,10 @@ template <class Launch>
 static hipError_t launch_ring16_planned(const GemmParams& p, hipStream_t s, Launch&& launch, int rect = RECT_NONE) {
     Ring16Plan pl = ring16_plan(p.M, p.N, p.K, p.batch, rect);
     if (p.cmode == C_PARTIAL || p.Aptr || p.Bptr || p.Cptr) pl.head = p.batch;
+    if (p.krange_items) {                                                            // (whole images: see ring_batch_range)
+        pl.head -= pl.head % p.krange_items;
+        if (pl.head == 0) pl.head = p.batch;
+    }
     if (pl.head >= p.batch) return launch(pl.edge, p);
     const hipError_t e = launch(pl.edge, ring_batch_range(p, 2, 0, pl.head));
     if (e != hipSuccess) return e;

@@ -230,7 +230,8 @@ int launch_gemm(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s) {
     } else {
         bool handled = false;
         // (the streaming kernels for up to 32 rows split k over their wavefronts: not for a caller who wants the one chain)
-        if (!(p.keep_k_order && dtype == ntg::DT_F32)) e = ntg::launch_gemm_skinny(dtype, ta, tb, p, s, &handled);
+        e = hipSuccess;
+        if (!(p.keep_k_order && dtype == ntg::DT_F32) && p.krange_items == 0) e = ntg::launch_gemm_skinny(dtype, ta, tb, p, s, &handled);
         if (e != hipSuccess) return hip_fail(e, "skinny gemm launch");
         if (handled) return finish();
         switch (dtype) {
@@ -667,6 +668,37 @@ int desc_to_params(const ntg_gemm_desc* d, ntg::GemmParams& p) {
     if (p.cmode == NTG_C_BIAS && !p.bias) return fail(NTG_ERR_INVALID_ARGUMENT, "c_mode is bias but bias is null");
     p.keep_k_order = (d->flags & NTG_GEMM_KEEP_K_ORDER) != 0;
     return NTG_OK;
+}
+
+// The groups of a convolution are items of its one launch: item image * groups + group has its operands at group * (its own stride) +
+// image * (the images' stride), its result at a uniform stride (rows of the groups follow each other in every layout used here).  A launch
+// a group is `groups` times the 4-5 us that a launch costs the host and as many half-empty rounds: training steps in groups, us before | now:
+// BFloat16 1 x 96 x 48 x 48 -> 16 by 3 x 3 in 4 groups 118 | 51, Float32 6 x 256 x 32 x 32 -> 96 by 5 x 5 at stride 2 in 4 groups 239 | 99,
+// Float16 10 x 64 x 216 x 216 -> 192 by 3 x 3 in 4 groups 854 | 814; 40 drawn ones 0.77 of their time.
+struct GroupStrides { int64_t a_group, a_image, b_group, b_image, c_item; };      // elements
+template <class Launch>
+static hipError_t launch_groups(ntg::GemmParams p, int dtype, int64_t batch, int64_t groups, const GroupStrides& st, Launch&& launch) {
+    const int64_t es = ntg::elem_size(dtype);
+    // (a grid's 2^31 workgroups hold 32 x 32 tiles of any result that fits the memory, unless the groups are tiny and there are 2^31 of them)
+    if ((double)((p.M + 31) / 32) * ((p.N + 31) / 32) * (double)batch * (double)groups < 2147483647.0) {
+        p.batch = (int)(batch * groups);
+        p.sC = st.c_item;
+        p.sA = groups > 1 ? st.a_group : st.a_image;
+        p.sB = groups > 1 ? st.b_group : st.b_image;
+        if (groups > 1) { p.krange_items = (int)groups; p.sAk = st.a_image; p.sBk = st.b_image; }
+        return launch(p);
+    }
+    for (int64_t g = 0; g < groups; ++g) {
+        ntg::GemmParams q = p;
+        q.batch = (int)batch;
+        q.A = static_cast<const char*>(p.A) + g * st.a_group * es;
+        q.B = static_cast<const char*>(p.B) + g * st.b_group * es;
+        q.C = static_cast<char*>(p.C) + g * st.c_item * (p.cmode == ntg::C_PARTIAL ? 4 : es);
+        q.sA = st.a_image; q.sB = st.b_image; q.sC = groups * st.c_item;
+        const hipError_t e = launch(q);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 }  // namespace
@@ -1281,6 +1313,40 @@ static void fill_conv_geom(ntg::ConvGeom& c, int64_t slice_channels, const Geo3&
     c.div_howo = ntg::make_fastdiv((uint32_t)c.HoWo);
 }
 
+// A plain product per (image, group), strides in elements; the floating types in one launch.
+static int gemm_per_group(int dtype, bool ta, bool tb, int cmode, int64_t m, int64_t k, int64_t n, int64_t lda, int64_t ldb, int64_t ldc, int64_t batch, int64_t groups,
+                          const void* A, int64_t a_group, int64_t a_image, const void* B, int64_t b_group, int64_t b_image, void* C, void* stream) {
+    const int64_t es = ntg::elem_size(dtype), c_item = m * ldc;
+    if (groups > 1 && !is_valu_dtype(dtype) && m > 0 && n > 0 && k > 0 && batch > 0) {
+        const int rc = check_sizes(m, k, n, batch);
+        if (rc) return rc;
+        ntg::GemmParams p;
+        std::memset(&p, 0, sizeof p);
+        p.M = (int)m; p.K = (int)k; p.N = (int)n;
+        p.A = A; p.B = B; p.C = C;
+        p.lda = lda; p.ldb = ldb; p.ldc = ldc;
+        p.cmode = cmode;
+        int status = NTG_OK;
+        const hipError_t e = launch_groups(p, dtype, batch, groups, {a_group, a_image, b_group, b_image, c_item}, [&](const ntg::GemmParams& q) {
+            status = launch_gemm(q, dtype, ta, tb, static_cast<hipStream_t>(stream));
+            return status == NTG_OK ? hipSuccess : hipErrorUnknown;
+        });
+        return e == hipSuccess ? NTG_OK : status;
+    }
+    for (int64_t g = 0; g < groups; ++g) {
+        ntg_gemm_desc d;
+        std::memset(&d, 0, sizeof d);
+        d.dtype = dtype; d.transpose_a = ta; d.transpose_b = tb; d.c_mode = cmode;
+        d.m = m; d.k = k; d.n = n;
+        d.lda = lda; d.ldb = ldb; d.ldc = ldc; d.batches = batch;
+        d.stride_a = a_image; d.stride_b = b_image; d.stride_c = groups * c_item;
+        const int rc = ntg_gemm_dev(&d, static_cast<const char*>(A) + g * a_group * es, static_cast<const char*>(B) + g * b_group * es,
+                                    static_cast<char*>(C) + g * c_item * es, stream);
+        if (rc) return rc;
+    }
+    return NTG_OK;
+}
+
 // out_b[g*og:(g+1)*og, L] = W_g[og, add] . col_b[g*add:(g+1)*add, L] with col_b gathered from the image by the B loader.
 // The reference forms (col_b^T . W_g^T) and swaps rows/columns afterwards (conv.cpp:94, :143); each output element is the
 // same ascending-k sum of the same products.
@@ -1288,21 +1354,17 @@ static int conv_forward_gather(int dtype, const void* image, const void* kernel,
                                int64_t out_channels, const Geo3& g, int64_t groups, hipStream_t hs) {
     const int64_t es = ntg::elem_size(dtype), cg = channels / groups, og = out_channels / groups;
     const int64_t L = g.L(), add = cg * g.taps(), vol = g.vol();
-    for (int64_t gi = 0; gi < groups; ++gi) {
-        ntg::GemmParams p;
-        std::memset(&p, 0, sizeof p);
-        p.M = (int)og; p.K = (int)add; p.N = (int)L; p.batch = (int)batch;
-        p.A = static_cast<const char*>(kernel) + gi * og * add * es;
-        p.B = static_cast<const char*>(image) + gi * cg * vol * es;
-        p.C = static_cast<char*>(out) + gi * og * L * es;
-        p.lda = add; p.ldb = L; p.ldc = L;
-        p.sA = 0; p.sB = channels * vol; p.sC = out_channels * L;
-        p.cmode = ntg::C_OVERWRITE;
-        p.vecA_ok = (add * es) % 16 == 0;
-        fill_conv_geom(p.conv, cg, g);
-        hipError_t e = ntg::launch_conv_mfma(dtype, false, g.nd, p, hs);
-        if (e != hipSuccess) return hip_fail(e, "implicit convolution launch");
-    }
+    ntg::GemmParams p;
+    std::memset(&p, 0, sizeof p);
+    p.M = (int)og; p.K = (int)add; p.N = (int)L;
+    p.A = kernel; p.B = image; p.C = out;
+    p.lda = add; p.ldb = L; p.ldc = L;
+    p.cmode = ntg::C_OVERWRITE;
+    p.vecA_ok = (add * es) % 16 == 0;
+    fill_conv_geom(p.conv, cg, g);
+    const hipError_t e = launch_groups(p, dtype, batch, groups, {og * add, 0, cg * vol, channels * vol, og * L},
+                                       [&](const ntg::GemmParams& q) { return ntg::launch_conv_mfma(dtype, false, g.nd, q, hs); });
+    if (e != hipSuccess) return hip_fail(e, "implicit convolution launch");
     return NTG_OK;
 }
 
@@ -1322,20 +1384,8 @@ static bool conv_pointwise_ok(int dtype, int64_t channels, int64_t groups, const
 }
 static int conv_forward_pointwise(int dtype, const void* image, const void* kernel, void* out, int64_t batch, int64_t channels,
                                   int64_t out_channels, const Geo3& g, int64_t groups, void* stream) {
-    const int64_t es = ntg::elem_size(dtype), cg = channels / groups, og = out_channels / groups, L = g.L();
-    for (int64_t gi = 0; gi < groups; ++gi) {
-        ntg_gemm_desc d;
-        std::memset(&d, 0, sizeof d);
-        d.dtype = dtype; d.c_mode = NTG_C_OVERWRITE;
-        d.m = og; d.k = cg; d.n = L;
-        d.lda = cg; d.ldb = L; d.ldc = L;
-        d.batches = batch;
-        d.stride_a = 0; d.stride_b = channels * L; d.stride_c = out_channels * L;
-        int rc = ntg_gemm_dev(&d, static_cast<const char*>(kernel) + gi * og * cg * es, static_cast<const char*>(image) + gi * cg * L * es,
-                              static_cast<char*>(out) + gi * og * L * es, stream);
-        if (rc) return rc;
-    }
-    return NTG_OK;
+    const int64_t cg = channels / groups, og = out_channels / groups, L = g.L();
+    return gemm_per_group(dtype, false, false, NTG_C_OVERWRITE, og, cg, L, cg, L, L, batch, groups, kernel, og * cg, 0, image, cg * L, channels * L, out, stream);
 }
 
 // Channels-last form of the same convolution, for the floating dtypes up to 32 bits: the image is first copied to
@@ -1445,25 +1495,20 @@ static int conv_forward_nhwc(int dtype, const void* image, const void* kernel, v
     if (mt) e = ntg::launch_weights_channels_last_rows(es, kernel, ws_w, out_channels, cg, cgp, g.k[1], g.k[2], mt->kq_pad, hs);
     else if (!took_along) e = ntg::launch_weights_channels_last(es, kernel, ws_w, out_channels, cg, cgp, taps, hs, wchunk);
     if (e != hipSuccess) return hip_fail(e, "weight permutation launch");
-    for (int64_t gi = 0; gi < groups; ++gi) {
-        ntg::GemmParams p;
-        std::memset(&p, 0, sizeof p);
-        p.M = (int)og; p.K = (int)K; p.N = (int)L; p.batch = (int)batch;
-        p.A = ws_w + gi * og * K * es;
-        p.B = ws_img + gi * cgp * es;
-        p.C = static_cast<char*>(out) + gi * og * L * es;
-        p.lda = K; p.ldb = chp; p.ldc = L;
-        p.sA = 0; p.sB = chp * volp; p.sC = out_channels * L;
-        p.cmode = ntg::C_OVERWRITE;
-        p.vecA_ok = 1; p.vecB_ok = 1;
-        fill_conv_geom(p.conv, cgp, halo.gp);
-        p.conv.chan = (int)chp;                    // elements from one pixel to the next
-        p.conv.halo = halo.on ? 1 : 0;
-        p.conv.tap_inner = tap_inner ? 1 : 0;
-        if (mt) { p.conv.tap_step = (int)mt->T; p.conv.kq_pad = (int)mt->kq_pad; }
-        e = ntg::launch_conv_nhwc(dtype, p, hs);
-        if (e != hipSuccess) return hip_fail(e, "channels-last convolution launch");
-    }
+    ntg::GemmParams p;
+    std::memset(&p, 0, sizeof p);
+    p.M = (int)og; p.K = (int)K; p.N = (int)L;
+    p.A = ws_w; p.B = ws_img; p.C = out;
+    p.lda = K; p.ldb = chp; p.ldc = L;
+    p.cmode = ntg::C_OVERWRITE;
+    p.vecA_ok = 1; p.vecB_ok = 1;
+    fill_conv_geom(p.conv, cgp, halo.gp);
+    p.conv.chan = (int)chp;                        // elements from one pixel to the next
+    p.conv.halo = halo.on ? 1 : 0;
+    p.conv.tap_inner = tap_inner ? 1 : 0;
+    if (mt) { p.conv.tap_step = (int)mt->T; p.conv.kq_pad = (int)mt->kq_pad; }
+    e = launch_groups(p, dtype, batch, groups, {og * K, 0, cgp, chp * volp, og * L}, [&](const ntg::GemmParams& q) { return ntg::launch_conv_nhwc(dtype, q, hs); });
+    if (e != hipSuccess) return hip_fail(e, "channels-last convolution launch");
     return NTG_OK;
 }
 
@@ -1474,22 +1519,18 @@ static int conv_dkernel_gather(int dtype, const void* image, const void* grad_ou
                                int64_t channels, int64_t out_channels, const Geo3& g, int64_t groups, int accumulate, hipStream_t hs) {
     const int64_t es = ntg::elem_size(dtype), cg = channels / groups, og = out_channels / groups;
     const int64_t L = g.L(), add = cg * g.taps(), vol = g.vol();
-    for (int64_t gi = 0; gi < groups; ++gi) {
-        ntg::GemmParams p;
-        std::memset(&p, 0, sizeof p);
-        p.M = (int)og; p.K = (int)L; p.N = (int)add; p.batch = (int)batch;
-        p.A = static_cast<const char*>(grad_out) + gi * og * L * es;
-        p.B = static_cast<const char*>(image) + gi * cg * vol * es;
-        p.C = static_cast<char*>(ws) + gi * og * add * es;
-        p.lda = L; p.ldb = L; p.ldc = add;
-        p.sA = out_channels * L; p.sB = channels * vol; p.sC = out_channels * add;
-        p.cmode = ntg::C_OVERWRITE;
-        p.vecA_ok = (L * es) % 16 == 0 && (p.sA * es) % 16 == 0;
-        fill_conv_geom(p.conv, cg, g);
-        hipError_t e = ntg::launch_conv_mfma(dtype, true, g.nd, p, hs);
-        if (e != hipSuccess) return hip_fail(e, "implicit conv_dkernel launch");
-    }
-    hipError_t e = ntg::launch_reduce_batch(dtype, ws, d_kernel, batch, out_channels * add, accumulate, hs);
+    ntg::GemmParams p;
+    std::memset(&p, 0, sizeof p);
+    p.M = (int)og; p.K = (int)L; p.N = (int)add;
+    p.A = grad_out; p.B = image; p.C = ws;
+    p.lda = L; p.ldb = L; p.ldc = add;
+    p.cmode = ntg::C_OVERWRITE;
+    p.vecA_ok = (L * es) % 16 == 0 && (out_channels * L * es) % 16 == 0;
+    fill_conv_geom(p.conv, cg, g);
+    hipError_t e = launch_groups(p, dtype, batch, groups, {og * L, out_channels * L, cg * vol, channels * vol, og * add},
+                                 [&](const ntg::GemmParams& q) { return ntg::launch_conv_mfma(dtype, true, g.nd, q, hs); });
+    if (e != hipSuccess) return hip_fail(e, "implicit conv_dkernel launch");
+    e = ntg::launch_reduce_batch(dtype, ws, d_kernel, batch, out_channels * add, accumulate, hs);
     if (e != hipSuccess) return hip_fail(e, "weight gradient reduction launch");
     return NTG_OK;
 }
@@ -1504,21 +1545,17 @@ static int conv_dimage_gather(int dtype, const void* kernel, const void* grad_ou
     hipError_t e = ntg::launch_flip_weights(es, kernel, ws, groups, og, cg, taps, hs);
     if (e != hipSuccess) return hip_fail(e, "weight flip launch");
     const Geo3 t = geo_dimage(g);
-    for (int64_t gi = 0; gi < groups; ++gi) {
-        ntg::GemmParams p;
-        std::memset(&p, 0, sizeof p);
-        p.M = (int)cg; p.K = (int)(og * taps); p.N = (int)vol; p.batch = (int)batch;
-        p.A = static_cast<const char*>(ws) + gi * cg * og * taps * es;
-        p.B = static_cast<const char*>(grad_out) + gi * og * L * es;
-        p.C = static_cast<char*>(d_image) + gi * cg * vol * es;
-        p.lda = og * taps; p.ldb = vol; p.ldc = vol;
-        p.sA = 0; p.sB = out_channels * L; p.sC = channels * vol;
-        p.cmode = accumulate ? ntg::C_ACCUMULATE : ntg::C_OVERWRITE;
-        p.vecA_ok = (og * taps * es) % 16 == 0;
-        fill_conv_geom(p.conv, og, t);
-        e = ntg::launch_conv_mfma(dtype, false, g.nd, p, hs);
-        if (e != hipSuccess) return hip_fail(e, "implicit conv_dimage launch");
-    }
+    ntg::GemmParams p;
+    std::memset(&p, 0, sizeof p);
+    p.M = (int)cg; p.K = (int)(og * taps); p.N = (int)vol;
+    p.A = ws; p.B = grad_out; p.C = d_image;
+    p.lda = og * taps; p.ldb = vol; p.ldc = vol;
+    p.cmode = accumulate ? ntg::C_ACCUMULATE : ntg::C_OVERWRITE;
+    p.vecA_ok = (og * taps * es) % 16 == 0;
+    fill_conv_geom(p.conv, og, t);
+    e = launch_groups(p, dtype, batch, groups, {cg * og * taps, 0, og * L, out_channels * L, cg * vol},
+                      [&](const ntg::GemmParams& q) { return ntg::launch_conv_mfma(dtype, false, g.nd, q, hs); });
+    if (e != hipSuccess) return hip_fail(e, "implicit conv_dimage launch");
     return NTG_OK;
 }
 
@@ -1554,24 +1591,19 @@ static int conv_dimage_nhwc(int dtype, const void* kernel, const void* grad_out,
     }
     if (!took_along) e = ntg::launch_flip_weights_channels_last(es, kernel, ws_w, groups, og, ogp, cg, taps, hs, wchunk);
     if (e != hipSuccess) return hip_fail(e, "weight flip launch");
-    for (int64_t gi = 0; gi < groups; ++gi) {
-        ntg::GemmParams p;
-        std::memset(&p, 0, sizeof p);
-        p.M = (int)cg; p.K = (int)K; p.N = (int)vol; p.batch = (int)batch;
-        p.A = ws_w + gi * cg * K * es;
-        p.B = ws_gy + gi * ogp * es;
-        p.C = static_cast<char*>(d_image) + gi * cg * vol * es;
-        p.lda = K; p.ldb = ochp; p.ldc = vol;
-        p.sA = 0; p.sB = ochp * Lp; p.sC = channels * vol;
-        p.cmode = accumulate ? ntg::C_ACCUMULATE : ntg::C_OVERWRITE;
-        p.vecA_ok = 1; p.vecB_ok = 1;
-        fill_conv_geom(p.conv, ogp, halo.gp);
-        p.conv.chan = (int)ochp;
-        p.conv.halo = halo.on ? 1 : 0;
-        p.conv.tap_inner = tap_inner ? 1 : 0;
-        e = ntg::launch_conv_nhwc(dtype, p, hs);
-        if (e != hipSuccess) return hip_fail(e, "channels-last conv_dimage launch");
-    }
+    ntg::GemmParams p;
+    std::memset(&p, 0, sizeof p);
+    p.M = (int)cg; p.K = (int)K; p.N = (int)vol;
+    p.A = ws_w; p.B = ws_gy; p.C = d_image;
+    p.lda = K; p.ldb = ochp; p.ldc = vol;
+    p.cmode = accumulate ? ntg::C_ACCUMULATE : ntg::C_OVERWRITE;
+    p.vecA_ok = 1; p.vecB_ok = 1;
+    fill_conv_geom(p.conv, ogp, halo.gp);
+    p.conv.chan = (int)ochp;
+    p.conv.halo = halo.on ? 1 : 0;
+    p.conv.tap_inner = tap_inner ? 1 : 0;
+    e = launch_groups(p, dtype, batch, groups, {cg * K, 0, ogp, ochp * Lp, cg * vol}, [&](const ntg::GemmParams& q) { return ntg::launch_conv_nhwc(dtype, q, hs); });
+    if (e != hipSuccess) return hip_fail(e, "channels-last conv_dimage launch");
     return NTG_OK;
 }
 
@@ -1804,9 +1836,8 @@ static DkernelPlan plan_dkernel(int dtype, int64_t batch, int64_t channels, int6
         const int64_t shortest = std::min<int64_t>(8, std::max<int64_t>(2, (L + bk - 1) / bk));
         double best = 0.0;
         const auto consider = [&](bool copy, int64_t ranges, int64_t items, int64_t kr, int edge) {
-            const int64_t tiles = ((og + edge - 1) / edge) * ((N + edge - 1) / edge) * items;
-            // (the groups' launches run one behind the other)
-            const double us = (copy ? 4.0 + 2.0 * (double)(total * out_channels * es) / 4.5e6 : 0.0) + groups * dkernel_cost_us(es, edge, tiles, kr) + 4.0 +
+            const int64_t tiles = ((og + edge - 1) / edge) * ((N + edge - 1) / edge) * items * groups;
+            const double us = (copy ? 4.0 + 2.0 * (double)(total * out_channels * es) / 4.5e6 : 0.0) + dkernel_cost_us(es, edge, tiles, kr) + 4.0 +
                               2.0 * (double)(items * out_channels * N * 4) / 4.0e6;
             if (pl.edge && us >= best) return;
             best = us;
@@ -1851,46 +1882,37 @@ static int conv_dkernel_nhwc(int dtype, const DkernelPlan& pl, const void* image
     if (e == hipSuccess && halo.on && volp != vol && !took_along) e = ntg::launch_halo_zero(es, ws_img, batch, chp, halo.hm, hs);
     if (e == hipSuccess && pl.copy_dy) e = ntg::launch_nchw_to_nhwc(es, grad_out, ws_gy, batch, out_channels, L, hs);
     if (e != hipSuccess) return hip_fail(e, "channels-last copy launch");
-    for (int64_t gi = 0; gi < groups; ++gi) {
-        ntg::GemmParams p;
-        std::memset(&p, 0, sizeof p);
-        p.M = (int)og; p.K = (int)(pl.ranges ? pl.kr : L); p.N = (int)N; p.batch = (int)pl.items;
-        if (pl.copy_dy) {
-            p.A = ws_gy + gi * og * es;
-            p.lda = out_channels;
-            p.sA = pl.kr * out_channels;
-        } else {
-            p.A = static_cast<const char*>(grad_out) + gi * og * L * es;
-            p.lda = L;
-            p.sA = pl.ranges ? 0 : out_channels * L;
+    ntg::GemmParams p;
+    std::memset(&p, 0, sizeof p);
+    p.M = (int)og; p.K = (int)(pl.ranges ? pl.kr : L); p.N = (int)N;
+    p.A = pl.copy_dy ? static_cast<const void*>(ws_gy) : grad_out;
+    p.lda = pl.copy_dy ? out_channels : L;
+    p.B = ws_img; p.C = ws_part;
+    p.ldb = chp; p.ldc = N;
+    const int64_t a_item = pl.copy_dy ? pl.kr * out_channels : pl.ranges ? 0 : out_channels * L;     // (a range: or an image)
+    p.cmode = ntg::C_PARTIAL;
+    p.vecA_ok = 1; p.vecB_ok = 1;
+    fill_conv_geom(p.conv, cgp, halo.gp);
+    p.conv.chan = (int)chp;                        // elements from one pixel to the next
+    p.conv.halo = halo.on ? 1 : 0;
+    if (halo.on && g.nd == 2 && L < (1 << 20) && (pl.ranges == 0 || L % bk == 0)) p.conv.pix_table = (int)L;     // (a K-step inside one image: see the kernel)
+    p.conv.tile_edge = pl.edge;
+    p.conv.k_segment = chain_steps(L);
+    if (pl.ranges) {
+        p.conv.k_ranges = 1;
+        p.conv.k_total = (int)(batch * L);
+        p.conv.fold_L = (int)L;
+        p.conv.div_fold = ntg::make_fastdiv((uint32_t)L);
+        p.conv.fold_stride = chp * volp;
+        if (!pl.copy_dy) {
+            p.conv.a_steps = (int)(L / bk);
+            p.conv.div_a_steps = ntg::make_fastdiv((uint32_t)(L / bk));
+            p.conv.a_image_stride = out_channels * L;
         }
-        p.B = ws_img + gi * cgp * es;
-        p.C = ws_part + gi * og * N * 4;
-        p.ldb = chp; p.ldc = N;
-        p.sB = pl.ranges ? 0 : chp * volp; p.sC = out_channels * N;
-        p.cmode = ntg::C_PARTIAL;
-        p.vecA_ok = 1; p.vecB_ok = 1;
-        fill_conv_geom(p.conv, cgp, halo.gp);
-        p.conv.chan = (int)chp;                    // elements from one pixel to the next
-        p.conv.halo = halo.on ? 1 : 0;
-        if (halo.on && g.nd == 2 && L < (1 << 20) && (pl.ranges == 0 || L % bk == 0)) p.conv.pix_table = (int)L;     // (a K-step inside one image: see the kernel)
-        p.conv.tile_edge = pl.edge;
-        p.conv.k_segment = chain_steps(L);
-        if (pl.ranges) {
-            p.conv.k_ranges = 1;
-            p.conv.k_total = (int)(batch * L);
-            p.conv.fold_L = (int)L;
-            p.conv.div_fold = ntg::make_fastdiv((uint32_t)L);
-            p.conv.fold_stride = chp * volp;
-            if (!pl.copy_dy) {
-                p.conv.a_steps = (int)(L / bk);
-                p.conv.div_a_steps = ntg::make_fastdiv((uint32_t)(L / bk));
-                p.conv.a_image_stride = out_channels * L;
-            }
-        }
-        e = ntg::launch_conv_nhwc_dw(dtype, pl.copy_dy, p, hs);
-        if (e != hipSuccess) return hip_fail(e, "channels-last conv_dkernel launch");
     }
+    e = launch_groups(p, dtype, pl.items, groups, {pl.copy_dy ? og : og * L, a_item, cgp, pl.ranges ? 0 : chp * volp, og * N},
+                      [&](const ntg::GemmParams& q) { return ntg::launch_conv_nhwc_dw(dtype, pl.copy_dy, q, hs); });
+    if (e != hipSuccess) return hip_fail(e, "channels-last conv_dkernel launch");
     // (groups are consecutive row blocks of both layouts, so one pass covers them all)
     e = ntg::launch_reduce_batch_taps_last(dtype, ws_part, d_kernel, pl.items, out_channels, cg, cgp, taps, accumulate, hs);
     if (e != hipSuccess) return hip_fail(e, "weight gradient reduction launch");
@@ -2218,20 +2240,14 @@ static int conv2d_backward_dev_impl(int dtype, const void* image, const void* ke
         ((reinterpret_cast<uintptr_t>(image) | reinterpret_cast<uintptr_t>(kernel) | reinterpret_cast<uintptr_t>(grad_out) |
           reinterpret_cast<uintptr_t>(d_image) | reinterpret_cast<uintptr_t>(d_kernel) | reinterpret_cast<uintptr_t>(ws)) & 15) == 0) {
         const int64_t cg = channels / groups;
-        for (int64_t g = 0; g < groups && d_image; ++g) {
-            std::memset(&d, 0, sizeof d);
-            d.dtype = dtype; d.transpose_a = 1; d.c_mode = accumulate ? NTG_C_ACCUMULATE : NTG_C_OVERWRITE;
-            d.m = cg; d.k = og; d.n = L; d.batches = batch;
-            d.stride_a = 0; d.stride_b = out_channels * L; d.stride_c = channels * L;
-            rc = ntg_gemm_dev(&d, kern + g * og * cg * es, gy + g * og * L * es, static_cast<char*>(d_image) + g * cg * L * es, stream);
+        if (d_image) {
+            rc = gemm_per_group(dtype, true, false, accumulate ? NTG_C_ACCUMULATE : NTG_C_OVERWRITE, cg, og, L, cg, L, L, batch, groups, kern, og * cg, 0,
+                                gy, og * L, out_channels * L, d_image, stream);
             if (rc) return rc;
         }
-        for (int64_t g = 0; g < groups && d_kernel; ++g) {
-            std::memset(&d, 0, sizeof d);
-            d.dtype = dtype; d.transpose_b = 1; d.c_mode = NTG_C_OVERWRITE;
-            d.m = og; d.k = L; d.n = cg; d.batches = batch;
-            d.stride_a = out_channels * L; d.stride_b = channels * L; d.stride_c = out_channels * cg;
-            rc = ntg_gemm_dev(&d, gy + g * og * L * es, static_cast<const char*>(image) + g * cg * L * es, ws + g * og * cg * es, stream);
+        if (d_kernel) {
+            rc = gemm_per_group(dtype, false, true, NTG_C_OVERWRITE, og, L, cg, L, L, cg, batch, groups, gy, og * L, out_channels * L,
+                                image, cg * L, channels * L, ws, stream);
             if (rc) return rc;
         }
         if (d_kernel) {
@@ -2276,15 +2292,9 @@ static int conv2d_backward_dev_impl(int dtype, const void* image, const void* ke
             hipError_t e = ntg::launch_nchw_to_nhwc(es, kern, ws + plan.wt_offset, groups, og, add, hs);
             if (e != hipSuccess) return hip_fail(e, "transposed weights launch");
         }
-        for (int64_t g = 0; g < groups; ++g) {
-            std::memset(&d, 0, sizeof d);
-            d.dtype = dtype; d.transpose_a = wt ? 0 : 1; d.c_mode = NTG_C_OVERWRITE;
-            d.m = add; d.k = og; d.n = L;
-            d.lda = wt ? og : add; d.ldb = L; d.ldc = L; d.batches = batch;
-            d.stride_a = 0; d.stride_b = out_channels * L; d.stride_c = ckk * L;
-            rc = ntg_gemm_dev(&d, (wt ? ws + plan.wt_offset : kern) + g * og * add * es, gy + g * og * L * es, ws + g * add * L * es, stream);
-            if (rc) return rc;
-        }
+        rc = gemm_per_group(dtype, !wt, false, NTG_C_OVERWRITE, add, og, L, wt ? og : add, L, L, batch, groups, wt ? ws + plan.wt_offset : kern, og * add, 0,
+                            gy, og * L, out_channels * L, ws, stream);
+        if (rc) return rc;
         rc = ntg_unfold2d_backward_dev(dtype, ws, d_image, batch, channels, height, width, k_r, k_c, s_r, s_c, p_r, p_c, d_r, d_c,
                                        accumulate, stream);
         if (rc) return rc;
@@ -2679,15 +2689,8 @@ static int convnd_backward_dev_impl(int dtype, const void* image, const void* ke
         if (rc) return rc;
     }
     if (d_image) {
-        for (int64_t g = 0; g < groups; ++g) {
-            std::memset(&d, 0, sizeof d);
-            d.dtype = dtype; d.transpose_a = 1; d.c_mode = NTG_C_OVERWRITE;
-            d.m = add; d.k = og; d.n = L;
-            d.lda = add; d.ldb = L; d.ldc = L; d.batches = batch;
-            d.stride_a = 0; d.stride_b = out_channels * L; d.stride_c = u.ccol * L;
-            rc = ntg_gemm_dev(&d, kern + g * og * add * es, gy + g * og * L * es, ws + g * add * L * es, stream);
-            if (rc) return rc;
-        }
+        rc = gemm_per_group(dtype, true, false, NTG_C_OVERWRITE, add, og, L, add, L, L, batch, groups, kern, og * add, 0, gy, og * L, out_channels * L, ws, stream);
+        if (rc) return rc;
         hipError_t e = ntg::launch_col2imnd(dtype, ws, d_image, u, accumulate, static_cast<hipStream_t>(stream));
         if (e != hipSuccess) return hip_fail(e, "col2imnd launch");
     }

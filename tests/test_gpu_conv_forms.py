@@ -1,0 +1,81 @@
+"""The forms a convolution is computed in on the device, each against the sums in 64 bits: groups as items of one launch.
+
+The bound: an output of n products is rounded once to its type (unit roundoff u; Float16 below 2^-14: 2^-25) after a sum in 32 bits whose error
+is at most n 2^-24 times the sum of the products' magnitudes.  Where parts of the sum are stored in the type on the way (the entries of a col
+matrix, the products per image of a layer of one tap) each is rounded too: u times those magnitudes more."""
+import pytest
+import torch
+
+from neurotensor_amd import functional as F
+
+pytestmark = pytest.mark.gpu
+
+UNIT = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -24}
+CONV = {1: torch.nn.functional.conv1d, 2: torch.nn.functional.conv2d, 3: torch.nn.functional.conv3d}
+TRANS = {1: torch.nn.functional.conv_transpose1d, 2: torch.nn.functional.conv_transpose2d, 3: torch.nn.functional.conv_transpose3d}
+OURS = {(1, False): (F.conv1d, F.conv1d_backward), (2, False): (F.conv2d, F.conv2d_backward), (3, False): (F.conv3d, F.conv3d_backward),
+        (1, True): (F.conv_transpose1d, F.conv_transpose1d_backward), (2, True): (F.conv_transpose2d, F.conv_transpose2d_backward),
+        (3, True): (F.conv_transpose3d, F.conv_transposend_backward)}
+
+
+def operands(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed, seed=1):
+    gen = torch.Generator().manual_seed(seed)
+    nd = len(size)
+    wshape = ((cin, cout // groups) if transposed else (cout, cin // groups)) + (kernel,) * nd
+    x = torch.randn((batch, cin) + size, generator=gen).to(dtype)
+    w = (torch.randn(wshape, generator=gen) * 0.2).to(dtype)
+    out = tuple((s - 1) * stride - 2 * pad + kernel if transposed else (s + 2 * pad - kernel) // stride + 1 for s in size)
+    return x, w, torch.randn((batch, cout) + out, generator=gen).to(dtype)
+
+
+def sums(x, w, dy, stride, pad, groups, transposed):
+    """(y, dx, dw) in float64 on the CPU."""
+    x, w = x.double().requires_grad_(), w.double().requires_grad_()
+    y = (TRANS if transposed else CONV)[x.dim() - 2](x, w, stride=stride, padding=pad, groups=groups)
+    dx, dw = torch.autograd.grad(y, (x, w), dy.double())
+    return y.detach(), dx, dw
+
+
+def check(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed, parts=()):
+    x, w, dy = operands(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed)
+    forward, backward = OURS[(len(size), transposed)]
+    opt = {"stride": stride, "padding": pad, "groups": groups}
+    dev = [t.cuda() for t in (x, w, dy)]
+    got = (forward(dev[0], dev[1], **opt),) + tuple(backward(*dev, **opt))
+    want = sums(x, w, dy, stride, pad, groups, transposed)
+    mags = sums(x.abs(), w.abs(), dy.abs(), stride, pad, groups, transposed)
+    taps = kernel ** len(size)
+    terms = (cin // groups * taps, cout // groups * taps, batch * dy[0, 0].numel() if not transposed else batch * x[0, 0].numel())
+    for name, g, r, m, n in zip(("y", "dx", "dw"), got, want, mags, terms):
+        assert g.shape == r.shape and g.dtype == dtype
+        bound = UNIT[dtype] * (r.abs() + (m if name in parts else 0.0)) + 2.0 ** -24 * (n + 32) * m + (2.0 ** -25 if dtype == torch.float16 else 0.0)
+        err = (g.double().cpu() - r).abs()
+        assert bool((err <= bound).all()), f"{name}: {float((err - bound).max())} over the bound"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("batch,cin,cout,size,kernel,stride,pad,groups,transposed,parts", [
+    (2, 64, 96, (13, 11), 3, 1, 1, 2, False, ()),        # channels-last, ragged pixels
+    (3, 128, 128, (17,), 5, 1, 2, 4, False, ()),
+    (2, 64, 64, (5, 6, 7), 3, 1, 1, 2, False, ()),
+    (3, 24, 32, (12, 12), 3, 2, 1, 4, False, ("dx",)),        # few channels a group: taps merged, image gradient through the col matrix
+    (2, 256, 144, (8, 8), 1, 1, 0, 4, False, ("dw",)),        # one tap: plain products
+    (5, 48, 48, (9, 9), 1, 1, 0, 3, False, ()),          # ... on rows that miss 16 bytes
+    (2, 64, 96, (6, 6), 4, 2, 1, 2, True, ()),
+    (2, 16, 16, (7, 5), 2, 2, 0, 4, True, ("y", "dw")),
+    (2, 30, 18, (10, 9), 3, 1, 1, 3, False, ("dw",)),         # element-wise gathers
+], ids=str)
+def test_groups_as_items_of_one_launch(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed, parts):
+    check(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed, parts)
+
+
+def test_a_batch_of_groups_split_in_two_launches_keeps_whole_images():
+    """One round of 256 x 256 tiles and a rest: the first launch takes whole images of all groups, each group with its own weights."""
+    batch, groups, c = 23, 3, 256
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn((batch, groups * c, 32, 32), generator=gen, device="cuda").to(torch.bfloat16)
+    w = (torch.randn((groups * c, c, 1, 1), generator=gen, device="cuda") * 0.1).to(torch.bfloat16)
+    y = F.conv2d(x, w, groups=groups)
+    for g in range(groups):
+        part = slice(g * c, (g + 1) * c)
+        assert torch.equal(y[:, part], F.conv2d(x[:, part].contiguous(), w[part].contiguous()))
