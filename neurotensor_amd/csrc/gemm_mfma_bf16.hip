@@ -19,6 +19,7 @@ hipError_t launch_conv_mfma_bf16(bool tb, int nd, const GemmParams& p, hipStream
     return tb ? launch_conv_cfg<DT_BF16, true, 2, 2, 2, 64>(p, s) : launch_conv_cfg<DT_BF16, false, 2, 2, 2, 64>(p, s);
 }
 hipError_t launch_conv_nhwc_bf16(const GemmParams& p, hipStream_t s) {
+    if (p.M <= 32) return ring16_flat_wide(p) ? launch_ring_nhwc_cfg<DT_BF16, 2, true>(p, s) : launch_ring_nhwc_cfg<DT_BF16, 1, true>(p, s);
     return launch_conv_nhwc16_planned(p, s, [&](int te, const GemmParams& q) {
         if (te == 256) return launch_ring_nhwc_cfg<DT_BF16, 4>(q, s);
         if (te == 64) return launch_ring_nhwc_cfg<DT_BF16, 1>(q, s);
@@ -28,6 +29,7 @@ hipError_t launch_conv_nhwc_bf16(const GemmParams& p, hipStream_t s) {
 hipError_t launch_conv_nhwc_items_bf16(int edge, const GemmParams& p, int64_t blocks, hipStream_t s) {
     if (edge == 256) return launch_ring_items_cfg<DT_BF16, 4>(p, blocks, s);
     if (edge == 64) return launch_ring_items_cfg<DT_BF16, 1>(p, blocks, s);
+    if (edge == 32) return launch_ring_items_cfg<DT_BF16, 1, true>(p, blocks, s);
     return launch_ring_items_cfg<DT_BF16, 2>(p, blocks, s);
 }
 hipError_t launch_conv_nhwc_dw_bf16(bool ta, const GemmParams& p, hipStream_t s) {

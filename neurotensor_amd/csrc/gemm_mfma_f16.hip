@@ -19,6 +19,7 @@ hipError_t launch_conv_mfma_f16(bool tb, int nd, const GemmParams& p, hipStream_
     return tb ? launch_conv_cfg<DT_F16, true, 2, 2, 2, 64>(p, s) : launch_conv_cfg<DT_F16, false, 2, 2, 2, 64>(p, s);
 }
 hipError_t launch_conv_nhwc_f16(const GemmParams& p, hipStream_t s) {
+    if (p.M <= 32) return ring16_flat_wide(p) ? launch_ring_nhwc_cfg<DT_F16, 2, true>(p, s) : launch_ring_nhwc_cfg<DT_F16, 1, true>(p, s);
     return launch_conv_nhwc16_planned(p, s, [&](int te, const GemmParams& q) {
         if (te == 256) return launch_ring_nhwc_cfg<DT_F16, 4>(q, s);
         if (te == 64) return launch_ring_nhwc_cfg<DT_F16, 1>(q, s);
@@ -28,6 +29,7 @@ hipError_t launch_conv_nhwc_f16(const GemmParams& p, hipStream_t s) {
 hipError_t launch_conv_nhwc_items_f16(int edge, const GemmParams& p, int64_t blocks, hipStream_t s) {
     if (edge == 256) return launch_ring_items_cfg<DT_F16, 4>(p, blocks, s);
     if (edge == 64) return launch_ring_items_cfg<DT_F16, 1>(p, blocks, s);
+    if (edge == 32) return launch_ring_items_cfg<DT_F16, 1, true>(p, blocks, s);
     return launch_ring_items_cfg<DT_F16, 2>(p, blocks, s);
 }
 hipError_t launch_conv_nhwc_dw_f16(bool ta, const GemmParams& p, hipStream_t s) {

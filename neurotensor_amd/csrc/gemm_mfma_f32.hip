@@ -7,9 +7,7 @@ namespace ntg {
 // times the tile's MFMA time; 64 x 64 tiles balance four times finer and lose about 7 % to their single
 // accumulator block per wavefront.
 static int ring_f32_tile_edge(const GemmParams& p) {
-    const int64_t t128 = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
-    const int64_t t64 = (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
-    const double cost128 = (double)((t128 + 255) / 256), cost64 = 1.07 * 0.25 * (double)((t64 + 255) / 256);
+    const double cost128 = ring_f32_cost(128, p.M, p.N, p.batch), cost64 = ring_f32_cost(64, p.M, p.N, p.batch);
     return cost64 < cost128 ? 64 : 128;
 }
 
@@ -275,9 +273,11 @@ hipError_t launch_conv_mfma_f32(bool tb, int nd, const GemmParams& p, hipStream_
     return nd == 3 ? launch_conv_nd_f32<3>(tb, p, s) : launch_conv_nd_f32<2>(tb, p, s);
 }
 hipError_t launch_conv_nhwc_f32(const GemmParams& p, hipStream_t s) {
-    return ring_f32_tile_edge(p) == 128 ? launch_ring_nhwc_cfg<DT_F32, 2>(p, s) : launch_ring_nhwc_cfg<DT_F32, 1>(p, s);
+    if (ring_f32_conv_edge(p.M, p.N, p.batch) == 32) return launch_ring_nhwc_cfg<DT_F32, 1, true>(p, s);
+    return ring_f32_conv_edge(p.M, p.N, p.batch) == 128 ? launch_ring_nhwc_cfg<DT_F32, 2>(p, s) : launch_ring_nhwc_cfg<DT_F32, 1>(p, s);
 }
 hipError_t launch_conv_nhwc_items_f32(int edge, const GemmParams& p, int64_t blocks, hipStream_t s) {
+    if (edge == 32) return launch_ring_items_cfg<DT_F32, 1, true>(p, blocks, s);
     return edge == 128 ? launch_ring_items_cfg<DT_F32, 2>(p, blocks, s) : launch_ring_items_cfg<DT_F32, 1>(p, blocks, s);
 }
 hipError_t launch_conv_nhwc_dw_f32(bool ta, const GemmParams& p, hipStream_t s) {

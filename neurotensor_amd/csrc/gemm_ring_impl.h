@@ -206,21 +206,24 @@ constexpr int dw_table_entries(int wb) { return wb == 4 ? 6144 : 3584; }
 // second set of sums (SEGMENTS below) and, unasked, takes a few registers more than two workgroups a CU can have.
 constexpr int ring_min_waves(int dt, int wb, int conv) { return dt == DT_F32 && wb == 2 && (conv == 4 || conv == 7) ? 2 : 0; }
 
-template <int DT, bool TA, bool TB, bool RAGGED, int WB_, int CONV = 0, int WBN_ = 0, int KD_ = 1>
-__global__ void __launch_bounds__(256, ring_min_waves(DT, WB_, CONV)) gemm_ring_kernel(const GemmParams pin) {
+// FLAT (gathering kernels, A stored [m][k]): the four wavefronts stand side by side, a tile is 32 rows x 128 WB_ columns.
+template <int DT, bool TA, bool TB, bool RAGGED, int WB_, int CONV = 0, int WBN_ = 0, int KD_ = 1, bool FLAT = false>
+__global__ void __launch_bounds__(256, ring_min_waves(DT, FLAT ? 1 : WB_, CONV)) gemm_ring_kernel(const GemmParams pin) {
     using E = Elem<DT>;
     using T = typename E::T;
     constexpr int ES = sizeof(T);
-    constexpr int WBM = WB_, WBN = WBN_ ? WBN_ : WB_;    // 32 x 32 blocks per wavefront along m / along n
-    constexpr int WB = WBN;                              // (the gathered operand is B; gathering kernels have square tiles)
-    static_assert(CONV == 0 || WBM == WBN, "gathering kernels have square tiles");
+    constexpr int WBM = FLAT ? 1 : WB_, WBN = WBN_ ? WBN_ : WB_;      // 32 x 32 blocks per wavefront along m / along n
+    constexpr int WB = FLAT ? 2 * WBN : WBN;             // DMA instructions per wavefront for 64 bytes of k of the B tile, whose 64 WB columns a gathering kernel fills
+    static_assert(CONV == 0 || FLAT || WBM == WBN, "gathering kernels have square tiles, or flat ones");
+    static_assert(!FLAT || ((CONV == 3 || CONV == 5 || CONV == 6 || CONV == 8) && !TA && WBN_ == 0 && KD_ == 1), "flat tiles: channels-last convolutions, A stored [m][k]");
     constexpr int KD = KD_;
     static_assert(KD == 1 || (KD == 2 && CONV == 0 && (ES == 2 || ES == 1) && WB_ == 2 && (WBN_ == 0 || WBN_ == 4)), "deep K-steps: 16- and 8-bit plain products on 128 x 128 and 128 x 256 tiles");
     constexpr bool RING3 = KD == 2 && WBN_ == 4;         // three stages of 48 KiB
-    using GA = RingGeom<WBM, ES, KD>;                    // geometry of the A tile
-    using G = RingGeom<WBN, ES, KD>;                     // geometry of the B tile
-    constexpr int A_TILE_BYTES = GA::TILE_BYTES, STAGE_BYTES = GA::TILE_BYTES + G::TILE_BYTES;
-    constexpr int WTM = GA::WT, WTN = G::WT;             // a wavefront's share of the tile: WTM rows x WTN columns
+    using GA = RingGeom<WBM, ES, KD>;                    // geometry of the A tile (flat: twice its rows)
+    using G = RingGeom<WB, ES, KD>;                      // geometry of the B tile
+    constexpr int BM = FLAT ? 32 : GA::BM;
+    constexpr int A_TILE_BYTES = BM * G::KB, STAGE_BYTES = A_TILE_BYTES + G::TILE_BYTES;
+    constexpr int WTM = 32 * WBM, WTN = 32 * WBN;        // a wavefront's share of the tile: WTM rows x WTN columns
     constexpr bool GATHER4 = CONV == 1 || CONV == 2;     // op(B) gathered element by element from an NCHW image
     constexpr bool ITEMS = CONV == 8;                    // several convolutions of one bordered image in one launch, each described by a RingItem
     constexpr bool GATHER16 = CONV == 3 || CONV == 5 || CONV == 6 || ITEMS;   // op(B) = col^T gathered in 16-byte pieces from a channels-last image
@@ -233,7 +236,7 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, WB_, CONV)) gemm_ring_
     static_assert(!GATHER4 || (ES == 4 && !TA && RAGGED), "gathered operands: Float32, A stored [m][k], guarded edges");
     static_assert(!GATHER16 || ((ES == 4 || ES == 2) && !TA && RAGGED), "channels-last gather: 16/32-bit floats, A stored [m][k], guarded edges");
     static_assert(!GATHERW || ((ES == 4 || ES == 2) && !TB && RAGGED), "channels-last weight gradient: 16/32-bit floats, guarded edges");
-    constexpr int NA = WBM * KD, NB = GATHER4 ? 4 * WB : WBN * KD;   // DMA instructions per wavefront and K-step for the A / B tile
+    constexpr int NA = WBM * KD, NB = GATHER4 ? 4 * WB : WB * KD;   // DMA instructions per wavefront and K-step for the A / B tile
     // B instructions issued in the first / second half-step (the second also carries the A tile's).  Splitting a gathered
     // tile between the two was measured slower than issuing all of it in the first.
     constexpr int NB1 = NB, NB2 = NB - NB1;
@@ -250,7 +253,7 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, WB_, CONV)) gemm_ring_
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wm = FLAT ? 0 : wave >> 1, wn = FLAT ? wave : wave & 1;
 
     int lid = pin.group_m < 0 ? (int)blockIdx.x : xcd_contiguous_id(blockIdx.x, gridDim.x);      // (group_m != 0: measurement only, see ring_tile_order_override)
     typename std::conditional<ITEMS, GemmParams, const GemmParams&>::type p = pin;
@@ -280,7 +283,7 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, WB_, CONV)) gemm_ring_
     const int b = lid / tiles;
     int tm, tn;
     tile_coords(lid - b * tiles, p.tiles_m, p.tiles_n, p.group_m > 0 ? p.group_m : p.group_m < 0 ? -p.group_m : 4, tm, tn);
-    const int m0 = tm * GA::BM, n0 = tn * G::BN;
+    const int m0 = tm * BM, n0 = tn * G::BN;
 
     // (pointer tables: one uniform load per operand; everything below is base + offset either way)
     const T* A = p.Aptr ? static_cast<const T*>(p.Aptr[b]) : static_cast<const T*>(p.A) + operand_offset(p, b, p.sA, p.sAk);
@@ -344,14 +347,17 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, WB_, CONV)) gemm_ring_
     const int KT = (K + BK - 1) / BK;
     const int last = KT - 1;
     const int kr = K - last * BK;                                    // k that exist in the last K-step (a multiple of one chunk, or the gathered operand is zero past it)
-    const int mvalid = p.M - m0 < GA::BM ? p.M - m0 : GA::BM;
+    const int mvalid = p.M - m0 < BM ? p.M - m0 : BM;
     const int nvalid = p.N - n0 < G::BN ? p.N - n0 : G::BN;
-    uint32_t offA[WBM * KD], offB[WBN * KD];      // K-steps before the last
-    uint32_t offAt[WBM * KD], offBt[WBN * KD];    // the last K-step (RAGGED: k clamped to what exists)
-    dma_offsets<A_KC, RAGGED, WBM, ES, KD>(offA, p.lda, wave, lane, mvalid, BK);
-    dma_offsets<B_KC, RAGGED, WBN, ES, KD>(offB, p.ldb, wave, lane, nvalid, BK);
-    dma_offsets<A_KC, RAGGED, WBM, ES, KD>(offAt, p.lda, wave, lane, mvalid, kr);
-    dma_offsets<B_KC, RAGGED, WBN, ES, KD>(offBt, p.ldb, wave, lane, nvalid, kr);
+    uint32_t offA[WBM * KD], offB[WB * KD];       // K-steps before the last
+    uint32_t offAt[WBM * KD], offBt[WB * KD];     // the last K-step (RAGGED: k clamped to what exists)
+    // (a flat tile's A is two instructions, which wavefronts 2 and 3 issue a second time: the same bytes to the same place, and every
+    //  wavefront counts the same loads)
+    const int wave_a = FLAT ? wave & 1 : wave, wave_a_u = FLAT ? wave_u & 1 : wave_u;
+    dma_offsets<A_KC, RAGGED, WBM, ES, KD>(offA, p.lda, wave_a, lane, mvalid, BK);
+    dma_offsets<B_KC, RAGGED, WB, ES, KD>(offB, p.ldb, wave, lane, nvalid, BK);
+    dma_offsets<A_KC, RAGGED, WBM, ES, KD>(offAt, p.lda, wave_a, lane, mvalid, kr);
+    dma_offsets<B_KC, RAGGED, WB, ES, KD>(offBt, p.ldb, wave, lane, nvalid, kr);
     const char* baseA = reinterpret_cast<const char*>(A) + (A_KC ? (int64_t)m0 * p.lda : (int64_t)m0) * ES;
     const char* baseB = reinterpret_cast<const char*>(B) + (B_KC ? (int64_t)n0 * p.ldb : (int64_t)n0) * ES;
     const int64_t advA = (A_KC ? (int64_t)BK : (int64_t)BK * p.lda) * ES;
@@ -805,7 +811,7 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, WB_, CONV)) gemm_ring_
 #pragma unroll
             for (int x = 0; x < WB; ++x) conv4_dma(x, lds_tile);
         }
-        else dma_tile<WBN * KD>(srcB(kt), kt >= last ? offBt : offB, lds_tile, wave_u);
+        else dma_tile<WB * KD>(srcB(kt), kt >= last ? offBt : offB, lds_tile, wave_u);
     };
     if constexpr (ES == 4 && std::is_same<AccS, float>::value) {
         if (p.cmode == C_ACCUMULATE || p.cmode == C_BIAS) {
@@ -818,9 +824,9 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, WB_, CONV)) gemm_ring_
                 for (int j = 0; j < WBN; ++j) asm volatile("" : "+v"(acc[i][j]));
         }
     }
-    dma_tile<NA>(srcA(0), 0 >= last ? offAt : offA, lds_addr_of(st0), wave_u);
+    dma_tile<NA>(srcA(0), 0 >= last ? offAt : offA, lds_addr_of(st0), wave_a_u);
     b_tile(0, lds_addr_of(st0) + A_TILE_BYTES);
-    dma_tile<NA>(srcA(1), 1 >= last ? offAt : offA, lds_addr_of(st1), wave_u);
+    dma_tile<NA>(srcA(1), 1 >= last ? offAt : offA, lds_addr_of(st1), wave_a_u);
     b_tile(1, lds_addr_of(st1) + A_TILE_BYTES);
     // instruction y (A's first, then B's) of this wavefront's share of tile kt, into the stage at lds_stage
     auto tile_dma = [&](int y, int kt, uint32_t lds_stage) __attribute__((always_inline)) {
@@ -832,9 +838,9 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, WB_, CONV)) gemm_ring_
 #pragma unroll
         for (int y = 0; y < (NA + NB) / 2; ++y) tile_dma(y, 2, lds_addr_of(st2));     // first half of tile 2
     } else {
-        dma_tile<NA>(srcA(2), 2 >= last ? offAt : offA, lds_addr_of(st2), wave_u);
+        dma_tile<NA>(srcA(2), 2 >= last ? offAt : offA, lds_addr_of(st2), wave_a_u);
         b_tile(2, lds_addr_of(st2) + A_TILE_BYTES);
-        if constexpr (KD == 1) dma_tile<NA>(srcA(3), 3 >= last ? offAt : offA, lds_addr_of(st3), wave_u);
+        if constexpr (KD == 1) dma_tile<NA>(srcA(3), 3 >= last ? offAt : offA, lds_addr_of(st3), wave_a_u);
     }
 
     constexpr int NBUF = 2 * KD;
@@ -959,7 +965,7 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, WB_, CONV)) gemm_ring_
             mma_step_prefetch(1, nxt, 0, 0, std::integral_constant<int, NB2 + NA>{}, std::integral_constant<int, NB2>{},
                               [&](int x) __attribute__((always_inline)) {
                 if (x < NB2) conv_dma(NB1 + x, lds_gather);       // rest of B(kt+3)
-                else dma_1k(src, (RAGGED && tail) ? offAt[x - NB2] : offA[x - NB2], lds_tile + (uint32_t)(wave_u * WBM + x - NB2) * 1024u);
+                else dma_1k(src, (RAGGED && tail) ? offAt[x - NB2] : offA[x - NB2], lds_tile + (uint32_t)(wave_a_u * WBM + x - NB2) * 1024u);
             });
         }
     };
@@ -1328,51 +1334,57 @@ static hipError_t launch_ring_conv_cfg(bool tb, const GemmParams& pin, hipStream
 }
 
 // ... from a channels-last image that carries its padding as zero pixels (CONV = 5; three spatial axes: 6)
-template <int DT, int WB>
+template <int DT, int WB, bool FLAT = false>
 static hipError_t launch_ring_nhwc_halo_cfg(const GemmParams& pin, hipStream_t s) {
-    constexpr int TE = RingGeom<WB, (int)sizeof(typename Elem<DT>::T)>::BM;
+    constexpr int TM = FLAT ? 32 : 64 * WB, TN = FLAT ? 128 * WB : 64 * WB;
     GemmParams p = pin;
-    p.tiles_m = (p.M + TE - 1) / TE;
-    p.tiles_n = (p.N + TE - 1) / TE;
+    p.tiles_m = (p.M + TM - 1) / TM;
+    p.tiles_n = (p.N + TN - 1) / TN;
     const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n * p.batch;
     if (blocks <= 0) return hipSuccess;
     if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    if (p.conv.k_d > 1 || p.conv.D > 1) hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 6>), dim3((unsigned)blocks), dim3(256), 0, s, p);
-    else hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 5>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+    if (p.conv.k_d > 1 || p.conv.D > 1) hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 6, 0, 1, FLAT>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 5, 0, 1, FLAT>), dim3((unsigned)blocks), dim3(256), 0, s, p);
     return hipGetLastError();
 }
 
 // several such convolutions in one launch (CONV = 8)
-template <int DT, int WB>
+template <int DT, int WB, bool FLAT = false>
 static hipError_t launch_ring_items_cfg(const GemmParams& pin, int64_t blocks, hipStream_t s) {
-    constexpr int TE = RingGeom<WB, (int)sizeof(typename Elem<DT>::T)>::BM;
+    constexpr int TM = FLAT ? 32 : 64 * WB;
     GemmParams p = pin;
-    p.tiles_m = (p.M + TE - 1) / TE;
+    p.tiles_m = (p.M + TM - 1) / TM;
     if (blocks <= 0) return hipSuccess;
     if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 8>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 8, 0, 1, FLAT>), dim3((unsigned)blocks), dim3(256), 0, s, p);
     return hipGetLastError();
 }
 
+// 16-bit convolutions of up to 32 rows take flat tiles: of square tiles half the rows or more would not exist.  us on 64 x 64 or 128 x 128 tiles |
+// 32 x 128 | 32 x 256, BFloat16: 64 x 192 x 64 x 64 -> 16 by 5 x 5 267 | 200 | 185, 4 x 64 x 32^3 -> 32 by 3 x 3 x 3 59 | 45 | 41, 4 x 32 x 128 x 128
+// -> 32 by 7 x 7 28 | 19 | 18, 16 x 16 x 64 x 64 -> 32 by 3 x 3 10.6 | 8.1 | 9.6, 2 x 32 x 28 x 28 -> 32 by 3 x 3 5.6 | 5.8 | 7.0: the wide one where there are
+// four of them for each CU or more.
+static inline bool ring16_flat_wide(const GemmParams& p) { return (int64_t)((p.N + 255) / 256) * p.batch >= 1024; }
+
 // convolution with op(B) gathered in 16-byte pieces from a channels-last image (see CONV = 3)
-template <int DT, int WB>
+template <int DT, int WB, bool FLAT = false>
 static hipError_t launch_ring_nhwc_cfg(const GemmParams& pin, hipStream_t s) {
-    if (pin.conv.halo) return launch_ring_nhwc_halo_cfg<DT, WB>(pin, s);
-    constexpr int TE = RingGeom<WB, (int)sizeof(typename Elem<DT>::T)>::BM;
+    if (pin.conv.halo) return launch_ring_nhwc_halo_cfg<DT, WB, FLAT>(pin, s);
+    constexpr int TM = FLAT ? 32 : 64 * WB, TN = FLAT ? 128 * WB : 64 * WB;
     GemmParams p = pin;
-    p.tiles_m = (p.M + TE - 1) / TE;
-    p.tiles_n = (p.N + TE - 1) / TE;
+    p.tiles_m = (p.M + TM - 1) / TM;
+    p.tiles_n = (p.N + TN - 1) / TN;
     const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n * p.batch;
     if (blocks <= 0) return hipSuccess;
     if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 3>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 3, 0, 1, FLAT>), dim3((unsigned)blocks), dim3(256), 0, s, p);
     return hipGetLastError();
 }
 
 // weight gradient of a convolution with op(B) gathered from a channels-last image (see CONV = 4 and 7)
 template <int DT, int WB, bool TA = false>
 static hipError_t launch_ring_nhwc_dw_cfg(const GemmParams& pin, hipStream_t s) {
-    constexpr int TE = RingGeom<WB, (int)sizeof(typename Elem<DT>::T)>::BM;
+    constexpr int TE = 64 * WB;
     GemmParams p = pin;
     p.tiles_m = (p.M + TE - 1) / TE;
     p.tiles_n = (p.N + TE - 1) / TE;

@@ -301,6 +301,19 @@ static inline Ring16Split ring16_split(int64_t M, int64_t N, int64_t K, int rect
     return sp;
 }
 
+// Float32 tiles by evenness: rounds over the CUs times a tile's time (128 x 128: 1).  A 64 x 64 tile takes 7 % more than its share of the
+// work; the flat tile of the channels-last convolutions, 32 rows x 128 columns (code 32), 17 %: 4 x 32 x 32^3 -> 64 by 3 x 3 x 3, whose image
+// gradient has 32 rows, 247 us on 64 x 64 tiles, half of them rows that do not exist, 144 on flat ones (the forward product, the same work on
+// whole 64 x 64 tiles: 132).
+static inline double ring_f32_cost(int t, int64_t M, int64_t N, int64_t batch) {
+    const int64_t r = t, c = t == 32 ? 128 : t, nt = ((M + r - 1) / r) * ((N + c - 1) / c) * batch;
+    return (t == 128 ? 1.0 : t == 64 ? 1.07 * 0.25 : 1.17 * 0.25) * (double)((nt + 255) / 256);
+}
+static inline int ring_f32_conv_edge(int64_t M, int64_t N, int64_t batch) {
+    const double c128 = ring_f32_cost(128, M, N, batch), c64 = ring_f32_cost(64, M, N, batch), c32 = ring_f32_cost(32, M, N, batch);
+    return c32 < c64 && c32 < c128 ? 32 : c64 < c128 ? 64 : 128;
+}
+
 static inline int64_t elem_size(int dt) {
     switch (dt) {
     case DT_I8: case DT_U8: return 1;

@@ -1700,20 +1700,17 @@ static PhasePlan plan_dimage_phases(int dtype, int64_t batch, int64_t channels, 
     if (q.phases == 0) return pp;
     // one tile for all items, as if they were equal
     const int64_t items = (int64_t)q.phases * groups;
-    if (es == 4) {
-        const int64_t t128 = ((cg + 127) / 128) * ((n_max + 127) / 128) * batch * items, t64 = ((cg + 63) / 64) * ((n_max + 63) / 64) * batch * items;
-        pp.edge = 1.07 * 0.25 * (double)((t64 + 255) / 256) < (double)((t128 + 255) / 256) ? 64 : 128;
-    } else {
-        pp.edge = ntg::ring16_tile_edge(cg, n_max, k_max, batch * items);
-    }
-    q.tile_rows = q.tile_cols = pp.edge;
+    if (es == 4) pp.edge = ntg::ring_f32_conv_edge(cg, n_max, batch * items);
+    else pp.edge = cg <= 32 ? 32 : ntg::ring16_tile_edge(cg, n_max, k_max, batch * items);      // (32: flat tiles)
+    q.tile_rows = pp.edge;
+    q.tile_cols = pp.edge == 32 ? 128 : pp.edge;
     const int64_t tiles_m = (cg + pp.edge - 1) / pp.edge;
     for (int e0 = 0; e0 < q.s[0]; ++e0)
         for (int e1 = 0; e1 < q.s[1]; ++e1)
             for (int e2 = 0; e2 < q.s[2]; ++e2) {
                 if (q.plane_off[(e0 * q.s[1] + e1) * q.s[2] + e2] < 0) continue;
                 const int64_t n = (int64_t)q.n[0][e0] * q.n[1][e1] * q.n[2][e2];
-                pp.blocks += tiles_m * ((n + pp.edge - 1) / pp.edge) * batch * groups;
+                pp.blocks += tiles_m * ((n + q.tile_cols - 1) / q.tile_cols) * batch * groups;
             }
     if (pp.blocks > 0x7fffffffLL) return pp;
     pp.gy_bytes = (int64_t)align_up((size_t)(batch * ochp * volp * es), 256);

@@ -79,3 +79,19 @@ def test_a_batch_of_groups_split_in_two_launches_keeps_whole_images():
     for g in range(groups):
         part = slice(g * c, (g + 1) * c)
         assert torch.equal(y[:, part], F.conv2d(x[:, part].contiguous(), w[part].contiguous()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("batch,cin,cout,size,kernel,stride,pad,groups,transposed", [
+    (1, 64, 1, (127,), 3, 1, 1, 1, False),           # 32 x 128 tiles: one row, one column short of a tile
+    (2, 32, 32, (129,), 5, 1, 2, 1, False),          # ... all rows, one column more
+    (3, 64, 33, (12, 12), 3, 1, 1, 1, False),        # one row too many
+    (2, 32, 24, (4, 5, 7), 3, 1, 1, 1, False),
+    (1040, 32, 31, (33,), 3, 1, 1, 1, False),        # 16 bits: 32 x 256 tiles
+    (2, 16, 96, (9, 10), 3, 2, 1, 1, False),         # image gradient by phases
+    (2, 64, 64, (16, 8), 4, 2, 1, 2, True),
+    (2, 20, 32, (4, 6, 6), 2, 2, 0, 1, False),
+    (2, 96, 96, (11, 12), 3, 1, 1, 1, False),        # Float32: three rows of flat tiles
+], ids=str)
+def test_flat_tiles(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed):
+    check(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed)
