@@ -1632,6 +1632,15 @@ struct PhasePlan {
     ntg::PhaseLayout lay;
     int64_t bytes() const { return gy_bytes + w_bytes + item_bytes + tmp_bytes; }
 };
+// Out channels of a group as the phases hold them, in whole 64-byte runs (0: not taken).  The alternative is the col matrix, which is ahead wherever
+// Float32 would have to pad (16 x 64 x 56 x 56 -> 24 by 3 x 3 at stride 2, a step: 83 us against 93 by phases; 4 x 32 x 24^3 -> 24 by 3 x 3 x 3 84 / 101)
+// except over three axes on images from 32 MiB on, the passes over col and image being the larger part there (9 x 256 x 29^3 -> 48 by one
+// tap in 2 groups 621 / 406, 42 x 256 x 24^3 -> 96 by 3 x 3 x 3 in 4 groups 3291 / 2571).
+static int64_t phase_padded_channels(int64_t es, int64_t og, int64_t batch, int64_t channels, const Geo3& g) {
+    const int64_t step = 64 / es, ogp = (og + step - 1) / step * step;
+    const int64_t most = es == 2 ? 4 : g.nd == 3 && batch * channels * g.vol() * es >= (1LL << 25) ? 2 : 1;
+    return og > 0 && ogp <= most * og ? ogp : 0;
+}
 static PhasePlan plan_dimage_phases(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
     PhasePlan pp;
     std::memset(&pp, 0, sizeof pp);
@@ -1640,7 +1649,7 @@ static PhasePlan plan_dimage_phases(int dtype, int64_t batch, int64_t channels, 
     for (int a = 0; a < 3; ++a)
         if (g.d[a] != 1 || g.s[a] > 4 || g.p[a] < 0 || g.sz[a] >= (1 << 24) || g.k[a] >= (1 << 16)) return pp;
     const int64_t es = ntg::elem_size(dtype), vel = 16 / es, og = out_channels / groups, cg = channels / groups;
-    const int64_t ogp = nhwc_padded_channels(es, og), ochp = groups * ogp;
+    const int64_t ogp = phase_padded_channels(es, og, batch, channels, g), ochp = groups * ogp;
     // (the interleaving pass counts image elements in 32 bits; one image's planes, whose pitches are 16-byte multiples, are indexed in 32 bits)
     if (ogp == 0 || batch * channels * g.vol() >= 0x7fffffffLL || channels * (g.vol() + 64 * vel) >= 0x7fffffffLL) return pp;
     // the image channels of a group are the rows of these products: with a handful of them (an RGB input layer) a 64-row

@@ -6,6 +6,8 @@
 // for stride 1, so are the loads.
 #include "ntg_common.h"
 
+#include <cstring>
+
 namespace ntg {
 
 // a 16-byte element that is only moved (Complex128)
@@ -264,6 +266,76 @@ __global__ void __launch_bounds__(256) col2imnd_kernel(const T* __restrict__ col
     }
 }
 
+// The undilated windows' gather over up to four axes (leading ones of size 1) in 32-bit arithmetic, like col2im_step_kernel: two divisions per axis for
+// the thread instead of three 64-bit ones per axis and tap, only the taps that exist, four loads in flight.  Bound by the reads of col.
+// Training steps that go through it, with the general kernel | with this one: Float32 42 x 256 x 24^3 -> 96 by 3 x 3 x 3 at stride 2 in 4 groups 29500 us |
+// 3290, BFloat16 2 x 16 x 20^3 transposed to 128 by 4 x 4 x 4 in 4 groups 7180 | 390, Float32 4 x 32 x 24^3 -> 8 by 3 x 3 x 3 at stride 2 409 | 86.
+struct Col2imNdStep {
+    int size[4], k[4], s[4], p[4], o[4];
+    FastDiv div_size[4], div_s[4], div_c;
+    int channels;
+    uint32_t total;
+    int64_t col_image, col_channel, step[4], tap[4], out[4];      // elements of col from a tap, an output position or the next pair of both to the next along an axis
+};
+template <class T, class Acc>
+__global__ void __launch_bounds__(256) col2imnd_step_kernel(const T* __restrict__ col, T* __restrict__ im, const Col2imNdStep u, const int accumulate) {
+    const uint32_t idx = blockIdx.x * 256u + threadIdx.x;
+    if (idx >= u.total) return;
+    uint32_t r = idx;
+    int lo[4], hi[4];
+    int64_t off = 0;
+#pragma unroll
+    for (int a = 3; a >= 0; --a) {
+        const uint32_t q = fast_div(r, u.div_size[a]), P = r - q * (uint32_t)u.size[a] + (uint32_t)u.p[a];
+        r = q;
+        const int h0 = (int)fast_div(P, u.div_s[a]), i0 = (int)P - h0 * u.s[a];
+        // tap i0 + s m reads output position h0 - m: inside the outputs and the kernel
+        lo[a] = h0 >= u.o[a] ? h0 - u.o[a] + 1 : 0;
+        hi[a] = i0 < u.k[a] ? (int)fast_div((uint32_t)(u.k[a] - 1 - i0), u.div_s[a]) : -1;
+        hi[a] = hi[a] > h0 ? h0 : hi[a];
+        off += (int64_t)i0 * u.tap[a] + (int64_t)h0 * u.out[a];
+    }
+    const uint32_t b = fast_div(r, u.div_c), c = r - b * (uint32_t)u.channels;
+    const T* base = col + (int64_t)b * u.col_image + (int64_t)c * u.col_channel + off;
+    Acc acc = accumulate ? (Acc)im[idx] : (Acc)0;
+    for (int m0 = lo[0]; m0 <= hi[0]; ++m0)
+        for (int m1 = lo[1]; m1 <= hi[1]; ++m1)
+            for (int m2 = lo[2]; m2 <= hi[2]; ++m2) {
+                const T* rowp = base + m0 * u.step[0] + m1 * u.step[1] + m2 * u.step[2];
+                for (int n = lo[3]; n <= hi[3]; n += 4) {
+                    T v[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (n + e <= hi[3]) v[e] = rowp[(int64_t)(n + e) * u.step[3]];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (n + e <= hi[3]) acc += (Acc)v[e];
+                }
+            }
+    im[idx] = (T)acc;
+}
+
+// (false: dilated windows, or sizes that the 32-bit arithmetic does not hold)
+static bool col2imnd_step_params(const UnfoldNdParams& u, Col2imNdStep& q) {
+    const int64_t total = u.batch * u.channels * u.vol, lim = 1LL << 30;
+    if (total >= 0x7fffffffLL || u.nd > 4) return false;
+    std::memset(&q, 0, sizeof q);
+    int64_t taps = 1, outs = 1;
+    for (int a = 3; a >= 0; --a) {
+        const int x = a - (4 - u.nd);                              // this axis of u; axes in front of its first are of size 1
+        const int64_t size = x >= 0 ? u.size[x] : 1, k = x >= 0 ? u.k[x] : 1, st = x >= 0 ? u.s[x] : 1, p = x >= 0 ? u.p[x] : 0, o = x >= 0 ? u.out[x] : 1;
+        if ((x >= 0 && u.d[x] != 1) || p < 0 || size + p >= lim || k >= lim || st >= lim || o * st >= lim) return false;
+        q.size[a] = (int)size; q.k[a] = (int)k; q.s[a] = (int)st; q.p[a] = (int)p; q.o[a] = (int)o;
+        q.div_size[a] = make_fastdiv((uint32_t)size); q.div_s[a] = make_fastdiv((uint32_t)st);
+        q.tap[a] = taps * u.L; q.out[a] = outs;
+        q.step[a] = st * taps * u.L - outs;
+        taps *= k; outs *= o;
+    }
+    q.div_c = make_fastdiv((uint32_t)u.channels);
+    q.channels = (int)u.channels; q.total = (uint32_t)total; q.col_image = u.ccol * u.L; q.col_channel = u.taps * u.L;
+    return true;
+}
+
 hipError_t launch_unfoldnd(int64_t es, const void* im, void* col, const UnfoldNdParams& u, hipStream_t s) {
     if (u.total == 0) return hipSuccess;
     const dim3 g(grid_for(u.total)), b(256);
@@ -282,21 +354,28 @@ hipError_t launch_col2imnd(int dtype, const void* col, void* im, const UnfoldNdP
     const int64_t total = u.batch * u.channels * u.vol;
     if (total == 0) return hipSuccess;
     const dim3 g(grid_for(total)), b(256);
+    Col2imNdStep q;
+    const bool step = col2imnd_step_params(u, q);
+    const dim3 gq((unsigned)((total + 255) / 256));
+#define NTG_COL2IMND(T, ACC) \
+    do { if (step) hipLaunchKernelGGL((col2imnd_step_kernel<T, ACC>), gq, b, 0, s, (const T*)col, (T*)im, q, accumulate); \
+         else hipLaunchKernelGGL((col2imnd_kernel<T, ACC>), g, b, 0, s, (const T*)col, (T*)im, u, accumulate); } while (0)
     switch (dtype) {
-    case DT_F32: hipLaunchKernelGGL((col2imnd_kernel<float, float>), g, b, 0, s, (const float*)col, (float*)im, u, accumulate); break;
-    case DT_F64: hipLaunchKernelGGL((col2imnd_kernel<double, double>), g, b, 0, s, (const double*)col, (double*)im, u, accumulate); break;
-    case DT_F16: hipLaunchKernelGGL((col2imnd_kernel<_Float16, float>), g, b, 0, s, (const _Float16*)col, (_Float16*)im, u, accumulate); break;
-    case DT_BF16: hipLaunchKernelGGL((col2imnd_kernel<__bf16, float>), g, b, 0, s, (const __bf16*)col, (__bf16*)im, u, accumulate); break;
-    case DT_I8: case DT_U8: hipLaunchKernelGGL((col2imnd_kernel<uint8_t, uint8_t>), g, b, 0, s, (const uint8_t*)col, (uint8_t*)im, u, accumulate); break;
-    case DT_I16: case DT_U16: hipLaunchKernelGGL((col2imnd_kernel<uint16_t, uint16_t>), g, b, 0, s, (const uint16_t*)col, (uint16_t*)im, u, accumulate); break;
-    case DT_I32: case DT_U32: hipLaunchKernelGGL((col2imnd_kernel<uint32_t, uint32_t>), g, b, 0, s, (const uint32_t*)col, (uint32_t*)im, u, accumulate); break;
-    case DT_I64: case DT_U64: hipLaunchKernelGGL((col2imnd_kernel<uint64_t, uint64_t>), g, b, 0, s, (const uint64_t*)col, (uint64_t*)im, u, accumulate); break;
+    case DT_F32: NTG_COL2IMND(float, float); break;
+    case DT_F64: NTG_COL2IMND(double, double); break;
+    case DT_F16: NTG_COL2IMND(_Float16, float); break;
+    case DT_BF16: NTG_COL2IMND(__bf16, float); break;
+    case DT_I8: case DT_U8: NTG_COL2IMND(uint8_t, uint8_t); break;
+    case DT_I16: case DT_U16: NTG_COL2IMND(uint16_t, uint16_t); break;
+    case DT_I32: case DT_U32: NTG_COL2IMND(uint32_t, uint32_t); break;
+    case DT_I64: case DT_U64: NTG_COL2IMND(uint64_t, uint64_t); break;
     // complex: the two lanes of an element are added separately in the lane's type, taps in the same ascending order
-    case DT_C32: hipLaunchKernelGGL((col2imnd_kernel<LanePair<_Float16>, LanePair<_Float16>>), g, b, 0, s, (const LanePair<_Float16>*)col, (LanePair<_Float16>*)im, u, accumulate); break;
-    case DT_C64: hipLaunchKernelGGL((col2imnd_kernel<LanePair<float>, LanePair<float>>), g, b, 0, s, (const LanePair<float>*)col, (LanePair<float>*)im, u, accumulate); break;
-    case DT_C128: hipLaunchKernelGGL((col2imnd_kernel<LanePair<double>, LanePair<double>>), g, b, 0, s, (const LanePair<double>*)col, (LanePair<double>*)im, u, accumulate); break;
+    case DT_C32: NTG_COL2IMND(LanePair<_Float16>, LanePair<_Float16>); break;
+    case DT_C64: NTG_COL2IMND(LanePair<float>, LanePair<float>); break;
+    case DT_C128: NTG_COL2IMND(LanePair<double>, LanePair<double>); break;
     default: return hipErrorInvalidValue;
     }
+#undef NTG_COL2IMND
     return hipGetLastError();
 }
 

@@ -3,9 +3,14 @@
 The bound: an output of n products is rounded once to its type (unit roundoff u; Float16 below 2^-14: 2^-25) after a sum in 32 bits whose error
 is at most n 2^-24 times the sum of the products' magnitudes.  Where parts of the sum are stored in the type on the way (the entries of a col
 matrix, the products per image of a layer of one tap) each is rounded too: u times those magnitudes more."""
+import ctypes
+
+import numpy as np
 import pytest
 import torch
 
+import oracle
+from neurotensor_amd import _lib
 from neurotensor_amd import functional as F
 
 pytestmark = pytest.mark.gpu
@@ -95,3 +100,24 @@ def test_a_batch_of_groups_split_in_two_launches_keeps_whole_images():
 ], ids=str)
 def test_flat_tiles(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed):
     check(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed)
+
+
+@pytest.mark.parametrize("size,kernel,stride,pad,dil", [
+    ((7,), (3,), (2,), (1,), (1,)), ((9,), (2,), (4,), (0,), (1,)),                     # (positions that no window reaches)
+    ((6, 9), (3, 5), (2, 1), (1, 2), (1, 1)),
+    ((5, 6, 7), (4, 4, 4), (2, 2, 2), (1, 1, 1), (1, 1, 1)), ((4, 8, 3), (1, 1, 1), (2, 2, 2), (0, 0, 0), (1, 1, 1)),
+    ((3, 5, 20), (2, 3, 9), (1, 3, 2), (0, 1, 5), (1, 1, 1)), ((6, 5, 7), (2, 3, 2), (1, 2, 1), (1, 0, 2), (2, 1, 1)),      # (dilated: the general kernel)
+    ((3, 4, 3, 5), (2, 2, 3, 3), (1, 2, 1, 2), (1, 0, 1, 1), (1, 1, 1, 1)),
+], ids=str)
+def test_col_matrix_back_onto_an_image_in_tap_order(size, kernel, stride, pad, dil):
+    """Up to four axes, bit for bit: every position adds its taps in ascending order."""
+    nd, batch, channels = len(size), 2, 3
+    out = [(s + 2 * p - d * (k - 1) - 1) // st + 1 for s, k, st, p, d in zip(size, kernel, stride, pad, dil)]
+    rng = np.random.default_rng(5)
+    col = rng.standard_normal((batch, channels * int(np.prod(kernel)), int(np.prod(out)))).astype(np.float32)
+    arr = lambda v: (ctypes.c_int64 * nd)(*v)
+    image = torch.empty((batch, channels) + size, device="cuda")
+    _lib.check(_lib.load().ntg_unfoldnd_backward_dev(_lib.FLOAT32, torch.from_numpy(col).cuda().data_ptr(), image.data_ptr(), batch, channels, nd, arr(size), arr(kernel),
+                                                     arr(stride), arr(pad), arr(dil), 0, torch.cuda.current_stream().cuda_stream))
+    want = oracle.unfoldnd_backward(col, size, kernel, dil, pad, stride)
+    assert np.array_equal(image.cpu().numpy().view(np.uint32), want.view(np.uint32))
