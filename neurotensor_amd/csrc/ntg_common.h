@@ -423,8 +423,8 @@ hipError_t launch_phase_setup(int64_t es, const void* w, void* wt, RingItem* ite
 hipError_t launch_phase_interleave(int dtype, const void* tmp, void* im, const PhaseLayout& q, int accumulate, hipStream_t s);
 hipError_t launch_conv_nhwc_items(int dtype, int edge, const GemmParams& p, int64_t blocks, hipStream_t s);
 hipError_t launch_conv_nhwc_dw(int dtype, bool ta, const GemmParams& p, hipStream_t s);   // ta: A (the output gradient) stored [k][m]
-// part rows hold cgp >= cg channels per tap; the partial sums are Float32 whatever the dtype
-hipError_t launch_reduce_batch_taps_last(int dtype, const void* part, void* out, int64_t batch, int64_t rows, int64_t cg, int64_t cgp,
+// part rows hold cgp >= cg channels per tap, and ogp >= og rows a group (rows: of all groups); the partial sums are Float32 whatever the dtype
+hipError_t launch_reduce_batch_taps_last(int dtype, const void* part, void* out, int64_t batch, int64_t rows, int64_t og, int64_t ogp, int64_t cg, int64_t cgp,
                                          int64_t taps, int accumulate, hipStream_t s);
 hipError_t launch_flip_weights(int64_t elem_size, const void* w, void* wt, int64_t groups, int64_t og, int64_t cg, int64_t taps, hipStream_t s);
 

@@ -1803,8 +1803,10 @@ static double dkernel_cost_us(int64_t es, int edge, int64_t tiles, int64_t K) {
     return 3.0 + k * std::max(0.009, 0.0042 * w);
 }
 // How dW is cut up: `ranges` k ranges of `kr` output pixels (0: one product per image), tiles of edge x edge, dY read where it
-// lies (its rows 16-byte multiples, an image a whole number of K-steps) or through a channels-last copy of its own (the out
-// channels of a group a 16-byte multiple; any range then).  The partial sums are Float32 whatever the type, so that a 16-bit gradient
+// lies (its rows 16-byte multiples, an image a whole number of K-steps) or through a channels-last copy of its own (any range then), with
+// the out channels of a group padded to 16 bytes: rows of zeros that the last pass skips.  Without that padding a layer with odd planes and odd
+// channels ran on the element-wise gather, one chain an image: BFloat16 5 x 192 x 125 x 125 -> 48 by one tap in 4 groups, a step 2033 us before, 153 with
+// it, Float32 2 x 24 x 63 x 63 transposed to 96 by 4 x 4 in 4 groups 773 | 100, BFloat16 1 x 223 x 223 -> 16 by 5 x 5 1518 | 60.  The partial sums are Float32 whatever the type, so that a 16-bit gradient
 // is rounded once (rounded to 16 bits each, they left sqrt(2) of one rounding's error in the sum: BFloat16 2 x 256 x 32 x 32 -> 1024
 // channels by 3 x 3 2.45e-3 against 1.66e-3).
 // One product per image left a small layer on a handful of workgroups, each with the whole image as its k (3 x 3 x 3 x 32 -> 64
@@ -1820,12 +1822,13 @@ static DkernelPlan plan_dkernel(int dtype, int64_t batch, int64_t channels, int6
     const int64_t es = ntg::elem_size(dtype), bk = 64 / es, cg = channels / groups, og = out_channels / groups, L = g.L();
     if (g.k[1] * g.d[1] >= 32768 || g.k[2] * g.d[2] >= 32768) return pl;         // tap reach packed in 16 bits
     const int64_t cgp = dkernel_padded_channels(es, cg), N = cgp * g.taps();
-    if (cgp > 4 * cg || N >= 0x7fffffffLL || !conv_nhwc_offsets_fit(groups * cgp, es, g)) return pl;
+    if (cgp > (es == 2 ? 8 : 4) * cg || N >= 0x7fffffffLL || !conv_nhwc_offsets_fit(groups * cgp, es, g)) return pl;
     if (g.nd == 3 && !dkernel_halo(es, cg, groups, g).on) return pl;             // (three axes: the bordered copy is the only form)
-    const bool rows_16 = (L * es) % 16 == 0, og_16 = (og * es) % 16 == 0;
+    const bool rows_16 = (L * es) % 16 == 0;
+    const int64_t ogp = dkernel_padded_channels(es, og);                         // (rows of a copied dY)
     const int64_t total = batch * L, steps = (total + bk - 1) / bk;
     const bool countable = total < (1LL << 30);
-    const bool lies = rows_16 && L % bk == 0 && countable, copied = og_16 && countable;
+    const bool lies = rows_16 && L % bk == 0 && countable, copied = countable;
     if (!rows_16 && !copied) return pl;
     pl.ok = true;
     // measurement and test knob: NTG_DW_RANGES=r forces r ranges of dY where it lies where r is admissible, 0 one product per image
@@ -1843,8 +1846,8 @@ static DkernelPlan plan_dkernel(int dtype, int64_t batch, int64_t channels, int6
         double best = 0.0;
         const auto consider = [&](bool copy, int64_t ranges, int64_t items, int64_t kr, int edge) {
             const int64_t tiles = ((og + edge - 1) / edge) * ((N + edge - 1) / edge) * items * groups;
-            const double us = (copy ? 4.0 + 2.0 * (double)(total * out_channels * es) / 4.5e6 : 0.0) + dkernel_cost_us(es, edge, tiles, kr) + 4.0 +
-                              2.0 * (double)(items * out_channels * N * 4) / 4.0e6;
+            const double us = (copy ? 4.0 + (double)(total * (out_channels + groups * ogp) * es) / 4.5e6 : 0.0) + dkernel_cost_us(es, edge, tiles, kr) + 4.0 +
+                              2.0 * (double)(items * groups * (copy ? ogp : og) * N * 4) / 4.0e6;
             if (pl.edge && us >= best) return;
             best = us;
             pl.copy_dy = copy; pl.ranges = ranges; pl.items = items; pl.kr = kr; pl.edge = edge;
@@ -1866,36 +1869,39 @@ static DkernelPlan plan_dkernel(int dtype, int64_t batch, int64_t channels, int6
 }
 static int64_t conv_dkernel_nhwc_workspace(int dtype, const DkernelPlan& pl, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
     const int64_t es = ntg::elem_size(dtype);
-    const int64_t gy = pl.copy_dy ? (int64_t)align_up((size_t)(batch * out_channels * g.L() * es), 256) : 0;
+    const int64_t rows = pl.copy_dy ? groups * dkernel_padded_channels(es, out_channels / groups) : out_channels;
+    const int64_t gy = pl.copy_dy ? (int64_t)align_up((size_t)(batch * rows * g.L() * es), 256) : 0;
     const int64_t cgp = dkernel_padded_channels(es, channels / groups);
     return (int64_t)align_up((size_t)(batch * groups * cgp * dkernel_halo(es, channels / groups, groups, g).vol * es), 256) + gy +
-           pl.items * out_channels * cgp * g.taps() * 4;
+           pl.items * rows * cgp * g.taps() * 4;
 }
 static int conv_dkernel_nhwc(int dtype, const DkernelPlan& pl, const void* image, const void* grad_out, void* d_kernel, void* ws, int64_t batch,
                              int64_t channels, int64_t out_channels, const Geo3& g, int64_t groups, int accumulate, hipStream_t hs) {
     const int64_t es = ntg::elem_size(dtype), bk = 64 / es, cg = channels / groups, og = out_channels / groups;
     const int64_t cgp = dkernel_padded_channels(es, cg), chp = groups * cgp;      // channels per group / per pixel in the copy
+    const int64_t ogr = pl.copy_dy ? dkernel_padded_channels(es, og) : og, rows = groups * ogr;     // rows of a group and in all: a copied dY's are whole 16 bytes
     const int64_t L = g.L(), taps = g.taps(), vol = g.vol(), N = taps * cgp;
     const HaloPlan halo = dkernel_halo(es, cg, groups, g);
     const int64_t volp = halo.vol;                                                         // pixels per image of the copy
     char* ws_img = static_cast<char*>(ws);
     char* ws_gy = ws_img + align_up((size_t)(batch * chp * volp * es), 256);
-    char* ws_part = ws_gy + (pl.copy_dy ? align_up((size_t)(batch * out_channels * L * es), 256) : 0);
+    char* ws_part = ws_gy + (pl.copy_dy ? align_up((size_t)(batch * rows * L * es), 256) : 0);
     const ntg::HaloMap* hm = halo.on ? &halo.hm : nullptr;
     bool took_along = false;
     hipError_t e = cgp == cg ? ntg::launch_nchw_to_nhwc(es, image, ws_img, batch, channels, vol, hs, hm, nullptr, &took_along)
                              : ntg::launch_nchw_to_nhwc_padded(es, image, ws_img, batch, groups, cg, cgp, vol, hs, hm);
     if (e == hipSuccess && halo.on && volp != vol && !took_along) e = ntg::launch_halo_zero(es, ws_img, batch, chp, halo.hm, hs);
-    if (e == hipSuccess && pl.copy_dy) e = ntg::launch_nchw_to_nhwc(es, grad_out, ws_gy, batch, out_channels, L, hs);
+    if (e == hipSuccess && pl.copy_dy)
+        e = ogr == og ? ntg::launch_nchw_to_nhwc(es, grad_out, ws_gy, batch, out_channels, L, hs) : ntg::launch_nchw_to_nhwc_padded(es, grad_out, ws_gy, batch, groups, og, ogr, L, hs);
     if (e != hipSuccess) return hip_fail(e, "channels-last copy launch");
     ntg::GemmParams p;
     std::memset(&p, 0, sizeof p);
-    p.M = (int)og; p.K = (int)(pl.ranges ? pl.kr : L); p.N = (int)N;
+    p.M = (int)ogr; p.K = (int)(pl.ranges ? pl.kr : L); p.N = (int)N;
     p.A = pl.copy_dy ? static_cast<const void*>(ws_gy) : grad_out;
-    p.lda = pl.copy_dy ? out_channels : L;
+    p.lda = pl.copy_dy ? rows : L;
     p.B = ws_img; p.C = ws_part;
     p.ldb = chp; p.ldc = N;
-    const int64_t a_item = pl.copy_dy ? pl.kr * out_channels : pl.ranges ? 0 : out_channels * L;     // (a range: or an image)
+    const int64_t a_item = pl.copy_dy ? pl.kr * rows : pl.ranges ? 0 : out_channels * L;     // (a range: or an image)
     p.cmode = ntg::C_PARTIAL;
     p.vecA_ok = 1; p.vecB_ok = 1;
     fill_conv_geom(p.conv, cgp, halo.gp);
@@ -1916,11 +1922,11 @@ static int conv_dkernel_nhwc(int dtype, const DkernelPlan& pl, const void* image
             p.conv.a_image_stride = out_channels * L;
         }
     }
-    e = launch_groups(p, dtype, pl.items, groups, {pl.copy_dy ? og : og * L, a_item, cgp, pl.ranges ? 0 : chp * volp, og * N},
+    e = launch_groups(p, dtype, pl.items, groups, {pl.copy_dy ? ogr : og * L, a_item, cgp, pl.ranges ? 0 : chp * volp, ogr * N},
                       [&](const ntg::GemmParams& q) { return ntg::launch_conv_nhwc_dw(dtype, pl.copy_dy, q, hs); });
     if (e != hipSuccess) return hip_fail(e, "channels-last conv_dkernel launch");
     // (groups are consecutive row blocks of both layouts, so one pass covers them all)
-    e = ntg::launch_reduce_batch_taps_last(dtype, ws_part, d_kernel, pl.items, out_channels, cg, cgp, taps, accumulate, hs);
+    e = ntg::launch_reduce_batch_taps_last(dtype, ws_part, d_kernel, pl.items, rows, og, ogr, cg, cgp, taps, accumulate, hs);
     if (e != hipSuccess) return hip_fail(e, "weight gradient reduction launch");
     return NTG_OK;
 }
@@ -1969,17 +1975,68 @@ static int conv_dkernel_from_col(int dtype, const char* gy, char* col, void* d_k
     return NTG_OK;
 }
 
+// dW of one tap on rows of 16-byte multiples: dY_b . X_b^T per image on the operands where they lie, every image's pixels in `splits` equal ranges of
+// whole K-steps so that tiles x images x groups x ranges fill the CUs, the Float32 sums of all of them added up in one pass.  With one range an
+// image a few large images were a few workgroups, each a chain of all its pixels (Float16 4 x 128 x 192 x 192 -> 96, a step: 231 us, 56 with
+// ranges; Float32 6 x 64 x 5992 -> 32 in 4 groups 299 | 139, 1 x 192 x 112 x 112 -> 48 104 | 37), and 16-bit gradients were rounded once an image.
+struct PointwiseDwPlan { int64_t splits, bytes; };                               // splits 0: one product an image in the element type
+static PointwiseDwPlan plan_pointwise_dw(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
+    PointwiseDwPlan pl = {0, 0};
+    if (dtype != ntg::DT_F32 && dtype != ntg::DT_F16 && dtype != ntg::DT_BF16) return pl;
+    const int64_t es = ntg::elem_size(dtype), bk = 64 / es, cg = channels / groups, og = out_channels / groups, L = g.L();
+    if (!conv_pointwise_ok(dtype, channels, groups, g) || (og * es) % 16 != 0 || batch <= 0 || og <= 0) return pl;
+    const int64_t tiles = ((og + 63) / 64) * ((cg + 63) / 64) * batch * groups;
+    if (tiles >= 0x7fffffffLL || L >= 0x7fffffffLL) return pl;
+    const uint32_t steps = L % bk == 0 ? (uint32_t)(L / bk) : 1u;
+    double best = 0.0;
+    for (uint32_t s = 1; s <= steps && (s == 1 || tiles * s <= 2048); ++s) {      // (eight tiles a CU: more only makes more partial sums)
+        if (steps % s != 0) continue;
+        const int64_t items = batch * groups * s, K = L / s;
+        double us;
+        if (es == 2) {
+            const int te = ntg::ring16_tile_edge(og, cg, K, items);
+            us = ntg::ring16_cost_us(te, ntg::ring16_tiles(te, og, cg, items), K);
+        } else {
+            us = std::min(ntg::ring_f32_cost(128, og, cg, items), ntg::ring_f32_cost(64, og, cg, items)) * ((double)K * 0.062 + 3.0);
+        }
+        us += 2.0 * (double)(items * og * cg * 4) / 4.0e6;
+        if (pl.splits == 0 || us < best) { best = us; pl.splits = s; }
+    }
+    pl.bytes = pl.splits * batch * out_channels * cg * 4;
+    return pl;
+}
+static int conv_dkernel_pointwise(int dtype, const PointwiseDwPlan& pl, const void* image, const void* grad_out, void* d_kernel, void* ws, int64_t batch,
+                                  int64_t channels, int64_t out_channels, const Geo3& g, int64_t groups, int accumulate, hipStream_t hs) {
+    const int64_t cg = channels / groups, og = out_channels / groups, L = g.L();
+    ntg::GemmParams p;
+    std::memset(&p, 0, sizeof p);
+    p.M = (int)og; p.K = (int)(L / pl.splits); p.N = (int)cg;
+    p.A = grad_out; p.B = image; p.C = ws;
+    p.lda = L; p.ldb = L; p.ldc = cg;
+    // launch index = range * (images * groups) + image * groups + group
+    p.batch = (int)(batch * groups * pl.splits);
+    p.krange_items = (int)(batch * groups);
+    p.sA = og * L; p.sB = cg * L; p.sAk = p.sBk = p.K; p.sC = og * cg;
+    p.cmode = dtype == ntg::DT_F32 ? ntg::C_OVERWRITE : ntg::C_PARTIAL;
+    const int rc = launch_gemm(p, dtype, false, true, hs);
+    if (rc) return rc;
+    hipError_t e = ntg::launch_reduce_batch_taps_last(dtype, ws, d_kernel, pl.splits * batch, out_channels, og, og, cg, cg, 1, accumulate, hs);
+    if (e != hipSuccess) return hip_fail(e, "weight gradient reduction launch");
+    return NTG_OK;
+}
+
 // Which backward gradients run as implicit GEMMs, and the workspace the call needs.
-struct ConvBackwardPlan { bool gather_dw, gather_dx, nhwc_dx, nhwc_dw, phase_dx; int64_t need, need_nhwc_dx, need_nhwc_dw, need_phase_dx, need_wt_dx, wt_offset; PhasePlan phases; DkernelPlan dkernel; };
+struct ConvBackwardPlan { bool gather_dw, gather_dx, nhwc_dx, nhwc_dw, phase_dx; int64_t need, need_nhwc_dx, need_nhwc_dw, need_phase_dx, need_wt_dx, wt_offset; PointwiseDwPlan pointwise; PhasePlan phases; DkernelPlan dkernel; };
 // reference_order (Float32 through the host entry points): the forms whose sums are the reference's own, bit for bit -- the
 // image gradient as W^T . dY into the col matrix + col2im (conv.cpp:318-346; the implicit forms run one chain over out
 // channels and taps where the reference rounds in between), the weight gradient per image with k = the output pixels +
 // the sum over the batch (conv.cpp:444-471; not the channels-last kernels, whose partial sums may span images).
 static ConvBackwardPlan plan_conv_backward_g(int dtype, bool want_dx, bool want_dw, int64_t batch, int64_t channels, int64_t out_channels,
-                                             const Geo3& g, int64_t groups, bool reference_order = false) {
+                                             const Geo3& g, int64_t groups, bool reference_order = false, bool in_place = false) {
     const int64_t es = ntg::elem_size(dtype);
     const int64_t cg = channels / groups, taps = g.taps();
     ConvBackwardPlan pl;
+    std::memset(&pl, 0, sizeof pl);
     pl.gather_dw = want_dw && conv_implicit_g(dtype, channels, g);
     pl.gather_dx = want_dx && !reference_order && g.s[0] == 1 && g.s[1] == 1 && g.s[2] == 1 && conv_implicit_g(dtype, out_channels, geo_dimage(g));
     const int64_t col = batch * channels * taps * g.L() * es;
@@ -1987,15 +2044,15 @@ static ConvBackwardPlan plan_conv_backward_g(int dtype, bool want_dx, bool want_
     if (want_dw) need = std::max(need, pl.gather_dw ? batch * out_channels * cg * taps * es : col + complex_dkernel_extra(dtype, batch, out_channels, cg * taps, col));
     if (want_dx) need = std::max(need, pl.gather_dx ? out_channels * cg * taps * es : col);
     pl.need = need;
+    pl.pointwise = want_dw && !reference_order ? plan_pointwise_dw(dtype, batch, channels, out_channels, groups, g) : PointwiseDwPlan{0, 0};
+    if (in_place) return pl;                       // (one tap on operands where they lie: the call takes none of the forms below)
     // the channels-last form of dX is taken when the caller's workspace also holds the copy of dY
     pl.nhwc_dx = pl.gather_dx && conv_dimage_nhwc_ok(dtype, channels, out_channels, groups, g);
     pl.need_nhwc_dx = pl.nhwc_dx ? conv_dimage_nhwc_workspace(dtype, batch, channels, out_channels, groups, g) : 0;
-    std::memset(&pl.dkernel, 0, sizeof pl.dkernel);
     if (pl.gather_dw && !reference_order) pl.dkernel = plan_dkernel(dtype, batch, channels, out_channels, groups, g);
     pl.nhwc_dw = pl.dkernel.ok;
     pl.need_nhwc_dw = pl.nhwc_dw ? conv_dkernel_nhwc_workspace(dtype, pl.dkernel, batch, channels, out_channels, groups, g) : 0;
     // strides > 1: dX phase by phase instead of GEMM + col2im, again when the workspace allows
-    std::memset(&pl.phases, 0, sizeof pl.phases);
     if (want_dx && !pl.gather_dx && !reference_order)
         pl.phases = plan_dimage_phases(dtype, batch, channels, out_channels, groups, g);
     pl.phase_dx = pl.phases.ok;
@@ -2191,9 +2248,9 @@ int ntg_unfold2d_backward(int dtype, const void* col, void* image,
 
 static ConvBackwardPlan plan_conv_backward(int dtype, bool want_dx, bool want_dw, int64_t batch, int64_t channels, int64_t height, int64_t width,
                                            int64_t out_channels, int64_t k_r, int64_t k_c, int64_t s_r, int64_t s_c, int64_t p_r, int64_t p_c,
-                                           int64_t d_r, int64_t d_c, int64_t groups, int64_t Ho, int64_t Wo, bool reference_order = false) {
+                                           int64_t d_r, int64_t d_c, int64_t groups, int64_t Ho, int64_t Wo, bool reference_order = false, bool in_place = false) {
     return plan_conv_backward_g(dtype, want_dx, want_dw, batch, channels, out_channels,
-                                geo2(height, width, k_r, k_c, s_r, s_c, p_r, p_c, d_r, d_c, Ho, Wo), groups, reference_order);
+                                geo2(height, width, k_r, k_c, s_r, s_c, p_r, p_c, d_r, d_c, Ho, Wo), groups, reference_order, in_place);
 }
 
 int64_t ntg_conv2d_backward_workspace_bytes(int dtype, int64_t batch, int64_t channels, int64_t height, int64_t width,
@@ -2205,7 +2262,7 @@ int64_t ntg_conv2d_backward_workspace_bytes(int dtype, int64_t batch, int64_t ch
     // the larger of what the call needs at least and what lets dX take its channels-last form (copy of dY + flipped weights)
     const ConvBackwardPlan pl = plan_conv_backward(dtype, true, true, batch, channels, height, width, out_channels, k_r, k_c, s_r, s_c, p_r, p_c,
                                                    d_r, d_c, groups, Ho, Wo);
-    return std::max(std::max(std::max(pl.need, pl.need_phase_dx), pl.need_wt_dx), std::max(pl.need_nhwc_dx, pl.need_nhwc_dw));
+    return std::max({pl.need, pl.need_phase_dx, pl.need_wt_dx, pl.need_nhwc_dx, pl.need_nhwc_dw, pl.pointwise.bytes});
 }
 
 static int conv2d_backward_dev_impl(int dtype, const void* image, const void* kernel, const void* grad_out,
@@ -2227,8 +2284,15 @@ static int conv2d_backward_dev_impl(int dtype, const void* image, const void* ke
     if (!kernel || !grad_out || (d_kernel && !image)) return fail(NTG_ERR_INVALID_ARGUMENT, "null pointer");
     const int64_t L = Ho * Wo, ckk = channels * k_r * k_c;
     const int64_t add = (channels / groups) * k_r * k_c, og = out_channels / groups;
+    const Geo3 geo = geo2(height, width, k_r, k_c, s_r, s_c, p_r, p_c, d_r, d_c, Ho, Wo);
+    // 1x1 kernel, unit stride, no padding (floating dtypes, 16-byte rows): col is the image itself, so both gradients are
+    // products on the tensors where they lie: dX_b = W_g^T . dY_b, and dW_g = sum_b dY_b . X_b^T through per-image results
+    // in the workspace (the amount the gathering form needs), summed in batch order, or through those of ranges of the images' pixels.
+    const bool in_place = !is_valu_dtype(dtype) && !(reference_order && accumulate) && conv_pointwise_ok(dtype, channels, groups, geo) && (og * es) % 16 == 0 &&
+                          ((reinterpret_cast<uintptr_t>(image) | reinterpret_cast<uintptr_t>(kernel) | reinterpret_cast<uintptr_t>(grad_out) |
+                            reinterpret_cast<uintptr_t>(d_image) | reinterpret_cast<uintptr_t>(d_kernel) | reinterpret_cast<uintptr_t>(workspace)) & 15) == 0;
     const ConvBackwardPlan plan = plan_conv_backward(dtype, d_image != nullptr, d_kernel != nullptr, batch, channels, height, width,
-                                                     out_channels, k_r, k_c, s_r, s_c, p_r, p_c, d_r, d_c, groups, Ho, Wo, reference_order);
+                                                     out_channels, k_r, k_c, s_r, s_c, p_r, p_c, d_r, d_c, groups, Ho, Wo, reference_order, in_place);
     if (plan.need > 0 && (!workspace || workspace_bytes < plan.need))
         return fail(NTG_ERR_INVALID_ARGUMENT, "workspace of %lld bytes needed, %lld given", (long long)plan.need, (long long)workspace_bytes);
     const char* kern = static_cast<const char*>(kernel);
@@ -2238,19 +2302,15 @@ static int conv2d_backward_dev_impl(int dtype, const void* image, const void* ke
     ntg_gemm_desc d;
     // Floating dtypes: neither gradient needs the stored im2col matrix (conv_dkernel_gather, conv_dimage_gather).
     bool gather_dw = plan.gather_dw, gather_dx = plan.gather_dx;
-    const Geo3 geo = geo2(height, width, k_r, k_c, s_r, s_c, p_r, p_c, d_r, d_c, Ho, Wo);
-    // 1x1 kernel, unit stride, no padding (floating dtypes, 16-byte rows): col is the image itself, so both gradients are
-    // products on the tensors where they lie: dX_b = W_g^T . dY_b, and dW_g = sum_b dY_b . X_b^T through per-image results
-    // in the workspace (the amount the gathering form needs), summed in batch order.
-    if (!is_valu_dtype(dtype) && !(reference_order && accumulate) && conv_pointwise_ok(dtype, channels, groups, geo) && (og * es) % 16 == 0 &&
-        ((reinterpret_cast<uintptr_t>(image) | reinterpret_cast<uintptr_t>(kernel) | reinterpret_cast<uintptr_t>(grad_out) |
-          reinterpret_cast<uintptr_t>(d_image) | reinterpret_cast<uintptr_t>(d_kernel) | reinterpret_cast<uintptr_t>(ws)) & 15) == 0) {
+    if (in_place) {
         const int64_t cg = channels / groups;
         if (d_image) {
             rc = gemm_per_group(dtype, true, false, accumulate ? NTG_C_ACCUMULATE : NTG_C_OVERWRITE, cg, og, L, cg, L, L, batch, groups, kern, og * cg, 0,
                                 gy, og * L, out_channels * L, d_image, stream);
             if (rc) return rc;
         }
+        if (d_kernel && plan.pointwise.splits > 0 && workspace_bytes >= plan.pointwise.bytes)
+            return conv_dkernel_pointwise(dtype, plan.pointwise, image, grad_out, d_kernel, ws, batch, channels, out_channels, geo, groups, accumulate, hs);
         if (d_kernel) {
             rc = gemm_per_group(dtype, false, true, NTG_C_OVERWRITE, og, L, cg, L, L, cg, batch, groups, gy, og * L, out_channels * L,
                                 image, cg * L, channels * L, ws, stream);

@@ -49,8 +49,8 @@ __global__ void __launch_bounds__(256) reduce_batch_sum_first_kernel(const T* __
 // 66 MB: four slices, 16.1 us).  The order of the additions depends on the sizes only.
 template <class T, int SLICES>
 __global__ void __launch_bounds__(256) reduce_batch_taps_last_kernel(const float* __restrict__ part, T* __restrict__ out, const int64_t batch,
-                                                                     const int64_t rows, const int64_t cg, const int64_t cgp, const int64_t taps,
-                                                                     const int accumulate) {
+                                                                     const int64_t rows, const int64_t og, const int64_t ogp, const int64_t cg, const int64_t cgp,
+                                                                     const int64_t taps, const int accumulate) {
     constexpr int VEC = 4;
     typedef float PV __attribute__((ext_vector_type(VEC)));
     constexpr int COLS = 256 / SLICES;                    // column groups of VEC elements per workgroup
@@ -88,7 +88,13 @@ __global__ void __launch_bounds__(256) reduce_batch_taps_last_kernel(const float
             for (int e = 0; e < VEC; ++e) acc[e] += sums[(e * SLICES + o) * COLS + col];
     }
     if (v >= nv) return;
-    const int64_t c = i % cgp, t = (i / cgp) % taps, o = i / (cgp * taps);
+    const int64_t c = i % cgp, t = (i / cgp) % taps;
+    int64_t o = i / (cgp * taps);
+    if (ogp != og) {                                      // (uniform; a group's rows may be padded too)
+        const int64_t g = o / ogp;
+        if (o - g * ogp >= og) return;
+        o -= g * (ogp - og);
+    }
     T* dst = out + (o * cg + c) * taps + t;
 #pragma unroll
     for (int e = 0; e < VEC; ++e)
@@ -283,24 +289,24 @@ hipError_t launch_reduce_batch(int dtype, const void* part, void* out, int64_t b
 }
 
 template <class T>
-static void launch_reduce_taps_last_t(const void* part, void* out, int64_t batch, int64_t rows, int64_t cg, int64_t cgp, int64_t taps, int accumulate, hipStream_t s) {
+static void launch_reduce_taps_last_t(const void* part, void* out, int64_t batch, int64_t rows, int64_t og, int64_t ogp, int64_t cg, int64_t cgp, int64_t taps, int accumulate, hipStream_t s) {
     const int64_t nv = rows * cgp * taps / 4;
 #define NTG_TAPS_LAST(S) \
-    hipLaunchKernelGGL((reduce_batch_taps_last_kernel<T, S>), dim3((unsigned)((nv * S + 255) / 256)), dim3(256), 0, s, (const float*)part, (T*)out, batch, rows, cg, cgp, taps, accumulate)
+    hipLaunchKernelGGL((reduce_batch_taps_last_kernel<T, S>), dim3((unsigned)((nv * S + 255) / 256)), dim3(256), 0, s, (const float*)part, (T*)out, batch, rows, og, ogp, cg, cgp, taps, accumulate)
     if (nv >= 256 * 1024 || batch < 8) NTG_TAPS_LAST(1);
     else if (nv * 4 >= 256 * 1024 || batch < 32) NTG_TAPS_LAST(4);
     else NTG_TAPS_LAST(16);
 #undef NTG_TAPS_LAST
 }
-hipError_t launch_reduce_batch_taps_last(int dtype, const void* part, void* out, int64_t batch, int64_t rows, int64_t cg, int64_t cgp,
+hipError_t launch_reduce_batch_taps_last(int dtype, const void* part, void* out, int64_t batch, int64_t rows, int64_t og, int64_t ogp, int64_t cg, int64_t cgp,
                                          int64_t taps, int accumulate, hipStream_t s) {
     const int64_t n = rows * cgp * taps;
     if (n == 0) return hipSuccess;
     if (cgp % 4 != 0 || (reinterpret_cast<uintptr_t>(part) & 15) != 0 || n / 64 >= 0x7fffffffLL) return hipErrorInvalidValue;
     switch (dtype) {
-    case DT_F32: launch_reduce_taps_last_t<float>(part, out, batch, rows, cg, cgp, taps, accumulate, s); break;
-    case DT_F16: launch_reduce_taps_last_t<_Float16>(part, out, batch, rows, cg, cgp, taps, accumulate, s); break;
-    case DT_BF16: launch_reduce_taps_last_t<__bf16>(part, out, batch, rows, cg, cgp, taps, accumulate, s); break;
+    case DT_F32: launch_reduce_taps_last_t<float>(part, out, batch, rows, og, ogp, cg, cgp, taps, accumulate, s); break;
+    case DT_F16: launch_reduce_taps_last_t<_Float16>(part, out, batch, rows, og, ogp, cg, cgp, taps, accumulate, s); break;
+    case DT_BF16: launch_reduce_taps_last_t<__bf16>(part, out, batch, rows, og, ogp, cg, cgp, taps, accumulate, s); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

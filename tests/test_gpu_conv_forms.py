@@ -64,11 +64,11 @@ def check(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed
     (3, 128, 128, (17,), 5, 1, 2, 4, False, ()),
     (2, 64, 64, (5, 6, 7), 3, 1, 1, 2, False, ()),
     (3, 24, 32, (12, 12), 3, 2, 1, 4, False, ("dx",)),        # few channels a group: taps merged, image gradient through the col matrix
-    (2, 256, 144, (8, 8), 1, 1, 0, 4, False, ("dw",)),        # one tap: plain products
+    (2, 256, 144, (8, 8), 1, 1, 0, 4, False, ("dw",)),        # one tap: plain products (36 out channels a group: the images' products are rounded)
     (5, 48, 48, (9, 9), 1, 1, 0, 3, False, ()),          # ... on rows that miss 16 bytes
     (2, 64, 96, (6, 6), 4, 2, 1, 2, True, ()),
-    (2, 16, 16, (7, 5), 2, 2, 0, 4, True, ("y", "dw")),
-    (2, 30, 18, (10, 9), 3, 1, 1, 3, False, ("dw",)),         # element-wise gathers
+    (2, 16, 16, (7, 5), 2, 2, 0, 4, True, ("y",)),
+    (2, 30, 18, (10, 9), 3, 1, 1, 3, False, ()),         # element-wise gathers
 ], ids=str)
 def test_groups_as_items_of_one_launch(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed, parts):
     check(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed, parts)
@@ -91,7 +91,7 @@ def test_a_batch_of_groups_split_in_two_launches_keeps_whole_images():
     (1, 64, 1, (127,), 3, 1, 1, 1, False),           # 32 x 128 tiles: one row, one column short of a tile
     (2, 32, 32, (129,), 5, 1, 2, 1, False),          # ... all rows, one column more
     (3, 64, 33, (12, 12), 3, 1, 1, 1, False),        # one row too many
-    (2, 32, 24, (4, 5, 7), 3, 1, 1, 1, False),
+    (2, 32, 17, (4, 5, 7), 3, 1, 1, 1, False),        # (out channels padded for the weight gradient)
     (1040, 32, 31, (33,), 3, 1, 1, 1, False),        # 16 bits: 32 x 256 tiles
     (2, 16, 96, (9, 10), 3, 2, 1, 1, False),         # image gradient by phases
     (2, 64, 64, (16, 8), 4, 2, 1, 2, True),
@@ -121,3 +121,25 @@ def test_col_matrix_back_onto_an_image_in_tap_order(size, kernel, stride, pad, d
                                                      arr(stride), arr(pad), arr(dil), 0, torch.cuda.current_stream().cuda_stream))
     want = oracle.unfoldnd_backward(col, size, kernel, dil, pad, stride)
     assert np.array_equal(image.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("batch,cin,cout,size,kernel,stride,pad,groups,transposed", [
+    (3, 16, 1, (9, 9), 3, 1, 1, 1, False),           # one out channel, planes that miss 16 bytes
+    (2, 1, 9, (11, 7), 5, 1, 2, 1, False),           # one channel
+    (2, 24, 21, (13,), 3, 2, 1, 3, False),
+    (2, 8, 10, (5, 5, 5), 3, 1, 1, 2, False),
+    (1, 6, 260, (15, 15), 3, 1, 1, 1, False),
+    (2, 18, 24, (6, 5), 4, 2, 1, 2, True),
+], ids=str)
+def test_weight_gradients_of_odd_planes_and_channels(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed):
+    parts = ("dx",) if stride > 1 and not transposed else ("y",) if transposed else ()      # (through the col matrix)
+    check(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed, parts)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("batch,cin,cout,size,groups", [
+    (1, 16, 16, (256,), 1), (2, 64, 136, (8, 24), 1), (3, 32, 48, (20, 10), 2), (1, 8, 264, (1024,), 1), (5, 24, 8, (4, 6), 1),
+], ids=str)
+def test_weight_gradient_of_one_tap_in_ranges(dtype, batch, cin, cout, size, groups):
+    check(dtype, batch, cin, cout, size, 1, 1, 0, groups, False)
