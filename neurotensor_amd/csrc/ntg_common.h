@@ -380,22 +380,19 @@ struct HaloMap {
     __host__ __device__ int64_t vol() const { return Dp * Hp * Wp; }
     __host__ __device__ int64_t border() const { return vol() - D * H * W; }
 };
-// A weight permutation that the launch of a channels-last copy can take along (its blocks share the elements after
-// their tiles): kind 1 = launch_weights_channels_last(w, wp, rows = a, cg, cgp, taps, chunk), kind 2 =
-// launch_flip_weights_channels_last(w, wp, groups = a, og, ogp, cg, taps, chunk).
-struct WeightsJob { int kind; const void* w; void* wp; int64_t a, og, ogp, cg, cgp, taps, chunk; };
-// With `halo`, pixels go to their places inside the bordered copy.  When the 16-byte kernel serves the copy it also zeroes
-// the border in the same launch, runs `job` (there too, or where the blocks are too few for it in a launch of its own) and
-// sets *took_along; otherwise the caller launches those two itself.
-hipError_t launch_nchw_to_nhwc(int64_t elem_size, const void* in, void* out, int64_t batch, int64_t C, int64_t P, hipStream_t s, const HaloMap* halo = nullptr,
-                               const WeightsJob* job = nullptr, bool* took_along = nullptr);
-hipError_t launch_halo_zero(int64_t elem_size, void* out, int64_t batch, int64_t C, const HaloMap& halo, hipStream_t s);   // zeros the border pixels
-hipError_t launch_weights_channels_last(int64_t es, const void* w, void* wp, int64_t rows, int64_t cg, int64_t cgp, int64_t taps, hipStream_t s, int64_t chunk = 0);
-hipError_t launch_weights_channels_last_rows(int64_t es, const void* w, void* wp, int64_t rows, int64_t cg, int64_t cgp, int64_t k_r, int64_t k_c,
-                                             int64_t kq_pad, hipStream_t s);   // tap rows padded from k_c to kq_pad taps
-hipError_t launch_nchw_to_nhwc_padded(int64_t es, const void* in, void* out, int64_t batch, int64_t groups, int64_t cg, int64_t cgp, int64_t P, hipStream_t s,
-                                      const HaloMap* halo = nullptr);
-hipError_t launch_flip_weights_channels_last(int64_t es, const void* w, void* wt, int64_t groups, int64_t og, int64_t ogp, int64_t cg, int64_t taps, hipStream_t s, int64_t chunk = 0);
+// One launch of channels_last.hip: up to three copies of [batch][groups * cg][P] to [batch][pixel][groups * cgp] (the channels of a group padded with
+// zeros to cgp, whole 16-byte vectors; `bordered`: pixels go to their places inside the border of zero pixels of `halo`), a weight permutation
+// (kinds 1 to 3: see ClWeights; wp in 16-byte vectors) or, with `phases`, the weights and the table of a strided image gradient (kind 4).
+struct ChannelsLastCopy { const void* in; void* out; int64_t batch, groups, cg, cgp, P; bool bordered; HaloMap halo; };
+struct WeightsJob { int kind; const void* w; void* wp; int64_t rows, cg, cgp, taps, other, k_r, k_c, kq_pad, chunk; };
+struct ChannelsLast {
+    ChannelsLastCopy copy[3];
+    int n;
+    WeightsJob weights;
+    const struct PhaseLayout* phases;
+    struct RingItem* items;
+};
+hipError_t launch_channels_last(int64_t elem_size, const ChannelsLast& job, hipStream_t s);
 // channels-last convolution (image [B][pixel][C], weights [O][(r, q, c)]); F16 / BF16 / F32, up to three spatial axes
 hipError_t launch_conv_nhwc(int dtype, const GemmParams& p, hipStream_t s);
 // Image gradient of a strided convolution as one stride-1 convolution per phase of the image (see conv_dimage_phases), up to
@@ -419,7 +416,6 @@ __host__ __device__ static inline int phase_plane(const PhaseLayout& q, int e0, 
 // One product of a launch that computes several convolutions of one bordered channels-last image (phases and groups): what
 // differs from item to item.  Offsets in elements from GemmParams::A / B / C; `first` = first workgroup.
 struct RingItem { int64_t a, b, c; int K, N, ldc, k_d, k_r, k_c, Wo, HoWo, first, tiles_n; FastDiv div_wo, div_howo; };
-hipError_t launch_phase_setup(int64_t es, const void* w, void* wt, RingItem* items, const PhaseLayout& q, hipStream_t s);
 hipError_t launch_phase_interleave(int dtype, const void* tmp, void* im, const PhaseLayout& q, int accumulate, hipStream_t s);
 hipError_t launch_conv_nhwc_items(int dtype, int edge, const GemmParams& p, int64_t blocks, hipStream_t s);
 hipError_t launch_conv_nhwc_dw(int dtype, bool ta, const GemmParams& p, hipStream_t s);   // ta: A (the output gradient) stored [k][m]

@@ -1450,7 +1450,7 @@ static bool conv_nhwc_merged(int dtype, int64_t channels, int64_t out_channels, 
     if (cg <= 0 || cg * es > 32) return false;
     const int64_t cb = cg * es <= 16 ? 16 : 32;
     mt.cgp = cb / es; mt.T = 64 / cb; mt.kq_pad = (g.k[2] + mt.T - 1) / mt.T * mt.T;
-    if (mt.kq_pad > 8 || mt.kq_pad * mt.cgp > 4 * g.k[2] * cg) return false;          // (padding: at most 4x the arithmetic)
+    if (mt.kq_pad > 8 || mt.kq_pad * mt.cgp > 4 * g.k[2] * cg || out_channels * g.k[1] * mt.kq_pad >= 0x7fffffffLL) return false;          // (padding: at most 4x the arithmetic)
     return conv_nhwc_offsets_fit(groups * mt.cgp, es, g);
 }
 static int64_t conv_nhwc_merged_workspace(int dtype, int64_t batch, int64_t out_channels, int64_t groups, const Geo3& g, const MergedTaps& mt) {
@@ -1463,11 +1463,15 @@ static bool conv_nhwc_ok(int dtype, int64_t channels, int64_t out_channels, int6
     const HaloPlan halo = conv_halo(g);
     if (g.nd == 3 && !halo.on) return false;                          // (three axes: the bordered copy is the only form)
     const int64_t es = ntg::elem_size(dtype), cgp = nhwc_padded_channels(es, channels / groups);
-    return cgp > 0 && out_channels > 0 && conv_nhwc_offsets_fit(groups * cgp, es, g) && conv_nhwc_offsets_fit(groups * cgp, es, halo.gp);
+    return cgp > 0 && out_channels > 0 && out_channels * g.taps() < 0x7fffffffLL && conv_nhwc_offsets_fit(groups * cgp, es, g) &&
+           conv_nhwc_offsets_fit(groups * cgp, es, halo.gp);
 }
 static int64_t conv_nhwc_workspace(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
     const int64_t es = ntg::elem_size(dtype), cgp = nhwc_padded_channels(es, channels / groups);
     return (int64_t)align_up((size_t)(batch * groups * cgp * conv_halo(g).vol * es), 256) + out_channels * cgp * g.taps() * es;
+}
+static void add_copy(ntg::ChannelsLast& cl, const void* in, void* out, int64_t batch, int64_t groups, int64_t cg, int64_t cgp, int64_t pixels, const HaloPlan& halo) {
+    cl.copy[cl.n++] = {in, out, batch, groups, cg, cgp, pixels, halo.on, halo.hm};
 }
 static int conv_forward_nhwc(int dtype, const void* image, const void* kernel, void* out, void* ws, int64_t batch, int64_t channels,
                              int64_t out_channels, const Geo3& g, int64_t groups, hipStream_t hs, const MergedTaps* mt = nullptr) {
@@ -1480,21 +1484,13 @@ static int conv_forward_nhwc(int dtype, const void* image, const void* kernel, v
     const bool tap_inner = halo.on && g.s[0] == 1 && g.s[1] == 1 && g.s[2] == 1;   // (neighbouring taps share pixels only at unit strides)
     char* ws_img = static_cast<char*>(ws);
     char* ws_w = ws_img + align_up((size_t)(batch * chp * volp * es), 256);
-    const ntg::HaloMap* hm = halo.on ? &halo.hm : nullptr;
-    // (the 16-byte copy kernel zeroes the border and permutes the weights in the same launch)
     const int64_t wchunk = tap_inner ? 64 / es : 0;                              // (taps inside a 64-byte run of channels)
-    const ntg::WeightsJob wjob = {mt ? 0 : 1, kernel, ws_w, out_channels, 0, 0, cg, cgp, taps, wchunk};
-    bool took_along = false;
-    hipError_t e = cgp == cg ? ntg::launch_nchw_to_nhwc(es, image, ws_img, batch, channels, vol, hs, hm, &wjob, &took_along)
-                             : ntg::launch_nchw_to_nhwc_padded(es, image, ws_img, batch, groups, cg, cgp, vol, hs, hm);
+    ntg::ChannelsLast cl;
+    std::memset(&cl, 0, sizeof cl);
+    add_copy(cl, image, ws_img, batch, groups, cg, cgp, vol, halo);
+    cl.weights = {mt ? 3 : 1, kernel, ws_w, out_channels, cg, cgp, taps, 0, g.k[1], g.k[2], mt ? mt->kq_pad : 0, wchunk};
+    hipError_t e = ntg::launch_channels_last(es, cl, hs);
     if (e != hipSuccess) return hip_fail(e, "channels-last copy launch");
-    if (halo.on && volp != vol && !took_along) {
-        e = ntg::launch_halo_zero(es, ws_img, batch, chp, halo.hm, hs);
-        if (e != hipSuccess) return hip_fail(e, "border fill launch");
-    }
-    if (mt) e = ntg::launch_weights_channels_last_rows(es, kernel, ws_w, out_channels, cg, cgp, g.k[1], g.k[2], mt->kq_pad, hs);
-    else if (!took_along) e = ntg::launch_weights_channels_last(es, kernel, ws_w, out_channels, cg, cgp, taps, hs, wchunk);
-    if (e != hipSuccess) return hip_fail(e, "weight permutation launch");
     ntg::GemmParams p;
     std::memset(&p, 0, sizeof p);
     p.M = (int)og; p.K = (int)K; p.N = (int)L;
@@ -1567,8 +1563,10 @@ static bool conv_dimage_nhwc_ok(int dtype, int64_t channels, int64_t out_channel
 static int64_t conv_dimage_nhwc_workspace(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
     return conv_nhwc_workspace(dtype, batch, out_channels, channels, groups, geo_dimage(g));
 }
+// (the image gradients and the channels-last weight gradient come in two parts, so that a call can make the copies of both in one launch:
+//  with `cl` they only add theirs to it, without it they run on copies that have been made)
 static int conv_dimage_nhwc(int dtype, const void* kernel, const void* grad_out, void* d_image, void* ws, int64_t batch,
-                            int64_t channels, int64_t out_channels, const Geo3& g, int64_t groups, int accumulate, hipStream_t hs) {
+                            int64_t channels, int64_t out_channels, const Geo3& g, int64_t groups, int accumulate, hipStream_t hs, ntg::ChannelsLast* cl) {
     const int64_t es = ntg::elem_size(dtype), cg = channels / groups, og = out_channels / groups;
     const int64_t ogp = nhwc_padded_channels(es, og), ochp = groups * ogp;      // out channels per group / per pixel in the copy
     const int64_t L = g.L(), taps = g.taps(), vol = g.vol(), K = taps * ogp;
@@ -1578,19 +1576,11 @@ static int conv_dimage_nhwc(int dtype, const void* kernel, const void* grad_out,
     const bool tap_inner = halo.on;                                             // (all strides are 1)
     char* ws_gy = static_cast<char*>(ws);
     char* ws_w = ws_gy + align_up((size_t)(batch * ochp * Lp * es), 256);
-    const ntg::HaloMap* hm = halo.on ? &halo.hm : nullptr;
-    const int64_t wchunk = tap_inner ? 64 / es : 0;
-    const ntg::WeightsJob wjob = {2, kernel, ws_w, groups, og, ogp, cg, 0, taps, wchunk};
-    bool took_along = false;                                                    // (border and weight flip inside the copy's launch)
-    hipError_t e = ogp == og ? ntg::launch_nchw_to_nhwc(es, grad_out, ws_gy, batch, out_channels, L, hs, hm, &wjob, &took_along)
-                             : ntg::launch_nchw_to_nhwc_padded(es, grad_out, ws_gy, batch, groups, og, ogp, L, hs, hm);
-    if (e != hipSuccess) return hip_fail(e, "channels-last copy launch");
-    if (halo.on && Lp != L && !took_along) {
-        e = ntg::launch_halo_zero(es, ws_gy, batch, ochp, halo.hm, hs);
-        if (e != hipSuccess) return hip_fail(e, "border fill launch");
+    if (cl) {
+        add_copy(*cl, grad_out, ws_gy, batch, groups, og, ogp, L, halo);
+        cl->weights = {2, kernel, ws_w, channels, og, ogp, taps, cg, 0, 0, 0, tap_inner ? 64 / es : 0};
+        return NTG_OK;
     }
-    if (!took_along) e = ntg::launch_flip_weights_channels_last(es, kernel, ws_w, groups, og, ogp, cg, taps, hs, wchunk);
-    if (e != hipSuccess) return hip_fail(e, "weight flip launch");
     ntg::GemmParams p;
     std::memset(&p, 0, sizeof p);
     p.M = (int)cg; p.K = (int)K; p.N = (int)vol;
@@ -1602,7 +1592,7 @@ static int conv_dimage_nhwc(int dtype, const void* kernel, const void* grad_out,
     p.conv.chan = (int)ochp;
     p.conv.halo = halo.on ? 1 : 0;
     p.conv.tap_inner = tap_inner ? 1 : 0;
-    e = launch_groups(p, dtype, batch, groups, {cg * K, 0, ogp, ochp * Lp, cg * vol}, [&](const ntg::GemmParams& q) { return ntg::launch_conv_nhwc(dtype, q, hs); });
+    const hipError_t e = launch_groups(p, dtype, batch, groups, {cg * K, 0, ogp, ochp * Lp, cg * vol}, [&](const ntg::GemmParams& q) { return ntg::launch_conv_nhwc(dtype, q, hs); });
     if (e != hipSuccess) return hip_fail(e, "channels-last conv_dimage launch");
     return NTG_OK;
 }
@@ -1721,7 +1711,7 @@ static PhasePlan plan_dimage_phases(int dtype, int64_t batch, int64_t channels, 
                 const int64_t n = (int64_t)q.n[0][e0] * q.n[1][e1] * q.n[2][e2];
                 pp.blocks += tiles_m * ((n + q.tile_cols - 1) / q.tile_cols) * batch * groups;
             }
-    if (pp.blocks > 0x7fffffffLL) return pp;
+    if (pp.blocks > 0x7fffffffLL || channels * g.taps() >= 0x7fffffffLL) return pp;
     pp.gy_bytes = (int64_t)align_up((size_t)(batch * ochp * volp * es), 256);
     pp.w_bytes = (int64_t)align_up((size_t)(w_elems * es), 256);
     pp.item_bytes = (int64_t)align_up((size_t)items * sizeof(ntg::RingItem), 256);
@@ -1730,21 +1720,20 @@ static PhasePlan plan_dimage_phases(int dtype, int64_t batch, int64_t channels, 
     return pp;
 }
 static int conv_dimage_phases(int dtype, const PhasePlan& pp, const void* kernel, const void* grad_out, void* d_image, void* ws, int64_t batch,
-                              int64_t channels, int64_t out_channels, const Geo3& g, int64_t groups, int accumulate, hipStream_t hs) {
+                              int64_t channels, const Geo3& g, int64_t groups, int accumulate, hipStream_t hs, ntg::ChannelsLast* cl) {
     const ntg::PhaseLayout& q = pp.lay;
-    const int64_t es = ntg::elem_size(dtype), og = q.og, ogp = q.ogp, ochp = groups * ogp, L = g.L();
+    const int64_t og = q.og, ogp = q.ogp, ochp = groups * ogp;
     char* ws_gy = static_cast<char*>(ws);
     char* ws_w = ws_gy + pp.gy_bytes;
-    char* ws_items = ws_w + pp.w_bytes;
-    char* ws_tmp = ws_items + pp.item_bytes;
-    bool took_along = false;
-    hipError_t e = ogp == og ? ntg::launch_nchw_to_nhwc(es, grad_out, ws_gy, batch, out_channels, L, hs, &pp.hm, nullptr, &took_along)
-                             : ntg::launch_nchw_to_nhwc_padded(es, grad_out, ws_gy, batch, groups, og, ogp, L, hs, &pp.hm);
-    if (e == hipSuccess && pp.hm.border() > 0 && !took_along) e = ntg::launch_halo_zero(es, ws_gy, batch, ochp, pp.hm, hs);
-    if (e != hipSuccess) return hip_fail(e, "channels-last copy launch");
-    ntg::RingItem* items = reinterpret_cast<ntg::RingItem*>(ws_items);
-    e = ntg::launch_phase_setup(es, kernel, ws_w, items, q, hs);
-    if (e != hipSuccess) return hip_fail(e, "phase weight launch");
+    ntg::RingItem* items = reinterpret_cast<ntg::RingItem*>(ws_w + pp.w_bytes);
+    char* ws_tmp = ws_w + pp.w_bytes + pp.item_bytes;
+    if (cl) {
+        cl->copy[cl->n++] = {grad_out, ws_gy, batch, groups, og, ogp, g.L(), true, pp.hm};
+        cl->weights = {4, kernel, ws_w, channels, og, ogp, g.taps(), q.cg, 0, 0, 0, 0};
+        cl->phases = &pp.lay;
+        cl->items = items;
+        return NTG_OK;
+    }
     ntg::GemmParams p;
     std::memset(&p, 0, sizeof p);
     p.M = q.cg; p.batch = (int)batch;
@@ -1759,7 +1748,7 @@ static int conv_dimage_phases(int dtype, const PhasePlan& pp, const void* kernel
     p.conv.halo = 1; p.conv.tap_inner = 1;
     p.conv.items = items; p.conv.n_items = q.phases * (int)groups;
     if (g.nd == 3) p.conv.k_segment = chain_steps(og);
-    e = ntg::launch_conv_nhwc_items(dtype, pp.edge, p, pp.blocks, hs);
+    hipError_t e = ntg::launch_conv_nhwc_items(dtype, pp.edge, p, pp.blocks, hs);
     if (e != hipSuccess) return hip_fail(e, "phase convolution launch");
     e = ntg::launch_phase_interleave(dtype, ws_tmp, d_image, q, accumulate, hs);
     if (e != hipSuccess) return hip_fail(e, "phase interleave launch");
@@ -1876,7 +1865,7 @@ static int64_t conv_dkernel_nhwc_workspace(int dtype, const DkernelPlan& pl, int
            pl.items * rows * cgp * g.taps() * 4;
 }
 static int conv_dkernel_nhwc(int dtype, const DkernelPlan& pl, const void* image, const void* grad_out, void* d_kernel, void* ws, int64_t batch,
-                             int64_t channels, int64_t out_channels, const Geo3& g, int64_t groups, int accumulate, hipStream_t hs) {
+                             int64_t channels, int64_t out_channels, const Geo3& g, int64_t groups, int accumulate, hipStream_t hs, ntg::ChannelsLast* cl) {
     const int64_t es = ntg::elem_size(dtype), bk = 64 / es, cg = channels / groups, og = out_channels / groups;
     const int64_t cgp = dkernel_padded_channels(es, cg), chp = groups * cgp;      // channels per group / per pixel in the copy
     const int64_t ogr = pl.copy_dy ? dkernel_padded_channels(es, og) : og, rows = groups * ogr;     // rows of a group and in all: a copied dY's are whole 16 bytes
@@ -1886,14 +1875,11 @@ static int conv_dkernel_nhwc(int dtype, const DkernelPlan& pl, const void* image
     char* ws_img = static_cast<char*>(ws);
     char* ws_gy = ws_img + align_up((size_t)(batch * chp * volp * es), 256);
     char* ws_part = ws_gy + (pl.copy_dy ? align_up((size_t)(batch * rows * L * es), 256) : 0);
-    const ntg::HaloMap* hm = halo.on ? &halo.hm : nullptr;
-    bool took_along = false;
-    hipError_t e = cgp == cg ? ntg::launch_nchw_to_nhwc(es, image, ws_img, batch, channels, vol, hs, hm, nullptr, &took_along)
-                             : ntg::launch_nchw_to_nhwc_padded(es, image, ws_img, batch, groups, cg, cgp, vol, hs, hm);
-    if (e == hipSuccess && halo.on && volp != vol && !took_along) e = ntg::launch_halo_zero(es, ws_img, batch, chp, halo.hm, hs);
-    if (e == hipSuccess && pl.copy_dy)
-        e = ogr == og ? ntg::launch_nchw_to_nhwc(es, grad_out, ws_gy, batch, out_channels, L, hs) : ntg::launch_nchw_to_nhwc_padded(es, grad_out, ws_gy, batch, groups, og, ogr, L, hs);
-    if (e != hipSuccess) return hip_fail(e, "channels-last copy launch");
+    if (cl) {
+        add_copy(*cl, image, ws_img, batch, groups, cg, cgp, vol, halo);
+        if (pl.copy_dy) cl->copy[cl->n++] = {grad_out, ws_gy, batch, groups, og, ogr, L, false, {}};
+        return NTG_OK;
+    }
     ntg::GemmParams p;
     std::memset(&p, 0, sizeof p);
     p.M = (int)ogr; p.K = (int)(pl.ranges ? pl.kr : L); p.N = (int)N;
@@ -1922,7 +1908,7 @@ static int conv_dkernel_nhwc(int dtype, const DkernelPlan& pl, const void* image
             p.conv.a_image_stride = out_channels * L;
         }
     }
-    e = launch_groups(p, dtype, pl.items, groups, {pl.copy_dy ? ogr : og * L, a_item, cgp, pl.ranges ? 0 : chp * volp, ogr * N},
+    hipError_t e = launch_groups(p, dtype, pl.items, groups, {pl.copy_dy ? ogr : og * L, a_item, cgp, pl.ranges ? 0 : chp * volp, ogr * N},
                       [&](const ntg::GemmParams& q) { return ntg::launch_conv_nhwc_dw(dtype, pl.copy_dy, q, hs); });
     if (e != hipSuccess) return hip_fail(e, "channels-last conv_dkernel launch");
     // (groups are consecutive row blocks of both layouts, so one pass covers them all)
@@ -2026,7 +2012,7 @@ static int conv_dkernel_pointwise(int dtype, const PointwiseDwPlan& pl, const vo
 }
 
 // Which backward gradients run as implicit GEMMs, and the workspace the call needs.
-struct ConvBackwardPlan { bool gather_dw, gather_dx, nhwc_dx, nhwc_dw, phase_dx; int64_t need, need_nhwc_dx, need_nhwc_dw, need_phase_dx, need_wt_dx, wt_offset; PointwiseDwPlan pointwise; PhasePlan phases; DkernelPlan dkernel; };
+struct ConvBackwardPlan { bool gather_dw, gather_dx, nhwc_dx, nhwc_dw, phase_dx; int64_t need, need_both, need_nhwc_dx, need_nhwc_dw, need_phase_dx, need_wt_dx, wt_offset; PointwiseDwPlan pointwise; PhasePlan phases; DkernelPlan dkernel; };
 // reference_order (Float32 through the host entry points): the forms whose sums are the reference's own, bit for bit -- the
 // image gradient as W^T . dY into the col matrix + col2im (conv.cpp:318-346; the implicit forms run one chain over out
 // channels and taps where the reference rounds in between), the weight gradient per image with k = the output pixels +
@@ -2057,6 +2043,10 @@ static ConvBackwardPlan plan_conv_backward_g(int dtype, bool want_dx, bool want_
         pl.phases = plan_dimage_phases(dtype, batch, channels, out_channels, groups, g);
     pl.phase_dx = pl.phases.ok;
     pl.need_phase_dx = pl.phase_dx ? pl.phases.bytes() : 0;
+    // both channels-last gradients with their copies side by side, made in one launch, as long as that is not much memory (the launch it saves is
+    // 1 % of a step from there on)
+    const int64_t both = (int64_t)align_up((size_t)pl.need_nhwc_dw, 256) + std::max(pl.need_nhwc_dx, pl.need_phase_dx);
+    pl.need_both = pl.nhwc_dw && (pl.nhwc_dx || pl.phase_dx) && both <= (1LL << 26) ? both : 0;
     // strides > 1 on few channels: W^T . dY + col2im.  W_g is stored [og][channels of the group * taps]; where those rows miss the
     // 16-byte rule (3 channels by 7 x 7: 147) the product would run on rows as they lie, so W is copied to [..][og] behind the col matrix
     // and dY and col, whose rows keep the rule, stay where they are.  From 2^30 multiply-adds on, where every layer timed gains; us per backward
@@ -2070,6 +2060,53 @@ static ConvBackwardPlan plan_conv_backward_g(int dtype, bool want_dx, bool want_
                     (g.L() * es) % 16 == 0 && (double)batch * (double)(og * add) * (double)g.L() >= 1073741824.0;
     pl.need_wt_dx = wt ? pl.wt_offset + groups * og * add * es : 0;
     return pl;
+}
+
+// The gradients that need no col matrix; d_image / d_kernel are set to null when done.  fast: the channels-last forms may be taken.
+static int conv_gradients_implicit(int dtype, const ConvBackwardPlan& plan, const void* image, const void* kernel, const void* grad_out, void*& d_image, void*& d_kernel,
+                                   char* ws, int64_t ws_bytes, int64_t batch, int64_t channels, int64_t out_channels, const Geo3& g, int64_t groups, int accumulate,
+                                   hipStream_t hs, bool fast) {
+    fast = fast && (reinterpret_cast<uintptr_t>(ws) & 15) == 0;
+    const bool dw = d_kernel && fast && plan.nhwc_dw && ws_bytes >= plan.need_nhwc_dw && (reinterpret_cast<uintptr_t>(grad_out) & 15) == 0;
+    const bool dx = d_image && fast && plan.nhwc_dx && ws_bytes >= plan.need_nhwc_dx, dx_phases = d_image && fast && plan.phase_dx && ws_bytes >= plan.need_phase_dx;
+    const bool together = dw && (dx || dx_phases) && plan.need_both > 0 && ws_bytes >= plan.need_both;
+    char* ws_dx = together ? ws + align_up((size_t)plan.need_nhwc_dw, 256) : ws;
+    ntg::ChannelsLast cl;
+    std::memset(&cl, 0, sizeof cl);
+    const auto dw_part = [&](ntg::ChannelsLast* c) {
+        return conv_dkernel_nhwc(dtype, plan.dkernel, image, grad_out, d_kernel, ws, batch, channels, out_channels, g, groups, accumulate, hs, c);
+    };
+    const auto dx_part = [&](ntg::ChannelsLast* c) {
+        return dx ? conv_dimage_nhwc(dtype, kernel, grad_out, d_image, ws_dx, batch, channels, out_channels, g, groups, accumulate, hs, c)
+                  : conv_dimage_phases(dtype, plan.phases, kernel, grad_out, d_image, ws_dx, batch, channels, g, groups, accumulate, hs, c);
+    };
+    const auto copies = [&]() -> int {
+        const hipError_t e = ntg::launch_channels_last(ntg::elem_size(dtype), cl, hs);
+        return e == hipSuccess ? NTG_OK : hip_fail(e, "channels-last copy launch");
+    };
+    int rc = NTG_OK;
+    if (dw) {
+        dw_part(&cl);
+        if (together) dx_part(&cl);
+        if ((rc = copies()) || (rc = dw_part(nullptr))) return rc;
+    } else if (d_kernel && plan.gather_dw) {
+        rc = conv_dkernel_gather(dtype, image, grad_out, d_kernel, ws, batch, channels, out_channels, g, groups, accumulate, hs);
+        if (rc) return rc;
+    }
+    if (plan.gather_dw) d_kernel = nullptr;
+    if (dx || dx_phases) {
+        if (!together) {
+            std::memset(&cl, 0, sizeof cl);
+            dx_part(&cl);
+            if ((rc = copies())) return rc;
+        }
+        rc = dx_part(nullptr);
+        d_image = nullptr;
+    } else if (d_image && plan.gather_dx) {
+        rc = conv_dimage_gather(dtype, kernel, grad_out, d_image, ws, batch, channels, out_channels, g, groups, accumulate, hs);
+        d_image = nullptr;
+    }
+    return rc;
 }
 
 int64_t ntg_conv2d_fast_workspace_bytes(int dtype, int64_t batch, int64_t channels, int64_t height, int64_t width,
@@ -2262,7 +2299,7 @@ int64_t ntg_conv2d_backward_workspace_bytes(int dtype, int64_t batch, int64_t ch
     // the larger of what the call needs at least and what lets dX take its channels-last form (copy of dY + flipped weights)
     const ConvBackwardPlan pl = plan_conv_backward(dtype, true, true, batch, channels, height, width, out_channels, k_r, k_c, s_r, s_c, p_r, p_c,
                                                    d_r, d_c, groups, Ho, Wo);
-    return std::max({pl.need, pl.need_phase_dx, pl.need_wt_dx, pl.need_nhwc_dx, pl.need_nhwc_dw, pl.pointwise.bytes});
+    return std::max({pl.need, pl.need_phase_dx, pl.need_wt_dx, pl.need_nhwc_dx, pl.need_nhwc_dw, pl.need_both, pl.pointwise.bytes});
 }
 
 static int conv2d_backward_dev_impl(int dtype, const void* image, const void* kernel, const void* grad_out,
@@ -2300,8 +2337,6 @@ static int conv2d_backward_dev_impl(int dtype, const void* image, const void* ke
     char* ws = static_cast<char*>(workspace);
     hipStream_t hs = static_cast<hipStream_t>(stream);
     ntg_gemm_desc d;
-    // Floating dtypes: neither gradient needs the stored im2col matrix (conv_dkernel_gather, conv_dimage_gather).
-    bool gather_dw = plan.gather_dw, gather_dx = plan.gather_dx;
     if (in_place) {
         const int64_t cg = channels / groups;
         if (d_image) {
@@ -2322,27 +2357,8 @@ static int conv2d_backward_dev_impl(int dtype, const void* image, const void* ke
         }
         return NTG_OK;
     }
-    if (gather_dw) {
-        if (plan.nhwc_dw && workspace_bytes >= plan.need_nhwc_dw && ((reinterpret_cast<uintptr_t>(ws) | reinterpret_cast<uintptr_t>(grad_out)) & 15) == 0)
-            rc = conv_dkernel_nhwc(dtype, plan.dkernel, image, grad_out, d_kernel, ws, batch, channels, out_channels, geo, groups, accumulate, hs);
-        else
-            rc = conv_dkernel_gather(dtype, image, grad_out, d_kernel, ws, batch, channels, out_channels, geo, groups, accumulate, hs);
-        if (rc) return rc;
-    }
-    if (gather_dx) {
-        if (plan.nhwc_dx && workspace_bytes >= plan.need_nhwc_dx && (reinterpret_cast<uintptr_t>(ws) & 15) == 0)
-            rc = conv_dimage_nhwc(dtype, kernel, grad_out, d_image, ws, batch, channels, out_channels, geo, groups, accumulate, hs);
-        else
-            rc = conv_dimage_gather(dtype, kernel, grad_out, d_image, ws, batch, channels, out_channels, geo, groups, accumulate, hs);
-        if (rc) return rc;
-    }
-    if (gather_dw) d_kernel = nullptr;    // done
-    if (gather_dx) d_image = nullptr;
-    if (d_image && plan.phase_dx && workspace_bytes >= plan.need_phase_dx && (reinterpret_cast<uintptr_t>(ws) & 15) == 0) {
-        rc = conv_dimage_phases(dtype, plan.phases, kernel, grad_out, d_image, ws, batch, channels, out_channels, geo, groups, accumulate, hs);
-        if (rc) return rc;
-        d_image = nullptr;
-    }
+    rc = conv_gradients_implicit(dtype, plan, image, kernel, grad_out, d_image, d_kernel, ws, workspace_bytes, batch, channels, out_channels, geo, groups, accumulate, hs, true);
+    if (rc) return rc;
     if (d_kernel) {
         // col = im2col(image); per group g:  dW_g [og, add] (+)= sum_b dY_{b,g} [og, L] . col_{b,g}^T  (col_{b,g} stored [add, L])
         rc = ntg_unfold2d_dev(dtype, image, ws, batch, channels, height, width, k_r, k_c, s_r, s_c, p_r, p_c, d_r, d_c, stream);
@@ -2355,7 +2371,10 @@ static int conv2d_backward_dev_impl(int dtype, const void* image, const void* ke
         const bool wt = plan.need_wt_dx > 0 && workspace_bytes >= plan.need_wt_dx &&
                         ((reinterpret_cast<uintptr_t>(ws) | reinterpret_cast<uintptr_t>(grad_out)) & 15) == 0;
         if (wt) {
-            hipError_t e = ntg::launch_nchw_to_nhwc(es, kern, ws + plan.wt_offset, groups, og, add, hs);
+            ntg::ChannelsLast cl;
+            std::memset(&cl, 0, sizeof cl);
+            cl.copy[cl.n++] = {kern, ws + plan.wt_offset, groups, 1, og, og, add, false, {}};
+            const hipError_t e = ntg::launch_channels_last(es, cl, hs);
             if (e != hipSuccess) return hip_fail(e, "transposed weights launch");
         }
         rc = gemm_per_group(dtype, !wt, false, NTG_C_OVERWRITE, add, og, L, wt ? og : add, L, L, batch, groups, wt ? ws + plan.wt_offset : kern, og * add, 0,
@@ -2629,7 +2648,7 @@ int64_t ntg_convnd_fast_workspace_bytes(int dtype, int64_t batch, int64_t channe
     const Geo3 g = geo_from(u);
     if (backward) {
         const ConvBackwardPlan pl = plan_conv_backward_g(dtype, true, true, batch, channels, out_channels, g, groups);
-        const int64_t fast = std::max(pl.need_phase_dx, std::max(pl.need_nhwc_dx, pl.need_nhwc_dw));
+        const int64_t fast = std::max({pl.need_phase_dx, pl.need_nhwc_dx, pl.need_nhwc_dw, pl.need_both});
         return fast > 0 ? std::max(fast, least + 256) : least;        // (more than `least` is what asks for the fast forms)
     }
     return conv_nhwc_ok(dtype, channels, out_channels, groups, g) ? conv_nhwc_workspace(dtype, batch, channels, out_channels, groups, g) : least;
@@ -2712,33 +2731,9 @@ static int convnd_backward_dev_impl(int dtype, const void* image, const void* ke
         // a workspace of ntg_convnd_workspace_bytes asks for the reference's order, even where a fast form would fit into it
         const bool fast = channels_last && workspace_bytes > ntg_convnd_workspace_bytes(dtype, batch, channels, out_channels, ndim, size, kernel_size, stride,
                                                                                         padding, dilation, groups, 1);
-        if (plan.gather_dw) {
-            if (fast && plan.nhwc_dw && workspace_bytes >= plan.need_nhwc_dw &&
-                ((reinterpret_cast<uintptr_t>(workspace) | reinterpret_cast<uintptr_t>(grad_out)) & 15) == 0)
-                rc = conv_dkernel_nhwc(dtype, plan.dkernel, image, grad_out, d_kernel, workspace, batch, channels, out_channels, g, groups, accumulate,
-                                       static_cast<hipStream_t>(stream));
-            else
-                rc = conv_dkernel_gather(dtype, image, grad_out, d_kernel, workspace, batch, channels, out_channels, g, groups, accumulate,
-                                         static_cast<hipStream_t>(stream));
-            if (rc) return rc;
-            d_kernel = nullptr;
-        }
-        if (plan.gather_dx) {
-            if (fast && plan.nhwc_dx && workspace_bytes >= plan.need_nhwc_dx && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0)
-                rc = conv_dimage_nhwc(dtype, kernel, grad_out, d_image, workspace, batch, channels, out_channels, g, groups, accumulate,
-                                      static_cast<hipStream_t>(stream));
-            else
-                rc = conv_dimage_gather(dtype, kernel, grad_out, d_image, workspace, batch, channels, out_channels, g, groups, accumulate,
-                                        static_cast<hipStream_t>(stream));
-            if (rc) return rc;
-            d_image = nullptr;
-        }
-        if (d_image && fast && plan.phase_dx && workspace_bytes >= plan.need_phase_dx && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0) {
-            rc = conv_dimage_phases(dtype, plan.phases, kernel, grad_out, d_image, workspace, batch, channels, out_channels, g, groups, accumulate,
-                                    static_cast<hipStream_t>(stream));
-            if (rc) return rc;
-            d_image = nullptr;
-        }
+        rc = conv_gradients_implicit(dtype, plan, image, kernel, grad_out, d_image, d_kernel, static_cast<char*>(workspace), workspace_bytes, batch, channels,
+                                     out_channels, g, groups, accumulate, static_cast<hipStream_t>(stream), fast);
+        if (rc) return rc;
         if (!d_kernel && !d_image) return NTG_OK;
     }
     if (!workspace || workspace_bytes < need)

@@ -325,332 +325,6 @@ hipError_t launch_flip_weights(int64_t es, const void* w, void* wt, int64_t grou
     return hipGetLastError();
 }
 
-// out[b][p][c] = in[b][c][p]: an image batch from channel planes to channels-last, 64 x 64 tiles through LDS so that
-// both the loads (along p) and the stores (along c) are coalesced.
-// Where pixel p of the source image goes in a copy that carries a border of zero pixels (on == 0: no border, Pp == P): every row
-// skips the Wp - W border pixels beside it, every depth slice the Hp - H border rows
-struct PixRemap { int64_t Pp; FastDiv div_w, div_hw; uint32_t on, row_skip, slice_skip, off0; };
-__device__ __forceinline__ int64_t remap_pixel(const PixRemap& r, int64_t p) {
-    if (!r.on) return p;
-    uint32_t skip = fast_div((uint32_t)p, r.div_w) * r.row_skip + r.off0;      // (a padded image has fewer than 2^31 pixels)
-    if (r.slice_skip) skip += fast_div((uint32_t)p, r.div_hw) * r.slice_skip;   // (uniform)
-    return p + skip;
-}
-static PixRemap make_remap(const HaloMap* h, int64_t P) {
-    PixRemap r;
-    std::memset(&r, 0, sizeof r);
-    r.Pp = P;
-    if (h && h->Wp) {
-        r.Pp = h->vol(); r.on = 1;
-        r.div_w = make_fastdiv((uint32_t)h->W); r.div_hw = make_fastdiv((uint32_t)(h->H * h->W));
-        r.row_skip = (uint32_t)(h->Wp - h->W); r.slice_skip = (uint32_t)((h->Hp - h->H) * h->Wp);
-        r.off0 = (uint32_t)((h->front * h->Hp + h->top) * h->Wp + h->left);
-    }
-    return r;
-}
-
-// zeros the border pixels of a channels-last copy [B][Dp * Hp * Wp][C] (16-byte pieces; C * sizeof(T) a multiple of 16).
-// Only the border is visited: its pixels are numbered front slices, back slices, then slice by slice the top rows, the bottom
-// rows and the left and right pieces of the image's rows.
-// (vectors first, first + step, ... of the per_image 16-byte vectors of one image's border)
-__device__ __forceinline__ void zero_border_vectors(uint4* __restrict__ img, const uint32_t per_image, const uint32_t vec_per_pixel, const HaloMap& h,
-                                                    const uint32_t first, const uint32_t step) {
-    const uint32_t top_n = (uint32_t)(h.top * h.Wp), bot_n = (uint32_t)((h.Hp - h.top - h.H) * h.Wp), side = (uint32_t)(h.Wp - h.W);
-    const uint32_t slice = (uint32_t)(h.Hp * h.Wp), slice_n = slice - (uint32_t)(h.H * h.W);
-    const uint32_t front_n = (uint32_t)h.front * slice, back_n = (uint32_t)(h.Dp - h.front - h.D) * slice;
-    for (uint32_t i = first; i < per_image; i += step) {
-        uint32_t j = i / vec_per_pixel, pix, d0 = 0u;
-        const uint32_t v = i - j * vec_per_pixel;
-        if (h.Dp > 1) {                                               // (uniform)
-            if (j < front_n + back_n) {
-                pix = j < front_n ? j : j + (uint32_t)h.D * slice;
-                img[(int64_t)pix * vec_per_pixel + v] = make_uint4(0u, 0u, 0u, 0u);
-                continue;
-            }
-            j -= front_n + back_n;
-            const uint32_t d = j / slice_n;
-            j -= d * slice_n;
-            d0 = ((uint32_t)h.front + d) * slice;
-        }
-        if (j < top_n) pix = j;
-        else if (j < top_n + bot_n) pix = (uint32_t)((h.top + h.H) * h.Wp) + (j - top_n);
-        else {
-            j -= top_n + bot_n;
-            const uint32_t row = j / side, c = j - row * side;
-            pix = (uint32_t)((h.top + row) * h.Wp) + (c < (uint32_t)h.left ? c : (uint32_t)h.W + c);
-        }
-        img[(int64_t)(d0 + pix) * vec_per_pixel + v] = make_uint4(0u, 0u, 0u, 0u);
-    }
-}
-__global__ void __launch_bounds__(256) halo_zero_kernel(uint4* __restrict__ out, const uint32_t per_image, const uint32_t vec_per_pixel, const HaloMap h) {
-    zero_border_vectors(out + (int64_t)blockIdx.y * h.vol() * vec_per_pixel, per_image, vec_per_pixel, h, blockIdx.x * 256u + threadIdx.x, gridDim.x * 256u);
-}
-hipError_t launch_halo_zero(int64_t es, void* out, int64_t batch, int64_t C, const HaloMap& h, hipStream_t s) {
-    if ((C * es) % 16 != 0 || (reinterpret_cast<uintptr_t>(out) & 15) != 0) return hipErrorInvalidValue;
-    const int64_t vpp = C * es / 16, border = h.border(), per_image = border * vpp;
-    if (batch <= 0 || per_image <= 0) return hipSuccess;
-    if (per_image > 0x7fffffffLL || h.vol() > 0x7fffffffLL) return hipErrorInvalidValue;
-    const int64_t gx = std::min<int64_t>((per_image + 255) / 256, 64);
-    for (int64_t b0 = 0; b0 < batch; b0 += 65535) {
-        const int64_t nb = std::min<int64_t>(batch - b0, 65535);
-        hipLaunchKernelGGL(halo_zero_kernel, dim3((unsigned)gx, (unsigned)nb), dim3(256), 0, s,
-                           (uint4*)out + b0 * h.vol() * vpp, (uint32_t)per_image, (uint32_t)vpp, h);
-    }
-    return hipGetLastError();
-}
-
-template <class T>
-__global__ void __launch_bounds__(256) nchw_to_nhwc_kernel(const T* __restrict__ in, T* __restrict__ out, const int64_t C, const int64_t P, const PixRemap r) {
-    __shared__ T tile[64][65];
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    const int64_t p0 = (int64_t)blockIdx.x * 64, c0 = (int64_t)blockIdx.y * 64, b = blockIdx.z;
-    const T* src = in + b * C * P;
-    T* dst = out + b * C * r.Pp;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int64_t c = c0 + ty + 4 * i, pp = p0 + tx;
-        if (c < C && pp < P) tile[ty + 4 * i][tx] = src[c * P + pp];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int64_t pp = p0 + ty + 4 * i, c = c0 + tx;
-        if (c < C && pp < P) dst[remap_pixel(r, pp) * C + c] = tile[tx][ty + 4 * i];
-    }
-}
-
-// element idx of the two weight permutations (see weights_channels_last_kernel, flip_weights_channels_last_kernel)
-template <class T>
-__device__ __forceinline__ void weights_channels_last_elem(const T* __restrict__ w, T* __restrict__ wp, const int64_t idx, const int64_t cg, const int64_t cgp,
-                                                           const int64_t taps, const int64_t chunk) {
-    const int64_t c = idx % cgp;
-    const int64_t t = (idx / cgp) % taps;
-    const int64_t o = idx / (cgp * taps);
-    // chunk != 0: the k order (run of `chunk` channels, tap, channel inside the run) instead of (tap, channel)
-    const int64_t dst = chunk ? o * taps * cgp + ((c / chunk) * taps + t) * chunk + c % chunk : idx;
-    wp[dst] = c < cg ? w[(o * cg + c) * taps + t] : (T)0;
-}
-template <class T>
-__device__ __forceinline__ void flip_weights_channels_last_elem(const T* __restrict__ w, T* __restrict__ wt, const int64_t idx, const int64_t og, const int64_t ogp,
-                                                                const int64_t cg, const int64_t taps, const int64_t chunk) {
-    const int64_t oc = idx % ogp;
-    int64_t r = idx / ogp;
-    const int64_t t = r % taps;
-    r /= taps;
-    const int64_t c = r % cg;
-    const int64_t g = r / cg;
-    // chunk != 0: the k order (run of `chunk` out channels, tap, out channel inside the run) instead of (tap, out channel)
-    const int64_t dst = chunk ? r * taps * ogp + ((oc / chunk) * taps + t) * chunk + oc % chunk : idx;
-    wt[dst] = oc < og ? w[((g * og + oc) * cg + c) * taps + (taps - 1 - t)] : (T)0;
-}
-// what a channels-last copy takes along: the border of zero pixels of its own output and a weight permutation
-struct CopyExtras { HaloMap h; uint32_t border_vecs, vpp; WeightsJob job; int64_t job_total; };
-
-// The same copy with 16-byte accesses on both sides (C and P multiples of one 16-byte vector, aligned pointers): a
-// thread loads VEC pixels of one channel, the tile goes through LDS as single elements (row pitch chosen so that the
-// column-wise read-back spreads over the banks), and a thread stores VEC channels of one pixel.
-template <class T>
-__global__ void __launch_bounds__(256) nchw_to_nhwc_vec_kernel(const T* __restrict__ in, T* __restrict__ out, const int64_t C, const int64_t P, const PixRemap r,
-                                                               const CopyExtras ex) {
-    constexpr int VEC = 16 / (int)sizeof(T), VPR = 64 / VEC;            // elements per vector, vectors per tile row
-    constexpr int PITCH = sizeof(T) == 2 ? 66 : 65;                     // elements: 33 / 65 words
-    typedef T TV __attribute__((ext_vector_type(VEC)));
-    __shared__ T tile[64 * PITCH];
-    const int64_t p0 = (int64_t)blockIdx.x * 64, c0 = (int64_t)blockIdx.y * 64, b = blockIdx.z;
-    const T* src = in + b * C * P;
-    T* dst = out + b * C * r.Pp;
-#pragma unroll
-    for (int i = 0; i < 64 * VPR / 256; ++i) {
-        const int v = threadIdx.x + 256 * i, c = v / VPR, pv = v % VPR;
-        if (c0 + c < C && p0 + pv * VEC < P) {
-            const TV x = *reinterpret_cast<const TV*>(src + (c0 + c) * P + p0 + pv * VEC);
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) tile[c * PITCH + pv * VEC + e] = x[e];
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 64 * VPR / 256; ++i) {
-        const int v = threadIdx.x + 256 * i, pp = v / VPR, cv = v % VPR;
-        if (c0 + cv * VEC < C && p0 + pp < P) {
-            TV x;
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) x[e] = tile[(cv * VEC + e) * PITCH + pp];
-            *reinterpret_cast<TV*>(dst + remap_pixel(r, p0 + pp) * C + c0 + cv * VEC) = x;
-        }
-    }
-    // the blocks of an image share its border, all blocks of the launch the weight permutation (a few elements each)
-    const uint32_t per_image = gridDim.x * gridDim.y, bid = blockIdx.y * gridDim.x + blockIdx.x;
-    if (ex.border_vecs)
-        zero_border_vectors(reinterpret_cast<uint4*>(dst), ex.border_vecs, ex.vpp, ex.h, bid * 256u + threadIdx.x, per_image * 256u);
-    if (ex.job.kind) {
-        const int64_t step = (int64_t)gridDim.z * per_image * 256;
-        for (int64_t idx = ((int64_t)blockIdx.z * per_image + bid) * 256 + threadIdx.x; idx < ex.job_total; idx += step) {
-            if (ex.job.kind == 1) weights_channels_last_elem<T>((const T*)ex.job.w, (T*)ex.job.wp, idx, ex.job.cg, ex.job.cgp, ex.job.taps, ex.job.chunk);
-            else flip_weights_channels_last_elem<T>((const T*)ex.job.w, (T*)ex.job.wp, idx, ex.job.og, ex.job.ogp, ex.job.cg, ex.job.taps, ex.job.chunk);
-        }
-    }
-}
-
-hipError_t launch_nchw_to_nhwc(int64_t es, const void* in, void* out, int64_t batch, int64_t C, int64_t P, hipStream_t s, const HaloMap* halo,
-                               const WeightsJob* job, bool* took_along) {
-    if (took_along) *took_along = false;
-    if (batch * C * P == 0) return hipSuccess;
-    const PixRemap r = make_remap(halo, P);
-    const int64_t gx = (P + 63) / 64, gy = (C + 63) / 64;
-    if (gx > 0x7fffffffLL || gy > 65535) return hipErrorInvalidValue;
-    const int64_t vec = 16 / es;
-    const bool vec_ok = C % vec == 0 && P % vec == 0 && ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
-    CopyExtras ex;
-    std::memset(&ex, 0, sizeof ex);
-    if (vec_ok && (es == 2 || es == 4) && took_along) {
-        // (the caller acts on *took_along: without it the copy stays what it was)
-        const int64_t vpp = C * es / 16, border = halo && halo->Wp ? halo->border() : 0;
-        if (border * vpp <= 0x7fffffffLL && (!halo || halo->vol() <= 0x7fffffffLL)) {
-            if (border > 0) { ex.h = *halo; ex.border_vecs = (uint32_t)(border * vpp); ex.vpp = (uint32_t)vpp; }
-            if (job && job->kind) {
-                ex.job = *job;
-                ex.job_total = job->kind == 1 ? job->a * job->cgp * job->taps : job->a * job->ogp * job->cg * job->taps;
-                // Small images have few blocks, and an element is a chain of divisions and a strided read, about 0.55 us: eight a thread
-                // take as long as a launch, beyond that the permutation goes out on its own (Float32 1 x 512 x 4 x 4 x 4 -> 128
-                // channels by 3 x 3 x 3, eight blocks: 864 elements a thread, image gradient 1960 us; on its own 84 us).
-                if (ex.job_total > 8 * 256 * gx * gy * std::min<int64_t>(batch, 65535)) {
-                    const WeightsJob& j = *job;
-                    const hipError_t e = j.kind == 1 ? launch_weights_channels_last(es, j.w, j.wp, j.a, j.cg, j.cgp, j.taps, s, j.chunk)
-                                                     : launch_flip_weights_channels_last(es, j.w, j.wp, j.a, j.og, j.ogp, j.cg, j.taps, s, j.chunk);
-                    if (e != hipSuccess) return e;
-                    ex.job.kind = 0;
-                }
-            }
-            *took_along = true;
-        }
-    }
-    for (int64_t b0 = 0; b0 < batch; b0 += 65535) {                    // (grid z limit)
-        const int64_t nb = batch - b0 < 65535 ? batch - b0 : 65535;
-        const dim3 g((unsigned)gx, (unsigned)gy, (unsigned)nb), t(256);
-        const char* src = static_cast<const char*>(in) + b0 * C * P * es;
-        char* dst = static_cast<char*>(out) + b0 * C * r.Pp * es;
-        if (es == 2 && vec_ok) hipLaunchKernelGGL(nchw_to_nhwc_vec_kernel<uint16_t>, g, t, 0, s, (const uint16_t*)src, (uint16_t*)dst, C, P, r, ex);
-        else if (es == 4 && vec_ok) hipLaunchKernelGGL(nchw_to_nhwc_vec_kernel<uint32_t>, g, t, 0, s, (const uint32_t*)src, (uint32_t*)dst, C, P, r, ex);
-        else if (es == 2) hipLaunchKernelGGL(nchw_to_nhwc_kernel<uint16_t>, g, t, 0, s, (const uint16_t*)src, (uint16_t*)dst, C, P, r);
-        else if (es == 4) hipLaunchKernelGGL(nchw_to_nhwc_kernel<uint32_t>, g, t, 0, s, (const uint32_t*)src, (uint32_t*)dst, C, P, r);
-        else return hipErrorInvalidValue;
-        ex.job.kind = 0;                                               // (the first launch has done the weights)
-    }
-    return hipGetLastError();
-}
-
-// wt[g][c][t][oc] = w[g*og + oc][c][taps-1-t]: the weights of the convolution that maps the output gradient back to the
-// image (channel axes swapped inside each group, taps reversed), with the out channels of one tap consecutive and
-// padded with zeros from og to ogp per tap.
-template <class T>
-__global__ void __launch_bounds__(256) flip_weights_channels_last_kernel(const T* __restrict__ w, T* __restrict__ wt, const int64_t groups,
-                                                                         const int64_t og, const int64_t ogp, const int64_t cg, const int64_t taps,
-                                                                         const int64_t chunk) {
-    const int64_t total = groups * ogp * cg * taps;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += stride)
-        flip_weights_channels_last_elem<T>(w, wt, idx, og, ogp, cg, taps, chunk);
-}
-
-hipError_t launch_flip_weights_channels_last(int64_t es, const void* w, void* wt, int64_t groups, int64_t og, int64_t ogp, int64_t cg, int64_t taps, hipStream_t s,
-                                             int64_t chunk) {
-    const int64_t total = groups * ogp * cg * taps;
-    if (total == 0) return hipSuccess;
-    const dim3 g(grid_for(total)), t(256);
-    switch (es) {
-    case 2: hipLaunchKernelGGL(flip_weights_channels_last_kernel<uint16_t>, g, t, 0, s, (const uint16_t*)w, (uint16_t*)wt, groups, og, ogp, cg, taps, chunk); break;
-    case 4: hipLaunchKernelGGL(flip_weights_channels_last_kernel<uint32_t>, g, t, 0, s, (const uint32_t*)w, (uint32_t*)wt, groups, og, ogp, cg, taps, chunk); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
-// Weights of all phases of a strided convolution's image gradient, and the table of their products.  Phase e has the taps
-// e + s (M - 1 - m) of w [g*og + oc][c][taps], reversed, as wt[g][c][(run, m0, m1, m2, oc in run)] with the out channels padded with
-// zeros from og to ogp and in runs of `chunk` (see ConvGeom::tap_inner).  One thread per (group, image channel, tap, out channel):
-// every tap belongs to one phase.  The table, one thread an item, is the work of the blocks behind those of the weights: an item is a
-// walk over the phases and four 64-bit divisions, which behind a weight of its own was the kernel's whole length; index arithmetic in
-// 32 bits (I) where the weights allow it, as a 64-bit division is some hundred instructions and a weight takes three
-// (Float16 128 x 64 x 4 x 4 at stride 2: 9.5 -> 8.2 us, the rest the latency of its strided reads).
-template <class T, class I>
-__global__ void __launch_bounds__(256) phase_setup_kernel(const T* __restrict__ w, T* __restrict__ wt, RingItem* __restrict__ items, const PhaseLayout q,
-                                                          const uint32_t weight_blocks) {
-    const int taps = q.k[0] * q.k[1] * q.k[2];
-    const int64_t total = (int64_t)q.groups * q.cg * taps * q.ogp;
-    const int64_t stride = (int64_t)weight_blocks * 256;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; blockIdx.x < weight_blocks && i < total; i += stride) {
-        const I idx = (I)i, row = idx / (I)q.ogp, gc = row / (I)taps;
-        const int oc = (int)(idx - row * (I)q.ogp);
-        int tap = (int)(row - gc * (I)taps);
-        const int src_tap = tap;
-        const int64_t r = (int64_t)gc;                                 // g * cg + c
-        int e[3], m[3];
-#pragma unroll
-        for (int a = 2; a >= 0; --a) {
-            const int i = tap % q.k[a];
-            tap /= q.k[a];
-            e[a] = i % q.s[a];
-            m[a] = q.M[a][e[a]] - 1 - i / q.s[a];
-        }
-        const int ph = (e[0] * q.s[1] + e[1]) * q.s[2] + e[2];
-        if (q.plane_off[ph] < 0) continue;
-        const int ptaps = q.M[0][e[0]] * q.M[1][e[1]] * q.M[2][e[2]], t = (m[0] * q.M[1][e[1]] + m[1]) * q.M[2][e[2]] + m[2];
-        const int64_t g = (int64_t)(gc / (I)q.cg), c = r - g * q.cg;
-        wt[q.w_off[ph] + r * ptaps * q.ogp + ((int64_t)(oc / q.chunk) * ptaps + t) * q.chunk + oc % q.chunk] =
-            oc < q.og ? w[((g * q.og + oc) * q.cg + c) * taps + src_tap] : (T)0;
-    }
-    // item (live phase, group)
-    if (blockIdx.x < weight_blocks) return;
-    const int64_t i = (int64_t)(blockIdx.x - weight_blocks) * 256 + threadIdx.x;
-    if (i < (int64_t)q.phases * q.groups) {
-        const int want = (int)(i / q.groups), g = (int)(i % q.groups);
-        const int tiles_m = (q.cg + q.tile_rows - 1) / q.tile_rows;
-        int64_t start = 0;
-        int live = 0;
-        for (int ph = 0; ph < q.s[0] * q.s[1] * q.s[2]; ++ph) {
-            if (q.plane_off[ph] < 0) continue;
-            const int e2 = ph % q.s[2], e1 = ph / q.s[2] % q.s[1], e0 = ph / (q.s[2] * q.s[1]);
-            const int N = q.n[0][e0] * q.n[1][e1] * q.n[2][e2], tiles_n = (N + q.tile_cols - 1) / q.tile_cols;
-            const int64_t per_group = (int64_t)tiles_m * tiles_n * q.batch;
-            if (live++ < want) { start += per_group * q.groups; continue; }
-            const int ptaps = q.M[0][e0] * q.M[1][e1] * q.M[2][e2], ochp = q.groups * q.ogp;
-            RingItem it;
-            it.K = ptaps * q.ogp; it.N = N; it.ldc = phase_plane(q, e0, e1, e2);
-            it.a = q.w_off[ph] + (int64_t)g * q.cg * it.K;
-            it.b = (((int64_t)q.org[0][e0] * q.yp[1] + q.org[1][e1]) * q.yp[2] + q.org[2][e2]) * ochp + (int64_t)g * q.ogp;
-            it.c = q.plane_off[ph] + (int64_t)g * q.cg * it.ldc;
-            it.k_d = q.M[0][e0]; it.k_r = q.M[1][e1]; it.k_c = q.M[2][e2];
-            it.Wo = q.n[2][e2]; it.HoWo = q.n[1][e1] * q.n[2][e2];
-            it.first = (int)(start + per_group * g); it.tiles_n = tiles_n;
-            it.div_wo = make_fastdiv((uint32_t)it.Wo); it.div_howo = make_fastdiv((uint32_t)it.HoWo);
-            items[i] = it;
-            break;
-        }
-    }
-}
-
-hipError_t launch_phase_setup(int64_t es, const void* w, void* wt, RingItem* items, const PhaseLayout& q, hipStream_t s) {
-    const int64_t total = (int64_t)q.groups * q.cg * q.k[0] * q.k[1] * q.k[2] * q.ogp;
-    const uint32_t wb = (uint32_t)grid_for(total);
-    const int64_t ib = ((int64_t)q.phases * q.groups + 255) / 256;
-    if (ib > 0x3fffffffLL) return hipErrorInvalidValue;
-    const dim3 g(wb + (uint32_t)ib), t(256);
-    const bool narrow = total <= 0x7fffffffLL;
-    switch (es) {
-    case 2:
-        if (narrow) hipLaunchKernelGGL((phase_setup_kernel<uint16_t, uint32_t>), g, t, 0, s, (const uint16_t*)w, (uint16_t*)wt, items, q, wb);
-        else hipLaunchKernelGGL((phase_setup_kernel<uint16_t, int64_t>), g, t, 0, s, (const uint16_t*)w, (uint16_t*)wt, items, q, wb);
-        break;
-    case 4:
-        if (narrow) hipLaunchKernelGGL((phase_setup_kernel<uint32_t, uint32_t>), g, t, 0, s, (const uint32_t*)w, (uint32_t*)wt, items, q, wb);
-        else hipLaunchKernelGGL((phase_setup_kernel<uint32_t, int64_t>), g, t, 0, s, (const uint32_t*)w, (uint32_t*)wt, items, q, wb);
-        break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
 // im[b][c][z][y][x] (+)= the element of the phase plane that holds it: phase e = (position + p) % s per axis stores the image
 // positions s (a0 + a) + e - p as its positions a; phases without taps contribute zero.  A thread does V consecutive elements of
 // an image row (16 bytes in one store where the rows allow it): the divisions are made once per row piece and the column phase
@@ -746,133 +420,6 @@ hipError_t launch_phase_interleave(int dtype, const void* tmp, void* im, const P
     case DT_BF16: return launch_phase_interleave_t<__bf16>(tmp, im, q, accumulate, s);
     default: return hipErrorInvalidValue;
     }
-}
-
-// wp[o][t][c] = w[o][c][t]: convolution weights with the channel index fastest (the k order of the channels-last gather),
-// the channels of one tap padded with zeros from cg to cgp
-template <class T>
-__global__ void __launch_bounds__(256) weights_channels_last_kernel(const T* __restrict__ w, T* __restrict__ wp, const int64_t rows,
-                                                                    const int64_t cg, const int64_t cgp, const int64_t taps, const int64_t chunk) {
-    const int64_t total = rows * cgp * taps;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += stride)
-        weights_channels_last_elem<T>(w, wp, idx, cg, cgp, taps, chunk);
-}
-
-hipError_t launch_weights_channels_last(int64_t es, const void* w, void* wp, int64_t rows, int64_t cg, int64_t cgp, int64_t taps, hipStream_t s, int64_t chunk) {
-    const int64_t total = rows * cgp * taps;
-    if (total == 0) return hipSuccess;
-    const dim3 g(grid_for(total)), t(256);
-    switch (es) {
-    case 2: hipLaunchKernelGGL(weights_channels_last_kernel<uint16_t>, g, t, 0, s, (const uint16_t*)w, (uint16_t*)wp, rows, cg, cgp, taps, chunk); break;
-    case 4: hipLaunchKernelGGL(weights_channels_last_kernel<uint32_t>, g, t, 0, s, (const uint32_t*)w, (uint32_t*)wp, rows, cg, cgp, taps, chunk); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
-// wp[o][r][q][c] = w[o][c][r][q] with every tap row padded with zeros from k_c to kq_pad taps and the channels from cg to cgp
-template <class T>
-__global__ void __launch_bounds__(256) weights_channels_last_rows_kernel(const T* __restrict__ w, T* __restrict__ wp, const int64_t rows, const int64_t cg,
-                                                                         const int64_t cgp, const int64_t k_r, const int64_t k_c, const int64_t kq_pad) {
-    const int64_t total = rows * k_r * kq_pad * cgp;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += stride) {
-        const int64_t c = idx % cgp;
-        int64_t t = idx / cgp;
-        const int64_t q = t % kq_pad;
-        t /= kq_pad;
-        const int64_t r = t % k_r, o = t / k_r;
-        wp[idx] = (c < cg && q < k_c) ? w[((o * cg + c) * k_r + r) * k_c + q] : (T)0;
-    }
-}
-
-hipError_t launch_weights_channels_last_rows(int64_t es, const void* w, void* wp, int64_t rows, int64_t cg, int64_t cgp, int64_t k_r, int64_t k_c,
-                                             int64_t kq_pad, hipStream_t s) {
-    const int64_t total = rows * k_r * kq_pad * cgp;
-    if (total == 0) return hipSuccess;
-    const dim3 g(grid_for(total)), t(256);
-    switch (es) {
-    case 2: hipLaunchKernelGGL(weights_channels_last_rows_kernel<uint16_t>, g, t, 0, s, (const uint16_t*)w, (uint16_t*)wp, rows, cg, cgp, k_r, k_c, kq_pad); break;
-    case 4: hipLaunchKernelGGL(weights_channels_last_rows_kernel<uint32_t>, g, t, 0, s, (const uint32_t*)w, (uint32_t*)wp, rows, cg, cgp, k_r, k_c, kq_pad); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
-// out[b][p][g*cgp + c] = in[b][g*cg + c][p] for c < cg, 0 for cg <= c < cgp: the channels-last copy with the channels of
-// every group padded to cgp.  64 x 64 tiles of (channel inside the group, pixel) through LDS, like the plain copy.
-template <class T>
-__global__ void __launch_bounds__(256) nchw_to_nhwc_pad_kernel(const T* __restrict__ in, T* __restrict__ out, const int64_t groups,
-                                                               const int64_t cg, const int64_t cgp, const int64_t P, const int cblocks, const PixRemap r) {
-    __shared__ T tile[64][65];
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    const int64_t g = blockIdx.y / cblocks, c0 = (int64_t)(blockIdx.y % cblocks) * 64;
-    const int64_t p0 = (int64_t)blockIdx.x * 64, b = blockIdx.z;
-    const T* src = in + (b * groups + g) * cg * P;
-    T* dst = out + b * r.Pp * groups * cgp + g * cgp;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int64_t c = c0 + ty + 4 * i, pp = p0 + tx;
-        tile[ty + 4 * i][tx] = (c < cg && pp < P) ? src[c * P + pp] : (T)0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int64_t pp = p0 + ty + 4 * i, c = c0 + tx;
-        if (c < cgp && pp < P) dst[remap_pixel(r, pp) * groups * cgp + c] = tile[tx][ty + 4 * i];
-    }
-}
-
-// The same for groups of at most 32 bytes of channels (padded to 16 or 32 bytes): one thread per pixel and group reads its
-// cg channels (each a coalesced stream over the pixels) and stores the padded run with 16-byte stores.
-template <class T, int CP>
-__global__ void __launch_bounds__(256) nchw_to_nhwc_few_kernel(const T* __restrict__ in, T* __restrict__ out, const int64_t total, const int64_t groups,
-                                                               const int64_t cg, const int64_t P, const PixRemap r) {
-    constexpr int VEC = 16 / (int)sizeof(T);
-    typedef T TV __attribute__((ext_vector_type(VEC)));
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= total) return;
-    const int64_t pp = idx % P, bg = idx / P, b = bg / groups, g = bg - b * groups;
-    const T* src = in + bg * cg * P + pp;
-    TV* dst = reinterpret_cast<TV*>(out + ((b * r.Pp + remap_pixel(r, pp)) * groups + g) * CP);
-#pragma unroll
-    for (int v = 0; v < CP / VEC; ++v) {
-        TV x;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) x[e] = (v * VEC + e) < cg ? src[(int64_t)(v * VEC + e) * P] : (T)0;
-        dst[v] = x;
-    }
-}
-
-hipError_t launch_nchw_to_nhwc_padded(int64_t es, const void* in, void* out, int64_t batch, int64_t groups, int64_t cg, int64_t cgp, int64_t P, hipStream_t s,
-                                      const HaloMap* halo) {
-    if (batch * groups * cgp * P == 0) return hipSuccess;
-    const PixRemap r = make_remap(halo, P);
-    if (cgp * es <= 32 && (cgp * es) % 16 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
-        const int64_t total = batch * groups * P, blocks = (total + 255) / 256;
-        if (blocks <= 0x7fffffffLL) {
-            const dim3 g((unsigned)blocks), t(256);
-            if (es == 2 && cgp == 8) hipLaunchKernelGGL((nchw_to_nhwc_few_kernel<uint16_t, 8>), g, t, 0, s, (const uint16_t*)in, (uint16_t*)out, total, groups, cg, P, r);
-            else if (es == 2) hipLaunchKernelGGL((nchw_to_nhwc_few_kernel<uint16_t, 16>), g, t, 0, s, (const uint16_t*)in, (uint16_t*)out, total, groups, cg, P, r);
-            else if (es == 4 && cgp == 4) hipLaunchKernelGGL((nchw_to_nhwc_few_kernel<uint32_t, 4>), g, t, 0, s, (const uint32_t*)in, (uint32_t*)out, total, groups, cg, P, r);
-            else if (es == 4) hipLaunchKernelGGL((nchw_to_nhwc_few_kernel<uint32_t, 8>), g, t, 0, s, (const uint32_t*)in, (uint32_t*)out, total, groups, cg, P, r);
-            else return hipErrorInvalidValue;
-            return hipGetLastError();
-        }
-    }
-    const int64_t cblocks = (cgp + 63) / 64, gx = (P + 63) / 64, gy = cblocks * groups;
-    if (gx > 0x7fffffffLL || gy > 65535) return hipErrorInvalidValue;
-    for (int64_t b0 = 0; b0 < batch; b0 += 65535) {                    // (grid z limit)
-        const int64_t nb = batch - b0 < 65535 ? batch - b0 : 65535;
-        const dim3 g((unsigned)gx, (unsigned)gy, (unsigned)nb), t(256);
-        const char* src = static_cast<const char*>(in) + b0 * groups * cg * P * es;
-        char* dst = static_cast<char*>(out) + b0 * groups * cgp * r.Pp * es;
-        if (es == 2) hipLaunchKernelGGL(nchw_to_nhwc_pad_kernel<uint16_t>, g, t, 0, s, (const uint16_t*)src, (uint16_t*)dst, groups, cg, cgp, P, (int)cblocks, r);
-        else if (es == 4) hipLaunchKernelGGL(nchw_to_nhwc_pad_kernel<uint32_t>, g, t, 0, s, (const uint32_t*)src, (uint32_t*)dst, groups, cg, cgp, P, (int)cblocks, r);
-        else return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
 }
 
 }  // namespace ntg

@@ -143,3 +143,33 @@ def test_weight_gradients_of_odd_planes_and_channels(dtype, batch, cin, cout, si
 ], ids=str)
 def test_weight_gradient_of_one_tap_in_ranges(dtype, batch, cin, cout, size, groups):
     check(dtype, batch, cin, cout, size, 1, 1, 0, groups, False)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32], ids=["f16", "f32"])
+@pytest.mark.parametrize("batch,cin,cout,size,kernel,stride,pad,groups,transposed", [
+    (3, 64, 64, (9, 15), 3, 1, 1, 1, False),         # planes that miss 16 bytes: the last piece of a row element by element
+    (2, 72, 72, (63,), 5, 1, 2, 1, False),           # a tile and a part in each direction
+    (2, 65, 70, (13, 5), 3, 1, 3, 5, False),         # padded channels of five groups in one tile, a border wider than the window
+    (4, 3, 64, (10, 9), 5, 1, 2, 1, False),          # a thread a pixel
+    (1, 5, 16, (300,), 7, 2, 3, 1, False),
+    (2, 64, 64, (3, 4, 5), 3, 1, 1, 1, False),       # slices in front and behind
+    (2, 32, 64, (7, 6, 5), 3, 3, 1, 2, False),       # phases of stride 3: their weights and table beside the copies
+    (1, 64, 48, (2, 3), 4, 4, 0, 1, True),
+], ids=str)
+def test_copies_borders_and_weights_in_one_launch(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed):
+    parts = ("dx",) if stride > 1 and not transposed else ()
+    check(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed, parts)
+
+
+def test_tensors_at_any_element_of_a_buffer():
+    """Images, weights and gradients two bytes off any alignment."""
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    x, w, dy = (torch.randn(s, generator=gen, device="cuda").to(torch.bfloat16) for s in ((2, 40, 12, 12), (24, 40, 3, 3), (2, 24, 12, 12)))
+    off = []
+    for t in (x, w, dy):
+        buf = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")
+        buf[1:].copy_(t.flatten())
+        off.append(buf[1:].view(t.shape))
+    assert torch.equal(F.conv2d(off[0], off[1], padding=1), F.conv2d(x, w, padding=1))
+    dx, _ = F.conv2d_backward(*off, padding=1)
+    assert torch.equal(dx, F.conv2d_backward(x, w, dy, padding=1)[0])
