@@ -7,6 +7,8 @@ conditions follow the reference (lines cited at each check); errors surface as
 ValueError where the reference throws from utils::throw_exception.
 """
 import ctypes
+import importlib.util
+import os
 
 import torch
 
@@ -39,6 +41,27 @@ else:
     def _stream():
         """The current stream's handle."""
         return _cuda_getCurrentRawStream(_cuda_getDevice())
+
+
+def _load_native():
+    """lib/_face.so: the usual calls in one native call each (face/face.cpp).  Without it everything goes the general ways below."""
+    path = os.path.join(os.path.dirname(_lib.LIB_PATH), "_face.so")
+    if not os.path.exists(path):
+        return None
+    spec = importlib.util.spec_from_file_location("neurotensor_amd._face", path)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    return module
+
+
+_face = _load_native()
+
+
+def _done(result):
+    """What a native call returned (not None): tensors, or the status of a call that failed."""
+    if result.__class__ is int:
+        check(result)
+    return result
 
 
 def _require_device(*ts):
@@ -94,20 +117,15 @@ def matmult(a, b, out=None, transpose_a=False, transpose_b=False, accumulate=Non
     Without `out`: returns op(a).op(b) (the reference allocates zeros and accumulates,
     matmult_cpu.cpp:110, :707; here the kernel overwrites, which is the same result).
     With `out`: out += op(a).op(b) -- the accumulate contract (matmult_cpu.cpp:123-153)."""
+    if out is None and _face is not None and a.is_cuda:
+        c = _face.gemm(a, b, None, bool(transpose_a), bool(transpose_b), False, _stream())
+        if c is not None:
+            return _done(c)
     _require_device(a, b)
     if a.dim() < 2 or b.dim() < 2:
         raise ValueError(f"Expected tensors to have dims greater than 1, but instead had dims of {a.dim()} and {b.dim()}")
     if a.dtype != b.dtype:
         raise ValueError(f"Expected both tensors to have the same dtype but got {a.dtype} and {b.dtype}")   # :868
-    if out is None and a.dim() == 2 and b.dim() == 2:
-        # two matrices: what the rules below come down to, without their bookkeeping
-        a_st, ta = _as_matrix_view(a, bool(transpose_a))
-        b_st, tb = _as_matrix_view(b, bool(transpose_b))
-        m, k, n = _logical(a_st.shape, b_st.shape, ta, tb)
-        c = torch.empty((m, n), dtype=a.dtype, device=a.device)
-        if m and n:
-            _launch(a_st, b_st, c, m, k, n, ta, tb, 1, m * k, k * n, m * n, _lib.C_OVERWRITE)
-        return c
     a_st, ta = _as_matrix_view(a, bool(transpose_a))
     b_st, tb = _as_matrix_view(b, bool(transpose_b))
     m, k, n = _logical(a_st.shape, b_st.shape, ta, tb)
@@ -188,6 +206,10 @@ def relu_(x):
 def linear(x, w, bias, transpose_a=False, transpose_b=False, _relu=False):
     """functional::linear -> cpu::linear (matmult_cpu.cpp:1624-1714): the bias, broadcast to the
     output shape, is the initial accumulator of the GEMM.  Done here in one pass (C_BIAS)."""
+    if _face is not None and x.is_cuda and bias is not None:
+        y = _face.gemm(x, w, bias, bool(transpose_a), bool(transpose_b), bool(_relu), _stream())
+        if y is not None:
+            return _done(y)
     _require_device(x, w, bias)
     if not (x.dtype == w.dtype == bias.dtype):
         raise ValueError("linear expects input, weight and bias of one dtype")
@@ -198,15 +220,6 @@ def linear(x, w, bias, transpose_a=False, transpose_b=False, _relu=False):
     def unsq(t):      # unsqueeze_as, matmult_cpu.cpp:1712-1713
         return t.reshape((1,) * (nd - t.dim()) + tuple(t.shape))
 
-    if x.dim() == 2 and w.dim() == 2 and bias.dim() == 1:
-        # a layer's own call: one bias row for a matrix (what the rules below come down to)
-        x_st, ta = _as_matrix_view(x, bool(transpose_a))
-        w_st, tb = _as_matrix_view(w, bool(transpose_b))
-        m, k, n = _logical(x_st.shape, w_st.shape, ta, tb)
-        if bias.shape[0] == n and m and n:
-            out = torch.empty((m, n), dtype=x.dtype, device=x.device)
-            _launch(x_st, w_st, out, m, k, n, ta, tb, 1, m * k, k * n, m * n, _lib.C_BIAS, bias=bias.contiguous(), bias_strides=(0, 0, 1), relu=_relu)
-            return out
     x, w, bias = unsq(x), unsq(w), unsq(bias)
     x_st, ta = _as_matrix_view(x, bool(transpose_a))
     w_st, tb = _as_matrix_view(w, bool(transpose_b))
@@ -288,6 +301,10 @@ def unfold2d(x, kernel_size, dilation=1, padding=0, stride=1, transpose_out=True
 
 def conv2d(image, kernel, stride=1, padding=0, dilation=1, groups=1):
     """functional::conv2d (tensor_files/conv.cpp:69-119): unfold2d then matmult; out [B,O,Ho,Wo]."""
+    if _face is not None and image.is_cuda:
+        y = _face.conv(2, image, kernel, stride, padding, dilation, groups, _stream())
+        if y is not None:
+            return _done(y)
     _require_device(image, kernel)
     if image.dim() < 3:
         raise ValueError(f"Expected to get a 3D or greater tensor as the input for a 2d convolution, but got {image.dim()}D")
@@ -351,6 +368,10 @@ def unfold2d_backward(col, output_size, kernel_size, dilation=1, padding=0, stri
 
 def conv2d_backward(image, kernel, grad, stride=1, padding=0, dilation=1, groups=1):
     """conv_dimage + conv_dkernel for dim == 2 (conv.cpp:318-346, 444-471): returns (d_image, d_kernel)."""
+    if _face is not None and image.is_cuda:
+        gradients = _face.conv_backward(2, image, kernel, grad, stride, padding, dilation, groups, _stream())
+        if gradients is not None:
+            return _done(gradients)
     return _conv2d_gradients(image, kernel, grad, stride, padding, dilation, groups)
 
 
@@ -385,6 +406,10 @@ def _conv2d_gradients(image, kernel, grad, stride, padding, dilation, groups, wa
 def conv1d(image, kernel, stride=1, padding=0, dilation=1, groups=1):
     """functional::conv1d (tensor_files/conv.cpp:13-67): unfold1d then matmult; image [.., C, W], kernel [O, C/groups, k]
     -> [B, O, Wo].  A convolution over one axis is the two-axis one with a single image row and a single tap row."""
+    if _face is not None and image.is_cuda:
+        y = _face.conv(1, image, kernel, stride, padding, dilation, groups, _stream())
+        if y is not None:
+            return _done(y)
     _require_device(image, kernel)
     if image.dim() < 2:
         raise ValueError(f"Expected to get a 2D or greater tensor as the input for a 1d convolution, but got {image.dim()}D")
@@ -404,6 +429,10 @@ def conv1d(image, kernel, stride=1, padding=0, dilation=1, groups=1):
 
 def conv1d_backward(image, kernel, grad, stride=1, padding=0, dilation=1, groups=1):
     """Gradients of conv1d with respect to image and kernel (conv_dimage / conv_dkernel with dim == 1)."""
+    if _face is not None and image.is_cuda:
+        gradients = _face.conv_backward(1, image, kernel, grad, stride, padding, dilation, groups, _stream())
+        if gradients is not None:
+            return _done(gradients)
     x = image.reshape((1,) + tuple(image.shape)) if image.dim() == 2 else image.reshape((-1,) + tuple(image.shape[-2:]))
     w = kernel.reshape((1,) + tuple(kernel.shape)) if kernel.dim() == 2 else kernel
     dx, dw = conv2d_backward(x.unsqueeze(2), w.unsqueeze(2), grad.reshape(x.shape[0], w.shape[0], 1, -1),
@@ -414,6 +443,10 @@ def conv1d_backward(image, kernel, grad, stride=1, padding=0, dilation=1, groups
 def conv_transpose2d(image, kernel, stride=1, padding=0, output_padding=0, dilation=1, groups=1):
     """functional::conv_transpose2d (tensor_files/conv.cpp:614-676): image [.., Cin, H, W], kernel [Cin, Cout/groups, kh, kw]
     -> [B, Cout, (H-1)*s - 2p + d(kh-1) + 1 + output_padding, ...]."""
+    if _face is not None and image.is_cuda:
+        y = _face.conv_transpose(2, image, kernel, stride, padding, output_padding, dilation, groups, _stream())
+        if y is not None:
+            return _done(y)
     _require_device(image, kernel)
     if image.dim() < 3:
         raise ValueError(f"Expected to get a 3D or greater tensor as the input for a conv2d transpose, but got {image.dim()}D")
@@ -459,6 +492,10 @@ def conv_transpose2d(image, kernel, stride=1, padding=0, output_padding=0, dilat
 def conv_transpose2d_backward(image, kernel, grad, stride=1, padding=0, output_padding=0, dilation=1, groups=1):
     """Gradients of conv_transpose2d: d_image = conv2d(grad, kernel) and d_kernel = conv_dkernel with the roles of image
     and output gradient exchanged (the transposed convolution is the adjoint of that convolution)."""
+    if _face is not None and image.is_cuda:
+        gradients = _face.conv_transpose_backward(2, image, kernel, grad, stride, padding, dilation, groups, _stream())
+        if gradients is not None:
+            return _done(gradients)
     s, p, d = _pair(stride), _pair(padding), _pair(dilation)
     x = image.reshape((1,) + tuple(image.shape)) if image.dim() == 3 else image.reshape((-1,) + tuple(image.shape[-3:]))
     w = kernel.reshape((1,) + tuple(kernel.shape)) if kernel.dim() == 3 else kernel
@@ -470,6 +507,10 @@ def conv_transpose2d_backward(image, kernel, grad, stride=1, padding=0, output_p
 
 def conv_transpose1d(image, kernel, stride=1, padding=0, output_padding=0, dilation=1, groups=1):
     """functional::conv_transpose1d (tensor_files/conv.cpp:538-612): image [.., Cin, W], kernel [Cin, Cout/groups, k]."""
+    if _face is not None and image.is_cuda:
+        y = _face.conv_transpose(1, image, kernel, stride, padding, output_padding, dilation, groups, _stream())
+        if y is not None:
+            return _done(y)
     x = image.reshape((1,) + tuple(image.shape)) if image.dim() == 2 else image.reshape((-1,) + tuple(image.shape[-2:]))
     w = kernel.reshape((1,) + tuple(kernel.shape)) if kernel.dim() == 2 else kernel
     out = conv_transpose2d(x.unsqueeze(2), w.unsqueeze(2), (1, stride), (0, padding), (0, output_padding), (1, dilation), groups)
@@ -477,6 +518,10 @@ def conv_transpose1d(image, kernel, stride=1, padding=0, output_padding=0, dilat
 
 
 def conv_transpose1d_backward(image, kernel, grad, stride=1, padding=0, output_padding=0, dilation=1, groups=1):
+    if _face is not None and image.is_cuda:
+        gradients = _face.conv_transpose_backward(1, image, kernel, grad, stride, padding, dilation, groups, _stream())
+        if gradients is not None:
+            return _done(gradients)
     x = image.reshape((1,) + tuple(image.shape)) if image.dim() == 2 else image.reshape((-1,) + tuple(image.shape[-2:]))
     w = kernel.reshape((1,) + tuple(kernel.shape)) if kernel.dim() == 2 else kernel
     dx, dw = conv_transpose2d_backward(x.unsqueeze(2), w.unsqueeze(2), grad.unsqueeze(-2), (1, stride), (0, padding),
@@ -561,6 +606,10 @@ def _convnd_gradients(image, kernel, grad, stride, padding, dilation, groups, wa
 
 def conv3d(image, kernel, stride=1, padding=0, dilation=1, groups=1):
     """functional::conv3d (conv.cpp:122-175): image [.., C, D, H, W], kernel [O, C/groups, kd, kh, kw]."""
+    if _face is not None and image.is_cuda:
+        y = _face.conv(3, image, kernel, stride, padding, dilation, groups, _stream())
+        if y is not None:
+            return _done(y)
     if image.dim() < 4:
         raise ValueError(f"Expected to get a 4D or greater tensor as the input for a 3d convolution, but got {image.dim()}D")
     if kernel.dim() not in (4, 5):
@@ -571,6 +620,10 @@ def conv3d(image, kernel, stride=1, padding=0, dilation=1, groups=1):
 
 
 def conv3d_backward(image, kernel, grad, stride=1, padding=0, dilation=1, groups=1):
+    if _face is not None and image.is_cuda:
+        gradients = _face.conv_backward(3, image, kernel, grad, stride, padding, dilation, groups, _stream())
+        if gradients is not None:
+            return _done(gradients)
     x = image.reshape((1,) + tuple(image.shape)) if image.dim() == 4 else image.reshape((-1,) + tuple(image.shape[-4:]))
     w = kernel.reshape((1,) + tuple(kernel.shape)) if kernel.dim() == 4 else kernel
     dx, dw = convnd_backward(x, w, grad, stride, padding, dilation, groups)
@@ -609,6 +662,10 @@ def conv_transposend(image, kernel, stride=1, padding=0, output_padding=0, dilat
 def conv_transposend_backward(image, kernel, grad, stride=1, padding=0, output_padding=0, dilation=1, groups=1):
     """Gradients of the transposed convolution through its adjoint: d_image = convnd(grad, kernel), d_kernel = conv_dkernel
     with image and output gradient exchanged."""
+    if _face is not None and image.is_cuda and kernel.dim() == 5:
+        gradients = _face.conv_transpose_backward(3, image, kernel, grad, stride, padding, dilation, groups, _stream())
+        if gradients is not None:
+            return _done(gradients)
     g = grad.contiguous()
     dx = convnd(g, kernel, stride, padding, dilation, groups)
     _, dw = _convnd_gradients(g, kernel, image.contiguous(), stride, padding, dilation, groups, want_dx=False)
@@ -616,6 +673,10 @@ def conv_transposend_backward(image, kernel, grad, stride=1, padding=0, output_p
 
 
 def conv_transpose3d(image, kernel, stride=1, padding=0, output_padding=0, dilation=1, groups=1):
+    if _face is not None and image.is_cuda:
+        y = _face.conv_transpose(3, image, kernel, stride, padding, output_padding, dilation, groups, _stream())
+        if y is not None:
+            return _done(y)
     if image.dim() < 4:
         raise ValueError(f"Expected to get a 4D or greater tensor as the input for a conv3d transpose, but got {image.dim()}D")
     if kernel.dim() not in (4, 5):
