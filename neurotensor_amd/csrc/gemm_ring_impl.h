@@ -215,7 +215,7 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, FLAT ? 1 : WB_, CONV))
     constexpr int WBM = FLAT ? 1 : WB_, WBN = WBN_ ? WBN_ : WB_;      // 32 x 32 blocks per wavefront along m / along n
     constexpr int WB = FLAT ? 2 * WBN : WBN;             // DMA instructions per wavefront for 64 bytes of k of the B tile, whose 64 WB columns a gathering kernel fills
     static_assert(CONV == 0 || FLAT || WBM == WBN, "gathering kernels have square tiles, or flat ones");
-    static_assert(!FLAT || ((CONV == 3 || CONV == 5 || CONV == 6 || CONV == 8) && !TA && WBN_ == 0 && KD_ == 1), "flat tiles: channels-last convolutions, A stored [m][k]");
+    static_assert(!FLAT || ((CONV == 3 || CONV == 5 || CONV == 6 || CONV == 8 || CONV == 9 || CONV == 10) && !TA && WBN_ == 0 && KD_ == 1), "flat tiles: channels-last convolutions, A stored [m][k]");
     constexpr int KD = KD_;
     static_assert(KD == 1 || (KD == 2 && CONV == 0 && (ES == 2 || ES == 1) && WB_ == 2 && (WBN_ == 0 || WBN_ == 4)), "deep K-steps: 16- and 8-bit plain products on 128 x 128 and 128 x 256 tiles");
     constexpr bool RING3 = KD == 2 && WBN_ == 4;         // three stages of 48 KiB
@@ -225,10 +225,11 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, FLAT ? 1 : WB_, CONV))
     constexpr int A_TILE_BYTES = BM * G::KB, STAGE_BYTES = A_TILE_BYTES + G::TILE_BYTES;
     constexpr int WTM = 32 * WBM, WTN = 32 * WBN;        // a wavefront's share of the tile: WTM rows x WTN columns
     constexpr bool GATHER4 = CONV == 1 || CONV == 2;     // op(B) gathered element by element from an NCHW image
-    constexpr bool ITEMS = CONV == 8;                    // several convolutions of one bordered image in one launch, each described by a RingItem
-    constexpr bool GATHER16 = CONV == 3 || CONV == 5 || CONV == 6 || ITEMS;   // op(B) = col^T gathered in 16-byte pieces from a channels-last image
-    constexpr bool HALO = CONV == 5 || CONV == 6 || ITEMS;   // ... whose copy carries the padding as pixels of zeros: every tap of every window exists
-    constexpr bool DEPTH = CONV == 6 || ITEMS;           // ... over three spatial axes
+    constexpr bool ITEMS = CONV == 8 || CONV == 10;      // several convolutions of one bordered image in one launch, each described by a RingItem
+    constexpr bool SLOTS = CONV == 9 || CONV == 10;      // channels of a tap in whole 16-byte slots instead of whole K-steps: a K-step's four slots may belong to several taps
+    constexpr bool GATHER16 = CONV == 3 || CONV == 5 || CONV == 6 || ITEMS || SLOTS;   // op(B) = col^T gathered in 16-byte pieces from a channels-last image
+    constexpr bool HALO = CONV == 5 || CONV == 6 || ITEMS || SLOTS;   // ... whose copy carries the padding as pixels of zeros: every tap of every window exists
+    constexpr bool DEPTH = CONV == 6 || ITEMS || SLOTS;  // ... over three spatial axes
     constexpr bool GATHERW = CONV == 4 || CONV == 7;     // op(B) = col^T of a channels-last image, 16-byte pieces along the channels (weight gradient)
     constexpr bool DEPTHW = CONV == 7;                   // ... of a bordered copy over two or three axes, pixel by division (no table of window origins)
     constexpr bool A_KC = !TA, B_KC = GATHER4 ? false : GATHER16 ? true : GATHERW ? false : TB;
@@ -248,6 +249,8 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, FLAT ? 1 : WB_, CONV))
     // channels-last weight gradient: byte offset of every output pixel's window origin inside one (bordered) image
     constexpr int DW_TABLE = CONV == 4 ? dw_table_entries(WB) : 1;   // (CONV = 7 has none)
     __shared__ int dw_tab[DW_TABLE];
+    // ... byte offset from a window's origin of every 16-byte slot of k
+    __shared__ int slot_tab[SLOTS ? NTG_SLOT_TABLE + 16 : 1];
 
     if (pin.gate && *pin.gate != pin.gate_want) return; // (uniform: the other kernel of a gated pair does this product)
     const int tid = threadIdx.x;
@@ -496,8 +499,8 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, FLAT ? 1 : WB_, CONV))
             }
             cmask3[x] = n < p.N ? m : 0u;
             const uint32_t kv = (uint32_t)((lane & 3) ^ km_swz<ES>(row));
-            uint32_t tq = 0u, cho = kv * 16u;
-            if (g.tap_step > 1) {
+            uint32_t tq = 0u, cho = SLOTS ? 0u : kv * 16u;
+            if (!SLOTS && g.tap_step > 1) {
                 const uint32_t cb = 64u / (uint32_t)g.tap_step;        // bytes of channels per pixel: 16 or 32
                 tq = cho / cb;
                 cho -= tq * cb;
@@ -507,11 +510,38 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, FLAT ? 1 : WB_, CONV))
                            (uint32_t)g.chan * (uint32_t)ES + cho;
         }
     }
+    // Slots (p.conv.slot_v of them a tap, taps outermost): a lane's slot of the K-step is the same in all its instructions (rows 16 apart), so one table
+    // entry, read a K-step ahead, and one addition an instruction place its 16 bytes.
+    int slot_n = 0, slot_off = 0;
+    const int slot_kv = (lane & 3) ^ km_swz<ES>(lane >> 2);
+    if constexpr (SLOTS) {
+        const ConvGeom& g = p.conv;
+        const int nslots = K / G::VEL;
+        for (int i = tid; i < nslots + 16; i += 256) {
+            int off = 0;                                            // (K-steps past the end read the first slot; nobody multiplies it)
+            if (i < nslots) {
+                const uint32_t tap = fast_div((uint32_t)i, g.div_slot), cv = (uint32_t)i - tap * (uint32_t)g.slot_v;
+                const uint32_t tr = tap / (uint32_t)g.k_c, q = tap - tr * (uint32_t)g.k_c, t = tr / (uint32_t)g.k_r, r = tr - t * (uint32_t)g.k_r;
+                off = (int)((((t * (uint32_t)g.d_d * (uint32_t)g.H + r * (uint32_t)g.d_r) * (uint32_t)g.W + q * (uint32_t)g.d_c) * (uint32_t)g.chan) * (uint32_t)ES + cv * 16u);
+            }
+            slot_tab[i] = off;
+        }
+        __syncthreads();
+        slot_off = slot_tab[slot_kv];
+    }
     // instruction x (0 .. WB - 1) of this wavefront's share of the NEXT gathered tile; the K-step's counters move on after the last
     auto conv3_dma = [&](int x, uint32_t lds_tile) __attribute__((always_inline)) {
         if constexpr (GATHER16) {
             const ConvGeom& g = p.conv;
             const char* img = reinterpret_cast<const char*>(B);
+            if constexpr (SLOTS) {
+                dma_1k(img, lanepart3[x] + (uint32_t)slot_off, lds_tile + (uint32_t)(wave_u * WB + x) * 1024u);
+                if (x == WB - 1) {
+                    slot_n = slot_n + 4 < K / G::VEL ? slot_n + 4 : slot_n;      // (uniform; the entries behind the last slot are zeros)
+                    slot_off = slot_tab[slot_n + slot_kv];
+                }
+                return;
+            }
             if constexpr (HALO) {
                 // the image carries its padding (p.conv describes the padded image, padding 0): no tap is ever outside, the
                 // address is a uniform base plus the lane's constant offset, exactly the DMA of a stored operand
@@ -1343,7 +1373,8 @@ static hipError_t launch_ring_nhwc_halo_cfg(const GemmParams& pin, hipStream_t s
     const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n * p.batch;
     if (blocks <= 0) return hipSuccess;
     if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    if (p.conv.k_d > 1 || p.conv.D > 1) hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 6, 0, 1, FLAT>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+    if (p.conv.slot_v) hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 9, 0, 1, FLAT>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+    else if (p.conv.k_d > 1 || p.conv.D > 1) hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 6, 0, 1, FLAT>), dim3((unsigned)blocks), dim3(256), 0, s, p);
     else hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 5, 0, 1, FLAT>), dim3((unsigned)blocks), dim3(256), 0, s, p);
     return hipGetLastError();
 }
@@ -1356,7 +1387,8 @@ static hipError_t launch_ring_items_cfg(const GemmParams& pin, int64_t blocks, h
     p.tiles_m = (p.M + TM - 1) / TM;
     if (blocks <= 0) return hipSuccess;
     if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 8, 0, 1, FLAT>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+    if (p.conv.slot_v) hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 10, 0, 1, FLAT>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((gemm_ring_kernel<DT, false, true, true, WB, 8, 0, 1, FLAT>), dim3((unsigned)blocks), dim3(256), 0, s, p);
     return hipGetLastError();
 }
 

@@ -83,7 +83,11 @@ struct ConvGeom {
     int n_items;
     int k_segment;           // Float32 weight gradients and `items`: K-steps of one chain of multiply-adds (a power of two; 0: all of them)
     int tile_edge;           // channels-last weight gradient: the edge of the tile the caller planned with
+    // channels-last convolution on a bordered copy, k in 16-byte slots (taps outermost): slots of a tap; 0: whole 64-byte runs
+    int slot_v;
+    FastDiv div_slot;
 };
+#define NTG_SLOT_TABLE 2048  // slots of k at most (8 KiB of LDS beside the ring)
 
 struct GemmParams {
     const void* A;

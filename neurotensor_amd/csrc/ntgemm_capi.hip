@@ -1439,15 +1439,29 @@ static HaloPlan conv_halo(const Geo3& g) {
     return h;
 }
 
+// How the copy holds the channels of a group (cgp 0: not at all): whole 64-byte runs, or behind a border in whole 16-byte slots (slot_v of them) where
+// that is less; the kernel's K-steps are then four slots of whatever taps.  us of the forward product and what it needs, as whole runs, merged taps or
+// element-wise gathers | in slots: BFloat16 16 x 24 x 56 x 56 -> 24 by 3 x 3 21 | 12, 16 x 48 x 47 x 47 -> 16 by 5 x 5 in 2 groups 43 | 18, 14 x 1 x 40^3 -> 32 by
+// 3 x 3 x 3 365 | 83, Float32 32 x 3 x 224 x 224 -> 64 by 7 x 7 at stride 2 144 | 126, 16 x 24 x 56 x 56 -> 24 29 | 19, 16 x 48 x 47 x 47 -> 16 in 2 groups 104 | 46,
+// 4 x 24 x 20^3 -> 40 47 | 33; equal on one or two tiles (Float32 1 x 24 x 12 x 12 -> 24 12 | 12).  Up to 128 output pixels, the columns of one
+// flat tile, the other forms stay with the workspaces that callers know: a step takes about as long (8 x 8 pixels so | 9 x 9 in slots: BFloat16 24 -> 24 29.0 | 29.1,
+// 16 -> 32 28.7 | 29.1, Float32 24 -> 24 38 | 34).
+struct NhwcForm { int64_t cgp, slot_v; };
+static NhwcForm nhwc_form(int64_t es, int64_t cg, int64_t taps, bool bordered, int64_t pixels) {
+    const int64_t vel = 16 / es, run = 64 / es, slots = (cg + vel - 1) / vel;
+    if (bordered && cg > 0 && pixels > 128 && slots * vel % run != 0 && taps * slots <= NTG_SLOT_TABLE) return {slots * vel, slots};
+    return {nhwc_padded_channels(es, cg), 0};
+}
+
 // Few channels per group (up to 32 bytes of them): a pixel of the copy holds 16 or 32 bytes and a K-step covers 4 or 2
 // consecutive taps of a tap row, the row padded to a multiple of that with zero weights -- an RGB 7 x 7 input layer in
 // BFloat16 runs on K = 7 * 8 * 8 instead of 49 * 32.  Forward only.
 struct MergedTaps { int64_t cgp, T, kq_pad; };
-static bool conv_nhwc_merged(int dtype, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g, MergedTaps& mt) {
+static bool conv_nhwc_merged(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g, MergedTaps& mt) {
     if (dtype != ntg::DT_F32 && dtype != ntg::DT_F16 && dtype != ntg::DT_BF16) return false;
     if (g.nd != 2 || !conv_implicit_g(dtype, channels, g) || out_channels <= 0) return false;
     const int64_t es = ntg::elem_size(dtype), cg = channels / groups;
-    if (cg <= 0 || cg * es > 32) return false;
+    if (cg <= 0 || cg * es > 32 || nhwc_form(es, cg, g.taps(), conv_halo(g).on, batch * g.L()).slot_v) return false;
     const int64_t cb = cg * es <= 16 ? 16 : 32;
     mt.cgp = cb / es; mt.T = 64 / cb; mt.kq_pad = (g.k[2] + mt.T - 1) / mt.T * mt.T;
     if (mt.kq_pad > 8 || mt.kq_pad * mt.cgp > 4 * g.k[2] * cg || out_channels * g.k[1] * mt.kq_pad >= 0x7fffffffLL) return false;          // (padding: at most 4x the arithmetic)
@@ -1457,18 +1471,23 @@ static int64_t conv_nhwc_merged_workspace(int dtype, int64_t batch, int64_t out_
     const int64_t es = ntg::elem_size(dtype);
     return (int64_t)align_up((size_t)(batch * groups * mt.cgp * g.vol() * es), 256) + out_channels * g.k[1] * mt.kq_pad * mt.cgp * es;
 }
-static bool conv_nhwc_ok(int dtype, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
+static bool conv_nhwc_ok(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
     if (dtype != ntg::DT_F32 && dtype != ntg::DT_F16 && dtype != ntg::DT_BF16) return false;
     if (!conv_implicit_g(dtype, channels, g)) return false;
     const HaloPlan halo = conv_halo(g);
     if (g.nd == 3 && !halo.on) return false;                          // (three axes: the bordered copy is the only form)
-    const int64_t es = ntg::elem_size(dtype), cgp = nhwc_padded_channels(es, channels / groups);
+    const int64_t es = ntg::elem_size(dtype), cgp = nhwc_form(es, channels / groups, g.taps(), halo.on, batch * g.L()).cgp;
     return cgp > 0 && out_channels > 0 && out_channels * g.taps() < 0x7fffffffLL && conv_nhwc_offsets_fit(groups * cgp, es, g) &&
            conv_nhwc_offsets_fit(groups * cgp, es, halo.gp);
 }
 static int64_t conv_nhwc_workspace(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
-    const int64_t es = ntg::elem_size(dtype), cgp = nhwc_padded_channels(es, channels / groups);
-    return (int64_t)align_up((size_t)(batch * groups * cgp * conv_halo(g).vol * es), 256) + out_channels * cgp * g.taps() * es;
+    const HaloPlan halo = conv_halo(g);
+    const int64_t es = ntg::elem_size(dtype), cgp = nhwc_form(es, channels / groups, g.taps(), halo.on, batch * g.L()).cgp;
+    return (int64_t)align_up((size_t)(batch * groups * cgp * halo.vol * es), 256) + out_channels * cgp * g.taps() * es;
+}
+static void set_slots(ntg::ConvGeom& c, const NhwcForm& form) {
+    c.slot_v = (int)form.slot_v;
+    c.div_slot = ntg::make_fastdiv((uint32_t)std::max<int64_t>(form.slot_v, 1));
 }
 static void add_copy(ntg::ChannelsLast& cl, const void* in, void* out, int64_t batch, int64_t groups, int64_t cg, int64_t cgp, int64_t pixels, const HaloPlan& halo) {
     cl.copy[cl.n++] = {in, out, batch, groups, cg, cgp, pixels, halo.on, halo.hm};
@@ -1476,12 +1495,13 @@ static void add_copy(ntg::ChannelsLast& cl, const void* in, void* out, int64_t b
 static int conv_forward_nhwc(int dtype, const void* image, const void* kernel, void* out, void* ws, int64_t batch, int64_t channels,
                              int64_t out_channels, const Geo3& g, int64_t groups, hipStream_t hs, const MergedTaps* mt = nullptr) {
     const int64_t es = ntg::elem_size(dtype), cg = channels / groups, og = out_channels / groups;
-    const int64_t cgp = mt ? mt->cgp : nhwc_padded_channels(es, cg), chp = groups * cgp;      // channels per group / per pixel in the copy
-    const int64_t L = g.L(), taps = g.taps(), vol = g.vol(), K = mt ? g.k[1] * mt->kq_pad * cgp : taps * cgp;
     HaloPlan halo = conv_halo(g);
+    const NhwcForm form = nhwc_form(es, cg, g.taps(), halo.on, batch * g.L());
+    const int64_t cgp = mt ? mt->cgp : form.cgp, chp = groups * cgp;      // channels per group / per pixel in the copy
+    const int64_t L = g.L(), taps = g.taps(), vol = g.vol(), K = mt ? g.k[1] * mt->kq_pad * cgp : taps * cgp;
     if (mt) { halo.on = false; halo.vol = vol; halo.gp = g; }                    // (the merged-tap form keeps its validity bits)
     const int64_t volp = halo.vol;                                               // pixels per image of the copy
-    const bool tap_inner = halo.on && g.s[0] == 1 && g.s[1] == 1 && g.s[2] == 1;   // (neighbouring taps share pixels only at unit strides)
+    const bool tap_inner = halo.on && !form.slot_v && g.s[0] == 1 && g.s[1] == 1 && g.s[2] == 1;   // (neighbouring taps share pixels only at unit strides)
     char* ws_img = static_cast<char*>(ws);
     char* ws_w = ws_img + align_up((size_t)(batch * chp * volp * es), 256);
     const int64_t wchunk = tap_inner ? 64 / es : 0;                              // (taps inside a 64-byte run of channels)
@@ -1503,6 +1523,7 @@ static int conv_forward_nhwc(int dtype, const void* image, const void* kernel, v
     p.conv.halo = halo.on ? 1 : 0;
     p.conv.tap_inner = tap_inner ? 1 : 0;
     if (mt) { p.conv.tap_step = (int)mt->T; p.conv.kq_pad = (int)mt->kq_pad; }
+    else set_slots(p.conv, form);
     e = launch_groups(p, dtype, batch, groups, {og * K, 0, cgp, chp * volp, og * L}, [&](const ntg::GemmParams& q) { return ntg::launch_conv_nhwc(dtype, q, hs); });
     if (e != hipSuccess) return hip_fail(e, "channels-last convolution launch");
     return NTG_OK;
@@ -1557,8 +1578,8 @@ static int conv_dimage_gather(int dtype, const void* kernel, const void* grad_ou
 
 // The same gradient through the channels-last kernel: dY is copied to [B][pixel][O] and the flipped weights to
 // [C][(taps, oc)] in the workspace (out channels of a group in whole 64-byte runs, padded like the forward copy).
-static bool conv_dimage_nhwc_ok(int dtype, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
-    return conv_nhwc_ok(dtype, out_channels, channels, groups, geo_dimage(g));
+static bool conv_dimage_nhwc_ok(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
+    return conv_nhwc_ok(dtype, batch, out_channels, channels, groups, geo_dimage(g));
 }
 static int64_t conv_dimage_nhwc_workspace(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
     return conv_nhwc_workspace(dtype, batch, out_channels, channels, groups, geo_dimage(g));
@@ -1568,12 +1589,13 @@ static int64_t conv_dimage_nhwc_workspace(int dtype, int64_t batch, int64_t chan
 static int conv_dimage_nhwc(int dtype, const void* kernel, const void* grad_out, void* d_image, void* ws, int64_t batch,
                             int64_t channels, int64_t out_channels, const Geo3& g, int64_t groups, int accumulate, hipStream_t hs, ntg::ChannelsLast* cl) {
     const int64_t es = ntg::elem_size(dtype), cg = channels / groups, og = out_channels / groups;
-    const int64_t ogp = nhwc_padded_channels(es, og), ochp = groups * ogp;      // out channels per group / per pixel in the copy
-    const int64_t L = g.L(), taps = g.taps(), vol = g.vol(), K = taps * ogp;
     const Geo3 t = geo_dimage(g);
     const HaloPlan halo = conv_halo(t);                                         // (the "image" of this convolution is dY)
+    const NhwcForm form = nhwc_form(es, og, g.taps(), halo.on, batch * t.L());
+    const int64_t ogp = form.cgp, ochp = groups * ogp;                          // out channels per group / per pixel in the copy
+    const int64_t L = g.L(), taps = g.taps(), vol = g.vol(), K = taps * ogp;
     const int64_t Lp = halo.vol;
-    const bool tap_inner = halo.on;                                             // (all strides are 1)
+    const bool tap_inner = halo.on && !form.slot_v;                             // (all strides are 1)
     char* ws_gy = static_cast<char*>(ws);
     char* ws_w = ws_gy + align_up((size_t)(batch * ochp * Lp * es), 256);
     if (cl) {
@@ -1592,6 +1614,7 @@ static int conv_dimage_nhwc(int dtype, const void* kernel, const void* grad_out,
     p.conv.chan = (int)ochp;
     p.conv.halo = halo.on ? 1 : 0;
     p.conv.tap_inner = tap_inner ? 1 : 0;
+    set_slots(p.conv, form);
     const hipError_t e = launch_groups(p, dtype, batch, groups, {cg * K, 0, ogp, ochp * Lp, cg * vol}, [&](const ntg::GemmParams& q) { return ntg::launch_conv_nhwc(dtype, q, hs); });
     if (e != hipSuccess) return hip_fail(e, "channels-last conv_dimage launch");
     return NTG_OK;
@@ -1617,6 +1640,7 @@ static int chain_steps(int64_t n) {
 struct PhasePlan {
     bool ok;
     int edge;
+    NhwcForm form;
     int64_t gy_bytes, w_bytes, item_bytes, tmp_bytes, blocks;
     ntg::HaloMap hm;
     ntg::PhaseLayout lay;
@@ -1626,10 +1650,14 @@ struct PhasePlan {
 // Float32 would have to pad (16 x 64 x 56 x 56 -> 24 by 3 x 3 at stride 2, a step: 83 us against 93 by phases; 4 x 32 x 24^3 -> 24 by 3 x 3 x 3 84 / 101)
 // except over three axes on images from 32 MiB on, the passes over col and image being the larger part there (9 x 256 x 29^3 -> 48 by one
 // tap in 2 groups 621 / 406, 42 x 256 x 24^3 -> 96 by 3 x 3 x 3 in 4 groups 3291 / 2571).
-static int64_t phase_padded_channels(int64_t es, int64_t og, int64_t batch, int64_t channels, const Geo3& g) {
+static NhwcForm phase_form(int64_t es, int64_t og, int64_t batch, int64_t channels, const Geo3& g) {
+    int64_t taps = 1;                                                             // of the largest phase
+    for (int a = 0; a < 3; ++a) taps *= (g.k[a] + g.s[a] - 1) / g.s[a];
+    const NhwcForm f = nhwc_form(es, og, taps, true, batch * g.vol());
+    if (f.slot_v) return f;
     const int64_t step = 64 / es, ogp = (og + step - 1) / step * step;
     const int64_t most = es == 2 ? 4 : g.nd == 3 && batch * channels * g.vol() * es >= (1LL << 25) ? 2 : 1;
-    return og > 0 && ogp <= most * og ? ogp : 0;
+    return {og > 0 && ogp <= most * og ? ogp : 0, 0};
 }
 static PhasePlan plan_dimage_phases(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
     PhasePlan pp;
@@ -1639,7 +1667,8 @@ static PhasePlan plan_dimage_phases(int dtype, int64_t batch, int64_t channels, 
     for (int a = 0; a < 3; ++a)
         if (g.d[a] != 1 || g.s[a] > 4 || g.p[a] < 0 || g.sz[a] >= (1 << 24) || g.k[a] >= (1 << 16)) return pp;
     const int64_t es = ntg::elem_size(dtype), vel = 16 / es, og = out_channels / groups, cg = channels / groups;
-    const int64_t ogp = phase_padded_channels(es, og, batch, channels, g), ochp = groups * ogp;
+    const NhwcForm form = phase_form(es, og, batch, channels, g);
+    const int64_t ogp = form.cgp, ochp = groups * ogp;
     // (the interleaving pass counts image elements in 32 bits; one image's planes, whose pitches are 16-byte multiples, are indexed in 32 bits)
     if (ogp == 0 || batch * channels * g.vol() >= 0x7fffffffLL || channels * (g.vol() + 64 * vel) >= 0x7fffffffLL) return pp;
     // the image channels of a group are the rows of these products: with a handful of them (an RGB input layer) a 64-row
@@ -1680,7 +1709,7 @@ static PhasePlan plan_dimage_phases(int dtype, int64_t batch, int64_t channels, 
     pp.hm.Wp = q.yp[2]; pp.hm.Hp = q.yp[1]; pp.hm.Dp = q.yp[0];
     pp.hm.left = front[2]; pp.hm.top = front[1]; pp.hm.front = front[0];
     q.groups = (int)groups; q.og = (int)og; q.ogp = (int)ogp; q.cg = (int)cg; q.batch = (int)batch;
-    q.chunk = (int)(64 / es); q.vel = (int)vel;
+    q.chunk = (int)(form.slot_v ? ogp : 64 / es); q.vel = (int)vel;
     int64_t w_elems = 0, tmp_elems = 0, n_max = 0, k_max = 0;
     for (int ph = 0; ph < NTG_MAX_PHASES; ++ph) q.plane_off[ph] = -1;
     for (int e0 = 0; e0 < q.s[0]; ++e0)
@@ -1712,6 +1741,7 @@ static PhasePlan plan_dimage_phases(int dtype, int64_t batch, int64_t channels, 
                 pp.blocks += tiles_m * ((n + q.tile_cols - 1) / q.tile_cols) * batch * groups;
             }
     if (pp.blocks > 0x7fffffffLL || channels * g.taps() >= 0x7fffffffLL) return pp;
+    pp.form = form;
     pp.gy_bytes = (int64_t)align_up((size_t)(batch * ochp * volp * es), 256);
     pp.w_bytes = (int64_t)align_up((size_t)(w_elems * es), 256);
     pp.item_bytes = (int64_t)align_up((size_t)items * sizeof(ntg::RingItem), 256);
@@ -1746,6 +1776,7 @@ static int conv_dimage_phases(int dtype, const PhasePlan& pp, const void* kernel
     p.conv.d_d = p.conv.d_r = p.conv.d_c = 1;
     p.conv.k_drc = 1;                                      // (the items set their own taps; k runs taps-inner, which does not use it)
     p.conv.halo = 1; p.conv.tap_inner = 1;
+    set_slots(p.conv, pp.form);
     p.conv.items = items; p.conv.n_items = q.phases * (int)groups;
     if (g.nd == 3) p.conv.k_segment = chain_steps(og);
     hipError_t e = ntg::launch_conv_nhwc_items(dtype, pp.edge, p, pp.blocks, hs);
@@ -2033,7 +2064,7 @@ static ConvBackwardPlan plan_conv_backward_g(int dtype, bool want_dx, bool want_
     pl.pointwise = want_dw && !reference_order ? plan_pointwise_dw(dtype, batch, channels, out_channels, groups, g) : PointwiseDwPlan{0, 0};
     if (in_place) return pl;                       // (one tap on operands where they lie: the call takes none of the forms below)
     // the channels-last form of dX is taken when the caller's workspace also holds the copy of dY
-    pl.nhwc_dx = pl.gather_dx && conv_dimage_nhwc_ok(dtype, channels, out_channels, groups, g);
+    pl.nhwc_dx = pl.gather_dx && conv_dimage_nhwc_ok(dtype, batch, channels, out_channels, groups, g);
     pl.need_nhwc_dx = pl.nhwc_dx ? conv_dimage_nhwc_workspace(dtype, batch, channels, out_channels, groups, g) : 0;
     if (pl.gather_dw && !reference_order) pl.dkernel = plan_dkernel(dtype, batch, channels, out_channels, groups, g);
     pl.nhwc_dw = pl.dkernel.ok;
@@ -2119,8 +2150,8 @@ int64_t ntg_conv2d_fast_workspace_bytes(int dtype, int64_t batch, int64_t channe
     const bool groups_ok = groups >= 1 && channels % groups == 0 && out_channels % groups == 0;      // (the call itself reports bad groups)
     if (groups_ok && conv_pointwise_ok(dtype, channels, groups, g)) return 0;
     MergedTaps mt;
-    if (groups_ok && conv_nhwc_merged(dtype, channels, out_channels, groups, g, mt)) return conv_nhwc_merged_workspace(dtype, batch, out_channels, groups, g, mt);
-    if (groups_ok && conv_nhwc_ok(dtype, channels, out_channels, groups, g)) return conv_nhwc_workspace(dtype, batch, channels, out_channels, groups, g);
+    if (groups_ok && conv_nhwc_merged(dtype, batch, channels, out_channels, groups, g, mt)) return conv_nhwc_merged_workspace(dtype, batch, out_channels, groups, g, mt);
+    if (groups_ok && conv_nhwc_ok(dtype, batch, channels, out_channels, groups, g)) return conv_nhwc_workspace(dtype, batch, channels, out_channels, groups, g);
     return ntg_conv2d_forward_workspace_bytes(dtype, batch, channels, height, width, k_r, k_c, s_r, s_c, p_r, p_c, d_r, d_c);
 }
 
@@ -2171,10 +2202,10 @@ int ntg_conv2d_dev(int dtype, const void* image, const void* kernel, void* out,
             return conv_forward_pointwise(dtype, image, kernel, out, batch, channels, out_channels, g, groups, stream);
         // with the workspace of ntg_conv2d_fast_workspace_bytes: channels-last copy of the image, 16-byte gathers
         MergedTaps mt;
-        if (conv_nhwc_merged(dtype, channels, out_channels, groups, g, mt) && workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
+        if (conv_nhwc_merged(dtype, batch, channels, out_channels, groups, g, mt) && workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
             workspace_bytes >= conv_nhwc_merged_workspace(dtype, batch, out_channels, groups, g, mt))
             return conv_forward_nhwc(dtype, image, kernel, out, workspace, batch, channels, out_channels, g, groups, static_cast<hipStream_t>(stream), &mt);
-        if (conv_nhwc_ok(dtype, channels, out_channels, groups, g) && workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
+        if (conv_nhwc_ok(dtype, batch, channels, out_channels, groups, g) && workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
             workspace_bytes >= conv_nhwc_workspace(dtype, batch, channels, out_channels, groups, g))
             return conv_forward_nhwc(dtype, image, kernel, out, workspace, batch, channels, out_channels, g, groups, static_cast<hipStream_t>(stream));
         if (conv_implicit_g(dtype, channels, g))      // col_b is never stored: the GEMM's B loader gathers it from the image
@@ -2651,7 +2682,7 @@ int64_t ntg_convnd_fast_workspace_bytes(int dtype, int64_t batch, int64_t channe
         const int64_t fast = std::max({pl.need_phase_dx, pl.need_nhwc_dx, pl.need_nhwc_dw, pl.need_both});
         return fast > 0 ? std::max(fast, least + 256) : least;        // (more than `least` is what asks for the fast forms)
     }
-    return conv_nhwc_ok(dtype, channels, out_channels, groups, g) ? conv_nhwc_workspace(dtype, batch, channels, out_channels, groups, g) : least;
+    return conv_nhwc_ok(dtype, batch, channels, out_channels, groups, g) ? conv_nhwc_workspace(dtype, batch, channels, out_channels, groups, g) : least;
 }
 
 int ntg_convnd_dev(int dtype, const void* image, const void* kernel, void* out, void* workspace, int64_t workspace_bytes,
@@ -2673,7 +2704,7 @@ int ntg_convnd_dev(int dtype, const void* image, const void* kernel, void* out, 
     if (!image || !kernel || !out) return fail(NTG_ERR_INVALID_ARGUMENT, "null pointer");
     if (ndim == 3) {
         const Geo3 g = geo_from(u);
-        if (conv_nhwc_ok(dtype, channels, out_channels, groups, g) && workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
+        if (conv_nhwc_ok(dtype, batch, channels, out_channels, groups, g) && workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
             workspace_bytes >= conv_nhwc_workspace(dtype, batch, channels, out_channels, groups, g))
             return conv_forward_nhwc(dtype, image, kernel, out, workspace, batch, channels, out_channels, g, groups, static_cast<hipStream_t>(stream));
         if (conv_implicit_g(dtype, channels, g))      // three axes, floating dtype: gathered inside the GEMM, no col buffer

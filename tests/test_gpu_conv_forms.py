@@ -173,3 +173,33 @@ def test_tensors_at_any_element_of_a_buffer():
     assert torch.equal(F.conv2d(off[0], off[1], padding=1), F.conv2d(x, w, padding=1))
     dx, _ = F.conv2d_backward(*off, padding=1)
     assert torch.equal(dx, F.conv2d_backward(x, w, dy, padding=1)[0])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("batch,cin,cout,size,kernel,stride,pad,groups,transposed", [
+    (2, 1, 1, (9, 15), 3, 1, 1, 1, False),           # one slot a tap, nine taps: K-steps across tap rows, a last one of a single slot
+    (2, 24, 40, (8, 9), 3, 1, 1, 1, False),          # three and five slots (Float32: six and ten)
+    (1, 3, 33, (40, 33), 7, 2, 3, 1, False),
+    (3, 20, 12, (60,), 5, 1, 2, 1, False),
+    (2, 12, 24, (6, 5, 7), 3, 1, 1, 2, False),       # three axes, two groups
+    (2, 24, 16, (12, 11), 3, 1, 2, 1, False),        # dilated windows below
+    (1, 48, 12, (5, 5, 6), 2, 2, 0, 3, False),       # phases
+    (5, 36, 20, (6, 5), 4, 2, 1, 1, True),
+    (2, 8, 24, (129, 1), 1, 1, 0, 1, False),         # one tap: a K-step that is mostly past the end
+    (1, 40, 300, (12, 12), 3, 1, 1, 1, False),       # larger tiles
+], ids=str)
+def test_taps_in_slots(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed):
+    parts = ("dx", "y") if stride > 1 or transposed else ("dw", "y", "dx") if kernel == 1 else ()
+    check(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed, parts)
+
+
+def test_taps_in_slots_dilated_and_the_longest_table():
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    for shape, w, opt in (((2, 24, 20, 20), (8, 24, 3, 3), {"dilation": 3, "padding": 3}), ((1, 40, 12, 12), (8, 40, 8, 8), {"padding": 3}),
+                          ((1, 328, 12, 12), (8, 328, 7, 7), {"padding": 3})):          # 320 and 2009 slots; 2048 at most
+        x = torch.randn(shape, generator=gen, device="cuda").to(torch.bfloat16)
+        k = torch.randn(w, generator=gen, device="cuda").to(torch.bfloat16)
+        want = torch.nn.functional.conv2d(x.double().cpu(), k.double().cpu(), **opt)
+        mags = torch.nn.functional.conv2d(x.double().abs().cpu(), k.double().abs().cpu(), **opt)
+        err = (F.conv2d(x, k, **opt).double().cpu() - want).abs()
+        assert bool((err <= 2.0 ** -8 * want.abs() + 2.0 ** -24 * (k[0].numel() + 32) * mags).all())
