@@ -1480,10 +1480,48 @@ static bool conv_nhwc_ok(int dtype, int64_t batch, int64_t channels, int64_t out
     return cgp > 0 && out_channels > 0 && out_channels * g.taps() < 0x7fffffffLL && conv_nhwc_offsets_fit(groups * cgp, es, g) &&
            conv_nhwc_offsets_fit(groups * cgp, es, halo.gp);
 }
+// Few output tiles and a deep k (a handful of small maps with many channels): the 64-byte runs of channels in `ranges` equal ranges, Float32 sums of
+// each, added up in order by a second pass.  A workgroup alone on its CU takes 0.32 us a K-step in Float32 and 0.2 in 16 bits whatever the others do (2 x 256 x
+// 13 x 13 -> 256 by 3 x 3: 24 tiles of 144 and 72 K-steps); shared by w workgroups a CU takes 0.25 w and 0.07 w.  The second pass costs 4.5 us and the traffic of
+// the sums.  Measured: that layer 47 -> 11 + 3 us and 18 -> 8 + 3; 192 x 17 x 17 -> 32 by 7 x 7, 3 tiles of 588, 169 -> 33 + 4 us.  The number of ranges does not depend on the number of images, only whether
+// there are any: up to 128 tiles an image's result is the same bits alone and among others.  Under 64 K-steps there is too little to win; groups would need a
+// third stride.
+static int64_t conv_k_ranges(int64_t es, int64_t batch, int64_t rows, int64_t pixels, int64_t groups, const NhwcForm& form, int64_t taps) {
+    const int64_t bk = 64 / es, runs = form.cgp / bk, steps = runs * taps, tiles = ((rows + 63) / 64) * ((pixels + 63) / 64) * batch;
+    if (groups != 1 || form.slot_v || tiles > 128 || steps < 64) return 1;
+    int64_t r = 8;
+    while (r > 1 && (runs % r != 0 || steps / r < 16)) --r;
+    const double shared = (double)((tiles * r + 255) / 256), step_us = es == 4 ? 0.32 : 0.2, shared_us = std::max(step_us, (es == 4 ? 0.25 : 0.07) * shared);
+    const double sums_us = 4.5 + 8.0 * (double)(r * batch * rows * pixels) / 4.0e6;
+    return (double)(steps / r) * shared_us + sums_us < 0.8 * (double)steps * step_us ? r : 1;
+}
+static int64_t conv_k_ranges_bytes(int64_t ranges, int64_t batch, int64_t rows, int64_t pixels) { return ranges > 1 ? ranges * batch * rows * ((pixels + 7) / 8 * 8) * 4 : 0; }
+// the product p (weights by image, `rows` x `pixels` an image) in ranges: partial sums at `part`, results at p.C in p.cmode
+static hipError_t launch_conv_k_ranges(ntg::GemmParams p, int dtype, int64_t batch, int64_t ranges, int64_t taps, int64_t b_image, int64_t c_image, char* part, hipStream_t hs) {
+    const int64_t ldp = (p.N + 7) / 8 * 8, K = p.K;
+    ntg::GemmParams q = p;
+    // launch index = range * images + image
+    q.K = (int)(K / ranges);
+    q.C = part;
+    q.ldc = ldp; q.sC = p.M * ldp;
+    q.cmode = ntg::C_PARTIAL;
+    q.batch = (int)(batch * ranges);
+    q.krange_items = (int)batch;
+    q.sA = 0; q.sAk = q.K;
+    q.sB = b_image; q.sBk = q.K / taps;
+    hipError_t e = ntg::launch_conv_nhwc(dtype, q, hs);
+    if (e != hipSuccess) return e;
+    p.batch = (int)batch;
+    p.sC = c_image;
+    return ntg::launch_splitk_reduce(dtype, part, (int)ranges, p, ldp, hs);
+}
 static int64_t conv_nhwc_workspace(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
     const HaloPlan halo = conv_halo(g);
-    const int64_t es = ntg::elem_size(dtype), cgp = nhwc_form(es, channels / groups, g.taps(), halo.on, batch * g.L()).cgp;
-    return (int64_t)align_up((size_t)(batch * groups * cgp * halo.vol * es), 256) + out_channels * cgp * g.taps() * es;
+    const int64_t es = ntg::elem_size(dtype);
+    const NhwcForm form = nhwc_form(es, channels / groups, g.taps(), halo.on, batch * g.L());
+    const int64_t cgp = form.cgp, weights = out_channels * cgp * g.taps() * es;
+    const int64_t sums = halo.on ? conv_k_ranges_bytes(conv_k_ranges(es, batch, out_channels, g.L(), groups, form, g.taps()), batch, out_channels, g.L()) : 0;
+    return (int64_t)align_up((size_t)(batch * groups * cgp * halo.vol * es), 256) + (sums ? (int64_t)align_up((size_t)weights, 256) + sums : weights);
 }
 static void set_slots(ntg::ConvGeom& c, const NhwcForm& form) {
     c.slot_v = (int)form.slot_v;
@@ -1501,7 +1539,9 @@ static int conv_forward_nhwc(int dtype, const void* image, const void* kernel, v
     const int64_t L = g.L(), taps = g.taps(), vol = g.vol(), K = mt ? g.k[1] * mt->kq_pad * cgp : taps * cgp;
     if (mt) { halo.on = false; halo.vol = vol; halo.gp = g; }                    // (the merged-tap form keeps its validity bits)
     const int64_t volp = halo.vol;                                               // pixels per image of the copy
-    const bool tap_inner = halo.on && !form.slot_v && g.s[0] == 1 && g.s[1] == 1 && g.s[2] == 1;   // (neighbouring taps share pixels only at unit strides)
+    const int64_t ranges = halo.on ? conv_k_ranges(es, batch, out_channels, L, groups, form, taps) : 1;
+    // (neighbouring taps share pixels only at unit strides; ranges are of whole runs with all their taps)
+    const bool tap_inner = halo.on && !form.slot_v && ((g.s[0] == 1 && g.s[1] == 1 && g.s[2] == 1) || ranges > 1);
     char* ws_img = static_cast<char*>(ws);
     char* ws_w = ws_img + align_up((size_t)(batch * chp * volp * es), 256);
     const int64_t wchunk = tap_inner ? 64 / es : 0;                              // (taps inside a 64-byte run of channels)
@@ -1524,7 +1564,8 @@ static int conv_forward_nhwc(int dtype, const void* image, const void* kernel, v
     p.conv.tap_inner = tap_inner ? 1 : 0;
     if (mt) { p.conv.tap_step = (int)mt->T; p.conv.kq_pad = (int)mt->kq_pad; }
     else set_slots(p.conv, form);
-    e = launch_groups(p, dtype, batch, groups, {og * K, 0, cgp, chp * volp, og * L}, [&](const ntg::GemmParams& q) { return ntg::launch_conv_nhwc(dtype, q, hs); });
+    if (ranges > 1) e = launch_conv_k_ranges(p, dtype, batch, ranges, taps, chp * volp, og * L, ws_w + align_up((size_t)(og * K * es), 256), hs);
+    else e = launch_groups(p, dtype, batch, groups, {og * K, 0, cgp, chp * volp, og * L}, [&](const ntg::GemmParams& q) { return ntg::launch_conv_nhwc(dtype, q, hs); });
     if (e != hipSuccess) return hip_fail(e, "channels-last convolution launch");
     return NTG_OK;
 }
@@ -1615,7 +1656,9 @@ static int conv_dimage_nhwc(int dtype, const void* kernel, const void* grad_out,
     p.conv.halo = halo.on ? 1 : 0;
     p.conv.tap_inner = tap_inner ? 1 : 0;
     set_slots(p.conv, form);
-    const hipError_t e = launch_groups(p, dtype, batch, groups, {cg * K, 0, ogp, ochp * Lp, cg * vol}, [&](const ntg::GemmParams& q) { return ntg::launch_conv_nhwc(dtype, q, hs); });
+    const int64_t ranges = halo.on ? conv_k_ranges(es, batch, channels, vol, groups, form, taps) : 1;
+    const hipError_t e = ranges > 1 ? launch_conv_k_ranges(p, dtype, batch, ranges, taps, ochp * Lp, cg * vol, ws_w + align_up((size_t)(cg * K * es), 256), hs)
+                                    : launch_groups(p, dtype, batch, groups, {cg * K, 0, ogp, ochp * Lp, cg * vol}, [&](const ntg::GemmParams& q) { return ntg::launch_conv_nhwc(dtype, q, hs); });
     if (e != hipSuccess) return hip_fail(e, "channels-last conv_dimage launch");
     return NTG_OK;
 }

@@ -203,3 +203,15 @@ def test_taps_in_slots_dilated_and_the_longest_table():
         mags = torch.nn.functional.conv2d(x.double().abs().cpu(), k.double().abs().cpu(), **opt)
         err = (F.conv2d(x, k, **opt).double().cpu() - want).abs()
         assert bool((err <= 2.0 ** -8 * want.abs() + 2.0 ** -24 * (k[0].numel() + 32) * mags).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("batch,cin,cout,size,kernel,stride,pad", [
+    (2, 256, 65, (13, 5), 3, 1, 1),                  # a tile and a part in each direction
+    (1, 256, 256, (9,), 7, 1, 3),                    # pixels that miss the rows of the sums
+    (3, 320, 24, (11, 12), 3, 2, 1),                 # five ranges in 16 bits; strides
+    (1, 64, 30, (9, 9), 7, 1, 3),                    # flat tiles; two ranges in 16 bits
+    (1, 128, 64, (4, 5, 6), 3, 1, 1),
+], ids=str)
+def test_channels_in_ranges(dtype, batch, cin, cout, size, kernel, stride, pad):
+    check(dtype, batch, cin, cout, size, kernel, stride, pad, 1, False, ("dx",) if stride > 1 else ())
