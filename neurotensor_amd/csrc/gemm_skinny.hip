@@ -10,20 +10,27 @@
 // Lane (c = lane%16, g = lane/16) holds, per k-step, A[row c][k0+4g .. k0+4g+3] and
 // B[k0+4g+e][n0 + CPL*c .. +CPL-1] for e = 0..3: MFMA e uses k = k0+4g+e for lane group g
 // on both operands, and MFMA column c stands for strip column CPL*c + j.
+//
+// Sizes and rows off every 16-byte boundary take the same loads: vectors are declared at the alignment of one element (the memory system takes them at any
+// address), rows and columns past the end are clamped onto the last ones and their sums not stored, and the one k-step that K does not fill is read element by
+// element, all of them in flight, by the wavefront whose turn it is.  A guard per element around every load, which such products had before, made each wait
+// one for everything.  (Whole strips and steps, RAGGED = false, leave the clamps out.)  Float16 on one card, before | now, us: 3 x 4352 x 10109 (B stored [n][k]) 129 | 19.3 (with the clamp of relu, which was a pass of its own), 6 x 5229 x 331 61 | 21.5, 8 x 1536 x 472 28.5 | 4.5.
 #include "ntg_common.h"
 
 namespace ntg {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx4e __attribute__((ext_vector_type(4), aligned(4)));          // at any element
 
-template <int MB, int CPL, bool TA, bool TB, bool FAST>
+template <int MB, int CPL, bool TA, bool TB, bool RAGGED>
 __global__ void __launch_bounds__(512) gemm_skinny_f32_kernel(const GemmParams p) {
     constexpr int NW = 8;
     constexpr int SW = 16 * CPL;
     __shared__ float part[NW][MB * CPL * 4][64];
 
     const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
+    // (the wavefront's number in a scalar register: the branches below must be real ones, a matrix instruction runs whatever the lane mask says)
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, g = lane >> 4;
     const int b = blockIdx.y;
     const int n0 = blockIdx.x * SW;
@@ -39,64 +46,65 @@ __global__ void __launch_bounds__(512) gemm_skinny_f32_kernel(const GemmParams p
 #pragma unroll
         for (int j = 0; j < CPL; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    const int steps = (p.K + 15) / 16;
+    const int steps = p.K / 16;                  // whole ones
     // D k-steps of loads are kept in flight per wavefront (a register ring), so that
-    // 8 wavefronts per CU cover the HBM latency-bandwidth product.
+    // 8 wavefronts per CU cover the HBM latency-bandwidth product.  (Up to 12 in 96 registers were slower: 8 x 4096 x 4096 22.5 | 24.5 us.)
     constexpr int D = 4;
     float a[D][MB][4];
     float bv[D][4][CPL];
+
+    int row[MB];                                 // (rows and columns past the end: the last ones, their sums are not stored)
+#pragma unroll
+    for (int i = 0; i < MB; ++i) row[i] = i * 16 + c < p.M ? i * 16 + c : p.M - 1;
+    // B stored [k][n]: this lane's first column (N >= CPL)
+    const int nb = !RAGGED || n0 + CPL * c < p.N - CPL ? n0 + CPL * c : p.N - CPL;
 
     auto load_step = [&](int d, int s) {
         const int kl = s * 16 + 4 * g;          // this lane's first k
 #pragma unroll
         for (int i = 0; i < MB; ++i) {
-            const int row = i * 16 + c;
-            if constexpr (FAST && !TA) {
-                const floatx4 t = (row < p.M) ? *(const NTG_GLOBAL floatx4*)(A + (int64_t)row * p.lda + kl) : floatx4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (!TA) {
+                const floatx4 t = i * 16 + c < p.M ? *(const NTG_GLOBAL floatx4e*)(A + (int64_t)row[i] * p.lda + kl) : floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int e = 0; e < 4; ++e) a[d][i][e] = t[e];
             } else {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int k = kl + e;
-                    float v = 0.f;
-                    if (row < p.M && k < p.K) v = TA ? A[(int64_t)k * p.lda + row] : A[(int64_t)row * p.lda + k];
-                    a[d][i][e] = v;
-                }
+                for (int e = 0; e < 4; ++e) a[d][i][e] = A[(int64_t)(kl + e) * p.lda + row[i]];
             }
         }
         if constexpr (!TB) {
-            typedef float fv __attribute__((ext_vector_type(CPL)));
+            typedef float fv __attribute__((ext_vector_type(CPL), aligned(4)));
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int k = kl + e;
-                if constexpr (FAST) {
-                    const fv t = *(const NTG_GLOBAL fv*)(B + (int64_t)k * p.ldb + n0 + CPL * c);
+                const fv t = *(const NTG_GLOBAL fv*)(B + (int64_t)(kl + e) * p.ldb + nb);
 #pragma unroll
-                    for (int j = 0; j < CPL; ++j) bv[d][e][j] = t[j];
-                } else {
-#pragma unroll
-                    for (int j = 0; j < CPL; ++j) {
-                        const int n = n0 + CPL * c + j;
-                        bv[d][e][j] = (k < p.K && n < p.N) ? B[(int64_t)k * p.ldb + n] : 0.f;
-                    }
-                }
+                for (int j = 0; j < CPL; ++j) bv[d][e][j] = t[j];
             }
         } else {
 #pragma unroll
             for (int j = 0; j < CPL; ++j) {
                 const int n = n0 + CPL * c + j;
-                if constexpr (FAST) {
-                    const floatx4 t = *(const NTG_GLOBAL floatx4*)(B + (int64_t)n * p.ldb + kl);
+                const floatx4 t = *(const NTG_GLOBAL floatx4e*)(B + (int64_t)(!RAGGED || n < p.N ? n : p.N - 1) * p.ldb + kl);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) bv[d][e][j] = t[e];
-                } else {
+                for (int e = 0; e < 4; ++e) bv[d][e][j] = t[e];
+            }
+        }
+    };
+    auto load_rest = [&]() {                     // the k-step that K does not fill, into slot 0
+        const int kl = steps * 16 + 4 * g;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int k = kl + e;
-                        bv[d][e][j] = (k < p.K && n < p.N) ? B[(int64_t)n * p.ldb + k] : 0.f;
-                    }
-                }
+        for (int e = 0; e < 4; ++e) {
+            const int k = kl + e < p.K ? kl + e : p.K - 1;
+#pragma unroll
+            for (int i = 0; i < MB; ++i) {
+                const float v = TA ? A[(int64_t)k * p.lda + row[i]] : A[(int64_t)row[i] * p.lda + k];
+                a[0][i][e] = kl + e < p.K ? v : 0.f;
+            }
+#pragma unroll
+            for (int j = 0; j < CPL; ++j) {
+                const int n = n0 + CPL * c + j;
+                const float v = TB ? B[(int64_t)(!RAGGED || n < p.N ? n : p.N - 1) * p.ldb + k] : B[(int64_t)k * p.ldb + nb + j];
+                bv[0][e][j] = kl + e < p.K ? v : 0.f;
             }
         }
     };
@@ -140,6 +148,12 @@ __global__ void __launch_bounds__(512) gemm_skinny_f32_kernel(const GemmParams p
             }
         }
     }
+    if constexpr (RAGGED) {
+        if (p.K > steps * 16 && wave == (steps & (NW - 1))) {      // (uniform per wavefront)
+            load_rest();
+            compute(0);
+        }
+    }
 
 #pragma unroll
     for (int i = 0; i < MB; ++i)
@@ -158,11 +172,13 @@ __global__ void __launch_bounds__(512) gemm_skinny_f32_kernel(const GemmParams p
         for (int w = 0; w < NW; ++w) sum += part[w][q][l];     // fixed order: deterministic
         const int r = q & 3, j = (q >> 2) % CPL, i = (q >> 2) / CPL;
         const int m = i * 16 + 4 * (l >> 4) + r;
-        const int n = n0 + CPL * (l & 15) + j;
-        if (m < p.M && n < p.N) {
+        // (a lane whose columns were moved back from the end leaves those that others have)
+        const int first = n0 + CPL * (l & 15), n = (TB || !RAGGED || first < p.N - CPL ? first : p.N - CPL) + j;
+        if (m < p.M && n < p.N && n >= first) {
             NTG_GLOBAL float* cp = C + (int64_t)m * p.ldc + n;
             if (p.cmode == C_ACCUMULATE) sum += *cp;
             else if (p.cmode == C_BIAS) sum += bias[(int64_t)b * p.bias_bs + (int64_t)m * p.bias_rs + (int64_t)n * p.bias_cs];
+            if (p.act == ACT_RELU) sum = sum > 0.f ? sum : 0.f;
             *cp = sum;
         }
     }
@@ -171,12 +187,8 @@ __global__ void __launch_bounds__(512) gemm_skinny_f32_kernel(const GemmParams p
 template <int MB, int CPL, bool TA, bool TB>
 static hipError_t launch_skinny_cfg(const GemmParams& p, hipStream_t s) {
     constexpr int SW = 16 * CPL;
-    const bool a_fast = TA || ((p.lda % 4 == 0) && !p.Aptr && ((reinterpret_cast<uintptr_t>(p.A) & 15) == 0) && (p.sA % 4 == 0));
-    const int bw = TB ? 4 : CPL;    // floats per vector load of B
-    const bool b_fast = (p.ldb % bw == 0) && !p.Bptr && ((reinterpret_cast<uintptr_t>(p.B) & 15) == 0) && (p.sB % 4 == 0);
-    const bool fast = a_fast && b_fast && (p.K % 16 == 0) && (p.N % SW == 0);
-    dim3 grid((unsigned)((p.N + SW - 1) / SW), (unsigned)p.batch);
-    if (fast) hipLaunchKernelGGL((gemm_skinny_f32_kernel<MB, CPL, TA, TB, true>), grid, dim3(512), 0, s, p);
+    const dim3 grid((unsigned)((p.N + SW - 1) / SW), (unsigned)p.batch);
+    if (p.K % 16 || p.N % SW) hipLaunchKernelGGL((gemm_skinny_f32_kernel<MB, CPL, TA, TB, true>), grid, dim3(512), 0, s, p);
     else hipLaunchKernelGGL((gemm_skinny_f32_kernel<MB, CPL, TA, TB, false>), grid, dim3(512), 0, s, p);
     return hipGetLastError();
 }
@@ -196,6 +208,7 @@ static hipError_t launch_skinny_t(bool ta, bool tb, const GemmParams& p, hipStre
 //       column CPL c + j.
 // fp32 accumulation over all of K, one rounding at the end (C0 added in fp32).
 typedef uint32_t su32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t su32x4e __attribute__((ext_vector_type(4), aligned(2)));        // at any element
 typedef __bf16 sbf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 shalfx8 __attribute__((ext_vector_type(8)));
 
@@ -213,7 +226,7 @@ template <> struct Skinny16<DT_BF16> {
     }
 };
 
-template <int DT, int MB, int CPL, bool TA, bool TB, bool FAST>
+template <int DT, int MB, int CPL, bool TA, bool TB, bool RAGGED>
 __global__ void __launch_bounds__(512) gemm_skinny16_kernel(const GemmParams p) {
     using S = Skinny16<DT>;
     using T = typename S::T;
@@ -224,7 +237,7 @@ __global__ void __launch_bounds__(512) gemm_skinny16_kernel(const GemmParams p) 
     __shared__ float part[NW][MB * CPL * 4][64];
 
     const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);      // (scalar: as in the Float32 kernel)
     const int c = lane & 15, g = lane >> 4;
     const int b = blockIdx.y;
     const int n0 = blockIdx.x * SW;
@@ -239,12 +252,17 @@ __global__ void __launch_bounds__(512) gemm_skinny16_kernel(const GemmParams p) 
 #pragma unroll
         for (int j = 0; j < CPL; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    const int steps = (p.K + 31) / 32;
+    const int steps = p.K / 32;                         // whole ones
     constexpr int D = (NB * BW >= 32 || MB * CPL >= 8) ? 2 : 4;   // k-steps of loads in flight per wavefront (register budget)
     su32x4 a[D][MB];
     uint32_t bv[D][NB][BW];
 
-    auto gather8 = [&](auto&& elem) -> su32x4 {          // 8 elements -> 4 packed dwords
+    int row[MB];                                        // (rows and columns past the end: as in the Float32 kernel)
+#pragma unroll
+    for (int i = 0; i < MB; ++i) row[i] = i * 16 + c < p.M ? i * 16 + c : p.M - 1;
+    const int nb = !RAGGED || n0 + CPL * c < p.N - CPL ? n0 + CPL * c : p.N - CPL;
+
+    auto pack8 = [&](auto&& elem) -> su32x4 {            // 8 elements -> 4 packed dwords
         T tmp[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) tmp[e] = elem(e);
@@ -257,54 +275,59 @@ __global__ void __launch_bounds__(512) gemm_skinny16_kernel(const GemmParams p) 
         const int kl = s * 32 + 8 * g;                   // this lane's first k
 #pragma unroll
         for (int i = 0; i < MB; ++i) {
-            const int row = i * 16 + c;
-            if constexpr (FAST && !TA) {
-                a[d][i] = (row < p.M) ? *(const NTG_GLOBAL su32x4*)(A + (int64_t)row * p.lda + kl) : su32x4{0u, 0u, 0u, 0u};
-            } else {
-                a[d][i] = gather8([&](int e) -> T {
-                    const int k = kl + e;
-                    if (row >= p.M || k >= p.K) return (T)0.0f;
-                    return TA ? A[(int64_t)k * p.lda + row] : A[(int64_t)row * p.lda + k];
-                });
-            }
+            // (a real branch: lanes without a row ask the cache for nothing, and the scheduler does not gather a round's requests behind its products,
+            //  which cost the linear layer of 16 x 4096 x 11008 3 %)
+            if constexpr (!TA) a[d][i] = i * 16 + c < p.M ? *(const NTG_GLOBAL su32x4e*)(A + (int64_t)row[i] * p.lda + kl) : su32x4{0u, 0u, 0u, 0u};
+            else a[d][i] = pack8([&](int e) -> T { return A[(int64_t)(kl + e) * p.lda + row[i]]; });
         }
         if constexpr (TB) {
 #pragma unroll
             for (int j = 0; j < CPL; ++j) {
                 const int n = n0 + c + 16 * j;
-                su32x4 t;
-                if constexpr (FAST) {
-                    t = *(const NTG_GLOBAL su32x4*)(B + (int64_t)n * p.ldb + kl);
-                } else {
-                    t = gather8([&](int e) -> T { return (n < p.N && kl + e < p.K) ? B[(int64_t)n * p.ldb + kl + e] : (T)0.0f; });
-                }
+                const su32x4 t = *(const NTG_GLOBAL su32x4e*)(B + (int64_t)(!RAGGED || n < p.N ? n : p.N - 1) * p.ldb + kl);
 #pragma unroll
                 for (int w = 0; w < 4; ++w) bv[d][j][w] = t[w];
             }
         } else {
+            typedef uint16_t bvec __attribute__((ext_vector_type(CPL), aligned(2)));
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const int k = kl + e;
-                const int n = n0 + CPL * c;
-                if constexpr (FAST) {
-                    if constexpr (CPL == 8) {
-                        const su32x4 t = *(const NTG_GLOBAL su32x4*)(B + (int64_t)k * p.ldb + n);
+                const bvec t = *(const NTG_GLOBAL bvec*)(B + (int64_t)(kl + e) * p.ldb + nb);
+                if constexpr (CPL == 1) bv[d][e][0] = t[0];
+                else __builtin_memcpy(&bv[d][e][0], &t, 2 * CPL);
+            }
+        }
+    };
+    auto load_rest = [&]() {                             // the k-step that K does not fill, into slot 0
+        const int kl = steps * 32 + 8 * g;
+        auto at = [&](int e) { return kl + e < p.K ? kl + e : p.K - 1; };
 #pragma unroll
-                        for (int w = 0; w < 4; ++w) bv[d][e][w] = t[w];
-                    } else if constexpr (CPL == 4) {
-                        typedef uint32_t u2 __attribute__((ext_vector_type(2)));
-                        const u2 t = *(const NTG_GLOBAL u2*)(B + (int64_t)k * p.ldb + n);
-                        bv[d][e][0] = t[0];
-                        bv[d][e][1] = t[1];
-                    } else {
-                        bv[d][e][0] = *(const NTG_GLOBAL uint32_t*)(B + (int64_t)k * p.ldb + n);
-                    }
-                } else {
-                    T tmp[2 * BW];
+        for (int i = 0; i < MB; ++i)
+            a[0][i] = pack8([&](int e) -> T {
+                const T v = TA ? A[(int64_t)at(e) * p.lda + row[i]] : A[(int64_t)row[i] * p.lda + at(e)];
+                return kl + e < p.K ? v : (T)0.0f;
+            });
+        if constexpr (TB) {
 #pragma unroll
-                    for (int j = 0; j < 2 * BW; ++j) tmp[j] = (j < CPL && k < p.K && n + j < p.N) ? B[(int64_t)k * p.ldb + n + j] : (T)0.0f;
-                    __builtin_memcpy(&bv[d][e][0], tmp, 4 * BW);
+            for (int j = 0; j < CPL; ++j) {
+                const int n = n0 + c + 16 * j;
+                const su32x4 t = pack8([&](int e) -> T {
+                    const T v = B[(int64_t)(!RAGGED || n < p.N ? n : p.N - 1) * p.ldb + at(e)];
+                    return kl + e < p.K ? v : (T)0.0f;
+                });
+#pragma unroll
+                for (int w = 0; w < 4; ++w) bv[0][j][w] = t[w];
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                T tmp[2 * BW];
+#pragma unroll
+                for (int j = 0; j < 2 * BW; ++j) {
+                    const T v = B[(int64_t)at(e) * p.ldb + nb + (j < CPL ? j : 0)];
+                    tmp[j] = kl + e < p.K ? v : (T)0.0f;
                 }
+                __builtin_memcpy(&bv[0][e][0], tmp, 4 * BW);
             }
         }
     };
@@ -356,6 +379,12 @@ __global__ void __launch_bounds__(512) gemm_skinny16_kernel(const GemmParams p) 
             }
         }
     }
+    if constexpr (RAGGED) {
+        if (p.K > steps * 32 && wave == (steps & (NW - 1))) {      // (uniform per wavefront)
+            load_rest();
+            compute(0);
+        }
+    }
 
 #pragma unroll
     for (int i = 0; i < MB; ++i)
@@ -374,11 +403,13 @@ __global__ void __launch_bounds__(512) gemm_skinny16_kernel(const GemmParams p) 
         for (int w = 0; w < NW; ++w) sum += part[w][q][l];     // fixed order: deterministic
         const int r = q & 3, j = (q >> 2) % CPL, i = (q >> 2) / CPL;
         const int m = i * 16 + 4 * (l >> 4) + r;
-        const int n = n0 + (TB ? (l & 15) + 16 * j : CPL * (l & 15) + j);
-        if (m < p.M && n < p.N) {
+        const int first = n0 + (TB ? (l & 15) : CPL * (l & 15));
+        const int n = TB ? first + 16 * j : (!RAGGED || first < p.N - CPL ? first : p.N - CPL) + j;
+        if (m < p.M && n < p.N && n >= first) {
             NTG_GLOBAL T* cp = C + (int64_t)m * p.ldc + n;
             if (p.cmode == C_ACCUMULATE) sum += (float)*cp;
             else if (p.cmode == C_BIAS) sum += (float)bias[(int64_t)b * p.bias_bs + (int64_t)m * p.bias_rs + (int64_t)n * p.bias_cs];
+            if (p.act == ACT_RELU) sum = sum > 0.f ? sum : 0.f;      // (before the one rounding: the same bits)
             *cp = (T)sum;
         }
     }
@@ -387,12 +418,8 @@ __global__ void __launch_bounds__(512) gemm_skinny16_kernel(const GemmParams p) 
 template <int DT, int MB, int CPL, bool TA, bool TB>
 static hipError_t launch_skinny16_cfg(const GemmParams& p, hipStream_t s) {
     constexpr int SW = 16 * CPL;
-    const bool a_fast = TA || ((p.lda % 8 == 0) && !p.Aptr && ((reinterpret_cast<uintptr_t>(p.A) & 15) == 0) && (p.sA % 8 == 0));
-    const int bw = TB ? 8 : CPL;    // elements per vector load of B
-    const bool b_fast = (p.ldb % bw == 0) && !p.Bptr && ((reinterpret_cast<uintptr_t>(p.B) & 15) == 0) && (p.sB % 8 == 0);
-    const bool fast = a_fast && b_fast && (p.K % 32 == 0) && (p.N % SW == 0);
-    dim3 grid((unsigned)((p.N + SW - 1) / SW), (unsigned)p.batch);
-    if (fast) hipLaunchKernelGGL((gemm_skinny16_kernel<DT, MB, CPL, TA, TB, true>), grid, dim3(512), 0, s, p);
+    const dim3 grid((unsigned)((p.N + SW - 1) / SW), (unsigned)p.batch);
+    if (p.K % 32 || p.N % SW) hipLaunchKernelGGL((gemm_skinny16_kernel<DT, MB, CPL, TA, TB, true>), grid, dim3(512), 0, s, p);
     else hipLaunchKernelGGL((gemm_skinny16_kernel<DT, MB, CPL, TA, TB, false>), grid, dim3(512), 0, s, p);
     return hipGetLastError();
 }
@@ -407,20 +434,25 @@ template <int DT>
 static hipError_t launch_skinny16(bool ta, bool tb, const GemmParams& p, hipStream_t s) {
     // Columns per lane (strip = 16 x that): as many workgroups as possible without exceeding one per CU -- a second
     // round of workgroups costs more than narrower strips gain.  B stored [k][n] is loaded with (2 x columns)-byte
-    // accesses, so 2 columns per lane (4-byte loads) is never worth it there.
-    const int widest = p.M > 16 ? 4 : 8, narrowest = tb ? 2 : 4;
+    // accesses, so 2 columns per lane (4-byte loads) is never worth it there; B stored [n][k] goes down to one column (a lane's load is a row's 16 bytes
+    // of k, a line of its own to the cache whatever the strip, so a CU's rate is what bounds a strip: 8 x 8192 x 480 20.7 us on 15 strips, 13.4 on 30;
+    // 32 x 8192 x 4096 31.0 on 128, 24.2 on 256; 6 x 5229 x 331, rows at any element, 33.8 | 21.5).
+    const int widest = p.M > 16 ? 4 : 8, narrowest = tb ? 1 : 4;
     int cpl = widest;
     for (int cand = widest; cand >= narrowest; cand >>= 1) {
         const int64_t wgs = ((p.N + 16 * cand - 1) / (16 * cand)) * (int64_t)p.batch;
         if (wgs <= 256) cpl = cand;
     }
+    while (!tb && cpl > p.N) cpl >>= 1;                 // (a lane's columns are one load)
     if (p.M <= 16) {
         if (cpl == 8) return launch_skinny16_t<DT, 1, 8>(ta, tb, p, s);
         if (cpl == 4) return launch_skinny16_t<DT, 1, 4>(ta, tb, p, s);
-        return launch_skinny16_t<DT, 1, 2>(ta, tb, p, s);
+        if (cpl == 2) return launch_skinny16_t<DT, 1, 2>(ta, tb, p, s);
+        return launch_skinny16_t<DT, 1, 1>(ta, tb, p, s);
     }
     if (cpl == 4) return launch_skinny16_t<DT, 2, 4>(ta, tb, p, s);
-    return launch_skinny16_t<DT, 2, 2>(ta, tb, p, s);
+    if (cpl == 2) return launch_skinny16_t<DT, 2, 2>(ta, tb, p, s);
+    return launch_skinny16_t<DT, 2, 1>(ta, tb, p, s);
 }
 
 hipError_t launch_gemm_skinny(int dtype, bool ta, bool tb, const GemmParams& p, hipStream_t s, bool* handled) {
@@ -437,6 +469,7 @@ hipError_t launch_gemm_skinny(int dtype, bool ta, bool tb, const GemmParams& p, 
     int cpl = 4;
     if (p.M > 16) cpl = 2;
     while (cpl > 1 && ((p.N + 16 * cpl - 1) / (16 * cpl)) * (int64_t)p.batch < want) cpl >>= 1;
+    while (!tb && cpl > p.N) cpl >>= 1;
     if (p.M <= 16) {
         if (cpl == 4) return launch_skinny_t<1, 4>(ta, tb, p, s);
         if (cpl == 2) return launch_skinny_t<1, 2>(ta, tb, p, s);

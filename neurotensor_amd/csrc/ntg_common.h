@@ -128,7 +128,7 @@ struct GemmParams {
                              // live in device memory, the host cannot look); lets table batches onto the DMA-fed kernels
     int group_m;             // DMA-fed kernels: tile rows per group of the tile order (0: the default, 4; see tile_coords)
     int act;                 // ACT_RELU: the stored result is max(result, 0) (relu_ of the reference = clamp_(x, 0): NaN and -0 become +0);
-                             // honoured by the DMA-fed Float16 / BFloat16 / Float32 kernels, gemm_any_impl.h and the split-K reduction only
+                             // honoured by the DMA-fed Float16 / BFloat16 / Float32 kernels, gemm_any_impl.h, gemm_skinny.hip and the split-K reduction only
     ConvGeom conv;           // used by the implicit-im2col kernels only: B = image, op(B) = col or col^T
 };
 enum { ACT_NONE = 0, ACT_RELU = 1 };

@@ -194,8 +194,8 @@ int launch_gemm(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s) {
     p.vecA_ok = (p.lda % ve == 0) && (p.Aptr || p.sA % ve == 0) && (p.krange_items == 0 || p.sAk % ve == 0);
     p.vecB_ok = (p.ldb % ve == 0) && (p.Bptr || p.sB % ve == 0) && (p.krange_items == 0 || p.sBk % ve == 0);
     hipError_t e;
-    // relu_ on the result: inside the DMA-fed kernel's epilogue where that kernel serves the product (more than 32 rows: the
-    // streaming kernels take the others), else as a pass over C after whichever kernel runs
+    // relu_ on the result: inside the epilogue of the DMA-fed kernels, of those for rows as they lie and of the streaming ones for up to 32 rows,
+    // else as a pass over C after whichever kernel runs
     const int act = p.act;
     p.act = ntg::ACT_NONE;
     if (act != ntg::ACT_NONE) {
@@ -231,9 +231,13 @@ int launch_gemm(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s) {
         bool handled = false;
         // (the streaming kernels for up to 32 rows split k over their wavefronts: not for a caller who wants the one chain)
         e = hipSuccess;
-        if (!(p.keep_k_order && dtype == ntg::DT_F32) && p.krange_items == 0) e = ntg::launch_gemm_skinny(dtype, ta, tb, p, s, &handled);
+        if (!(p.keep_k_order && dtype == ntg::DT_F32) && p.krange_items == 0) {
+            p.act = act;                                                   // (its epilogue clamps)
+            e = ntg::launch_gemm_skinny(dtype, ta, tb, p, s, &handled);
+            p.act = ntg::ACT_NONE;
+        }
         if (e != hipSuccess) return hip_fail(e, "skinny gemm launch");
-        if (handled) return finish();
+        if (handled) return NTG_OK;
         switch (dtype) {
         case ntg::DT_F32: e = ntg::launch_gemm_mfma_f32(ta, tb, p, s); break;
         case ntg::DT_F64: e = ntg::launch_gemm_mfma_f64(ta, tb, p, s); break;
