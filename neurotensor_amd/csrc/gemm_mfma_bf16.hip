@@ -32,15 +32,5 @@ hipError_t launch_conv_nhwc_items_bf16(int edge, const GemmParams& p, int64_t bl
     if (edge == 32) return launch_ring_items_cfg<DT_BF16, 1, true>(p, blocks, s);
     return launch_ring_items_cfg<DT_BF16, 2>(p, blocks, s);
 }
-hipError_t launch_conv_nhwc_dw_bf16(bool ta, const GemmParams& p, hipStream_t s) {
-    const int te = p.conv.tile_edge;
-    if (ta) {
-        if (te == 256) return launch_ring_nhwc_dw_cfg<DT_BF16, 4, true>(p, s);
-        if (te == 64) return launch_ring_nhwc_dw_cfg<DT_BF16, 1, true>(p, s);
-        return launch_ring_nhwc_dw_cfg<DT_BF16, 2, true>(p, s);
-    }
-    if (te == 256) return launch_ring_nhwc_dw_cfg<DT_BF16, 4>(p, s);
-    if (te == 64) return launch_ring_nhwc_dw_cfg<DT_BF16, 1>(p, s);
-    return launch_ring_nhwc_dw_cfg<DT_BF16, 2>(p, s);
-}
+hipError_t launch_conv_nhwc_dw_bf16(bool ta, const GemmParams& p, hipStream_t s) { return launch_ring_nhwc_dw<DT_BF16>(ta, p, s); }
 }  // namespace ntg

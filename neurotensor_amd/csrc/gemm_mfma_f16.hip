@@ -32,15 +32,5 @@ hipError_t launch_conv_nhwc_items_f16(int edge, const GemmParams& p, int64_t blo
     if (edge == 32) return launch_ring_items_cfg<DT_F16, 1, true>(p, blocks, s);
     return launch_ring_items_cfg<DT_F16, 2>(p, blocks, s);
 }
-hipError_t launch_conv_nhwc_dw_f16(bool ta, const GemmParams& p, hipStream_t s) {
-    const int te = p.conv.tile_edge;
-    if (ta) {
-        if (te == 256) return launch_ring_nhwc_dw_cfg<DT_F16, 4, true>(p, s);
-        if (te == 64) return launch_ring_nhwc_dw_cfg<DT_F16, 1, true>(p, s);
-        return launch_ring_nhwc_dw_cfg<DT_F16, 2, true>(p, s);
-    }
-    if (te == 256) return launch_ring_nhwc_dw_cfg<DT_F16, 4>(p, s);
-    if (te == 64) return launch_ring_nhwc_dw_cfg<DT_F16, 1>(p, s);
-    return launch_ring_nhwc_dw_cfg<DT_F16, 2>(p, s);
-}
+hipError_t launch_conv_nhwc_dw_f16(bool ta, const GemmParams& p, hipStream_t s) { return launch_ring_nhwc_dw<DT_F16>(ta, p, s); }
 }  // namespace ntg

@@ -280,9 +280,5 @@ hipError_t launch_conv_nhwc_items_f32(int edge, const GemmParams& p, int64_t blo
     if (edge == 32) return launch_ring_items_cfg<DT_F32, 1, true>(p, blocks, s);
     return edge == 128 ? launch_ring_items_cfg<DT_F32, 2>(p, blocks, s) : launch_ring_items_cfg<DT_F32, 1>(p, blocks, s);
 }
-hipError_t launch_conv_nhwc_dw_f32(bool ta, const GemmParams& p, hipStream_t s) {
-    const bool big = p.conv.tile_edge == 128;
-    if (ta) return big ? launch_ring_nhwc_dw_cfg<DT_F32, 2, true>(p, s) : launch_ring_nhwc_dw_cfg<DT_F32, 1, true>(p, s);
-    return big ? launch_ring_nhwc_dw_cfg<DT_F32, 2>(p, s) : launch_ring_nhwc_dw_cfg<DT_F32, 1>(p, s);
-}
+hipError_t launch_conv_nhwc_dw_f32(bool ta, const GemmParams& p, hipStream_t s) { return launch_ring_nhwc_dw<DT_F32>(ta, p, s); }
 }  // namespace ntg

@@ -191,22 +191,22 @@ __device__ __forceinline__ uint32_t lds_addr_of(const char* p) {
 // (convolution: the tap (c, r, q) is uniform, the pixel per lane; weight gradient: the other way round).  Padding taps
 // and columns / k-rows past the edge read a zero word instead, so the tile in LDS is exact and the multiply loop is the
 // plain one.  Wavefront w gathers k-rows 4 w .. 4 w + 3 of every K-step.
-// WBN_ != 0: a rectangular tile, 64 WB_ rows x 64 WBN_ columns (plain products only).
+// WBN_ != 0: a rectangular tile, 64 WB_ rows x 64 WBN_ columns (plain products and weight gradients).
 // KD_ = 2 (16-bit plain products on 128 x 128 tiles): a K-step is 128 bytes of k per row, so a K-contiguous operand is
 // fetched in whole 128-byte cache lines (half the requests to L2 of the 64-byte K-step) and the one barrier of a K-step
 // comes every sixteen MFMAs instead of every eight; the four stages are 32 KiB each (one workgroup per CU).  Fragments
 // are read two quarter-steps ahead (four sets in registers), the whole of tile kt + 3 is fetched during K-step kt.
 // With WBN_ = 4 (128 x 256 tiles) the stages are 48 KiB and there are three of them: tile kt + 2 is fetched from the
 // barrier of K-step kt - 1 (which frees its stage) to the barrier of K-step kt.
-// entries of the weight gradient's LDS table of window origins (16 + 128 KiB beside the 256 x 256 tile's ring; 14 + 64 KiB
-// on the smaller tiles, so that two workgroups still share a CU)
-constexpr int dw_table_entries(int wb) { return wb == 4 ? 6144 : 3584; }
+// output pixels in a half of the weight gradient's LDS table of window origins (4 KiB: as many workgroups to a CU as without it)
+constexpr int DW_CHUNK = 512;
 
 // Wavefronts per SIMD that an instantiation must leave room for (0: as the compiler sees fit): the 128 x 128 weight gradient in Float32 holds a
 // second set of sums (SEGMENTS below) and, unasked, takes a few registers more than two workgroups a CU can have.
 constexpr int ring_min_waves(int dt, int wb, int conv) { return dt == DT_F32 && wb == 2 && (conv == 4 || conv == 7) ? 2 : 0; }
 
-// FLAT (gathering kernels, A stored [m][k]): the four wavefronts stand side by side, a tile is 32 rows x 128 WB_ columns.
+// FLAT (gathering kernels): the four wavefronts stand side by side, a tile is 32 rows x 128 WB_ columns.  An A stored [k][m] is staged 64 rows wide, of
+// which the first 32 are multiplied (one DMA instruction a wavefront either way).
 template <int DT, bool TA, bool TB, bool RAGGED, int WB_, int CONV = 0, int WBN_ = 0, int KD_ = 1, bool FLAT = false>
 __global__ void __launch_bounds__(256, ring_min_waves(DT, FLAT ? 1 : WB_, CONV)) gemm_ring_kernel(const GemmParams pin) {
     using E = Elem<DT>;
@@ -214,15 +214,15 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, FLAT ? 1 : WB_, CONV))
     constexpr int ES = sizeof(T);
     constexpr int WBM = FLAT ? 1 : WB_, WBN = WBN_ ? WBN_ : WB_;      // 32 x 32 blocks per wavefront along m / along n
     constexpr int WB = FLAT ? 2 * WBN : WBN;             // DMA instructions per wavefront for 64 bytes of k of the B tile, whose 64 WB columns a gathering kernel fills
-    static_assert(CONV == 0 || FLAT || WBM == WBN, "gathering kernels have square tiles, or flat ones");
-    static_assert(!FLAT || ((CONV == 3 || CONV == 5 || CONV == 6 || CONV == 8 || CONV == 9 || CONV == 10) && !TA && WBN_ == 0 && KD_ == 1), "flat tiles: channels-last convolutions, A stored [m][k]");
+    static_assert(CONV == 0 || FLAT || WBM == WBN || CONV == 4 || CONV == 7, "convolutions have square tiles, or flat ones");
+    static_assert(!FLAT || (CONV >= 3 && WBN_ == 0 && KD_ == 1), "flat tiles: channels-last convolutions and weight gradients");
     constexpr int KD = KD_;
     static_assert(KD == 1 || (KD == 2 && CONV == 0 && (ES == 2 || ES == 1) && WB_ == 2 && (WBN_ == 0 || WBN_ == 4)), "deep K-steps: 16- and 8-bit plain products on 128 x 128 and 128 x 256 tiles");
     constexpr bool RING3 = KD == 2 && WBN_ == 4;         // three stages of 48 KiB
     using GA = RingGeom<WBM, ES, KD>;                    // geometry of the A tile (flat: twice its rows)
     using G = RingGeom<WB, ES, KD>;                      // geometry of the B tile
     constexpr int BM = FLAT ? 32 : GA::BM;
-    constexpr int A_TILE_BYTES = BM * G::KB, STAGE_BYTES = A_TILE_BYTES + G::TILE_BYTES;
+    constexpr int A_TILE_BYTES = (TA ? GA::BM : BM) * G::KB, STAGE_BYTES = A_TILE_BYTES + G::TILE_BYTES;
     constexpr int WTM = 32 * WBM, WTN = 32 * WBN;        // a wavefront's share of the tile: WTM rows x WTN columns
     constexpr bool GATHER4 = CONV == 1 || CONV == 2;     // op(B) gathered element by element from an NCHW image
     constexpr bool ITEMS = CONV == 8 || CONV == 10;      // several convolutions of one bordered image in one launch, each described by a RingItem
@@ -231,7 +231,7 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, FLAT ? 1 : WB_, CONV))
     constexpr bool HALO = CONV == 5 || CONV == 6 || ITEMS || SLOTS;   // ... whose copy carries the padding as pixels of zeros: every tap of every window exists
     constexpr bool DEPTH = CONV == 6 || ITEMS || SLOTS;  // ... over three spatial axes
     constexpr bool GATHERW = CONV == 4 || CONV == 7;     // op(B) = col^T of a channels-last image, 16-byte pieces along the channels (weight gradient)
-    constexpr bool DEPTHW = CONV == 7;                   // ... of a bordered copy over two or three axes, pixel by division (no table of window origins)
+    constexpr bool HALOW = CONV == 7;                    // ... of a bordered copy over one to three axes
     constexpr bool A_KC = !TA, B_KC = GATHER4 ? false : GATHER16 ? true : GATHERW ? false : TB;
     constexpr int BK = G::BK;
     static_assert(!GATHER4 || (ES == 4 && !TA && RAGGED), "gathered operands: Float32, A stored [m][k], guarded edges");
@@ -246,9 +246,8 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, FLAT ? 1 : WB_, CONV))
     __shared__ __attribute__((aligned(1024))) char st1[STAGE_BYTES];
     __shared__ __attribute__((aligned(1024))) char st2[STAGE_BYTES];
     __shared__ __attribute__((aligned(1024))) char st3[RING3 ? 1024 : STAGE_BYTES];
-    // channels-last weight gradient: byte offset of every output pixel's window origin inside one (bordered) image
-    constexpr int DW_TABLE = CONV == 4 ? dw_table_entries(WB) : 1;   // (CONV = 7 has none)
-    __shared__ int dw_tab[DW_TABLE];
+    // bordered weight gradient: offset of the output pixels' window origins, in 16 bytes, two chunks of them
+    __shared__ uint32_t dw_tab[HALOW ? 2 * DW_CHUNK : 1];
     // ... byte offset from a window's origin of every 16-byte slot of k
     __shared__ int slot_tab[SLOTS ? NTG_SLOT_TABLE + 16 : 1];
 
@@ -354,9 +353,9 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, FLAT ? 1 : WB_, CONV))
     const int nvalid = p.N - n0 < G::BN ? p.N - n0 : G::BN;
     uint32_t offA[WBM * KD], offB[WB * KD];       // K-steps before the last
     uint32_t offAt[WBM * KD], offBt[WB * KD];     // the last K-step (RAGGED: k clamped to what exists)
-    // (a flat tile's A is two instructions, which wavefronts 2 and 3 issue a second time: the same bytes to the same place, and every
+    // (a flat tile's A stored [m][k] is two instructions, which wavefronts 2 and 3 issue a second time: the same bytes to the same place, and every
     //  wavefront counts the same loads)
-    const int wave_a = FLAT ? wave & 1 : wave, wave_a_u = FLAT ? wave_u & 1 : wave_u;
+    const int wave_a = FLAT && !TA ? wave & 1 : wave, wave_a_u = FLAT && !TA ? wave_u & 1 : wave_u;
     dma_offsets<A_KC, RAGGED, WBM, ES, KD>(offA, p.lda, wave_a, lane, mvalid, BK);
     dma_offsets<B_KC, RAGGED, WB, ES, KD>(offB, p.ldb, wave, lane, nvalid, BK);
     dma_offsets<A_KC, RAGGED, WBM, ES, KD>(offAt, p.lda, wave_a, lane, mvalid, kr);
@@ -609,8 +608,10 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, FLAT ? 1 : WB_, CONV))
     // split into (row, column) with one multiply-shift division per instruction.  Padding and k >= K read zeros.
     // Items that are k ranges (p.conv.k_ranges, fold_L = output pixels per image) count k through the output pixels of all
     // images, and one more division gives the image, p.conv.fold_stride elements apart.
-    // CONV = 7: the copy carries its padding as zeros (the only form for three spatial axes, and what large output planes take),
-    // which needs no validity test; without the table its LDS lets a fourth 64 x 64 workgroup onto the CU.
+    // CONV = 7: the copy carries its padding as zeros (the only form for three spatial axes), so every tap of every window exists, and the pixels' window
+    // origins come from a table in LDS: chunks of DW_CHUNK output pixels, two at a time, written by all threads while the chunk before is being read; a lane
+    // reads its pixel's entry one K-step ahead, and an instruction's address is one addition.  Three divisions an instruction, which large planes
+    // and three axes took before, were several times the matrix work of a 16-bit K-step and half of a Float32 one.
     int krow4[WB], noff4[WB];
     uint32_t tap4[WB];
     int k4_k = 0, k4_base = 0;
@@ -635,79 +636,63 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, FLAT ? 1 : WB_, CONV))
                        (int)c * ES;
         }
     }
-    // Table form (p.conv.pix_table = output pixels per image, at most DW_TABLE - BK; the copy of the image carries its padding
-    // as pixels of zeros, so every tap of every window exists): the window origin's byte offset of each output pixel is
-    // computed once per workgroup into LDS, BK entries of zeros behind them.  A K-step then lies inside ONE image (per-image
-    // items, or k ranges whose images are whole K-steps): image and first pixel are wave-uniform counters, a lane reads its
-    // pixel's entry one K-step ahead, and the per-instruction work is two additions instead of two divisions and the tests.
-    int pre4[WB];
-    int t4_pix = 0, t4_pixn = 0;
-    int64_t t4_img = 0, t4_imgn = 0;
-    if constexpr (GATHERW) {
-        const ConvGeom& g = p.conv;
-        if (!DEPTHW && g.pix_table) {                             // (uniform)
-            const int Lp = g.pix_table;
-            for (int i = tid; i < Lp + BK; i += 256) {
-                const uint32_t oh = fast_div((uint32_t)i, g.div_wo), ow = (uint32_t)i - oh * (uint32_t)g.Wo;
-                dw_tab[i] = i < Lp ? (int)((oh * (uint32_t)g.s_r * (uint32_t)g.W + ow * (uint32_t)g.s_c) * (uint32_t)g.chan * (uint32_t)ES) : 0;
-            }
-            __syncthreads();
-            if (g.k_ranges) {
-                const uint32_t im0 = fast_div((uint32_t)k4_base, g.div_fold);
-                t4_pix = k4_base - (int)im0 * Lp;
-                t4_img = (int64_t)im0 * g.fold_stride * ES;
-            }
-            t4_pixn = t4_pix + BK;
-            t4_imgn = t4_img;
-            if (g.k_ranges && t4_pixn >= Lp) { t4_pixn -= Lp; t4_imgn += g.fold_stride * ES; }
+    uint32_t pre4[WB];
+    const char* tap_base[WB];
+    const uint32_t im0 = HALOW && p.conv.k_ranges ? fast_div((uint32_t)k4_base, p.conv.div_fold) : 0u;      // the image of the item's first pixel
+    auto fill_pixels = [&](int chunk) __attribute__((always_inline)) {
+        if constexpr (HALOW) {
+            const ConvGeom& g = p.conv;
 #pragma unroll
-            for (int x = 0; x < WB; ++x) pre4[x] = dw_tab[t4_pix + (krow4[x] & 63)];
+            for (int i = 0; i < DW_CHUNK / 256; ++i) {
+                const uint32_t j = (uint32_t)(chunk * DW_CHUNK + 256 * i + tid);
+                uint32_t li = j + (uint32_t)k4_base, im = 0u;
+                if (g.k_ranges) {                                  // (uniform)
+                    im = fast_div(li, g.div_fold);
+                    li -= im * (uint32_t)g.fold_L;
+                    im -= im0;
+                }
+                const uint32_t od = fast_div(li, g.div_howo);
+                li -= od * (uint32_t)g.HoWo;
+                const uint32_t oh = fast_div(li, g.div_wo), ow = li - oh * (uint32_t)g.Wo;
+                const uint32_t row = oh * (uint32_t)g.s_r + od * (uint32_t)(g.s_d * g.H);
+                // (a pixel of the copy is whole 16 bytes; pixels past the last one are never used)
+                dw_tab[j & (2 * DW_CHUNK - 1)] = im * (uint32_t)(g.fold_stride * ES / 16) + (row * (uint32_t)g.W + ow * (uint32_t)g.s_c) * (uint32_t)(g.chan * ES / 16);
+            }
+        }
+    };
+    if constexpr (HALOW) {
+        fill_pixels(0);
+        fill_pixels(1);
+        __syncthreads();
+#pragma unroll
+        for (int x = 0; x < WB; ++x) {
+            pre4[x] = dw_tab[krow4[x] & 63];
+            tap_base[x] = reinterpret_cast<const char*>(B) + (int64_t)im0 * p.conv.fold_stride * ES + (int64_t)noff4[x];
         }
     }
     auto conv4_dma = [&](int x, uint32_t lds_tile) __attribute__((always_inline)) {
         if constexpr (GATHERW) {
             const ConvGeom& g = p.conv;
-            const char* img = reinterpret_cast<const char*>(B);
-            if (!DEPTHW && g.pix_table) {                          // (uniform)
-                const uint32_t lk = (uint32_t)(k4_k + krow4[x]);
-                const char* src = lk < (uint32_t)K ? img + (t4_img + (int64_t)(pre4[x] + noff4[x])) : reinterpret_cast<const char*>(ring_zero_word);
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                             :: "s"(lds_tile + (uint32_t)(wave_u * WB + x) * 1024u), "v"(src) : "memory");
-                const int pn = t4_pixn < g.pix_table ? t4_pixn : g.pix_table;      // (K-steps past the end: the zeros behind the table)
-                pre4[x] = dw_tab[pn + (krow4[x] & 63)];
-                if (x == WB - 1) {
-                    k4_k += BK;
-                    t4_pix = t4_pixn; t4_img = t4_imgn;
-                    t4_pixn += BK;
-                    if (g.k_ranges && t4_pixn >= g.pix_table) { t4_pixn -= g.pix_table; t4_imgn += g.fold_stride * ES; }
-                }
-                return;
-            }
-            const uint32_t lk = (uint32_t)(k4_k + krow4[x]), l = lk + (uint32_t)k4_base;
-            uint32_t li = l, im = 0u;
-            if (g.k_ranges) {                                      // (uniform)
-                im = fast_div(l, g.div_fold);
-                li = l - im * (uint32_t)g.fold_L;
-            }
-            bool ok = lk < (uint32_t)K;
-            uint32_t oh, ow;
-            if constexpr (DEPTHW) {
-                const uint32_t od = fast_div(li, g.div_howo);
-                li -= od * (uint32_t)g.HoWo;
-                oh = fast_div(li, g.div_wo);
-                ow = li - oh * (uint32_t)g.Wo;
-                oh = oh * (uint32_t)g.s_r + od * (uint32_t)(g.s_d * g.H);
+            const uint32_t lk = (uint32_t)(k4_k + krow4[x]);
+            const char* src;
+            if constexpr (HALOW) {
+                src = lk < (uint32_t)K ? tap_base[x] + ((uint64_t)pre4[x] << 4) : reinterpret_cast<const char*>(ring_zero_word);
             } else {
-                oh = fast_div(li, g.div_wo);
-                ow = li - oh * (uint32_t)g.Wo;
-                oh *= (uint32_t)g.s_r;
-                const int ih0 = (int)oh - g.p_r, iw0 = (int)ow * g.s_c - g.p_c;
-                ok = ok & ((uint32_t)(ih0 + (int)(tap4[x] & 0xffffu)) < (uint32_t)g.H) & ((uint32_t)(iw0 + (int)(tap4[x] >> 16)) < (uint32_t)g.W);
+                const uint32_t l = lk + (uint32_t)k4_base;
+                uint32_t li = l, im = 0u;
+                if (g.k_ranges) {                                  // (uniform)
+                    im = fast_div(l, g.div_fold);
+                    li = l - im * (uint32_t)g.fold_L;
+                }
+                const uint32_t oh = fast_div(li, g.div_wo), ow = li - oh * (uint32_t)g.Wo;
+                const int ih0 = (int)(oh * (uint32_t)g.s_r) - g.p_r, iw0 = (int)ow * g.s_c - g.p_c;
+                const bool ok = (lk < (uint32_t)K) & ((uint32_t)(ih0 + (int)(tap4[x] & 0xffffu)) < (uint32_t)g.H) & ((uint32_t)(iw0 + (int)(tap4[x] >> 16)) < (uint32_t)g.W);
+                const int off = (int)((oh * (uint32_t)g.s_r * (uint32_t)g.W + ow * (uint32_t)g.s_c) * (uint32_t)g.chan * (uint32_t)ES) + noff4[x];
+                src = ok ? reinterpret_cast<const char*>(B) + ((int64_t)im * g.fold_stride * ES + (int64_t)off) : reinterpret_cast<const char*>(ring_zero_word);
             }
-            const int off = (int)((oh * (uint32_t)g.W + ow * (uint32_t)g.s_c) * (uint32_t)g.chan * (uint32_t)ES) + noff4[x];
-            const char* src = ok ? img + ((int64_t)im * g.fold_stride * ES + (int64_t)off) : reinterpret_cast<const char*>(ring_zero_word);
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
                          :: "s"(lds_tile + (uint32_t)(wave_u * WB + x) * 1024u), "v"(src) : "memory");
+            if constexpr (HALOW) pre4[x] = dw_tab[((k4_k + BK) & (2 * DW_CHUNK - 1)) + (krow4[x] & 63)];
             if (x == WB - 1) k4_k += BK;
         }
     };
@@ -926,7 +911,7 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, FLAT ? 1 : WB_, CONV))
             else if (nrd == 1) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             if constexpr (NGATHER > 0) {
                 // the gather's address arithmetic, dealt out evenly: what does not fit under one MFMA delays the next
-                constexpr int VPG = GATHERW ? 20 : 8;          // vector instructions per gathering DMA, roughly
+                constexpr int VPG = CONV == 4 ? 20 : 8;          // vector instructions per gathering DMA, roughly
                 __builtin_amdgcn_sched_group_barrier(0x002, (VPG * NGATHER + NMMA - 1) / NMMA + 1, 0);   // VALU
                 __builtin_amdgcn_sched_group_barrier(0x004, (10 * NGATHER + NMMA - 1) / NMMA, 0);      // SALU
             }
@@ -1097,6 +1082,13 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, FLAT ? 1 : WB_, CONV))
         }
     } else
     for (int kt = 0; kt < KT; kt += 4) {
+        if constexpr (HALOW) {
+            // K-step kt reads the entries of K-step kt + 4.  Where those are a chunk's first, every wavefront read its last entry of the chunk before
+            // ahead of the barrier of K-step kt - 1: the chunk after the next takes its place, many barriers before it is read.
+            constexpr int S = DW_CHUNK / BK;
+            static_assert(S % 4 == 0, "a chunk of pixels is whole rounds of this loop");
+            if ((kt + 4) % S == 0 && (kt + 4) * BK + DW_CHUNK < K) fill_pixels((kt + 4) / S + 1);      // (uniform)
+        }
         if constexpr (KD == 2) {
             iteration_deep(kt, st0, st1, st3);
             if (kt + 1 < KT) iteration_deep(kt + 1, st1, st2, st0);
@@ -1414,20 +1406,33 @@ static hipError_t launch_ring_nhwc_cfg(const GemmParams& pin, hipStream_t s) {
 }
 
 // weight gradient of a convolution with op(B) gathered from a channels-last image (see CONV = 4 and 7)
-template <int DT, int WB, bool TA = false>
+template <int DT, bool TA, int WB, int WBN = 0, bool FLAT = false>
 static hipError_t launch_ring_nhwc_dw_cfg(const GemmParams& pin, hipStream_t s) {
-    constexpr int TE = 64 * WB;
+    constexpr int WBC = FLAT ? 2 * WB : WBN ? WBN : WB, TM = FLAT ? 32 : 64 * WB, TN = 64 * WBC;
     GemmParams p = pin;
-    p.tiles_m = (p.M + TE - 1) / TE;
-    p.tiles_n = (p.N + TE - 1) / TE;
+    p.tiles_m = (p.M + TM - 1) / TM;
+    p.tiles_n = (p.N + TN - 1) / TN;
     const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n * p.batch;
     if (blocks <= 0) return hipSuccess;
     if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    // (more output pixels per image than the table holds: the divisions per instruction, which serve a bordered copy as well)
-    if (p.conv.pix_table + 64 > dw_table_entries(WB)) p.conv.pix_table = 0;
-    if (p.conv.halo && !p.conv.pix_table) hipLaunchKernelGGL((gemm_ring_kernel<DT, TA, false, true, WB, 7>), dim3((unsigned)blocks), dim3(256), 0, s, p);
-    else hipLaunchKernelGGL((gemm_ring_kernel<DT, TA, false, true, WB, 4>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+    if (p.conv.halo) hipLaunchKernelGGL((gemm_ring_kernel<DT, TA, false, true, WB, 7, WBN, 1, FLAT>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((gemm_ring_kernel<DT, TA, false, true, WB, 4, WBN, 1, FLAT>), dim3((unsigned)blocks), dim3(256), 0, s, p);
     return hipGetLastError();
+}
+// ... on the tile that the caller planned with (p.conv.tile_rows x tile_cols)
+template <int DT, bool TA>
+static hipError_t launch_ring_nhwc_dw_tile(const GemmParams& p, hipStream_t s) {
+    const int rows = p.conv.tile_rows, cols = p.conv.tile_cols;
+    if (rows == 32) return launch_ring_nhwc_dw_cfg<DT, TA, 1, 0, true>(p, s);
+    if (rows == 64) return cols == 128 ? launch_ring_nhwc_dw_cfg<DT, TA, 1, 2>(p, s) : launch_ring_nhwc_dw_cfg<DT, TA, 1>(p, s);
+    if constexpr (DT != DT_F32) {
+        if (rows == 256) return launch_ring_nhwc_dw_cfg<DT, TA, 4>(p, s);
+    }
+    return launch_ring_nhwc_dw_cfg<DT, TA, 2>(p, s);
+}
+template <int DT>
+static hipError_t launch_ring_nhwc_dw(bool ta, const GemmParams& p, hipStream_t s) {
+    return ta ? launch_ring_nhwc_dw_tile<DT, true>(p, s) : launch_ring_nhwc_dw_tile<DT, false>(p, s);
 }
 
 template <int DT, int WB, int WBN = 0, int KD = 1>

@@ -75,14 +75,11 @@ struct ConvGeom {
     int k_ranges, k_total, a_steps;
     FastDiv div_a_steps;
     int64_t a_image_stride;
-    // channels-last weight gradient on a copy that carries the padding as pixels of zeros (H, W describe the padded image,
-    // p_r = p_c = 0): output pixels per image when the kernel keeps their window origins in an LDS table, 0: off
-    int pix_table;
     // channels-last convolution, several products in one launch: their table in device memory (see RingItem)
     const struct RingItem* items;
     int n_items;
     int k_segment;           // Float32 weight gradients and `items`: K-steps of one chain of multiply-adds (a power of two; 0: all of them)
-    int tile_edge;           // channels-last weight gradient: the edge of the tile the caller planned with
+    int tile_rows, tile_cols;      // channels-last weight gradient: the tile the caller planned with
     // channels-last convolution on a bordered copy, k in 16-byte slots (taps outermost): slots of a tap; 0: whole 64-byte runs
     int slot_v;
     FastDiv div_slot;

@@ -1851,23 +1851,29 @@ static HaloPlan dkernel_halo(int64_t es, int64_t cg, int64_t groups, const Geo3&
     }
     return h;
 }
-// What a launch of the gathering kernel takes: microseconds for `tiles` tiles of edge x edge with K output pixels each, by how many
-// workgroups share a CU; the writes of the partial sums are the caller's.  Float32, from profiles/conv_weight_gradient_gather_sweep.txt without
-// those writes (4.7 TB/s): 8 us and, per pixel, 29 ns for a 64 x 64 tile alone on its CU, 22 ns each for several; 128 x 128: 79 and 68, so large
-// tiles where the gradient has the rows and columns for them (64 x 128 x 28 x 28 -> 128 by 3 x 3, a step: 438 us on
-// 64 x 64 tiles, 419).  16-bit: 0.41 of a CU's MFMA
-// peak on 256 x 256 tiles; 0.35 on 128 x 128 tiles when two workgroups share a CU, 0.245 when one has it alone; a 64 x 64 tile 9 ns per
-// pixel alone, 4.2 ns each for several, and 3 us (the sweep reads 0.46, 0.41, 0.29, 7.5 and 5.1 ns, and 8 us).
-static double dkernel_cost_us(int64_t es, int edge, int64_t tiles, int64_t K) {
+// What a launch of the gathering kernel takes: microseconds for `tiles` tiles of rows x cols with K output pixels each, by how many workgroups share a
+// CU; the writes of the partial sums are the caller's.  Nanoseconds a pixel and tile, alone on its CU and for each of several:
+//   Float32  64 x 64 25, 18.5 (the matrix pipe takes 13.3)   64 x 128 40, 33   32 x 128 26, 19.5   128 x 128 72, 60
+//   16-bit   64 x 64 7.5, 3.5                                64 x 128 8.5, 5.5   32 x 128 7.5, 4.6   larger ones by their share of a CU's MFMA peak
+// Wide tiles read the output gradient and wait at the barrier half as often, flat ones do half the work where a group has up to 32 out channels.  us of the
+// gradient on 64 x 64 | 64 x 128 | 32 x 128: Float32 4 x 32 x 32^3 -> 64 by 3 x 3 x 3 158 | 144 | 171, 32 x 3 x 224 x 224 -> 64 by 7 x 7 at stride 2 142 | 134 |
+// 151, 20 x 256 x 193 x 193 -> 16 by 3 x 3 in 4 groups 2216 | 2227 | 1433, 32 x 32 x 64 x 64 -> 32 by 5 x 5 139 | 143 | 95; Float16 8 x 64 x 32^3 -> 64 by 3 x 3 x 3
+// 130 | 110 | 146, 13 x 48 x 128 x 128 -> 48 by 5 x 5 in 2 groups 82 | 64 | 57.  (32 x 256 was never the fastest.)
+static double dkernel_cost_us(int64_t es, int rows, int cols, int64_t tiles, int64_t K) {
     const double w = (double)((tiles + 255) / 256), k = (double)K;
-    if (es == 4) return 8.0 + k * (edge == 128 ? std::max(0.079, 0.068 * w) : std::max(0.029, 0.022 * w));
-    const double cu_flops_per_us = 9.77e6, area = (double)edge * edge;
-    if (edge == 256) return w * (2.0 * area * k / (cu_flops_per_us * 0.41) + 6.0);
-    if (edge == 128) {
-        if (tiles <= 256) return 2.0 * area * k / (cu_flops_per_us * 0.245) + 3.0;
-        return (double)((tiles + 511) / 512) * (4.0 * area * k / (cu_flops_per_us * 0.35) + 3.0);
+    if (es == 4) {
+        const double alone = rows == 128 ? 0.072 : rows == 32 ? 0.026 : cols == 128 ? 0.040 : 0.025;
+        const double each = rows == 128 ? 0.060 : rows == 32 ? 0.0195 : cols == 128 ? 0.033 : 0.0185;
+        return 8.0 + k * std::max(alone, each * w);
     }
-    return 3.0 + k * std::max(0.009, 0.0042 * w);
+    const double cu_flops_per_us = 9.77e6, area = (double)rows * cols;
+    if (rows == 256) return w * (2.0 * area * k / (cu_flops_per_us * 0.45) + 6.0);
+    if (rows == 128) {
+        if (tiles <= 256) return 2.0 * area * k / (cu_flops_per_us * 0.27) + 3.0;
+        return (double)((tiles + 511) / 512) * (4.0 * area * k / (cu_flops_per_us * 0.41) + 3.0);
+    }
+    const double alone = cols == 64 || rows == 32 ? 0.0075 : 0.0085, each = cols == 64 ? 0.0035 : rows == 32 ? 0.0046 : 0.0055;
+    return 3.0 + k * std::max(alone, each * w);
 }
 // How dW is cut up: `ranges` k ranges of `kr` output pixels (0: one product per image), tiles of edge x edge, dY read where it
 // lies (its rows 16-byte multiples, an image a whole number of K-steps) or through a channels-last copy of its own (any range then), with
@@ -1880,7 +1886,7 @@ static double dkernel_cost_us(int64_t es, int edge, int64_t tiles, int64_t K) {
 // channels on 4 volumes of 32^3 in Float32: 56 workgroups of 32768 pixels, 1285 us), and a 7 x 7 map of 64 images with 64
 // times the partial sums it needs; the ranges are chosen so that tiles x ranges fill whole rounds over the CUs, against the
 // cost of writing and reading the partial sums (4 TB/s) and of the copy of dY.
-struct DkernelPlan { bool ok, copy_dy; int64_t ranges, kr, items; int edge; };
+struct DkernelPlan { bool ok, copy_dy; int64_t ranges, kr, items; int rows, cols; };      // rows x cols: the tile
 static DkernelPlan plan_dkernel(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
     DkernelPlan pl;
     std::memset(&pl, 0, sizeof pl);
@@ -1897,6 +1903,7 @@ static DkernelPlan plan_dkernel(int dtype, int64_t batch, int64_t channels, int6
     const bool countable = total < (1LL << 30);
     const bool lies = rows_16 && L % bk == 0 && countable, copied = countable;
     if (!rows_16 && !copied) return pl;
+    const int64_t volp = dkernel_halo(es, cg, groups, g).vol;
     pl.ok = true;
     // measurement and test knob: NTG_DW_RANGES=r forces r ranges of dY where it lies where r is admissible, 0 one product per image
     const char* env = rows_16 ? std::getenv("NTG_DW_RANGES") : nullptr;
@@ -1904,33 +1911,36 @@ static DkernelPlan plan_dkernel(int dtype, int64_t batch, int64_t channels, int6
     if (lies && forced > 0 && steps % forced == 0) {
         pl.ranges = pl.items = forced;
         pl.kr = total / forced;
-        pl.edge = es == 2 ? ntg::ring16_tile_edge(og, N, pl.kr, forced) : 64;
+        pl.rows = pl.cols = es == 2 ? ntg::ring16_tile_edge(og, N, pl.kr, forced) : 64;
     } else {
         // A range has the pixels of an image at least, where those are two to eight K-steps: over small maps longer ranges are few and cost
         // time, as the groups run one behind the other (58 x 64 x 17 -> 64 by 5 in 8 groups: backward 136 us, 108 with short ranges), while
         // shorter ones ask for a larger workspace than one gradient per image.
         const int64_t shortest = std::min<int64_t>(8, std::max<int64_t>(2, (L + bk - 1) / bk));
         double best = 0.0;
-        const auto consider = [&](bool copy, int64_t ranges, int64_t items, int64_t kr, int edge) {
-            const int64_t tiles = ((og + edge - 1) / edge) * ((N + edge - 1) / edge) * items * groups;
-            const double us = (copy ? 4.0 + (double)(total * (out_channels + groups * ogp) * es) / 4.5e6 : 0.0) + dkernel_cost_us(es, edge, tiles, kr) + 4.0 +
+        const auto consider = [&](bool copy, int64_t ranges, int64_t items, int64_t kr, int rows, int cols) {
+            const int64_t tiles = ((og + rows - 1) / rows) * ((N + cols - 1) / cols) * items * groups;
+            const double us = (copy ? 4.0 + (double)(total * (out_channels + groups * ogp) * es) / 4.5e6 : 0.0) + dkernel_cost_us(es, rows, cols, tiles, kr) + 4.0 +
                               2.0 * (double)(items * groups * (copy ? ogp : og) * N * 4) / 4.0e6;
-            if (pl.edge && us >= best) return;
+            if (pl.rows && us >= best) return;
+            if ((kr / L + 2) * groups * cgp * volp * es >= (1LL << 36)) return;  // (window origins in 16 bytes from the range's first image: 32 bits)
             best = us;
-            pl.copy_dy = copy; pl.ranges = ranges; pl.items = items; pl.kr = kr; pl.edge = edge;
+            pl.copy_dy = copy; pl.ranges = ranges; pl.items = items; pl.kr = kr; pl.rows = rows; pl.cols = cols;
         };
-        for (int edge : {256, 128, 64}) {
-            if (es == 4 && edge == 256) continue;
-            if (rows_16) consider(false, 0, batch, L, edge);
+        struct { int rows, cols; } const shapes[] = {{256, 256}, {128, 128}, {64, 64}, {64, 128}, {32, 128}};
+        for (const auto [rows, cols] : shapes) {
+            if (es == 4 && rows == 256) continue;
+            if (rows_16) consider(false, 0, batch, L, rows, cols);
             if (env) continue;
-            const int64_t tiles = ((og + edge - 1) / edge) * ((N + edge - 1) / edge) * groups;
+            const int64_t tiles = ((og + rows - 1) / rows) * ((N + cols - 1) / cols) * groups;
             for (int64_t target : {256, 512, 768, 1024, 1536, 2048}) {
                 const int64_t want = std::min(std::max<int64_t>(target / tiles, 1), std::max<int64_t>(steps / shortest, 1));
                 const int64_t per = (steps + want - 1) / want, r = (steps + per - 1) / per;
-                if (lies) consider(false, r, r, per * bk, edge);
-                if (copied) consider(true, r, r, per * bk, edge);
+                if (lies) consider(false, r, r, per * bk, rows, cols);
+                if (copied) consider(true, r, r, per * bk, rows, cols);
             }
         }
+        pl.ok = pl.rows != 0;
     }
     return pl;
 }
@@ -1971,8 +1981,7 @@ static int conv_dkernel_nhwc(int dtype, const DkernelPlan& pl, const void* image
     fill_conv_geom(p.conv, cgp, halo.gp);
     p.conv.chan = (int)chp;                        // elements from one pixel to the next
     p.conv.halo = halo.on ? 1 : 0;
-    if (halo.on && g.nd == 2 && L < (1 << 20) && (pl.ranges == 0 || L % bk == 0)) p.conv.pix_table = (int)L;     // (a K-step inside one image: see the kernel)
-    p.conv.tile_edge = pl.edge;
+    p.conv.tile_rows = pl.rows; p.conv.tile_cols = pl.cols;
     p.conv.k_segment = chain_steps(L);
     if (pl.ranges) {
         p.conv.k_ranges = 1;

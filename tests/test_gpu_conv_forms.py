@@ -215,3 +215,21 @@ def test_taps_in_slots_dilated_and_the_longest_table():
 ], ids=str)
 def test_channels_in_ranges(dtype, batch, cin, cout, size, kernel, stride, pad):
     check(dtype, batch, cin, cout, size, kernel, stride, pad, 1, False, ("dx",) if stride > 1 else ())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("ranges", [None, "0", "1"])
+@pytest.mark.parametrize("batch,cin,cout,size,kernel,stride,pad,groups", [
+    (3, 16, 16, (1600,), 3, 1, 1, 1),            # chunks of 512 pixels that images cross, one row of flat tiles
+    (2, 24, 33, (40, 40), 3, 1, 1, 1),           # one row past a flat tile
+    (5, 8, 64, (32, 32), 5, 1, 2, 1),            # 200 columns: a wide tile and part of one
+    (2, 32, 65, (65, 63), 3, 2, 1, 1),           # strides, one row past a tile
+    (2, 16, 48, (12, 16, 20), 3, 1, 1, 2),       # three axes, groups of 24 rows
+    (1, 8, 8, (23, 41), 1, 1, 0, 1),             # under two chunks
+    (40, 64, 128, (8, 8), 3, 1, 1, 1),           # many images a chunk
+])
+def test_weight_gradients_through_the_table_of_pixels(monkeypatch, dtype, ranges, batch, cin, cout, size, kernel, stride, pad, groups):
+    """As planned, one product an image, and one range over all images (the last two where the gradient's rows allow)."""
+    if ranges is not None:
+        monkeypatch.setenv("NTG_DW_RANGES", ranges)
+    check(dtype, batch, cin, cout, size, kernel, stride, pad, groups, False)
