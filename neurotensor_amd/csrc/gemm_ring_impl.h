@@ -1480,7 +1480,7 @@ static hipError_t launch_conv_nhwc16_planned(const GemmParams& p, hipStream_t s,
     head.N = (int)head_cols;
     tail.N = p.N - (int)head_cols;
     tail.conv.n_base = p.conv.n_base + (int)head_cols;
-    tail.C = static_cast<char*>(p.C) + head_cols * 2;
+    tail.C = static_cast<char*>(p.C) + head_cols * (p.cmode == C_PARTIAL ? 4 : 2);      // (partial sums are Float32)
     if (p.bias) tail.bias = static_cast<const char*>(p.bias) + head_cols * p.bias_cs * 2;
     const hipError_t e = launch_ring16_planned(head, s, launch);
     if (e != hipSuccess) return e;

@@ -233,3 +233,13 @@ def test_weight_gradients_through_the_table_of_pixels(monkeypatch, dtype, ranges
     if ranges is not None:
         monkeypatch.setenv("NTG_DW_RANGES", ranges)
     check(dtype, batch, cin, cout, size, kernel, stride, pad, groups, False)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+def test_channels_in_ranges_with_the_columns_split(dtype):
+    """289 output pixels of 1536 rows of partial sums go out as 256 columns and a rest, whose sums start 256 Float32 elements in."""
+    x, w, _ = operands(dtype, 8, 256, 192, (17, 17), 7, 1, 3, 1, False)
+    got = F.conv2d(x.cuda(), w.cuda(), padding=3)[::7].double().cpu()
+    want, mags = (CONV[2](a.double(), b.double(), padding=3) for a, b in ((x[::7], w), (x[::7].abs(), w.abs())))
+    bound = UNIT[dtype] * want.abs() + 2.0 ** -24 * (256 * 49 + 32) * mags + (2.0 ** -25 if dtype == torch.float16 else 0.0)
+    assert bool(((got - want).abs() <= bound).all())
