@@ -290,6 +290,13 @@ __global__ void __launch_bounds__(256, ring_min_waves(DT, FLAT ? 1 : WB_, CONV))
     // (pointer tables: one uniform load per operand; everything below is base + offset either way)
     const T* A = p.Aptr ? static_cast<const T*>(p.Aptr[b]) : static_cast<const T*>(p.A) + operand_offset(p, b, p.sA, p.sAk);
     const T* B = p.Bptr ? static_cast<const T*>(p.Bptr[b]) : static_cast<const T*>(p.B) + operand_offset(p, b, p.sB, p.sBk);
+    if constexpr (GATHER16 && !ITEMS) {
+        if (p.conv.range_groups > 1) {                   // (uniform) channels in ranges, an item of a range is (image, group)
+            const int range = b / p.krange_items, of = b - range * p.krange_items, image = of / p.conv.range_groups, group = of - image * p.conv.range_groups;
+            A = static_cast<const T*>(p.A) + (int64_t)range * p.sAk + (int64_t)group * p.sA;
+            B = static_cast<const T*>(p.B) + (int64_t)range * p.sBk + (int64_t)image * p.conv.range_image + (int64_t)group * p.sB;
+        }
+    }
     T* C = p.Cptr ? static_cast<T*>(p.Cptr[b]) : static_cast<T*>(p.C) + (int64_t)b * p.sC;
     const int item = GATHERW && p.krange_items ? b / p.krange_items : b;      // (weight gradient: the k range or image; its groups follow each other)
 

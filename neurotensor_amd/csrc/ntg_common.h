@@ -78,6 +78,9 @@ struct ConvGeom {
     // channels-last convolution, several products in one launch: their table in device memory (see RingItem)
     const struct RingItem* items;
     int n_items;
+    // channels-last convolution in ranges of channels: groups (0, 1: none) and the elements from one image to the next; sA and sB step the groups
+    int range_groups;
+    int64_t range_image;
     int k_segment;           // Float32 weight gradients and `items`: K-steps of one chain of multiply-adds (a power of two; 0: all of them)
     int tile_rows, tile_cols;      // channels-last weight gradient: the tile the caller planned with
     // channels-last convolution on a bordered copy, k in 16-byte slots (taps outermost): slots of a tap; 0: whole 64-byte runs

@@ -1432,8 +1432,10 @@ static HaloPlan conv_halo(const Geo3& g) {
     }
     const int64_t vol = ext[0] * ext[1] * ext[2];
     // (a border larger than the image: not worth the copy on two axes, where the validity bits serve; three axes have no such form,
-    //  and the element-wise gather they fall back to loses more than the copy of three times the image costs)
-    if (vol > (g.nd == 3 ? 4 : 2) * g.vol() + 64) return h;
+    //  and the element-wise gather they fall back to loses more than the copy of three times the image costs; small maps under wide windows,
+    //  where the copy is next to nothing, need it for their channels to go out in ranges: a step of Float16 4 x 1 x 8 x 8 -> 256 by 7 x 7 130 -> 36 us, BFloat16
+    //  2 x 256 x 8 x 8 -> 192 by 7 x 7 in 2 groups 113 -> 59)
+    if (vol > (g.nd == 3 || vol <= 1024 ? 4 : 2) * g.vol() + 64) return h;
     h.hm.W = g.sz[2]; h.hm.H = g.sz[1]; h.hm.D = g.sz[0];
     h.hm.Wp = ext[2]; h.hm.Hp = ext[1]; h.hm.Dp = ext[0];
     h.hm.left = g.p[2]; h.hm.top = g.p[1]; h.hm.front = g.p[0];
@@ -1488,11 +1490,11 @@ static bool conv_nhwc_ok(int dtype, int64_t batch, int64_t channels, int64_t out
 // each, added up in order by a second pass.  A workgroup alone on its CU takes 0.32 us a K-step in Float32 and 0.2 in 16 bits whatever the others do (2 x 256 x
 // 13 x 13 -> 256 by 3 x 3: 24 tiles of 144 and 72 K-steps); shared by w workgroups a CU takes 0.25 w and 0.07 w.  The second pass costs 4.5 us and the traffic of
 // the sums.  Measured: that layer 47 -> 11 + 3 us and 18 -> 8 + 3; 192 x 17 x 17 -> 32 by 7 x 7, 3 tiles of 588, 169 -> 33 + 4 us.  The number of ranges does not depend on the number of images, only whether
-// there are any: up to 128 tiles an image's result is the same bits alone and among others.  Under 64 K-steps there is too little to win; groups would need a
-// third stride.
+// there are any: up to 128 tiles an image's result is the same bits alone and among others.  Under 64 K-steps there is too little to win.  Layers in groups
+// alike (Float32 256 x 11^3 -> 128 by 3 x 3 x 3 at stride 2 in 4 groups, a step, 85 -> 62 us, 4 x 96 x 8 x 8 -> 16 by 5 x 5 at stride 2 in 2 56 -> 44).
 static int64_t conv_k_ranges(int64_t es, int64_t batch, int64_t rows, int64_t pixels, int64_t groups, const NhwcForm& form, int64_t taps) {
-    const int64_t bk = 64 / es, runs = form.cgp / bk, steps = runs * taps, tiles = ((rows + 63) / 64) * ((pixels + 63) / 64) * batch;
-    if (groups != 1 || form.slot_v || tiles > 128 || steps < 64) return 1;
+    const int64_t bk = 64 / es, runs = form.cgp / bk, steps = runs * taps, tiles = ((rows / groups + 63) / 64) * ((pixels + 63) / 64) * batch * groups;
+    if (form.slot_v || tiles > 128 || steps < 64) return 1;
     int64_t r = 8;
     while (r > 1 && (runs % r != 0 || steps / r < 16)) --r;
     const double shared = (double)((tiles * r + 255) / 256), step_us = es == 4 ? 0.32 : 0.2, shared_us = std::max(step_us, (es == 4 ? 0.25 : 0.07) * shared);
@@ -1500,23 +1502,25 @@ static int64_t conv_k_ranges(int64_t es, int64_t batch, int64_t rows, int64_t pi
     return (double)(steps / r) * shared_us + sums_us < 0.8 * (double)steps * step_us ? r : 1;
 }
 static int64_t conv_k_ranges_bytes(int64_t ranges, int64_t batch, int64_t rows, int64_t pixels) { return ranges > 1 ? ranges * batch * rows * ((pixels + 7) / 8 * 8) * 4 : 0; }
-// the product p (weights by image, `rows` x `pixels` an image) in ranges: partial sums at `part`, results at p.C in p.cmode
-static hipError_t launch_conv_k_ranges(ntg::GemmParams p, int dtype, int64_t batch, int64_t ranges, int64_t taps, int64_t b_image, int64_t c_image, char* part, hipStream_t hs) {
+// the product p (weights by image, p.M rows a group; strides as in launch_groups) in ranges: partial sums at `part`, results at p.C in p.cmode
+static hipError_t launch_conv_k_ranges(ntg::GemmParams p, int dtype, int64_t batch, int64_t groups, int64_t ranges, int64_t taps, const GroupStrides& st, char* part, hipStream_t hs) {
     const int64_t ldp = (p.N + 7) / 8 * 8, K = p.K;
     ntg::GemmParams q = p;
-    // launch index = range * images + image
+    // launch index = (range * images + image) * groups + group
     q.K = (int)(K / ranges);
     q.C = part;
     q.ldc = ldp; q.sC = p.M * ldp;
     q.cmode = ntg::C_PARTIAL;
-    q.batch = (int)(batch * ranges);
-    q.krange_items = (int)batch;
-    q.sA = 0; q.sAk = q.K;
-    q.sB = b_image; q.sBk = q.K / taps;
+    q.batch = (int)(batch * groups * ranges);
+    q.krange_items = (int)(batch * groups);
+    q.sA = groups > 1 ? st.a_group : 0; q.sAk = q.K;
+    q.sB = groups > 1 ? st.b_group : st.b_image; q.sBk = q.K / taps;
+    q.conv.range_groups = (int)groups;
+    q.conv.range_image = st.b_image;
     hipError_t e = ntg::launch_conv_nhwc(dtype, q, hs);
     if (e != hipSuccess) return e;
-    p.batch = (int)batch;
-    p.sC = c_image;
+    p.batch = (int)(batch * groups);
+    p.sC = st.c_item;
     return ntg::launch_splitk_reduce(dtype, part, (int)ranges, p, ldp, hs);
 }
 static int64_t conv_nhwc_workspace(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
@@ -1568,8 +1572,9 @@ static int conv_forward_nhwc(int dtype, const void* image, const void* kernel, v
     p.conv.tap_inner = tap_inner ? 1 : 0;
     if (mt) { p.conv.tap_step = (int)mt->T; p.conv.kq_pad = (int)mt->kq_pad; }
     else set_slots(p.conv, form);
-    if (ranges > 1) e = launch_conv_k_ranges(p, dtype, batch, ranges, taps, chp * volp, og * L, ws_w + align_up((size_t)(og * K * es), 256), hs);
-    else e = launch_groups(p, dtype, batch, groups, {og * K, 0, cgp, chp * volp, og * L}, [&](const ntg::GemmParams& q) { return ntg::launch_conv_nhwc(dtype, q, hs); });
+    const GroupStrides st = {og * K, 0, cgp, chp * volp, og * L};
+    if (ranges > 1) e = launch_conv_k_ranges(p, dtype, batch, groups, ranges, taps, st, ws_w + align_up((size_t)(out_channels * K * es), 256), hs);
+    else e = launch_groups(p, dtype, batch, groups, st, [&](const ntg::GemmParams& q) { return ntg::launch_conv_nhwc(dtype, q, hs); });
     if (e != hipSuccess) return hip_fail(e, "channels-last convolution launch");
     return NTG_OK;
 }
@@ -1661,8 +1666,9 @@ static int conv_dimage_nhwc(int dtype, const void* kernel, const void* grad_out,
     p.conv.tap_inner = tap_inner ? 1 : 0;
     set_slots(p.conv, form);
     const int64_t ranges = halo.on ? conv_k_ranges(es, batch, channels, vol, groups, form, taps) : 1;
-    const hipError_t e = ranges > 1 ? launch_conv_k_ranges(p, dtype, batch, ranges, taps, ochp * Lp, cg * vol, ws_w + align_up((size_t)(cg * K * es), 256), hs)
-                                    : launch_groups(p, dtype, batch, groups, {cg * K, 0, ogp, ochp * Lp, cg * vol}, [&](const ntg::GemmParams& q) { return ntg::launch_conv_nhwc(dtype, q, hs); });
+    const GroupStrides st = {cg * K, 0, ogp, ochp * Lp, cg * vol};
+    const hipError_t e = ranges > 1 ? launch_conv_k_ranges(p, dtype, batch, groups, ranges, taps, st, ws_w + align_up((size_t)(channels * K * es), 256), hs)
+                                    : launch_groups(p, dtype, batch, groups, st, [&](const ntg::GemmParams& q) { return ntg::launch_conv_nhwc(dtype, q, hs); });
     if (e != hipSuccess) return hip_fail(e, "channels-last conv_dimage launch");
     return NTG_OK;
 }

@@ -218,6 +218,19 @@ def test_channels_in_ranges(dtype, batch, cin, cout, size, kernel, stride, pad):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("batch,cin,cout,size,kernel,stride,pad,groups", [
+    (2, 256, 130, (13, 5), 5, 1, 2, 2),              # 65 rows a group
+    (3, 192, 9, (9, 10), 5, 2, 2, 3),                # three rows a group
+    (1, 256, 128, (5, 6, 7), 3, 2, 1, 4),
+    (2, 512, 32, (11,), 7, 1, 3, 2),                 # (an axis of more than eight taps has no such form: its image gradient goes through a col matrix)
+    (4, 1, 256, (8, 8), 7, 1, 3, 1),                 # a border of twice the map
+    (2, 128, 96, (8, 8), 7, 1, 3, 2),
+], ids=str)
+def test_channels_of_groups_in_ranges(dtype, batch, cin, cout, size, kernel, stride, pad, groups):
+    check(dtype, batch, cin, cout, size, kernel, stride, pad, groups, False, ("dx",) if stride > 1 else ())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
 @pytest.mark.parametrize("ranges", [None, "0", "1"])
 @pytest.mark.parametrize("batch,cin,cout,size,kernel,stride,pad,groups", [
     (3, 16, 16, (1600,), 3, 1, 1, 1),            # chunks of 512 pixels that images cross, one row of flat tiles
