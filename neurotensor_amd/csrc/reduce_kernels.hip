@@ -327,17 +327,27 @@ hipError_t launch_flip_weights(int64_t es, const void* w, void* wt, int64_t grou
 
 // im[b][c][z][y][x] (+)= the element of the phase plane that holds it: phase e = (position + p) % s per axis stores the image
 // positions s (a0 + a) + e - p as its positions a; phases without taps contribute zero.  A thread does V consecutive elements of
-// an image row (16 bytes in one store where the rows allow it): the divisions are made once per row piece and the column phase
+// an image row (16 bytes in one store at any element; the last piece of a row that is no whole pieces moves back over the one before, which stores the
+// same values, or adds to C element by element; rows shorter than a piece go four elements at a time): the divisions are made once per row piece and the column phase
 // advances by counting (Float16 32 x 64 x 56 x 56: one element per thread with all its divisions 19.8 us, this 12.9).  At a column
 // stride of two, the one in common use, a piece is half a chunk of one phase's row and half a chunk of the other's: two loads at any element
-// where the counting makes one of two bytes for each of its elements, 8.5 us (25.7 MB: 5.5 at the rate of a large copy).
+// where the counting makes one of two bytes for each of its elements, 8.5 us (25.7 MB: 5.5 at the rate of a large copy).  Rows of 52, element by element
+// before: BFloat16 53 x 256 x 52 x 52 81 us, 33 now (73 MB each way: 31).
 template <class T, int V, bool STORE16>
 __global__ void __launch_bounds__(256) phase_interleave_kernel(const T* __restrict__ tmp, T* __restrict__ im, const PhaseLayout q, const uint32_t total,
                                                                const FastDiv div_pieces, const int accumulate) {
     const uint32_t idx = blockIdx.x * 256u + threadIdx.x;
     if (idx >= total) return;
     const uint32_t pieces = (uint32_t)(q.sz[2] + V - 1) / V;
-    const uint32_t row = fast_div(idx, div_pieces), x0 = (idx - row * pieces) * V;
+    const uint32_t row = fast_div(idx, div_pieces);
+    uint32_t x0 = (idx - row * pieces) * V;
+    bool whole = STORE16;
+    if constexpr (STORE16) {
+        if (x0 + V > (uint32_t)q.sz[2]) {
+            whole = !accumulate;
+            if (whole) x0 = (uint32_t)q.sz[2] - V;
+        }
+    }
     const uint32_t t1 = fast_div(row, q.div_rows[1]), y = row - t1 * (uint32_t)q.sz[1];
     const uint32_t bc = fast_div(t1, q.div_rows[0]), z = t1 - bc * (uint32_t)q.sz[0];
     const uint32_t Z = z + (uint32_t)q.p[0], Y = y + (uint32_t)q.p[1], X = x0 + (uint32_t)q.p[2];
@@ -355,8 +365,8 @@ __global__ void __launch_bounds__(256) phase_interleave_kernel(const T* __restri
                   ? q.plane_off[rphase + e] + (int64_t)bc * phase_plane(q, (int)ez, (int)ey, e) + ((int64_t)rz * q.n[1][ey] + ry) * q.n[2][e] - q.a0[2][e] : none;
     T* dst = im + (int64_t)row * q.sz[2] + x0;
     if constexpr (STORE16) {
-        if (q.s[2] == 2) {                                             // (uniform)
-            typedef T TV __attribute__((ext_vector_type(V)));
+        if (q.s[2] == 2 && whole) {
+            typedef T TV __attribute__((ext_vector_type(V), aligned(sizeof(T))));
             typedef T TH __attribute__((ext_vector_type(V / 2), aligned(sizeof(T))));
             const int64_t o0 = (ex ? rowoff[1] : rowoff[0]), o1 = (ex ? rowoff[0] : rowoff[1]);
             TH f0, f1;
@@ -386,8 +396,8 @@ __global__ void __launch_bounds__(256) phase_interleave_kernel(const T* __restri
         v[i] = (T)f;
         if (++ex == (uint32_t)q.s[2]) { ex = 0u; ++ax; }
     }
-    if constexpr (STORE16) {
-        typedef T TV __attribute__((ext_vector_type(V)));
+    if (whole) {
+        typedef T TV __attribute__((ext_vector_type(V), aligned(sizeof(T))));
         TV o;
 #pragma unroll
         for (int i = 0; i < V; ++i) o[i] = v[i];
@@ -403,8 +413,8 @@ template <class T>
 static hipError_t launch_phase_interleave_t(const void* tmp, void* im, const PhaseLayout& q, int accumulate, hipStream_t s) {
     constexpr int V16 = 16 / (int)sizeof(T), V = 4;
     const int64_t rows = (int64_t)q.batch * q.groups * q.cg * q.sz[0] * q.sz[1];
-    const bool vec = q.sz[2] % V16 == 0 && (reinterpret_cast<uintptr_t>(im) & 15) == 0;
-    const int64_t pieces = vec ? q.sz[2] / V16 : (q.sz[2] + V - 1) / V, total = rows * pieces;
+    const bool vec = q.sz[2] >= V16;
+    const int64_t pieces = (q.sz[2] + (vec ? V16 : V) - 1) / (vec ? V16 : V), total = rows * pieces;
     if (total == 0) return hipSuccess;
     if (total >= 0x7fffffffLL) return hipErrorInvalidValue;
     const dim3 g((unsigned)((total + 255) / 256)), t(256);

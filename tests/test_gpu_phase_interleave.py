@@ -102,3 +102,18 @@ def test_rows_from_two_column_phases_over_three_axes(geom, dtype):
     bound = UNIT[dtype] * exact.abs() + (k + 8) * 2.0 ** -24 * terms + (2.0 ** -24 if dtype == torch.float16 else 0)
     assert ((out[0, 0].double() - exact).abs() <= bound).all()
     assert torch.equal(out[1, 0], (out[0, 0].float() + c0.float()).to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("geom", [
+    # rows shorter than a piece, a piece and one element, one less than two: the last piece moves back over the one before, or adds element by element
+    (2, 16, 4, 3, 16, 3, 3, 2, 1, 1),
+    (2, 16, 5, 7, 16, 3, 3, 2, 1, 1),
+    (1, 32, 5, 9, 32, 4, 4, 2, 1, 1),
+    (2, 16, 6, 15, 32, 2, 2, 2, 0, 0),
+    (3, 32, 3, 17, 16, 3, 1, 1, 1, 0),
+    (1, 16, 9, 52, 48, 5, 7, 3, 2, 3),
+    (2, 16, 7, 41, 16, 1, 3, 2, 0, 2),
+], ids=lambda g: "x".join(map(str, g)))
+def test_rows_that_are_no_whole_pieces(geom, dtype):
+    test_rows_from_two_column_phases(geom, dtype)
