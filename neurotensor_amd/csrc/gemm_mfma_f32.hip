@@ -236,11 +236,24 @@ static hipError_t launch_small16_f32(bool ta, bool tb, const GemmParams& pin, hi
     return hipGetLastError();
 }
 
+// Up to 64 k on many tiles (col matrices of strided image gradients): a tile is four K-steps and as long again to fill the ring and to store; tiles of 64
+// rows x 128 columns have half as many of those.  The same chains.  us on 64 x 64 | 64 x 128 tiles: 32 x (160 x 64 x 12544) A^T.B 142 | 132, 8 x (64 x 64 x
+// 50000) 47.3 | 45.8, 64 x (192 x 32 x 3200) 44.9 | 42.7.  Under 3072 wide tiles, four rounds of three on each CU, a last round that is nearly empty costs
+// more (64 x (448 x 64 x 640), 2240 of them, 30.7 | 32.3), and so do columns that they waste (60 x (320 x 48 x 1088), 9 tiles for 8.5, 30.6 | 32.9); a deeper k
+// gains nothing (64 x (192 x 128 x 3136) 98.5 | 99.5).  64 x 256 tiles: 137 and 51.6 on the first two.
+static bool ring_f32_wide(const GemmParams& p) {
+    const int64_t cols = ((int64_t)p.N + 127) / 128;
+    return p.K <= 64 && 128 * cols * 100 <= 101 * (int64_t)p.N && (int64_t)((p.M + 63) / 64) * cols * p.batch >= 3072;
+}
+static hipError_t launch_ring_f32(bool ta, bool tb, const GemmParams& p, hipStream_t s) {
+    if (ring_f32_tile_edge(p) == 128) return launch_ring_wb<DT_F32, 2>(ta, tb, p, s);
+    return ring_f32_wide(p) ? launch_ring_wb<DT_F32, 1, 2>(ta, tb, p, s) : launch_ring_wb<DT_F32, 1>(ta, tb, p, s);
+}
+
 hipError_t launch_gemm_mfma_f32(bool ta, bool tb, const GemmParams& p, hipStream_t s) {
     if ((p.tailA || p.tailB) && !ring_eligible(p, ta, 4)) return hipErrorInvalidValue;       // (only the DMA-fed kernel reads copied tail rows)
     if (ring_eligible(p, ta, 4) && small16_f32_wins(p)) return launch_small16_f32(ta, tb, p, s);
-    if (ring_eligible(p, ta, 4))
-        return ring_f32_tile_edge(p) == 64 ? launch_ring_wb<DT_F32, 1>(ta, tb, p, s) : launch_ring_wb<DT_F32, 2>(ta, tb, p, s);
+    if (ring_eligible(p, ta, 4)) return launch_ring_f32(ta, tb, p, s);
     if (any_eligible(p, DT_F32, ta, tb)) return launch_gemm_any(DT_F32, ta, tb, p, s);
     // rows shorter than a 16-byte chunk, pitches from 8 MiB on: register-staged kernel, 64 x 64 x 32 (128 x 128: 2048 x 3 x 2048 11.9 us against 9.6, 2048 x 2048 x
     // 2048 at such a pitch 167 / 161)
@@ -250,7 +263,7 @@ hipError_t launch_gemm_ring_only_f32(bool ta, bool tb, const GemmParams& p, hipS
     *taken = ring_eligible(p, ta, 4);
     if (!*taken) return hipSuccess;
     if (small16_f32_wins(p)) return launch_small16_f32(ta, tb, p, s);
-    return ring_f32_tile_edge(p) == 64 ? launch_ring_wb<DT_F32, 1>(ta, tb, p, s) : launch_ring_wb<DT_F32, 2>(ta, tb, p, s);
+    return launch_ring_f32(ta, tb, p, s);
 }
 // convolution / conv_dkernel with op(B) gathered from the image (tb: col^T), nd = 2 or 3 spatial axes
 template <int ND>

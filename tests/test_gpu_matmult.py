@@ -1341,3 +1341,20 @@ def test_pointer_tables_without_a_vouch_find_their_alignment_on_the_device(dtype
         torch.cuda.synchronize()
         for i in range(nb):
             assert torch.equal(bits(c[i]), bits(alone[i])), (dtype, "shift", shift, "item", i)
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("batch,m,k,n", [(33, 68, 60, 8004), (20, 160, 64, 12544), (3080, 64, 4, 128), (70, 132, 32, 1920)])
+def test_fp32_short_k_on_many_tiles(batch, m, k, n, ta, tb):
+    """Up to 64 k on 3072 tiles of 64 x 128 or more: the chain of an item that is alone (and then on other tiles), overwriting and from C on; and within
+    k + 1 roundings of the product in 64 bits."""
+    gen = torch.Generator(device=DEV).manual_seed(m + n)
+    a = torch.randn((batch, k, m) if ta else (batch, m, k), device=DEV, generator=gen)
+    b = torch.randn((batch, n, k) if tb else (batch, k, n), device=DEV, generator=gen)
+    c = torch.randn((batch, m, n), device=DEV, generator=gen)
+    got, acc = F.matmult(a, b, None, ta, tb), F.matmult(a, b, c.clone(), ta, tb)
+    for i in (0, batch // 2, batch - 1):
+        assert torch.equal(F.matmult(a[i], b[i], None, ta, tb), got[i])
+        assert torch.equal(F.matmult(a[i], b[i], c[i].clone(), ta, tb), acc[i])
+        x, w = (t.double().cpu() for t in ((a[i].t() if ta else a[i]), (b[i].t() if tb else b[i])))
+        assert bool(((got[i].double().cpu() - x @ w).abs() <= (k + 1) * 2.0 ** -24 * (x.abs() @ w.abs())).all())
