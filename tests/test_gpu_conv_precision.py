@@ -311,6 +311,43 @@ def test_fp32_gradients_are_as_close_as_sums_per_tap_and_per_image(geom):
         assert ours <= 1.15 * reference, (name, ours, reference)
 
 
+@pytest.mark.parametrize("geom", [
+    # (B, C, size, O, kernel, stride, groups): out channels of a group that are no multiple of 16
+    (8, 32, (56, 56), 24, (3, 3), 2, 1),
+    (8, 32, (56, 56), 24, (7, 7), 2, 1),
+    (8, 64, (56, 56), 48, (5, 5), 2, 2),
+    (8, 48, (28, 28), 72, (4, 4), 2, 1),                   # 72: two K-steps and a half
+    (8, 32, (56, 56), 8, (3, 3), 2, 1),                    # fewer than a K-step's 16
+    (8, 64, (40, 40), 16, (4, 4), 2, 4),
+    (8, 32, (33, 35), 24, (3, 3), 2, 2),
+    (4, 24, (4000,), 24, (7,), 2, 1),
+    (2, 16, (24, 24, 24), 8, (3, 3, 3), 2, 1),
+    (2, 16, (24, 24, 24), 16, (3, 3, 3), 2, 4),
+], ids=str)
+def test_fp32_strided_image_gradients_of_any_channels_are_as_close_as_sums_per_tap(geom):
+    """Image gradients at strides, and the transposed convolution that is the same sum: the col matrix adds up one product per tap, and the
+    host entry point forms it.  The phases' chains are no longer than that, so the two norms' ratio is 1 within some percent; one chain through all
+    taps was 1.4 (3 x 3) to 2.7 (7 x 7)."""
+    B, C, size, O, k, s, groups = geom
+    nd, p = len(size), tuple(v // 2 for v in k)
+    out = tuple((size[a] + 2 * p[a] - k[a]) // s + 1 for a in range(nd))
+    x, w, g = randn((B, C) + size, torch.float32, 1), randn((O, C // groups) + k, torch.float32, 2, 0.05), randn((B, O) + out, torch.float32, 3)
+    dx, _ = backward(nd)(x, w, g, stride=s, padding=p[0], groups=groups)
+    rest = {size[a] - ((out[a] - 1) * s - 2 * p[a] + k[a]) for a in range(nd)}
+    hx, hw, hg = (t.cpu().numpy() for t in (x, w, g))
+    hdx, hdw = np.empty_like(hx), np.empty_like(hw)
+    vp = lambda a: a.ctypes.data_as(ctypes.c_void_p)
+    geo = tuple(_arr(v) for v in (size, k, (s,) * nd, p, (1,) * nd))
+    _lib.check(_lib.load().ntg_convnd_backward(_lib.FLOAT32, vp(hx), vp(hw), vp(hg), vp(hdx), vp(hdw), B, C, O, nd, *geo, groups, 0))
+    want = exact_dx(size, w, g, k, (s,) * nd, p, (1,) * nd, groups)
+    reference = relative(torch.from_numpy(hdx).to(DEV), want)
+    assert relative(dx, want) <= 1.15 * reference, (relative(dx, want), reference)
+    if len(rest) == 1:
+        transposed = {1: F.conv_transpose1d, 2: F.conv_transpose2d, 3: F.conv_transpose3d}[nd]
+        y = transposed(g, w, stride=s, padding=p[0], output_padding=rest.pop(), groups=groups)
+        assert relative(y, want) <= 1.15 * reference, (relative(y, want), reference)
+
+
 def test_fp32_weight_gradient_takes_the_large_tiles_where_they_are_faster(monkeypatch):
     """128 x 128 tiles take 77 % of the time of four 64 x 64 ones (profiles/conv_weight_gradient_gather_sweep.txt): the planned gradient of this
     layer is faster than fourteen ranges on 64 x 64 tiles (the knob's tile), which a plan that charged both alike chose; by 15 % without
