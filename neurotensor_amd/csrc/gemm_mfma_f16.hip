@@ -5,6 +5,7 @@ hipError_t launch_gemm_mfma_f16(bool ta, bool tb, const GemmParams& p, hipStream
     if ((p.tailA || p.tailB) && !ring_eligible(p, ta)) return hipErrorInvalidValue;       // (only the DMA-fed kernel reads copied tail rows)
     if (ring_eligible(p, ta)) return launch_ring16<DT_F16>(ta, tb, p, s);   // DMA-fed LDS ring; the tile (256 x 256 .. 64 x 64, 192 x 256, 128 x 256) follows ring16_tile_edge
     if (any_eligible(p, DT_F16, ta, tb)) return launch_gemm_any(DT_F16, ta, tb, p, s);
+    if (p.cmode == C_PARTIAL) return hipErrorInvalidValue;      // (this kernel would round the sums to 16 bits)
     // rows shorter than a 16-byte chunk, pitches from 8 MiB on: 128 x 128 x 64 (256 x 256: 8192 x 4 x 8192 127 us against 78, 4096 x 2048 x 4096 at such a pitch 98 / 100)
     return launch_trans<DT_F16, 2, 2, 64>(ta, tb, p, s);
 }

@@ -2070,6 +2070,7 @@ static PointwiseDwPlan plan_pointwise_dw(int dtype, int64_t batch, int64_t chann
     if (!conv_pointwise_ok(dtype, channels, groups, g) || (og * es) % 16 != 0 || batch <= 0 || og <= 0) return pl;
     const int64_t tiles = ((og + 63) / 64) * ((cg + 63) / 64) * batch * groups;
     if (tiles >= 0x7fffffffLL || L >= 0x7fffffffLL) return pl;
+    if (es == 2 && L >= (1 << 23) / es) return pl;       // (the rows are the operands' pitch, and no kernel for pitches from 8 MiB on writes Float32 sums of 16-bit operands)
     const uint32_t steps = L % bk == 0 ? (uint32_t)(L / bk) : 1u;
     double best = 0.0;
     for (uint32_t s = 1; s <= steps && (s == 1 || tiles * s <= 2048); ++s) {      // (eight tiles a CU: more only makes more partial sums)

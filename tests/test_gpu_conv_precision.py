@@ -311,6 +311,19 @@ def test_fp32_gradients_are_as_close_as_sums_per_tap_and_per_image(geom):
         assert ours <= 1.15 * reference, (name, ours, reference)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("width", [2040, 2048])
+@pytest.mark.parametrize("groups", [1, 2])
+def test_16_bit_weight_gradients_of_one_tap_on_rows_of_8_mib(width, dtype, groups):
+    """Rows of 2^23 bytes are the first that the kernels that can write Float32 sums do not take as a pitch.  One rounding to 16 bits, on both sides of it (one
+    image); the sums of 2^22 products in 32 bits add at most 2^-24 sqrt(2^22) = 1.2e-4 of the result, 1 / 2 of Float16's rounding in the norm of both."""
+    x, g = randn((1, 16, 2048, width), dtype, 1), randn((1, 16, 2048, width), dtype, 3)
+    w = randn((16, 16 // groups, 1, 1), dtype, 2)
+    _, dw = F.conv2d_backward(x, w, g, groups=groups)
+    want = exact_dw(x, g, (1, 1), (1, 1), (0, 0), (1, 1), groups)
+    assert relative(dw, want) <= 1.25 * relative(want.to(dtype), want), (relative(dw, want), relative(want.to(dtype), want))
+
+
 @pytest.mark.parametrize("geom", [
     # (B, C, size, O, kernel, stride, groups): out channels of a group that are no multiple of 16
     (8, 32, (56, 56), 24, (3, 3), 2, 1),
