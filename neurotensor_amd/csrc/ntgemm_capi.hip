@@ -1317,9 +1317,10 @@ static void fill_conv_geom(ntg::ConvGeom& c, int64_t slice_channels, const Geo3&
     c.div_howo = ntg::make_fastdiv((uint32_t)c.HoWo);
 }
 
-// A plain product per (image, group), strides in elements; the floating types in one launch.
+// A plain product per (image, group), strides in elements; the floating types in one launch.  reference_order: NTG_GEMM_KEEP_K_ORDER (a convolution of one tap
+// through the host entry points is unfold + matmult bit for bit).
 static int gemm_per_group(int dtype, bool ta, bool tb, int cmode, int64_t m, int64_t k, int64_t n, int64_t lda, int64_t ldb, int64_t ldc, int64_t batch, int64_t groups,
-                          const void* A, int64_t a_group, int64_t a_image, const void* B, int64_t b_group, int64_t b_image, void* C, void* stream) {
+                          const void* A, int64_t a_group, int64_t a_image, const void* B, int64_t b_group, int64_t b_image, void* C, void* stream, bool reference_order) {
     const int64_t es = ntg::elem_size(dtype), c_item = m * ldc;
     if (groups > 1 && !is_valu_dtype(dtype) && m > 0 && n > 0 && k > 0 && batch > 0) {
         const int rc = check_sizes(m, k, n, batch);
@@ -1330,6 +1331,7 @@ static int gemm_per_group(int dtype, bool ta, bool tb, int cmode, int64_t m, int
         p.A = A; p.B = B; p.C = C;
         p.lda = lda; p.ldb = ldb; p.ldc = ldc;
         p.cmode = cmode;
+        p.keep_k_order = reference_order;
         int status = NTG_OK;
         const hipError_t e = launch_groups(p, dtype, batch, groups, {a_group, a_image, b_group, b_image, c_item}, [&](const ntg::GemmParams& q) {
             status = launch_gemm(q, dtype, ta, tb, static_cast<hipStream_t>(stream));
@@ -1344,6 +1346,7 @@ static int gemm_per_group(int dtype, bool ta, bool tb, int cmode, int64_t m, int
         d.m = m; d.k = k; d.n = n;
         d.lda = lda; d.ldb = ldb; d.ldc = ldc; d.batches = batch;
         d.stride_a = a_image; d.stride_b = b_image; d.stride_c = groups * c_item;
+        d.flags = reference_order ? NTG_GEMM_KEEP_K_ORDER : 0;
         const int rc = ntg_gemm_dev(&d, static_cast<const char*>(A) + g * a_group * es, static_cast<const char*>(B) + g * b_group * es,
                                     static_cast<char*>(C) + g * c_item * es, stream);
         if (rc) return rc;
@@ -1387,9 +1390,10 @@ static bool conv_pointwise_ok(int dtype, int64_t channels, int64_t groups, const
     return (g.L() * es) % 16 == 0 && (channels / groups * es) % 16 == 0;
 }
 static int conv_forward_pointwise(int dtype, const void* image, const void* kernel, void* out, int64_t batch, int64_t channels,
-                                  int64_t out_channels, const Geo3& g, int64_t groups, void* stream) {
+                                  int64_t out_channels, const Geo3& g, int64_t groups, void* stream, bool reference_order) {
     const int64_t cg = channels / groups, og = out_channels / groups, L = g.L();
-    return gemm_per_group(dtype, false, false, NTG_C_OVERWRITE, og, cg, L, cg, L, L, batch, groups, kernel, og * cg, 0, image, cg * L, channels * L, out, stream);
+    return gemm_per_group(dtype, false, false, NTG_C_OVERWRITE, og, cg, L, cg, L, L, batch, groups, kernel, og * cg, 0, image, cg * L, channels * L, out, stream,
+                          reference_order);
 }
 
 // Channels-last form of the same convolution, for the floating dtypes up to 32 bits: the image is first copied to
@@ -2242,12 +2246,12 @@ int64_t ntg_conv2d_workspace_bytes(int dtype, int64_t batch, int64_t channels, i
     return batch * channels * k_r * k_c * Ho * Wo * es;
 }
 
-int ntg_conv2d_dev(int dtype, const void* image, const void* kernel, void* out,
+static int conv2d_dev_impl(int dtype, const void* image, const void* kernel, void* out,
                    void* workspace, int64_t workspace_bytes,
                    int64_t batch, int64_t channels, int64_t height, int64_t width,
                    int64_t out_channels, int64_t k_r, int64_t k_c,
                    int64_t s_r, int64_t s_c, int64_t p_r, int64_t p_c, int64_t d_r, int64_t d_c,
-                   int64_t groups, void* stream) {
+                   int64_t groups, void* stream, bool reference_order) {
     const int64_t es = ntg::elem_size(dtype);
     if (es == 0) return fail(NTG_ERR_UNSUPPORTED_DTYPE, "dtype %d is not supported", dtype);
     if (batch < 0 || channels < 0 || out_channels < 0 || height < 0 || width < 0) return fail(NTG_ERR_INVALID_ARGUMENT, "negative size");
@@ -2266,7 +2270,7 @@ int ntg_conv2d_dev(int dtype, const void* image, const void* kernel, void* out,
         const Geo3 g = geo2(height, width, k_r, k_c, s_r, s_c, p_r, p_c, d_r, d_c, Ho, Wo);
         if (conv_pointwise_ok(dtype, channels, groups, g) &&
             (is_valu_dtype(dtype) || ((reinterpret_cast<uintptr_t>(image) | reinterpret_cast<uintptr_t>(kernel) | reinterpret_cast<uintptr_t>(out)) & 15) == 0))
-            return conv_forward_pointwise(dtype, image, kernel, out, batch, channels, out_channels, g, groups, stream);
+            return conv_forward_pointwise(dtype, image, kernel, out, batch, channels, out_channels, g, groups, stream, reference_order);
         // with the workspace of ntg_conv2d_fast_workspace_bytes: channels-last copy of the image, 16-byte gathers
         MergedTaps mt;
         if (conv_nhwc_merged(dtype, batch, channels, out_channels, groups, g, mt) && workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
@@ -2297,6 +2301,16 @@ int ntg_conv2d_dev(int dtype, const void* image, const void* kernel, void* out,
         if (rc) return rc;
     }
     return NTG_OK;
+}
+
+int ntg_conv2d_dev(int dtype, const void* image, const void* kernel, void* out,
+                   void* workspace, int64_t workspace_bytes,
+                   int64_t batch, int64_t channels, int64_t height, int64_t width,
+                   int64_t out_channels, int64_t k_r, int64_t k_c,
+                   int64_t s_r, int64_t s_c, int64_t p_r, int64_t p_c, int64_t d_r, int64_t d_c,
+                   int64_t groups, void* stream) {
+    return conv2d_dev_impl(dtype, image, kernel, out, workspace, workspace_bytes, batch, channels, height, width, out_channels, k_r, k_c, s_r, s_c, p_r, p_c, d_r, d_c,
+                           groups, stream, false);
 }
 
 int ntg_conv2d(int dtype, const void* image, const void* kernel, void* out,
@@ -2330,8 +2344,8 @@ int ntg_conv2d(int dtype, const void* image, const void* kernel, void* out,
     HIP_TRY(mem.reserve(ow + (size_t)ws));
     if (im_bytes) HIP_TRY(mem.upload(0, image, im_bytes));
     if (k_bytes) HIP_TRY(mem.upload(ok_, kernel, k_bytes));
-    rc = ntg_conv2d_dev(dtype, mem.at(0), mem.at(ok_), mem.at(oo), mem.at(ow), ws, batch, channels, height, width,
-                        out_channels, k_r, k_c, s_r, s_c, p_r, p_c, d_r, d_c, groups, mem.stream());
+    rc = conv2d_dev_impl(dtype, mem.at(0), mem.at(ok_), mem.at(oo), mem.at(ow), ws, batch, channels, height, width,
+                         out_channels, k_r, k_c, s_r, s_c, p_r, p_c, d_r, d_c, groups, mem.stream(), dtype == ntg::DT_F32);
     if (rc) return rc;
     HIP_TRY(mem.download(out, oo, o_bytes));
     return NTG_OK;
@@ -2439,14 +2453,14 @@ static int conv2d_backward_dev_impl(int dtype, const void* image, const void* ke
         const int64_t cg = channels / groups;
         if (d_image) {
             rc = gemm_per_group(dtype, true, false, accumulate ? NTG_C_ACCUMULATE : NTG_C_OVERWRITE, cg, og, L, cg, L, L, batch, groups, kern, og * cg, 0,
-                                gy, og * L, out_channels * L, d_image, stream);
+                                gy, og * L, out_channels * L, d_image, stream, reference_order);
             if (rc) return rc;
         }
         if (d_kernel && plan.pointwise.splits > 0 && workspace_bytes >= plan.pointwise.bytes)
             return conv_dkernel_pointwise(dtype, plan.pointwise, image, grad_out, d_kernel, ws, batch, channels, out_channels, geo, groups, accumulate, hs);
         if (d_kernel) {
             rc = gemm_per_group(dtype, false, true, NTG_C_OVERWRITE, og, L, cg, L, L, cg, batch, groups, gy, og * L, out_channels * L,
-                                image, cg * L, channels * L, ws, stream);
+                                image, cg * L, channels * L, ws, stream, reference_order);
             if (rc) return rc;
         }
         if (d_kernel) {
@@ -2476,7 +2490,7 @@ static int conv2d_backward_dev_impl(int dtype, const void* image, const void* ke
             if (e != hipSuccess) return hip_fail(e, "transposed weights launch");
         }
         rc = gemm_per_group(dtype, !wt, false, NTG_C_OVERWRITE, add, og, L, wt ? og : add, L, L, batch, groups, wt ? ws + plan.wt_offset : kern, og * add, 0,
-                            gy, og * L, out_channels * L, ws, stream);
+                            gy, og * L, out_channels * L, ws, stream, reference_order);
         if (rc) return rc;
         rc = ntg_unfold2d_backward_dev(dtype, ws, d_image, batch, channels, height, width, k_r, k_c, s_r, s_c, p_r, p_c, d_r, d_c,
                                        accumulate, stream);
@@ -2820,6 +2834,7 @@ static int convnd_backward_dev_impl(int dtype, const void* image, const void* ke
     if (batch == 0 || out_channels == 0 || channels == 0) return NTG_OK;
     if (!kernel || !grad_out || (d_kernel && !image)) return fail(NTG_ERR_INVALID_ARGUMENT, "null pointer");
     int64_t need = u.total * es + (d_kernel ? complex_dkernel_extra(dtype, batch, out_channels, (channels / groups) * u.taps, u.total * es) : 0);
+    bool reference_order = !channels_last && dtype == ntg::DT_F32;
     if (ndim == 3) {
         const Geo3 g = geo_from(u);
         const ConvBackwardPlan plan = plan_conv_backward_g(dtype, d_image != nullptr, d_kernel != nullptr, batch, channels, out_channels, g, groups);
@@ -2829,6 +2844,7 @@ static int convnd_backward_dev_impl(int dtype, const void* image, const void* ke
         // a workspace of ntg_convnd_workspace_bytes asks for the reference's order, even where a fast form would fit into it
         const bool fast = channels_last && workspace_bytes > ntg_convnd_workspace_bytes(dtype, batch, channels, out_channels, ndim, size, kernel_size, stride,
                                                                                         padding, dilation, groups, 1);
+        reference_order = !fast && dtype == ntg::DT_F32;
         rc = conv_gradients_implicit(dtype, plan, image, kernel, grad_out, d_image, d_kernel, static_cast<char*>(workspace), workspace_bytes, batch, channels,
                                      out_channels, g, groups, accumulate, static_cast<hipStream_t>(stream), fast);
         if (rc) return rc;
@@ -2848,7 +2864,8 @@ static int convnd_backward_dev_impl(int dtype, const void* image, const void* ke
         if (rc) return rc;
     }
     if (d_image) {
-        rc = gemm_per_group(dtype, true, false, NTG_C_OVERWRITE, add, og, L, add, L, L, batch, groups, kern, og * add, 0, gy, og * L, out_channels * L, ws, stream);
+        rc = gemm_per_group(dtype, true, false, NTG_C_OVERWRITE, add, og, L, add, L, L, batch, groups, kern, og * add, 0, gy, og * L, out_channels * L, ws, stream,
+                            reference_order);
         if (rc) return rc;
         hipError_t e = ntg::launch_col2imnd(dtype, ws, d_image, u, accumulate, static_cast<hipStream_t>(stream));
         if (e != hipSuccess) return hip_fail(e, "col2imnd launch");
@@ -2938,8 +2955,14 @@ int ntg_convnd(int dtype, const void* image, const void* kernel, void* out, int6
     HIP_TRY(mem.reserve(o_ws + (size_t)wsb));
     if (im_bytes) HIP_TRY(mem.upload(0, image, im_bytes));
     if (k_bytes) HIP_TRY(mem.upload(o_k, kernel, k_bytes));
-    rc = ntg_convnd_dev(dtype, mem.at(0), mem.at(o_k), mem.at(o_o), mem.at(o_ws), wsb, batch, channels, out_channels, ndim, size, kernel_size,
-                        stride, padding, dilation, groups, mem.stream());
+    if (ndim <= 2) {
+        const Geo2 g = as_2d(ndim, size, kernel_size, stride, padding, dilation);
+        rc = conv2d_dev_impl(dtype, mem.at(0), mem.at(o_k), mem.at(o_o), mem.at(o_ws), wsb, batch, channels, g.h, g.w, out_channels, g.kr, g.kc,
+                             g.sr, g.sc, g.pr, g.pc, g.dr, g.dc, groups, mem.stream(), dtype == ntg::DT_F32);
+    } else {
+        rc = ntg_convnd_dev(dtype, mem.at(0), mem.at(o_k), mem.at(o_o), mem.at(o_ws), wsb, batch, channels, out_channels, ndim, size, kernel_size,
+                            stride, padding, dilation, groups, mem.stream());
+    }
     if (rc) return rc;
     HIP_TRY(mem.download(out, o_o, o_bytes));
     return NTG_OK;

@@ -311,6 +311,30 @@ def test_fp32_gradients_are_as_close_as_sums_per_tap_and_per_image(geom):
         assert ours <= 1.15 * reference, (name, ours, reference)
 
 
+@pytest.mark.parametrize("geom", [
+    # (B, C, size, O, groups): 32 rows and fewer in the forward product, in the image gradient
+    (2, 128, (8, 12), 16, 1), (2, 256, (8, 12), 32, 2), (1, 64, (96,), 8, 1), (3, 16, (8, 12), 192, 1), (2, 32, (96,), 256, 2),
+], ids=str)
+def test_fp32_one_tap_through_the_host_entry_points_is_the_reference_product(geom):
+    """unfold + matmult bit for bit, also where the device entry points split k over the wavefronts of the kernels for few rows."""
+    B, C, size, O, groups = geom
+    nd, L, cg, og = len(size), int(np.prod(size)), C // groups, O // groups
+    x, w, g = (randn(shape, torch.float32, i).cpu().numpy() for i, shape in enumerate(((B, C) + size, (O, cg) + (1,) * nd, (B, O) + size)))
+    y, dx = np.empty_like(g), np.empty_like(x)
+    vp = lambda a: a.ctypes.data_as(ctypes.c_void_p)
+    geo = tuple(_arr(v) for v in (size, (1,) * nd, (1,) * nd, (0,) * nd, (1,) * nd))
+    lib = _lib.load()
+    _lib.check(lib.ntg_convnd(_lib.FLOAT32, vp(x), vp(w), vp(y), B, C, O, nd, *geo, groups))
+    _lib.check(lib.ntg_convnd_backward(_lib.FLOAT32, vp(x), vp(w), vp(g), vp(dx), None, B, C, O, nd, *geo, groups, 0))
+    for b in range(B):
+        for q in range(groups):
+            wq = np.ascontiguousarray(w.reshape(O, cg)[q * og:(q + 1) * og])
+            for got, a, rhs, m, k in ((y, wq, x, og, cg), (dx, np.ascontiguousarray(wq.T), g, cg, og)):
+                want, rhs = np.zeros((m, L), np.float32), np.ascontiguousarray(rhs.reshape(B, groups, k, L)[b, q])
+                _lib.check(lib.ntg_matmult(_lib.FLOAT32, vp(a), vp(rhs), vp(want), m, k, k, L, 0, 0))
+                assert np.array_equal(got.reshape(B, groups, m, L)[b, q], want), (b, q, m, k)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("width", [2040, 2048])
 @pytest.mark.parametrize("groups", [1, 2])
