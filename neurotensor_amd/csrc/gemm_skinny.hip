@@ -36,8 +36,8 @@ __global__ void __launch_bounds__(512) gemm_skinny_f32_kernel(const GemmParams p
     const int n0 = blockIdx.x * SW;
 
     // (global pointers: the waits of the register ring below are per k-step only if the loads are not FLAT instructions)
-    const NTG_GLOBAL float* A = (const NTG_GLOBAL float*)(p.Aptr ? static_cast<const float*>(p.Aptr[b]) : static_cast<const float*>(p.A) + (int64_t)b * p.sA);
-    const NTG_GLOBAL float* B = (const NTG_GLOBAL float*)(p.Bptr ? static_cast<const float*>(p.Bptr[b]) : static_cast<const float*>(p.B) + (int64_t)b * p.sB);
+    const NTG_GLOBAL float* A = (const NTG_GLOBAL float*)(p.Aptr ? static_cast<const float*>(p.Aptr[b]) : static_cast<const float*>(p.A) + operand_offset(p, b, p.sA, p.sAk));
+    const NTG_GLOBAL float* B = (const NTG_GLOBAL float*)(p.Bptr ? static_cast<const float*>(p.Bptr[b]) : static_cast<const float*>(p.B) + operand_offset(p, b, p.sB, p.sBk));
     NTG_GLOBAL float* C = (NTG_GLOBAL float*)(p.Cptr ? static_cast<float*>(p.Cptr[b]) : static_cast<float*>(p.C) + (int64_t)b * p.sC);
 
     floatx4 acc[MB][CPL];
@@ -457,7 +457,7 @@ static hipError_t launch_skinny16(bool ta, bool tb, const GemmParams& p, hipStre
 
 hipError_t launch_gemm_skinny(int dtype, bool ta, bool tb, const GemmParams& p, hipStream_t s, bool* handled) {
     *handled = false;
-    if (p.M > 32 || p.batch > 65535) return hipSuccess;
+    if (p.M > 32 || p.batch > NTG_SKINNY_MAX_ITEMS) return hipSuccess;
     if ((dtype == DT_F16 || dtype == DT_BF16) && p.K >= 128) {
         *handled = true;
         return dtype == DT_F16 ? launch_skinny16<DT_F16>(ta, tb, p, s) : launch_skinny16<DT_BF16>(ta, tb, p, s);

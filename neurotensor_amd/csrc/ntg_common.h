@@ -345,6 +345,7 @@ hipError_t launch_relu_inplace(int dtype, void* C, int64_t ldc, int64_t sC, int6
 hipError_t launch_gemm_valu(int dtype, bool ta, bool tb, const GemmParams& p, hipStream_t s);
 hipError_t launch_gemm_mfma_i8(int dtype, bool ta, bool tb, const GemmParams& p, hipStream_t s);   // Int8 / UInt8: MFMA where rows are 16-byte multiples
 hipError_t launch_gemm_complex(int dtype, bool ta, bool tb, const GemmParams& p, hipStream_t s);   // Complex32 / 64 / 128: lane-wise products on (re, im) pairs
+#define NTG_SKINNY_MAX_ITEMS 65535      // (a grid's second axis)
 hipError_t launch_gemm_skinny(int dtype, bool ta, bool tb, const GemmParams& p, hipStream_t s, bool* handled);
 // op(B) is the im2col matrix of the image at p.B (tb: its transpose); floating dtypes only
 hipError_t launch_conv_mfma(int dtype, bool tb, const GemmParams& p, hipStream_t s);

@@ -229,9 +229,11 @@ int launch_gemm(ntg::GemmParams p, int dtype, bool ta, bool tb, hipStream_t s) {
         e = ntg::launch_gemm_complex(dtype, ta, tb, p, s);
     } else {
         bool handled = false;
-        // (the streaming kernels for up to 32 rows split k over their wavefronts: not for a caller who wants the one chain)
+        // (the streaming kernels for up to 32 rows split k over their wavefronts: not for a caller who wants the one chain.  Items in groups or k ranges go there
+        //  in Float32, where the eight short chains are what a result errs by: 2 x 512 x 28 x 28 -> 32 by one tap in 2 groups 1.17e-7 against 2.87e-7; 16-bit
+        //  results err by their rounding, and the tiles' kernels are faster)
         e = hipSuccess;
-        if (!(p.keep_k_order && dtype == ntg::DT_F32) && p.krange_items == 0) {
+        if (dtype == ntg::DT_F32 ? !p.keep_k_order : p.krange_items == 0) {
             p.act = act;                                                   // (its epilogue clamps)
             e = ntg::launch_gemm_skinny(dtype, ta, tb, p, s, &handled);
             p.act = ntg::ACT_NONE;
@@ -1322,7 +1324,8 @@ static void fill_conv_geom(ntg::ConvGeom& c, int64_t slice_channels, const Geo3&
 static int gemm_per_group(int dtype, bool ta, bool tb, int cmode, int64_t m, int64_t k, int64_t n, int64_t lda, int64_t ldb, int64_t ldc, int64_t batch, int64_t groups,
                           const void* A, int64_t a_group, int64_t a_image, const void* B, int64_t b_group, int64_t b_image, void* C, void* stream, bool reference_order) {
     const int64_t es = ntg::elem_size(dtype), c_item = m * ldc;
-    if (groups > 1 && !is_valu_dtype(dtype) && m > 0 && n > 0 && k > 0 && batch > 0) {
+    const bool streaming = dtype != ntg::DT_F32 || m > 32 || batch * groups <= NTG_SKINNY_MAX_ITEMS;      // (in Float32 the kernels for few rows decide the sums)
+    if (groups > 1 && !is_valu_dtype(dtype) && streaming && m > 0 && n > 0 && k > 0 && batch > 0) {
         const int rc = check_sizes(m, k, n, batch);
         if (rc) return rc;
         ntg::GemmParams p;
@@ -2075,6 +2078,7 @@ static PointwiseDwPlan plan_pointwise_dw(int dtype, int64_t batch, int64_t chann
     const int64_t tiles = ((og + 63) / 64) * ((cg + 63) / 64) * batch * groups;
     if (tiles >= 0x7fffffffLL || L >= 0x7fffffffLL) return pl;
     if (es == 2 && L >= (1 << 23) / es) return pl;       // (the rows are the operands' pitch, and no kernel for pitches from 8 MiB on writes Float32 sums of 16-bit operands)
+    if (es == 4 && og <= 32 && batch * groups > NTG_SKINNY_MAX_ITEMS) return pl;
     const uint32_t steps = L % bk == 0 ? (uint32_t)(L / bk) : 1u;
     double best = 0.0;
     for (uint32_t s = 1; s <= steps && (s == 1 || tiles * s <= 2048); ++s) {      // (eight tiles a CU: more only makes more partial sums)

@@ -335,6 +335,41 @@ def test_fp32_one_tap_through_the_host_entry_points_is_the_reference_product(geo
                 assert np.array_equal(got.reshape(B, groups, m, L)[b, q], want), (b, q, m, k)
 
 
+@pytest.mark.parametrize("geom", [
+    # (B, C, size, O, groups): up to 32 rows in the forward product or the image gradient, 64 k and more; a pitch of one strip, of odd strips, of one column block
+    (8, 256, (28, 28), 64, 4), (3, 64, (32, 5), 256, 2), (2, 512, (28, 28), 32, 2), (5, 1040, (4,), 32, 4), (2, 128, (2044,), 16, 1),
+    (6, 64, (5992,), 32, 4), (2, 256, (4004,), 16, 1),
+], ids=str)
+def test_fp32_few_rows_in_groups_err_no_more_than_the_products_of_each_group(geom):
+    """The kernels for up to 32 rows add up eight short chains, and layers in groups go through them in one launch: the same bits as each group's layer
+    by itself.  The weight gradient of one tap is no further from the sums in 64 bits than the images' products added up (ratio 1 within some percent; one
+    chain an image was 2.9)."""
+    B, C, size, O, groups = geom
+    nd, cg, og = len(size), C // groups, O // groups
+    forward = {1: F.conv1d, 2: F.conv2d}[nd]
+    x, w, g = (randn(shape, torch.float32, i) for i, shape in enumerate(((B, C) + size, (O, cg) + (1,) * nd, (B, O) + size)))
+    y = forward(x, w, groups=groups)
+    dx, dw = backward(nd)(x, w, g, groups=groups)
+    per_image = torch.zeros_like(dw)
+    for q in range(groups):
+        c, o = slice(q * cg, (q + 1) * cg), slice(q * og, (q + 1) * og)
+        xq, wq, gq = x[:, c].contiguous(), w[o].contiguous(), g[:, o].contiguous()
+        assert torch.equal(y[:, o], forward(xq, wq)), q
+        assert torch.equal(dx[:, c], backward(nd)(xq, wq, gq)[0]), q
+        for b in range(B):
+            per_image[o] += F.matmult(gq[b].reshape(og, -1), xq[b].reshape(cg, -1), None, False, True).reshape(wq.shape)
+    want = exact_dw(x, g, (1,) * nd, (1,) * nd, (0,) * nd, (1,) * nd, groups)
+    assert relative(dw, want) <= 1.15 * relative(per_image, want), (relative(dw, want), relative(per_image, want))
+
+
+def test_fp32_few_rows_in_groups_of_more_images_than_a_launch_holds():
+    """65535 items: 33000 images in two groups go out group by group."""
+    x, w = randn((33000, 128, 4), torch.float32, 1), randn((32, 64, 1), torch.float32, 2)
+    y = F.conv1d(x, w, groups=2)
+    for q in range(2):
+        assert torch.equal(y[:, 16 * q:16 * q + 16], F.conv1d(x[:, 64 * q:64 * q + 64].contiguous(), w[16 * q:16 * q + 16].contiguous())), q
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("width", [2040, 2048])
 @pytest.mark.parametrize("groups", [1, 2])
