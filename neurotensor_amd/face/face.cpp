@@ -144,18 +144,22 @@ struct Geometry {
     int64_t B, C, O, groups, size[3], k[3], s[3], p[3], d[3], out[3];
 };
 
+// Options, sizes and kernels from here on go the general way, where no sum or product of them wraps: a padding of 2^63 - 1 must not come out as -1.
+constexpr int64_t LARGE = int64_t(1) << 31;
+
 bool options(Geometry& g, PyObject* stride, PyObject* padding, PyObject* dilation, PyObject* groups) {
     if (!per_axis(stride, g.nd, g.s) || !per_axis(padding, g.nd, g.p) || !per_axis(dilation, g.nd, g.d) || !whole(groups, g.groups) || g.groups < 1) return false;
     for (int a = 0; a < g.nd; ++a)
-        if (g.s[a] < 1 || g.d[a] < 1 || g.p[a] < 0) return false;
+        if (g.s[a] < 1 || g.d[a] < 1 || g.p[a] < 0 || g.s[a] >= LARGE || g.d[a] >= LARGE || g.p[a] >= LARGE) return false;
     return true;
 }
 // image and kernel as they are given; the outputs' sizes
 bool shapes(Geometry& g, at::IntArrayRef image, at::IntArrayRef kernel) {
     g.B = image[0]; g.C = image[1]; g.O = kernel[0];
-    if (g.B < 1 || g.C < 1 || g.O < 1 || g.C % g.groups != 0 || kernel[1] * g.groups != g.C || g.O % g.groups != 0) return false;
+    if (g.B < 1 || g.C < 1 || g.O < 1 || g.C % g.groups != 0 || kernel[1] != g.C / g.groups || g.O % g.groups != 0) return false;
     for (int a = 0; a < g.nd; ++a) {
         g.size[a] = image[2 + a]; g.k[a] = kernel[2 + a];
+        if (g.size[a] >= LARGE || g.k[a] >= LARGE) return false;
         const int64_t reach = g.size[a] + 2 * g.p[a] - g.d[a] * (g.k[a] - 1) - 1;
         if (g.size[a] < 1 || g.k[a] < 1 || reach < 0) return false;
         g.out[a] = reach / g.s[a] + 1;
@@ -257,10 +261,11 @@ PyObject* conv_backward(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const at::Tensor *x = dense(args[1], g.nd), *w = dense(args[2], g.nd), *dy = plain(args[3]);
     if (!x || !w || !dy || !dy->is_contiguous() || x->scalar_type() != w->scalar_type() || x->scalar_type() != dy->scalar_type() ||
         !options(g, args[4], args[5], args[6], args[7]) || !whole(args[8], stream) || !shapes(g, x->sizes(), w->sizes())) Py_RETURN_NONE;
-    int64_t numel = g.B * g.O;
-    for (int a = 0; a < g.nd; ++a) numel *= g.out[a];
+    int64_t numel = g.B;
+    bool wraps = __builtin_mul_overflow(numel, g.O, &numel);
+    for (int a = 0; a < g.nd; ++a) wraps |= __builtin_mul_overflow(numel, g.out[a], &numel);
     const int dt = ntg_dtype(x->scalar_type());
-    if (dt < 0 || dy->numel() != numel) Py_RETURN_NONE;
+    if (dt < 0 || wraps || dy->numel() != numel) Py_RETURN_NONE;
     at::Tensor dx, dw;
     int status;
     {
@@ -283,11 +288,13 @@ PyObject* conv_transpose(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     if (!x || !w || x->scalar_type() != w->scalar_type() || !options(g, args[3], args[4], args[6], args[7]) || !per_axis(args[5], g.nd, op) ||
         !whole(args[8], stream)) Py_RETURN_NONE;
     const int dt = ntg_dtype(x->scalar_type());
-    g.B = x->size(0); g.C = x->size(1); g.O = w->size(1) * g.groups;
-    if (dt < 0 || g.B < 1 || g.C < 1 || g.O < 1 || w->size(0) != g.C || g.C % g.groups != 0) Py_RETURN_NONE;
+    g.B = x->size(0); g.C = x->size(1);
+    if (dt < 0 || g.B < 1 || g.C < 1 || w->size(1) < 1 || w->size(0) != g.C || g.C % g.groups != 0) Py_RETURN_NONE;
+    g.O = w->size(1) * g.groups;                                   // (at most the kernel's elements: groups <= its first size)
     c10::SmallVector<int64_t, 5> size = {g.B, g.O};
     for (int a = 0; a < g.nd; ++a) {
         g.size[a] = x->size(2 + a); g.k[a] = w->size(2 + a);
+        if (g.size[a] >= LARGE || g.k[a] >= LARGE || op[a] >= LARGE) Py_RETURN_NONE;
         const int64_t out = (g.size[a] - 1) * g.s[a] - 2 * g.p[a] + g.d[a] * (g.k[a] - 1) + 1 + op[a];
         if (g.size[a] < 1 || g.k[a] < 1 || op[a] < 0 || out < 1) Py_RETURN_NONE;
         size.push_back(out);

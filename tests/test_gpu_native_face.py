@@ -128,3 +128,21 @@ def test_the_native_side_leaves_everything_but_plain_device_tensors_to_the_gener
     assert F._face.conv(2, torch.ones(1, 1, 3, 3), torch.ones(1, 1, 1, 1), 1, 0, 1, 1, 0) is None
     assert F._face.conv(7, m, m, 1, 0, 1, 1, 0) is None
     assert F._face.conv_backward(2, m, m) is None
+
+
+@gpu
+@pytest.mark.parametrize("large", [2 ** 31, 2 ** 62, 2 ** 63 - 1], ids=hex)
+def test_options_whose_sums_would_wrap_are_left_to_the_general_ways(large):
+    """(2 x padding and dilation x (kernel - 1) of 2^63 - 1 are -2 in 64 bits: a geometry that looks sound.)"""
+    for axes in (1, 2, 3):
+        x, w = t(2, 8, *(8,) * axes), t(8, 8, *(3,) * axes)
+        for options in ((1, large, 1, 1), (1, large, large, 1), (large, 0, large, 1), (1, 0, 1, large), (1, (large,) * axes, 1, 1)):
+            assert F._face.conv(axes, x, w, *options, 0) is None, options
+            assert F._face.conv_backward(axes, x, w, t(2, 8, *(6,) * axes), *options, 0) is None, options
+            assert F._face.conv_backward(axes, x, w, t(0), *options, 0) is None, options
+            s, p, d, groups = options
+            assert F._face.conv_transpose(axes, x, w, s, p, 0, d, groups, 0) is None, options
+            assert F._face.conv_transpose_backward(axes, x, w, t(2, 8, *(10,) * axes), *options, 0) is None, options
+        assert F._face.conv_transpose(axes, x, w, 2, 0, large, 1, 1, 0) is None
+    # two output sizes of 2^32 are no pixels in 64 bits
+    assert F._face.conv_backward(2, t(2, 8, 8, 8), t(8, 8, 1, 1), t(0), 1, 2 ** 31 - 4, 1, 1, 0) is None
