@@ -9,6 +9,7 @@ ValueError where the reference throws from utils::throw_exception.
 import ctypes
 import importlib.util
 import os
+import warnings
 
 import torch
 
@@ -44,13 +45,18 @@ else:
 
 
 def _load_native():
-    """lib/_face.so: the usual calls in one native call each (face/face.cpp).  Without it everything goes the general ways below."""
+    """_face.so beside libntgemm.so: the usual calls in one native call each (face/face.cpp).  Without it, where it does not load (built for another torch or
+    Python), and with a library of another name, which it would not call, everything goes the general ways below."""
     path = os.path.join(os.path.dirname(_lib.LIB_PATH), "_face.so")
-    if not os.path.exists(path):
+    if os.path.basename(_lib.LIB_PATH) != "libntgemm.so" or not os.path.exists(path):
         return None
     spec = importlib.util.spec_from_file_location("neurotensor_amd._face", path)
-    module = importlib.util.module_from_spec(spec)
-    spec.loader.exec_module(module)
+    try:
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+    except (ImportError, OSError) as e:
+        warnings.warn(f"{path} does not load, calls take more time on the host: {e}", RuntimeWarning)
+        return None
     return module
 
 

@@ -1,7 +1,10 @@
 """The native side of functional.py (face/face.cpp) against the general Python ways: the same results, the same refusals."""
+import os
+
 import pytest
 import torch
 
+from neurotensor_amd import _lib
 from neurotensor_amd import functional as F
 
 gpu = pytest.mark.gpu
@@ -146,3 +149,15 @@ def test_options_whose_sums_would_wrap_are_left_to_the_general_ways(large):
         assert F._face.conv_transpose(axes, x, w, 2, 0, large, 1, 1, 0) is None
     # two output sizes of 2^32 are no pixels in 64 bits
     assert F._face.conv_backward(2, t(2, 8, 8, 8), t(8, 8, 1, 1), t(0), 1, 2 ** 31 - 4, 1, 1, 0) is None
+
+
+def test_a_native_side_that_does_not_load_is_done_without(monkeypatch, tmp_path):
+    assert F._load_native() is not None
+    monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "libntgemm.so"))
+    assert F._load_native() is None                                     # none there
+    (tmp_path / "_face.so").write_bytes(b"built for something else")
+    with pytest.warns(RuntimeWarning, match="_face.so does not load"):
+        assert F._load_native() is None
+    # another build of the library in the same directory: the native side calls libntgemm.so only
+    monkeypatch.setattr(_lib, "LIB_PATH", os.path.join(os.path.dirname(_lib.__file__), "lib", "libntgemm_other.so"))
+    assert F._load_native() is None
