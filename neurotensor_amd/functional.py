@@ -226,6 +226,15 @@ def linear(x, w, bias, transpose_a=False, transpose_b=False, _relu=False):
     def unsq(t):      # unsqueeze_as, matmult_cpu.cpp:1712-1713
         return t.reshape((1,) * (nd - t.dim()) + tuple(t.shape))
 
+    if x.dim() == 2 and w.dim() == 2 and bias.dim() == 1:
+        # a layer's call that the native side left (a slice, an active mode): one bias row for a matrix, what the rules below come down to
+        x_st, ta = _as_matrix_view(x, bool(transpose_a))
+        w_st, tb = _as_matrix_view(w, bool(transpose_b))
+        m, k, n = _logical(x_st.shape, w_st.shape, ta, tb)
+        if bias.shape[0] == n and m and n:
+            out = torch.empty((m, n), dtype=x.dtype, device=x.device)
+            _launch(x_st, w_st, out, m, k, n, ta, tb, 1, m * k, k * n, m * n, _lib.C_BIAS, bias=bias.contiguous(), bias_strides=(0, 0, 1), relu=_relu)
+            return out
     x, w, bias = unsq(x), unsq(w), unsq(bias)
     x_st, ta = _as_matrix_view(x, bool(transpose_a))
     w_st, tb = _as_matrix_view(w, bool(transpose_b))
