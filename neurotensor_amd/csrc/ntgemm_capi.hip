@@ -1496,16 +1496,18 @@ static bool conv_nhwc_ok(int dtype, int64_t batch, int64_t channels, int64_t out
 // Few output tiles and a deep k (a handful of small maps with many channels): the 64-byte runs of channels in `ranges` equal ranges, Float32 sums of
 // each, added up in order by a second pass.  A workgroup alone on its CU takes 0.32 us a K-step in Float32 and 0.2 in 16 bits whatever the others do (2 x 256 x
 // 13 x 13 -> 256 by 3 x 3: 24 tiles of 144 and 72 K-steps); shared by w workgroups a CU takes 0.25 w and 0.07 w.  The second pass costs 4.5 us and the traffic of
-// the sums.  Measured: that layer 47 -> 11 + 3 us and 18 -> 8 + 3; 192 x 17 x 17 -> 32 by 7 x 7, 3 tiles of 588, 169 -> 33 + 4 us.  The number of ranges does not depend on the number of images, only whether
-// there are any: up to 128 tiles an image's result is the same bits alone and among others.  Under 64 K-steps there is too little to win.  Layers in groups
-// alike (Float32 256 x 11^3 -> 128 by 3 x 3 x 3 at stride 2 in 4 groups, a step, 85 -> 62 us, 4 x 96 x 8 x 8 -> 16 by 5 x 5 at stride 2 in 2 56 -> 44).
+// the sums.  Measured: that layer 47 -> 11 + 3 us and 18 -> 8 + 3; 192 x 17 x 17 -> 32 by 7 x 7, 3 tiles of 588, 169 -> 33 + 4 us.  Under 64 K-steps there is too little
+// to win.  Layers in groups alike (Float32 256 x 11^3 -> 128 by 3 x 3 x 3 at stride 2 in 4 groups, a step, 85 -> 62 us, 4 x 96 x 8 x 8 -> 16 by 5 x 5 at stride 2 in 2
+// 56 -> 44).  Whether there are ranges, and how many, follows from one image, so up to 128 tiles in all an image's result is the same bits alone and among
+// others (in whole runs: nhwc_form looks at all images' pixels).  That is ahead all the way: BFloat16 n x 256 x 13 x 13 -> 256 by
+// 3 x 3, a step, without | with ranges in the products: 10 images 64.0 | 55.6 us; 256 x 16 x 16 -> 256, 8 images 62.8 | 58.9.
 static int64_t conv_k_ranges(int64_t es, int64_t batch, int64_t rows, int64_t pixels, int64_t groups, const NhwcForm& form, int64_t taps) {
-    const int64_t bk = 64 / es, runs = form.cgp / bk, steps = runs * taps, tiles = ((rows / groups + 63) / 64) * ((pixels + 63) / 64) * batch * groups;
-    if (form.slot_v || tiles > 128 || steps < 64) return 1;
+    const int64_t bk = 64 / es, runs = form.cgp / bk, steps = runs * taps, tiles = ((rows / groups + 63) / 64) * ((pixels + 63) / 64) * groups;
+    if (form.slot_v || tiles * batch > 128 || steps < 64) return 1;
     int64_t r = 8;
     while (r > 1 && (runs % r != 0 || steps / r < 16)) --r;
     const double shared = (double)((tiles * r + 255) / 256), step_us = es == 4 ? 0.32 : 0.2, shared_us = std::max(step_us, (es == 4 ? 0.25 : 0.07) * shared);
-    const double sums_us = 4.5 + 8.0 * (double)(r * batch * rows * pixels) / 4.0e6;
+    const double sums_us = 4.5 + 8.0 * (double)(r * rows * pixels) / 4.0e6;
     return (double)(steps / r) * shared_us + sums_us < 0.8 * (double)steps * step_us ? r : 1;
 }
 static int64_t conv_k_ranges_bytes(int64_t ranges, int64_t batch, int64_t rows, int64_t pixels) { return ranges > 1 ? ranges * batch * rows * ((pixels + 7) / 8 * 8) * 4 : 0; }

@@ -256,3 +256,22 @@ def test_channels_in_ranges_with_the_columns_split(dtype):
     want, mags = (CONV[2](a.double(), b.double(), padding=3) for a, b in ((x[::7], w), (x[::7].abs(), w.abs())))
     bound = UNIT[dtype] * want.abs() + 2.0 ** -24 * (256 * 49 + 32) * mags + (2.0 ** -25 if dtype == torch.float16 else 0.0)
     assert bool(((got - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("cin,cout,size,kernel,batches", [
+    (256, 256, (13, 13), 3, (1, 9, 10)),             # 12 tiles an image
+    (256, 256, (16, 16), 3, (1, 6, 7, 8)),           # 16: 128 of them
+    (512, 32, (9,), 3, (1, 2, 128)),
+    (64, 64, (11, 11), 7, (1, 3, 64)),
+], ids=str)
+def test_an_image_is_the_same_bits_alone_and_among_others(dtype, cin, cout, size, kernel, batches):
+    """Channels in ranges, up to 128 tiles in all: forward product and image gradient."""
+    x, w, dy = (t.cuda() for t in operands(dtype, max(batches), cin, cout, size, kernel, 1, kernel // 2, 1, False))
+    forward, backward = OURS[(len(size), False)]
+    opt = {"padding": kernel // 2}
+    alone = [(forward(x[i:i + 1], w, **opt)[0], backward(x[i:i + 1], w, dy[i:i + 1], **opt)[0][0]) for i in (0, max(batches) - 1)]
+    for n in batches:
+        y, dx = forward(x[:n], w, **opt), backward(x[:n], w, dy[:n], **opt)[0]
+        assert torch.equal(y[0], alone[0][0]) and torch.equal(dx[0], alone[0][1]), n
+    assert torch.equal(y[-1], alone[1][0]) and torch.equal(dx[-1], alone[1][1])
