@@ -1456,13 +1456,17 @@ static HaloPlan conv_halo(const Geo3& g) {
 // that is less; the kernel's K-steps are then four slots of whatever taps.  us of the forward product and what it needs, as whole runs, merged taps or
 // element-wise gathers | in slots: BFloat16 16 x 24 x 56 x 56 -> 24 by 3 x 3 21 | 12, 16 x 48 x 47 x 47 -> 16 by 5 x 5 in 2 groups 43 | 18, 14 x 1 x 40^3 -> 32 by
 // 3 x 3 x 3 365 | 83, Float32 32 x 3 x 224 x 224 -> 64 by 7 x 7 at stride 2 144 | 126, 16 x 24 x 56 x 56 -> 24 29 | 19, 16 x 48 x 47 x 47 -> 16 in 2 groups 104 | 46,
-// 4 x 24 x 20^3 -> 40 47 | 33; equal on one or two tiles (Float32 1 x 24 x 12 x 12 -> 24 12 | 12).  Up to 128 output pixels, the columns of one
-// flat tile, the other forms stay with the workspaces that callers know: a step takes about as long (8 x 8 pixels so | 9 x 9 in slots: BFloat16 24 -> 24 29.0 | 29.1,
-// 16 -> 32 28.7 | 29.1, Float32 24 -> 24 38 | 34).
+// 4 x 24 x 20^3 -> 40 47 | 33; equal on one or two tiles (Float32 1 x 24 x 12 x 12 -> 24 12 | 12).  Up to 128 output pixels the other forms stay for the
+// workspaces that callers know (tests/test_abi.py holds some), not for speed: steps of n x 24 x 8 x 8 -> 24 take 21.0 us so | 20.2 in slots with one image in BFloat16,
+// 21.7 | 20.9 with four, Float32 35.0 | 28.9 and 35.5 | 29.6, 72 -> 72 63 | 46.
+// In 16 bits wide groups lose little to whole runs, whose taps meet a pixel's line while it is in L2: there slots are taken where they save a quarter of k, or on few
+// pixels.  Steps in BFloat16, whole runs | slots: 72 channels (9 slots of 12) 32 x 56 x 56 by 3 x 3 131 | 125, 16 x 28 x 28 46 | 41; 104 (13 of 16) 168 | 178 and 53 | 51,
+// 20^3 104 | 111; 168 (21 of 24) 343 | 347 and 77 | 90, 161 | 185; 232 (29 of 32) 476 | 486 and 98 | 107, 224 | 259; 4 x 28 x 28 of 104, 168, 232 37.7 | 35.1, 51 | 47, 64 | 60.
 struct NhwcForm { int64_t cgp, slot_v; };
-static NhwcForm nhwc_form(int64_t es, int64_t cg, int64_t taps, bool bordered, int64_t pixels) {
-    const int64_t vel = 16 / es, run = 64 / es, slots = (cg + vel - 1) / vel;
-    if (bordered && cg > 0 && pixels > 128 && slots * vel % run != 0 && taps * slots <= NTG_SLOT_TABLE) return {slots * vel, slots};
+static NhwcForm nhwc_form(int64_t es, int64_t cg, int64_t taps, int nd, bool bordered, int64_t pixels) {
+    const int64_t vel = 16 / es, slots = (cg + vel - 1) / vel, in_runs = (slots + 3) / 4 * 4;
+    const bool fewer = es == 4 ? slots < in_runs : 4 * slots <= 3 * in_runs || (slots < in_runs && pixels < (in_runs <= 16 && nd < 3 ? 32768 : 8192));
+    if (bordered && cg > 0 && pixels > 128 && fewer && taps * slots <= NTG_SLOT_TABLE) return {slots * vel, slots};
     return {nhwc_padded_channels(es, cg), 0};
 }
 
@@ -1474,7 +1478,7 @@ static bool conv_nhwc_merged(int dtype, int64_t batch, int64_t channels, int64_t
     if (dtype != ntg::DT_F32 && dtype != ntg::DT_F16 && dtype != ntg::DT_BF16) return false;
     if (g.nd != 2 || !conv_implicit_g(dtype, channels, g) || out_channels <= 0) return false;
     const int64_t es = ntg::elem_size(dtype), cg = channels / groups;
-    if (cg <= 0 || cg * es > 32 || nhwc_form(es, cg, g.taps(), conv_halo(g).on, batch * g.L()).slot_v) return false;
+    if (cg <= 0 || cg * es > 32 || nhwc_form(es, cg, g.taps(), g.nd, conv_halo(g).on, batch * g.L()).slot_v) return false;
     const int64_t cb = cg * es <= 16 ? 16 : 32;
     mt.cgp = cb / es; mt.T = 64 / cb; mt.kq_pad = (g.k[2] + mt.T - 1) / mt.T * mt.T;
     if (mt.kq_pad > 8 || mt.kq_pad * mt.cgp > 4 * g.k[2] * cg || out_channels * g.k[1] * mt.kq_pad >= 0x7fffffffLL) return false;          // (padding: at most 4x the arithmetic)
@@ -1489,7 +1493,7 @@ static bool conv_nhwc_ok(int dtype, int64_t batch, int64_t channels, int64_t out
     if (!conv_implicit_g(dtype, channels, g)) return false;
     const HaloPlan halo = conv_halo(g);
     if (g.nd == 3 && !halo.on) return false;                          // (three axes: the bordered copy is the only form)
-    const int64_t es = ntg::elem_size(dtype), cgp = nhwc_form(es, channels / groups, g.taps(), halo.on, batch * g.L()).cgp;
+    const int64_t es = ntg::elem_size(dtype), cgp = nhwc_form(es, channels / groups, g.taps(), g.nd, halo.on, batch * g.L()).cgp;
     return cgp > 0 && out_channels > 0 && out_channels * g.taps() < 0x7fffffffLL && conv_nhwc_offsets_fit(groups * cgp, es, g) &&
            conv_nhwc_offsets_fit(groups * cgp, es, halo.gp);
 }
@@ -1535,7 +1539,7 @@ static hipError_t launch_conv_k_ranges(ntg::GemmParams p, int dtype, int64_t bat
 static int64_t conv_nhwc_workspace(int dtype, int64_t batch, int64_t channels, int64_t out_channels, int64_t groups, const Geo3& g) {
     const HaloPlan halo = conv_halo(g);
     const int64_t es = ntg::elem_size(dtype);
-    const NhwcForm form = nhwc_form(es, channels / groups, g.taps(), halo.on, batch * g.L());
+    const NhwcForm form = nhwc_form(es, channels / groups, g.taps(), g.nd, halo.on, batch * g.L());
     const int64_t cgp = form.cgp, weights = out_channels * cgp * g.taps() * es;
     const int64_t sums = halo.on ? conv_k_ranges_bytes(conv_k_ranges(es, batch, out_channels, g.L(), groups, form, g.taps()), batch, out_channels, g.L()) : 0;
     return (int64_t)align_up((size_t)(batch * groups * cgp * halo.vol * es), 256) + (sums ? (int64_t)align_up((size_t)weights, 256) + sums : weights);
@@ -1551,7 +1555,7 @@ static int conv_forward_nhwc(int dtype, const void* image, const void* kernel, v
                              int64_t out_channels, const Geo3& g, int64_t groups, hipStream_t hs, const MergedTaps* mt = nullptr) {
     const int64_t es = ntg::elem_size(dtype), cg = channels / groups, og = out_channels / groups;
     HaloPlan halo = conv_halo(g);
-    const NhwcForm form = nhwc_form(es, cg, g.taps(), halo.on, batch * g.L());
+    const NhwcForm form = nhwc_form(es, cg, g.taps(), g.nd, halo.on, batch * g.L());
     const int64_t cgp = mt ? mt->cgp : form.cgp, chp = groups * cgp;      // channels per group / per pixel in the copy
     const int64_t L = g.L(), taps = g.taps(), vol = g.vol(), K = mt ? g.k[1] * mt->kq_pad * cgp : taps * cgp;
     if (mt) { halo.on = false; halo.vol = vol; halo.gp = g; }                    // (the merged-tap form keeps its validity bits)
@@ -1650,7 +1654,7 @@ static int conv_dimage_nhwc(int dtype, const void* kernel, const void* grad_out,
     const int64_t es = ntg::elem_size(dtype), cg = channels / groups, og = out_channels / groups;
     const Geo3 t = geo_dimage(g);
     const HaloPlan halo = conv_halo(t);                                         // (the "image" of this convolution is dY)
-    const NhwcForm form = nhwc_form(es, og, g.taps(), halo.on, batch * t.L());
+    const NhwcForm form = nhwc_form(es, og, g.taps(), g.nd, halo.on, batch * t.L());
     const int64_t ogp = form.cgp, ochp = groups * ogp;                          // out channels per group / per pixel in the copy
     const int64_t L = g.L(), taps = g.taps(), vol = g.vol(), K = taps * ogp;
     const int64_t Lp = halo.vol;
@@ -1718,7 +1722,7 @@ struct PhasePlan {
 static NhwcForm phase_form(int64_t es, int64_t og, int64_t batch, int64_t channels, const Geo3& g) {
     int64_t taps = 1;                                                             // of the largest phase
     for (int a = 0; a < 3; ++a) taps *= (g.k[a] + g.s[a] - 1) / g.s[a];
-    const NhwcForm f = nhwc_form(es, og, taps, true, batch * g.vol());
+    const NhwcForm f = nhwc_form(es, og, taps, g.nd, true, batch * g.vol());
     // (a chain ends with a K-step at the earliest: in slots it would run through several taps of fewer than 16 channels)
     if (es == 4 && og < 16 && f.slot_v) return {16, 0};
     if (f.slot_v) return f;

@@ -193,6 +193,18 @@ def test_taps_in_slots(dtype, batch, cin, cout, size, kernel, stride, pad, group
     check(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed, parts)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("batch,cin,cout,size,kernel,stride,pad,groups,transposed", [
+    (8, 104, 8, (64, 63), 3, 1, 1, 1, False), (8, 104, 8, (64, 64), 3, 1, 1, 1, False),      # 13 slots of 16: under 32768 pixels and from there
+    (2, 8, 136, (64, 63), 3, 1, 1, 1, False), (2, 8, 136, (64, 64), 3, 1, 1, 1, False),      # 17 of 20, the image gradient: 8192
+    (1, 104, 24, (16, 16, 31), 3, 1, 1, 1, False), (1, 104, 24, (16, 16, 32), 3, 1, 1, 1, False),
+    (2, 24, 104, (128, 128), 3, 2, 1, 1, False),                                             # the phases of 32768 image pixels
+    (2, 208, 16, (64, 64), 2, 2, 0, 2, True),
+], ids=str)
+def test_wide_groups_in_slots_or_whole_runs(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed):
+    check(dtype, batch, cin, cout, size, kernel, stride, pad, groups, transposed)
+
+
 def test_taps_in_slots_dilated_and_the_longest_table():
     gen = torch.Generator(device="cuda").manual_seed(6)
     for shape, w, opt in (((2, 24, 20, 20), (8, 24, 3, 3), {"dilation": 3, "padding": 3}), ((1, 40, 12, 12), (8, 40, 8, 8), {"padding": 3}),
