@@ -287,12 +287,16 @@ int64_t ntg_conv2d_forward_workspace_bytes(int dtype, int64_t batch, int64_t cha
                                            int64_t k_r, int64_t k_c, int64_t s_r, int64_t s_c,
                                            int64_t p_r, int64_t p_c, int64_t d_r, int64_t d_c);
 
-/* Bytes of device workspace with which ntg_conv2d_dev runs its fastest form.  For Float32 whose channels per group are a
- * multiple of 16, Float16 / BFloat16 with at least 8 channels per group (padded with zeros to a multiple of 32 in the
- * copy), and groups of up to 32 bytes of channels in all three (RGB input layers: pixels of 16 or 32 bytes, several taps
- * per K-step), that is a channels-last copy of the image (with the padding as a border of zero pixels where the channels
- * of a group fill whole 64-byte runs) plus the weights with the channel index fastest; the convolution (conv.cpp:86-118)
- * then gathers its operand in 16-byte pieces.  Otherwise the figure of
+/* Bytes of device workspace with which ntg_conv2d_dev runs its fastest form.  For Float32, Float16 and BFloat16 (kernels up
+ * to 8 taps an axis) that is a channels-last copy of the image plus the weights in the order of the product's k; the
+ * convolution (conv.cpp:86-118) then gathers its operand in 16-byte pieces.  The copy carries the padding as a border of
+ * zero pixels unless that makes it more than twice the image (four times up to 1024 pixels), and the channels of a group
+ *   in whole 64-byte runs where they fill them, or where 16-bit ones nearly do (padded with zeros),
+ *   else, behind a border, in whole 16-byte slots (four or eight channels), whatever the number of channels.
+ * Up to 128 output pixels in all, and without a border, whole runs (in 16 bits padded, up to four times) or pixels of 16 or 32
+ * bytes (groups of up to 32 bytes of channels) take the place of slots; other Float32 groups have no such form there.  A few
+ * small maps with many channels add Float32 partial sums of up to eight ranges of channels, 4 bytes an output each.
+ * Which form it is follows from all sizes, the number of images included: ask for the sizes of the call.  Otherwise the figure of
  * ntg_conv2d_forward_workspace_bytes.  ntg_conv2d_dev accepts any smaller workspace and falls back to its other forms. */
 int64_t ntg_conv2d_fast_workspace_bytes(int dtype, int64_t batch, int64_t channels, int64_t height, int64_t width,
                                         int64_t out_channels, int64_t k_r, int64_t k_c, int64_t s_r, int64_t s_c,
@@ -315,18 +319,23 @@ int ntg_unfold2d_backward_dev(int dtype, const void* col, void* image,
                               int64_t k_r, int64_t k_c, int64_t s_r, int64_t s_c,
                               int64_t p_r, int64_t p_c, int64_t d_r, int64_t d_c, int accumulate, void* stream);
 
-/* Bytes of device workspace ntg_conv2d_backward_dev needs when both gradients are requested.  Floating dtypes with
- * kernels up to 8x8 compute conv_dkernel (conv.cpp:444-471) without the stored im2col matrix (workspace = the per-image
- * weight gradients, batch * out_channels * channels/groups * k_r * k_c elements) and, at stride 1, conv_dimage
- * (conv.cpp:318-346) as well; every other case needs the im2col-sized buffer (ntg_conv2d_workspace_bytes).  Where
- * conv_dimage can run in its channels-last form (Float32 / Float16 / BFloat16, two axes, stride 1, the out channels of a
- * group filling whole 64-byte runs) the figure also covers a channels-last copy of grad_out plus the flipped weights; the
- * call still accepts the smaller amount and then gathers from grad_out as it lies. */
+/* Bytes of device workspace with which ntg_conv2d_backward_dev runs its fastest forms, both gradients requested: the largest of
+ *   what the call needs at least: floating dtypes with kernels up to 8x8 compute conv_dkernel (conv.cpp:444-471) without the
+ *     stored im2col matrix (the per-image weight gradients, batch * out_channels * channels/groups * k_r * k_c elements) and,
+ *     at stride 1, conv_dimage (conv.cpp:318-346) as well; every other case needs the im2col-sized buffer
+ *     (ntg_conv2d_workspace_bytes),
+ *   and, for Float32, Float16 and BFloat16,
+ *     conv_dkernel: a channels-last copy of the image (channels padded to 16 bytes, bordered), one of grad_out where that is
+ *       read so, and Float32 partial sums of up to some 2048 tiles; one tap: those of ranges of the images' pixels alone,
+ *     conv_dimage at stride 1: the forward form (ntg_conv2d_fast_workspace_bytes) of the convolution of grad_out that it is,
+ *     conv_dimage at strides up to 4: a bordered channels-last copy of grad_out, the weights and the phases of the image,
+ *     the copies of both gradients side by side, made in one launch, while that is 64 MiB at most.
+ * The call accepts every amount from the least on and takes the forms that fit. */
 int64_t ntg_conv2d_backward_workspace_bytes(int dtype, int64_t batch, int64_t channels, int64_t height, int64_t width,
                                             int64_t out_channels, int64_t k_r, int64_t k_c, int64_t s_r, int64_t s_c,
                                             int64_t p_r, int64_t p_c, int64_t d_r, int64_t d_c, int64_t groups);
 
-/* workspace: at least ntg_conv2d_backward_workspace_bytes */
+/* workspace: ntg_conv2d_backward_workspace_bytes, or as little as its first item */
 int ntg_conv2d_backward_dev(int dtype, const void* image, const void* kernel, const void* grad_out,
                             void* d_image, void* d_kernel, void* workspace, int64_t workspace_bytes,
                             int64_t batch, int64_t channels, int64_t height, int64_t width,
@@ -365,7 +374,7 @@ int ntg_conv_transpose2d(int dtype, const void* input, const void* kernel, void*
  *   with ntg_convnd_workspace_bytes -- element by element: a Float32 result is unfold + matmult bit for bit, a weight
  *     gradient sums the output pixels of one image in ascending order and then the images (like the host entry points);
  *   with ntg_convnd_fast_workspace_bytes -- Float32 / Float16 / BFloat16 from channels-last copies that carry the padding:
- *     k runs (channels of one 64-byte run, tap) in the forward call and the image gradient, which at strides > 1 is one
+ *     k runs (channels of one 64-byte run, tap), or (tap, channels in 16-byte slots), in the forward call and the image gradient, which at strides > 1 is one
  *     convolution per residue of the image position; the weight gradient's sums run through the pixels of all images in
  *     equal ranges, `accumulate` adds the incoming value last.  Float32 chains of the gradients (at strides > 1 of the image's) end every 16 to
  *     128 multiply-adds and are added up, no longer ones than one tap's or one image's.  Where there is no such form the two figures are equal.

@@ -680,7 +680,7 @@ int desc_to_params(const ntg_gemm_desc* d, ntg::GemmParams& p) {
 // image * (the images' stride), its result at a uniform stride (rows of the groups follow each other in every layout used here).  A launch
 // a group is `groups` times the 4-5 us that a launch costs the host and as many half-empty rounds: training steps in groups, us before | now:
 // BFloat16 1 x 96 x 48 x 48 -> 16 by 3 x 3 in 4 groups 118 | 51, Float32 6 x 256 x 32 x 32 -> 96 by 5 x 5 at stride 2 in 4 groups 239 | 99,
-// Float16 10 x 64 x 216 x 216 -> 192 by 3 x 3 in 4 groups 854 | 814; 40 drawn ones 0.77 of their time.
+// Float16 10 x 64 x 216 x 216 -> 192 by 3 x 3 in 4 groups 854 | 814.
 struct GroupStrides { int64_t a_group, a_image, b_group, b_image, c_item; };      // elements
 template <class Launch>
 static hipError_t launch_groups(ntg::GemmParams p, int dtype, int64_t batch, int64_t groups, const GroupStrides& st, Launch&& launch) {
@@ -1867,10 +1867,9 @@ static int64_t dkernel_padded_channels(int64_t es, int64_t cg) { const int64_t v
 static HaloPlan dkernel_halo(int64_t es, int64_t cg, int64_t groups, const Geo3& g) {
     HaloPlan h = conv_halo(g);
     const int64_t cgp = dkernel_padded_channels(es, cg);
-    // (a copy that pads the channels grows by its border as well, which takes a launch of its own: on one and two axes only where the border
-    //  is a quarter of the image at most, as it is from 17 x 17 pixels on for a 3 x 3 window.  Validity tests against the border, us per
-    //  weight gradient: Float32 64 x 3 x 16 x 16 -> 64 by 3 x 3 20.1 | 23.1, 256 x 6 x 16 x 16 -> 96 35.9 | 36.5, 64 x 60 x 16 x 16 -> 128
-    //  41.9 | 41.9, 256 x 3 x 32 x 32 -> 64 by 5 x 5 56.2 | 55.3; BFloat16 20.4 | 23.2, 20.3 | 23.0, 25.2 | 27.7, 37.6 | 37.7)
+    // (a copy that pads the channels grows by its border as well: on one and two axes that is kept to a quarter of the image, as it is from 17 x 17 pixels on for a
+    //  3 x 3 window, for the workspace alone.  Steps with validity tests | with the border, us: BFloat16 64 x 3 x 16 x 16 -> 64 by 3 x 3 26.1 | 25.8, 256 x 3 x 32 x 32 ->
+    //  64 by 5 x 5 132 | 128, Float32 39.5 | 39.0, 331 | 324, 256 x 6 x 16 x 16 -> 96 100 | 94, 64 x 102 x 14 x 14 -> 128 134 | 129; equal on 8 x 8)
     const bool wide_border = g.nd < 3 && cgp != cg && 4 * h.vol > 5 * g.vol();
     if (h.on && (wide_border || !conv_nhwc_offsets_fit(groups * cgp, es, h.gp))) {
         h.on = false; h.gp = g; h.vol = g.vol();
@@ -1901,7 +1900,7 @@ static double dkernel_cost_us(int64_t es, int rows, int cols, int64_t tiles, int
     const double alone = cols == 64 || rows == 32 ? 0.0075 : 0.0085, each = cols == 64 ? 0.0035 : rows == 32 ? 0.0046 : 0.0055;
     return 3.0 + k * std::max(alone, each * w);
 }
-// How dW is cut up: `ranges` k ranges of `kr` output pixels (0: one product per image), tiles of edge x edge, dY read where it
+// How dW is cut up: `ranges` k ranges of `kr` output pixels (0: one product per image), tiles of rows x cols, dY read where it
 // lies (its rows 16-byte multiples, an image a whole number of K-steps) or through a channels-last copy of its own (any range then), with
 // the out channels of a group padded to 16 bytes: rows of zeros that the last pass skips.  Without that padding a layer with odd planes and odd
 // channels ran on the element-wise gather, one chain an image: BFloat16 5 x 192 x 125 x 125 -> 48 by one tap in 4 groups, a step 2033 us before, 153 with
@@ -1939,9 +1938,9 @@ static DkernelPlan plan_dkernel(int dtype, int64_t batch, int64_t channels, int6
         pl.kr = total / forced;
         pl.rows = pl.cols = es == 2 ? ntg::ring16_tile_edge(og, N, pl.kr, forced) : 64;
     } else {
-        // A range has the pixels of an image at least, where those are two to eight K-steps: over small maps longer ranges are few and cost
-        // time, as the groups run one behind the other (58 x 64 x 17 -> 64 by 5 in 8 groups: backward 136 us, 108 with short ranges), while
-        // shorter ones ask for a larger workspace than one gradient per image.
+        // A range has the pixels of an image at least, where those are two to eight K-steps: over small maps ranges of eight are too few (a step of 58 x 64 x 17 -> 64
+        // by 5 in 8 groups, in ranges from an image's pixels | from eight K-steps on: BFloat16 23.7 | 25.0 us, Float32 27.4 | 30.4; without groups 24.8 | 26.1, 36.4 |
+        // 38.7), while shorter ones gain nothing and ask for a larger workspace than one gradient per image.
         const int64_t shortest = std::min<int64_t>(8, std::max<int64_t>(2, (L + bk - 1) / bk));
         double best = 0.0;
         const auto consider = [&](bool copy, int64_t ranges, int64_t items, int64_t kr, int rows, int cols) {
