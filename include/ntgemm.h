@@ -377,7 +377,7 @@ int ntg_conv_transpose2d(int dtype, const void* input, const void* kernel, void*
  *     k runs (channels of one 64-byte run, tap), or (tap, channels in 16-byte slots), in the forward call and the image gradient, which at strides > 1 is one
  *     convolution per residue of the image position; the weight gradient's sums run through the pixels of all images in
  *     equal ranges, `accumulate` adds the incoming value last.  Float32 chains of the gradients (at strides > 1 of the image's) end every 16 to
- *     128 multiply-adds and are added up, no longer ones than one tap's or one image's.  Where there is no such form the two figures are equal.
+ *     256 multiply-adds and are added up, no longer ones than one tap's or one image's.  Where there is no such form the two figures are equal.
  * ndim <= 2: the first is ntg_conv2d_forward_workspace_bytes, the second ntg_conv2d_fast_workspace_bytes; both are
  * ntg_conv2d_backward_workspace_bytes for the gradients.  `backward` selects the workspace of the gradient call.  The
  * calls accept every amount from the first figure on; ntg_conv_transposend_workspace_bytes is that of the fast forms. */

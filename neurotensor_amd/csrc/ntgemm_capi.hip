@@ -1687,13 +1687,13 @@ static int conv_dimage_nhwc(int dtype, const void* kernel, const void* grad_out,
 }
 
 // Float32: K-steps (16 multiply-adds) of one chain in a gathered product that stands for shorter ones of `n` multiply-adds each, added
-// up: the largest power of two within n, from one K-step to eight.  Sixteen gain no time (4 x 32 x 32^3 -> 64 by 3 x 3 x 3, a step, 392 us | 393 with eight, 32 x 3 x
-// 224 x 224 -> 64 by 7 x 7 at stride 2 418 | 420, 16 x 128 x 28 x 28 -> 128 by 3 x 3 145 | 146), and weight gradients whose ranges are longer than one are further off:
-// 3.00e-7 | 2.32e-7 from the sums in 64 bits, 3.08 | 2.42, 2.78 | 2.13; layers in groups, which have fewer ranges as items of one launch, 3.01 | 2.23
-// (4 x 24 x 64 x 64 -> 32 by 5 x 5 in 4 groups; 2.26 with a launch and ranges of its own for each group).
-static int chain_steps(int64_t n) {
+// up: the largest power of two within n, from one K-step to sixteen (256 multiply-adds; longer chains gain no time), to eight in the weight
+// gradients of layers in groups, which share the ranges that fill the CUs: theirs are fewer and longer.  Relative error with ranges for each group |
+// shared ones in chains of 256 | of 128: 4 x 24 x 64 x 64 -> 32 by 5 x 5 in 4 groups 2.26e-7 | 3.01e-7 | 2.23e-7, 192 x 29^3 -> 48 by 3 x 3 x 3 at stride 2
+// in 4 groups 2.14e-7 | 2.59e-7 | 1.95e-7.  Without groups 128 costs 0.6 % of a step (4 x 32 x 32^3 -> 64 by 3 x 3 x 3 395.3 | 397.7 us).
+static int chain_steps(int64_t n, int most = 16) {
     int steps = 1;
-    while (steps < 8 && 32 * steps <= n) steps *= 2;
+    while (steps < most && 32 * steps <= n) steps *= 2;
     return steps;
 }
 
@@ -2007,7 +2007,7 @@ static int conv_dkernel_nhwc(int dtype, const DkernelPlan& pl, const void* image
     p.conv.chan = (int)chp;                        // elements from one pixel to the next
     p.conv.halo = halo.on ? 1 : 0;
     p.conv.tile_rows = pl.rows; p.conv.tile_cols = pl.cols;
-    p.conv.k_segment = chain_steps(L);
+    p.conv.k_segment = chain_steps(L, groups > 1 ? 8 : 16);
     if (pl.ranges) {
         p.conv.k_ranges = 1;
         p.conv.k_total = (int)(batch * L);
