@@ -1,4 +1,5 @@
-"""The forms a convolution is computed in on the device, each against the sums in 64 bits: groups as items of one launch.
+"""The forms a convolution is computed in on the device, each against the sums in 64 bits: that every product is there once, at the edges of tiles, slots,
+ranges and groups.  (The bound holds for any order of summation; what an order costs in precision is held to in test_gpu_conv_precision.py.)
 
 The bound: an output of n products is rounded once to its type (unit roundoff u; Float16 below 2^-14: 2^-25) after a sum in 32 bits whose error
 is at most n 2^-24 times the sum of the products' magnitudes.  Where parts of the sum are stored in the type on the way (the entries of a col
